@@ -44,17 +44,17 @@ def _case(name, model, layers, users=0, context=0, prompts=0, length=0):
 def listed():
     return [
         # one person chatting with the flagship model
-        _case("8b, 1 user", "llama3-8b", 0, 1, 300),
+        _case("8b 1 user", "llama3-8b", 0, 1, 300),
         # the headline workload: 32 concurrent users of the flagship model
-        _case("8b, 32 users", "llama3-8b", 0, 32, 512),
+        _case("8b 32 users", "llama3-8b", 0, 32, 512),
         # a busy node: the largest batches that a worker captures
-        _case("busy node, 128 users", "llama3-8b", 4, 128, 700),
+        _case("busy node 128 users", "llama3-8b", 4, 128, 700),
         # questions about long documents: the cache outweighs the weights
-        _case("long context, 12 users", "llama3.1-8b", 4, 12, 8192),
+        _case("long context 12 users", "llama3.1-8b", 4, 12, 8192),
         # grouped heads in sevens, biases, and an odd batch above 32
-        _case("qwen2, 45 users", "qwen2-7b", 4, 45, 600),
+        _case("qwen2 45 users", "qwen2-7b", 4, 45, 600),
         # no grouped heads: four times the keys and values per token
-        _case("llama2, 20 users", "llama2-7b", 4, 20, 1100),
+        _case("llama2 20 users", "llama2-7b", 4, 20, 1100),
         # the first line of a chat, nobody else there
         _case("short prompt", "llama3-8b", 4, prompts=1, length=37),
         # several requests admitted together
@@ -64,9 +64,9 @@ def listed():
         # a prompt admitted while others are being answered
         _case("prompt among 24 users", "llama3-8b", 4, 24, 800, 1, 517),
         # recurrent, softmax and latent layers: a small model's decode ...
-        _case("kavedra 1b, 32 users", "kavedra-1b", 4, 32, 512),
+        _case("kavedra 1b 32 users", "kavedra-1b", 4, 32, 512),
         # ... and a large one's prompts
-        _case("kavedra 8b, prompts", "kavedra-8b", 4, prompts=2,
+        _case("kavedra 8b prompts", "kavedra-8b", 4, prompts=2,
               length=2048),
     ]
 
