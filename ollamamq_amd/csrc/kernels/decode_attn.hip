@@ -1,400 +1,256 @@
-// gfx950 decode attention with KV-length splitting (flash-decoding style).
+// gfx950 decode attention over paged keys and values, heads of 128.
 //
-// Problem shape: B sequences × Hq heads × 1 query token, paged KV pool,
-// GQA group G = Hq/KVH.  Memory-bound: the whole job is streaming each
-// sequence's K+V (seq_len × 512 B per kv-head) once.  A (seq, kv-head)
-// grid alone gives B×KVH blocks (256 at B=32 ⇒ 1 workgroup/CU, far too
-// few to hide HBM latency — measured 0.65 TB/s).  Splitting the KV length
-// into SPLIT segments multiplies parallelism: each block computes a
-// partial (o, m, l) over its segment; a small combine kernel merges the
-// online-softmax partials exactly.
+// One query token per sequence, G = Hq / KVH query heads per key/value head:
+// the work is to read every cached key and value once, 512 bytes per token
+// and key/value head.  A block of eight waves takes a (sequence, key/value
+// head), or one of `split` parts of it; its G heads are the columns of a
+// 16-wide matrix tile, so a byte is read once for all of them.
 //
-// LDS: K/V chunk tiles shared by the group's G waves (each KV byte read
-// once per kv-head, not per q-head); rows padded +4 bf16 to keep per-lane
-// row reads conflict-free (guide §6 G4).
-#include <hip/hip_runtime.h>
-#include <hip/hip_bf16.h>
-#include <cstdint>
+// Every wave walks its own steps of 32 keys with its own maximum and sum, and
+// nothing passes through LDS before the one merge at the end:
+//  * a key row is the row operand of mfma_16x16x32 as it lies in memory;
+//  * values are loaded as whole rows (four of them per instruction) and
+//    turned in registers: a lane holds columns 8c..8c+7 of the eight keys
+//    whose weights it holds, and 32 byte permutes make of them the operands
+//    of eight value tiles (tile v has the columns 8c + v);
+//  * both are requested a step ahead, 16 KB in flight per wave.
+// Weights stay fp32: they enter the product with the values as three bf16
+// terms, which hold all 24 bits.
+//
+// Bound by memory: 5.2 TB/s over large caches, where a device copy makes 4.7.
+// Before, keys and values went through LDS for products on the vector units,
+// one head a wave (32 heads, 8 of them key/value heads, unless said):
+//   32 users, 256 to 768 tokens                34.2 us, now 17.5
+//   128 users, 350 to 1050                      131 us, now 70
+//   12 users, 4096 to 12288                     144 us, now 83
+//   45 users, 300 to 900, 28 / 4 heads           46 us, now 18.5
+//   20 users, 550 to 1650, 32 / 32 heads        282 us, now 69
+// Loading values through wave-private LDS tiles instead is no faster and
+// costs 70 KB of LDS; non-temporal loads gain 2 us at 128 users and lose as
+// much at 45.
+#include "tile_mma.h"
 
-typedef __hip_bfloat16 bf16;
-typedef __hip_bfloat162 bf162;
+#define NEG (-3.0e38f)
 
-#define DEV static __device__ __forceinline__
-DEV float bf2f(bf16 x) { return __bfloat162float(x); }
+constexpr int D = 128, NW = 8, KT = 32;
 
-DEV void load8f_lds(const bf16* p, float* out) {
-    const bf162* v = reinterpret_cast<const bf162*>(p);
-    float2 f0 = __bfloat1622float2(v[0]), f1 = __bfloat1622float2(v[1]);
-    float2 f2 = __bfloat1622float2(v[2]), f3 = __bfloat1622float2(v[3]);
-    out[0] = f0.x; out[1] = f0.y; out[2] = f1.x; out[3] = f1.y;
-    out[4] = f2.x; out[5] = f2.y; out[6] = f3.x; out[7] = f3.y;
-}
+typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
 
-// fused-chain frag layout for the attention OUTPUT (o-GEMM streams it
-// linearly; see wstream_gemm.hip frag_off): element (m, kcol) ->
-// 16 B unit ((b*4+j)*64 + h*32 + m), kcol = b*64 + j*16 + h*8 + e
-DEV int64_t attn_frag_off(int m, int kcol) {
-    const int b = kcol >> 6, j = (kcol >> 4) & 3, h = (kcol >> 3) & 1;
-    return ((((int64_t)b * 4 + j) * 64) + h * 32 + m) * 8 + (kcol & 7);
-}
-
-DEV float wave_max(float x) {
-    #pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-        x = fmaxf(x, __shfl_down(x, off, 64));
-    return __shfl(x, 0, 64);
-}
-DEV float wave_sum(float x) {
-    #pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-        x += __shfl_down(x, off, 64);
-    return __shfl(x, 0, 64);
-}
-
-#define DCHUNK 64
-#define DHEAD 128
-#define DKPAD 4
-
-// grid: (n_seqs * split, KVH); block: G*64 threads (G templated: the
-// next-chunk register-prefetch array must be compile-time sized, guide
-// rule 20 — runtime-indexed arrays land in scratch).
-// Partials: o_part [S][Hq][split][128] f32, ml_part [S][Hq][split][2] f32.
-// When split == 1, writes normalized bf16 straight to out.
-// launch_bounds min-waves/EU = 1: LDS (~37 KB/block) already caps
-// residency at 4 blocks/CU, so a high compiler occupancy target only
-// forces the prefetch registers to spill (measured 144 B/lane scratch)
-template <int GT, int CH>
-__global__ __launch_bounds__(GT * 64, 1) void k_decode_attn(
-    bf16* __restrict__ out,               // [S, Hq, D] (split==1)
-    float* __restrict__ o_part,           // split>1 partials
-    float* __restrict__ ml_part,
-    const bf16* __restrict__ q,           // [S, Hq, D] (row stride qs)
+// Pages: with SH they are 1 << pshift tokens and no smaller than a tile of
+// 16 keys, so a tile's page number is the same for the whole wave; otherwise
+// any number of tokens, looked up key by key.
+template <bool SH>
+__global__ __launch_bounds__(NW * 64, 2) void k_decode_attn(
+    bf16* __restrict__ out,               // [S, Hq, D] (split == 1)
+    float* __restrict__ o_part,           // [S, Hq, split, D]
+    float* __restrict__ ml_part,          // [S, Hq, split, 2] maximum, sum
+    const bf16* __restrict__ q,           // [S, Hq, D], rows qs apart
     const bf16* __restrict__ kpool,       // [P][KVH][page][D]
     const bf16* __restrict__ vpool,
     const int* __restrict__ page_table,   // [slots][max_pages]
-    const int* __restrict__ slot_ids,     // [S]
-    const int* __restrict__ seq_lens,     // [S] (kv length incl. this tok)
-    int Hq, int KVH, int page, int max_pages, float scale,
-    int64_t qs, int split, int window,    // window 0 = full causal
-    unsigned* __restrict__ sem,           // [S*KVH] tickets (fused combine)
-    int fragout)                          // out in fused-chain frag layout
+    const int* __restrict__ slot_ids, const int* __restrict__ seq_lens,
+    int G, int KVH, int page, int pshift, int max_pages, float unit,
+    int64_t qs, int window, int fragout)
 {
-    const int S_idx = blockIdx.x / split;
-    const int seg = blockIdx.x % split;
-    const int kvh = blockIdx.y;
-    constexpr int G = GT;
-    const int wid = threadIdx.x >> 6;
-    const int lane = threadIdx.x & 63;
-    const int qh = kvh * G + wid;
+    const int kvh = blockIdx.x, seq = blockIdx.y;
+    const int split = gridDim.z, Hq = G * KVH;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, lr = lane & 15, g = lane >> 4;
+    const int kv_len = seq_lens[seq], last = kv_len - 1;
+    const int* pt = page_table + (int64_t)slot_ids[seq] * max_pages;
+    // first key that the query, at kv_len - 1, sees
+    const int lo = window > 0 ? max(0, kv_len - window) : 0;
+    const int first = lo / KT, steps = (kv_len + KT - 1) / KT - first;
+    const int GW = split * NW;            // a wave's steps: every GW-th
+    // a part without keys; the first writes zeros where there are none at all
+    if (blockIdx.z && (int)blockIdx.z * NW >= steps) return;
 
-    constexpr int NTHR = GT * 64;
-    constexpr int NSLOT = CH * (DHEAD / 8);       // uint4 slots per tile
-    constexpr int NPF = (NSLOT + NTHR - 1) / NTHR;  // prefetch regs/thread
-    // Register-prefetch pipeline for every GQA group a preset uses.
-    // Non-dividing groups (G=7, Qwen2: 1024 slots over 448 threads)
-    // clamp the tail slot exactly like the prefill stager — duplicate
-    // threads re-load/re-write identical bytes, which is benign, while a
-    // guarded load/write would de-pipeline the stage (traps (c)).
-    // NPF=8 (G=1 at chunk 32, G=2 at chunk 64) costs 64 VGPRs — free at
-    // the 1-2 wave/SIMD occupancy LDS already imposes there.
-    constexpr bool PF =
-        (NPF <= 8) && (NSLOT % NTHR == 0 || NPF == 3);
+    __shared__ __attribute__((aligned(16))) float o_s[NW * 8 * D];
+    __shared__ float ml_s[NW * 8 * 2];
 
-    const int slot = slot_ids[S_idx];
-    const int kv_len = seq_lens[S_idx];
-    // balanced segment bounds in whole chunks (pages don't straddle
-    // chunks): ceil-div per_seg gave e.g. 9 chunks @ split 4 -> 3,3,3,0
-    // with a whole workgroup idle; floor-interpolated bounds give 2,2,2,3
-    const int n_chunks = (kv_len + CH - 1) / CH;
-    // sliding window: the (single) query sits at kv_len-1, so only keys
-    // >= lo_tok participate; split the ACTIVE chunk range
-    const int lo_tok = (window > 0 && kv_len > window) ? kv_len - window : 0;
-    const int ch_base = lo_tok / CH;
-    const int n_act = n_chunks - ch_base;
-    const int c0 = ch_base + (int)(((int64_t)n_act * seg) / split);
-    const int c1 = ch_base + (int)(((int64_t)n_act * (seg + 1)) / split);
+    bf16x8 qf[4], kf[2][4];
+    u32x4 vr[8];
+    const bf16* qr = q + seq * qs + (kvh * G + min(lr, G - 1)) * D + g * 8;
+    #pragma unroll
+    for (int d = 0; d < 4; d++) qf[d] = frag8(qr + d * 32);
 
-    extern __shared__ __attribute__((aligned(16))) char smem[];
-    const int KROW = DHEAD + DKPAD;
-    bf16* k_tile = reinterpret_cast<bf16*>(smem);
-    bf16* v_tile = k_tile + CH * KROW;
-    float* q_lds = reinterpret_cast<float*>(v_tile + CH * KROW); // [G][128]
-    // p row is per-LANE (65 = 64+pad), NOT per-chunk-key: every lane
-    // stores its p (dead lanes 0.0), so a CH=32 row of 33 floats would
-    // send lanes 32-63 past the row (OOB at G=1, cross-wave race at G>1)
-    float* p_lds = q_lds + (int64_t)G * DHEAD;                       // [G][65]
-
-    // stage q (fp32 in LDS: repeated broadcast reads in the score loop)
-    if (wid < G) {
-        const bf16* qsrc = q + (int64_t)S_idx * qs + (int64_t)qh * DHEAD;
-        q_lds[wid * DHEAD + lane] = bf2f(qsrc[lane]);
-        q_lds[wid * DHEAD + lane + 64] = bf2f(qsrc[lane + 64]);
-    }
-    __syncthreads();
-
-    float m = -3.0e38f, l = 0.f, o0 = 0.f, o1 = 0.f;
-
-    // clamp instead of guarding: a conditional load would de-pipeline the
-    // whole stage (guide §5 traps (c)); the duplicated tail rows are
-    // masked to p=0 by the softmax
-    auto src_of = [&](int base, int u) -> int64_t {
-        const int tok = u / (DHEAD / 8), dv = u % (DHEAD / 8);
-        const int tk = base + tok < kv_len ? base + tok : kv_len - 1;
-        const int gp = page_table[(int64_t)slot * max_pages + tk / page];
-        return (((int64_t)gp * KVH + kvh) * page + tk % page) * DHEAD
-               + dv * 8;
-    };
-    auto stage_direct = [&](int ch2) {
-        const int base2 = ch2 * CH;
-        for (int u = threadIdx.x; u < NSLOT; u += NTHR) {
-            const int tok = u / (DHEAD / 8), dv = u % (DHEAD / 8);
-            const int64_t src = src_of(base2, u);
-            *reinterpret_cast<uint4*>(k_tile + tok * KROW + dv * 8) =
-                *reinterpret_cast<const uint4*>(kpool + src);
-            *reinterpret_cast<uint4*>(v_tile + tok * KROW + dv * 8) =
-                *reinterpret_cast<const uint4*>(vpool + src);
+    // SH: pages of a step's tiles, looked up a step before they are needed
+    int pg[2], next[2];
+    auto pages = [&](int st) {
+        #pragma unroll
+        for (int t = 0; SH && t < 2; t++) {
+            pg[t] = next[t];
+            next[t] = pt[min((first + st) * KT + t * 16, last) >> pshift];
         }
     };
-
-    if (c0 < c1) stage_direct(c0);
-    __syncthreads();
-
-    for (int ch = c0; ch < c1; ch++) {
-        const int base = ch * CH;
-        const int n_here = min(CH, kv_len - base);
-        // ---- issue next chunk's HBM loads NOW, write to LDS after the
-        // compute phase (T14 issue-early/write-late): the fetch rides
-        // under the score/PV work instead of serializing with it.
-        // Named registers, not an array — hipcc demotes even
-        // constant-indexed uint4 arrays here to scratch (24 scratch ops,
-        // 144 B/lane), and a spilled prefetch is HBM traffic, not a win.
-        uint4 k0, k1, k2, k3, v0, v1, v2, v3;
-        uint4 k4, k5, k6, k7, v4, v5, v6, v7;
-        const bool have_next = PF && (ch + 1 < c1);
-        if (have_next) {
-            const int nbase = (ch + 1) * CH;
-            const int64_t s0 = src_of(nbase, threadIdx.x);
-            const int64_t s1 = NPF >= 2 ? src_of(nbase, threadIdx.x + NTHR)
-                                        : s0;
-            k0 = *reinterpret_cast<const uint4*>(kpool + s0);
-            v0 = *reinterpret_cast<const uint4*>(vpool + s0);
-            if constexpr (NPF >= 2) {
-                k1 = *reinterpret_cast<const uint4*>(kpool + s1);
-                v1 = *reinterpret_cast<const uint4*>(vpool + s1);
-            }
-            if constexpr (NPF >= 3) {
-                const int64_t s2 = src_of(
-                    nbase, min((int)threadIdx.x + 2 * NTHR, NSLOT - 1));
-                k2 = *reinterpret_cast<const uint4*>(kpool + s2);
-                v2 = *reinterpret_cast<const uint4*>(vpool + s2);
-            }
-            if constexpr (NPF >= 4) {
-                const int64_t s3 = src_of(nbase, threadIdx.x + 3 * NTHR);
-                k3 = *reinterpret_cast<const uint4*>(kpool + s3);
-                v3 = *reinterpret_cast<const uint4*>(vpool + s3);
-            }
-            if constexpr (NPF >= 8) {
-                const int64_t s4 = src_of(nbase, threadIdx.x + 4 * NTHR);
-                const int64_t s5 = src_of(nbase, threadIdx.x + 5 * NTHR);
-                const int64_t s6 = src_of(nbase, threadIdx.x + 6 * NTHR);
-                const int64_t s7 = src_of(nbase, threadIdx.x + 7 * NTHR);
-                k4 = *reinterpret_cast<const uint4*>(kpool + s4);
-                v4 = *reinterpret_cast<const uint4*>(vpool + s4);
-                k5 = *reinterpret_cast<const uint4*>(kpool + s5);
-                v5 = *reinterpret_cast<const uint4*>(vpool + s5);
-                k6 = *reinterpret_cast<const uint4*>(kpool + s6);
-                v6 = *reinterpret_cast<const uint4*>(vpool + s6);
-                k7 = *reinterpret_cast<const uint4*>(kpool + s7);
-                v7 = *reinterpret_cast<const uint4*>(vpool + s7);
-            }
-        }
-
-        // ---- score for key j = lane ----
-        float s = 0.f;
-        const bool live = lane < n_here && base + lane >= lo_tok;
-        {
-            const bf16* krow = k_tile + lane * KROW;
-            const float* qrow = q_lds + wid * DHEAD;
+    // row of a key within one of the pools
+    auto row = [&](const bf16* pool, int t, int key) {
+        if (SH)
+            return pool + (((int64_t)pg[t] * KVH + kvh) << pshift) * D
+                   + (key & ((1 << pshift) - 1)) * D;
+        return pool + (((int64_t)pt[key / page] * KVH + kvh) * page
+                       + key % page) * D;
+    };
+    // keys past the last are the last again, with a weight of zero
+    auto load_k = [&](int st) {
+        #pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int key = min((first + st) * KT + t * 16 + lr, last);
+            const bf16* r = row(kpool, t, key) + g * 8;
             #pragma unroll
-            for (int d = 0; d < DHEAD; d += 8) {
-                float k8[8];
-                load8f_lds(krow + d, k8);
-                s += k8[0] * qrow[d] + k8[1] * qrow[d + 1]
-                   + k8[2] * qrow[d + 2] + k8[3] * qrow[d + 3]
-                   + k8[4] * qrow[d + 4] + k8[5] * qrow[d + 5]
-                   + k8[6] * qrow[d + 6] + k8[7] * qrow[d + 7];
-            }
-            s = live ? s * scale : -3.0e38f;
+            for (int d = 0; d < 4; d++) kf[t][d] = frag8(r + d * 32);
         }
+    };
+    auto load_v = [&](int st) {
+        #pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const int key = min((first + st) * KT + (e >> 2) * 16 + g * 4
+                                + (e & 3), last);
+            vr[e] = *reinterpret_cast<const u32x4*>(
+                row(vpool, e >> 2, key) + lr * 8);
+        }
+    };
 
-        // ---- online softmax ----
-        const float smax = wave_max(s);
-        float p = 0.f;
-        if (smax > -3.0e38f) {
-            const float mn = fmaxf(m, smax);
-            const float corr = __expf(m - mn);
-            p = live ? __expf(s - mn) : 0.f;
-            l = l * corr + wave_sum(p);
-            o0 *= corr; o1 *= corr;
-            m = mn;
+    float m = NEG, l = 0.f;
+    f32x4 acc[8] = {};
+    int st = blockIdx.z * NW + wid;
+    if (st < steps) {
+        pages(st);
+        pages(st + GW);
+        load_k(st);
+        load_v(st);
+    }
+    for (; st < steps; st += GW) {
+        const bool more = st + GW < steps;
+        f32x4 s[2] = {};
+        #pragma unroll
+        for (int d = 0; d < 4; d++) {
+            s[0] = mma(kf[0][d], qf[d], s[0]);
+            s[1] = mma(kf[1][d], qf[d], s[1]);
         }
-        p_lds[wid * 65 + lane] = p;
-
-        // ---- PV: lane accumulates dims (2*lane, 2*lane+1) ----
-        // fixed bound + full unroll: a runtime bound left this loop a
-        // serial ds_read latency chain (PMC: 25% SQ_WAIT_INST_ANY);
-        // dead keys contribute p=0 so looping to CH is exact
-        const float* prow = p_lds + wid * 65;
-        #pragma unroll 8
-        for (int j = 0; j < CH; j++) {
-            const bf162 v2 = *reinterpret_cast<const bf162*>(
-                v_tile + j * KROW + 2 * lane);
-            const float pj = prow[j];
-            o0 = fmaf(pj, bf2f(v2.x), o0);
-            o1 = fmaf(pj, bf2f(v2.y), o1);
+        if (more) {
+            pages(st + 2 * GW);
+            load_k(st + GW);
         }
-        __syncthreads();  // every wave done reading the k/v tiles
-        if (have_next) {
-            auto put = [&](int u, uint4 kx, uint4 vx) {
-                const int tok = u / (DHEAD / 8), dv = u % (DHEAD / 8);
-                *reinterpret_cast<uint4*>(k_tile + tok * KROW + dv * 8)
-                    = kx;
-                *reinterpret_cast<uint4*>(v_tile + tok * KROW + dv * 8)
-                    = vx;
-            };
-            put(threadIdx.x, k0, v0);
-            if constexpr (NPF >= 2) put(threadIdx.x + NTHR, k1, v1);
-            if constexpr (NPF >= 3)
-                put(min((int)threadIdx.x + 2 * NTHR, NSLOT - 1), k2, v2);
-            if constexpr (NPF >= 4) put(threadIdx.x + 3 * NTHR, k3, v3);
-            if constexpr (NPF >= 8) {
-                put(threadIdx.x + 4 * NTHR, k4, v4);
-                put(threadIdx.x + 5 * NTHR, k5, v5);
-                put(threadIdx.x + 6 * NTHR, k6, v6);
-                put(threadIdx.x + 7 * NTHR, k7, v7);
+        // scores of the keys base + 16 j + 4 g + i for head lr
+        const int base = (first + st) * KT;
+        const bool inside = base >= lo && base + KT <= kv_len;
+        float mx = NEG;
+        #pragma unroll
+        for (int j = 0; j < 2; j++)
+            #pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int key = base + j * 16 + g * 4 + i;
+                float v = s[j][i] * unit;
+                if (!inside && (key < lo || key > last)) v = NEG;
+                s[j][i] = v;
+                mx = fmaxf(mx, v);
             }
-            __syncthreads();  // tiles ready for next iteration
-        } else if (!PF && ch + 1 < c1) {
-            stage_direct(ch + 1);
-            __syncthreads();
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float mn = fmaxf(m, mx), ref = mn > NEG ? mn : 0.f;
+        const float f = __builtin_amdgcn_exp2f(m - ref);
+        m = mn;
+        float sum = 0.f;
+        bf16x8 w0, w1, w2;
+        #pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float p = __builtin_amdgcn_exp2f(s[e >> 2][e & 3] - ref);
+            sum += p;
+            w0[e] = (__bf16)p;
+            const float r = p - (float)w0[e];
+            w1[e] = (__bf16)r;
+            w2[e] = (__bf16)(r - (float)w1[e]);
+        }
+        l = l * f + sum;                  // of this lane's keys only
+        #pragma unroll
+        for (int v = 0; v < 8; v++) acc[v] *= f;
+        #pragma unroll
+        for (int v = 0; v < 8; v++) {
+            u32x4 a;
+            #pragma unroll
+            for (int k = 0; k < 4; k++)
+                a[k] = __builtin_amdgcn_perm(
+                    vr[2 * k + 1][v >> 1], vr[2 * k][v >> 1],
+                    v & 1 ? 0x07060302u : 0x05040100u);
+            const bf16x8 af = __builtin_bit_cast(bf16x8, a);
+            acc[v] = mma(af, w2, acc[v]);
+            acc[v] = mma(af, w1, acc[v]);
+            acc[v] = mma(af, w0, acc[v]);
+        }
+        if (more) load_v(st + GW);
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+
+    // the waves meet: head lr, columns 8 (4 g + i) + v
+    if (lr < G) {
+        #pragma unroll
+        for (int i = 0; i < 4; i++) {
+            f32x4* d = reinterpret_cast<f32x4*>(
+                o_s + (wid * G + lr) * D + (g * 4 + i) * 8);
+            d[0] = f32x4{acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
+            d[1] = f32x4{acc[4][i], acc[5][i], acc[6][i], acc[7][i]};
+        }
+        if (g == 0) {
+            ml_s[(wid * G + lr) * 2] = m;
+            ml_s[(wid * G + lr) * 2 + 1] = l;
         }
     }
-
-    // ---- emit ----
+    __syncthreads();
+    if (threadIdx.x >= G * (D / 4)) return;
+    const int h = threadIdx.x / (D / 4), c = (threadIdx.x % (D / 4)) * 4;
+    float top = NEG, den = 0.f;
+    #pragma unroll
+    for (int w = 0; w < NW; w++) top = fmaxf(top, ml_s[(w * G + h) * 2]);
+    f32x4 sum = {};
+    #pragma unroll
+    for (int w = 0; w < NW; w++) {
+        const float f = __builtin_amdgcn_exp2f(ml_s[(w * G + h) * 2] - top);
+        den += f * ml_s[(w * G + h) * 2 + 1];
+        sum += f * *reinterpret_cast<const f32x4*>(o_s + (w * G + h) * D + c);
+    }
+    const int hq = kvh * G + h;
     if (split == 1) {
-        const float linv = l > 0.f ? 1.f / l : 0.f;
-        const bf162 ov =
-            __float22bfloat162_rn(make_float2(o0 * linv, o1 * linv));
-        if (fragout)
-            *reinterpret_cast<bf162*>(
-                out + (int64_t)(S_idx >> 5) * 32 * Hq * DHEAD
-                    + attn_frag_off(S_idx & 31, qh * DHEAD + 2 * lane))
-                = ov;
-        else
-            reinterpret_cast<bf162*>(
-                out + ((int64_t)S_idx * Hq + qh) * DHEAD)[lane] = ov;
+        sum *= den > 0.f ? 1.f / den : 0.f;
+        put_out(out, seq, hq, c, Hq, D, sum, fragout);
         return;
     }
-    {
-        const int64_t pi = (((int64_t)S_idx * Hq + qh) * split + seg);
-        float* op = o_part + pi * DHEAD;
-        op[2 * lane] = o0;
-        op[2 * lane + 1] = o1;
-        ml_part[pi * 2] = m;
-        ml_part[pi * 2 + 1] = l;
-    }
-    if (sem == nullptr) return;   // separate k_decode_combine pass (A/B)
-
-    // ---- in-launch combine (guide §6 G16 split-K recipe): publish the
-    // partials with an agent-scope release BEFORE the ticket fetch_add;
-    // the block that draws split-1 acquires and reduces its (seq, kvh)
-    // group — saves the combine kernel's launch boundary + HBM round trip
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();              // all waves' partials issued
-    int* flag = reinterpret_cast<int*>(smem);   // tiles are dead; reuse
-    if (threadIdx.x == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        // restate the post-wbl2 wait the compiler may drop (pitfall 12)
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        const unsigned t = __hip_atomic_fetch_add(
-            &sem[(int64_t)S_idx * gridDim.y + kvh], 1u,
-            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        *flag = (t == (unsigned)(split - 1)) ? 1 : 0;
-    }
-    __syncthreads();
-    if (*flag == 0) return;
-    if (threadIdx.x == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        // reset for the next launch (stream-ordered; all arrivals done)
-        __hip_atomic_store(&sem[(int64_t)S_idx * gridDim.y + kvh], 0u,
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();              // acquire visible to the whole block
-    {
-        // wave `wid` reduces its head, lane covers dims (2*lane, 2*lane+1)
-        const int64_t sh = (int64_t)S_idx * Hq + qh;
-        float mm = -3.0e38f;
-        for (int i = 0; i < split; i++)
-            mm = fmaxf(mm, ml_part[(sh * split + i) * 2]);
-        float ll = 0.f, a0 = 0.f, a1 = 0.f;
-        for (int i = 0; i < split; i++) {
-            const int64_t pi = sh * split + i;
-            const float mi = ml_part[pi * 2];
-            if (mi <= -3.0e38f) continue;
-            const float w = __expf(mi - mm);
-            ll += w * ml_part[pi * 2 + 1];
-            const float* op = o_part + pi * DHEAD;
-            a0 = fmaf(w, op[2 * lane], a0);
-            a1 = fmaf(w, op[2 * lane + 1], a1);
-        }
-        const float linv = ll > 0.f ? 1.f / ll : 0.f;
-        if (fragout) {
-            *reinterpret_cast<bf162*>(
-                out + (int64_t)(S_idx >> 5) * 32 * Hq * DHEAD
-                    + attn_frag_off(S_idx & 31, qh * DHEAD + 2 * lane)) =
-                __float22bfloat162_rn(
-                    make_float2(a0 * linv, a1 * linv));
-            return;
-        }
-        reinterpret_cast<bf162*>(out + sh * DHEAD)[lane] =
-            __float22bfloat162_rn(make_float2(a0 * linv, a1 * linv));
+    const int64_t part = ((int64_t)seq * Hq + hq) * split + blockIdx.z;
+    *reinterpret_cast<f32x4*>(o_part + part * D + c) = sum;
+    if (c == 0) {
+        ml_part[part * 2] = top;
+        ml_part[part * 2 + 1] = den;
     }
 }
 
-// combine: one wave per (seq, head); merges the split online-softmax
-// partials exactly: m* = max m_i; o = Σ e^{m_i-m*} o_i; l = Σ e^{m_i-m*} l_i
+// merge of the parts: 32 lanes per (sequence, head)
 __global__ __launch_bounds__(256) void k_decode_combine(
     bf16* __restrict__ out, const float* __restrict__ o_part,
-    const float* __restrict__ ml_part, int total, int split,
-    int Hq, int fragout)
+    const float* __restrict__ ml_part, const int* __restrict__ seq_lens,
+    int total, int split, int Hq, int window, int fragout)
 {
-    const int sh = blockIdx.x * 4 + (threadIdx.x >> 6);  // seq*Hq + head
-    const int lane = threadIdx.x & 63;
+    const int sh = blockIdx.x * 8 + threadIdx.x / 32;
+    const int c = (threadIdx.x % 32) * 4;
     if (sh >= total) return;
-    float m = -3.0e38f;
-    for (int i = 0; i < split; i++)
-        m = fmaxf(m, ml_part[((int64_t)sh * split + i) * 2]);
-    float l = 0.f, a0 = 0.f, a1 = 0.f;
-    for (int i = 0; i < split; i++) {
-        const int64_t pi = (int64_t)sh * split + i;
-        const float mi = ml_part[pi * 2];
-        if (mi <= -3.0e38f) continue;
-        const float w = __expf(mi - m);
-        l += w * ml_part[pi * 2 + 1];
-        const float* op = o_part + pi * DHEAD;
-        a0 = fmaf(w, op[2 * lane], a0);
-        a1 = fmaf(w, op[2 * lane + 1], a1);
+    // parts that have keys: the first step of the last of them exists
+    const int kv_len = seq_lens[sh / Hq];
+    const int lo = window > 0 ? max(0, kv_len - window) : 0;
+    const int steps = (kv_len + KT - 1) / KT - lo / KT;
+    const int parts = min(split, (steps + NW - 1) / NW);
+    const float* ml = ml_part + (int64_t)sh * split * 2;
+    const float* o = o_part + (int64_t)sh * split * D + c;
+    float top = NEG, den = 0.f;
+    for (int i = 0; i < parts; i++) top = fmaxf(top, ml[i * 2]);
+    f32x4 sum = {};
+    #pragma unroll 4
+    for (int i = 0; i < parts; i++) {
+        const float f = __builtin_amdgcn_exp2f(ml[i * 2] - top);
+        den += f * ml[i * 2 + 1];
+        sum += f * *reinterpret_cast<const f32x4*>(o + i * D);
     }
-    const float linv = l > 0.f ? 1.f / l : 0.f;
-    const bf162 ov =
-        __float22bfloat162_rn(make_float2(a0 * linv, a1 * linv));
-    if (fragout)
-        *reinterpret_cast<bf162*>(
-            out + (int64_t)((sh / Hq) >> 5) * 32 * Hq * DHEAD
-                + attn_frag_off((sh / Hq) & 31,
-                                (sh % Hq) * DHEAD + 2 * lane)) = ov;
-    else
-        reinterpret_cast<bf162*>(out + (int64_t)sh * DHEAD)[lane] = ov;
+    sum *= den > 0.f ? 1.f / den : 0.f;
+    put_out(out, sh / Hq, sh % Hq, c, Hq, D, sum, fragout);
 }
 
 extern "C" int decode_attn_bf16(
@@ -402,98 +258,24 @@ extern "C" int decode_attn_bf16(
     const void* kpool, const void* vpool, const void* page_table,
     const void* slot_ids, const void* seq_lens, int S, int Hq, int KVH,
     int page, int max_pages, float scale, int64_t q_stride, int split,
-    int window, int chunk, void* sem, int fragout, hipStream_t stream)
+    int window, int fragout, hipStream_t stream)
 {
     const int G = Hq / KVH;
-    const int lds = 2 * chunk * (DHEAD + DKPAD) * 2 + G * DHEAD * 4
-                  + G * 65 * 4;
-    dim3 grid(S * split, KVH);
-#define DA_LAUNCH1(GT, CH)                                                \
-    k_decode_attn<GT, CH><<<grid, GT * 64, lds, stream>>>(                \
-        (bf16*)out, (float*)o_part, (float*)ml_part, (const bf16*)q,      \
-        (const bf16*)kpool, (const bf16*)vpool, (const int*)page_table,   \
-        (const int*)slot_ids, (const int*)seq_lens, Hq, KVH, page,        \
-        max_pages, scale, q_stride, split, window, (unsigned*)sem,     \
-        fragout)
-// chunk is capped at 64: the score phase assigns ONE key per lane of a
-// wave64, so a larger staged chunk would silently drop keys 64+ (a 128
-// arm measured wrong before this guard)
-#define DA_LAUNCH(GT)                                                     \
-    switch (chunk) {                                                      \
-        case 32: DA_LAUNCH1(GT, 32); break;                               \
-        default: DA_LAUNCH1(GT, 64); break;                               \
-    }
-    switch (G) {
-        case 1: DA_LAUNCH(1); break;
-        case 2: DA_LAUNCH(2); break;
-        case 3: DA_LAUNCH(3); break;
-        case 4: DA_LAUNCH(4); break;
-        case 5: DA_LAUNCH(5); break;
-        case 6: DA_LAUNCH(6); break;
-        case 7: DA_LAUNCH(7); break;
-        case 8: DA_LAUNCH(8); break;
-        default: return (int)hipErrorInvalidValue;
-    }
-#undef DA_LAUNCH
-#undef DA_LAUNCH1
-    if (split > 1 && sem == nullptr) {
-        const int waves = S * Hq;
-        k_decode_combine<<<(waves + 3) / 4, 256, 0, stream>>>(
-            (bf16*)out, (const float*)o_part, (const float*)ml_part, waves,
-            split, Hq, fragout);
-    }
-    return (int)hipGetLastError();
-}
-
-// Pure-stage diagnostic: identical grid/segmentation/addressing to
-// k_decode_attn but ONLY the KV loads (no LDS, no score/PV, no
-// barriers) — the staging stream ceiling of this geometry.  If this
-// matches the real kernel's time, the kernel is geometry/bandwidth
-// capped and compute-side pipelining cannot help.
-__global__ __launch_bounds__(256) void k_decode_pure(
-    float* __restrict__ sink, const bf16* __restrict__ kpool,
-    const bf16* __restrict__ vpool, const int* __restrict__ page_table,
-    const int* __restrict__ slot_ids, const int* __restrict__ seq_lens,
-    int KVH, int page, int max_pages, int split, int chunk)
-{
-    const int S_idx = blockIdx.x / split;
-    const int seg = blockIdx.x % split;
-    const int kvh = blockIdx.y;
-    const int slot = slot_ids[S_idx];
-    const int kv_len = seq_lens[S_idx];
-    const int n_chunks = (kv_len + chunk - 1) / chunk;
-    const int c0 = (int)(((int64_t)n_chunks * seg) / split);
-    const int c1 = (int)(((int64_t)n_chunks * (seg + 1)) / split);
-    const int nslot = chunk * 16;
-    unsigned acc = 0;
-    for (int ch = c0; ch < c1; ch++) {
-        const int base = ch * chunk;
-        for (int u = threadIdx.x; u < nslot; u += 256) {
-            const int tok = u >> 4, dv = u & 15;
-            const int tk = base + tok < kv_len ? base + tok : kv_len - 1;
-            const int gp = page_table[(int64_t)slot * max_pages
-                                      + tk / page];
-            const int64_t src =
-                (((int64_t)gp * KVH + kvh) * page + tk % page) * 128
-                + dv * 8;
-            const uint4 k = *reinterpret_cast<const uint4*>(kpool + src);
-            const uint4 v = *reinterpret_cast<const uint4*>(vpool + src);
-            acc ^= k.x ^ k.w ^ v.x ^ v.w;
-        }
-    }
-    if (acc == 0xDEADBEEFu) sink[0] = 1.f;
-}
-
-extern "C" int decode_pure_bf16(
-    void* sink, const void* kpool, const void* vpool,
-    const void* page_table, const void* slot_ids, const void* seq_lens,
-    int S, int KVH, int page, int max_pages, int split, int chunk,
-    hipStream_t stream)
-{
-    dim3 grid(S * split, KVH);
-    k_decode_pure<<<grid, 256, 0, stream>>>(
-        (float*)sink, (const bf16*)kpool, (const bf16*)vpool,
-        (const int*)page_table, (const int*)slot_ids,
-        (const int*)seq_lens, KVH, page, max_pages, split, chunk);
+    if (G < 1 || G > 8 || G * KVH != Hq || page < 1
+        || (reinterpret_cast<uintptr_t>(q) & 15) || q_stride % 8)
+        return (int)hipErrorInvalidValue;
+    const bool sh = page >= 16 && !(page & (page - 1));
+    const float unit = scale * 1.4426950408889634f;
+    auto go = sh ? k_decode_attn<true> : k_decode_attn<false>;
+    go<<<dim3(KVH, S, split), NW * 64, 0, stream>>>(
+        (bf16*)out, (float*)o_part, (float*)ml_part, (const bf16*)q,
+        (const bf16*)kpool, (const bf16*)vpool, (const int*)page_table,
+        (const int*)slot_ids, (const int*)seq_lens, G, KVH, page,
+        sh ? __builtin_ctz(page) : 0, max_pages, unit, q_stride, window,
+        fragout);
+    if (split > 1)
+        k_decode_combine<<<(S * Hq + 7) / 8, 256, 0, stream>>>(
+            (bf16*)out, (const float*)o_part, (const float*)ml_part,
+            (const int*)seq_lens, S * Hq, split, Hq, window, fragout);
     return (int)hipGetLastError();
 }

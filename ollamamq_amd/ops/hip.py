@@ -48,8 +48,7 @@ def _try_load():
     lib.argmax_bf16.argtypes = [vp, vp, i, i, vp, vp, i, vp]
     lib.argmax_f32.argtypes = lib.argmax_bf16.argtypes
     lib.decode_attn_bf16.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp,
-                                     i, i, i, i, i, f, i64, i, i, i, vp,
-                                     i, vp]
+                                     i, i, i, i, i, f, i64, i, i, i, vp]
     lib.skinny_gemm_bf16.argtypes = [vp, vp, vp, vp, i, i, i, i64, i, vp]
     lib.skinny_direct_bf16.argtypes = [vp, vp, vp, vp, i, i, i, i64, i, vp]
     lib.rope_append_bf16.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp, vp,
@@ -66,8 +65,6 @@ def _try_load():
     lib.fragify_sumsq_bf16.argtypes = [vp, vp, vp, i, i, vp]
     lib.sample_gumbel_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i, i,
                                        vp, vp, i, vp]
-    lib.decode_pure_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i, i, i, i,
-                                     i, i, vp]
     lib.wstream_qkv_rope_bf16.argtypes = [vp, vp, vp, vp, i, i, i, i64,
                                           vp, i, f, f, vp, vp, vp, vp,
                                           vp, vp, vp, i, i, i, i, i, vp]
@@ -320,84 +317,46 @@ def _attention(q, cache, layer, meta, qt):
     return out
 
 
-_scratch = {}
+def _decode_split(pairs, max_kv):
+    """Parts of a context, for `pairs` (sequence, key/value head) pairs.  From
+    192 pairs on the chip has a block a CU and one part is best (32 users of
+    about 512 tokens, 8 key/value heads: 18.2 us against 20.9 with two and
+    their merge); below, up to 768 blocks help where contexts are long or
+    ragged (12 users of 4096 to 12288: 149 us whole, 91 in two, 80 in
+    eight).  A part has at least a step of 32 keys for each of its eight
+    waves."""
+    env = os.environ.get("OLLAMAMQ_DECODE_SPLIT")
+    if env:                       # tuning override (tools/perf_decode.py)
+        want = int(env)
+    else:
+        want = 1 if pairs >= 192 else 768 // max(1, pairs)
+    return min(want, max(1, (max_kv + 255) // 256), 32)
 
 
-def _decode_scratch(S, Hq, split, dev):
-    key = (S, Hq, split, str(dev))
-    t = _scratch.get(key)
-    if t is None:
-        t = (torch.empty(S * Hq * split * 128, dtype=torch.float32,
-                         device=dev),
-             torch.empty(S * Hq * split * 2, dtype=torch.float32,
-                         device=dev))
-        _scratch[key] = t
-    return t
-
-
-def _combine_sem(S, KVH, dev):
-    """Ticket counters for the in-launch split-K combine: zero-initialized
-    once; the last-arriving block resets its counter, so the buffer is
-    always all-zero between launches (guide G16 counter recipe)."""
-    key = ("sem", S, KVH, str(dev))
-    t = _scratch.get(key)
-    if t is None:
-        t = torch.zeros(S * KVH, dtype=torch.int32, device=dev)
-        _scratch[key] = t
-    return t
-
-
-# staged KV chunk length (tokens) per pipeline stage; 32/64 compiled
-# (the kernel scores one key per wave64 lane, so 64 is the ceiling).
-# 64 wins for GQA groups >= 2 (sweep in NOTES.md); G=1 (MHA, Llama-2)
-# takes 32 so the register-prefetch pipeline fits (NPF=8) — measured
-# 142.9 -> 101.4 us at ctx 512 (see NOTES.md)
-_CHUNK_ENV = os.environ.get("OLLAMAMQ_DECODE_CHUNK")
-
-
-def _decode_chunk(G):
-    if _CHUNK_ENV:
-        return min(64, int(_CHUNK_ENV))
-    return 32 if G == 1 else 64
-
-
-def attention_decode(q, cache, layer, meta, fragout=False):
-    """Flash-decoding: KV-split partials + exact online-softmax combine.
-
-    The split factor targets ≥1024 workgroups so the memory-bound KV sweep
-    fills the 256-CU chip (a bare (seq, kv-head) grid at batch 32 is 1
-    workgroup/CU and runs at ~10% of HBM bandwidth).
+def attention_decode(q, cache, layer, meta, fragout=False, out=None):
+    """Attention of one query token per sequence over its paged keys and
+    values, the context of a (sequence, key/value head) in parts while there
+    are few of them.
     fragout: emit the output in the fused-chain 32-row frag layout (the
     o GEMM streams it linearly like packed weights)."""
     S, Hq, D = q.shape
     assert D == 128
-    out = torch.empty((((S + 31) // 32) * 32 * Hq * D,)
-                      if fragout else (S, Hq, D),
-                      dtype=q.dtype, device=q.device)
+    if out is None:
+        out = torch.empty((((S + 31) // 32) * 32 * Hq * D,)
+                          if fragout else (S, Hq, D),
+                          dtype=q.dtype, device=q.device)
+    if not S:
+        return out
+    if q.data_ptr() % 16 or _row_stride(q, D) % 8:
+        q = q.clone(memory_format=torch.contiguous_format)
     kp, vp = _layer_ptrs(cache, layer)
     kvh = cache.n_kv_heads
-    # target ~1024 blocks; under graph capture max_kv is the pool's
-    # max_ctx, so an unconditional max-split would freeze in dozens of
-    # empty segments per sequence (measured: 5.55k -> 4.3k tok/s)
-    want = max(1, 1024 // max(1, S * kvh))
-    env = os.environ.get("OLLAMAMQ_DECODE_SPLIT")
-    if env:                       # tuning override (tools/perf_decode.py)
-        want = int(env)
-    max_seg = max(1, (meta.max_kv + 63) // 64)
-    split = int(min(want, max_seg, 32))
-    o_part, ml_part = (None, None)
+    split = _decode_split(S * kvh, meta.max_kv)
     op = mp = ctypes.c_void_p(0)
-    sem = ctypes.c_void_p(0)
     if split > 1:
-        o_part, ml_part = _decode_scratch(S, Hq, split, q.device)
-        op, mp = _p(o_part), _p(ml_part)
-        # in-launch combine measured WORSE (41.8 vs 29.3 us @ctx512 B32;
-        # bench 5131 vs 5580): all S*split*KVH blocks pay the agent-scope
-        # release fence (buffer_wbl2, ~1.7-6.5 us at 4 blocks/CU) to save
-        # one 5 us combine launch. Kept for re-evaluation on shapes with
-        # fewer, longer blocks.
-        if os.environ.get("OLLAMAMQ_FUSED_COMBINE") == "1":
-            sem = _p(_combine_sem(S, kvh, q.device))
+        part = torch.empty(S * Hq * split * (D + 2), dtype=torch.float32,
+                           device=q.device)
+        op, mp = _p(part), _p(part[S * Hq * split * D:])
     slot32 = meta.slot_ids.int() if meta.slot_ids.dtype != torch.int32 \
         else meta.slot_ids
     len32 = meta.seq_lens.int() if meta.seq_lens.dtype != torch.int32 \
@@ -406,8 +365,7 @@ def attention_decode(q, cache, layer, meta, fragout=False):
         _p(out), op, mp, _p(q), kp, vp, _p(cache.page_table),
         _p(slot32), _p(len32), S, Hq, kvh, cache.page_size,
         cache.page_table.shape[1], 1.0 / (D ** 0.5), _row_stride(q, D),
-        split, meta.window, _decode_chunk(Hq // kvh), sem,
-        1 if fragout else 0, _stream()),
+        split, meta.window, 1 if fragout else 0, _stream()),
         "decode_attn")
     return out
 
@@ -429,7 +387,7 @@ def attention_mixed(q, cache, layer, meta):
             max_kv=meta.max_kv, window=meta.window)
         meta._mixed_dec = sub
     if nd:
-        out[:nd] = attention_decode(q[:nd], cache, layer, sub)
+        attention_decode(q[:nd], cache, layer, sub, out=out)
     # ---- prefill part (tiles over sequences nd..) ----
     plan = getattr(meta, "_mixed_plan", None)
     if plan is None:
@@ -1958,6 +1916,9 @@ def moe_experts(h, w, chosen, share, packs):
     return Weighted(out, share)
 
 
+_scratch = {}
+
+
 def sample_gumbel(logits, temps, seeds, ctrs, noise=None, out=None):
     """Exact temperature sampling (Gumbel-max): token ~ softmax(l/T) per
     row; rows with temps<=0 are greedy argmax.  Counter-based noise from
@@ -2054,17 +2015,3 @@ def sample(logits, temperature, top_k, top_p, generator=None):
         return out_s
     # greedy rows override with the true argmax
     return torch.where(stoch, out_s, l.argmax(-1))
-
-
-def decode_pure(cache, layer, meta, split, chunk=64):
-    """Staging-only diagnostic for decode attention (see decode_attn.hip
-    k_decode_pure)."""
-    sink = torch.zeros(1, dtype=torch.float32, device=cache.k_pool.device)
-    kp, vp = _layer_ptrs(cache, layer)
-    S = meta.slot_ids.shape[0]
-    _check(_lib.decode_pure_bf16(
-        _p(sink), kp, vp, _p(cache.page_table), _p(meta.slot_ids.int()),
-        _p(meta.seq_lens.int()), S, cache.n_kv_heads, cache.page_size,
-        cache.page_table.shape[1], split, chunk, _stream()),
-        "decode_pure")
-    return sink

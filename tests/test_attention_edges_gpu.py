@@ -1,0 +1,118 @@
+"""The attention kernels of the Llama path at the edges of their tiles, against
+float64.
+
+Tolerance: the result is rounded once to bf16 (relative 2^-9, doubled for ties
+and for sums of fp32 products), decode keeps weights in fp32; the absolute part
+covers results that cancel: 128 to 4000 products of size one with errors of
+2^-24 each.
+"""
+import pytest
+import torch
+
+from ollamamq_amd.engine.kvcache import PagedKVCache
+from ollamamq_amd.ops.interface import AttnMeta
+
+pytestmark = pytest.mark.gpu
+D = 128
+
+
+def _hip():
+    from ollamamq_amd.ops import hip
+    hip.require()
+    return hip
+
+
+def _cache(lens, heads, page, seed):
+    cache = PagedKVCache(2, heads, D, page_size=page,
+                         n_pages=sum(-(-n // page) for n in lens) + 2,
+                         max_slots=len(lens) + 1, max_ctx=max(lens) + page,
+                         device="cuda", dtype=torch.bfloat16)
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    for pool in (cache.k_pool, cache.v_pool):
+        pool.normal_(generator=g)
+    slots = [cache.alloc_slot() for _ in lens]
+    cache.alloc_slot()
+    for at in range(0, max(lens), 3 * page):        # pages interleave
+        for slot, n in zip(slots, lens):
+            if at < n:
+                cache.ensure(slot, min(n, at + 3 * page))
+    return cache, slots
+
+
+def _meta(slots, lens, q_lens, window, mode):
+    def i32(v):
+        return torch.tensor(v, dtype=torch.int32, device="cuda")
+    cu = [0]
+    for n in q_lens:
+        cu.append(cu[-1] + n)
+    return AttnMeta(mode=mode, slot_ids=i32(slots), seq_lens=i32(lens),
+                    cu_q=i32(cu), logits_idx=None, max_q=max(q_lens),
+                    max_kv=max(lens), window=window)
+
+
+def _exact(q, cache, layer, slots, lens, q_lens, window):
+    """q [T, Hq, D]; float64."""
+    out, at = [], 0
+    for slot, n, m in zip(slots, lens, q_lens):
+        pages = cache.page_table[slot, :-(-n // cache.page_size)].long()
+        k, v = (pool[layer][pages].transpose(1, 2).flatten(0, 1)[:n].double()
+                for pool in (cache.k_pool, cache.v_pool))
+        group = q.shape[1] // k.shape[1]
+        k, v = (t.repeat_interleave(group, 1).transpose(0, 1).contiguous()
+                for t in (k, v))
+        pos = torch.arange(n - m, n, device="cuda")[:, None]
+        key = torch.arange(n, device="cuda")[None]
+        gone = key > pos
+        if window:
+            gone |= key <= pos - window
+        x = q[at:at + m].double().transpose(0, 1).contiguous()
+        s = (x @ k.transpose(1, 2).contiguous()) / D ** 0.5
+        s = s.masked_fill(gone, float("-inf")).softmax(-1)
+        out.append((s @ v).transpose(0, 1))
+        at += m
+    return torch.cat(out)
+
+
+def _defrag(buf, rows, cols):
+    x = buf.view(-1, cols // 64, 4, 2, 32, 8).permute(0, 4, 1, 2, 3, 5)
+    return x.reshape(-1, cols)[:rows]
+
+
+STEPS = [1, 15, 16, 17, 31, 32, 33, 64, 255, 256, 257, 511, 700]
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(1, 1), (6, 3), (3, 1), (8, 2),
+                                            (5, 1), (6, 1), (14, 2), (16, 2)])
+@pytest.mark.parametrize("page,window", [(16, 0), (64, 0), (16, 33),
+                                         (24, 0), (8, 100)])
+def test_decode(heads, kv_heads, page, window):
+    hip = _hip()
+    cache, slots = _cache(STEPS, kv_heads, page, 7)
+    q = torch.randn(len(STEPS), heads, D, device="cuda").bfloat16()
+    meta = _meta(slots, STEPS, [1] * len(STEPS), window, "decode")
+    want = _exact(q, cache, 1, slots, STEPS, meta.q_lens or [1] * len(STEPS),
+                  window)
+    got = hip.attention_decode(q, cache, 1, meta)
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=1e-5)
+    frag = hip.attention_decode(q, cache, 1, meta, fragout=True)
+    assert torch.equal(_defrag(frag, len(STEPS), heads * D),
+                       got.flatten(1))
+
+
+@pytest.mark.parametrize("split", [1, 2, 3, 32])
+def test_decode_parts(split, monkeypatch):
+    """Any number of parts, some of them without keys, and queries that lie
+    anywhere in their projection."""
+    hip = _hip()
+    lens = [1, 200, 257, 3000, 8100]
+    cache, slots = _cache(lens, 2, 16, 8)
+    monkeypatch.setenv("OLLAMAMQ_DECODE_SPLIT", str(split))
+    whole = torch.randn(len(lens), 11 * D + 3, device="cuda").bfloat16()
+    for first, stride in ((0, 11 * D + 3), (1, 11 * D + 3), (8, 11 * D)):
+        q = whole.flatten()[first:].as_strided((len(lens), 8, D),
+                                               (stride, D, 1))
+        meta = _meta(slots, lens, [1] * len(lens), 0, "decode")
+        got = hip.attention_decode(q, cache, 0, meta)
+        want = _exact(q, cache, 0, slots, lens, [1] * len(lens), 0)
+        torch.testing.assert_close(got.double(), want, rtol=2 ** -8,
+                                   atol=1e-5)
