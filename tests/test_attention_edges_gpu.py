@@ -116,3 +116,44 @@ def test_decode_parts(split, monkeypatch):
         want = _exact(q, cache, 0, slots, lens, [1] * len(lens), 0)
         torch.testing.assert_close(got.double(), want, rtol=2 ** -8,
                                    atol=1e-5)
+
+
+# queries, cached tokens before them
+PORTIONS = [(1, 0), (2, 63), (31, 0), (32, 1), (33, 31), (64, 0), (65, 64),
+            (127, 130), (200, 57), (300, 0)]
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(1, 1), (4, 2), (3, 1), (8, 2),
+                                            (5, 1), (6, 1), (14, 2), (8, 1)])
+@pytest.mark.parametrize("page,window", [(16, 0), (128, 0), (16, 1),
+                                         (16, 40), (24, 0), (8, 129)])
+def test_portions(heads, kv_heads, page, window):
+    """Weights are rounded to bf16 before they meet the values: relative 2^-9
+    of a sum of weighted values of size one, doubled for the result's own."""
+    hip = _hip()
+    q_lens = [m for m, _ in PORTIONS]
+    lens = [m + n for m, n in PORTIONS]
+    cache, slots = _cache(lens, kv_heads, page, 9)
+    q = torch.randn(sum(q_lens), heads, D, device="cuda").bfloat16()
+    meta = _meta(slots, lens, q_lens, window, "prefill")
+    got = hip.attention_prefill(q, cache, 1, meta)
+    want = _exact(q, cache, 1, slots, lens, q_lens, window)
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -8,
+                               atol=2 ** -7)
+    assert ((got - want).norm() / want.norm()).item() < 2 ** -8
+
+
+@pytest.mark.parametrize("singles", [1, 5])
+def test_single_tokens_before_portions(singles):
+    hip = _hip()
+    lens = [90 + 40 * i for i in range(singles)] + [70, 400]
+    q_lens = [1] * singles + [70, 33]
+    cache, slots = _cache(lens, 2, 16, 10)
+    whole = torch.randn(sum(q_lens), 12 * D, device="cuda").bfloat16()
+    q = whole[:, :8 * D].view(-1, 8, D)
+    meta = _meta(slots, lens, q_lens, 0, "mixed")
+    meta.n_decode = singles
+    got = hip.attention_mixed(q, cache, 0, meta)
+    want = _exact(q, cache, 0, slots, lens, q_lens, 0)
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -8,
+                               atol=2 ** -7)
