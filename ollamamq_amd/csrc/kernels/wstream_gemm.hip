@@ -18,15 +18,15 @@
 // The stream is then PERFECTLY linear: each wave reads consecutive 1 KiB
 // vectors (full 128 B line use per instruction), tagged non-temporal
 // (MI355X_MICROARCH "nt-weights": one-time-read stream, -18% landed
-// traffic), with no LDS staging, no barriers, and a register prefetch one
-// 4 KiB iteration deep per wave (8 waves x ~2 blocks/CU ~= 64 KiB in
-// flight/CU -> "streaming" regime, MICROARCH price-table preamble).
+// traffic), with no LDS staging, no barriers, and a register prefetch of
+// one to four 4 KiB iterations per wave.
 //
 // Geometry: grid (N/32, ksplit) x 512 threads (8 waves).  The K/64
 // k-blocks are range-partitioned over ksplit*8 waves (uneven ranges OK:
 // any K%64==0, N%32==0, M<=64).  Wave partials meet in a single
 // end-of-kernel LDS reduce (the ONE barrier, after all streaming).
-// ksplit>1 writes fp32 partials; k_wstream_combine folds them (+bias).
+// ksplit>1 writes fp32 partials; the consumer folds them, or the block that
+// arrives last at a tile (x in fragment layout), or k_wstream_combine (+bias).
 #include "act.h"
 #include "tile_mma.h"
 
@@ -73,9 +73,12 @@ extern "C" int wstream_pure_bf16(void* sink, const void* wp, int N, int K,
 }
 
 // MT: m-tiles of 32 rows (1: M<=32, 2: M<=64).
-// DEPTH: weight prefetch depth in 4 KiB iterations (1 or 2); 2 doubles
-// the b-register ring so a whole iteration's loads stay in flight across
-// one full compute iteration (covers ~2x the HBM latency per wave).
+// DEPTH: weights under way per wave, in 4 KiB iterations.
+// XLDS == 2: x in fragment layout (the decode chain).  A CU's loads are what
+// bounds it, x counted: rows past M repeat row M - 1, so few rows cost few
+// cache lines.  4 iterations ahead for 32 rows, 2 for 64 (registers).  Alone,
+// 28672 x 4096: 47 us before for any M, now 43 for 32 rows, 41 for 8;
+// 4096 x 4096: 12.5, now 8.5 and 7.8 in two parts.
 // XLDS (requires MT==1): stage the x fragments through a wave-PRIVATE
 // LDS tile instead of loading them in MFMA layout.  The direct x
 // fragment load is 32 rows x 16 B at an 8 KB stride = 32 cache-line
@@ -128,7 +131,8 @@ __global__ __launch_bounds__(512) void k_wstream_gemm(
     int M, int N, int K, int64_t xs, int ksplit,
     const float* __restrict__ rstd_parts, int rstd_nt, float inv_h,
     float eps, const bf16* __restrict__ res_in,
-    float* __restrict__ sq_parts, RopeEpi rp = {}, int yfrag = 0)
+    float* __restrict__ sq_parts, RopeEpi rp = {}, int yfrag = 0,
+    int* __restrict__ sem = nullptr) // ksplit > 1: tickets per tile, zero
 {
     const int t = blockIdx.x;              // n-tile (32 cols of y)
     const int ks = blockIdx.y;
@@ -161,20 +165,65 @@ __global__ __launch_bounds__(512) void k_wstream_gemm(
     extern __shared__ __align__(16) char smem[];
 
     f32x16 acc0 = {}, acc1 = {};
-    if (b_lo < b_hi) {
+    if (XLDS == 2 && b_lo < b_hi) {
+        // x in fragment layout: DEPTH iterations of weights and up to two of x
+        // are under way.  The first round may begin before b_lo: those slots
+        // repeat the first block and are not used.
+        const u32x4* wq = wp + (int64_t)t * NB * 256 + lane;
+        const u32x4* xq[MT];
+        #pragma unroll
+        for (int m = 0; m < MT; m++)
+            xq[m] = reinterpret_cast<const u32x4*>(x) + (int64_t)m * K * 4
+                    + (lane & 32) + min(row, max(M - m * 32, 1) - 1);
+        constexpr int XS = DEPTH < 2 ? 1 : 2;
+        u4bf8 w[DEPTH][4], xr[XS][MT][4];
+        auto ldw = [&](int s, int b) {
+            #pragma unroll
+            for (int j = 0; j < 4; j++)
+                w[s][j].u = __builtin_nontemporal_load(
+                    wq + (int64_t)b * 256 + j * 64);
+        };
+        auto ldx = [&](int s, int b) {
+            #pragma unroll
+            for (int m = 0; m < MT; m++)
+                #pragma unroll
+                for (int j = 0; j < 4; j++)
+                    xr[s][m][j].u = xq[m][(int64_t)b * 256 + j * 64];
+        };
+        auto mul = [&](int s) {
+            #pragma unroll
+            for (int j = 0; j < 4; j++) {
+                acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    xr[s % XS][0][j].v, w[s][j].v, acc0, 0, 0, 0);
+                if (MT == 2)
+                    acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        xr[s % XS][MT - 1][j].v, w[s][j].v, acc1, 0, 0, 0);
+            }
+        };
+        int b = b_hi - (b_hi - b_lo + DEPTH - 1) / DEPTH * DEPTH;
+        #pragma unroll
+        for (int s = 0; s < DEPTH; s++) ldw(s, max(b + s, b_lo));
+        #pragma unroll
+        for (int s = 0; s < XS; s++) ldx(s, max(b + s, b_lo));
+        for (; b + DEPTH < b_hi; b += DEPTH) {
+            #pragma unroll
+            for (int s = 0; s < DEPTH; s++) {
+                if (b + s >= b_lo) mul(s);
+                ldw(s, b + s + DEPTH);
+                ldx(s % XS, max(b + s + XS, b_lo));
+            }
+        }
+        #pragma unroll
+        for (int s = 0; s < DEPTH; s++) {
+            if (b + s >= b_lo) mul(s);
+            if (s + XS < DEPTH) ldx(s % XS, max(b + s + XS, b_lo));
+        }
+    }
+    if (XLDS != 2 && b_lo < b_hi) {
         const u32x4* wbase = wp + ((int64_t)t * NB * 4) * 64 + lane;
         u4bf8 br[DEPTH][4];
         bf16x8 a0[2], a1[2], a2[2], a3[2];
-        const u4bf8* xf = reinterpret_cast<const u4bf8*>(x);
         auto lda16 = [&](bf16x8* d, int b, int off) {
-            if (XLDS == 2) {   // frag input: linear like the weights
-                const int64_t u = ((int64_t)b * 4 + (off >> 4)) * 64
-                                  + lane;
-                d[0] = xf[u].v;
-                if (MT == 2)   // second 32-row frag half
-                    d[1] = xf[u + (int64_t)4 * K].v;
-                return;
-            }
             const int64_t k = ((int64_t)b << 6) + off;
             d[0] = *reinterpret_cast<const bf16x8*>(xr0 + k);
             if (MT == 2) d[1] = *reinterpret_cast<const bf16x8*>(xr1 + k);
@@ -445,6 +494,35 @@ __global__ __launch_bounds__(512) void k_wstream_gemm(
     }
     __syncthreads();
     const int n0 = t * 32;
+    // row mr of half mt, column n: the finished sum
+    auto finish = [&](int mt, int mr, int n, float s) {
+        const int m = mr + mt * 32;
+        if (rstd_parts) s *= rstd_sh[m];
+        if (bias) s += __bfloat162float(bias[n0 + n]);
+        const int64_t yo = yfrag ? (int64_t)mt * 32 * N + frag_off(mr, n0 + n)
+                                 : (int64_t)m * N + n0 + n;
+        if (res_in) s += __bfloat162float(res_in[yo]);
+        y[yo] = __float2bfloat16(s);
+        return s * s;
+    };
+    // this block's sums of squares of half mt, from two values per thread
+    auto squares = [&](int mt, const float* rsq) {
+        __syncthreads();
+        float (*sqt)[32] = reinterpret_cast<float (*)[32]>(smem);
+        sqt[tid >> 5][tid & 31] = rsq[0];          // rows 0..15
+        sqt[(tid >> 5) + 16][tid & 31] = rsq[1];   // rows 16..31
+        __syncthreads();
+        if (tid < 32) {
+            float s = 0.f;
+            #pragma unroll
+            for (int n2 = 0; n2 < 32; n2++) s += sqt[tid][n2];
+            // m-major [M][n_tiles]: the consumer's fold walks tiles
+            // CONTIGUOUSLY (a tile-major layout cost 1 float per
+            // 128 B line and ~3 us per consumer block)
+            sq_parts[(int64_t)(tid + mt * 32) * gridDim.x + t] = s;
+        }
+        if (MT == 2 && mt == 0) __syncthreads();   // sqt reused
+    };
     for (int mt = 0; mt < MT; ++mt) {
         const f32x16& acc = mt ? acc1 : acc0;
         if (mt) __syncthreads();
@@ -460,46 +538,63 @@ __global__ __launch_bounds__(512) void k_wstream_gemm(
             const int e = tid + ee * 512;
             const int mr = e >> 5, n = e & 31;
             const int m = mr + mt * 32;
-            if (m < M) {
-                float s = 0.f;
-                #pragma unroll
-                for (int wv = 0; wv < 8; wv++)
-                    s += red8[wv][mr][n];
-                if (ksplit == 1 && y) {
-                    if (rstd_parts) s *= rstd_sh[m];
-                    if (bias) s += __bfloat162float(bias[n0 + n]);
-                    const int64_t yo =
-                        yfrag ? (int64_t)mt * 32 * N + frag_off(mr, n0 + n)
-                              : (int64_t)m * N + n0 + n;
-                    if (res_in) {
-                        s += __bfloat162float(res_in[yo]);
-                        rsq[ee] = s * s;
-                    }
-                    y[yo] = __float2bfloat16(s);
-                } else {
-                    part[((int64_t)ks * M + m) * N + n0 + n] = s;
-                }
-            }
+            if (m >= M) continue;
+            float s = 0.f;
+            #pragma unroll
+            for (int wv = 0; wv < 8; wv++) s += red8[wv][mr][n];
+            if (ksplit == 1 && y) rsq[ee] = finish(mt, mr, n, s);
+            else if (sem)
+                __hip_atomic_store(
+                    part + (((int64_t)ks * gridDim.x + t) * MT + mt) * 1024
+                        + e, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            else part[((int64_t)ks * M + m) * N + n0 + n] = s;
         }
-        // emit this block's sum-of-squares partials for the mt rows
-        if (sq_parts && ksplit == 1) {
-            __syncthreads();
-            float (*sqt)[32] = reinterpret_cast<float (*)[32]>(smem);
-            sqt[tid >> 5][tid & 31] = rsq[0];          // rows 0..15
-            sqt[(tid >> 5) + 16][tid & 31] = rsq[1];   // rows 16..31
-            __syncthreads();
-            if (tid < 32) {
-                float s = 0.f;
-                #pragma unroll
-                for (int n2 = 0; n2 < 32; n2++) s += sqt[tid][n2];
-                // m-major [M][n_tiles]: the consumer's fold walks tiles
-                // CONTIGUOUSLY (a tile-major layout cost 1 float per
-                // 128 B line and ~3 us per consumer block)
-                sq_parts[(int64_t)(tid + mt * 32) * gridDim.x + t] = s;
-            }
-            if (MT == 2 && mt == 0) __syncthreads();  // sqt reused
-        }
+        if (sq_parts && ksplit == 1) squares(mt, rsq);
     }
+    if (!sem) return;
+    // The block that arrives last adds up the parts of its tile, in their
+    // order.  Parts are written through and read past the caches (agent
+    // scope), so the ticket needs no write-back of a whole L2: the stores
+    // have only to be complete before it is drawn.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int* drawn = reinterpret_cast<int*>(smem);
+    if (tid == 0)
+        *drawn = __hip_atomic_fetch_add(sem + t, 1, __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (*drawn != ksplit - 1) return;
+    if (tid == 0)                        // ready for the next launch
+        __hip_atomic_store(sem + t, 0, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    for (int mt = 0; mt < MT; ++mt) {
+        float rsq[2] = {0.f, 0.f};
+        #pragma unroll
+        for (int ee = 0; ee < 2; ee++) {
+            const int e = tid + ee * 512;
+            const int mr = e >> 5;
+            if (mr + mt * 32 >= M) continue;
+            float v[8], s = 0.f;
+            #pragma unroll
+            for (int k = 0; k < 8; k++)
+                v[k] = k < ksplit ? __hip_atomic_load(
+                    part + (((int64_t)k * gridDim.x + t) * MT + mt) * 1024
+                        + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                    : 0.f;
+            #pragma unroll
+            for (int k = 0; k < 8; k++) s += v[k];
+            rsq[ee] = finish(mt, mr, e & 31, s);
+        }
+        if (sq_parts) squares(mt, rsq);
+    }
+}
+
+// Iterations ahead for 32 rows in fragment layout: no more than a wave has,
+// as the slots of a first round that it does not have are loaded all the same
+static int frag_depth(int K, int ksplit)
+{
+    const int n = K / 64 / (8 * ksplit);
+    return n >= 4 ? 4 : n >= 2 ? 2 : 1;
 }
 
 // Fused gate_up @ SwiGLU over GU-interleaved packed weights.
@@ -515,7 +610,7 @@ static int wstream_gu(
     const int lds = (xlds == 1 ? 16 * 4096 : 8 * 32 * 32 * 4) + 256;
     if (M > 32) {
         if (xlds == 2) {       // frag chain at batches 33..64
-            k_wstream_gemm<2, 1, 2, GU><<<grid, 512, lds, stream>>>(
+            k_wstream_gemm<2, 2, 2, GU><<<grid, 512, lds, stream>>>(
                 (bf16*)act, nullptr, (const bf16*)x, (const u32x4*)wp,
                 nullptr, M, N, K, xs, 1, (const float*)rstd_parts,
                 rstd_nt, inv_h, eps, nullptr, nullptr, {}, yfrag);
@@ -530,13 +625,16 @@ static int wstream_gu(
             nullptr, nullptr, {}, 0);
         return (int)hipGetLastError();
     }
-    auto go = xlds == 2 ? k_wstream_gemm<1, 1, 2, GU>
+    const int d = frag_depth(K, 1);
+    auto go = xlds == 2 ? (d == 4   ? k_wstream_gemm<1, 4, 2, GU>
+                           : d == 2 ? k_wstream_gemm<1, 2, 2, GU>
+                                    : k_wstream_gemm<1, 1, 2, GU>)
               : xlds == 1 ? k_wstream_gemm<1, 1, 1, GU>
                           : k_wstream_gemm<1, 1, 0, GU>;
     go<<<grid, 512, lds, stream>>>(
         (bf16*)act, nullptr, (const bf16*)x, (const u32x4*)wp,
         nullptr, M, N, K, xs, 1, (const float*)rstd_parts, rstd_nt,
-        inv_h, eps, nullptr, nullptr, {}, yfrag);
+        inv_h, eps, nullptr, nullptr, {}, yfrag, nullptr);
     return (int)hipGetLastError();
 }
 
@@ -565,73 +663,37 @@ __global__ __launch_bounds__(256) void k_wstream_combine(
     }
 }
 
-// Tile-structured combine for the fused chain (M <= 32): folds the
-// k-split partials, adds the residual stream in place and emits per-tile
-// sum-of-squares partials for the next GEMM's rstd.
-__global__ __launch_bounds__(256) void k_wstream_combine_tiles(
-    bf16* __restrict__ y, const float* __restrict__ part,
-    const bf16* __restrict__ res_in, float* __restrict__ sq_parts,
-    int M, int N, int ksplit, int yfrag)
-{
-    const int t = blockIdx.x;
-    const int tid = threadIdx.x;
-    __shared__ float sqt[32][32];
-    const int n0 = t * 32;
-    const int mts = (M + 31) >> 5;          // 1 or 2 m-halves
-    for (int mt = 0; mt < mts; ++mt) {
-        if (mt) __syncthreads();
-        #pragma unroll
-        for (int ee = 0; ee < 4; ee++) {
-            const int e = tid + ee * 256;
-            const int mr = e >> 5, n = e & 31;
-            const int m = mr + mt * 32;
-            float rsq = 0.f;
-            if (m < M) {
-                float s = 0.f;
-                for (int k = 0; k < ksplit; k++)
-                    s += part[((int64_t)k * M + m) * N + n0 + n];
-                const int64_t yo =
-                    yfrag ? (int64_t)mt * 32 * N + frag_off(mr, n0 + n)
-                          : (int64_t)m * N + n0 + n;
-                if (res_in)
-                    s += __bfloat162float(res_in[yo]);
-                y[yo] = __float2bfloat16(s);
-                rsq = s * s;
-            }
-            sqt[mr][n] = rsq;
-        }
-        if (sq_parts) {
-            __syncthreads();
-            if (tid < 32) {
-                float s = 0.f;
-                #pragma unroll
-                for (int n2 = 0; n2 < 32; n2++) s += sqt[tid][n2];
-                sq_parts[(int64_t)(tid + mt * 32) * gridDim.x + t] = s;
-            }
-        }
-    }
-}
-
-// y == null: the partial sums, fp32, are the result
+// y == null: the partial sums, fp32, are the result.  sem (x in fragment
+// layout): zeros, one per 32 columns; the product adds up its own parts, then
+// part holds ksplit * N * 32 floats for every 32 rows.
 extern "C" int wstream_gemm_bf16(
     void* y, void* part, const void* x, const void* wp, const void* bias,
     int M, int N, int K, int64_t xs, int ksplit, int depth, int xlds,
     const void* rstd_parts, int rstd_nt, float inv_h, float eps,
-    const void* res_in, void* sq_parts, int yfrag, hipStream_t stream)
+    const void* res_in, void* sq_parts, int yfrag, void* sem_,
+    hipStream_t stream)
 {
     dim3 grid(N / 32, ksplit);
+    int* sem = ksplit > 1 && y ? (int*)sem_ : nullptr;
+    if (sem && (xlds != 2 || ksplit > 8)) return -103;
     const int lds_red = 8 * 32 * 32 * 4 + 256;     // reduce + rstd tail
     const int lds_x = 16 * 4096 + 256;             // + 8x2 x tiles
     const float* rp = (const float*)rstd_parts;
-    const bf16* ri = ksplit == 1 ? (const bf16*)res_in : nullptr;
-    float* sq = ksplit == 1 ? (float*)sq_parts : nullptr;
-    if (ksplit > 1 && rstd_parts) return -100;     // fused rstd needs ks==1
+    const bf16* ri = (const bf16*)res_in;
+    float* sq = (float*)sq_parts;
+    // what is fused needs the finished sums
+    if (ksplit > 1 && !sem && (rstd_parts || res_in || sq_parts))
+        return -100;
+    const int d = frag_depth(K, ksplit);
     if (M <= 32) {
         if (xlds == 2)
-            k_wstream_gemm<1, 1, 2><<<grid, 512, lds_red, stream>>>(
+            (d == 4   ? k_wstream_gemm<1, 4, 2>
+             : d == 2 ? k_wstream_gemm<1, 2, 2>
+                      : k_wstream_gemm<1, 1, 2>)
+                <<<grid, 512, lds_red, stream>>>(
                 (bf16*)y, (float*)part, (const bf16*)x, (const u32x4*)wp,
                 (const bf16*)bias, M, N, K, xs, ksplit, rp, rstd_nt,
-                inv_h, eps, ri, sq, {}, yfrag);
+                inv_h, eps, ri, sq, {}, yfrag, sem);
         else if (xlds == 1)
             k_wstream_gemm<1, 1, 1><<<grid, 512, lds_x, stream>>>(
                 (bf16*)y, (float*)part, (const bf16*)x, (const u32x4*)wp,
@@ -649,10 +711,10 @@ extern "C" int wstream_gemm_bf16(
                 inv_h, eps, ri, sq, {}, yfrag);
     } else {
         if (xlds == 2) {
-            k_wstream_gemm<2, 1, 2><<<grid, 512, lds_red, stream>>>(
+            k_wstream_gemm<2, 2, 2><<<grid, 512, lds_red, stream>>>(
                 (bf16*)y, (float*)part, (const bf16*)x, (const u32x4*)wp,
                 (const bf16*)bias, M, N, K, xs, ksplit, rp, rstd_nt,
-                inv_h, eps, ri, sq, {}, yfrag);
+                inv_h, eps, ri, sq, {}, yfrag, sem);
         } else if (rstd_parts || res_in || sq_parts || yfrag) {
             return -101;           // fusion needs the frag path at MT2
         } else if (depth == 2)
@@ -666,19 +728,13 @@ extern "C" int wstream_gemm_bf16(
                 (const bf16*)bias, M, N, K, xs, ksplit, nullptr, 0,
                 0.f, 0.f, nullptr, nullptr);
     }
-    if (ksplit > 1 && y != nullptr) {
-        if (res_in || sq_parts) {
-            k_wstream_combine_tiles<<<N / 32, 256, 0, stream>>>(
-                (bf16*)y, (const float*)part, (const bf16*)res_in,
-                (float*)sq_parts, M, N, ksplit, yfrag);
-        } else {
-            const int64_t mn = (int64_t)M * N;
-            const int64_t want = (mn + 255) / 256;
-            const int blocks = (int)(want < 1024 ? want : 1024);
-            k_wstream_combine<<<blocks, 256, 0, stream>>>(
-                (bf16*)y, (const float*)part, (const bf16*)bias, mn, mn,
-                N, ksplit);
-        }
+    if (ksplit > 1 && y && !sem) {
+        const int64_t mn = (int64_t)M * N;
+        const int64_t want = (mn + 255) / 256;
+        const int blocks = (int)(want < 1024 ? want : 1024);
+        k_wstream_combine<<<blocks, 256, 0, stream>>>(
+            (bf16*)y, (const float*)part, (const bf16*)bias, mn, mn, N,
+            ksplit);
     }
     return (int)hipGetLastError();
 }
@@ -700,16 +756,21 @@ extern "C" int wstream_qkv_rope_bf16(
     RopeEpi rp{(const float*)rcos, (const float*)rsin, (const int*)pos,
                (const int*)slot, (const int*)ptab, (bf16*)kp, (bf16*)vp,
                nl, nkl, psz, maxp};
+    const int d = frag_depth(K, 1);
     if (xf && M > 32)
-        k_wstream_gemm<2, 1, 2, 0, 1><<<grid, 512, lds, stream>>>(
+        k_wstream_gemm<2, 2, 2, 0, 1><<<grid, 512, lds, stream>>>(
             (bf16*)y, nullptr, (const bf16*)x, (const u32x4*)wp,
             (const bf16*)bias, M, N, K, xs, 1, (const float*)rstd_parts,
             rstd_nt, inv_h, eps, nullptr, nullptr, rp);
     else if (xf)
-        k_wstream_gemm<1, 1, 2, 0, 1><<<grid, 512, lds, stream>>>(
+        (d == 4   ? k_wstream_gemm<1, 4, 2, 0, 1>
+         : d == 2 ? k_wstream_gemm<1, 2, 2, 0, 1>
+                  : k_wstream_gemm<1, 1, 2, 0, 1>)
+            <<<grid, 512, lds, stream>>>(
             (bf16*)y, nullptr, (const bf16*)x, (const u32x4*)wp,
             (const bf16*)bias, M, N, K, xs, 1, (const float*)rstd_parts,
-            rstd_nt, inv_h, eps, nullptr, nullptr, rp);
+            rstd_nt, inv_h, eps, nullptr, nullptr, rp, 0,
+            nullptr);
     else
         k_wstream_gemm<1, 1, 0, 0, 1><<<grid, 512, lds, stream>>>(
             (bf16*)y, nullptr, (const bf16*)x, (const u32x4*)wp,

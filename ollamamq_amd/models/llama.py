@@ -352,6 +352,9 @@ class LlamaModel:
             self._sq_a = torch.zeros(max(th, 1) * 64, dtype=torch.float32,
                                      device=self.device)
             self._sq_b = torch.zeros_like(self._sq_a)
+            # tickets of the split products, zero between them
+            self._tickets = torch.zeros(max(th, 1), dtype=torch.int32,
+                                        device=self.device)
             # frag-layout residual stream: two 32-row halves (the MT2
             # chain serves batches up to 64; rows >= batch hold garbage
             # that only dead accumulator rows ever see)
@@ -482,14 +485,16 @@ class LlamaModel:
             q = qkv[:, :nl * d].view(-1, nl, d)
             attn = ops.attention_decode_frag(q, kv_cache, li, attn_meta)
             ops.linear_fused(attn, layer.wo_pk, H, res=res, sq_out=sq_b,
-                             y=res, yfrag=1, K=nl * d, xlds=2, M_frag=B)
+                             y=res, yfrag=1, K=nl * d, xlds=2, M_frag=B,
+                             sem=self._tickets)
             act = ops.gu_fused(res, layer.wgu_pk,
                                layer.wgate_up.shape[0], rstd=sq_b,
                                rstd_nt=tiles_h, inv_h=inv_h, eps=eps,
                                K=H, yfrag=1, M_frag=B)
             ops.linear_fused(act, layer.wdown_pk, H, res=res,
                              sq_out=sq_a, y=res, yfrag=1,
-                             K=layer.wdown.shape[1], xlds=2, M_frag=B)
+                             K=layer.wdown.shape[1], xlds=2, M_frag=B,
+                             sem=self._tickets)
             nt = tiles_h
         logits = ops.linear_fused(res, self.lm_head_pk,
                                   self.lm_head.shape[0], rstd=sq_a,

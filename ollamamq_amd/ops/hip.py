@@ -57,7 +57,7 @@ def _try_load():
                                       i, f, i64, i, vp]
     lib.embed_gather_bf16.argtypes = [vp, vp, vp, i, i, vp]
     lib.wstream_gemm_bf16.argtypes = [vp, vp, vp, vp, vp, i, i, i, i64, i,
-                                      i, i, vp, i, f, f, vp, vp, i, vp]
+                                      i, i, vp, i, f, f, vp, vp, i, vp, vp]
     lib.wstream_pure_bf16.argtypes = [vp, vp, i, i, i, vp]
     lib.wstream_gu_bf16.argtypes = [vp, vp, vp, i, i, i, i64, i,
                                     vp, i, f, f, i, i, vp]
@@ -622,17 +622,31 @@ _WS_KS = os.environ.get("OLLAMAMQ_WS_KS")   # sweep override
 _WS_MAX_N = int(os.environ.get("OLLAMAMQ_WS_MAX_N", "16384"))
 
 
+def _frag_ksplit(N, K):
+    """Parts of a product over an activation in fragment layout, which adds
+    up its own parts: two halves of 128 tiles keep all CUs loading (4096 x
+    4096, 32 rows: 8.5 us against 11.5 whole; 4096 x 14336: 22 against 38),
+    more than 200 tiles do so by themselves.  A wave keeps at least two
+    iterations of 64 columns."""
+    ks = 1
+    while ks < 8 and N // 32 * ks < 200 and K // 64 // (ks * 16) >= 2:
+        ks *= 2
+    return ks
+
+
 def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
                   rstd=None, rstd_nt=0, inv_h=0.0, eps=0.0,
                   res=None, sq_out=None, y=None, yfrag=0, K=None,
-                  M_frag=32):
+                  M_frag=32, sem=None):
     """y = x @ W^T via the weight-streaming kernel over pre-packed W.
 
-    Fused-chain extras (decode, M<=32): `rstd`/`rstd_nt`/`inv_h`/`eps`
+    Fused-chain extras (decode, M<=64): `rstd`/`rstd_nt`/`inv_h`/`eps`
     apply rmsnorm scaling of the raw-residual input x (norm weight must
     be folded into the pack); `res` adds the residual stream into the
     output (pass y=res for the in-place residual update) and `sq_out`
-    emits per-tile sum-of-squares partials for the next GEMM."""
+    emits per-tile sum-of-squares partials for the next GEMM.  `sem`: int32
+    zeros, one per 32 columns, for a split product over a fragment-layout x;
+    they are zero again when it ends, so a stream's products can share them."""
     if K is None:
         M, K = x.shape
         xs = x.stride(0)
@@ -646,29 +660,30 @@ def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
         per_k = os.environ.get(f"OLLAMAMQ_WS_KS_{K}")   # per-shape tuning
         if per_k:
             ks = int(per_k)
+        elif _WS_KS:
+            ks = int(_WS_KS)
         else:
-            ks = int(_WS_KS) if _WS_KS else _wstream_ksplit(N, K)
+            ks = _frag_ksplit(N, K) if xlds == 2 else _wstream_ksplit(N, K)
     if rstd is not None:
-        ks = 1            # rstd fusion requires ks == 1
-    part = ctypes.c_void_p(0)
+        ks = 1            # every part would have to scale its rows
+    part = None
     if ks > 1:
-        key = ("ws", M, N, ks, str(x.device))
-        t = _gemm_scratch.get(key)
-        if t is None:
-            t = torch.empty(ks * M * N, dtype=torch.float32,
-                            device=x.device)
-            _gemm_scratch[key] = t
-        part = _p(t)
+        rows = -(-M // 32) * 32 if xlds == 2 else M
+        part = torch.empty(ks * rows * N, dtype=torch.float32,
+                           device=x.device)
+        if xlds == 2 and sem is None:
+            sem = torch.zeros(N // 32, dtype=torch.int32, device=x.device)
+        assert sem is None or sem.numel() >= N // 32
     if xlds is None:
         # measured (profiles/r02_gemm_sweep.md): LDS x-staging pays on
         # long streams (down/gate_up/logits), the direct fragment load
         # wins on the short ramp-bound ones (qkv/o)
         xlds = (_WS_XLDS if M <= 32 and N * K * 2 > (64 << 20) else 0)
     _check(_lib.wstream_gemm_bf16(
-        _p(y), part, _p(x), _p(packed), _p(bias), M, N, K, xs,
+        _p(y), _p(part), _p(x), _p(packed), _p(bias), M, N, K, xs,
         ks, depth if depth is not None else _WS_DEPTH, xlds,
         _p(rstd), rstd_nt, float(inv_h), float(eps), _p(res), _p(sq_out),
-        yfrag, _stream()), "wstream_gemm")
+        yfrag, _p(sem), _stream()), "wstream_gemm")
     return y
 
 
@@ -809,7 +824,7 @@ def _linear_frag(x, N, packed, parts, most=8):
     _check(_lib.wstream_gemm_bf16(
         _p(y), _p(part), _p(x.buf), _p(packed), _p(None), M, N, K, 0, ks,
         _WS_DEPTH, 2, _p(None), 0, 0.0, 0.0, _p(None), _p(None), 0,
-        _stream()), "wstream_gemm")
+        _p(None), _stream()), "wstream_gemm")
     return y if y is not None else Partials(part)
 
 
@@ -824,7 +839,7 @@ def linear_f32(x, weight, packed=None):
         _check(_lib.wstream_gemm_bf16(
             _p(None), _p(part), _p(x.buf), _p(packed), _p(None), M, N, K, 0,
             part.shape[0], _WS_DEPTH, 2, _p(None), 0, 0.0, 0.0, _p(None),
-            _p(None), 0, _stream()), "wstream_gemm")
+            _p(None), 0, _p(None), _stream()), "wstream_gemm")
         return Partials(part)
     if x.dtype == torch.float32:
         return torch.nn.functional.linear(x, weight)
@@ -855,7 +870,7 @@ def linear_parts(x, weight, packed=None, most=8):
             _check(_lib.wstream_gemm_bf16(
                 _p(None), _p(part), _p(x), _p(packed), _p(None), M, N, K,
                 x.stride(0), ks, _WS_DEPTH, xlds, _p(None), 0, 0.0, 0.0,
-                _p(None), _p(None), 0, _stream()), "wstream_gemm")
+                _p(None), _p(None), 0, _p(None), _stream()), "wstream_gemm")
             return Partials(part)
     return linear(x, weight, packed=packed)
 

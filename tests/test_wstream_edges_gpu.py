@@ -1,0 +1,105 @@
+"""Weight-streaming products over activations in fragment layout at the edges
+of their tiles, against float64.
+
+Tolerance: fp32 sums of K products of about 1/sqrt(K), then one rounding to
+bf16 (relative 2^-9; doubled, as the sum's own error can cross a tie).
+"""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+CLOSE = dict(rtol=2 ** -8, atol=1e-4)
+
+
+def _hip():
+    from ollamamq_amd.ops import hip
+    hip.require()
+    return hip
+
+
+def _frag(x):
+    """x in fragment layout; rows that do not exist are NaN."""
+    rows = -(-x.shape[0] // 32) * 32
+    full = torch.full((rows, x.shape[1]), float("nan"), dtype=x.dtype,
+                      device=x.device)
+    full[:x.shape[0]] = x
+    return full.view(rows // 32, 32, -1, 4, 2, 8).permute(0, 2, 3, 4, 1, 5) \
+        .contiguous().flatten()
+
+
+def _defrag(buf, rows, cols):
+    x = buf.view(-1, cols // 64, 4, 2, 32, 8).permute(0, 4, 1, 2, 3, 5)
+    return x.reshape(-1, cols)[:rows]
+
+
+def _case(M, N, K, seed=3):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).bfloat16()
+    return x, w, x.double() @ w.double().T
+
+
+@pytest.mark.parametrize("M", [1, 2, 15, 16, 17, 31, 32, 33, 48, 63, 64])
+@pytest.mark.parametrize("N,K", [(32, 64), (64, 448), (96, 576), (64, 1088),
+                                 (128, 4096), (64, 4160)])
+def test_whole(M, N, K):
+    hip = _hip()
+    x, w, want = _case(M, N, K)
+    pk = hip.pack_weight(w)
+    got = hip.linear_packed(_frag(x), pk, None, N, ks=1, K=K, xlds=2,
+                            M_frag=M)
+    torch.testing.assert_close(got.double(), want, **CLOSE)
+    rows = -(-M // 32) * 32
+    norms = torch.rand(rows, 3, device="cuda") + 0.1     # three partials
+    bias = torch.randn(N, device="cuda").bfloat16()
+    got = hip.linear_packed(_frag(x), pk, bias, N, K=K, xlds=2, M_frag=M,
+                            rstd=norms, rstd_nt=3, inv_h=1 / K, eps=1e-5)
+    scale = (norms.double().sum(1) / K + 1e-5).rsqrt()[:M, None]
+    # the scale is the hardware's reciprocal root: relative 1e-6 more
+    torch.testing.assert_close(got.double(), want * scale + bias.double(),
+                               rtol=2 ** -8, atol=2e-3)
+
+
+@pytest.mark.parametrize("M", [1, 17, 32, 33, 64])
+@pytest.mark.parametrize("ks", [2, 3, 4, 8])
+@pytest.mark.parametrize("N,K", [(64, 512), (192, 1088), (128, 4160)])
+def test_parts_add_themselves_up(M, ks, N, K):
+    """The residual sum in place, sums of squares, and tickets that are zero
+    again, over several products that share them."""
+    hip = _hip()
+    x, w, want = _case(M, N, K)
+    pk, xf = hip.pack_weight(w), _frag(x)
+    sem = torch.zeros(N // 32, dtype=torch.int32, device="cuda")
+    base = torch.randn(M, N, device="cuda").bfloat16()
+    rows = -(-M // 32) * 32
+    first = None
+    for _ in range(4):
+        res = _frag(base)
+        sq = torch.zeros(rows, N // 32, device="cuda")
+        y = hip.linear_packed(xf, pk, None, N, ks=ks, res=res, y=res,
+                              sq_out=sq, yfrag=1, K=K, xlds=2, M_frag=M,
+                              sem=sem)
+        total = want + base.double()
+        got = _defrag(y, M, N).double()
+        torch.testing.assert_close(got, total, **CLOSE)
+        torch.testing.assert_close(
+            sq[:M].double(), total.square().unflatten(1, (-1, 32)).sum(2),
+            rtol=1e-4, atol=1e-3)
+        assert not sem.any()
+        # whoever comes last adds up in the same order
+        assert first is None or torch.equal(first, got)
+        first = got
+    plain = hip.linear_packed(xf, pk, None, N, ks=ks, K=K, xlds=2, M_frag=M)
+    torch.testing.assert_close(plain.double(), want, **CLOSE)
+
+
+@pytest.mark.parametrize("M", [1, 16, 32, 33, 64])
+@pytest.mark.parametrize("F,K", [(16, 64), (48, 576), (160, 4160)])
+def test_gate_up(M, F, K):
+    hip = _hip()
+    x, w, want = _case(M, 2 * F, K)
+    gate, up = want.chunk(2, 1)
+    want = torch.nn.functional.silu(gate) * up
+    got = hip.linear_gu(_frag(x), hip.pack_weight_gu(w), 2 * F, K=K,
+                        M_frag=M)
+    torch.testing.assert_close(got.double(), want, **CLOSE)
