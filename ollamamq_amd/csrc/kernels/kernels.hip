@@ -622,9 +622,22 @@ __global__ __launch_bounds__(256) void k_argmax_part(
     }
 }
 
-__global__ __launch_bounds__(256) void k_argmax_comb(
+// What a decode step does with the tokens it picked: they are the next step's
+// input, one position on.  Padding rows have adv = 0.
+struct Advance {
+    int* tok;
+    int64_t* out;
+    int* pos;
+    int* lens;
+    const int* adv;
+};
+
+// The best of a row's SP <= 64 slices, one wave a row: the token goes to `out`
+// or, with `step`, to the next step's inputs (five launches of torch and 22 us
+// a step as separate operations).
+__global__ __launch_bounds__(256) void k_pick(
     int* __restrict__ out, const float* __restrict__ pb,
-    const int* __restrict__ pi, int B, int SP)
+    const int* __restrict__ pi, int B, int SP, Advance step)
 {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
@@ -637,37 +650,56 @@ __global__ __launch_bounds__(256) void k_argmax_comb(
         const int oi = __shfl_down(bidx, off, 64);
         if (ob > best || (ob == best && oi < bidx)) { best = ob; bidx = oi; }
     }
-    if (lane == 0) out[row] = bidx;
+    if (lane) return;
+    if (out) out[row] = bidx;
+    if (!step.tok) return;
+    const int n = step.adv[row];
+    step.tok[row] = bidx;
+    step.out[row] = bidx;
+    step.pos[row] += n;
+    step.lens[row] += n;
 }
 
 template <typename T>
 static int argmax_go(void* out, const void* logits, int B, int V,
-                     void* pb, void* pi, int SP, hipStream_t stream)
+                     void* pb, void* pi, int SP, Advance step,
+                     hipStream_t stream)
 {
-    if (SP > 1 && pb != nullptr) {
-        int seg = (V / SP + 2047) & ~2047;          // 256-thread x8 rounds
+    if (step.tok && !pb) return (int)hipErrorInvalidValue;
+    if (pb != nullptr) {
+        // 256-thread x8 rounds; a small vocabulary is one slice
+        int seg = V < SP ? 2048 : (V / SP + 2047) & ~2047;
         while ((int64_t)(SP - 1) * seg >= V) SP--;  // drop empty slices
         dim3 grid(B, SP);
         k_argmax_part<T><<<grid, 256, 0, stream>>>(
             (float*)pb, (int*)pi, (const T*)logits, V, seg);
-        k_argmax_comb<<<(B + 3) / 4, 256, 0, stream>>>(
-            (int*)out, (const float*)pb, (const int*)pi, B, SP);
+        k_pick<<<(B + 3) / 4, 256, 0, stream>>>(
+            (int*)out, (const float*)pb, (const int*)pi, B, SP, step);
     } else {
         k_argmax<T><<<B, 256, 0, stream>>>((int*)out, (const T*)logits, V);
     }
     return (int)hipGetLastError();
 }
 
+// tok: null, or the next step's inputs (see Advance)
 extern "C" int argmax_bf16(void* out, const void* logits, int B, int V,
-                            void* pb, void* pi, int SP, hipStream_t stream)
+                            void* pb, void* pi, int SP, void* tok,
+                            void* out64, void* pos, void* lens,
+                            const void* adv, hipStream_t stream)
 {
-    return argmax_go<bf16>(out, logits, B, V, pb, pi, SP, stream);
+    return argmax_go<bf16>(out, logits, B, V, pb, pi, SP,
+                           {(int*)tok, (int64_t*)out64, (int*)pos,
+                            (int*)lens, (const int*)adv}, stream);
 }
 
 extern "C" int argmax_f32(void* out, const void* logits, int B, int V,
-                          void* pb, void* pi, int SP, hipStream_t stream)
+                          void* pb, void* pi, int SP, void* tok,
+                          void* out64, void* pos, void* lens,
+                          const void* adv, hipStream_t stream)
 {
-    return argmax_go<float>(out, logits, B, V, pb, pi, SP, stream);
+    return argmax_go<float>(out, logits, B, V, pb, pi, SP,
+                            {(int*)tok, (int64_t*)out64, (int*)pos,
+                             (int*)lens, (const int*)adv}, stream);
 }
 
 // ---------------------------------------------------------------------
@@ -900,41 +932,24 @@ __global__ __launch_bounds__(256) void k_gumbel_part(
     }
 }
 
-__global__ __launch_bounds__(64) void k_gumbel_comb(
-    int* __restrict__ out, const float* __restrict__ pb,
-    const int* __restrict__ pi, int sp)
-{
-    const int row = blockIdx.x;
-    float best = -3.0e38f;
-    int bidx = 0;
-    for (int s = threadIdx.x; s < sp; s += 64) {
-        const float v = pb[row * sp + s];
-        const int ix = pi[row * sp + s];
-        if (v > best || (v == best && ix < bidx)) { best = v; bidx = ix; }
-    }
-    #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const float ob = __shfl_down(best, off, 64);
-        const int oi = __shfl_down(bidx, off, 64);
-        if (ob > best || (ob == best && oi < bidx)) { best = ob; bidx = oi; }
-    }
-    if (threadIdx.x == 0) out[row] = bidx;
-}
-
 extern "C" int sample_gumbel_bf16(
     void* out, const void* logits, const void* temps, const void* seeds,
     const void* ctrs, const void* noise, int B, int V,
-    void* pb, void* pi, int sp, hipStream_t stream)
+    void* pb, void* pi, int sp, void* tok, void* out64, void* pos,
+    void* lens, const void* adv, hipStream_t stream)
 {
-    if (sp > 1) {
+    if ((tok && !pb) || sp > 64) return (int)hipErrorInvalidValue;
+    if (pb) {
         const int seg = (V + sp - 1) / sp;
         dim3 grid(B, sp);
         k_gumbel_part<true><<<grid, 256, 0, stream>>>(
             nullptr, (float*)pb, (int*)pi, (const bf16*)logits,
             (const float*)temps, (const unsigned long long*)seeds,
             (const int*)ctrs, (const float*)noise, V, seg);
-        k_gumbel_comb<<<B, 64, 0, stream>>>(
-            (int*)out, (const float*)pb, (const int*)pi, sp);
+        k_pick<<<(B + 3) / 4, 256, 0, stream>>>(
+            (int*)out, (const float*)pb, (const int*)pi, B, sp,
+            {(int*)tok, (int64_t*)out64, (int*)pos, (int*)lens,
+             (const int*)adv});
     } else {
         k_gumbel_part<false><<<B, 256, 0, stream>>>(
             (int*)out, nullptr, nullptr, (const bf16*)logits,
@@ -948,14 +963,15 @@ extern "C" int sample_gumbel_bf16(
 // Fragify + row sum-of-squares: convert a standard [M, H] activation into
 // the 32-row MFMA fragment layout the fused decode chain streams
 // (wstream_gemm.hip frag_off) AND emit sq[m] = sum(x[m]^2) — one read of
-// the embedding output seeds the whole chain.
+// the embedding output seeds the whole chain.  With tokens, x is the
+// embedding table and its rows are gathered on the way.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_fragify_sumsq(
-    const bf16* __restrict__ x, bf16* __restrict__ xf,
-    float* __restrict__ sq, int H)
+    const bf16* __restrict__ x, const int* __restrict__ tokens,
+    bf16* __restrict__ xf, float* __restrict__ sq, int H)
 {
     const int m = blockIdx.x;
-    const bf16* row = x + (int64_t)m * H;
+    const bf16* row = x + (int64_t)(tokens ? tokens[m] : m) * H;
     // rows 32-63 land in the second 32-row frag half (MT2 chain)
     bf16* xfh = xf + (int64_t)(m >> 5) * 32 * H;
     const int mr = m & 31;
@@ -981,9 +997,10 @@ __global__ __launch_bounds__(256) void k_fragify_sumsq(
 }
 
 extern "C" int fragify_sumsq_bf16(void* xf, void* sq, const void* x,
-                                  int M, int H, hipStream_t stream)
+                                  const void* tokens, int M, int H,
+                                  hipStream_t stream)
 {
     k_fragify_sumsq<<<M, 256, 0, stream>>>(
-        (const bf16*)x, (bf16*)xf, (float*)sq, H);
+        (const bf16*)x, (const int*)tokens, (bf16*)xf, (float*)sq, H);
     return (int)hipGetLastError();
 }

@@ -246,23 +246,25 @@ class LlamaEngine:
         seqs = [parts[i][0] for i in order]
         q_lens = [len(parts[i][1]) for i in order]
         tokens = [t for i in order for t in parts[i][1]]
-        pos, first, at = [], {}, 0
-        for i, s, n in zip(order, seqs, q_lens):
-            done = self.kv.seq_lens[s.slot]
-            pos.extend(range(done, done + n))
+        starts = [self.kv.seq_lens[s.slot] for s in seqs]
+        first, at = {}, 0
+        for i, n in zip(order, q_lens):
             first[i] = at
             at += n
         rows = [first[i] + w for i, p in enumerate(parts) for w in p[2]]
         nd = sum(n == 1 for n in q_lens)
         if nd == len(parts):
             if self.use_graphs and nd <= self.max_batch:
-                for s in seqs:
-                    self.kv.ensure(s.slot, self.kv.seq_lens[s.slot] + 1)
-                logits = self._decode_forward_graphed(seqs, tokens, pos)
+                self._one_more(seqs)
+                logits = self._decode_forward_graphed(seqs, tokens, starts)
             else:
-                logits = self._forward(seqs, tokens, pos, q_lens, "decode")
+                logits = self._forward(seqs, tokens, starts, q_lens,
+                                       "decode")
+            if rows and rows == list(range(rows[0], rows[0] + len(rows))):
+                # a copy: the next step writes over the captured logits
+                return logits[rows[0]:rows[0] + len(rows)].clone()
             return logits[rows]
-        logits = self._forward(seqs, tokens, pos, q_lens,
+        logits = self._forward(seqs, tokens, starts, q_lens,
                                "mixed" if nd else "prefill", n_decode=nd,
                                rows=rows or [at - 1])
         return logits[:len(rows)]
@@ -315,15 +317,15 @@ class LlamaEngine:
         dec = [s for s in self.running
                if s.total_len < self.kv.max_ctx]
         token_list = [s.generated[-1] for s in dec]
-        pos_list = [s.total_len - 1 for s in dec]
+        starts = [s.total_len - 1 for s in dec]
         q_lens = [1] * len(dec)
         for s in batch:
             take = s._chunk
             start = s.prefill_done
             token_list.extend(s.prompt[start:start + take])
-            pos_list.extend(range(start, start + take))
+            starts.append(start)
             q_lens.append(take)
-        logits = self._forward(dec + batch, token_list, pos_list, q_lens,
+        logits = self._forward(dec + batch, token_list, starts, q_lens,
                                "mixed", n_decode=len(dec))
         # sample decode rows + finishing-prefill rows
         fin_rows = [len(dec) + i for i, s in enumerate(batch)
@@ -355,48 +357,52 @@ class LlamaEngine:
                 if s.on_token:
                     s.on_token(int(tok), False)
 
-    def _build_meta(self, seqs, q_lens, mode, n_decode=0,
-                    rows=None) -> AttnMeta:
-        dev = self.dev
-        slot_ids = torch.tensor([s.slot for s in seqs], dtype=torch.int32,
-                                device=dev)
-        seq_lens = torch.tensor([self.kv.seq_lens[s.slot] for s in seqs],
-                                dtype=torch.int32, device=dev)
-        cu = [0]
-        for ql in q_lens:
-            cu.append(cu[-1] + ql)
-        cu_q = torch.tensor(cu, dtype=torch.int32, device=dev)
-        # default: every sequence's last token
-        logits_idx = torch.tensor(
-            [c - 1 for c in cu[1:]] if rows is None else rows,
-            dtype=torch.long, device=dev)
-        return AttnMeta(
-            mode=mode, slot_ids=slot_ids, seq_lens=seq_lens, cu_q=cu_q,
-            logits_idx=logits_idx, max_q=max(q_lens),
-            max_kv=int(max(self.kv.seq_lens[s.slot] for s in seqs)),
-            n_decode=n_decode,
-            window=getattr(self.model.cfg, "sliding_window", 0),
-            q_lens=list(q_lens),
-            kv_lens=[self.kv.seq_lens[s.slot] for s in seqs],
-            slots=[s.slot for s in seqs],
-        )
+    def _one_more(self, seqs):
+        """Room for another token of every sequence."""
+        self.kv.ensure_all([(s.slot, self.kv.seq_lens[s.slot] + 1)
+                            for s in seqs])
 
-    def _forward(self, seqs, token_list, pos_list, q_lens, mode,
+    def _forward(self, seqs, token_list, starts, q_lens, mode,
                  n_decode=0, rows=None):
-        dev = self.dev
-        tokens = torch.tensor(token_list, dtype=torch.int32, device=dev)
-        positions = torch.tensor(pos_list, dtype=torch.int32, device=dev)
-        slot_per_tok = torch.tensor(
-            [s.slot for s, ql in zip(seqs, q_lens) for _ in range(ql)],
-            dtype=torch.int32, device=dev)
-        for s, ql in zip(seqs, q_lens):
-            self.kv.ensure(s.slot, self.kv.seq_lens[s.slot] + ql)
-        meta = self._build_meta(seqs, q_lens, mode, n_decode, rows)
-        logits = self.model.forward(tokens, positions, self.kv, slot_per_tok,
-                                    meta)
-        return logits
+        """One forward of token_list, q_lens tokens per sequence from position
+        starts on; logits of every sequence's last token, or of `rows`.  The
+        batch goes to the device in one piece."""
+        slots = [s.slot for s in seqs]
+        self.kv.ensure_all([(slot, self.kv.seq_lens[slot] + ql)
+                            for slot, ql in zip(slots, q_lens)])
+        kv_lens = [self.kv.seq_lens[slot] for slot in slots]
+        cu = [0, *itertools.accumulate(q_lens)]
+        want = [c - 1 for c in cu[1:]] if rows is None else rows
+        n, T = len(seqs), len(token_list)
+        host = torch.empty(2 * len(want) + 3 * T + 3 * n + 1,
+                           dtype=torch.int32,
+                           pin_memory=self.dev.type == "cuda")
+        sizes = [2 * len(want), T, T, T, n, n, n + 1]
+        i32 = torch.int32
+        for part, value in zip(host.split(sizes), (
+                torch.tensor(want, dtype=torch.long).view(i32),
+                torch.tensor(token_list, dtype=i32),
+                torch.cat([torch.arange(p, p + ql, dtype=i32)
+                           for p, ql in zip(starts, q_lens)]),
+                torch.repeat_interleave(torch.tensor(slots, dtype=i32),
+                                        torch.tensor(q_lens)),
+                *(torch.tensor(v, dtype=i32)
+                  for v in (slots, kv_lens, cu)))):
+            part.copy_(value)
+        idx, tokens, positions, slot_per_tok, slot_ids, seq_lens, cu_q = \
+            host.to(self.dev, non_blocking=True).split(sizes)
+        meta = AttnMeta(
+            mode=mode, slot_ids=slot_ids, seq_lens=seq_lens, cu_q=cu_q,
+            logits_idx=idx.view(torch.long), max_q=max(q_lens),
+            max_kv=max(kv_lens), n_decode=n_decode,
+            window=getattr(self.model.cfg, "sliding_window", 0),
+            q_lens=list(q_lens), kv_lens=kv_lens, slots=slots)
+        return self.model.forward(tokens, positions, self.kv, slot_per_tok,
+                                  meta)
 
     def _sample(self, seqs, logits):
+        if all(s.params.temperature <= 0 for s in seqs):
+            return ops.sample(logits, 0.0, 0, 1.0, self._gen).tolist()
         dev = logits.device
         temps = torch.tensor([s.params.temperature for s in seqs],
                              dtype=torch.float32, device=dev)
@@ -428,14 +434,14 @@ class LlamaEngine:
 
     def _prefill_step(self, batch: List[Sequence]):
         self._drain_pipe()
-        token_list, pos_list, q_lens = [], [], []
+        token_list, starts, q_lens = [], [], []
         for s in batch:
             take = s._chunk
             start = s.prefill_done
             token_list.extend(s.prompt[start:start + take])
-            pos_list.extend(range(start, start + take))
+            starts.append(start)
             q_lens.append(take)
-        logits = self._forward(batch, token_list, pos_list, q_lens, "prefill")
+        logits = self._forward(batch, token_list, starts, q_lens, "prefill")
         # Only sequences whose whole prompt is now in KV emit a token.
         rows = [i for i, s in enumerate(batch)
                 if s.prefill_done + s._chunk == len(s.prompt)]
@@ -501,16 +507,18 @@ class LlamaEngine:
         if entry is not None:
             return entry
         dev = self.dev
+        # filled in one copy
+        inputs = torch.zeros(5, B, dtype=torch.int32, device=dev)
         bufs = {
-            "tok": torch.zeros(B, dtype=torch.int32, device=dev),
-            "pos": torch.zeros(B, dtype=torch.int32, device=dev),
-            "slot": torch.zeros(B, dtype=torch.int32, device=dev),
-            "lens": torch.zeros(B, dtype=torch.int32, device=dev),
-            "temps": torch.zeros(B, dtype=torch.float32, device=dev),
-            "seeds": torch.zeros(B, dtype=torch.int64, device=dev),
+            "inputs": inputs,
+            "tok": inputs[0], "pos": inputs[1], "slot": inputs[2],
+            "lens": inputs[3],
             # 1 for live rows, 0 for bucket padding: the in-graph
             # advance applies it so pad rows never grow their dummy slot
-            "adv": torch.ones(B, dtype=torch.int32, device=dev),
+            "adv": inputs[4].fill_(1),
+            "temps": torch.zeros(B, dtype=torch.float32, device=dev),
+            "seeds": torch.zeros(B, dtype=torch.int64, device=dev),
+            "out": torch.zeros(B, dtype=torch.int64, device=dev),
         }
         meta = AttnMeta(
             mode="decode", slot_ids=bufs["slot"], seq_lens=bufs["lens"],
@@ -519,7 +527,7 @@ class LlamaEngine:
             max_q=1, max_kv=self.kv.max_ctx,
             window=getattr(self.model.cfg, "sliding_window", 0))
         entry = {"bufs": bufs, "meta": meta, "graph": None, "logits": None,
-                 "out": None, "ring_i": 0, "klass": klass,
+                 "out": bufs["out"], "ring_i": 0, "klass": klass,
                  "pinned": [torch.empty(B, dtype=torch.int64,
                                         pin_memory=True) for _ in range(2)],
                  "events": [torch.cuda.Event() for _ in range(2)]}
@@ -537,12 +545,7 @@ class LlamaEngine:
              [s.slot for s in seqs] + [dummy] * pad,
              [self.kv.seq_lens[s.slot] for s in seqs] + [1] * pad,
              [1] * len(seqs) + [0] * pad], dtype=torch.int32)
-        staged = host.to(self.dev, non_blocking=True)
-        bufs["tok"].copy_(staged[0])
-        bufs["pos"].copy_(staged[1])
-        bufs["slot"].copy_(staged[2])
-        bufs["lens"].copy_(staged[3])
-        bufs["adv"].copy_(staged[4])
+        bufs["inputs"].copy_(host.pin_memory(), non_blocking=True)
         if entry["klass"] >= 1:
             bufs["temps"].copy_(torch.tensor(
                 [s.params.temperature for s in seqs] + [0.0] * pad,
@@ -552,25 +555,27 @@ class LlamaEngine:
                 + [0] * pad,
                 dtype=torch.int64).to(self.dev, non_blocking=True))
 
-    def _graph_tail(self, entry, logits):
-        """The in-graph sampling tail: class 0 = greedy argmax; class 1 =
-        exact Gumbel-max temperature sampling (kernels.hip sample_gumbel,
-        greedy rows ride the same kernel with T<=0), noise keyed by
-        (per-seq seed, kv length) so replays draw fresh randomness with
-        no host RNG.
-
-        This MUST also run once EAGERLY in the pre-capture warmup: the
-        samplers cache split-scratch buffers (ops/hip.py _scratch), and a
-        first allocation INSIDE capture would live in one graph's private
-        memory pool while every other graph and the eager path reuse the
-        cached tensor — undefined, and it produced real memory faults
-        under mixed sampled serving (r02 stress)."""
-        bufs = entry["bufs"]
-        if entry["klass"] == 1:
-            from ..ops import hip as _hip
-            return _hip.sample_gumbel(logits, bufs["temps"],
-                                      bufs["seeds"], bufs["lens"])
-        return ops.sample(logits, 0.0, 0, 1.0, None).int()
+    def _graph_tail(self, klass, logits, bufs):
+        """The in-graph end of a step: the picked tokens become the next
+        step's inputs, so a steady decode batch replays back-to-back with no
+        host round-trip.  Class 0 = greedy argmax; class 1 = exact Gumbel-max
+        temperature sampling (kernels.hip sample_gumbel, greedy rows ride the
+        same kernel with T<=0), noise keyed by (per-seq seed, kv length) so
+        replays draw fresh randomness with no host RNG."""
+        from ..ops import hip as _hip
+        step = _hip.StepInputs(*(bufs[k] for k in (
+            "tok", "out", "pos", "lens", "adv")))
+        sampled = (bufs["temps"], bufs["seeds"]) if klass == 1 else ()
+        if _hip.pick_and_advance(logits, step, *sampled):
+            return
+        if klass == 1:
+            toks = _hip.sample_gumbel(logits, *sampled, bufs["lens"])
+        else:
+            toks = ops.sample(logits, 0.0, 0, 1.0, None)
+        bufs["tok"].copy_(toks)
+        bufs["out"].copy_(toks)
+        bufs["pos"] += bufs["adv"]
+        bufs["lens"] += bufs["adv"]
 
     def _graph_replay(self, entry):
         bufs, meta = entry["bufs"], entry["meta"]
@@ -597,8 +602,10 @@ class LlamaEngine:
                     warm_logits = self.model.forward(
                         bufs["tok"], bufs["pos"], self.kv, bufs["slot"],
                         meta)
-                    # eager tail warmup — see _graph_tail docstring
-                    self._graph_tail(entry, warm_logits)
+                    # the end of the step too, so that its kernels are
+                    # loaded, but on copies: it moves the batch on
+                    self._graph_tail(entry["klass"], warm_logits,
+                                     {k: v.clone() for k, v in bufs.items()})
             torch.cuda.current_stream().wait_stream(s)
             for k, v in live.items():
                 bufs[k].copy_(v)
@@ -610,15 +617,7 @@ class LlamaEngine:
                     entry["logits"] = self.model.forward(
                         bufs["tok"], bufs["pos"], self.kv, bufs["slot"],
                         meta)
-                    # self-advancing tail: sample in-graph and stage the
-                    # NEXT step's inputs on-device, so a steady decode
-                    # batch replays back-to-back with no host round-trip
-                    toks32 = self._graph_tail(entry, entry["logits"])
-                    toks = toks32.long()
-                    bufs["tok"].copy_(toks32)
-                    entry["out"] = toks
-                    bufs["pos"] += bufs["adv"]
-                    bufs["lens"] += bufs["adv"]
+                    self._graph_tail(entry["klass"], entry["logits"], bufs)
             finally:
                 gc.enable()
             entry["graph"] = g
@@ -684,12 +683,11 @@ class LlamaEngine:
         pos_list = [s.total_len - 1 for s in seqs]
         q_lens = [1] * len(seqs)
         if self.use_graphs:
-            for s in seqs:
-                self.kv.ensure(s.slot, self.kv.seq_lens[s.slot] + 1)
+            self._one_more(seqs)
             logits = self._decode_forward_graphed(seqs, token_list, pos_list)
         else:
             logits = self._forward(seqs, token_list, pos_list, q_lens,
-                                   "decode")
+                                   "decode")    # one position each
         toks = self._sample(seqs, logits)
         now = time.monotonic()
         for s, tok in zip(seqs, toks):
@@ -713,8 +711,7 @@ class LlamaEngine:
         if self._pipe is not None and self._pipe["key"] != key:
             self._drain_pipe()
         # host/device page bookkeeping for the token this replay appends
-        for s in seqs:
-            self.kv.ensure(s.slot, self.kv.seq_lens[s.slot] + 1)
+        self._one_more(seqs)
         entry = self._graph_entry(self._bucket(len(seqs)), key[1])
         if self._pipe is None:
             # (re)sync device input buffers from host truth

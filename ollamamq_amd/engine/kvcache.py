@@ -68,21 +68,40 @@ class SequenceCache:
 
     def ensure(self, slot: int, new_len: int) -> None:
         """Grow slot's page list to cover new_len tokens."""
-        if new_len > self.max_ctx:
-            raise RuntimeError(f"sequence exceeds max_ctx {self.max_ctx}")
-        need = (new_len + self.page_size - 1) // self.page_size
-        pages = self._slot_pages[slot]
-        had = len(pages)
-        if need - had > len(self._free_pages):
-            raise RuntimeError("KV cache: out of pages")
-        while len(pages) < need:
-            pages.append(self._free_pages.pop())
-        if need == had + 1:
-            self.page_table[slot, had] = pages[had]
-        elif need > had:
-            self.page_table[slot, had:need] = torch.tensor(
-                pages[had:], dtype=torch.int32)
-        self.seq_lens[slot] = new_len
+        self.ensure_all([(slot, new_len)])
+
+    def ensure_all(self, wanted: List[Tuple[int, int]]) -> None:
+        """Grow page lists to cover new_len tokens each, (slot, new_len)
+        pairs.  New entries of the page table go to the device together, and
+        nothing waits for what it still has to do."""
+        width = self.page_table.shape[1]
+        places: List[int] = []
+        values: List[int] = []
+        try:
+            for slot, new_len in wanted:
+                if new_len > self.max_ctx:
+                    raise RuntimeError(
+                        f"sequence exceeds max_ctx {self.max_ctx}")
+                need = (new_len + self.page_size - 1) // self.page_size
+                pages = self._slot_pages[slot]
+                had = len(pages)
+                if need - had > len(self._free_pages):
+                    raise RuntimeError("KV cache: out of pages")
+                while len(pages) < need:
+                    pages.append(self._free_pages.pop())
+                places.extend(range(slot * width + had, slot * width + need))
+                values.extend(pages[had:])
+                self.seq_lens[slot] = new_len
+        finally:
+            table = self.page_table.view(-1)
+            if len(places) == 1:
+                table[places[0]] = values[0]
+            elif places:
+                both = torch.tensor([places, values], dtype=torch.int64)
+                if table.is_cuda:
+                    both = both.pin_memory()
+                both = both.to(table.device, non_blocking=True)
+                table.index_copy_(0, both[0], both[1].int())
 
     def can_fit(self, extra_tokens: int) -> bool:
         return len(self._free_pages) * self.page_size >= extra_tokens

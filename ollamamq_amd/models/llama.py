@@ -460,15 +460,13 @@ class LlamaModel:
         B = tokens.shape[0]
         H = cfg.hidden
         nl, nkl, d = self.n_local_heads, self.n_local_kv_heads, cfg.head_dim
-        emb = ops.embedding(tokens, self.embed)
-        if not emb.is_contiguous():
-            emb = emb.contiguous()
         sq_a, sq_b = self._sq_a, self._sq_b
         # res lives in the 32-row frag layout for the WHOLE chain: every
         # consumer GEMM streams its activation input linearly exactly
         # like packed weights (the scattered x machinery measured 15-30%
         # on top of the pure stream rate — profiles/r02_gemm_sweep.md)
-        res = ops.fragify_sumsq(emb, xf=self._res_frag, sq=sq_a[:B])[0]
+        res = ops.fragify_sumsq(self.embed, self._res_frag, sq_a[:B],
+                                tokens)[0]
         nt = 1                      # embed stats = one partial tile
         inv_h = 1.0 / H
         eps = cfg.norm_eps

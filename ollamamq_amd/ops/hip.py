@@ -45,7 +45,7 @@ def _try_load():
                                     i, i, i, i, i, i, f, i64, vp]
     lib.swiglu_bf16.argtypes = [vp, vp, i, i, i, vp]
     lib.swiglu_f32.argtypes = lib.swiglu_bf16.argtypes
-    lib.argmax_bf16.argtypes = [vp, vp, i, i, vp, vp, i, vp]
+    lib.argmax_bf16.argtypes = [vp, vp, i, i, vp, vp, i, *[vp] * 6]
     lib.argmax_f32.argtypes = lib.argmax_bf16.argtypes
     lib.decode_attn_bf16.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp,
                                      i, i, i, i, i, f, i64, i, i, i, vp]
@@ -62,9 +62,9 @@ def _try_load():
     lib.wstream_gu_bf16.argtypes = [vp, vp, vp, i, i, i, i64, i,
                                     vp, i, f, f, i, i, vp]
     lib.row_sumsq_bf16.argtypes = [vp, vp, i, i, vp]
-    lib.fragify_sumsq_bf16.argtypes = [vp, vp, vp, i, i, vp]
+    lib.fragify_sumsq_bf16.argtypes = [vp, vp, vp, vp, i, i, vp]
     lib.sample_gumbel_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i, i,
-                                       vp, vp, i, vp]
+                                       vp, vp, i, *[vp] * 6]
     lib.wstream_qkv_rope_bf16.argtypes = [vp, vp, vp, vp, i, i, i, i64,
                                           vp, i, f, f, vp, vp, vp, vp,
                                           vp, vp, vp, i, i, i, i, i, vp]
@@ -367,6 +367,13 @@ def attention_decode(q, cache, layer, meta, fragout=False, out=None):
     return out
 
 
+def upload(values, dev):
+    """int32 tensor of host values, without waiting for what the device still
+    has to do."""
+    t = torch.tensor(values, dtype=torch.int32)
+    return t.pin_memory().to(dev, non_blocking=True)
+
+
 def _prefill_plan(meta, first, G, KVH, dev):
     """(tiles, waves a block) of the sequences from `first` on, the longest
     walks first; cached on the meta object (one build per forward, shared by
@@ -387,8 +394,7 @@ def _prefill_plan(meta, first, G, KVH, dev):
             items.append((slot, tok, kv - n, row, min(rows, n * G - row)))
         tok += n
     items.sort(key=lambda it: -(it[2] + (it[3] + it[4]) // G))
-    plan = (torch.tensor(items, dtype=torch.int32).to(dev) if items
-            else None), waves
+    plan = (upload(items, dev) if items else None), waves
     meta._prefill = plan
     return plan
 
@@ -687,16 +693,21 @@ def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
     return y
 
 
-def fragify_sumsq(x, xf=None, sq=None):
+def fragify_sumsq(x, xf=None, sq=None, tokens=None):
     """Standard [M, H] -> 32-row frag layout + per-row sum of squares
-    (seeds the fused decode chain after the embedding gather)."""
+    (seeds the fused decode chain); with tokens, of their rows of the
+    embedding table x."""
     M, H = x.shape
+    if tokens is not None:
+        M, tokens = tokens.shape[0], _i32(tokens)
+        assert tokens.is_contiguous()
+    assert x.is_contiguous() and H % 8 == 0
     if xf is None:
         xf = torch.empty(((M + 31) // 32) * 32 * H, dtype=x.dtype,
                          device=x.device)
     if sq is None:
         sq = torch.empty(M, dtype=torch.float32, device=x.device)
-    _check(_lib.fragify_sumsq_bf16(_p(xf), _p(sq), _p(x), M, H,
+    _check(_lib.fragify_sumsq_bf16(_p(xf), _p(sq), _p(x), _p(tokens), M, H,
                                    _stream()), "fragify_sumsq")
     return xf, sq
 
@@ -1211,8 +1222,7 @@ def _chunk_plan(meta, dev, step_tokens):
         seqs.append((len(chunks), (n + 63) // 64))
         chunks += [(row + t, min(64, n - t)) for t in range(0, n, 64)]
         row += n
-    t32 = lambda x: torch.tensor(x, dtype=torch.int32).to(dev) \
-        if x else None
+    t32 = lambda x: upload(x, dev) if x else None
     plan = (t32(spans), t32(chunks), t32(seqs), base, row - base)
     setattr(meta, key, plan)
     return plan
@@ -1705,8 +1715,7 @@ def _tile_plan(meta, R, rows, dev):
         lo, hi = row * R, (row + n) * R
         long_ += [(r, min(rows, hi - r)) for r in range(lo, hi, rows)]
         row += n
-    t32 = lambda x: torch.tensor(x, dtype=torch.int32).to(dev) \
-        if x else None
+    t32 = lambda x: upload(x, dev) if x else None
     plan = (t32(short), n_short, kv, t32(long_))
     setattr(meta, key, plan)
     return plan
@@ -1930,33 +1939,66 @@ def moe_experts(h, w, chosen, share, packs):
     return Weighted(out, share)
 
 
-_scratch = {}
+class StepInputs(NamedTuple):
+    """Device inputs of a decode step that a step's picks are written to: tok,
+    pos, lens int32 and out int64 per row; adv: how far a row moves on."""
+    tok: torch.Tensor
+    out: torch.Tensor
+    pos: torch.Tensor
+    lens: torch.Tensor
+    adv: torch.Tensor
 
 
-def sample_gumbel(logits, temps, seeds, ctrs, noise=None, out=None):
+def _slices(B, like):
+    """Slices of a row (B blocks alone underfill the chip at decode batch
+    sizes) and room for the best value and index of each."""
+    sp = min(32, max(1, 768 // max(1, B)))
+    best = torch.empty(2, B * sp, dtype=torch.float32, device=like.device)
+    return sp, best
+
+
+def _step_ptrs(step):
+    return [_p(t) for t in (step or (None,) * 5)]
+
+
+def _argmax(logits, out, step=None):
+    B, V = logits.shape
+    l = logits if logits.dtype in (torch.float32, torch.bfloat16) \
+        else logits.bfloat16()
+    sp, best = _slices(B, l)
+    fn = _lib.argmax_f32 if l.dtype == torch.float32 else _lib.argmax_bf16
+    _check(fn(_p(out), _p(l), B, V, _p(best[0]), _p(best[1]), sp,
+              *_step_ptrs(step), _stream()), "argmax")
+
+
+def pick_and_advance(logits, step, temps=None, seeds=None):
+    """Greedy tokens, or sampled ones where temps > 0 (see sample_gumbel, the
+    counters are the lengths), become the next step's inputs.  False if the
+    logits' rows are not aligned for the kernel."""
+    if logits.shape[1] % 8 or not logits.is_contiguous():
+        return False
+    if temps is None:
+        _argmax(logits, None, step)
+    else:
+        sample_gumbel(logits, temps, seeds, step.lens, step=step)
+    return True
+
+
+def sample_gumbel(logits, temps, seeds, ctrs, noise=None, out=None,
+                  step=None):
     """Exact temperature sampling (Gumbel-max): token ~ softmax(l/T) per
     row; rows with temps<=0 are greedy argmax.  Counter-based noise from
     (seeds[row], ctrs[row], v) — graph-replay-safe and reproducible per
     request.  noise: optional [B,V] uniform(0,1) override (tests)."""
     B, V = logits.shape
     l = logits if logits.dtype == torch.bfloat16 else logits.bfloat16()
-    if out is None:
+    if out is None and step is None:
         out = torch.empty(B, dtype=torch.int32, device=logits.device)
-    sp = min(32, max(1, 768 // max(1, B)))
-    pb = pi = ctypes.c_void_p(0)
-    if sp > 1:
-        key = ("gmb", B, sp, str(logits.device))
-        t = _scratch.get(key)
-        if t is None:
-            t = (torch.empty(B * sp, dtype=torch.float32,
-                             device=logits.device),
-                 torch.empty(B * sp, dtype=torch.int32,
-                             device=logits.device))
-            _scratch[key] = t
-        pb, pi = _p(t[0]), _p(t[1])
+    sp, best = _slices(B, l)
     _check(_lib.sample_gumbel_bf16(
         _p(out), _p(l), _p(temps), _p(seeds), _p(ctrs), _p(noise),
-        B, V, pb, pi, sp, _stream()), "sample_gumbel")
+        B, V, _p(best[0]), _p(best[1]), sp, *_step_ptrs(step), _stream()),
+        "sample_gumbel")
     return out
 
 
@@ -1970,24 +2012,7 @@ def sample(logits, temperature, top_k, top_p, generator=None):
         if V % 8 or not logits.is_contiguous():
             return logits.argmax(-1)     # rows not aligned for the kernel
         out = torch.empty(B, dtype=torch.int32, device=logits.device)
-        f32 = logits.dtype == torch.float32
-        l = logits if f32 or logits.dtype == torch.bfloat16 \
-            else logits.bfloat16()
-        # split-V: B blocks alone underfill the chip at decode batch sizes
-        sp = min(32, max(1, 768 // max(1, B)))
-        pb = pi = ctypes.c_void_p(0)
-        if sp > 1:
-            key = ("amax", B, sp, str(logits.device))
-            t = _scratch.get(key)
-            if t is None:
-                t = (torch.empty(B * sp, dtype=torch.float32,
-                                 device=logits.device),
-                     torch.empty(B * sp, dtype=torch.int32,
-                                 device=logits.device))
-                _scratch[key] = t
-            pb, pi = _p(t[0]), _p(t[1])
-        fn = _lib.argmax_f32 if f32 else _lib.argmax_bf16
-        _check(fn(_p(out), _p(l), B, V, pb, pi, sp, _stream()), "argmax")
+        _argmax(logits, out)
         return out.long()
     # stochastic host path.  When every stochastic row carries
     # 0 < top_k <= 256 the sampling is EXACT over the top-256 candidates

@@ -742,10 +742,11 @@ def linear_fused(x, packed, N, bias=None, rstd=None, rstd_nt=0,
                              K=K, xlds=xlds, M_frag=M_frag, sem=sem)
 
 
-def fragify_sumsq(x, xf=None, sq=None):
-    """Standard [M, H] -> 32-row frag layout + per-row sum of squares."""
+def fragify_sumsq(x, xf=None, sq=None, tokens=None):
+    """Standard [M, H] -> 32-row frag layout + per-row sum of squares; with
+    tokens, of their rows of the embedding table x."""
     from . import hip
-    return hip.fragify_sumsq(x, xf, sq)
+    return hip.fragify_sumsq(x, xf, sq, tokens)
 
 
 def attention_decode_frag(q, cache, layer, meta):
