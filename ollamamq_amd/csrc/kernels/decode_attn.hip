@@ -36,6 +36,20 @@ constexpr int D = 128, NW = 8, KT = 32;
 
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
 
+// two floats that other blocks write or read in the same launch
+DEV void put2(float* p, float a, float b) {
+    const uint64_t v = (uint64_t)__float_as_uint(b) << 32
+                       | __float_as_uint(a);
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(p), v, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+DEV float2 get2(const float* p) {
+    const uint64_t v = __hip_atomic_load(
+        reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED,
+        __HIP_MEMORY_SCOPE_AGENT);
+    return {__uint_as_float((unsigned)v), __uint_as_float(v >> 32)};
+}
+
 // Pages: with SH they are 1 << pshift tokens and no smaller than a tile of
 // 16 keys, so a tile's page number is the same for the whole wave; otherwise
 // any number of tokens, looked up key by key.
@@ -44,6 +58,7 @@ __global__ __launch_bounds__(NW * 64, 2) void k_decode_attn(
     bf16* __restrict__ out,               // [S, Hq, D] (split == 1)
     float* __restrict__ o_part,           // [S, Hq, split, D]
     float* __restrict__ ml_part,          // [S, Hq, split, 2] maximum, sum
+    int* __restrict__ sem,                // [S, KVH] tickets, zero
     const bf16* __restrict__ q,           // [S, Hq, D], rows qs apart
     const bf16* __restrict__ kpool,       // [P][KVH][page][D]
     const bf16* __restrict__ vpool,
@@ -61,9 +76,11 @@ __global__ __launch_bounds__(NW * 64, 2) void k_decode_attn(
     // first key that the query, at kv_len - 1, sees
     const int lo = window > 0 ? max(0, kv_len - window) : 0;
     const int first = lo / KT, steps = (kv_len + KT - 1) / KT - first;
-    const int GW = split * NW;            // a wave's steps: every GW-th
-    // a part without keys; the first writes zeros where there are none at all
-    if (blockIdx.z && (int)blockIdx.z * NW >= steps) return;
+    // parts in use: every wave has a step (300 tokens of one user: 7.3 us in
+    // one part, 8.2 in two)
+    const int parts = max(1, min(split, steps / NW));
+    if ((int)blockIdx.z >= parts) return;
+    const int GW = parts * NW;            // a wave's steps: every GW-th
 
     __shared__ __attribute__((aligned(16))) float o_s[NW * 8 * D];
     __shared__ float ml_s[NW * 8 * 2];
@@ -198,8 +215,9 @@ __global__ __launch_bounds__(NW * 64, 2) void k_decode_attn(
         }
     }
     __syncthreads();
-    if (threadIdx.x >= G * (D / 4)) return;
-    const int h = threadIdx.x / (D / 4), c = (threadIdx.x % (D / 4)) * 4;
+    const bool live = threadIdx.x < G * (D / 4);
+    const int h = live ? threadIdx.x / (D / 4) : 0;
+    const int c = (threadIdx.x % (D / 4)) * 4, hq = kvh * G + h;
     float top = NEG, den = 0.f;
     #pragma unroll
     for (int w = 0; w < NW; w++) top = fmaxf(top, ml_s[(w * G + h) * 2]);
@@ -210,72 +228,72 @@ __global__ __launch_bounds__(NW * 64, 2) void k_decode_attn(
         den += f * ml_s[(w * G + h) * 2 + 1];
         sum += f * *reinterpret_cast<const f32x4*>(o_s + (w * G + h) * D + c);
     }
-    const int hq = kvh * G + h;
-    if (split == 1) {
-        sum *= den > 0.f ? 1.f / den : 0.f;
-        put_out(out, seq, hq, c, Hq, D, sum, fragout);
-        return;
+    if (parts > 1) {
+        // The block that arrives last merges the parts, in their order.  They
+        // are written through and read past the caches (agent scope), so the
+        // stores have only to be complete before the ticket is drawn.
+        const int64_t at = ((int64_t)seq * Hq + hq) * split;
+        if (live) {
+            put2(o_part + (at + blockIdx.z) * D + c, sum[0], sum[1]);
+            put2(o_part + (at + blockIdx.z) * D + c + 2, sum[2], sum[3]);
+            if (c == 0) put2(ml_part + (at + blockIdx.z) * 2, top, den);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        int* drawn = reinterpret_cast<int*>(o_s);
+        if (threadIdx.x == 0)
+            *drawn = __hip_atomic_fetch_add(
+                sem + seq * KVH + kvh, 1, __ATOMIC_RELAXED,
+                __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (*drawn != parts - 1) return;
+        if (threadIdx.x == 0)             // ready for the next launch
+            __hip_atomic_store(sem + seq * KVH + kvh, 0, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        top = NEG;
+        den = 0.f;
+        sum = f32x4{};
+        #pragma unroll 4
+        for (int i = 0; i < parts; i++) {
+            const float2 ml = get2(ml_part + (at + i) * 2);
+            const float2 a = get2(o_part + (at + i) * D + c);
+            const float2 b = get2(o_part + (at + i) * D + c + 2);
+            const float mn = fmaxf(top, ml.x);
+            const float f = __builtin_amdgcn_exp2f(top - mn);
+            const float w = __builtin_amdgcn_exp2f(ml.x - mn);
+            top = mn;
+            den = den * f + ml.y * w;
+            sum = sum * f + f32x4{a.x, a.y, b.x, b.y} * w;
+        }
     }
-    const int64_t part = ((int64_t)seq * Hq + hq) * split + blockIdx.z;
-    *reinterpret_cast<f32x4*>(o_part + part * D + c) = sum;
-    if (c == 0) {
-        ml_part[part * 2] = top;
-        ml_part[part * 2 + 1] = den;
-    }
-}
-
-// merge of the parts: 32 lanes per (sequence, head)
-__global__ __launch_bounds__(256) void k_decode_combine(
-    bf16* __restrict__ out, const float* __restrict__ o_part,
-    const float* __restrict__ ml_part, const int* __restrict__ seq_lens,
-    int total, int split, int Hq, int window, int fragout)
-{
-    const int sh = blockIdx.x * 8 + threadIdx.x / 32;
-    const int c = (threadIdx.x % 32) * 4;
-    if (sh >= total) return;
-    // parts that have keys: the first step of the last of them exists
-    const int kv_len = seq_lens[sh / Hq];
-    const int lo = window > 0 ? max(0, kv_len - window) : 0;
-    const int steps = (kv_len + KT - 1) / KT - lo / KT;
-    const int parts = min(split, (steps + NW - 1) / NW);
-    const float* ml = ml_part + (int64_t)sh * split * 2;
-    const float* o = o_part + (int64_t)sh * split * D + c;
-    float top = NEG, den = 0.f;
-    for (int i = 0; i < parts; i++) top = fmaxf(top, ml[i * 2]);
-    f32x4 sum = {};
-    #pragma unroll 4
-    for (int i = 0; i < parts; i++) {
-        const float f = __builtin_amdgcn_exp2f(ml[i * 2] - top);
-        den += f * ml[i * 2 + 1];
-        sum += f * *reinterpret_cast<const f32x4*>(o + i * D);
-    }
+    if (!live) return;
     sum *= den > 0.f ? 1.f / den : 0.f;
-    put_out(out, sh / Hq, sh % Hq, c, Hq, D, sum, fragout);
+    put_out(out, seq, hq, c, Hq, D, sum, fragout);
 }
 
+// part: S * Hq * split * (D + 2) floats, sem: S * KVH zeros, which are zero
+// again at the end; neither is used with split 1
 extern "C" int decode_attn_bf16(
-    void* out, void* o_part, void* ml_part, const void* q,
-    const void* kpool, const void* vpool, const void* page_table,
-    const void* slot_ids, const void* seq_lens, int S, int Hq, int KVH,
-    int page, int max_pages, float scale, int64_t q_stride, int split,
-    int window, int fragout, hipStream_t stream)
+    void* out, void* part, void* sem, const void* q, const void* kpool,
+    const void* vpool, const void* page_table, const void* slot_ids,
+    const void* seq_lens, int S, int Hq, int KVH, int page, int max_pages,
+    float scale, int64_t q_stride, int split, int window, int fragout,
+    hipStream_t stream)
 {
     const int G = Hq / KVH;
     if (G < 1 || G > 8 || G * KVH != Hq || page < 1
-        || (reinterpret_cast<uintptr_t>(q) & 15) || q_stride % 8)
+        || (reinterpret_cast<uintptr_t>(q) & 15) || q_stride % 8
+        || split < 1 || (split > 1 && (!part || !sem)))
         return (int)hipErrorInvalidValue;
     const bool sh = page >= 16 && !(page & (page - 1));
     const float unit = scale * 1.4426950408889634f;
     auto go = sh ? k_decode_attn<true> : k_decode_attn<false>;
     go<<<dim3(KVH, S, split), NW * 64, 0, stream>>>(
-        (bf16*)out, (float*)o_part, (float*)ml_part, (const bf16*)q,
-        (const bf16*)kpool, (const bf16*)vpool, (const int*)page_table,
+        (bf16*)out, (float*)part, (float*)part + (int64_t)S * Hq * split * D,
+        (int*)sem, (const bf16*)q, (const bf16*)kpool, (const bf16*)vpool,
+        (const int*)page_table,
         (const int*)slot_ids, (const int*)seq_lens, G, KVH, page,
         sh ? __builtin_ctz(page) : 0, max_pages, unit, q_stride, window,
         fragout);
-    if (split > 1)
-        k_decode_combine<<<(S * Hq + 7) / 8, 256, 0, stream>>>(
-            (bf16*)out, (const float*)o_part, (const float*)ml_part,
-            (const int*)seq_lens, S * Hq, split, Hq, window, fragout);
     return (int)hipGetLastError();
 }

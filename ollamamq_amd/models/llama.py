@@ -352,8 +352,9 @@ class LlamaModel:
             self._sq_a = torch.zeros(max(th, 1) * 64, dtype=torch.float32,
                                      device=self.device)
             self._sq_b = torch.zeros_like(self._sq_a)
-            # tickets of the split products, zero between them
-            self._tickets = torch.zeros(max(th, 1), dtype=torch.int32,
+            # tickets of products and attention in parts, zero between them
+            self._tickets = torch.zeros(max(th, 64 * self.n_local_kv_heads),
+                                        dtype=torch.int32,
                                         device=self.device)
             # frag-layout residual stream: two 32-row halves (the MT2
             # chain serves batches up to 64; rows >= batch hold garbage
@@ -481,7 +482,8 @@ class LlamaModel:
                 rstd=sq_a, rstd_nt=nt, inv_h=inv_h, eps=eps,
                 K=H, M_real=B)
             q = qkv[:, :nl * d].view(-1, nl, d)
-            attn = ops.attention_decode_frag(q, kv_cache, li, attn_meta)
+            attn = ops.attention_decode_frag(q, kv_cache, li, attn_meta,
+                                             self._tickets)
             ops.linear_fused(attn, layer.wo_pk, H, res=res, sq_out=sq_b,
                              y=res, yfrag=1, K=nl * d, xlds=2, M_frag=B,
                              sem=self._tickets)

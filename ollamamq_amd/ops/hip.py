@@ -317,8 +317,8 @@ def _attention(q, cache, layer, meta, qt):
 def _decode_split(pairs, max_kv):
     """Parts of a context, for `pairs` (sequence, key/value head) pairs.  From
     192 pairs on the chip has a block a CU and one part is best (32 users of
-    about 512 tokens, 8 key/value heads: 18.2 us against 20.9 with two and
-    their merge); below, up to 768 blocks help where contexts are long or
+    about 512 tokens, 8 key/value heads: 18.2 us against 20.9 with two);
+    below, up to 768 blocks help where contexts are long or
     ragged (12 users of 4096 to 12288: 149 us whole, 91 in two, 80 in
     eight).  A part has at least a step of 32 keys for each of its eight
     waves."""
@@ -330,12 +330,15 @@ def _decode_split(pairs, max_kv):
     return min(want, max(1, (max_kv + 255) // 256), 32)
 
 
-def attention_decode(q, cache, layer, meta, fragout=False, out=None):
+def attention_decode(q, cache, layer, meta, fragout=False, out=None,
+                     sem=None):
     """Attention of one query token per sequence over its paged keys and
     values, the context of a (sequence, key/value head) in parts while there
     are few of them.
     fragout: emit the output in the fused-chain 32-row frag layout (the
-    o GEMM streams it linearly like packed weights)."""
+    o GEMM streams it linearly like packed weights).  sem: int32 zeros, one per
+    (sequence, key/value head); they are zero again at the end, so a stream's
+    launches can share them."""
     S, Hq, D = q.shape
     assert D == 128
     if out is None:
@@ -349,17 +352,19 @@ def attention_decode(q, cache, layer, meta, fragout=False, out=None):
     kp, vp = _layer_ptrs(cache, layer)
     kvh = cache.n_kv_heads
     split = _decode_split(S * kvh, meta.max_kv)
-    op = mp = ctypes.c_void_p(0)
+    part = None
     if split > 1:
         part = torch.empty(S * Hq * split * (D + 2), dtype=torch.float32,
                            device=q.device)
-        op, mp = _p(part), _p(part[S * Hq * split * D:])
+        if sem is None:
+            sem = torch.zeros(S * kvh, dtype=torch.int32, device=q.device)
+        assert sem.numel() >= S * kvh
     slot32 = meta.slot_ids.int() if meta.slot_ids.dtype != torch.int32 \
         else meta.slot_ids
     len32 = meta.seq_lens.int() if meta.seq_lens.dtype != torch.int32 \
         else meta.seq_lens
     _check(_lib.decode_attn_bf16(
-        _p(out), op, mp, _p(q), kp, vp, _p(cache.page_table),
+        _p(out), _p(part), _p(sem), _p(q), kp, vp, _p(cache.page_table),
         _p(slot32), _p(len32), S, Hq, kvh, cache.page_size,
         cache.page_table.shape[1], 1.0 / (D ** 0.5), _row_stride(q, D),
         split, meta.window, 1 if fragout else 0, _stream()),

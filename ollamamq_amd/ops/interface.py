@@ -749,10 +749,11 @@ def fragify_sumsq(x, xf=None, sq=None, tokens=None):
     return hip.fragify_sumsq(x, xf, sq, tokens)
 
 
-def attention_decode_frag(q, cache, layer, meta):
-    """Decode attention emitting its output in frag layout."""
+def attention_decode_frag(q, cache, layer, meta, sem=None):
+    """Decode attention emitting its output in frag layout; sem: see
+    hip.attention_decode."""
     from . import hip
-    return hip.attention_decode(q, cache, layer, meta, fragout=True)
+    return hip.attention_decode(q, cache, layer, meta, fragout=True, sem=sem)
 
 
 def gu_fused(x, packed, N, rstd, rstd_nt, inv_h, eps, K=None, yfrag=0,

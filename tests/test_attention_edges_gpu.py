@@ -112,10 +112,13 @@ def test_decode_parts(split, monkeypatch):
         q = whole.flatten()[first:].as_strided((len(lens), 8, D),
                                                (stride, D, 1))
         meta = _meta(slots, lens, [1] * len(lens), 0, "decode")
-        got = hip.attention_decode(q, cache, 0, meta)
         want = _exact(q, cache, 0, slots, lens, [1] * len(lens), 0)
-        torch.testing.assert_close(got.double(), want, rtol=2 ** -8,
-                                   atol=1e-5)
+        sem = torch.zeros(2 * len(lens), dtype=torch.int32, device="cuda")
+        for tickets in (None, sem, sem, sem):       # given and shared
+            got = hip.attention_decode(q, cache, 0, meta, sem=tickets)
+            torch.testing.assert_close(got.double(), want, rtol=2 ** -8,
+                                       atol=1e-5)
+            assert not sem.any()
 
 
 # queries, cached tokens before them
