@@ -76,9 +76,10 @@ extern "C" int wstream_pure_bf16(void* sink, const void* wp, int N, int K,
 // DEPTH: weights under way per wave, in 4 KiB iterations.
 // XLDS == 2: x in fragment layout (the decode chain).  A CU's loads are what
 // bounds it, x counted: rows past M repeat row M - 1, so few rows cost few
-// cache lines.  4 iterations ahead for 32 rows, 2 for 64 (registers).  Alone,
-// 28672 x 4096: 47 us before for any M, now 43 for 32 rows, 41 for 8;
-// 4096 x 4096: 12.5, now 8.5 and 7.8 in two parts.
+// cache lines.  4 iterations ahead for 32 rows, in registers for two blocks a
+// CU; 2 for 64, where one block a CU with two of x under way beats two with
+// one (37888 x 3584: 70 us against 79).  28672 x 4096 with its norm and
+// activation: 46 us before for any M, now 44 for 32 rows, 39 for 1.
 // XLDS (requires MT==1): stage the x fragments through a wave-PRIVATE
 // LDS tile instead of loading them in MFMA layout.  The direct x
 // fragment load is 32 rows x 16 B at an 8 KB stride = 32 cache-line
@@ -122,7 +123,8 @@ struct RopeEpi {
 };
 
 template <int MT, int DEPTH = 1, int XLDS = 0, int GU = 0, int RP = 0>
-__global__ __launch_bounds__(512) void k_wstream_gemm(
+__global__ __launch_bounds__(512, XLDS == 2 && MT == 1 ? 4 : 1)
+void k_wstream_gemm(
     bf16* __restrict__ y,            // [M, N] (ksplit == 1)
     float* __restrict__ part,        // [ksplit, M, N] (ksplit > 1)
     const bf16* __restrict__ x,      // [M, K], row stride xs
@@ -165,6 +167,28 @@ __global__ __launch_bounds__(512) void k_wstream_gemm(
     extern __shared__ __align__(16) char smem[];
 
     f32x16 acc0 = {}, acc1 = {};
+    // rmsnorm scale of the raw-residual input: this row's sq partials from
+    // the producing GEMM, FL lanes a row, several loads at a time.  The frag
+    // path loads them beside its first weights: behind the stream they cost
+    // every block another memory latency (gate-up 46.7 us for 32 rows, 41.6
+    // for 1; now 43.8 and 38.9).
+    constexpr int FL = MT == 2 ? 8 : 16;
+    float rsum = 0.f;
+    auto fold = [&]() {
+        const int m = tid / FL;
+        if (!rstd_parts || m >= M) return;
+        const float* p = rstd_parts + (int64_t)m * rstd_nt;
+        int i = tid % FL;
+        for (; i + 7 * FL < rstd_nt; i += 8 * FL) {
+            float v[8];
+            #pragma unroll
+            for (int k = 0; k < 8; k++) v[k] = p[i + k * FL];
+            #pragma unroll
+            for (int k = 0; k < 8; k++) rsum += v[k];
+        }
+        for (; i + FL < rstd_nt; i += 2 * FL) rsum += p[i] + p[i + FL];
+        if (i < rstd_nt) rsum += p[i];
+    };
     if (XLDS == 2 && b_lo < b_hi) {
         // x in fragment layout: DEPTH iterations of weights and up to two of x
         // are under way.  The first round may begin before b_lo: those slots
@@ -205,6 +229,7 @@ __global__ __launch_bounds__(512) void k_wstream_gemm(
         for (int s = 0; s < DEPTH; s++) ldw(s, max(b + s, b_lo));
         #pragma unroll
         for (int s = 0; s < XS; s++) ldx(s, max(b + s, b_lo));
+        fold();
         for (; b + DEPTH < b_hi; b += DEPTH) {
             #pragma unroll
             for (int s = 0; s < DEPTH; s++) {
@@ -352,27 +377,15 @@ __global__ __launch_bounds__(512) void k_wstream_gemm(
     // ---- reduce 8 wave partials through LDS (aliases the x tiles: the
     // barrier closes the streaming epoch before anyone writes) ----
     float (*red8)[32][32] = reinterpret_cast<float (*)[32][32]>(smem);
-    // rmsnorm scale of the raw-residual input: sum this row's sq
-    // partials from the producing GEMM (L2-hot, overlapped with other
-    // waves' stream drain), publish rstd through the smem tail
     float* rstd_sh = reinterpret_cast<float*>(
         smem + (XLDS == 1 ? 16 * 4096 : 8 * 32 * 32 * 4));
     if (rstd_parts) {
-        // parallel partial fold: 8-16 lanes per row (each <= nt/L loads,
-        // independent), group-reduced with wave shuffles — a serial
-        // 32-thread loop here measurably stalled short-stream blocks.
-        // MT==2 folds 64 rows with 8 lanes each (512 threads exactly).
-        const int L = MT == 2 ? 8 : 16;
-        const int m2 = tid / L, c2 = tid % L;
-        float s = 0.f;
-        if (m2 < MT * 32)
-            for (int i = c2; i < rstd_nt; i += L)
-                s += rstd_parts[(int64_t)m2 * rstd_nt + i];
+        if (XLDS != 2 || b_lo >= b_hi) fold();
         #pragma unroll
-        for (int off = 8; off; off >>= 1)
-            if (off < L) s += __shfl_down(s, off, 64);
-        if (m2 < MT * 32 && c2 == 0)
-            rstd_sh[m2] = rsqrtf(s * inv_h + eps);
+        for (int off = FL / 2; off; off >>= 1)
+            rsum += __shfl_down(rsum, off, 64);
+        if (tid % FL == 0 && tid / FL < MT * 32)
+            rstd_sh[tid / FL] = rsqrtf(rsum * inv_h + eps);
     }
     if (GU) {
         const int F = N >> 1;                  // ffn width
