@@ -996,6 +996,41 @@ __global__ __launch_bounds__(256) void k_fragify_sumsq(
         sq[m] = red[0] + red[1] + red[2] + red[3];
 }
 
+// Selected rows of an activation in fragment layout, in that layout, and
+// their sums of squares
+__global__ __launch_bounds__(256) void k_frag_rows(
+    const uint4* __restrict__ x, const int64_t* __restrict__ rows,
+    uint4* __restrict__ xf, float* __restrict__ sq, int H)
+{
+    const int m = blockIdx.x, from = (int)rows[m];
+    const uint4* src = x + (int64_t)(from >> 5) * 4 * H + (from & 31);
+    uint4* dst = xf + (int64_t)(m >> 5) * 4 * H + (m & 31);
+    float s = 0.f;
+    for (int c = threadIdx.x; c < H / 8; c += 256) {
+        const uint4 v = src[(int64_t)c * 32];
+        float f[8];
+        load8f(reinterpret_cast<const bf16*>(&v), f);
+        #pragma unroll
+        for (int e = 0; e < 8; e++) s += f[e] * f[e];
+        dst[(int64_t)c * 32] = v;
+    }
+    __shared__ float red[4];
+    s = wave_reduce_sum(s);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        sq[m] = red[0] + red[1] + red[2] + red[3];
+}
+
+extern "C" int frag_rows_bf16(void* xf, void* sq, const void* x,
+                              const void* rows, int M, int H,
+                              hipStream_t stream)
+{
+    k_frag_rows<<<M, 256, 0, stream>>>((const uint4*)x, (const int64_t*)rows,
+                                       (uint4*)xf, (float*)sq, H);
+    return (int)hipGetLastError();
+}
+
 extern "C" int fragify_sumsq_bf16(void* xf, void* sq, const void* x,
                                   const void* tokens, int M, int H,
                                   hipStream_t stream)

@@ -56,12 +56,12 @@ struct Item { int slot, tok0, pos0, row0, rows; };
 
 template <bool SH, int NW>
 __global__ __launch_bounds__(NW * 64, 2) void k_prefill_attn(
-    bf16* __restrict__ out,               // [T, Hq, D]
+    bf16* __restrict__ out,               // [T, Hq, D], or its fragments
     const bf16* __restrict__ q,           // [T, Hq, D], rows qs apart
     const bf16* __restrict__ kpool,       // [P][KVH][page][D]
     const bf16* __restrict__ vpool, const int* __restrict__ page_table,
     const Item* __restrict__ items, int G, int KVH, int page, int pshift,
-    int max_pages, float unit, int64_t qs, int window)
+    int max_pages, float unit, int64_t qs, int window, int fragout)
 {
     const int kvh = blockIdx.x, Hq = G * KVH;
     const Item it = items[blockIdx.y];
@@ -189,15 +189,13 @@ __global__ __launch_bounds__(NW * 64, 2) void k_prefill_attn(
     l += __shfl_xor(l, 32, 64);
     if (w0 + col > end) return;
     const float f = l > 0.f ? 1.f / l : 0.f;
-    bf16* dst = out + ((int64_t)tok * Hq + head) * D + 4 * h;
     #pragma unroll
     for (int t = 0; t < 4; t++)
         #pragma unroll
-        for (int r = 0; r < 16; r += 4) {
-            const float v[4] = {o[t][r] * f, o[t][r + 1] * f,
-                                o[t][r + 2] * f, o[t][r + 3] * f};
-            stv<4>(dst + t * 32 + 2 * r, v);
-        }
+        for (int r = 0; r < 16; r += 4)
+            put_out(out, tok, head, t * 32 + 2 * r + 4 * h, Hq, D,
+                    f32x4{o[t][r], o[t][r + 1], o[t][r + 2], o[t][r + 3]}
+                        * f, fragout);
 }
 
 // items: int32 [n, 5]: slot, flat index and position of the portion's first
@@ -207,7 +205,7 @@ extern "C" int prefill_attn_bf16(
     void* out, const void* q, const void* kpool, const void* vpool,
     const void* page_table, const void* items, int n_items, int waves,
     int Hq, int KVH, int page, int max_pages, float scale, int64_t q_stride,
-    int window, hipStream_t stream)
+    int window, int fragout, hipStream_t stream)
 {
     const int G = Hq / KVH;
     if (G < 1 || G > 8 || G * KVH != Hq || page < 1
@@ -228,7 +226,7 @@ extern "C" int prefill_attn_bf16(
                     (const bf16*)vpool, (const int*)page_table,            \
                     (const Item*)items, G, KVH, page,                      \
                     sh ? __builtin_ctz(page) : 0, max_pages, unit,         \
-                    q_stride, window);                                     \
+                    q_stride, window, fragout);                            \
         } while (0)
     #define PF_W(SH)                                                       \
         do {                                                               \

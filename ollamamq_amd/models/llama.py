@@ -397,10 +397,12 @@ class LlamaModel:
         """Returns logits [T_last, vocab_full] for the tokens attn_meta
         selects as "last" (decode: all; prefill: final token per seq)."""
         cfg = self.cfg
-        if (self.fused_chain and attn_meta.mode == "decode"
-                and tokens.shape[0] <= 64 and not return_hidden):
-            return self._forward_decode_fused(tokens, positions, kv_cache,
-                                              slot_ids, attn_meta)
+        idx = attn_meta.logits_idx
+        if (self.fused_chain and 0 < tokens.shape[0] <= 64
+                and (idx is None or idx.shape[0] <= 64)
+                and not return_hidden):
+            return self._forward_fused(tokens, positions, kv_cache,
+                                       slot_ids, attn_meta)
         x = ops.embedding(tokens, self.embed)
         residual = None
         for li, layer in enumerate(self.layers):
@@ -430,7 +432,6 @@ class LlamaModel:
             self._allreduce(x)  # RCCL all-reduce #2 (TP)
 
         # Only the last token of each sequence needs logits.
-        idx = attn_meta.logits_idx
         if idx is not None:
             h = x[idx] + residual[idx]
         else:
@@ -448,10 +449,11 @@ class LlamaModel:
             logits = torch.cat(shards, dim=-1)
         return logits
 
-    def _forward_decode_fused(self, tokens, positions, kv_cache, slot_ids,
-                              attn_meta):
-        """Decode step as a fused weight-streaming chain (tp=1, B<=32):
-        4 GEMM-class kernels per layer, zero rmsnorm/swiglu kernels.
+    def _forward_fused(self, tokens, positions, kv_cache, slot_ids,
+                       attn_meta):
+        """A step of few tokens, decode or short portions of prompts, as a
+        fused weight-streaming chain (tp=1, up to 64 rows): 4 GEMM-class
+        kernels per layer, zero rmsnorm/swiglu kernels.
         rmsnorm weights are folded into the packs; the rstd scale rides
         each consumer GEMM's epilogue from sum-of-squares partials the
         producer GEMM emitted; residual adds happen in place inside the
@@ -482,8 +484,8 @@ class LlamaModel:
                 rstd=sq_a, rstd_nt=nt, inv_h=inv_h, eps=eps,
                 K=H, M_real=B)
             q = qkv[:, :nl * d].view(-1, nl, d)
-            attn = ops.attention_decode_frag(q, kv_cache, li, attn_meta,
-                                             self._tickets)
+            attn = ops.attention_frag(q, kv_cache, li, attn_meta,
+                                      self._tickets)
             ops.linear_fused(attn, layer.wo_pk, H, res=res, sq_out=sq_b,
                              y=res, yfrag=1, K=nl * d, xlds=2, M_frag=B,
                              sem=self._tickets)
@@ -496,8 +498,12 @@ class LlamaModel:
                              K=layer.wdown.shape[1], xlds=2, M_frag=B,
                              sem=self._tickets)
             nt = tiles_h
-        logits = ops.linear_fused(res, self.lm_head_pk,
-                                  self.lm_head.shape[0], rstd=sq_a,
-                                  rstd_nt=nt, inv_h=inv_h, eps=eps,
-                                  K=H, xlds=2, M_frag=B)
-        return logits[:B]
+        idx = attn_meta.logits_idx
+        if not attn_meta.one_each and idx is not None:
+            # the rows whose logits are wanted
+            res, sq_a = ops.frag_rows(res, idx, H)
+            nt, B = 1, idx.shape[0]
+        return ops.linear_fused(res, self.lm_head_pk,
+                                self.lm_head.shape[0], rstd=sq_a,
+                                rstd_nt=nt, inv_h=inv_h, eps=eps,
+                                K=H, xlds=2, M_frag=B)

@@ -54,7 +54,7 @@ def _try_load():
     lib.rope_append_bf16.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp, vp,
                                      i, i, i, i, i, i, i64, i64, i64, vp]
     lib.prefill_attn_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i, i, i, i, i,
-                                      i, f, i64, i, vp]
+                                      i, f, i64, i, i, vp]
     lib.embed_gather_bf16.argtypes = [vp, vp, vp, i, i, vp]
     lib.wstream_gemm_bf16.argtypes = [vp, vp, vp, vp, vp, i, i, i, i64, i,
                                       i, i, vp, i, f, f, vp, vp, i, vp, vp]
@@ -62,6 +62,7 @@ def _try_load():
     lib.wstream_gu_bf16.argtypes = [vp, vp, vp, i, i, i, i64, i,
                                     vp, i, f, f, i, i, vp]
     lib.row_sumsq_bf16.argtypes = [vp, vp, i, i, vp]
+    lib.frag_rows_bf16.argtypes = [vp, vp, vp, vp, i, i, vp]
     lib.fragify_sumsq_bf16.argtypes = [vp, vp, vp, vp, i, i, vp]
     lib.sample_gumbel_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i, i,
                                        vp, vp, i, *[vp] * 6]
@@ -404,7 +405,7 @@ def _prefill_plan(meta, first, G, KVH, dev):
     return plan
 
 
-def _prefill_rows(out, q, cache, layer, meta, first):
+def _prefill_rows(out, q, cache, layer, meta, first, fragout=False):
     """Attention of the sequences from `first` on, into their rows of out."""
     T, Hq, D = q.shape
     kvh = cache.n_kv_heads
@@ -418,17 +419,18 @@ def _prefill_rows(out, q, cache, layer, meta, first):
         _p(out), _p(q), kp, vp, _p(cache.page_table), _p(items),
         items.shape[0], waves, Hq, kvh, cache.page_size,
         cache.page_table.shape[1], 1.0 / (D ** 0.5), _row_stride(q, D),
-        meta.window, _stream()), "prefill_attn")
+        meta.window, int(fragout), _stream()), "prefill_attn")
 
 
-def attention_mixed(q, cache, layer, meta):
+def attention_mixed(q, cache, layer, meta, fragout=False, sem=None):
     """Mixed batch: decode kernel over the first n_decode rows, MFMA
     prefill kernel over the remaining chunk rows — both write into one
-    output tensor."""
+    output tensor.  fragout, sem: see attention_decode."""
     T, Hq, D = q.shape
     assert D == 128
-    nd = meta.n_decode
-    out = torch.empty((T, Hq, D), dtype=q.dtype, device=q.device)
+    nd = meta.n_single
+    out = torch.empty((-(-T // 32) * 32 * Hq * D,) if fragout
+                      else (T, Hq, D), dtype=q.dtype, device=q.device)
     sub = getattr(meta, "_mixed_dec", None)
     if sub is None:
         sub = AttnMeta(
@@ -438,8 +440,8 @@ def attention_mixed(q, cache, layer, meta):
             max_kv=meta.max_kv, window=meta.window)
         meta._mixed_dec = sub
     if nd:
-        attention_decode(q[:nd], cache, layer, sub, out=out)
-    _prefill_rows(out, q, cache, layer, meta, nd)
+        attention_decode(q[:nd], cache, layer, sub, fragout, out, sem)
+    _prefill_rows(out, q, cache, layer, meta, nd, fragout)
     return out
 
 
@@ -715,6 +717,19 @@ def fragify_sumsq(x, xf=None, sq=None, tokens=None):
     _check(_lib.fragify_sumsq_bf16(_p(xf), _p(sq), _p(x), _p(tokens), M, H,
                                    _stream()), "fragify_sumsq")
     return xf, sq
+
+
+def frag_rows(xf, rows, H):
+    """Rows (int64) of an activation in fragment layout, in that layout, and
+    their sums of squares."""
+    M = rows.shape[0]
+    assert rows.dtype == torch.int64 and rows.is_contiguous() and H % 64 == 0
+    out = torch.empty(-(-M // 32) * 32 * H, dtype=xf.dtype, device=xf.device)
+    sq = torch.empty(M, dtype=torch.float32, device=xf.device)
+    if M:
+        _check(_lib.frag_rows_bf16(_p(out), _p(sq), _p(xf), _p(rows), M, H,
+                                   _stream()), "frag_rows")
+    return out, sq
 
 
 def row_sumsq(x, out=None):

@@ -749,11 +749,20 @@ def fragify_sumsq(x, xf=None, sq=None, tokens=None):
     return hip.fragify_sumsq(x, xf, sq, tokens)
 
 
-def attention_decode_frag(q, cache, layer, meta, sem=None):
-    """Decode attention emitting its output in frag layout; sem: see
+def attention_frag(q, cache, layer, meta, sem=None):
+    """Attention emitting its output in frag layout; sem: see
     hip.attention_decode."""
     from . import hip
-    return hip.attention_decode(q, cache, layer, meta, fragout=True, sem=sem)
+    if meta.one_each:
+        return hip.attention_decode(q, cache, layer, meta, True, sem=sem)
+    return hip.attention_mixed(q, cache, layer, meta, True, sem)
+
+
+def frag_rows(xf, rows, H):
+    """Rows of an activation in frag layout, in that layout, and their sums
+    of squares."""
+    from . import hip
+    return hip.frag_rows(xf, rows, H)
 
 
 def gu_fused(x, packed, N, rstd, rstd_nt, inv_h, eps, K=None, yfrag=0,

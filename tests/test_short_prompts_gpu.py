@@ -1,0 +1,84 @@
+"""Steps of few tokens take the fused chain whatever they are made of: the same
+logits, keys and values as the general path gives.
+
+Tolerance: both paths round the residual stream and the operands of every
+product to bf16, at other places: some 12 roundings a path and layer, each off
+by 2^-9 / sqrt(3) of a value's size in the mean, sum to sqrt(2 * 2 * 12) times
+that or 2^-7 of the logits' norm; twice that is allowed.  Single values differ
+like normal ones: of 30000 the furthest lies 4.5 times the mean off, 8 are
+allowed.
+"""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(a, b):
+    size = b.square().mean().sqrt()
+    off = (a - b).abs()
+    assert off.square().mean().sqrt() <= 2 ** -6 * size
+    assert off.max() <= 8 * 2 ** -7 * size
+
+
+def _run(model, cfg, fused, steps):
+    """Logits of every step, and the keys and values at the end; a step is a
+    list of (stream, tokens, wanted places)."""
+    from ollamamq_amd.engine import LlamaEngine, PagedKVCache
+    model.fused_chain = fused
+    kv = PagedKVCache.for_model(cfg, n_pages=96, max_slots=6, max_ctx=256,
+                                device="cuda:0", dtype=torch.bfloat16)
+    eng = LlamaEngine(model, kv, max_batch=4)
+    eng.use_graphs = False
+    streams = [eng.open_stream() for _ in range(5)]
+    out = [eng.feed([(streams[i], list(t), list(w)) for i, t, w in step])
+           for step in steps]
+    return out, kv.k_pool.float(), kv.v_pool.float()
+
+
+STEPS = [
+    # one portion, its last place wanted; every place; none
+    [(0, range(1, 38), [36])],
+    [(0, range(9, 41), range(32))],
+    [(1, range(64), [])],
+    # portions and single tokens, unsorted, places repeated and out of order
+    [(2, range(3, 20), [16, 2, 2]), (0, [5], [0]), (3, range(40), [39]),
+     (1, [7], [0])],
+    # one token too many for the chain, and more places than it takes
+    [(4, range(65), [64, 0])],
+    [(4, range(12), [3] * 70)],
+    [(i, [i], [0]) for i in range(5)],
+]
+
+
+@pytest.mark.parametrize("name", ["tiny", "tiny-qwen", "tiny-swa"])
+def test_chain_and_general_path(name):
+    from ollamamq_amd.models import LlamaModel, PRESETS
+    cfg = PRESETS[name]
+    model = LlamaModel(cfg, device="cuda:0", dtype=torch.bfloat16, seed=5)
+    assert model.fused_chain
+    got, k1, v1 = _run(model, cfg, True, STEPS)
+    want, k2, v2 = _run(model, cfg, False, STEPS)
+    for a, b, step in zip(got, want, STEPS):
+        assert a.shape == b.shape == (sum(len(w) for _, _, w in step),
+                                      cfg.vocab)
+        if len(b):
+            _close(a.float(), b.float())
+    # the pools hold zeros where nothing was cached
+    _close(k1[k2 != 0], k2[k2 != 0])
+    _close(v1[v2 != 0], v2[v2 != 0])
+    assert torch.equal(k1 != 0, k2 != 0) and torch.equal(v1 != 0, v2 != 0)
+
+
+@pytest.mark.parametrize("H", [64, 512, 4096])
+def test_rows(H):
+    from ollamamq_amd.ops import hip
+    hip.require()
+    x = torch.randn(64, H, device="cuda").bfloat16()
+    xf, sq = hip.fragify_sumsq(x)
+    for idx in ([0], [63, 0, 31, 32], list(range(64)), [5] * 40, []):
+        rows = torch.tensor(idx, dtype=torch.long, device="cuda")
+        got, n = hip.frag_rows(xf, rows, H)
+        d = got.view(-1, H // 64, 4, 2, 32, 8).permute(0, 4, 1, 2, 3, 5)
+        assert torch.equal(d.reshape(-1, H)[:len(idx)], x[rows])
+        assert torch.equal(n, sq[rows])
