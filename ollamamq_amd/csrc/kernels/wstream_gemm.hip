@@ -1,7 +1,8 @@
-// gfx950 weight-streaming decode GEMM: y[M,N] = x[M,K] @ W[N,K]^T, M <= 64.
+// gfx950 weight-streaming decode GEMM: y[M,N] = x[M,K] @ W[N,K]^T, M <= 64
+// (128 with x in fragment layout).
 //
 // The decode projections are pure weight streaming (each weight byte is
-// used M<=64 times; compute is nothing next to the 8 TB/s HBM pull), and
+// used M times; compute is nothing next to the 8 TB/s HBM pull), and
 // round-1 measured hipBLASLt at 1.8-4.6 TB/s on these shapes with a
 // ~19 us floor on qkv/o (profiles/r01_decode_step_budget.md).  Two
 // hand-written attempts also lost:
@@ -23,7 +24,7 @@
 //
 // Geometry: grid (N/32, ksplit) x 512 threads (8 waves).  The K/64
 // k-blocks are range-partitioned over ksplit*8 waves (uneven ranges OK:
-// any K%64==0, N%32==0, M<=64).  Wave partials meet in a single
+// any K%64==0, N%32==0).  Wave partials meet in a single
 // end-of-kernel LDS reduce (the ONE barrier, after all streaming).
 // ksplit>1 writes fp32 partials; the consumer folds them, or the block that
 // arrives last at a tile (x in fragment layout), or k_wstream_combine (+bias).
@@ -72,7 +73,7 @@ extern "C" int wstream_pure_bf16(void* sink, const void* wp, int N, int K,
     return (int)hipGetLastError();
 }
 
-// MT: m-tiles of 32 rows (1: M<=32, 2: M<=64).
+// MT: m-tiles of 32 rows (up to 64 rows, 128 in fragment layout).
 // DEPTH: weights under way per wave, in 4 KiB iterations.
 // XLDS == 2: x in fragment layout (the decode chain).  A CU's loads are what
 // bounds it, x counted: rows past M repeat row M - 1, so few rows cost few
@@ -88,7 +89,7 @@ extern "C" int wstream_pure_bf16(void* sink, const void* wp, int N, int K,
 // minimum-phase swizzled ds_read (u = r*8 + (c ^ (r&7))).  Wave-private
 // double-buffered tiles -> NO barrier anywhere in the stream (a
 // __syncthreads would drain vmcnt and kill the weight prefetch).
-// GU (requires MT==1, ksplit==1): fused gate_up@SwiGLU.  The weights are
+// GU (requires ksplit==1): fused gate_up@SwiGLU.  The weights are
 // packed with gate and up INTERLEAVED (tile t = 16 gate rows f=t*16..+16
 // then the 16 matching up rows — ops/hip.py pack_weight_gu), so each
 // block's 32-column output tile holds the (gate, up) pairs of 16 ffn
@@ -166,13 +167,13 @@ void k_wstream_gemm(
     // a __syncthreads separates the stream epoch from the reduce epoch)
     extern __shared__ __align__(16) char smem[];
 
-    f32x16 acc0 = {}, acc1 = {};
+    f32x16 acc[MT] = {};
     // rmsnorm scale of the raw-residual input: this row's sq partials from
     // the producing GEMM, FL lanes a row, several loads at a time.  The frag
     // path loads them beside its first weights: behind the stream they cost
     // every block another memory latency (gate-up 46.7 us for 32 rows, 41.6
     // for 1; now 43.8 and 38.9).
-    constexpr int FL = MT == 2 ? 8 : 16;
+    constexpr int FL = MT == 1 ? 16 : MT == 2 ? 8 : 4;
     float rsum = 0.f;
     auto fold = [&]() {
         const int m = tid / FL;
@@ -216,13 +217,11 @@ void k_wstream_gemm(
         };
         auto mul = [&](int s) {
             #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                    xr[s % XS][0][j].v, w[s][j].v, acc0, 0, 0, 0);
-                if (MT == 2)
-                    acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        xr[s % XS][MT - 1][j].v, w[s][j].v, acc1, 0, 0, 0);
-            }
+            for (int j = 0; j < 4; j++)
+                #pragma unroll
+                for (int m = 0; m < MT; m++)
+                    acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        xr[s % XS][m][j].v, w[s][j].v, acc[m], 0, 0, 0);
         };
         int b = b_hi - (b_hi - b_lo + DEPTH - 1) / DEPTH * DEPTH;
         #pragma unroll
@@ -244,6 +243,7 @@ void k_wstream_gemm(
             if (s + XS < DEPTH) ldx(s % XS, max(b + s + XS, b_lo));
         }
     }
+    f32x16 &acc0 = acc[0], &acc1 = acc[MT - 1];     // XLDS < 2: MT <= 2
     if (XLDS != 2 && b_lo < b_hi) {
         const u32x4* wbase = wp + ((int64_t)t * NB * 4) * 64 + lane;
         u4bf8 br[DEPTH][4];
@@ -389,13 +389,13 @@ void k_wstream_gemm(
     }
     if (GU) {
         const int F = N >> 1;                  // ffn width
+        #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            const f32x16& acc = mt ? acc1 : acc0;
             __syncthreads();
             #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int crow = (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
-                red8[wid][crow][lane & 31] = acc[r];
+                red8[wid][crow][lane & 31] = acc[mt][r];
             }
             __syncthreads();
             const int m = tid >> 4, c = tid & 15;  // 512 thr = 32 x 16
@@ -423,13 +423,13 @@ void k_wstream_gemm(
     }
     if (RP) {
         const int qt = rp.nl * 4, kt = rp.nkl * 4;   // tiles per section
+        #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            const f32x16& acc = mt ? acc1 : acc0;
             __syncthreads();
             #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int crow = (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
-                red8[wid][crow][lane & 31] = acc[r];
+                red8[wid][crow][lane & 31] = acc[mt][r];
             }
             __syncthreads();
             if (t < qt + kt) {
@@ -534,15 +534,15 @@ void k_wstream_gemm(
             // 128 B line and ~3 us per consumer block)
             sq_parts[(int64_t)(tid + mt * 32) * gridDim.x + t] = s;
         }
-        if (MT == 2 && mt == 0) __syncthreads();   // sqt reused
+        if (mt + 1 < MT) __syncthreads();          // sqt reused
     };
+    #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-        const f32x16& acc = mt ? acc1 : acc0;
         if (mt) __syncthreads();
         #pragma unroll
         for (int r = 0; r < 16; r++) {
             const int crow = (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
-            red8[wid][crow][lane & 31] = acc[r];
+            red8[wid][crow][lane & 31] = acc[mt][r];
         }
         __syncthreads();
         float rsq[2] = {0.f, 0.f};
@@ -602,6 +602,207 @@ void k_wstream_gemm(
     }
 }
 
+// ---------------------------------------------------------------------------
+// Many columns for 33 to 128 rows in fragment layout: gate-up and logits.  A
+// CU moves some 20 bytes a clock through its vector loads whatever they are,
+// and k_wstream_gemm reads all rows for every 32 columns: three units of 4 KB
+// a step of 64 with 64 rows, five with 128, of which one is weights.  Here a
+// block takes CW tiles of 32 columns and its waves share the activations
+// through LDS, CW + rows / 32 units for CW of weights: 8 / CW groups of CW
+// waves walk parts of K, a step of every group staged at a time, the next one
+// on its way in registers.  The barrier leaves loads in flight.  With norm and
+// activation, K 4096, us for 64 and 128 rows:
+//   16384   36 and 42 (k_wstream_gemm 36 and 50)
+//   28672   47 and 57 (64 and 93; library product, norm and activation 63)
+//  128256  179 and 200 (250 and 362)
+// Products in parts stay with k_wstream_gemm: adding up the parts of several
+// tiles costs one block more than the loads saved (4096 x 14336, 128 rows:
+// 56 us against 49).  More weights or activations under way give nothing.
+// bytes for two stages of activations, or the sums that follow them
+static constexpr __host__ __device__ int wide_lds(int mt, int cw)
+{
+    const int x = 2 * (8 / cw) * mt * 4096, sums = 8 * 32 * 33 * 4;
+    return x > sums ? x : sums;
+}
+
+template <int MT, int CW, int GU>
+__global__ __launch_bounds__(512, 1) void k_wide(
+    bf16* __restrict__ y,            // [M, N], with GU [M, N / 2]
+    const u32x4* __restrict__ x,     // [M, K] in fragment layout
+    const u32x4* __restrict__ wp, int M, int N, int K,
+    const float* __restrict__ rstd_parts, int rstd_nt, float inv_h,
+    float eps, int yfrag)
+{
+    constexpr int KW = 8 / CW, DEPTH = CW == 4 ? 2 : 4;
+    constexpr int STAGE = KW * MT * 256;               // 16-byte units
+    constexpr int NX = (STAGE + 511) / 512;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int cw = wid % CW, kw = wid / CW;
+    const int NB = K >> 6, tiles = N >> 5;
+    auto from = [&](int k) { return (int)((int64_t)k * NB / KW); };
+    const int lo = from(kw), hi = from(kw + 1), steps = (NB + KW - 1) / KW;
+    // tiles past the last repeat it and are not stored
+    const int t0 = blockIdx.x * CW;
+    const u32x4* wq = wp + (int64_t)min(t0 + cw, tiles - 1) * NB * 256 + lane;
+    extern __shared__ __align__(16) char smem[];
+    u32x4* x_s = reinterpret_cast<u32x4*>(smem);       // [2][KW][MT][256]
+    float* rstd_s = reinterpret_cast<float*>(smem + wide_lds(MT, CW));
+
+    u4bf8 w[DEPTH][4];
+    u32x4 xr[NX];
+    f32x16 acc[MT] = {};
+    auto ldw = [&](int s, int b) {
+        #pragma unroll
+        for (int j = 0; j < 4; j++)
+            w[s][j].u = __builtin_nontemporal_load(
+                wq + (int64_t)min(b, max(hi, 1) - 1) * 256 + j * 64);
+    };
+    auto ldx = [&](int r) {
+        #pragma unroll
+        for (int i = 0; i < NX; i++) {
+            const int u = (tid >> 8) + i * 2;          // group and row tile
+            if (u >= KW * MT) break;
+            const int b = min(from(u / MT) + r, NB - 1);
+            xr[i] = x[(int64_t)(u % MT) * K * 4 + (int64_t)b * 256
+                      + (tid & 255)];
+        }
+    };
+    auto stx = [&](int r) {
+        #pragma unroll
+        for (int i = 0; i < NX; i++)
+            if ((tid >> 8) + i * 2 < KW * MT)
+                x_s[(r & 1) * STAGE + i * 512 + tid] = xr[i];
+    };
+    #pragma unroll
+    for (int s = 0; s < DEPTH; s++) ldw(s, lo + s);
+    ldx(0);
+    // the norm's partial sums, FL lanes a row
+    constexpr int FL = MT == 2 ? 8 : 4;
+    float rsum = 0.f;
+    if (rstd_parts && tid / FL < M) {
+        const float* p = rstd_parts + (int64_t)(tid / FL) * rstd_nt;
+        int i = tid % FL;
+        for (; i + 7 * FL < rstd_nt; i += 8 * FL) {
+            float v[8];
+            #pragma unroll
+            for (int k = 0; k < 8; k++) v[k] = p[i + k * FL];
+            #pragma unroll
+            for (int k = 0; k < 8; k++) rsum += v[k];
+        }
+        for (; i < rstd_nt; i += FL) rsum += p[i];
+    }
+    stx(0);
+    ldx(1);
+    lds_barrier();
+    for (int r0 = 0; r0 < steps; r0 += DEPTH) {
+        #pragma unroll
+        for (int s = 0; s < DEPTH; s++) {
+            const int r = r0 + s;
+            if (r >= steps) break;
+            if (r + 1 < steps) stx(r + 1);
+            ldx(r + 2);
+            const u32x4* xb = x_s + (r & 1) * STAGE + kw * MT * 256 + lane;
+            if (lo + r < hi) {
+                #pragma unroll
+                for (int j = 0; j < 4; j++)
+                    #pragma unroll
+                    for (int m = 0; m < MT; m++)
+                        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            __builtin_bit_cast(bf16x8, xb[m * 256 + j * 64]),
+                            w[s][j].v, acc[m], 0, 0, 0);
+            }
+            ldw(s, lo + r + DEPTH);
+            lds_barrier();
+        }
+    }
+    #pragma unroll
+    for (int off = FL / 2; off; off >>= 1) rsum += __shfl_down(rsum, off, 64);
+    if (tid % FL == 0 && tid / FL < MT * 32)
+        rstd_s[tid / FL] = rstd_parts ? rsqrtf(rsum * inv_h + eps) : 1.f;
+
+    // 32 rows at a time: the groups' sums meet in LDS
+    float (*sum)[32][33] = reinterpret_cast<float (*)[32][33]>(smem);
+    #pragma unroll
+    for (int m = 0; m < MT; m++) {
+        __syncthreads();
+        #pragma unroll
+        for (int r = 0; r < 16; r++)
+            sum[wid][(r & 3) + 8 * (r >> 2) + 4 * (lane >> 5)][lane & 31] =
+                acc[m][r];
+        __syncthreads();
+        auto total = [&](int c, int mr, int n) {
+            float s = 0.f;
+            #pragma unroll
+            for (int k = 0; k < KW; k++) s += sum[k * CW + c][mr][n];
+            return s;
+        };
+        constexpr int C = GU ? 16 : 32;                // columns of a tile
+        const int cols = GU ? N / 2 : N;
+        #pragma unroll
+        for (int e = tid; e < CW * 32 * C; e += 512) {
+            const int n = e % C, c = e / C % CW, mr = e / (C * CW);
+            const int row = m * 32 + mr, col = (t0 + c) * C + n;
+            if (row >= M || t0 + c >= tiles) continue;
+            float v = total(c, mr, n) * rstd_s[row];
+            if (GU) {
+                const float up = total(c, mr, n + 16) * rstd_s[row];
+                const float z = GU == 2 ? gelu_arg(v) : v;
+                v = v / (1.f + __expf(-z)) * up;
+            }
+            y[yfrag ? (int64_t)m * 32 * cols + frag_off(mr, col)
+                    : (int64_t)row * cols + col] = __float2bfloat16(v);
+        }
+    }
+}
+
+// Tiles a block: those with which the busiest CU loads least, counted in
+// units of 4 KB a step of K.  k_wstream_gemm (1) has two blocks a CU and reads
+// no rows past M; its loads may be a tenth more, for the steps' barriers
+// (37888 columns: 33 rows 70 us against 80, 45 rows 69 against 59; 16384: 33
+// rows 32 against 36).
+static int wide_tiles(int M, int N)
+{
+    const int tiles = N / 32, mt = (M + 31) / 32;
+    int best = 1;
+    double least = tiles / 256. * (1 + M / 32.) / 1.1;
+    for (int cw = 2; cw <= 8; cw *= 2) {
+        const int blocks = (tiles + cw - 1) / cw;
+        const double units = (blocks + 255) / 256 * (cw + mt);
+        if (units < least) {
+            least = units;
+            best = cw;
+        }
+    }
+    return best;
+}
+
+template <int GU>
+static int wide(int cw, void* y, const void* x, const void* wp, int M, int N,
+                int K, const void* rstd_parts, int rstd_nt, float inv_h,
+                float eps, int yfrag, hipStream_t stream)
+{
+    const int mt = (M + 31) / 32;
+    const int lds = wide_lds(mt, cw) + 512;            // + a scale per row
+    auto go = [&](auto k) {
+        const hipError_t e = hipFuncSetAttribute(
+            (const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return (int)e;
+        k<<<(N / 32 + cw - 1) / cw, 512, lds, stream>>>(
+            (bf16*)y, (const u32x4*)x, (const u32x4*)wp, M, N, K,
+            (const float*)rstd_parts, rstd_nt, inv_h, eps, yfrag);
+        return (int)hipGetLastError();
+    };
+    #define WIDE(MT)                                                       \
+        return cw == 8   ? go(k_wide<MT, 8, GU>)                           \
+               : cw == 4 ? go(k_wide<MT, 4, GU>)                           \
+                         : go(k_wide<MT, 2, GU>)
+    if (mt == 2) WIDE(2);
+    if (mt == 3) WIDE(3);
+    WIDE(4);
+    #undef WIDE
+}
+
 // Iterations ahead for 32 rows in fragment layout: no more than a wave has,
 // as the slots of a first round that it does not have are loaded all the same
 static int frag_depth(int K, int ksplit)
@@ -620,13 +821,21 @@ static int wstream_gu(
     float inv_h, float eps, int yfrag, hipStream_t stream)
 {
     dim3 grid(N / 32, 1);
-    const int lds = (xlds == 1 ? 16 * 4096 : 8 * 32 * 32 * 4) + 256;
+    const int lds = (xlds == 1 ? 16 * 4096 : 8 * 32 * 32 * 4) + 512;
     if (M > 32) {
-        if (xlds == 2) {       // frag chain at batches 33..64
-            k_wstream_gemm<2, 2, 2, GU><<<grid, 512, lds, stream>>>(
+        if (xlds == 2) {       // frag chain at batches 33..128
+            if (M > 128) return -104;
+            const int cw = wide_tiles(M, N);
+            if (cw > 1)
+                return wide<GU>(cw, act, x, wp, M, N, K, rstd_parts, rstd_nt,
+                                inv_h, eps, yfrag, stream);
+            (M <= 64   ? k_wstream_gemm<2, 2, 2, GU>
+             : M <= 96 ? k_wstream_gemm<3, 2, 2, GU>
+                       : k_wstream_gemm<4, 2, 2, GU>)
+                <<<grid, 512, lds, stream>>>(
                 (bf16*)act, nullptr, (const bf16*)x, (const u32x4*)wp,
                 nullptr, M, N, K, xs, 1, (const float*)rstd_parts,
-                rstd_nt, inv_h, eps, nullptr, nullptr, {}, yfrag);
+                rstd_nt, inv_h, eps, nullptr, nullptr, {}, yfrag, nullptr);
             return (int)hipGetLastError();
         }
         // generic-path fused product and activation, direct x loads (unused
@@ -689,8 +898,8 @@ extern "C" int wstream_gemm_bf16(
     dim3 grid(N / 32, ksplit);
     int* sem = ksplit > 1 && y ? (int*)sem_ : nullptr;
     if (sem && (xlds != 2 || ksplit > 8)) return -103;
-    const int lds_red = 8 * 32 * 32 * 4 + 256;     // reduce + rstd tail
-    const int lds_x = 16 * 4096 + 256;             // + 8x2 x tiles
+    const int lds_red = 8 * 32 * 32 * 4 + 512;     // reduce + rstd tail
+    const int lds_x = 16 * 4096 + 512;             // + 8x2 x tiles
     const float* rp = (const float*)rstd_parts;
     const bf16* ri = (const bf16*)res_in;
     float* sq = (float*)sq_parts;
@@ -724,7 +933,15 @@ extern "C" int wstream_gemm_bf16(
                 inv_h, eps, ri, sq, {}, yfrag);
     } else {
         if (xlds == 2) {
-            k_wstream_gemm<2, 2, 2><<<grid, 512, lds_red, stream>>>(
+            if (M > 128) return -104;
+            const int cw = wide_tiles(M, N);
+            if (ksplit == 1 && y && !bias && !ri && !sq && cw > 1)
+                return wide<0>(cw, y, x, wp, M, N, K, rp, rstd_nt, inv_h,
+                               eps, yfrag, stream);
+            (M <= 64   ? k_wstream_gemm<2, 2, 2>
+             : M <= 96 ? k_wstream_gemm<3, 2, 2>
+                       : k_wstream_gemm<4, 2, 2>)
+                <<<grid, 512, lds_red, stream>>>(
                 (bf16*)y, (float*)part, (const bf16*)x, (const u32x4*)wp,
                 (const bf16*)bias, M, N, K, xs, ksplit, rp, rstd_nt,
                 inv_h, eps, ri, sq, {}, yfrag, sem);
@@ -765,16 +982,20 @@ extern "C" int wstream_qkv_rope_bf16(
     int nl, int nkl, int psz, int maxp, int xf, hipStream_t stream)
 {
     dim3 grid(N / 32, 1);
-    const int lds = 8 * 32 * 32 * 4 + 256;
+    const int lds = 8 * 32 * 32 * 4 + 512;
     RopeEpi rp{(const float*)rcos, (const float*)rsin, (const int*)pos,
                (const int*)slot, (const int*)ptab, (bf16*)kp, (bf16*)vp,
                nl, nkl, psz, maxp};
     const int d = frag_depth(K, 1);
+    if (xf && M > 128) return -104;
     if (xf && M > 32)
-        k_wstream_gemm<2, 2, 2, 0, 1><<<grid, 512, lds, stream>>>(
+        (M <= 64   ? k_wstream_gemm<2, 2, 2, 0, 1>
+         : M <= 96 ? k_wstream_gemm<3, 2, 2, 0, 1>
+                   : k_wstream_gemm<4, 2, 2, 0, 1>)
+            <<<grid, 512, lds, stream>>>(
             (bf16*)y, nullptr, (const bf16*)x, (const u32x4*)wp,
             (const bf16*)bias, M, N, K, xs, 1, (const float*)rstd_parts,
-            rstd_nt, inv_h, eps, nullptr, nullptr, rp);
+            rstd_nt, inv_h, eps, nullptr, nullptr, rp, 0, nullptr);
     else if (xf)
         (d == 4   ? k_wstream_gemm<1, 4, 2, 0, 1>
          : d == 2 ? k_wstream_gemm<1, 2, 2, 0, 1>

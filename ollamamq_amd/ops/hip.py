@@ -653,7 +653,7 @@ def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
                   M_frag=32, sem=None):
     """y = x @ W^T via the weight-streaming kernel over pre-packed W.
 
-    Fused-chain extras (decode, M<=64): `rstd`/`rstd_nt`/`inv_h`/`eps`
+    Fused-chain extras (M<=128): `rstd`/`rstd_nt`/`inv_h`/`eps`
     apply rmsnorm scaling of the raw-residual input x (norm weight must
     be folded into the pack); `res` adds the residual stream into the
     output (pass y=res for the in-place residual update) and `sq_out`
