@@ -19,6 +19,7 @@
 #include <hip/hip_bf16.h>
 #include <cstdint>
 #include "act.h"
+#include "tile_mma.h"
 
 typedef __hip_bfloat16 bf16;
 typedef __hip_bfloat162 bf162;
@@ -703,63 +704,60 @@ extern "C" int argmax_f32(void* out, const void* logits, int B, int V,
 }
 
 // ---------------------------------------------------------------------
-// Fused RoPE + paged-KV append: one pass over the fresh q/k/v heads.
+// Fused RoPE + paged-KV append: one pass over the fresh q/k/v heads of 128.
 // q heads: rotate in place.  k heads: rotate, then write BOTH the rotated
 // value in place and into the pool (k read once instead of twice).
 // v heads: copy to the pool.  One launch replaces rope_bf16 + kv_append.
+//
+// Bound by memory: a token's 48 heads (32 and 8) move 26 KB.  A head is 64 / VEC
+// lanes, VEC elements of either half each: with 16-byte loads 2310 tokens
+// take 13.5 us (4.5 TB/s), with 2-byte ones, left for rows that do not lie on
+// 16 bytes, 30.
+template <int VEC>
 __global__ __launch_bounds__(256) void k_rope_append(
     bf16* __restrict__ q, bf16* __restrict__ k, const bf16* __restrict__ v,
     bf16* __restrict__ kp, bf16* __restrict__ vp,
     const int* __restrict__ pos, const int* __restrict__ slot,
     const int* __restrict__ page_table,
     const float* __restrict__ cost, const float* __restrict__ sint,
-    int T, int Hq, int KVH, int D, int page, int max_pages,
+    int T, int Hq, int KVH, int page, int max_pages,
     int64_t qs, int64_t ks, int64_t vs)
 {
-    const int gid = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
+    constexpr int D = 128, L = 64 / VEC;
+    const int gid = blockIdx.x * (256 / L) + threadIdx.x / L;
+    const int d = threadIdx.x % L * VEC;
     const int Htot = Hq + 2 * KVH;
     if (gid >= T * Htot) return;
     const int t = gid / Htot, h = gid % Htot;
-    const int d2 = D / 2;
     const int p = pos[t];
-
-    if (h < Hq) {                        // q head: rope in place
-        bf16* base = q + (int64_t)t * qs + (int64_t)h * D;
-        const float c = cost[(int64_t)p * d2 + lane];
-        const float s = sint[(int64_t)p * d2 + lane];
-        const float x1 = bf2f(base[lane]);
-        const float x2 = bf2f(base[lane + d2]);
-        base[lane] = f2bf(x1 * c - x2 * s);
-        base[lane + d2] = f2bf(x2 * c + x1 * s);
-        return;
+    const bool isq = h < Hq, isv = h >= Hq + KVH;
+    const int kh = isv ? h - Hq - KVH : h - Hq;       // key/value head
+    bf16* base = isq ? q + (int64_t)t * qs + (int64_t)h * D
+                     : isv ? const_cast<bf16*>(v) + (int64_t)t * vs
+                                 + (int64_t)kh * D
+                           : k + (int64_t)t * ks + (int64_t)kh * D;
+    float lo[VEC], hi[VEC];
+    ldv<VEC>(base + d, lo);
+    ldv<VEC>(base + d + D / 2, hi);
+    if (!isv) {
+        float c[VEC], s[VEC];
+        ldv<VEC>(cost + (int64_t)p * (D / 2) + d, c);
+        ldv<VEC>(sint + (int64_t)p * (D / 2) + d, s);
+        #pragma unroll
+        for (int i = 0; i < VEC; i++) {
+            const float x1 = lo[i], x2 = hi[i];
+            lo[i] = x1 * c[i] - x2 * s[i];
+            hi[i] = x2 * c[i] + x1 * s[i];
+        }
+        stv<VEC>(base + d, lo);
+        stv<VEC>(base + d + D / 2, hi);
+        if (isq) return;
     }
     const int pg = page_table[(int64_t)slot[t] * max_pages + p / page];
-    const int off = p % page;
-    if (h < Hq + KVH) {                  // k head: rope + pool write
-        const int kh = h - Hq;
-        bf16* base = k + (int64_t)t * ks + (int64_t)kh * D;
-        bf16* dst = kp + (((int64_t)pg * KVH + kh) * page + off) * D;
-        const float c = cost[(int64_t)p * d2 + lane];
-        const float s = sint[(int64_t)p * d2 + lane];
-        const float x1 = bf2f(base[lane]);
-        const float x2 = bf2f(base[lane + d2]);
-        const bf16 lo = f2bf(x1 * c - x2 * s);
-        const bf16 hi = f2bf(x2 * c + x1 * s);
-        base[lane] = lo;
-        base[lane + d2] = hi;
-        dst[lane] = lo;
-        dst[lane + d2] = hi;
-        return;
-    }
-    {                                    // v head: pool copy
-        const int vh = h - Hq - KVH;
-        const bf162* src = reinterpret_cast<const bf162*>(
-            v + (int64_t)t * vs + (int64_t)vh * D);
-        bf162* dst = reinterpret_cast<bf162*>(
-            vp + (((int64_t)pg * KVH + vh) * page + off) * D);
-        dst[lane] = src[lane];
-    }
+    bf16* dst = (isv ? vp : kp)
+                + (((int64_t)pg * KVH + kh) * page + p % page) * D + d;
+    stv<VEC>(dst, lo);
+    stv<VEC>(dst + D / 2, hi);
 }
 
 extern "C" int rope_append_bf16(
@@ -768,12 +766,19 @@ extern "C" int rope_append_bf16(
     const void* sint, int T, int Hq, int KVH, int D, int page,
     int max_pages, int64_t qs, int64_t ks, int64_t vs, hipStream_t stream)
 {
-    const int waves = T * (Hq + 2 * KVH);
-    k_rope_append<<<(waves + 3) / 4, 256, 0, stream>>>(
+    if (D != 128) return (int)hipErrorInvalidValue;
+    const bool wide = !(((uintptr_t)q | (uintptr_t)k | (uintptr_t)v
+                         | (uintptr_t)kp | (uintptr_t)vp | (uintptr_t)cost
+                         | (uintptr_t)sint) & 15)
+                      && !((qs | ks | vs) & 7);
+    const int64_t heads = (int64_t)T * (Hq + 2 * KVH);
+    const int per = wide ? 32 : 4;                    // heads a block
+    (wide ? k_rope_append<8> : k_rope_append<1>)
+        <<<(heads + per - 1) / per, 256, 0, stream>>>(
         (bf16*)q, (bf16*)k, (const bf16*)v, (bf16*)kp, (bf16*)vp,
         (const int*)pos, (const int*)slot, (const int*)page_table,
         (const float*)cost, (const float*)sint,
-        T, Hq, KVH, D, page, max_pages, qs, ks, vs);
+        T, Hq, KVH, page, max_pages, qs, ks, vs);
     return (int)hipGetLastError();
 }
 
