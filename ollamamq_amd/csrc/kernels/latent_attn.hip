@@ -16,7 +16,7 @@
 // In both a query may see a window of tokens only, itself included, and the
 // result may be gated by the sigmoid of a column of the fused projection.
 // Cached rows are KW wide, R + Dr filled up with zeros.
-#include "tile_mma.h"
+#include "flash32.h"
 
 #define NEG (-3.0e38f)
 
@@ -809,8 +809,7 @@ extern "C" int latent_attn(
 // the lanes already hold P.
 // ---------------------------------------------------------------------------
 template <typename T, int DT, int VT, int NQ>
-__global__ __launch_bounds__(256, sizeof(T) == 2 && DT <= 6 && VT <= 8
-                                      ? 2 : 1) void k_flash(
+__global__ __launch_bounds__(256, 1) void k_flash(
     T* __restrict__ out,               // [T, H, V]
     const T* __restrict__ q,           // [T, ..] row stride qs, head h at
                                        // h * (D + Dr)
@@ -1018,6 +1017,96 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 && DT <= 6 && VT <= 8
     }
 }
 
+// ---------------------------------------------------------------------------
+// The same for bf16 keys of at most 192 and values of at most 128, see
+// flash32.h.  32 heads, 192 / 128 wide, prompts of 1024 and 3072 tokens: 192 us
+// within a model, 370 with k_flash; alone 136 (0.8 PFLOP/s).  Tiles of 128
+// queries leave a CU half its waves, as LDS holds one block: 67 us against 48
+// for 7 prompts, 2310 tokens together, and no gain for one of 37.
+// VEC: whole vectors of queries and keys.
+// ---------------------------------------------------------------------------
+template <int DK, int DV, bool VEC>
+__global__ __launch_bounds__(512, 2) void k_flash32(
+    bf16* __restrict__ out, const bf16* __restrict__ q,
+    const bf16* __restrict__ k, const bf16* __restrict__ kr,
+    const bf16* __restrict__ vt, Rows<bf16> gate, int og,
+    const int* __restrict__ tiles, int H, int D, int Dr, int V, int64_t qs,
+    int64_t krs, int64_t kv_ld, float scale, int window)
+{
+    const int DD = D + Dr;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 31, g = lane >> 5;
+    const int h = blockIdx.x;
+    const int* tl = tiles + (int64_t)(gridDim.y - 1 - blockIdx.y) * 4;
+    const int q0 = tl[0], pos0 = tl[1], rows = tl[2];
+    const int64_t kv0 = tl[3];
+    auto first_seen = [&](int p) {
+        return window > 0 ? max(0, p - window + 1) : 0;
+    };
+    const int w0 = wid * 32, r = min(w0 + col, rows - 1);
+    const int w_lo = pos0 + min(w0, rows - 1);
+    const int w_hi = pos0 + min(w0 + 31, rows - 1);
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    bf16x8 qf[DK / 16];
+    const bf16* qr = q + (int64_t)(q0 + r) * qs + (int64_t)h * DD;
+    #pragma unroll
+    for (int i = 0; i < DK / 16; i++) {
+        const int c = i * 16 + g * 8;
+        if (VEC) qf[i] = c < DD ? frag8(qr + c) : frag_zero<bf16>();
+        else qf[i] = frag_guard(qr, c, DD);
+    }
+    const bf16* kh = k + kv0 * H * D + (int64_t)h * D;
+    const bf16* krh = kr + kv0 * krs - D;
+    const bf16* vh = vt + (int64_t)h * V * kv_ld + kv0;
+    const int kv_len = pos0 + rows;
+    const Seen see{first_seen(pos0 + r), pos0 + r, first_seen(w_lo),
+                   first_seen(w_hi), w_lo, w0 >= rows ? -1 : w_hi};
+    float m = NEG, l = 0.f;
+    f32x16 o[DV / 32] = {};
+    Flash32<DK, DV, 8, true>::walk(
+        reinterpret_cast<bf16*>(smem), qf, first_seen(pos0) / 64,
+        (kv_len + 63) / 64, scale * 1.4426950408889634f,
+        [&](int base, int, int key, int c) {
+            const bf16* src = kh + (int64_t)(base + key) * H * D;
+            const bf16* shared = krh + (base + key) * krs;
+            bf16x8 f;
+            if (VEC)
+                f = c < D ? frag8(src + c)
+                    : c < DD ? frag8(shared + c) : frag_zero<bf16>();
+            else
+                #pragma unroll
+                for (int e = 0; e < 8; e++)
+                    frag_set(f, e, c + e < D ? ldf(src + c + e)
+                             : c + e < DD ? ldf(shared + c + e) : 0.f);
+            return __builtin_bit_cast(u32x4, f);
+        },
+        [&](int base, int, int v, int c) {
+            return v < V ? *reinterpret_cast<const u32x4*>(
+                               vh + (int64_t)v * kv_ld + base + c)
+                         : u32x4{};
+        },
+        see, m, l, o);
+    if (w0 + col >= rows) return;
+    const float inv = 1.f / l;
+    #pragma unroll
+    for (int t = 0; t < DV / 32; t++)
+        #pragma unroll
+        for (int i = 0; i < 16; i += 4) {
+            const int c = t * 32 + 2 * i + 4 * g;
+            f32x4 v{o[t][i], o[t][i + 1], o[t][i + 2], o[t][i + 3]};
+            if (gate.p)
+                #pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    float z;
+                    if (c + e >= V) break;
+                    ldrow<1>(gate, q0 + r, og + h * V + c + e, &z);
+                    v[e] *= sigmoid_of<bf16>(z);
+                }
+            put_out(out, q0 + r, h, c, H, V, v * inv, false);
+        }
+}
+
 template <typename T, int DT, int VT, int NQ>
 static int flash_go(void* out, const void* q, const void* k, const void* kr,
                     const void* vt, const void* gate, int64_t gate_ld,
@@ -1025,29 +1114,41 @@ static int flash_go(void* out, const void* q, const void* k, const void* kr,
                     int Dr, int V, int64_t qs, int64_t krs, int64_t kv_ld,
                     float scale, int window, hipStream_t stream)
 {
-    const int pad = 16 / sizeof(T);
-    const int lds = (64 * (DT * 32 + pad) + VT * 16 * (64 + pad))
-                    * (int)sizeof(T);
-    static bool once = false;
-    if (!once) {
+    auto go = [&](auto kern, int threads, int lds) {
         (void)hipFuncSetAttribute(
-            (const void*)k_flash<T, DT, VT, NQ>,
-            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        once = true;
+            (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+            160 * 1024);
+        kern<<<dim3(H, n_tiles), threads, lds, stream>>>(
+            (T*)out, (const T*)q, (const T*)k, (const T*)kr, (const T*)vt,
+            Rows<T>{(const T*)gate, 1, 0, gate_ld}, og, (const int*)tiles, H,
+            D, Dr, V, qs, krs, kv_ld, scale, window);
+    };
+    if constexpr (sizeof(T) == 2 && DT <= 6 && VT <= 8) {
+        constexpr int DK = DT * 32, DV = VT * 16;
+        constexpr int lds = Flash32<DK, DV, 8, true>::LDS;
+        // whole vectors of queries and keys
+        const bool vec = D % 8 == 0 && Dr % 8 == 0 && qs % 8 == 0
+                         && (!Dr || (krs % 8 == 0 && (uintptr_t)kr % 16 == 0));
+        vec ? go(k_flash32<DK, DV, true>, 512, lds)
+            : go(k_flash32<DK, DV, false>, 512, lds);
+    } else {
+        const int pad = 16 / sizeof(T);
+        go(k_flash<T, DT, VT, NQ>, 256,
+           (64 * (DT * 32 + pad) + VT * 16 * (64 + pad)) * (int)sizeof(T));
     }
-    k_flash<T, DT, VT, NQ><<<dim3(H, n_tiles), 256, lds, stream>>>(
-        (T*)out, (const T*)q, (const T*)k, (const T*)kr, (const T*)vt,
-        Rows<T>{(const T*)gate, 1, 0, gate_ld}, og, (const int*)tiles, H, D,
-        Dr, V, qs, krs, kv_ld, scale, window);
     return (int)hipGetLastError();
 }
 
-// queries per tile; tiles: int32 [n, 4] (first q row, its position, rows, row
+// queries per tile
+extern "C" int flash_rows(int f32, int DD, int V)
+{
+    return f32 ? 64 : DD > 192 || V > 128 ? 128 : 256;
+}
+
+// tiles: int32 [n, 4] (first q row, its position, rows, row
 // of position 0 in k / kr / vt); these hold every sequence from a multiple of
 // 64 positions on, no later than the first key any query sees, padded to
 // another; D + Dr, V <= 256; gate may be null
-extern "C" int flash_rows(int f32) { return f32 ? 64 : 128; }
-
 extern "C" int flash_attn(
     int f32, void* out, const void* q, const void* k, const void* kr,
     const void* vt, const void* gate, int64_t gate_ld, int og,

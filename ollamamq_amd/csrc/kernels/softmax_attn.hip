@@ -12,7 +12,7 @@
 // All heads of a key/value head are rows of one tile: row = token * R + head
 // within the group, R = H / G, so a staged key serves the whole group.
 // Pools are [page][G][page_size][width], widths filled up to multiples of 8.
-#include "tile_mma.h"
+#include "flash32.h"
 
 #define NEG (-3.0e38f)
 
@@ -112,9 +112,8 @@ DEV float finish(float m, float l, const float* sink, int h) {
 // the weights stay in registers as the operand of the value product.
 // Dp <= 32 * DT, Vp <= 16 * VT.
 // ---------------------------------------------------------------------------
-template <typename T, int DT, int VT, int NQ>
-__global__ __launch_bounds__(256, sizeof(T) == 2 && DT <= 4 && VT <= 8
-                                       ? 4 - NQ : 1) void k_softmax_flash(
+template <typename T, int DT, int VT>
+__global__ __launch_bounds__(256) void k_softmax_flash(
     T* __restrict__ out,               // [T, H, V]
     const T* __restrict__ q,           // [T, H, Dp]
     const T* __restrict__ kpool, const T* __restrict__ vpool,
@@ -124,7 +123,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 && DT <= 4 && VT <= 8
     int H, int G, int V, int Dp, int Vp, int pshift, int maxp, Soft rule,
     HeadGate gate)
 {
-    constexpr int KT = 64;
+    constexpr int KT = 64, NQ = 1;
     constexpr int PAD = 16 / sizeof(T);
     constexpr int KS = DT * 32 + PAD, VS = VT * 16 + PAD;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -277,6 +276,78 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 && DT <= 4 && VT <= 8
             put_out(out, tok[n], head[n], v * 16 + g * 4, H, V, o[n][v] * f,
                     false);
     }
+}
+
+// ---------------------------------------------------------------------------
+// The same for bf16 heads of at most 128, see flash32.h.  32 heads of 128, 8 of
+// them key/value heads, prompts of 1024 and 3072 tokens: 135 us within a model,
+// 214 with k_softmax_flash; alone 124 (0.7 PFLOP/s).
+// ---------------------------------------------------------------------------
+// EVEN: heads are DK and DV wide and eight keys are on one page.
+template <int DK, int DV, int NW, bool EVEN>
+__global__ __launch_bounds__(NW * 64, 2) void k_softmax_flash32(
+    bf16* __restrict__ out,            // [T, H, V]
+    const bf16* __restrict__ q,        // [T, H, Dp]
+    const bf16* __restrict__ kpool, const bf16* __restrict__ vpool,
+    const int* __restrict__ ptab, const int* __restrict__ slot,
+    const int* __restrict__ pos,
+    const int* __restrict__ items,     // [n, 2] first row, rows
+    int H, int G, int V, int Dp, int Vp, int pshift, int maxp, Soft rule,
+    HeadGate gate)
+{
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 31, h = lane >> 5;
+    const int kvh = blockIdx.x, R = H / G;
+    const int* it = items + (int64_t)(gridDim.y - 1 - blockIdx.y) * 2;
+    const int row0 = it[0], end = row0 + it[1] - 1;
+    const int kv_len = pos[end / R] + 1;
+    const int* pt = ptab + (int64_t)slot[row0 / R] * maxp;
+    // the wave's rows
+    const int w0 = row0 + wid * 32;
+    const int w_lo = pos[min(w0, end) / R], w_hi = pos[min(w0 + 31, end) / R];
+    const int row = min(w0 + col, end);
+    const int tok = row / R, head = kvh * R + row % R, qpos = pos[tok];
+
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    bf16x8 qf[DK / 16];
+    const bf16* qr = q + ((int64_t)tok * H + head) * Dp;
+    #pragma unroll
+    for (int c = 0; c < DK / 16; c++) {
+        const int d = c * 16 + h * 8;
+        qf[c] = EVEN || d < Dp ? frag8(qr + d) : frag_zero<bf16>();
+    }
+    auto at = [&](const bf16* pool, int width, int base, int w, int k, int c) {
+        const int key = min(base + k, kv_len - 1);
+        const int pg = pt[(EVEN ? min(base + w, kv_len - 1) : key) >> pshift];
+        const int64_t r = (((int64_t)pg * G + kvh) << pshift)
+                          + (key & ((1 << pshift) - 1));
+        return EVEN || c < width
+            ? *reinterpret_cast<const u32x4*>(pool + r * width + c) : u32x4{};
+    };
+    const Seen see{first_seen(rule, qpos), qpos, first_seen(rule, w_lo),
+                   first_seen(rule, w_hi), w_lo, w0 > end ? -1 : w_hi};
+    float m = NEG, l = 0.f;
+    f32x16 o[DV / 32] = {};
+    Flash32<DK, DV, NW, false>::walk(
+        reinterpret_cast<bf16*>(smem), qf,
+        first_seen(rule, pos[row0 / R]) / 64, (kv_len + 63) / 64,
+        rule.scale * Expo<bf16>::unit,
+        [&](int base, int w, int k, int c) {
+            return at(kpool, Dp, base, w, k, c); },
+        [&](int base, int w, int k, int c) {
+            return at(vpool, Vp, base, w, k, c); },
+        see, m, l, o);
+    if (w0 + col > end) return;
+    const float f = finish<bf16>(m, l, rule.sink, head)
+                    * gate_of<bf16>(gate, tok, head);
+    #pragma unroll
+    for (int t = 0; t < DV / 32; t++)
+        #pragma unroll
+        for (int r = 0; r < 16; r += 4)
+            put_out(out, tok, head, t * 32 + 2 * r + 4 * h, H, V,
+                    f32x4{o[t][r], o[t][r + 1], o[t][r + 2], o[t][r + 3]} * f,
+                    false);
 }
 
 // ---------------------------------------------------------------------------
@@ -515,39 +586,47 @@ static int softmax_go(
                 (const int*)pos, (const int*)items, per_seq, T_rows, H, G, V,
                 Dp, Vp, pshift, maxp, split, frag, rule, gate);
     } else {
-        constexpr int NQ = sizeof(T) == 4 || DT == 8 || VT == 16 ? 1 : 2;
-        auto go = item_rows > 64 ? k_softmax_flash<T, DT, VT, NQ>
-                                   : k_softmax_flash<T, DT, VT, 1>;
-        const int lds = 64 * (DT * 32 + VT * 16 + 2 * PAD) * (int)sizeof(T);
-        static bool once = false;
-        if (!once) {
+        auto go = [&](auto kern, int threads, int lds) {
             (void)hipFuncSetAttribute(
-                (const void*)k_softmax_flash<T, DT, VT, NQ>,
+                (const void*)kern,
                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-            (void)hipFuncSetAttribute(
-                (const void*)k_softmax_flash<T, DT, VT, 1>,
-                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-            once = true;
-        }
-        go<<<dim3(G, n_items), 256, lds, stream>>>(
+            kern<<<dim3(G, n_items), threads, lds, stream>>>(
                 (T*)out, (const T*)q, (const T*)kpool, (const T*)vpool,
                 (const int*)ptab, (const int*)slot, (const int*)pos,
                 (const int*)items, H, G, V, Dp, Vp, pshift, maxp, rule,
                 gate);
+        };
+        if constexpr (sizeof(T) == 2 && DT <= 4 && VT <= 8) {
+            constexpr int DK = DT <= 2 ? 64 : 128, DV = VT * 16;
+            constexpr int lds = Flash32<DK, DV, 8, false>::LDS;
+            const bool even = Dp == DK && Vp == DV && pshift >= 3;
+            if (item_rows == 256)
+                even ? go(k_softmax_flash32<DK, DV, 8, true>, 512, lds)
+                     : go(k_softmax_flash32<DK, DV, 8, false>, 512, lds);
+            else
+                even ? go(k_softmax_flash32<DK, DV, 4, true>, 256, lds)
+                     : go(k_softmax_flash32<DK, DV, 4, false>, 256, lds);
+        } else
+            go(k_softmax_flash<T, DT, VT>, 256,
+               64 * (DT * 32 + VT * 16 + 2 * PAD) * (int)sizeof(T));
     }
     return (int)hipGetLastError();
 }
 
-// most rows of an item of the flash kernel; all of one sequence
-extern "C" int softmax_rows(int f32, int Dp, int Vp)
+// rows of an item of the flash kernels, all of one sequence, for T_rows tokens
+// of R heads a key/value head.  256 rows a block stage a chunk once for twice
+// the work of 128 (2 x 2048 tokens, 32 heads: 126 us against 140), but 517 tokens
+// are 72 blocks of them (30 us against 27)
+extern "C" int softmax_rows(int f32, int Dp, int Vp, int T_rows, int R, int G)
 {
-    return f32 || Dp > 128 || Vp > 128 ? 64 : 128;
+    if (f32 || Dp > 128 || Vp > 128) return 64;
+    return ((int64_t)T_rows * R + 255) / 256 * G >= 256 ? 256 : 128;
 }
 // keys a block of the decode kernel takes in one go
 extern "C" int softmax_step(int f32) { return f32 ? 128 : 256; }
 
 // item_rows 16: the decode kernel, items null, every token its own sequence,
-// or int32 [n, 2] (first row, rows); 64 or 128: the flash kernel.  Tokens
+// or int32 [n, 2] (first row, rows); else the flash kernels.  Tokens
 // t0 .. t0 + n_tok - 1 of `out` are written.
 extern "C" int softmax_attn(
     int f32, int item_rows, void* out, void* part, void* ml, const void* q,
@@ -560,8 +639,10 @@ extern "C" int softmax_attn(
 {
     if (psz & (psz - 1) || Dp % 8 || Vp % 8 || Dp > 256 || Vp > 256
         || (frag && (f32 || V % 4))
-        || (item_rows != 16 && item_rows != 64
-            && item_rows != softmax_rows(f32, Dp, Vp)))
+        || (item_rows != 16
+            && (f32 || Dp > 128 || Vp > 128
+                    ? item_rows != 64
+                    : item_rows != 128 && item_rows != 256)))
         return (int)hipErrorInvalidValue;
     const int pshift = __builtin_ctz(psz);
     const int per_seq = (H / G + 15) / 16;

@@ -87,7 +87,7 @@ def _try_load():
                                        i, i, i, i, i, i, i, i, f, vp]
     lib.rope_qkv_append.argtypes = [i, vp, vp, vp, *rows, vp, vp, i, vp, vp,
                                     vp, i, i, i, i, i, i, i, i, i, vp]
-    lib.softmax_rows.argtypes = [i, i, i]
+    lib.softmax_rows.argtypes = [i, i, i, i, i, i]
     lib.softmax_step.argtypes = [i]
     lib.softmax_attn.argtypes = [i, i, vp, vp, vp, vp, vp, vp, vp, vp, vp,
                                  vp, i, i, i, i, i, i, i, i, i, i, i, i, i,
@@ -120,7 +120,7 @@ def _try_load():
                                      vp, vp, vp, i, i, i, i, i, i, vp]
     lib.lightning_scratch.argtypes = [i, i, i, i]
     lib.lightning_scratch.restype = i64
-    lib.flash_rows.argtypes = [i]
+    lib.flash_rows.argtypes = [i, i, i]
     lib.flash_attn.argtypes = [i, vp, vp, vp, vp, vp, vp, i64, i, vp, i, i,
                                i, i, i, i64, i64, i64, f, i, vp]
     lib.gla_step.argtypes = [i, vp, vp, i64, i, i, i, i, i, i, vp, vp, vp,
@@ -1076,7 +1076,7 @@ def _latent_plan(meta, w, KW, f32, dev):
         row += q_lens[i]
         i += 1
     n_absorbed = row
-    QT = _lib.flash_rows(f32)
+    QT = _lib.flash_rows(f32, D + E, V)
     esz = 4 if f32 else 2
     groups = []            # (gather rows, tiles, padded keys) per batch
     gather, tiles, kv0 = [], [], 0
@@ -1084,6 +1084,8 @@ def _latent_plan(meta, w, KW, f32, dev):
     def flush():
         nonlocal gather, tiles, kv0
         if tiles:
+            # the kernels take the last first: the longest walks
+            tiles.sort(key=lambda t: t[1] + t[2])
             groups.append((
                 torch.tensor(gather, dtype=torch.int32).to(dev),
                 torch.tensor(tiles, dtype=torch.int32).to(dev), kv0))
@@ -1731,10 +1733,14 @@ def _tile_plan(meta, R, rows, dev):
         row += q_lens[i]
         i += 1
     n_short = row
-    for n in q_lens[i:]:
+    for n, seen in zip(q_lens[i:], kv_lens[i:]):
         lo, hi = row * R, (row + n) * R
-        long_ += [(r, min(rows, hi - r)) for r in range(lo, hi, rows)]
+        for r in range(lo, hi, rows):
+            end = min(r + rows, hi)
+            long_.append((seen - n + (end - lo) // R, r, end - r))
         row += n
+    # the kernels take the last first: the longest walks
+    long_ = [item[1:] for item in sorted(long_, key=lambda item: item[0])]
     t32 = lambda x: upload(x, dev) if x else None
     plan = (t32(short), n_short, kv, t32(long_))
     setattr(meta, key, plan)
@@ -1867,7 +1873,7 @@ def softmax_attention(q, cache, run, w, slot_ids, positions, meta, frag,
         n_items, n_tok, kv = T * -(-R // 16), T, meta.max_kv
         short = long_ = None
     else:
-        rows = _lib.softmax_rows(f32, Dp, Vp) if T * H >= ATTN_LARGE else 64
+        rows = _lib.softmax_rows(f32, Dp, Vp, T, R, G)
         short, n_tok, kv, long_ = _tile_plan(meta, R, rows, q.device)
         n_items = 0 if short is None else short.shape[0]
 
