@@ -177,12 +177,17 @@ def require():
         )
 
 
+# A step of few tokens is bound by the host: some 25 launches of 10 to 25 us,
+# each with its stream and ten pointers.  Every function's argument types are
+# declared, so plain integers serve as pointers, and the stream's handle needs
+# no stream object (a prompt of 77 tokens, kavedra 8b, 4 layers: 1173 us
+# before, 1078 now).
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _p(t: Optional[torch.Tensor]):
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 # ---------------------------------------------------------------------------
