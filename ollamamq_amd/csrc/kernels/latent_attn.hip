@@ -820,7 +820,7 @@ __global__ __launch_bounds__(256, 1) void k_flash(
     const int* __restrict__ tiles,     // [n, 4] q row, pos, rows, row of
                                        // position 0 in k, kr and vt
     int H, int D, int Dr, int V, int64_t qs, int64_t krs, int64_t kv_ld,
-    float scale, int window)
+    float scale, int window, int frag)
 {
     const int DD = D + Dr;
     constexpr int KT = 64;
@@ -989,7 +989,6 @@ __global__ __launch_bounds__(256, 1) void k_flash(
         const int r = (wid * NQ + n) * 16 + lr;
         if (r >= rows) continue;
         const float inv = 1.f / l[n];
-        T* orow = out + ((int64_t)(q0 + r) * H + h) * V;
         #pragma unroll
         for (int v = 0; v < VT; v++) {
             const int c = v * 16 + g * 4;
@@ -1002,17 +1001,7 @@ __global__ __launch_bounds__(256, 1) void k_flash(
                     o[n][v][i] *= sigmoid_of<T>(z);
                 }
             }
-            if (V % 4 == 0) {
-                if (c < V) {
-                    float w[4];
-                    #pragma unroll
-                    for (int i = 0; i < 4; i++) w[i] = o[n][v][i] * inv;
-                    stv<4>(orow + c, w);
-                }
-            } else
-                #pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (c + i < V) stf(orow + c + i, o[n][v][i] * inv);
+            put_out(out, q0 + r, h, c, H, V, o[n][v] * inv, frag);
         }
     }
 }
@@ -1031,7 +1020,7 @@ __global__ __launch_bounds__(512, 2) void k_flash32(
     const bf16* __restrict__ k, const bf16* __restrict__ kr,
     const bf16* __restrict__ vt, Rows<bf16> gate, int og,
     const int* __restrict__ tiles, int H, int D, int Dr, int V, int64_t qs,
-    int64_t krs, int64_t kv_ld, float scale, int window)
+    int64_t krs, int64_t kv_ld, float scale, int window, int frag)
 {
     const int DD = D + Dr;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1103,7 +1092,7 @@ __global__ __launch_bounds__(512, 2) void k_flash32(
                     ldrow<1>(gate, q0 + r, og + h * V + c + e, &z);
                     v[e] *= sigmoid_of<bf16>(z);
                 }
-            put_out(out, q0 + r, h, c, H, V, v * inv, false);
+            put_out(out, q0 + r, h, c, H, V, v * inv, frag);
         }
 }
 
@@ -1112,7 +1101,7 @@ static int flash_go(void* out, const void* q, const void* k, const void* kr,
                     const void* vt, const void* gate, int64_t gate_ld,
                     int og, const void* tiles, int n_tiles, int H, int D,
                     int Dr, int V, int64_t qs, int64_t krs, int64_t kv_ld,
-                    float scale, int window, hipStream_t stream)
+                    float scale, int window, int frag, hipStream_t stream)
 {
     auto go = [&](auto kern, int threads, int lds) {
         (void)hipFuncSetAttribute(
@@ -1121,7 +1110,7 @@ static int flash_go(void* out, const void* q, const void* k, const void* kr,
         kern<<<dim3(H, n_tiles), threads, lds, stream>>>(
             (T*)out, (const T*)q, (const T*)k, (const T*)kr, (const T*)vt,
             Rows<T>{(const T*)gate, 1, 0, gate_ld}, og, (const int*)tiles, H,
-            D, Dr, V, qs, krs, kv_ld, scale, window);
+            D, Dr, V, qs, krs, kv_ld, scale, window, frag);
     };
     if constexpr (sizeof(T) == 2 && DT <= 6 && VT <= 8) {
         constexpr int DK = DT * 32, DV = VT * 16;
@@ -1148,19 +1137,21 @@ extern "C" int flash_rows(int f32, int DD, int V)
 // tiles: int32 [n, 4] (first q row, its position, rows, row
 // of position 0 in k / kr / vt); these hold every sequence from a multiple of
 // 64 positions on, no later than the first key any query sees, padded to
-// another; D + Dr, V <= 256; gate may be null
+// another; D + Dr, V <= 256; gate may be null; frag: out in the activation-
+// fragment layout
 extern "C" int flash_attn(
     int f32, void* out, const void* q, const void* k, const void* kr,
     const void* vt, const void* gate, int64_t gate_ld, int og,
     const void* tiles, int n_tiles, int H, int D, int Dr, int V, int64_t qs,
-    int64_t krs, int64_t kv_ld, float scale, int window, hipStream_t stream)
+    int64_t krs, int64_t kv_ld, float scale, int window, int frag,
+    hipStream_t stream)
 {
-    if (D + Dr > 256 || V > 256) return (int)hipErrorInvalidValue;
+    if (D + Dr > 256 || V > 256 || (frag && (f32 || V % 4))) return (int)hipErrorInvalidValue;
     int err;
     #define FA(T, D_, V_, Q)                                               \
         err = flash_go<T, D_, V_, Q>(                                      \
             out, q, k, kr, vt, gate, gate_ld, og, tiles, n_tiles, H, D,    \
-            Dr, V, qs, krs, kv_ld, scale, window, stream)
+            Dr, V, qs, krs, kv_ld, scale, window, frag, stream)
     #define FA_V(T, D_, Q)                                                 \
         do {                                                               \
             if (V <= 64) FA(T, D_, 4, Q);                                  \

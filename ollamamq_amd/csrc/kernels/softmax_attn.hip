@@ -120,8 +120,8 @@ __global__ __launch_bounds__(256) void k_softmax_flash(
     const int* __restrict__ ptab, const int* __restrict__ slot,
     const int* __restrict__ pos,
     const int* __restrict__ items,     // [n, 2] first row, rows
-    int H, int G, int V, int Dp, int Vp, int pshift, int maxp, Soft rule,
-    HeadGate gate)
+    int H, int G, int V, int Dp, int Vp, int pshift, int maxp, int frag,
+    Soft rule, HeadGate gate)
 {
     constexpr int KT = 64, NQ = 1;
     constexpr int PAD = 16 / sizeof(T);
@@ -274,7 +274,7 @@ __global__ __launch_bounds__(256) void k_softmax_flash(
         #pragma unroll
         for (int v = 0; v < VT; v++)
             put_out(out, tok[n], head[n], v * 16 + g * 4, H, V, o[n][v] * f,
-                    false);
+                    frag);
     }
 }
 
@@ -292,8 +292,8 @@ __global__ __launch_bounds__(NW * 64, 2) void k_softmax_flash32(
     const int* __restrict__ ptab, const int* __restrict__ slot,
     const int* __restrict__ pos,
     const int* __restrict__ items,     // [n, 2] first row, rows
-    int H, int G, int V, int Dp, int Vp, int pshift, int maxp, Soft rule,
-    HeadGate gate)
+    int H, int G, int V, int Dp, int Vp, int pshift, int maxp, int frag,
+    Soft rule, HeadGate gate)
 {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -347,7 +347,7 @@ __global__ __launch_bounds__(NW * 64, 2) void k_softmax_flash32(
         for (int r = 0; r < 16; r += 4)
             put_out(out, tok, head, t * 32 + 2 * r + 4 * h, H, V,
                     f32x4{o[t][r], o[t][r + 1], o[t][r + 2], o[t][r + 3]} * f,
-                    false);
+                    frag);
 }
 
 // ---------------------------------------------------------------------------
@@ -593,7 +593,7 @@ static int softmax_go(
             kern<<<dim3(G, n_items), threads, lds, stream>>>(
                 (T*)out, (const T*)q, (const T*)kpool, (const T*)vpool,
                 (const int*)ptab, (const int*)slot, (const int*)pos,
-                (const int*)items, H, G, V, Dp, Vp, pshift, maxp, rule,
+                (const int*)items, H, G, V, Dp, Vp, pshift, maxp, frag, rule,
                 gate);
         };
         if constexpr (sizeof(T) == 2 && DT <= 4 && VT <= 8) {

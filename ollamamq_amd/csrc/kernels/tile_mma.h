@@ -124,7 +124,7 @@ DEV int64_t frag_off(int m, int kcol) {
     const int b = kcol >> 6, j = (kcol >> 4) & 3, h = (kcol >> 3) & 1;
     return ((((int64_t)b * 4 + j) * 64) + h * 32 + m) * 8 + (kcol & 7);
 }
-// row r of a batch of up to 64: two halves of 32 rows, `cols` wide
+// row r of a batch: 32 rows after 32 rows, `cols` wide
 DEV int64_t frag_row_off(int r, int c, int cols) {
     return (int64_t)(r >> 5) * 32 * cols + frag_off(r & 31, c);
 }

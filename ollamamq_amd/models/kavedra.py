@@ -330,6 +330,7 @@ class KavedraModel(HybridModel):
         self.head_norm = self.final_norm * cfg.logit_scale
         self.head = put(get("head", (cfg.vocab, W))).contiguous()
         self._pack_weights()
+        self.whole_heads = all(s.vdim % 8 == 0 for s in cfg.layers)
 
     def matrices(self):
         return {} if self.loop_in is None else {"loop_in": self.loop_in}
@@ -368,8 +369,11 @@ class KavedraModel(HybridModel):
         selects.  layer_out collects the residual stream after every layer
         run."""
         meta = attn_meta
-        frag = (self.frag_decode and meta.one_each
-                and tokens.shape[0] <= 64)
+        idx = meta.logits_idx
+        # few tokens, portions of prompts too: activations in fragment layout
+        frag = (self.frag_decode and 0 < tokens.shape[0] <= ops.CHAIN_ROWS
+                and (idx is None or 0 < idx.shape[0] <= ops.CHAIN_ROWS)
+                and (meta.one_each or self.whole_heads))
 
         def join(x, y, pre, **kw):
             return ops.rms_residual(x, y, None, pre, 1.0, self.cfg.eps,
@@ -398,7 +402,7 @@ class KavedraModel(HybridModel):
                 layer_out.append(join(x, y, None, frag=False)[0])
         frag = frag and not return_hidden and self.head_pk is not None
         _, h = join(x, y, self.final_norm if return_hidden
-                    else self.head_norm, rows=meta.logits_idx, need_x=False,
+                    else self.head_norm, rows=idx, need_x=False,
                     frag=frag)
         if return_hidden:
             return h

@@ -144,10 +144,6 @@ PRESETS = {
 }
 
 
-# steps of at most so many tokens take the fused chain
-CHAIN_ROWS = 128
-
-
 def _randn(shape, dev, dtype, gen, scale):
     # generate on the generator's own device (CPU gen => bit-identical
     # weights across CPU/GPU test runs; CUDA gen => fast 16 GB init for the
@@ -353,17 +349,17 @@ class LlamaModel:
                     for l in self.layers))
         if self.fused_chain:
             th = self.cfg.hidden // 32
-            self._sq_a = torch.zeros(max(th, 1) * CHAIN_ROWS, dtype=torch.float32,
+            rows = ops.CHAIN_ROWS
+            self._sq_a = torch.zeros(max(th, 1) * rows, dtype=torch.float32,
                                      device=self.device)
             self._sq_b = torch.zeros_like(self._sq_a)
             # tickets of products and attention in parts, zero between them
-            self._tickets = torch.zeros(max(th, CHAIN_ROWS
-                                            * self.n_local_kv_heads),
+            self._tickets = torch.zeros(max(th, rows * self.n_local_kv_heads),
                                         dtype=torch.int32,
                                         device=self.device)
             # frag-layout residual stream, 32 rows after 32 rows; those past
             # the batch hold garbage that only dead accumulator rows ever see
-            self._res_frag = torch.zeros(CHAIN_ROWS * self.cfg.hidden,
+            self._res_frag = torch.zeros(rows * self.cfg.hidden,
                                          dtype=self.dtype,
                                          device=self.device)
 
@@ -402,8 +398,9 @@ class LlamaModel:
         selects as "last" (decode: all; prefill: final token per seq)."""
         cfg = self.cfg
         idx = attn_meta.logits_idx
-        if (self.fused_chain and 0 < tokens.shape[0] <= CHAIN_ROWS
-                and (idx is None or idx.shape[0] <= CHAIN_ROWS)
+        if (self.fused_chain and 0 < tokens.shape[0] <= ops.CHAIN_ROWS
+                and (attn_meta.one_each or idx is None
+                     or 0 < idx.shape[0] <= ops.CHAIN_ROWS)
                 and not return_hidden):
             return self._forward_fused(tokens, positions, kv_cache,
                                        slot_ids, attn_meta)
@@ -456,8 +453,8 @@ class LlamaModel:
     def _forward_fused(self, tokens, positions, kv_cache, slot_ids,
                        attn_meta):
         """A step of few tokens, decode or short portions of prompts, as a
-        fused weight-streaming chain (tp=1, up to CHAIN_ROWS rows): 4 GEMM-class
-        kernels per layer, zero rmsnorm/swiglu kernels.
+        fused weight-streaming chain (tp=1, up to ops.CHAIN_ROWS rows): 4
+        GEMM-class kernels per layer, zero rmsnorm/swiglu kernels.
         rmsnorm weights are folded into the packs; the rstd scale rides
         each consumer GEMM's epilogue from sum-of-squares partials the
         producer GEMM emitted; residual adds happen in place inside the

@@ -122,7 +122,7 @@ def _try_load():
     lib.lightning_scratch.restype = i64
     lib.flash_rows.argtypes = [i, i, i]
     lib.flash_attn.argtypes = [i, vp, vp, vp, vp, vp, vp, i64, i, vp, i, i,
-                               i, i, i, i64, i64, i64, f, i, vp]
+                               i, i, i, i64, i64, i64, f, i, i, vp]
     lib.gla_step.argtypes = [i, vp, vp, i64, i, i, i, i, i, i, vp, vp, vp,
                              vp, vp, vp, vp, i, i, i, i, f, f, f, i, vp]
     lib.gla_chunks.argtypes = [i, vp, vp, vp, vp, i64, i, i, i, i, i, i,
@@ -1153,7 +1153,6 @@ def latent_attention(q, cache, run, w, slot_ids, positions, meta,
     if KW > LATENT_MAX_R and (max(DD, V) > FLASH_MAX or meta.n_single):
         raise ValueError(f"latent attention with rank {R}, head widths "
                          f"{DD}/{V}: no kernel")
-    assert not frag or meta.one_each
     if frag:
         res = _frag_rows(T, H * V, q)
         out = res.buf
@@ -1182,8 +1181,6 @@ def latent_attention(q, cache, run, w, slot_ids, positions, meta,
                              kv_abs)
         head_gemm(o.view(n_abs, H, R), w.uv, out if frag else out[:n_abs],
                   frag, gate=gate)
-        if frag:
-            return res
     g, og = (None, 0) if gate is None else gate
     if groups and isinstance(g, Partials):
         g, og = g.parts[:, :, og:og + H * V].sum(0).to(q.dtype), 0
@@ -1202,8 +1199,8 @@ def latent_attention(q, cache, run, w, slot_ids, positions, meta,
             f32, _p(out), _p(q), _p(k), _p(c[:, R:] if E else None), _p(vt),
             _p(g), 0 if g is None else g.stride(0), og, _p(tiles),
             tiles.shape[0], H, D, E, V, q.stride(0), KW, kv, float(w.scale),
-            w.window, _stream()), "flash_attn")
-    return out.view(T, H * V)
+            w.window, int(frag), _stream()), "flash_attn")
+    return res if frag else out.view(T, H * V)
 
 
 def latent_rope_append(p, cache, run, w, norm, eps, rope, slot_ids,
@@ -1313,7 +1310,6 @@ def lightning(p, w, state, slot_ids, positions, meta, frag=False):
         and w.powers.shape == (H, LIGHTNING_CHUNK + 1) \
         and w.powers.is_contiguous() \
         and max(oq + H * D, ok + H * D, ov + H * V, og + H * V) <= t.shape[-1]
-    assert not frag or meta.one_each
     o = torch.empty((T, H * V), dtype=torch.float32, device=t.device)
     slots, pos = _i32(slot_ids), _i32(positions)
     head = (*rows, oq, ok, ov, int(w.act), _p(w.powers), _p(state),
@@ -1868,7 +1864,6 @@ def softmax_attention(q, cache, run, w, slot_ids, positions, meta, frag,
         and (w.sink is None or w.sink.numel() == H)
     gp, og = (None, 0) if gate is None else gate
     assert gp is None or og + H <= _cols(gp)
-    assert not frag or meta.one_each
     if frag:
         res = _frag_rows(T, H * V, q)
         out = res.buf

@@ -108,9 +108,13 @@ class Weighted(NamedTuple):
     share: torch.Tensor
 
 
+# rows that the products over activations in fragment layout take
+CHAIN_ROWS = 128
+
+
 class FragRows(NamedTuple):
     """A bf16 activation [rows, cols] in the layout in which the
-    weight-streaming product reads it (GPU decode, up to 64 rows)."""
+    weight-streaming product reads it (GPU, up to CHAIN_ROWS rows)."""
     buf: torch.Tensor
     rows: int
     cols: int

@@ -127,8 +127,18 @@ def test_expanded(D, E, V, window, scale):
         1, (H, V))
     tl = torch.tensor(tiles, dtype=torch.int32, device="cuda")
     p = hip._p
-    hip._check(hip._lib.flash_attn(
-        0, p(out), p(q), p(k), p(kr if E else None), p(vt), p(gate),
-        gate.stride(0), 8, p(tl), len(tiles), H, D, E, V, q.stride(0),
-        kr.stride(0), n_kv, scale, window, hip._stream()), "flash_attn")
+    def launch(frag):
+        hip._check(hip._lib.flash_attn(
+            0, p(out), p(q), p(k), p(kr if E else None), p(vt), p(gate),
+            gate.stride(0), 8, p(tl), len(tiles), H, D, E, V, q.stride(0),
+            kr.stride(0), n_kv, scale, window, frag, hip._stream()),
+            "flash_attn")
+
+    launch(0)
     assert _rel(out, want) < CLOSE
+    if H * V % 64 == 0:
+        plain, T = out, out.shape[0]
+        out = torch.zeros(-(-T // 32) * 32, H * V, device="cuda").bfloat16()
+        launch(1)
+        out = out.view(-1, H * V // 64, 4, 2, 32, 8).permute(0, 4, 1, 2, 3, 5)
+        assert torch.equal(out.reshape(-1, H, V)[:T], plain)

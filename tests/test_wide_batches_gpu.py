@@ -160,3 +160,26 @@ def test_chain_and_general_path(name):
     _close(k1[k2 != 0], k2[k2 != 0])
     _close(v1[v2 != 0], v2[v2 != 0])
     assert torch.equal(k1 != 0, k2 != 0) and torch.equal(v1 != 0, v2 != 0)
+
+
+@pytest.mark.parametrize("T", [1, 5, 128, 129])
+def test_no_logits_wanted(T):
+    """A portion none of whose logits are wanted is refused on either path."""
+    from ollamamq_amd.engine import PagedKVCache
+    from ollamamq_amd.models import LlamaModel, PRESETS
+    from ollamamq_amd.ops.interface import AttnMeta
+    cfg = PRESETS["tiny"]
+    model = LlamaModel(cfg, device="cuda:0", dtype=torch.bfloat16, seed=5)
+    kv = PagedKVCache.for_model(cfg, n_pages=16, max_slots=1, max_ctx=256,
+                                device="cuda:0", dtype=torch.bfloat16)
+    slot = kv.alloc_slot()
+    kv.ensure(slot, T)
+    i32 = dict(dtype=torch.int32, device="cuda:0")
+    meta = AttnMeta(
+        mode="prefill", slot_ids=torch.tensor([slot], **i32),
+        seq_lens=torch.tensor([T], **i32), cu_q=torch.tensor([0, T], **i32),
+        logits_idx=torch.empty(0, dtype=torch.long, device="cuda:0"),
+        max_q=T, max_kv=T)
+    with pytest.raises(RuntimeError, match="launch failed"):
+        model.forward(torch.arange(T, **i32), torch.arange(T, **i32), kv,
+                      torch.full((T,), slot, **i32), meta)
