@@ -969,24 +969,46 @@ extern "C" int sample_gumbel_bf16(
 // the 32-row MFMA fragment layout the fused decode chain streams
 // (wstream_gemm.hip frag_off) AND emit sq[m] = sum(x[m]^2) — one read of
 // the embedding output seeds the whole chain.  With tokens, x is the
-// embedding table and its rows are gathered on the way.
+// embedding table and its rows are gathered on the way; with rows, x and what
+// is added to it are [T, H] and these of their sums are taken, the wanted rows
+// of a step whose logits leave the general path (gather, sum and norm as
+// launches of their own: 20 us).
 // ---------------------------------------------------------------------------
+// a row by its index, from the end where that is negative; others do not exist
+DEV int64_t row_at(const int64_t* rows, int m, int T) {
+    const int64_t r = rows[m];
+    return max((int64_t)0, min(r < 0 ? r + T : r, (int64_t)T - 1));
+}
+
 __global__ __launch_bounds__(256) void k_fragify_sumsq(
     const bf16* __restrict__ x, const int* __restrict__ tokens,
+    const int64_t* __restrict__ rows, const bf16* __restrict__ add, int T,
     bf16* __restrict__ xf, float* __restrict__ sq, int H)
 {
     const int m = blockIdx.x;
-    const bf16* row = x + (int64_t)(tokens ? tokens[m] : m) * H;
-    // rows 32-63 land in the second 32-row frag half (MT2 chain)
+    const int64_t at = rows ? row_at(rows, m, T) : tokens ? tokens[m] : m;
+    const bf16* row = x + at * H;
+    // rows land 32 after 32
     bf16* xfh = xf + (int64_t)(m >> 5) * 32 * H;
     const int mr = m & 31;
     float s = 0.f;
     // 16-byte chunk c covers k = c*8..c*8+8: frag unit
     // ((c>>3)*4 + ((c>>1)&3))*64 + (c&1)*32 + mr
     for (int c = threadIdx.x; c < H / 8; c += 256) {
-        const uint4 v = *reinterpret_cast<const uint4*>(row + c * 8);
+        uint4 v = *reinterpret_cast<const uint4*>(row + c * 8);
         float f[8];
         load8f(row + c * 8, f);
+        if (add) {
+            float g[8];
+            load8f(add + at * H + c * 8, g);
+            bf16 t[8];
+            #pragma unroll
+            for (int e = 0; e < 8; e++) {
+                t[e] = f2bf(f[e] + g[e]);
+                f[e] = bf2f(t[e]);
+            }
+            __builtin_memcpy(&v, t, 16);
+        }
         #pragma unroll
         for (int e = 0; e < 8; e++) s += f[e] * f[e];
         const int64_t u = ((int64_t)(c >> 3) * 4 + ((c >> 1) & 3)) * 64
@@ -1004,10 +1026,10 @@ __global__ __launch_bounds__(256) void k_fragify_sumsq(
 // Selected rows of an activation in fragment layout, in that layout, and
 // their sums of squares
 __global__ __launch_bounds__(256) void k_frag_rows(
-    const uint4* __restrict__ x, const int64_t* __restrict__ rows,
+    const uint4* __restrict__ x, const int64_t* __restrict__ rows, int T,
     uint4* __restrict__ xf, float* __restrict__ sq, int H)
 {
-    const int m = blockIdx.x, from = (int)rows[m];
+    const int m = blockIdx.x, from = (int)row_at(rows, m, T);
     const uint4* src = x + (int64_t)(from >> 5) * 4 * H + (from & 31);
     uint4* dst = xf + (int64_t)(m >> 5) * 4 * H + (m & 31);
     float s = 0.f;
@@ -1028,19 +1050,21 @@ __global__ __launch_bounds__(256) void k_frag_rows(
 }
 
 extern "C" int frag_rows_bf16(void* xf, void* sq, const void* x,
-                              const void* rows, int M, int H,
+                              const void* rows, int T, int M, int H,
                               hipStream_t stream)
 {
     k_frag_rows<<<M, 256, 0, stream>>>((const uint4*)x, (const int64_t*)rows,
-                                       (uint4*)xf, (float*)sq, H);
+                                       T, (uint4*)xf, (float*)sq, H);
     return (int)hipGetLastError();
 }
 
 extern "C" int fragify_sumsq_bf16(void* xf, void* sq, const void* x,
-                                  const void* tokens, int M, int H,
+                                  const void* tokens, const void* rows,
+                                  const void* add, int T, int M, int H,
                                   hipStream_t stream)
 {
     k_fragify_sumsq<<<M, 256, 0, stream>>>(
-        (const bf16*)x, (const int*)tokens, (bf16*)xf, (float*)sq, H);
+        (const bf16*)x, (const int*)tokens, (const int64_t*)rows,
+        (const bf16*)add, T, (bf16*)xf, (float*)sq, H);
     return (int)hipGetLastError();
 }

@@ -400,7 +400,11 @@ class KavedraModel(HybridModel):
                                      layer.packs.get("w_down"))
             if layer_out is not None:
                 layer_out.append(join(x, y, None, frag=False)[0])
-        frag = frag and not return_hidden and self.head_pk is not None
+        # the logits of few rows, of whatever step
+        frag = (self.frag_decode and not return_hidden
+                and self.head_pk is not None
+                and 0 < (tokens if idx is None else idx).shape[0]
+                <= ops.CHAIN_ROWS)
         _, h = join(x, y, self.final_norm if return_hidden
                     else self.head_norm, rows=idx, need_x=False,
                     frag=frag)

@@ -62,8 +62,8 @@ def _try_load():
     lib.wstream_gu_bf16.argtypes = [vp, vp, vp, i, i, i, i64, i,
                                     vp, i, f, f, i, i, vp]
     lib.row_sumsq_bf16.argtypes = [vp, vp, i, i, vp]
-    lib.frag_rows_bf16.argtypes = [vp, vp, vp, vp, i, i, vp]
-    lib.fragify_sumsq_bf16.argtypes = [vp, vp, vp, vp, i, i, vp]
+    lib.frag_rows_bf16.argtypes = [vp, vp, vp, vp, i, i, i, vp]
+    lib.fragify_sumsq_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i, i, i, vp]
     lib.sample_gumbel_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i, i,
                                        vp, vp, i, *[vp] * 6]
     lib.wstream_qkv_rope_bf16.argtypes = [vp, vp, vp, vp, i, i, i, i64,
@@ -705,34 +705,41 @@ def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
     return y
 
 
-def fragify_sumsq(x, xf=None, sq=None, tokens=None):
+def fragify_sumsq(x, xf=None, sq=None, tokens=None, rows=None, add=None):
     """Standard [M, H] -> 32-row frag layout + per-row sum of squares
     (seeds the fused decode chain); with tokens, of their rows of the
-    embedding table x."""
-    M, H = x.shape
+    embedding table x; with rows, of these rows of x + add."""
+    T, H = x.shape
+    M = T
     if tokens is not None:
         M, tokens = tokens.shape[0], _i32(tokens)
         assert tokens.is_contiguous()
+    if rows is not None:
+        M, rows = rows.shape[0], rows.long().contiguous()
+    assert add is None or (add.shape == x.shape and add.dtype == x.dtype
+                           and add.is_contiguous() and tokens is None)
     assert x.is_contiguous() and H % 8 == 0
     if xf is None:
         xf = torch.empty(((M + 31) // 32) * 32 * H, dtype=x.dtype,
                          device=x.device)
     if sq is None:
         sq = torch.empty(M, dtype=torch.float32, device=x.device)
-    _check(_lib.fragify_sumsq_bf16(_p(xf), _p(sq), _p(x), _p(tokens), M, H,
-                                   _stream()), "fragify_sumsq")
+    _check(_lib.fragify_sumsq_bf16(_p(xf), _p(sq), _p(x), _p(tokens),
+                                   _p(rows), _p(add), T, M, H, _stream()),
+           "fragify_sumsq")
     return xf, sq
 
 
-def frag_rows(xf, rows, H):
-    """Rows (int64) of an activation in fragment layout, in that layout, and
-    their sums of squares."""
-    M = rows.shape[0]
-    assert rows.dtype == torch.int64 and rows.is_contiguous() and H % 64 == 0
+def frag_rows(xf, rows, H, T=None):
+    """Rows (int64) of an activation of T rows in fragment layout, in that
+    layout, and their sums of squares."""
+    M, rows = rows.shape[0], rows.long().contiguous()
+    T = xf.numel() // H if T is None else T
+    assert H % 64 == 0
     out = torch.empty(-(-M // 32) * 32 * H, dtype=xf.dtype, device=xf.device)
     sq = torch.empty(M, dtype=torch.float32, device=xf.device)
     if M:
-        _check(_lib.frag_rows_bf16(_p(out), _p(sq), _p(xf), _p(rows), M, H,
+        _check(_lib.frag_rows_bf16(_p(out), _p(sq), _p(xf), _p(rows), T, M, H,
                                    _stream()), "frag_rows")
     return out, sq
 

@@ -746,11 +746,12 @@ def linear_fused(x, packed, N, bias=None, rstd=None, rstd_nt=0,
                              K=K, xlds=xlds, M_frag=M_frag, sem=sem)
 
 
-def fragify_sumsq(x, xf=None, sq=None, tokens=None):
+def fragify_sumsq(x, xf=None, sq=None, tokens=None, rows=None, add=None):
     """Standard [M, H] -> 32-row frag layout + per-row sum of squares; with
-    tokens, of their rows of the embedding table x."""
+    tokens, of their rows of the embedding table x; with rows, of these rows
+    of x + add."""
     from . import hip
-    return hip.fragify_sumsq(x, xf, sq, tokens)
+    return hip.fragify_sumsq(x, xf, sq, tokens, rows, add)
 
 
 def attention_frag(q, cache, layer, meta, sem=None):
@@ -762,11 +763,11 @@ def attention_frag(q, cache, layer, meta, sem=None):
     return hip.attention_mixed(q, cache, layer, meta, True, sem)
 
 
-def frag_rows(xf, rows, H):
-    """Rows of an activation in frag layout, in that layout, and their sums
-    of squares."""
+def frag_rows(xf, rows, H, T=None):
+    """Rows of an activation of T rows in frag layout, in that layout, and
+    their sums of squares."""
     from . import hip
-    return hip.frag_rows(xf, rows, H)
+    return hip.frag_rows(xf, rows, H, T)
 
 
 def gu_fused(x, packed, N, rstd, rstd_nt, inv_h, eps, K=None, yfrag=0,

@@ -109,5 +109,7 @@ def test_heads_of_odd_width():
     assert model.frag_decode and not model.whole_heads
     got = _run(model, cfg, True, STEPS[:2])
     want = _run(model, cfg, False, STEPS[:2])
+    # the same but for the logits' product, whose fp32 sums round to the same
+    # bf16 number or a neighbour, at most 2^-7 away
     for a, b in zip(got[0], want[0]):
-        assert torch.equal(a, b)
+        torch.testing.assert_close(a, b, rtol=2 ** -7, atol=1e-4)

@@ -183,3 +183,22 @@ def test_no_logits_wanted(T):
     with pytest.raises(RuntimeError, match="launch failed"):
         model.forward(torch.arange(T, **i32), torch.arange(T, **i32), kv,
                       torch.full((T,), slot, **i32), meta)
+
+
+@pytest.mark.parametrize("T,H", [(1, 64), (200, 512), (130, 4096)])
+def test_rows_of_a_sum(T, H):
+    """Rows by their indexes, from the end where these are negative."""
+    hip = _hip()
+    x, y = torch.randn(2, T, H, device="cuda").bfloat16()
+    for idx in ([0], [-1, 0, T - 1, -T], [T - 1] * 40, list(range(T))):
+        rows = torch.tensor(idx, device="cuda")
+        want = x[rows] + y[rows]
+        for form in (rows, rows.int(), rows.repeat_interleave(2)[::2]):
+            xf, sq = hip.fragify_sumsq(x, rows=form, add=y)
+            assert torch.equal(_defrag(xf, len(idx), H), want)
+            torch.testing.assert_close(
+                sq.double(), want.double().square().sum(1), rtol=1e-5,
+                atol=0)
+        if T <= 128:
+            got, _ = hip.frag_rows(_frag(x), rows, H, T)
+            assert torch.equal(_defrag(got, len(idx), H), x[rows])
