@@ -253,17 +253,25 @@ __global__ __launch_bounds__(NW * 64, 2) void k_decode_attn(
         top = NEG;
         den = 0.f;
         sum = f32x4{};
-        #pragma unroll 4
-        for (int i = 0; i < parts; i++) {
-            const float2 ml = get2(ml_part + (at + i) * 2);
-            const float2 a = get2(o_part + (at + i) * D + c);
-            const float2 b = get2(o_part + (at + i) * D + c + 2);
-            const float mn = fmaxf(top, ml.x);
-            const float f = __builtin_amdgcn_exp2f(top - mn);
-            const float w = __builtin_amdgcn_exp2f(ml.x - mn);
-            top = mn;
-            den = den * f + ml.y * w;
-            sum = sum * f + f32x4{a.x, a.y, b.x, b.y} * w;
+        for (int i = 0; i < parts; i += 8) {
+            float2 ml[8], a[8], b[8];     // all under way together
+            #pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int64_t p = at + min(i + j, parts - 1);
+                ml[j] = get2(ml_part + p * 2);
+                a[j] = get2(o_part + p * D + c);
+                b[j] = get2(o_part + p * D + c + 2);
+            }
+            #pragma unroll
+            for (int j = 0; j < 8; j++) {
+                if (i + j >= parts) break;
+                const float mn = fmaxf(top, ml[j].x);
+                const float f = __builtin_amdgcn_exp2f(top - mn);
+                const float w = __builtin_amdgcn_exp2f(ml[j].x - mn);
+                top = mn;
+                den = den * f + ml[j].y * w;
+                sum = sum * f + f32x4{a[j].x, a[j].y, b[j].x, b[j].y} * w;
+            }
         }
     }
     if (!live) return;

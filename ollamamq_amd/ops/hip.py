@@ -323,16 +323,18 @@ def _attention(q, cache, layer, meta, qt):
 def _decode_split(pairs, max_kv):
     """Parts of a context, for `pairs` (sequence, key/value head) pairs.  From
     192 pairs on the chip has a block a CU and one part is best (32 users of
-    about 512 tokens, 8 key/value heads: 18.2 us against 20.9 with two);
-    below, up to 768 blocks help where contexts are long or
-    ragged (12 users of 4096 to 12288: 149 us whole, 91 in two, 80 in
-    eight).  A part has at least a step of 32 keys for each of its eight
-    waves."""
+    about 512 tokens, 8 key/value heads: 18.2 us against 20.9 with two).  Up to
+    64, a block a CU in all: more parts are more to add up (4 users of 10000
+    tokens: 40 us in 8, 47 in 24; 8 of 2000: 18 in 4, 25 in 12).  Between
+    them up to 768 blocks even out ragged contexts (12 users of 4096 to 12288:
+    149 us whole, 91 in two, 80 in eight).  A part has at least a step of 32
+    keys for each of its eight waves."""
     env = os.environ.get("OLLAMAMQ_DECODE_SPLIT")
     if env:                       # tuning override (tools/perf_decode.py)
         want = int(env)
     else:
-        want = 1 if pairs >= 192 else 768 // max(1, pairs)
+        want = 1 if pairs >= 192 else (
+            min(256 // max(1, pairs), 24) if pairs <= 64 else 768 // pairs)
     return min(want, max(1, (max_kv + 255) // 256), 32)
 
 
