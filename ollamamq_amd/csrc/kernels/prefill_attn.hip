@@ -9,23 +9,23 @@
 //   2 x 2048                      335 us (205 TF), now 86 (800)
 //   7 prompts, 2310 together       66 us (106 TF), now 23 (300)
 //   2048, 32 / 32 heads          1777 us, now 66
-#include "flash32.h"
+#include "decode_attn.h"
 
 constexpr int D = 128;
 
 struct Item { int slot, tok0, pos0, row0, rows; };
 
 template <bool SH, int NW>
-__global__ __launch_bounds__(NW * 64, 2) void k_prefill_attn(
+DEV void prefill_block(
+    char* smem, int kvh, const Item it,
     bf16* __restrict__ out,               // [T, Hq, D], or its fragments
     const bf16* __restrict__ q,           // [T, Hq, D], rows qs apart
     const bf16* __restrict__ kpool,       // [P][KVH][page][D]
     const bf16* __restrict__ vpool, const int* __restrict__ page_table,
-    const Item* __restrict__ items, int G, int KVH, int page, int pshift,
-    int max_pages, float unit, int64_t qs, int window, int fragout)
+    int G, int KVH, int page, int pshift, int max_pages, float unit,
+    int64_t qs, int window, int fragout)
 {
-    const int kvh = blockIdx.x, Hq = G * KVH;
-    const Item it = items[blockIdx.y];
+    const int Hq = G * KVH;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, h = lane >> 5;
@@ -43,7 +43,6 @@ __global__ __launch_bounds__(NW * 64, 2) void k_prefill_attn(
     const int tok = it.tok0 + row / G, head = kvh * G + row % G;
     const int qpos = it.pos0 + row / G;
 
-    extern __shared__ __attribute__((aligned(16))) char smem[];
     bf16x8 qf[8];
     const bf16* qr = q + tok * qs + head * D + h * 8;
     #pragma unroll
@@ -81,6 +80,49 @@ __global__ __launch_bounds__(NW * 64, 2) void k_prefill_attn(
             put_out(out, tok, head, t * 32 + 2 * r + 4 * h, Hq, D,
                     f32x4{o[t][r], o[t][r + 1], o[t][r + 2], o[t][r + 3]}
                         * f, fragout);
+}
+
+template <bool SH, int NW>
+__global__ __launch_bounds__(NW * 64, 2) void k_prefill_attn(
+    bf16* __restrict__ out, const bf16* __restrict__ q,
+    const bf16* __restrict__ kpool, const bf16* __restrict__ vpool,
+    const int* __restrict__ page_table, const Item* __restrict__ items, int G,
+    int KVH, int page, int pshift, int max_pages, float unit, int64_t qs,
+    int window, int fragout)
+{
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    prefill_block<SH, NW>(smem, blockIdx.x, items[blockIdx.y], out, q, kpool,
+                          vpool, page_table, G, KVH, page, pshift, max_pages,
+                          unit, qs, window, fragout);
+}
+
+// Both kinds of a mixed batch in one launch: neither fills the chip where a
+// prompt joins a few users, and each is a latency of its own (24 users of 400
+// to 1200 tokens and a prompt of 517 within a step: 24 and 19 us one after the
+// other, 30 together).  Blocks of prompts come first, the longest walks; registers
+// leave one block of eight waves a CU, as decode alone has.
+template <bool SH>
+__global__ __launch_bounds__(512, 2) void k_mixed_attn(
+    bf16* __restrict__ out, float* __restrict__ o_part,
+    float* __restrict__ ml_part, int* __restrict__ sem,
+    const bf16* __restrict__ q, const bf16* __restrict__ kpool,
+    const bf16* __restrict__ vpool, const int* __restrict__ page_table,
+    const Item* __restrict__ items, int n_items,
+    const int* __restrict__ slot_ids, const int* __restrict__ seq_lens,
+    int split, int G, int KVH, int page, int pshift, int max_pages, float unit,
+    int64_t qs, int window, int fragout)
+{
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int b = blockIdx.y - n_items;
+    if (b < 0)
+        prefill_block<SH, 8>(smem, blockIdx.x, items[blockIdx.y], out, q,
+                             kpool, vpool, page_table, G, KVH, page, pshift,
+                             max_pages, unit, qs, window, fragout);
+    else
+        decode_block<SH>(reinterpret_cast<float*>(smem), blockIdx.x, b / split,
+                         b % split, split, out, o_part, ml_part, sem, q,
+                         kpool, vpool, page_table, slot_ids, seq_lens, G, KVH,
+                         page, pshift, max_pages, unit, qs, window, fragout);
 }
 
 // items: int32 [n, 5]: slot, flat index and position of the portion's first
@@ -124,5 +166,36 @@ extern "C" int prefill_attn_bf16(
     if (sh) PF_W(true); else PF_W(false);
     #undef PF_W
     #undef PF
+    return (int)hipGetLastError();
+}
+
+// S single tokens, rows 0 .. S - 1, and items of 256 rows; part and sem as for
+// decode_attn_bf16
+extern "C" int mixed_attn_bf16(
+    void* out, void* part, void* sem, const void* q, const void* kpool,
+    const void* vpool, const void* page_table, const void* items, int n_items,
+    const void* slot_ids, const void* seq_lens, int S, int split, int Hq,
+    int KVH, int page, int max_pages, float scale, int64_t q_stride,
+    int window, int fragout, hipStream_t stream)
+{
+    const int G = Hq / KVH;
+    if (G < 1 || G > 8 || G * KVH != Hq || page < 1 || S < 1 || n_items < 1
+        || (reinterpret_cast<uintptr_t>(q) & 15) || q_stride % 8
+        || split < 1 || (split > 1 && (!part || !sem)))
+        return (int)hipErrorInvalidValue;
+    const bool sh = page >= 16 && !(page & (page - 1));
+    constexpr int flash = Flash32<D, D, 8, false>::LDS;
+    const int lds = flash > DECODE_LDS ? flash : DECODE_LDS;
+    auto go = sh ? k_mixed_attn<true> : k_mixed_attn<false>;
+    const hipError_t ok = hipFuncSetAttribute(
+        (const void*)go, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (ok != hipSuccess) return (int)ok;
+    go<<<dim3(KVH, n_items + S * split), 512, lds, stream>>>(
+        (bf16*)out, (float*)part, (float*)part + (int64_t)S * Hq * split * D,
+        (int*)sem, (const bf16*)q, (const bf16*)kpool, (const bf16*)vpool,
+        (const int*)page_table, (const Item*)items, n_items,
+        (const int*)slot_ids, (const int*)seq_lens, split, G, KVH, page,
+        sh ? __builtin_ctz(page) : 0, max_pages,
+        scale * 1.4426950408889634f, q_stride, window, fragout);
     return (int)hipGetLastError();
 }

@@ -55,6 +55,8 @@ def _try_load():
                                      i, i, i, i, i, i, i64, i64, i64, vp]
     lib.prefill_attn_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i, i, i, i, i,
                                       i, f, i64, i, i, vp]
+    lib.mixed_attn_bf16.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, i, vp, vp,
+                                    i, i, i, i, i, i, f, i64, i, i, vp]
     lib.embed_gather_bf16.argtypes = [vp, vp, vp, i, i, vp]
     lib.wstream_gemm_bf16.argtypes = [vp, vp, vp, vp, vp, i, i, i, i64, i,
                                       i, i, vp, i, f, f, vp, vp, i, vp, vp]
@@ -338,6 +340,19 @@ def _decode_split(pairs, max_kv):
     return min(want, max(1, (max_kv + 255) // 256), 32)
 
 
+def _decode_parts(S, Hq, kvh, meta, sem, dev):
+    """(parts of a context, scratch for them, tickets, slots, lengths)"""
+    split = _decode_split(S * kvh, meta.max_kv)
+    part = None
+    if split > 1:
+        part = torch.empty(S * Hq * split * 130, dtype=torch.float32,
+                           device=dev)
+        if sem is None:
+            sem = torch.zeros(S * kvh, dtype=torch.int32, device=dev)
+        assert sem.numel() >= S * kvh
+    return split, part, sem, _i32(meta.slot_ids), _i32(meta.seq_lens)
+
+
 def attention_decode(q, cache, layer, meta, fragout=False, out=None,
                      sem=None):
     """Attention of one query token per sequence over its paged keys and
@@ -359,18 +374,8 @@ def attention_decode(q, cache, layer, meta, fragout=False, out=None,
         q = q.clone(memory_format=torch.contiguous_format)
     kp, vp = _layer_ptrs(cache, layer)
     kvh = cache.n_kv_heads
-    split = _decode_split(S * kvh, meta.max_kv)
-    part = None
-    if split > 1:
-        part = torch.empty(S * Hq * split * (D + 2), dtype=torch.float32,
-                           device=q.device)
-        if sem is None:
-            sem = torch.zeros(S * kvh, dtype=torch.int32, device=q.device)
-        assert sem.numel() >= S * kvh
-    slot32 = meta.slot_ids.int() if meta.slot_ids.dtype != torch.int32 \
-        else meta.slot_ids
-    len32 = meta.seq_lens.int() if meta.seq_lens.dtype != torch.int32 \
-        else meta.seq_lens
+    split, part, sem, slot32, len32 = _decode_parts(S, Hq, kvh, meta, sem,
+                                                    q.device)
     _check(_lib.decode_attn_bf16(
         _p(out), _p(part), _p(sem), _p(q), kp, vp, _p(cache.page_table),
         _p(slot32), _p(len32), S, Hq, kvh, cache.page_size,
@@ -390,7 +395,7 @@ def upload(values, dev):
 def _prefill_plan(meta, first, G, KVH, dev):
     """(tiles, waves a block) of the sequences from `first` on, the longest
     walks first; cached on the meta object (one build per forward, shared by
-    every layer)."""
+    every layer).  Beside single tokens blocks are as large as theirs."""
     plan = getattr(meta, "_prefill", None)
     if plan is not None:
         return plan
@@ -400,7 +405,7 @@ def _prefill_plan(meta, first, G, KVH, dev):
     # whole CUs: best from two blocks a CU on (2 x 2048 tokens, 8 key/value
     # heads: 86 us against 90; 7 prompts, 2310 together: 26 against 23)
     blocks = KVH * sum(-(-n * G // 256) for _, n, _ in parts)
-    waves = 8 if blocks >= 512 else 4
+    waves = 8 if first or blocks >= 512 else 4
     items, tok, rows = [], first, 32 * waves
     for slot, n, kv in parts:
         for row in range(0, n * G, rows):
@@ -430,12 +435,16 @@ def _prefill_rows(out, q, cache, layer, meta, first, fragout=False):
 
 
 def attention_mixed(q, cache, layer, meta, fragout=False, sem=None):
-    """Mixed batch: decode kernel over the first n_decode rows, MFMA
-    prefill kernel over the remaining chunk rows — both write into one
-    output tensor.  fragout, sem: see attention_decode."""
+    """Mixed batch: the first n_decode rows are single tokens, the others
+    portions of prompts.  One launch for both while the prompts are less than
+    two blocks a CU (32 heads, 8 of them key/value heads; 24 users of 800
+    tokens and a prompt of 517: 27 us against 38 one after the other, 48 of 700
+    and 2048: 77 against 96); more fill the chip by themselves, and single
+    tokens at their end then only leave it emptier (4 of 8000 and 7000: 508
+    against 499).  fragout, sem: see attention_decode."""
     T, Hq, D = q.shape
     assert D == 128
-    nd = meta.n_single
+    nd, kvh = meta.n_single, cache.n_kv_heads
     out = torch.empty((-(-T // 32) * 32 * Hq * D,) if fragout
                       else (T, Hq, D), dtype=q.dtype, device=q.device)
     sub = getattr(meta, "_mixed_dec", None)
@@ -446,9 +455,24 @@ def attention_mixed(q, cache, layer, meta, fragout=False, sem=None):
             cu_q=meta.cu_q[:nd + 1], logits_idx=None, max_q=1,
             max_kv=meta.max_kv, window=meta.window)
         meta._mixed_dec = sub
-    if nd:
+    items, _ = _prefill_plan(meta, nd, Hq // kvh, kvh, q.device)
+    if not nd:
+        _prefill_rows(out, q, cache, layer, meta, 0, fragout)
+    elif items is None or items.shape[0] * kvh >= 512:
         attention_decode(q[:nd], cache, layer, sub, fragout, out, sem)
-    _prefill_rows(out, q, cache, layer, meta, nd, fragout)
+        _prefill_rows(out, q, cache, layer, meta, nd, fragout)
+    else:
+        if q.data_ptr() % 16 or _row_stride(q, D) % 8:
+            q = q.clone(memory_format=torch.contiguous_format)
+        kp, vp = _layer_ptrs(cache, layer)
+        split, part, sem, slots, lens = _decode_parts(nd, Hq, kvh, sub, sem,
+                                                      q.device)
+        _check(_lib.mixed_attn_bf16(
+            _p(out), _p(part), _p(sem), _p(q), kp, vp, _p(cache.page_table),
+            _p(items), items.shape[0], _p(slots), _p(lens), nd, split, Hq,
+            kvh, cache.page_size, cache.page_table.shape[1], D ** -0.5,
+            _row_stride(q, D), meta.window, int(fragout), _stream()),
+            "mixed_attn")
     return out
 
 

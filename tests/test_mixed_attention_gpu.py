@@ -1,0 +1,85 @@
+"""Single tokens and portions of prompts in one launch: as each kind alone.
+
+A single token's sum is the same numbers in the same order.  A prompt's row may
+keep an older maximum where it shares a block with other rows: weights and
+results are rounded to bf16 as before, each 2^-9, four roundings of the two
+together.
+"""
+import pytest
+import torch
+
+from ollamamq_amd.engine import PagedKVCache
+from ollamamq_amd.ops.interface import AttnMeta
+
+pytestmark = pytest.mark.gpu
+D = 128
+
+
+def _meta(slots, q_lens, kv_lens, nd, window):
+    i32 = dict(dtype=torch.int32, device="cuda")
+    cu = [0]
+    for n in q_lens:
+        cu.append(cu[-1] + n)
+    return AttnMeta(
+        mode="mixed" if nd < len(slots) else "decode",
+        slot_ids=torch.tensor(slots, **i32),
+        seq_lens=torch.tensor(kv_lens, **i32), cu_q=torch.tensor(cu, **i32),
+        logits_idx=None, max_q=max(q_lens), max_kv=max(kv_lens),
+        n_decode=nd, window=window)
+
+
+@pytest.mark.parametrize("Hq,KVH,page", [
+    (32, 8, 16), (28, 4, 16), (8, 8, 32), (5, 1, 16), (8, 2, 5), (4, 4, 8)])
+@pytest.mark.parametrize("window", [0, 70])
+@pytest.mark.parametrize("singles,prompts", [
+    ([300], [(37, 37)]),
+    ([1, 16, 33, 500, 1100], [(2, 90), (130, 130), (65, 400)]),
+    ([20] * 60, [(300, 300)]),
+    ([1900, 5], [(2, 2)]),
+    # prompts of 512 blocks and more go by themselves
+    ([40, 900], [(2048, 2048), (2047, 2048)])])
+def test_as_each_alone(Hq, KVH, page, window, singles, prompts):
+    from ollamamq_amd.ops import hip
+    hip.require()
+    torch.manual_seed(6)
+    q_lens = [1] * len(singles) + [n for n, _ in prompts]
+    kv_lens = singles + [kv for _, kv in prompts]
+    cache = PagedKVCache(2, KVH, D, page_size=page,
+                         n_pages=sum(n // page + 1 for n in kv_lens),
+                         max_slots=len(kv_lens), max_ctx=2064, device="cuda",
+                         dtype=torch.bfloat16)
+    slots = [cache.alloc_slot() for _ in kv_lens]
+    for s, n in zip(slots, kv_lens):
+        cache.ensure(s, n)
+    cache.k_pool.normal_()
+    cache.v_pool.normal_()
+    T, nd = sum(q_lens), len(singles)
+    qkv = torch.randn(T, (Hq + 2 * KVH) * D, device="cuda").bfloat16()
+    q = qkv[:, :Hq * D].view(T, Hq, D)
+    sem = torch.zeros(len(kv_lens) * KVH, dtype=torch.int32, device="cuda")
+    alone = hip.attention_decode(
+        q[:nd], cache, 1, _meta(slots[:nd], q_lens[:nd], kv_lens[:nd], nd,
+                                window))
+    rest = hip.attention_mixed(q[nd:], cache, 1, _meta(
+        slots[nd:], q_lens[nd:], kv_lens[nd:], 0, window))
+    for _ in range(3):
+        got = hip.attention_mixed(q, cache, 1, _meta(
+            slots, q_lens, kv_lens, nd, window), sem=sem)
+        assert not sem.any()
+        close = dict(rtol=0, atol=0) if hip._decode_split(
+            nd * KVH, max(kv_lens)) == hip._decode_split(
+            nd * KVH, max(singles)) else dict(rtol=2 ** -7, atol=1e-4)
+        torch.testing.assert_close(got[:nd], alone, **close)
+        torch.testing.assert_close(got[nd:], rest, rtol=2 ** -7, atol=2e-3)
+    frag = hip.attention_mixed(q, cache, 1, _meta(
+        slots, q_lens, kv_lens, nd, window), True, sem)
+    if Hq * D % 64 == 0:
+        frag = frag.view(-1, Hq * D // 64, 4, 2, 32, 8) \
+            .permute(0, 4, 1, 2, 3, 5).reshape(-1, Hq, D)
+        assert torch.equal(frag[:T], got)
+    # rows that do not lie on 16 bytes
+    odd = torch.empty(T * Hq * D + 1, dtype=q.dtype, device="cuda")[1:]
+    odd = odd.view(T, Hq, D).copy_(q)
+    again = hip.attention_mixed(odd, cache, 1, _meta(
+        slots, q_lens, kv_lens, nd, window))
+    assert torch.equal(again, got)
