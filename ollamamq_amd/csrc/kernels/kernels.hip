@@ -972,7 +972,7 @@ extern "C" int sample_gumbel_bf16(
 // embedding table and its rows are gathered on the way; with rows, x and what
 // is added to it are [T, H] and these of their sums are taken, the wanted rows
 // of a step whose logits leave the general path (gather, sum and norm as
-// launches of their own: 20 us).
+// launches of their own: 20 us).  clear: ints that the chain needs as zeros.
 // ---------------------------------------------------------------------------
 // a row by its index, from the end where that is negative; others do not exist
 DEV int64_t row_at(const int64_t* rows, int m, int T) {
@@ -983,9 +983,12 @@ DEV int64_t row_at(const int64_t* rows, int m, int T) {
 __global__ __launch_bounds__(256) void k_fragify_sumsq(
     const bf16* __restrict__ x, const int* __restrict__ tokens,
     const int64_t* __restrict__ rows, const bf16* __restrict__ add, int T,
-    bf16* __restrict__ xf, float* __restrict__ sq, int H)
+    bf16* __restrict__ xf, float* __restrict__ sq, int H,
+    int* __restrict__ clear, int n_clear)
 {
     const int m = blockIdx.x;
+    for (int i = m * 256 + threadIdx.x; i < n_clear; i += gridDim.x * 256)
+        clear[i] = 0;
     const int64_t at = rows ? row_at(rows, m, T) : tokens ? tokens[m] : m;
     const bf16* row = x + at * H;
     // rows land 32 after 32
@@ -1061,10 +1064,11 @@ extern "C" int frag_rows_bf16(void* xf, void* sq, const void* x,
 extern "C" int fragify_sumsq_bf16(void* xf, void* sq, const void* x,
                                   const void* tokens, const void* rows,
                                   const void* add, int T, int M, int H,
+                                  void* clear, int n_clear,
                                   hipStream_t stream)
 {
     k_fragify_sumsq<<<M, 256, 0, stream>>>(
         (const bf16*)x, (const int*)tokens, (const int64_t*)rows,
-        (const bf16*)add, T, (bf16*)xf, (float*)sq, H);
+        (const bf16*)add, T, (bf16*)xf, (float*)sq, H, (int*)clear, n_clear);
     return (int)hipGetLastError();
 }

@@ -347,21 +347,6 @@ class LlamaModel:
             and all(l.wqkv_pk is not None and l.wo_pk is not None
                     and l.wgu_pk is not None and l.wdown_pk is not None
                     for l in self.layers))
-        if self.fused_chain:
-            th = self.cfg.hidden // 32
-            rows = ops.CHAIN_ROWS
-            self._sq_a = torch.zeros(max(th, 1) * rows, dtype=torch.float32,
-                                     device=self.device)
-            self._sq_b = torch.zeros_like(self._sq_a)
-            # tickets of products and attention in parts, zero between them
-            self._tickets = torch.zeros(max(th, rows * self.n_local_kv_heads),
-                                        dtype=torch.int32,
-                                        device=self.device)
-            # frag-layout residual stream, 32 rows after 32 rows; those past
-            # the batch hold garbage that only dead accumulator rows ever see
-            self._res_frag = torch.zeros(rows * self.cfg.hidden,
-                                         dtype=self.dtype,
-                                         device=self.device)
 
     # -- helpers -----------------------------------------------------------
     def _allreduce(self, x: torch.Tensor) -> torch.Tensor:
@@ -472,17 +457,26 @@ class LlamaModel:
         B = tokens.shape[0]
         H = cfg.hidden
         nl, nkl, d = self.n_local_heads, self.n_local_kv_heads, cfg.head_dim
-        sq_a, sq_b = self._sq_a, self._sq_b
+        # Scratch of this call alone: sums of squares, tickets of products and
+        # attention in parts (zero between them) and the residual stream, 32
+        # rows after 32 rows; those past the batch hold garbage that only dead
+        # accumulator rows ever see
+        tiles_h = H // 32
+        dev = self.embed.device
+        rows = -(-B // 32) * 32          # the products write these of sq
+        sq_a, sq_b = torch.empty((2, rows * tiles_h), dtype=torch.float32,
+                                 device=dev)
+        tickets = torch.empty(max(tiles_h, B * nkl), dtype=torch.int32,
+                              device=dev)
         # res lives in the 32-row frag layout for the WHOLE chain: every
         # consumer GEMM streams its activation input linearly exactly
         # like packed weights (the scattered x machinery measured 15-30%
         # on top of the pure stream rate — profiles/r02_gemm_sweep.md)
-        res = ops.fragify_sumsq(self.embed, self._res_frag, sq_a[:B],
-                                tokens)[0]
+        res = ops.fragify_sumsq(self.embed, sq=sq_a[:B], tokens=tokens,
+                                clear=tickets)[0]
         nt = 1                      # embed stats = one partial tile
         inv_h = 1.0 / H
         eps = cfg.norm_eps
-        tiles_h = H // 32
         for li, layer in enumerate(self.layers):
             # fused rmsnorm -> qkv -> RoPE -> paged KV append: q comes
             # back rotated in standard layout, k/v land in the pool
@@ -494,10 +488,10 @@ class LlamaModel:
                 K=H, M_real=B)
             q = qkv[:, :nl * d].view(-1, nl, d)
             attn = ops.attention_frag(q, kv_cache, li, attn_meta,
-                                      self._tickets)
+                                      tickets)
             ops.linear_fused(attn, layer.wo_pk, H, res=res, sq_out=sq_b,
                              y=res, yfrag=1, K=nl * d, xlds=2, M_frag=B,
-                             sem=self._tickets)
+                             sem=tickets)
             act = ops.gu_fused(res, layer.wgu_pk,
                                layer.wgate_up.shape[0], rstd=sq_b,
                                rstd_nt=tiles_h, inv_h=inv_h, eps=eps,
@@ -505,7 +499,7 @@ class LlamaModel:
             ops.linear_fused(act, layer.wdown_pk, H, res=res,
                              sq_out=sq_a, y=res, yfrag=1,
                              K=layer.wdown.shape[1], xlds=2, M_frag=B,
-                             sem=self._tickets)
+                             sem=tickets)
             nt = tiles_h
         idx = attn_meta.logits_idx
         if not attn_meta.one_each and idx is not None:

@@ -65,7 +65,8 @@ def _try_load():
                                     vp, i, f, f, i, i, vp]
     lib.row_sumsq_bf16.argtypes = [vp, vp, i, i, vp]
     lib.frag_rows_bf16.argtypes = [vp, vp, vp, vp, i, i, i, vp]
-    lib.fragify_sumsq_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i, i, i, vp]
+    lib.fragify_sumsq_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i, i, i, vp, i,
+                                       vp]
     lib.sample_gumbel_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i, i,
                                        vp, vp, i, *[vp] * 6]
     lib.wstream_qkv_rope_bf16.argtypes = [vp, vp, vp, vp, i, i, i, i64,
@@ -731,10 +732,12 @@ def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
     return y
 
 
-def fragify_sumsq(x, xf=None, sq=None, tokens=None, rows=None, add=None):
+def fragify_sumsq(x, xf=None, sq=None, tokens=None, rows=None, add=None,
+                  clear=None):
     """Standard [M, H] -> 32-row frag layout + per-row sum of squares
     (seeds the fused decode chain); with tokens, of their rows of the
-    embedding table x; with rows, of these rows of x + add."""
+    embedding table x; with rows, of these rows of x + add.  clear: int32
+    scratch to set to zero on the way."""
     T, H = x.shape
     M = T
     if tokens is not None:
@@ -751,8 +754,9 @@ def fragify_sumsq(x, xf=None, sq=None, tokens=None, rows=None, add=None):
     if sq is None:
         sq = torch.empty(M, dtype=torch.float32, device=x.device)
     _check(_lib.fragify_sumsq_bf16(_p(xf), _p(sq), _p(x), _p(tokens),
-                                   _p(rows), _p(add), T, M, H, _stream()),
-           "fragify_sumsq")
+                                   _p(rows), _p(add), T, M, H, _p(clear),
+                                   0 if clear is None else clear.numel(),
+                                   _stream()), "fragify_sumsq")
     return xf, sq
 
 
