@@ -451,8 +451,7 @@ class LlamaModel:
         rmsnorm weights are folded into the packs; the rstd scale rides
         each consumer GEMM's epilogue from sum-of-squares partials the
         producer GEMM emitted; residual adds happen in place inside the
-        o/down epilogues (SURVEY.md §2 kernel-table GEMM rows — this is
-        the MFMA-native decode path)."""
+        o/down epilogues."""
         cfg = self.cfg
         B = tokens.shape[0]
         H = cfg.hidden
