@@ -53,7 +53,7 @@ constexpr int DECODE_LDS = 8 * 8 * (128 + 2) * 4;
 
 template <bool SH>
 DEV void decode_block(
-    float* s, int kvh, int seq, int z, int split,
+    float* s, int kvh, int seq, int z, int split, int least,
     bf16* __restrict__ out,               // [S, Hq, D] (split == 1)
     float* __restrict__ o_part,           // [S, Hq, split, D]
     float* __restrict__ ml_part,          // [S, Hq, split, 2] maximum, sum
@@ -76,9 +76,9 @@ DEV void decode_block(
     // first key that the query, at kv_len - 1, sees
     const int lo = window > 0 ? max(0, kv_len - window) : 0;
     const int first = lo / KT, steps = (kv_len + KT - 1) / KT - first;
-    // parts in use: every wave has a step (300 tokens of one user: 7.3 us in
-    // one part, 8.2 in two)
-    const int parts = max(1, min(split, steps / NW));
+    // parts in use: each has `least` steps, at least one a wave (300 tokens of
+    // one user: 7.3 us in one part, 8.2 in two)
+    const int parts = max(1, min(split, steps / least));
     if (z >= parts) return;
     const int GW = parts * NW;            // a wave's steps: every GW-th
 

@@ -39,7 +39,7 @@ template <int DK, int DV, int NW, bool VT> struct Flash32 {
     static constexpr int NK = DK / 8 / NW, NV = DV / 8 / NW;
 
     // lane (col, h) <- values col of keys k0 + 4h .. and k0 + 8 + 4h ..
-    static DEV bf16x8 values(const bf16* v_s, int k0, int v0, int lane) {
+    DEV bf16x8 values(const bf16* v_s, int k0, int v0, int lane) {
         const int h = lane >> 5;
         if constexpr (VT) {
             const bf16* p = v_s + (v0 + (lane & 31)) * VS + k0 + 4 * h;
@@ -62,7 +62,7 @@ template <int DK, int DV, int NW, bool VT> struct Flash32 {
     // keys, for transposed values columns); unit: of a score, in octaves.  m:
     // the row's maximum, at most 8 octaves old; l: this lane's sum of weights.
     template <class K, class V>
-    static DEV void walk(bf16* lds, bf16x8* qf, int c_lo, int c_hi,
+    DEV void walk(bf16* lds, bf16x8* qf, int c_lo, int c_hi,
                          float unit, K kat, V vat, const Seen& see, float& m,
                          float& l, f32x16* o)
     {

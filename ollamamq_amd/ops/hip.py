@@ -48,7 +48,7 @@ def _try_load():
     lib.argmax_bf16.argtypes = [vp, vp, i, i, vp, vp, i, *[vp] * 6]
     lib.argmax_f32.argtypes = lib.argmax_bf16.argtypes
     lib.decode_attn_bf16.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp,
-                                     i, i, i, i, i, f, i64, i, i, i, vp]
+                                     i, i, i, i, i, f, i64, i, i, i, i, vp]
     lib.skinny_gemm_bf16.argtypes = [vp, vp, vp, vp, i, i, i, i64, i, vp]
     lib.skinny_direct_bf16.argtypes = [vp, vp, vp, vp, i, i, i, i64, i, vp]
     lib.rope_append_bf16.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp, vp,
@@ -56,7 +56,7 @@ def _try_load():
     lib.prefill_attn_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i, i, i, i, i,
                                       i, f, i64, i, i, vp]
     lib.mixed_attn_bf16.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, i, vp, vp,
-                                    i, i, i, i, i, i, f, i64, i, i, vp]
+                                    i, i, i, i, i, i, i, f, i64, i, i, vp]
     lib.embed_gather_bf16.argtypes = [vp, vp, vp, i, i, vp]
     lib.wstream_gemm_bf16.argtypes = [vp, vp, vp, vp, vp, i, i, i, i64, i,
                                       i, i, vp, i, f, f, vp, vp, i, vp, vp]
@@ -324,25 +324,34 @@ def _attention(q, cache, layer, meta, qt):
 
 
 def _decode_split(pairs, max_kv):
-    """Parts of a context, for `pairs` (sequence, key/value head) pairs.  From
-    192 pairs on the chip has a block a CU and one part is best (32 users of
-    about 512 tokens, 8 key/value heads: 18.2 us against 20.9 with two).  Up to
-    64, a block a CU in all: more parts are more to add up (4 users of 10000
-    tokens: 40 us in 8, 47 in 24; 8 of 2000: 18 in 4, 25 in 12).  Between
-    them up to 768 blocks even out ragged contexts (12 users of 4096 to 12288:
-    149 us whole, 91 in two, 80 in eight).  A part has at least a step of 32
-    keys for each of its eight waves."""
+    """Parts of a context, for `pairs` (sequence, key/value head) pairs, each
+    of at least _decode_least steps of 32 keys.  Up to 64 pairs, a block a CU
+    in all: more parts are more to add up (4 users of 10000 tokens, 8 key/value
+    heads: 40 us in 8, 47 in 24; 8 of 2000: 18 in 4, 25 in 12).  Up to 191, 768
+    blocks even out ragged contexts (12 users of 4096 to 12288: 149 us whole,
+    91 in two, 80 in eight).  From 192 on one part is best where its blocks
+    fill whole rounds of the 256 CUs (32 users of about 512 tokens: 17 us
+    against 20 in two short ones); where they do not, long parts fill the last
+    round (34 users of 2500: 73 us against 88 whole, 24 of 4000: 82 against
+    92)."""
     env = os.environ.get("OLLAMAMQ_DECODE_SPLIT")
     if env:                       # tuning override (tools/perf_decode.py)
         want = int(env)
     else:
-        want = 1 if pairs >= 192 else (
-            min(256 // max(1, pairs), 24) if pairs <= 64 else 768 // pairs)
+        want = (min(256 // max(1, pairs), 24) if pairs <= 64
+                else 768 // pairs if pairs < 192
+                else 4 if pairs < 512 and -pairs % 256 > 25 else 1)
     return min(want, max(1, (max_kv + 255) // 256), 32)
 
 
+def _decode_least(pairs):
+    """Steps of a part: one for each of its eight waves, or so many that short
+    contexts stay whole (24, 32 and 48 tried)."""
+    return 48 if pairs >= 192 else 8
+
+
 def _decode_parts(S, Hq, kvh, meta, sem, dev):
-    """(parts of a context, scratch for them, tickets, slots, lengths)"""
+    """(parts of a context, steps of one, scratch, tickets, slots, lengths)"""
     split = _decode_split(S * kvh, meta.max_kv)
     part = None
     if split > 1:
@@ -351,7 +360,8 @@ def _decode_parts(S, Hq, kvh, meta, sem, dev):
         if sem is None:
             sem = torch.zeros(S * kvh, dtype=torch.int32, device=dev)
         assert sem.numel() >= S * kvh
-    return split, part, sem, _i32(meta.slot_ids), _i32(meta.seq_lens)
+    return (split, _decode_least(S * kvh), part, sem, _i32(meta.slot_ids),
+            _i32(meta.seq_lens))
 
 
 def attention_decode(q, cache, layer, meta, fragout=False, out=None,
@@ -375,13 +385,13 @@ def attention_decode(q, cache, layer, meta, fragout=False, out=None,
         q = q.clone(memory_format=torch.contiguous_format)
     kp, vp = _layer_ptrs(cache, layer)
     kvh = cache.n_kv_heads
-    split, part, sem, slot32, len32 = _decode_parts(S, Hq, kvh, meta, sem,
-                                                    q.device)
+    split, least, part, sem, slot32, len32 = _decode_parts(
+        S, Hq, kvh, meta, sem, q.device)
     _check(_lib.decode_attn_bf16(
         _p(out), _p(part), _p(sem), _p(q), kp, vp, _p(cache.page_table),
         _p(slot32), _p(len32), S, Hq, kvh, cache.page_size,
         cache.page_table.shape[1], 1.0 / (D ** 0.5), _row_stride(q, D),
-        split, meta.window, 1 if fragout else 0, _stream()),
+        split, least, meta.window, 1 if fragout else 0, _stream()),
         "decode_attn")
     return out
 
@@ -466,12 +476,12 @@ def attention_mixed(q, cache, layer, meta, fragout=False, sem=None):
         if q.data_ptr() % 16 or _row_stride(q, D) % 8:
             q = q.clone(memory_format=torch.contiguous_format)
         kp, vp = _layer_ptrs(cache, layer)
-        split, part, sem, slots, lens = _decode_parts(nd, Hq, kvh, sub, sem,
-                                                      q.device)
+        split, least, part, sem, slots, lens = _decode_parts(
+            nd, Hq, kvh, sub, sem, q.device)
         _check(_lib.mixed_attn_bf16(
             _p(out), _p(part), _p(sem), _p(q), kp, vp, _p(cache.page_table),
-            _p(items), items.shape[0], _p(slots), _p(lens), nd, split, Hq,
-            kvh, cache.page_size, cache.page_table.shape[1], D ** -0.5,
+            _p(items), items.shape[0], _p(slots), _p(lens), nd, split, least,
+            Hq, kvh, cache.page_size, cache.page_table.shape[1], D ** -0.5,
             _row_stride(q, D), meta.window, int(fragout), _stream()),
             "mixed_attn")
     return out

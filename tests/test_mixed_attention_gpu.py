@@ -83,3 +83,45 @@ def test_as_each_alone(Hq, KVH, page, window, singles, prompts):
     again = hip.attention_mixed(odd, cache, 1, _meta(
         slots, q_lens, kv_lens, nd, window))
     assert torch.equal(again, got)
+
+
+@pytest.mark.parametrize("S,KVH", [(48, 4), (25, 8), (40, 8), (61, 8)])
+@pytest.mark.parametrize("window", [0, 1600])
+def test_long_parts_of_many_users(S, KVH, window):
+    """Between 192 and 511 pairs contexts of 96 steps and more go in parts of
+    at least 48, against float64; tickets are zero again."""
+    from ollamamq_amd.ops import hip
+    hip.require()
+    assert hip._decode_split(S * KVH, 4000) == (1 if S == 61 else 4)
+    torch.manual_seed(7)
+    G = 2
+    lens = [(1, 1535, 1536, 1537, 3071, 3072, 3300, 40)[i % 8]
+            for i in range(S)]
+    cache = PagedKVCache(1, KVH, D, page_size=16,
+                         n_pages=sum(n // 16 + 1 for n in lens), max_slots=S,
+                         max_ctx=4000, device="cuda", dtype=torch.bfloat16)
+    slots = [cache.alloc_slot() for _ in lens]
+    for s, n in zip(slots, lens):
+        cache.ensure(s, n)
+    cache.k_pool.normal_()
+    cache.v_pool.normal_()
+    q = torch.randn(S, G * KVH, D, device="cuda").bfloat16()
+    sem = torch.zeros(S * KVH, dtype=torch.int32, device="cuda")
+    meta = _meta(slots, [1] * S, lens, S, window)
+    first = None
+    for _ in range(3):
+        got = hip.attention_decode(q, cache, 0, meta, sem=sem)
+        assert not sem.any()
+        assert first is None or torch.equal(first, got)
+        first = got
+    for i, n in enumerate(lens):
+        pages = cache.page_table[slots[i], :-(-n // 16)].long()
+        k, v = (p[0][pages].transpose(1, 2).flatten(0, 1)[:n].double()
+                for p in (cache.k_pool, cache.v_pool))
+        lo = max(0, n - window) if window else 0
+        s = torch.einsum("hgd,nhd->hgn", q[i].double().view(KVH, G, D),
+                         k[lo:]) / D ** 0.5
+        want = torch.einsum("hgn,nhd->hgd", s.softmax(-1), v[lo:])
+        # one rounding to bf16, and fp32 sums
+        torch.testing.assert_close(got[i].double(), want.flatten(0, 1),
+                                   rtol=2 ** -8, atol=1e-5)
