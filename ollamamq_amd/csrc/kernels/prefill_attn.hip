@@ -5,10 +5,10 @@
 // token * G + head), so a staged key serves all of them, whatever G is.
 // Before, a wave had one head's 32 tokens, weights went through LDS and values
 // were transposed by 2-byte stores (32 heads, 8 of them key/value heads):
-//   8100 tokens, window 4096     1301 us (312 TF), now 427 (952)
-//   2 x 2048                      335 us (205 TF), now 86 (800)
-//   7 prompts, 2310 together       66 us (106 TF), now 23 (300)
-//   2048, 32 / 32 heads          1777 us, now 66
+//   8100 tokens, window 4096     1288 us (315 TF), now 456 (891)
+//   2 x 2048                      334 us (205 TF), now 101 (680)
+//   7 prompts, 2310 together       68 us (103 TF), now 26 (270)
+//   2048, 32 / 32 heads          1781 us, now 67
 #include "decode_attn.h"
 
 constexpr int D = 128;

@@ -615,8 +615,8 @@ static int softmax_go(
 
 // rows of an item of the flash kernels, all of one sequence, for T_rows tokens
 // of R heads a key/value head.  256 rows a block stage a chunk once for twice
-// the work of 128 (2 x 2048 tokens, 32 heads: 126 us against 140), but 517 tokens
-// are 72 blocks of them (30 us against 27)
+// the work of 128 (2 x 2048 tokens, 32 heads: 106 us against 112), but 517 tokens
+// are 72 blocks of them (26 us against 20)
 extern "C" int softmax_rows(int f32, int Dp, int Vp, int T_rows, int R, int G)
 {
     if (f32 || Dp > 128 || Vp > 128) return 64;

@@ -414,7 +414,7 @@ def _prefill_plan(meta, first, G, KVH, dev):
     parts = list(zip(slots, q_lens, kv_lens))[first:]
     # 256 rows a block stage a chunk once for twice the work of 128, but take
     # whole CUs: best from two blocks a CU on (2 x 2048 tokens, 8 key/value
-    # heads: 86 us against 90; 7 prompts, 2310 together: 26 against 23)
+    # heads: 107 us against 118; 7 prompts, 2310 together: 28 against 27)
     blocks = KVH * sum(-(-n * G // 256) for _, n, _ in parts)
     waves = 8 if first or blocks >= 512 else 4
     items, tok, rows = [], first, 32 * waves

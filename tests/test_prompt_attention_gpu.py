@@ -142,3 +142,26 @@ def test_expanded(D, E, V, window, scale):
         launch(1)
         out = out.view(-1, H * V // 64, 4, 2, 32, 8).permute(0, 4, 1, 2, 3, 5)
         assert torch.equal(out.reshape(-1, H, V)[:T], plain)
+
+
+def test_largest_weight_is_exact():
+    """Rows whose maximum grows by less than 8 octaves after their first 64
+    keys, at a key that alone has the value: the largest weight is 1, so what
+    is left is the result's rounding to bf16, of 8 bits: half a unit, 2^-8 of
+    it at most, and fp32's."""
+    hip, n, D = _hip(), 128, 128
+    g = torch.Generator(device="cuda").manual_seed(6)
+    peak = 3.5 + 1.9 * torch.rand(n, generator=g, device="cuda")
+    mass = 1 + torch.rand(n, generator=g, device="cuda")
+    q, vt = torch.diag(peak).bfloat16(), torch.diag(mass).bfloat16()
+    k = torch.eye(n, device="cuda").bfloat16()
+    out = torch.zeros(n, D, device="cuda").bfloat16()
+    tile = torch.tensor([[0, 0, n, 0]], dtype=torch.int32, device="cuda")
+    p = hip._p
+    hip._check(hip._lib.flash_attn(
+        0, p(out), p(q), p(k), None, p(vt), None, 0, 0, p(tile), 1, 1, D, 0,
+        D, D, 0, n, 1.0, 0, 0, hip._stream()), "flash_attn")
+    pos = torch.arange(n, device="cuda")
+    want = _attend(q, k, vt.T, 1.0, pos, pos * 0).diag()
+    off = (out.diag().double() - want).abs() / want
+    assert off.max().item() < 2 ** -8 * 1.01

@@ -5,8 +5,9 @@ Tolerance: both paths round the residual stream and the operands of every
 product to bf16, at other places: some 12 roundings a path and layer, each off
 by 2^-9 / sqrt(3) of a value's size in the mean, sum to sqrt(2 * 2 * 12) times
 that or 2^-7 of the logits' norm; twice that is allowed.  Single values differ
-like normal ones: of 30000 the furthest lies 4.5 times the mean off, 8 are
-allowed.
+like normal ones: they are nearly alike in the first layer and up to the
+allowed 2^-6 off in the mean in the last, and of 300000 normal values the
+furthest lies 5 times the mean off: 10 times 2^-7.
 """
 import pytest
 import torch
@@ -18,7 +19,7 @@ def _close(a, b):
     size = b.square().mean().sqrt()
     off = (a - b).abs()
     assert off.square().mean().sqrt() <= 2 ** -6 * size
-    assert off.max() <= 8 * 2 ** -7 * size
+    assert off.max() <= 10 * 2 ** -7 * size
 
 
 def _run(model, cfg, fused, steps):
