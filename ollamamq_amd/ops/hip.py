@@ -406,8 +406,10 @@ def upload(values, dev):
 def _prefill_plan(meta, first, G, KVH, dev):
     """(tiles, waves a block) of the sequences from `first` on, the longest
     walks first; cached on the meta object (one build per forward, shared by
-    every layer).  Beside single tokens blocks are as large as theirs."""
-    plan = getattr(meta, "_prefill", None)
+    the layers whose heads group alike: a tile's rows are token * G + head).
+    Beside single tokens blocks are as large as theirs."""
+    key = f"_prefill_{first}_{G}_{KVH}"
+    plan = getattr(meta, key, None)
     if plan is not None:
         return plan
     slots, q_lens, kv_lens = meta.layout()
@@ -424,7 +426,7 @@ def _prefill_plan(meta, first, G, KVH, dev):
         tok += n
     items.sort(key=lambda it: -(it[2] + (it[3] + it[4]) // G))
     plan = (upload(items, dev) if items else None), waves
-    meta._prefill = plan
+    setattr(meta, key, plan)
     return plan
 
 
