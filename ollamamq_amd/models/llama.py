@@ -383,10 +383,15 @@ class LlamaModel:
         selects as "last" (decode: all; prefill: final token per seq)."""
         cfg = self.cfg
         idx = attn_meta.logits_idx
-        if (self.fused_chain and 0 < tokens.shape[0] <= ops.CHAIN_ROWS
+        # The chain has its own attention, so a switch that asks for another
+        # one takes the general path; not for a decode step of up to 64, whose
+        # captured form has none
+        chain = (self.fused_chain and not return_hidden
+                 and (attn_meta.one_each and tokens.shape[0] <= 64
+                      or not ops.other_attention(attn_meta)))
+        if (chain and 0 < tokens.shape[0] <= ops.CHAIN_ROWS
                 and (attn_meta.one_each or idx is None
-                     or 0 < idx.shape[0] <= ops.CHAIN_ROWS)
-                and not return_hidden):
+                     or 0 < idx.shape[0] <= ops.CHAIN_ROWS)):
             return self._forward_fused(tokens, positions, kv_cache,
                                        slot_ids, attn_meta)
         x = ops.embedding(tokens, self.embed)
@@ -420,8 +425,7 @@ class LlamaModel:
         # Only the last token of each sequence needs logits: as few rows as
         # the fused chain takes go through its product (25 rows, 32000
         # columns, with gather, sum and norm: 47 us, the library's 85)
-        if (self.fused_chain and idx is not None and not return_hidden
-                and 0 < idx.shape[0] <= ops.CHAIN_ROWS):
+        if chain and idx is not None and 0 < idx.shape[0] <= ops.CHAIN_ROWS:
             h, sq = ops.fragify_sumsq(x, rows=idx, add=residual)
             return ops.linear_fused(h, self.lm_head_pk,
                                     self.lm_head.shape[0], rstd=sq, rstd_nt=1,

@@ -489,11 +489,16 @@ def attention_mixed(q, cache, layer, meta, fragout=False, sem=None):
     return out
 
 
+def valu_prefill(meta):
+    """The VALU paged_attn path is asked for (A/B + debugging) and can take
+    the batch: it predates sliding windows."""
+    return os.environ.get("OLLAMAMQ_VALU_PREFILL") == "1" and not meta.window
+
+
 def attention_prefill(q, cache, layer, meta):
     """MFMA flash prefill (prefill_attn.hip); set OLLAMAMQ_VALU_PREFILL=1
-    to fall back to the VALU paged_attn path (A/B + debugging)."""
-    if os.environ.get("OLLAMAMQ_VALU_PREFILL") == "1" \
-            and not meta.window:   # VALU fallback predates sliding window
+    to fall back to the VALU paged_attn path."""
+    if valu_prefill(meta):
         return _attention(q, cache, layer, meta, 16)
     T, Hq, D = q.shape
     assert D == 128

@@ -16,10 +16,12 @@ import torch
 from . import reference as ref
 
 
+def force_ref() -> bool:
+    return os.environ.get("OLLAMAMQ_FORCE_REF") == "1"
+
+
 def _use_hip(t: torch.Tensor) -> bool:
-    if not t.is_cuda:
-        return False
-    if os.environ.get("OLLAMAMQ_FORCE_REF") == "1":
+    if not t.is_cuda or force_ref():
         return False
     from . import hip  # deferred: imports/builds the extension
     hip.require()      # raises if the extension is missing on a GPU box
@@ -753,6 +755,13 @@ def fragify_sumsq(x, xf=None, sq=None, tokens=None, rows=None, add=None,
     of x + add; clear: int32 scratch to set to zero on the way."""
     from . import hip
     return hip.fragify_sumsq(x, xf, sq, tokens, rows, add, clear)
+
+
+def other_attention(meta) -> bool:
+    """A triage switch has another attention take this step."""
+    from . import hip
+    return force_ref() or (meta.mode == "prefill"
+                           and hip.valu_prefill(meta))
 
 
 def attention_frag(q, cache, layer, meta, sem=None):
