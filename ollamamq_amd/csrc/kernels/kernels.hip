@@ -974,11 +974,18 @@ extern "C" int sample_gumbel_bf16(
 // of a step whose logits leave the general path (gather, sum and norm as
 // launches of their own: 20 us).  clear: ints that the chain needs as zeros.
 // ---------------------------------------------------------------------------
-// a row by its index, from the end where that is negative; others do not exist
-DEV int64_t row_at(const int64_t* rows, int m, int T) {
-    const int64_t r = rows[m];
-    return max((int64_t)0, min(r < 0 ? r + T : r, (int64_t)T - 1));
-}
+// A row by its index, from the end where that is negative.  For an index that
+// does not exist it is row 0, and the sum of squares is NaN: so are the logits,
+// which are scaled by it.
+struct RowAt {
+    int64_t row;
+    bool bad;
+    __device__ RowAt(int64_t r, int T) {
+        if (r < 0) r += T;
+        bad = r < 0 || r >= T;
+        row = bad ? 0 : r;
+    }
+};
 
 __global__ __launch_bounds__(256) void k_fragify_sumsq(
     const bf16* __restrict__ x, const int* __restrict__ tokens,
@@ -989,7 +996,8 @@ __global__ __launch_bounds__(256) void k_fragify_sumsq(
     const int m = blockIdx.x;
     for (int i = m * 256 + threadIdx.x; i < n_clear; i += gridDim.x * 256)
         clear[i] = 0;
-    const int64_t at = rows ? row_at(rows, m, T) : tokens ? tokens[m] : m;
+    const RowAt wanted(rows ? rows[m] : 0, T);
+    const int64_t at = rows ? wanted.row : tokens ? tokens[m] : m;
     const bf16* row = x + at * H;
     // rows land 32 after 32
     bf16* xfh = xf + (int64_t)(m >> 5) * 32 * H;
@@ -1023,7 +1031,7 @@ __global__ __launch_bounds__(256) void k_fragify_sumsq(
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
     __syncthreads();
     if (threadIdx.x == 0)
-        sq[m] = red[0] + red[1] + red[2] + red[3];
+        sq[m] = wanted.bad ? NAN : red[0] + red[1] + red[2] + red[3];
 }
 
 // Selected rows of an activation in fragment layout, in that layout, and
@@ -1032,7 +1040,9 @@ __global__ __launch_bounds__(256) void k_frag_rows(
     const uint4* __restrict__ x, const int64_t* __restrict__ rows, int T,
     uint4* __restrict__ xf, float* __restrict__ sq, int H)
 {
-    const int m = blockIdx.x, from = (int)row_at(rows, m, T);
+    const int m = blockIdx.x;
+    const RowAt wanted(rows[m], T);
+    const int from = (int)wanted.row;
     const uint4* src = x + (int64_t)(from >> 5) * 4 * H + (from & 31);
     uint4* dst = xf + (int64_t)(m >> 5) * 4 * H + (m & 31);
     float s = 0.f;
@@ -1049,7 +1059,7 @@ __global__ __launch_bounds__(256) void k_frag_rows(
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
     __syncthreads();
     if (threadIdx.x == 0)
-        sq[m] = red[0] + red[1] + red[2] + red[3];
+        sq[m] = wanted.bad ? NAN : red[0] + red[1] + red[2] + red[3];
 }
 
 extern "C" int frag_rows_bf16(void* xf, void* sq, const void* x,

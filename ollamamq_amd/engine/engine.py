@@ -396,7 +396,7 @@ class LlamaEngine:
             logits_idx=idx.view(torch.long), max_q=max(q_lens),
             max_kv=max(kv_lens), n_decode=n_decode,
             window=getattr(self.model.cfg, "sliding_window", 0),
-            q_lens=list(q_lens), kv_lens=kv_lens, slots=slots)
+            q_lens=list(q_lens), kv_lens=kv_lens, slots=slots, rows=want)
         return self.model.forward(tokens, positions, self.kv, slot_per_tok,
                                   meta)
 
@@ -525,7 +525,8 @@ class LlamaEngine:
             cu_q=torch.arange(B + 1, dtype=torch.int32, device=dev),
             logits_idx=torch.arange(B, dtype=torch.long, device=dev),
             max_q=1, max_kv=self.kv.max_ctx,
-            window=getattr(self.model.cfg, "sliding_window", 0))
+            window=getattr(self.model.cfg, "sliding_window", 0),
+            rows=list(range(B)))
         entry = {"bufs": bufs, "meta": meta, "graph": None, "logits": None,
                  "out": bufs["out"], "ring_i": 0, "klass": klass,
                  "pinned": [torch.empty(B, dtype=torch.int64,

@@ -389,6 +389,8 @@ class LlamaModel:
         chain = (self.fused_chain and not return_hidden
                  and (attn_meta.one_each and tokens.shape[0] <= 64
                       or not ops.other_attention(attn_meta)))
+        if chain and idx is not None:
+            attn_meta.check_rows(tokens.shape[0])
         if (chain and 0 < tokens.shape[0] <= ops.CHAIN_ROWS
                 and (attn_meta.one_each or idx is None
                      or 0 < idx.shape[0] <= ops.CHAIN_ROWS)):

@@ -753,8 +753,8 @@ def fragify_sumsq(x, xf=None, sq=None, tokens=None, rows=None, add=None,
                   clear=None):
     """Standard [M, H] -> 32-row frag layout + per-row sum of squares
     (seeds the fused decode chain); with tokens, of their rows of the
-    embedding table x; with rows, of these rows of x + add.  clear: int32
-    scratch to set to zero on the way."""
+    embedding table x; with rows, of these rows of x + add (their sum NaN where
+    there is no such row).  clear: int32 scratch to set to zero on the way."""
     T, H = x.shape
     M = T
     if tokens is not None:
@@ -779,7 +779,7 @@ def fragify_sumsq(x, xf=None, sq=None, tokens=None, rows=None, add=None,
 
 def frag_rows(xf, rows, H, T=None):
     """Rows (int64) of an activation of T rows in fragment layout, in that
-    layout, and their sums of squares."""
+    layout, and their sums of squares (NaN for a row that does not exist)."""
     M, rows = rows.shape[0], rows.long().contiguous()
     T = xf.numel() // H if T is None else T
     assert H % 64 == 0

@@ -39,7 +39,7 @@ class AttnMeta:
     seq_lens : [S] int32  total KV length per slot AFTER the kv_append
     cu_q     : [S+1] int32 exclusive prefix sum of per-seq query counts
     logits_idx: [S] int64 flat indices of each sequence's last token
-                (None = all tokens get logits)
+                (None = all tokens get logits), from the end where negative
     """
     mode: str
     slot_ids: torch.Tensor
@@ -57,6 +57,8 @@ class AttnMeta:
     q_lens: Optional[List[int]] = None
     kv_lens: Optional[List[int]] = None
     slots: Optional[List[int]] = None
+    # host copy of logits_idx
+    rows: Optional[List[int]] = None
 
     @property
     def one_each(self) -> bool:
@@ -77,6 +79,17 @@ class AttnMeta:
             self.kv_lens = self.seq_lens.tolist()
             self.slots = self.slot_ids.tolist()
         return self.slots, self.q_lens, self.kv_lens
+
+    def check_rows(self, n: int) -> None:
+        """IndexError where logits_idx names a row that n tokens do not have.
+        A decode step reads nothing from the device, so there only the host
+        copy tells; without one the kernels give NaN for such a row."""
+        rows = self.rows
+        if rows is None and not self.one_each:
+            rows = self.logits_idx.tolist()
+        if rows and not -n <= min(rows) <= max(rows) < n:
+            raise IndexError(f"logits of rows {min(rows)} to {max(rows)} "
+                             f"wanted of a batch of {n} tokens")
 
 
 class DyT(NamedTuple):
@@ -775,7 +788,7 @@ def attention_frag(q, cache, layer, meta, sem=None):
 
 def frag_rows(xf, rows, H, T=None):
     """Rows of an activation of T rows in frag layout, in that layout, and
-    their sums of squares."""
+    their sums of squares (NaN for a row that does not exist)."""
     from . import hip
     return hip.frag_rows(xf, rows, H, T)
 
