@@ -380,7 +380,7 @@ class LlamaModel:
         return_hidden: bool = False,
     ) -> torch.Tensor:
         """Returns logits [T_last, vocab_full] for the tokens attn_meta
-        selects as "last" (decode: all; prefill: final token per seq)."""
+        selects (of a sequence its last one), or of all."""
         cfg = self.cfg
         idx = attn_meta.logits_idx
         # The chain has its own attention, so a switch that asks for another
@@ -507,7 +507,8 @@ class LlamaModel:
                              sem=tickets)
             nt = tiles_h
         idx = attn_meta.logits_idx
-        if not attn_meta.one_each and idx is not None:
+        if (idx is not None and 0 < idx.shape[0] <= ops.CHAIN_ROWS
+                and attn_meta.rows != list(range(B))):
             # the rows whose logits are wanted
             res, sq_a = ops.frag_rows(res, idx, H, B)
             nt, B = 1, idx.shape[0]

@@ -85,3 +85,34 @@ def test_refused(T, host):
                           torch.zeros(T, **i32),
                           _meta("prefill", "cuda:0", [T], [T], idx,
                                 rows=idx if host else None))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S", [3, 64, 70, 128])
+def test_decode_rows(S):
+    """Of a decode step too: some of them, repeated and in another order."""
+    model = _model()
+    kv = _cache(model, S)
+    g = torch.Generator().manual_seed(2)
+    i32 = dict(dtype=torch.int32, device="cuda:0")
+    tok = torch.randint(0, model.cfg.vocab, (S,), generator=g).to(**i32)
+    for s in range(S):
+        kv.ensure(s, 1)
+    slots = torch.arange(S, **i32)
+
+    def go(idx, **kw):
+        return model.forward(tok, torch.zeros(S, **i32), kv, slots, _meta(
+            "decode", "cuda:0", [1] * S, [1] * S, idx, **kw))
+
+    whole = go(list(range(S)), rows=list(range(S)))
+    assert whole.shape[0] == S
+    for idx in ([S - 1], list(range(S))[::-1], [2, 0, -1, 2],
+                list(range(S))):
+        got = go(idx)
+        assert got.shape[0] == len(idx)
+        # the rows' sums of squares are taken before or after their rounding
+        # to bf16: 2^-9 of a value, far less of a row's root mean square, and
+        # one more rounding of a logit
+        torch.testing.assert_close(got.float(), whole[idx].float(),
+                                   rtol=2 ** -7, atol=2 ** -8)
+    assert go([S, 0]).isnan().any(1).tolist() == [True, False]
