@@ -27,7 +27,8 @@
 // any K%64==0, N%32==0).  Wave partials meet in a single
 // end-of-kernel LDS reduce (the ONE barrier, after all streaming).
 // ksplit>1 writes fp32 partials; the consumer folds them, or the block that
-// arrives last at a tile (x in fragment layout), or k_wstream_combine (+bias).
+// arrives last at a tile (x in fragment layout, or with a fused epilogue), or
+// k_wstream_combine (+bias).
 #include "act.h"
 #include "tile_mma.h"
 
@@ -902,8 +903,8 @@ __global__ __launch_bounds__(256) void k_wstream_combine(
 }
 
 // y == null: the partial sums, fp32, are the result.  sem (x in fragment
-// layout): zeros, one per 32 columns; the product adds up its own parts, then
-// part holds ksplit * N * 32 floats for every 32 rows.
+// layout, or up to 32 rows): zeros, one per 32 columns; the product adds up its
+// own parts, then part holds ksplit * N * 32 floats for every 32 rows.
 extern "C" int wstream_gemm_bf16(
     void* y, void* part, const void* x, const void* wp, const void* bias,
     int M, int N, int K, int64_t xs, int ksplit, int depth, int xlds,
@@ -913,7 +914,7 @@ extern "C" int wstream_gemm_bf16(
 {
     dim3 grid(N / 32, ksplit);
     int* sem = ksplit > 1 && y ? (int*)sem_ : nullptr;
-    if (sem && (xlds != 2 || ksplit > 8)) return -103;
+    if (sem && ((xlds != 2 && M > 32) || ksplit > 8)) return -103;
     const int lds_red = 8 * 32 * 32 * 4 + 512;     // reduce + rstd tail
     const int lds_x = 16 * 4096 + 512;             // + 8x2 x tiles
     const float* rp = (const float*)rstd_parts;
@@ -936,17 +937,17 @@ extern "C" int wstream_gemm_bf16(
             k_wstream_gemm<1, 1, 1><<<grid, 512, lds_x, stream>>>(
                 (bf16*)y, (float*)part, (const bf16*)x, (const u32x4*)wp,
                 (const bf16*)bias, M, N, K, xs, ksplit, rp, rstd_nt,
-                inv_h, eps, ri, sq, {}, yfrag);
+                inv_h, eps, ri, sq, {}, yfrag, sem);
         else if (depth == 2)
             k_wstream_gemm<1, 2><<<grid, 512, lds_red, stream>>>(
                 (bf16*)y, (float*)part, (const bf16*)x, (const u32x4*)wp,
                 (const bf16*)bias, M, N, K, xs, ksplit, rp, rstd_nt,
-                inv_h, eps, ri, sq, {}, yfrag);
+                inv_h, eps, ri, sq, {}, yfrag, sem);
         else
             k_wstream_gemm<1, 1><<<grid, 512, lds_red, stream>>>(
                 (bf16*)y, (float*)part, (const bf16*)x, (const u32x4*)wp,
                 (const bf16*)bias, M, N, K, xs, ksplit, rp, rstd_nt,
-                inv_h, eps, ri, sq, {}, yfrag);
+                inv_h, eps, ri, sq, {}, yfrag, sem);
     } else {
         if (xlds == 2) {
             if (M > 128) return -104;

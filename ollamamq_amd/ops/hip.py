@@ -707,7 +707,7 @@ def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
     be folded into the pack); `res` adds the residual stream into the
     output (pass y=res for the in-place residual update) and `sq_out`
     emits per-tile sum-of-squares partials for the next GEMM.  `sem`: int32
-    zeros, one per 32 columns, for a split product over a fragment-layout x;
+    zeros, one per 32 columns, for a split product that adds up its own parts;
     they are zero again when it ends, so a stream's products can share them."""
     if K is None:
         M, K = x.shape
@@ -728,19 +728,24 @@ def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
             ks = _frag_ksplit(N, K) if xlds == 2 else _wstream_ksplit(N, K)
     if rstd is not None:
         ks = 1            # every part would have to scale its rows
-    part = None
-    if ks > 1:
-        rows = -(-M // 32) * 32 if xlds == 2 else M
-        part = torch.empty(ks * rows * N, dtype=torch.float32,
-                           device=x.device)
-        if xlds == 2 and sem is None:
-            sem = torch.zeros(N // 32, dtype=torch.int32, device=x.device)
-        assert sem is None or sem.numel() >= N // 32
     if xlds is None:
         # measured (profiles/r02_gemm_sweep.md): LDS x-staging pays on
         # long streams (down/gate_up/logits), the direct fragment load
         # wins on the short ramp-bound ones (qkv/o)
         xlds = (_WS_XLDS if M <= 32 and N * K * 2 > (64 << 20) else 0)
+    part = None
+    # what is fused needs the finished sums: the product adds up its own parts
+    if ks > 1 and (xlds == 2 or res is not None or sq_out is not None):
+        part = torch.empty(ks * -(-M // 32) * 32 * N, dtype=torch.float32,
+                           device=x.device)
+        if sem is None:
+            sem = torch.zeros(N // 32, dtype=torch.int32, device=x.device)
+        assert sem.numel() >= N // 32
+    else:
+        sem = None
+        if ks > 1:
+            part = torch.empty(ks * M * N, dtype=torch.float32,
+                               device=x.device)
     _check(_lib.wstream_gemm_bf16(
         _p(y), _p(part), _p(x), _p(packed), _p(bias), M, N, K, xs,
         ks, depth if depth is not None else _WS_DEPTH, xlds,

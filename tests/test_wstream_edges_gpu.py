@@ -93,6 +93,44 @@ def test_parts_add_themselves_up(M, ks, N, K):
     torch.testing.assert_close(plain.double(), want, **CLOSE)
 
 
+@pytest.mark.parametrize("M", [1, 17, 32])
+@pytest.mark.parametrize("xlds,depth", [(0, 1), (0, 2), (1, 1)])
+@pytest.mark.parametrize("ks,N,K", [(2, 64, 512), (3, 192, 1088),
+                                    (8, 128, 4160), (None, 4096, 14336)])
+def test_parts_of_plain_rows(M, xlds, depth, ks, N, K):
+    """The residual sum and sums of squares of a split product over rows that
+    lie in memory one after another, strided ones too."""
+    hip = _hip()
+    x, w, want = _case(M, N, K)
+    x = torch.cat([x, x], 1)[:, :K]
+    pk = hip.pack_weight(w)
+    assert (ks or hip._wstream_ksplit(N, K)) > 1
+    base = torch.randn(M, N, device="cuda").bfloat16()
+    bias = torch.randn(N, device="cuda").bfloat16()
+    total = want + base.double() + bias.double()
+    sem = torch.zeros(N // 32, dtype=torch.int32, device="cuda")
+    for tickets in (None, sem):
+        res = base.clone()
+        sq = torch.zeros(32, N // 32, device="cuda")
+        y = hip.linear_packed(x, pk, bias, N, ks=ks, depth=depth, xlds=xlds,
+                              res=res, y=res, sq_out=sq, sem=tickets)
+        assert y is res and not sem.any()
+        torch.testing.assert_close(y.double(), total, **CLOSE)
+        torch.testing.assert_close(
+            sq[:M].double(), total.square().unflatten(1, (-1, 32)).sum(2),
+            rtol=1e-4, atol=1e-3)
+    # one of the two alone
+    y = hip.linear_packed(x, pk, None, N, ks=ks, depth=depth, xlds=xlds,
+                          res=base)
+    torch.testing.assert_close(y.double(), want + base.double(), **CLOSE)
+    sq = torch.zeros(32, N // 32, device="cuda")
+    hip.linear_packed(x, pk, None, N, ks=ks, depth=depth, xlds=xlds,
+                      sq_out=sq)
+    torch.testing.assert_close(
+        sq[:M].double(), want.square().unflatten(1, (-1, 32)).sum(2),
+        rtol=1e-4, atol=1e-3)
+
+
 @pytest.mark.parametrize("M", [1, 16, 32, 33, 64])
 @pytest.mark.parametrize("F,K", [(16, 64), (48, 576), (160, 4160)])
 def test_gate_up(M, F, K):
