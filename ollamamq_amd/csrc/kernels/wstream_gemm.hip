@@ -920,8 +920,8 @@ extern "C" int wstream_gemm_bf16(
     const float* rp = (const float*)rstd_parts;
     const bf16* ri = (const bf16*)res_in;
     float* sq = (float*)sq_parts;
-    // what is fused needs the finished sums
-    if (ksplit > 1 && !sem && (rstd_parts || res_in || sq_parts))
+    // what is fused needs the finished sums, and k_wstream_combine writes rows
+    if (ksplit > 1 && !sem && (rstd_parts || res_in || sq_parts || yfrag))
         return -100;
     const int d = frag_depth(K, ksplit);
     if (M <= 32) {

@@ -735,7 +735,8 @@ def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
         xlds = (_WS_XLDS if M <= 32 and N * K * 2 > (64 << 20) else 0)
     part = None
     # what is fused needs the finished sums: the product adds up its own parts
-    if ks > 1 and (xlds == 2 or res is not None or sq_out is not None):
+    if ks > 1 and (xlds == 2 or res is not None or sq_out is not None
+                   or yfrag):
         part = torch.empty(ks * -(-M // 32) * 32 * N, dtype=torch.float32,
                            device=x.device)
         if sem is None:

@@ -123,12 +123,38 @@ def test_parts_of_plain_rows(M, xlds, depth, ks, N, K):
     y = hip.linear_packed(x, pk, None, N, ks=ks, depth=depth, xlds=xlds,
                           res=base)
     torch.testing.assert_close(y.double(), want + base.double(), **CLOSE)
+    if N % 64 == 0:                      # whole blocks of the layout
+        y = hip.linear_packed(x, pk, bias, N, ks=ks, depth=depth, xlds=xlds,
+                              yfrag=1)
+        torch.testing.assert_close(_defrag(y, M, N).double(),
+                                   want + bias.double(), **CLOSE)
     sq = torch.zeros(32, N // 32, device="cuda")
     hip.linear_packed(x, pk, None, N, ks=ks, depth=depth, xlds=xlds,
                       sq_out=sq)
     torch.testing.assert_close(
         sq[:M].double(), want.square().unflatten(1, (-1, 32)).sum(2),
         rtol=1e-4, atol=1e-3)
+
+
+def test_parts_without_tickets_are_refused_what_needs_sums():
+    """Nothing runs: fragment layout, a residual, norms or their sums, asked
+    of parts that nobody adds up."""
+    hip = _hip()
+    x, w, _ = _case(8, 64, 512)
+    pk, y = hip.pack_weight(w), torch.zeros(32 * 64, device="cuda").bfloat16()
+    part = torch.empty(2 * 32 * 64, device="cuda")
+    one = torch.zeros(64, device="cuda")
+
+    def go(xlds, norm=None, res=None, sq=None, yfrag=0):
+        return hip._lib.wstream_gemm_bf16(
+            *map(hip._p, (y, part, x, pk, None)), 8, 64, 512, 512, 2, 1, xlds,
+            hip._p(norm), 1, 1.0, 1.0, hip._p(res), hip._p(sq), yfrag, None,
+            hip._stream())
+
+    for xlds in (0, 1):
+        for kw in (dict(norm=one), dict(res=y), dict(sq=one), dict(yfrag=1)):
+            assert go(xlds, **kw) != 0
+    assert not y.any()
 
 
 @pytest.mark.parametrize("M", [1, 16, 32, 33, 64])
