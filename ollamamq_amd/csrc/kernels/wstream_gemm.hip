@@ -914,7 +914,7 @@ extern "C" int wstream_gemm_bf16(
 {
     dim3 grid(N / 32, ksplit);
     int* sem = ksplit > 1 && y ? (int*)sem_ : nullptr;
-    if (sem && ((xlds != 2 && M > 32) || ksplit > 8)) return -103;
+    if (sem && xlds != 2 && M > 32) return -103;
     const int lds_red = 8 * 32 * 32 * 4 + 512;     // reduce + rstd tail
     const int lds_x = 16 * 4096 + 512;             // + 8x2 x tiles
     const float* rp = (const float*)rstd_parts;

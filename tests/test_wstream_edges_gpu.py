@@ -61,11 +61,12 @@ def test_whole(M, N, K):
 
 
 @pytest.mark.parametrize("M", [1, 17, 32, 33, 64])
-@pytest.mark.parametrize("ks", [2, 3, 4, 8])
+@pytest.mark.parametrize("ks", [2, 3, 4, 8, 9, 16])
 @pytest.mark.parametrize("N,K", [(64, 512), (192, 1088), (128, 4160)])
 def test_parts_add_themselves_up(M, ks, N, K):
     """The residual sum in place, sums of squares, and tickets that are zero
-    again, over several products that share them."""
+    again, over several products that share them.  More parts than blocks of
+    64 columns leave some empty."""
     hip = _hip()
     x, w, want = _case(M, N, K)
     pk, xf = hip.pack_weight(w), _frag(x)
