@@ -839,9 +839,9 @@ static int wstream_gu(
 {
     dim3 grid(N / 32, 1);
     const int lds = (xlds == 1 ? 16 * 4096 : 8 * 32 * 32 * 4) + 512;
+    if (M > (xlds == 2 ? 128 : 64)) return -104;   // rows of a block
     if (M > 32) {
         if (xlds == 2) {       // frag chain at batches 33..128
-            if (M > 128) return -104;
             const int cw = wide_tiles(M, N);
             if (cw > 1)
                 return wide<GU>(cw, act, x, wp, M, N, K, rstd_parts, rstd_nt,
@@ -914,6 +914,7 @@ extern "C" int wstream_gemm_bf16(
 {
     dim3 grid(N / 32, ksplit);
     int* sem = ksplit > 1 && y ? (int*)sem_ : nullptr;
+    if (M > (xlds == 2 ? 128 : 64)) return -104;   // rows of a block
     if (sem && xlds != 2 && M > 32) return -103;
     const int lds_red = 8 * 32 * 32 * 4 + 512;     // reduce + rstd tail
     const int lds_x = 16 * 4096 + 512;             // + 8x2 x tiles
@@ -950,7 +951,6 @@ extern "C" int wstream_gemm_bf16(
                 inv_h, eps, ri, sq, {}, yfrag, sem);
     } else {
         if (xlds == 2) {
-            if (M > 128) return -104;
             const int cw = wide_tiles(M, N);
             if (ksplit == 1 && y && !bias && !ri && !sq && cw > 1)
                 return wide<0>(cw, y, x, wp, M, N, K, rp, rstd_nt, inv_h,
@@ -1004,7 +1004,7 @@ extern "C" int wstream_qkv_rope_bf16(
                (const int*)slot, (const int*)ptab, (bf16*)kp, (bf16*)vp,
                nl, nkl, psz, maxp};
     const int d = frag_depth(K, 1);
-    if (xf && M > 128) return -104;
+    if (M > (xf ? 128 : 32)) return -104;          // rows of a block
     if (xf && M > 32)
         (M <= 64   ? k_wstream_gemm<2, 2, 2, 0, 1>
          : M <= 96 ? k_wstream_gemm<3, 2, 2, 0, 1>

@@ -158,6 +158,25 @@ def test_parts_without_tickets_are_refused_what_needs_sums():
     assert not y.any()
 
 
+def test_more_plain_rows_are_refused():
+    """A block has 64 rows of them, with rope 32; none are left out."""
+    hip = _hip()
+    x, w, want = _case(65, 64, 512)
+    pk, gu = hip.pack_weight(w), hip.pack_weight_gu(w)
+    got = hip.linear_packed(x[:64], pk, None, 64)
+    torch.testing.assert_close(got.double(), want[:64], **CLOSE)
+    hip.linear_gu(x[:64], gu, 64)
+    for go in (lambda: hip.linear_packed(x, pk, None, 64),
+               lambda: hip.linear_packed(x, pk, None, 64, ks=2),
+               lambda: hip.linear_gu(x, gu, 64)):
+        with pytest.raises(RuntimeError):
+            go()
+    none = [hip._p(None)]
+    assert hip._lib.wstream_qkv_rope_bf16(
+        *none * 4, 33, 384, 512, 512, *none, 1, 1.0, 1.0, *none * 7, 1, 1, 16,
+        1, 0, hip._stream()) != 0
+
+
 @pytest.mark.parametrize("M", [1, 16, 32, 33, 64])
 @pytest.mark.parametrize("F,K", [(16, 64), (48, 576), (160, 4160)])
 def test_gate_up(M, F, K):
