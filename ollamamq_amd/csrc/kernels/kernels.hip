@@ -896,12 +896,13 @@ __global__ __launch_bounds__(256) void k_gumbel_part(
     const uint64_t sd = seeds ? seeds[row] : 1234567ULL;
     const uint64_t ct = ctrs ? (uint64_t)(unsigned)ctrs[row] : 0ULL;
     const int64_t noff = (int64_t)row * V;
+    const bool vec = ((uintptr_t)lr & 15) == 0;
     float best = -3.0e38f;
     int bidx = 0;
     for (int i = lo + threadIdx.x * 8; i < hi; i += blockDim.x * 8) {
         const int n = min(8, hi - i);
         float v[8];
-        if (n == 8) load8f(lr + i, v);
+        if (n == 8 && vec) load8f(lr + i, v);
         else for (int e = 0; e < n; e++) v[e] = bf2f(lr[i + e]);
         for (int e = 0; e < n; e++) {
             float s = v[e] * invT;
@@ -945,7 +946,8 @@ extern "C" int sample_gumbel_bf16(
 {
     if ((tok && !pb) || sp > 64) return (int)hipErrorInvalidValue;
     if (pb) {
-        const int seg = (V + sp - 1) / sp;
+        const int seg = ((V + sp - 1) / sp + 7) & ~7;   // whole vectors
+        while ((int64_t)(sp - 1) * seg >= V) sp--;      // drop empty slices
         dim3 grid(B, sp);
         k_gumbel_part<true><<<grid, 256, 0, stream>>>(
             nullptr, (float*)pb, (int*)pi, (const bf16*)logits,

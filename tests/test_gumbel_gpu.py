@@ -39,6 +39,41 @@ def test_gumbel_matches_fp32_reference_with_noise():
                            logits.float().argmax(-1).cpu())
 
 
+@pytest.mark.parametrize("B,V", [(1, 7), (1, 264), (5, 1003), (3, 8 * 513),
+                                 (32, 32000), (64, 32000), (128, 32000),
+                                 (2, 128256)])
+def test_gumbel_slices(B, V):
+    """Slices begin at whole vectors of eight, and the pick does not depend on
+    them; rows that do not lie on 16 bytes too."""
+    hip = _hip()
+    p, sp = hip._p, min(32, max(1, 768 // B))
+    best = torch.empty(B, sp, device="cuda")
+    at = torch.full((B, sp), -1, dtype=torch.int32, device="cuda")
+    out = torch.empty(B, dtype=torch.int32, device="cuda")
+    g = torch.Generator().manual_seed(V)
+
+    def pick(logits, parts, temps, noise=None):
+        hip._check(hip._lib.sample_gumbel_bf16(
+            p(out), p(logits), p(temps), None, None, p(noise), B, V, p(best),
+            p(at), parts, *[None] * 5, hip._stream()), "sample_gumbel")
+        return out.clone()
+
+    # of equal logits a slice's first is its best
+    pick(torch.zeros(B, V, device="cuda").bfloat16(), sp,
+         torch.zeros(B, device="cuda"))
+    first = at.flatten()[at.flatten() >= 0]
+    assert (first % 8 == 0).all() and first.max() < V
+    logits = (torch.randn(B, V, generator=g) * 3).bfloat16().cuda()
+    temps = (torch.rand(B, generator=g) * 1.5 + 0.05).cuda()
+    noise = torch.rand(B, V, generator=g).clamp(1e-7, 1 - 1e-7).cuda()
+    odd = torch.empty(B * V + 1, device="cuda").bfloat16()[1:].view(B, V)
+    odd.copy_(logits)
+    for t in (temps, torch.zeros_like(temps)):
+        want = pick(logits, 1, t, noise)
+        assert torch.equal(pick(logits, sp, t, noise), want)
+        assert torch.equal(pick(odd, sp, t, noise), want)
+
+
 def test_gumbel_counter_noise_reproducible_and_distributed():
     hip = _hip()
     B, V = 8, 512
