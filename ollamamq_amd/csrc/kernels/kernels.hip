@@ -523,55 +523,9 @@ extern "C" int swiglu_bf16(void* out, const void* gu, int T, int F, int gelu,
 }
 
 // ---------------------------------------------------------------------------
-// Greedy sampler: per-row argmax over the vocab, bf16 or fp32 logits.
-// One 256-thread block per row; ties resolve to the LOWEST index (matches
-// torch.argmax on the reference path).
+// Greedy sampler: per-row argmax over the vocab, bf16 or fp32 logits; ties
+// resolve to the LOWEST index (matches torch.argmax on the reference path).
 // ---------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(256) void k_argmax(
-    int* __restrict__ out, const T* __restrict__ logits, int V)
-{
-    const int row = blockIdx.x;
-    const T* lr = logits + (int64_t)row * V;
-    float best = -3.0e38f;
-    int bidx = 0;
-    for (int i = threadIdx.x * 8; i < V; i += blockDim.x * 8) {
-        if (i + 8 <= V) {
-            float v[8];
-            load8f(lr + i, v);
-            #pragma unroll
-            for (int e = 0; e < 8; e++)
-                if (v[e] > best || (v[e] == best && i + e < bidx)) {
-                    best = v[e]; bidx = i + e;
-                }
-        } else {
-            for (int e = i; e < V; e++) {
-                const float v = tof(lr[e]);
-                if (v > best || (v == best && e < bidx)) { best = v; bidx = e; }
-            }
-        }
-    }
-    // wave reduce (value, index), lowest index wins ties
-    #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const float ob = __shfl_down(best, off, 64);
-        const int oi = __shfl_down(bidx, off, 64);
-        if (ob > best || (ob == best && oi < bidx)) { best = ob; bidx = oi; }
-    }
-    __shared__ float wb[4];
-    __shared__ int wi[4];
-    const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 0) { wb[wid] = best; wi[wid] = bidx; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int wv = 1; wv < 4; wv++)
-            if (wb[wv] > best || (wb[wv] == best && wi[wv] < bidx)) {
-                best = wb[wv]; bidx = wi[wv];
-            }
-        out[row] = bidx;
-    }
-}
-
 // Split-V argmax: B blocks alone (decode B=32) light 32 of 256 CUs and
 // serialize ~V/2048 load rounds each (measured 45 us at V=128256).
 // Stage 1: (B, SP) blocks scan V/SP slices; stage 2: one wave per row
@@ -666,23 +620,20 @@ static int argmax_go(void* out, const void* logits, int B, int V,
                      void* pb, void* pi, int SP, Advance step,
                      hipStream_t stream)
 {
-    if (step.tok && !pb) return (int)hipErrorInvalidValue;
-    if (pb != nullptr) {
-        // 256-thread x8 rounds; a small vocabulary is one slice
-        int seg = V < SP ? 2048 : (V / SP + 2047) & ~2047;
-        while ((int64_t)(SP - 1) * seg >= V) SP--;  // drop empty slices
-        dim3 grid(B, SP);
-        k_argmax_part<T><<<grid, 256, 0, stream>>>(
-            (float*)pb, (int*)pi, (const T*)logits, V, seg);
-        k_pick<<<(B + 3) / 4, 256, 0, stream>>>(
-            (int*)out, (const float*)pb, (const int*)pi, B, SP, step);
-    } else {
-        k_argmax<T><<<B, 256, 0, stream>>>((int*)out, (const T*)logits, V);
-    }
+    if (!pb || !pi || SP < 1 || SP > 64) return (int)hipErrorInvalidValue;
+    // 256-thread x8 rounds; a small vocabulary is one slice
+    int seg = V < SP ? 2048 : (V / SP + 2047) & ~2047;
+    while ((int64_t)(SP - 1) * seg >= V) SP--;  // drop empty slices
+    dim3 grid(B, SP);
+    k_argmax_part<T><<<grid, 256, 0, stream>>>(
+        (float*)pb, (int*)pi, (const T*)logits, V, seg);
+    k_pick<<<(B + 3) / 4, 256, 0, stream>>>(
+        (int*)out, (const float*)pb, (const int*)pi, B, SP, step);
     return (int)hipGetLastError();
 }
 
-// tok: null, or the next step's inputs (see Advance)
+// pb, pi: room for the best and its index of SP <= 64 slices a row; tok: null,
+// or the next step's inputs (see Advance)
 extern "C" int argmax_bf16(void* out, const void* logits, int B, int V,
                             void* pb, void* pi, int SP, void* tok,
                             void* out64, void* pos, void* lens,
@@ -859,8 +810,8 @@ extern "C" int row_sumsq_bf16(void* sq, const void* x, int M, int H,
 // batch composition (ctr = the sequence's own length that step).
 // Rows with temps[row] <= 0 take the pure argmax path (greedy), so ONE
 // captured graph serves mixed greedy/sampled batches.
-// Split-V two-stage exactly like argmax (the noise is recomputed from
-// (row, v) so partials stay exact).  noise_override (tests): u = that
+// Split-V two-stage exactly like argmax (the noise is that of (row, v), so a
+// pick does not depend on the slices).  noise_override (tests): u = that
 // buffer instead of the hash.
 // ---------------------------------------------------------------------------
 DEV float u01_hash(uint64_t key) {
@@ -879,15 +830,14 @@ DEV float gumbel_of(uint64_t seed, uint64_t ctr, int v,
     return -__logf(-__logf(u));
 }
 
-template <bool PART>
 __global__ __launch_bounds__(256) void k_gumbel_part(
-    int* __restrict__ out, float* __restrict__ pb, int* __restrict__ pi,
+    float* __restrict__ pb, int* __restrict__ pi,
     const bf16* __restrict__ logits, const float* __restrict__ temps,
     const unsigned long long* __restrict__ seeds,
     const int* __restrict__ ctrs, const float* __restrict__ noise,
     int V, int seg)
 {
-    const int row = blockIdx.x, slice = PART ? blockIdx.y : 0;
+    const int row = blockIdx.x, slice = blockIdx.y;
     const int lo = slice * seg, hi = min(V, lo + seg);
     const bf16* lr = logits + (int64_t)row * V;
     const float T = temps ? temps[row] : 0.f;
@@ -929,12 +879,8 @@ __global__ __launch_bounds__(256) void k_gumbel_part(
             if (wb[wv] > best || (wb[wv] == best && wi[wv] < bidx)) {
                 best = wb[wv]; bidx = wi[wv];
             }
-        if (PART) {
-            pb[row * gridDim.y + slice] = best;
-            pi[row * gridDim.y + slice] = bidx;
-        } else {
-            out[row] = bidx;
-        }
+        pb[row * gridDim.y + slice] = best;
+        pi[row * gridDim.y + slice] = bidx;
     }
 }
 
@@ -944,25 +890,18 @@ extern "C" int sample_gumbel_bf16(
     void* pb, void* pi, int sp, void* tok, void* out64, void* pos,
     void* lens, const void* adv, hipStream_t stream)
 {
-    if ((tok && !pb) || sp > 64) return (int)hipErrorInvalidValue;
-    if (pb) {
-        const int seg = ((V + sp - 1) / sp + 7) & ~7;   // whole vectors
-        while ((int64_t)(sp - 1) * seg >= V) sp--;      // drop empty slices
-        dim3 grid(B, sp);
-        k_gumbel_part<true><<<grid, 256, 0, stream>>>(
-            nullptr, (float*)pb, (int*)pi, (const bf16*)logits,
-            (const float*)temps, (const unsigned long long*)seeds,
-            (const int*)ctrs, (const float*)noise, V, seg);
-        k_pick<<<(B + 3) / 4, 256, 0, stream>>>(
-            (int*)out, (const float*)pb, (const int*)pi, B, sp,
-            {(int*)tok, (int64_t*)out64, (int*)pos, (int*)lens,
-             (const int*)adv});
-    } else {
-        k_gumbel_part<false><<<B, 256, 0, stream>>>(
-            (int*)out, nullptr, nullptr, (const bf16*)logits,
-            (const float*)temps, (const unsigned long long*)seeds,
-            (const int*)ctrs, (const float*)noise, V, V);
-    }
+    if (!pb || !pi || sp < 1 || sp > 64) return (int)hipErrorInvalidValue;
+    const int seg = ((V + sp - 1) / sp + 7) & ~7;   // whole vectors
+    while ((int64_t)(sp - 1) * seg >= V) sp--;      // drop empty slices
+    dim3 grid(B, sp);
+    k_gumbel_part<<<grid, 256, 0, stream>>>(
+        (float*)pb, (int*)pi, (const bf16*)logits, (const float*)temps,
+        (const unsigned long long*)seeds, (const int*)ctrs,
+        (const float*)noise, V, seg);
+    k_pick<<<(B + 3) / 4, 256, 0, stream>>>(
+        (int*)out, (const float*)pb, (const int*)pi, B, sp,
+        {(int*)tok, (int64_t*)out64, (int*)pos, (int*)lens,
+         (const int*)adv});
     return (int)hipGetLastError();
 }
 

@@ -755,8 +755,7 @@ def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
     return y
 
 
-def fragify_sumsq(x, xf=None, sq=None, tokens=None, rows=None, add=None,
-                  clear=None):
+def fragify_sumsq(x, sq=None, tokens=None, rows=None, add=None, clear=None):
     """Standard [M, H] -> 32-row frag layout + per-row sum of squares
     (seeds the fused decode chain); with tokens, of their rows of the
     embedding table x; with rows, of these rows of x + add (their sum NaN where
@@ -771,9 +770,8 @@ def fragify_sumsq(x, xf=None, sq=None, tokens=None, rows=None, add=None,
     assert add is None or (add.shape == x.shape and add.dtype == x.dtype
                            and add.is_contiguous() and tokens is None)
     assert x.is_contiguous() and H % 8 == 0
-    if xf is None:
-        xf = torch.empty(((M + 31) // 32) * 32 * H, dtype=x.dtype,
-                         device=x.device)
+    xf = torch.empty(((M + 31) // 32) * 32 * H, dtype=x.dtype,
+                     device=x.device)
     if sq is None:
         sq = torch.empty(M, dtype=torch.float32, device=x.device)
     _check(_lib.fragify_sumsq_bf16(_p(xf), _p(sq), _p(x), _p(tokens),

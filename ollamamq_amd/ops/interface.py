@@ -761,13 +761,12 @@ def linear_fused(x, packed, N, bias=None, rstd=None, rstd_nt=0,
                              K=K, xlds=xlds, M_frag=M_frag, sem=sem)
 
 
-def fragify_sumsq(x, xf=None, sq=None, tokens=None, rows=None, add=None,
-                  clear=None):
+def fragify_sumsq(x, sq=None, tokens=None, rows=None, add=None, clear=None):
     """Standard [M, H] -> 32-row frag layout + per-row sum of squares; with
     tokens, of their rows of the embedding table x; with rows, of these rows
     of x + add; clear: int32 scratch to set to zero on the way."""
     from . import hip
-    return hip.fragify_sumsq(x, xf, sq, tokens, rows, add, clear)
+    return hip.fragify_sumsq(x, sq, tokens, rows, add, clear)
 
 
 def other_attention(meta) -> bool:
