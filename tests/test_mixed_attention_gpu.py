@@ -1,9 +1,10 @@
-"""Single tokens and portions of prompts in one launch: as each kind alone.
+"""Single tokens and portions of prompts in one launch: as each kind alone,
+which other tests compare with float64.
 
-A single token's sum is the same numbers in the same order.  A prompt's row may
-keep an older maximum where it shares a block with other rows: weights and
-results are rounded to bf16 as before, each 2^-9, four roundings of the two
-together.
+A single token's sum is the same numbers in the same order, unless its context
+goes in other parts: then fp32 sums in another order, and a rounding to bf16
+(relative 2^-9) on either side.  A prompt's row shares its wave with the same
+rows in blocks of any size, so it is the same bits.
 """
 import pytest
 import torch
@@ -68,9 +69,9 @@ def test_as_each_alone(Hq, KVH, page, window, singles, prompts):
         assert not sem.any()
         close = dict(rtol=0, atol=0) if hip._decode_split(
             nd * KVH, max(kv_lens)) == hip._decode_split(
-            nd * KVH, max(singles)) else dict(rtol=2 ** -7, atol=1e-4)
+            nd * KVH, max(singles)) else dict(rtol=2 ** -8, atol=1e-5)
         torch.testing.assert_close(got[:nd], alone, **close)
-        torch.testing.assert_close(got[nd:], rest, rtol=2 ** -7, atol=2e-3)
+        assert torch.equal(got[nd:], rest)
     frag = hip.attention_mixed(q, cache, 1, _meta(
         slots, q_lens, kv_lens, nd, window), True, sem)
     if Hq * D % 64 == 0:

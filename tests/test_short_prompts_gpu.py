@@ -45,10 +45,14 @@ STEPS = [
     # portions and single tokens, unsorted, places repeated and out of order
     [(2, range(3, 20), [16, 2, 2]), (0, [5], [0]), (3, range(40), [39]),
      (1, [7], [0])],
-    # one token too many for the chain, and more places than it takes
+    # more than 64 tokens, and places
     [(4, range(65), [64, 0])],
     [(4, range(12), [3] * 70)],
     [(i, [i], [0]) for i in range(5)],
+    # as many tokens as the chain takes, one too many, and more places
+    [(1, range(128), [127])],
+    [(2, range(129), [128, 0])],
+    [(3, range(20), [11] * 129)],
 ]
 
 
