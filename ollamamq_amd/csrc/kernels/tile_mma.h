@@ -114,7 +114,7 @@ template <typename T> DEV float silu_of(float x) {
 // Activation-fragment layout ("frag"): the SAME MFMA fragment order the
 // weight packs use, applied to a [32, K] activation: element (m, k) with
 // k = b*64 + j*16 + h*8 + e lives at 16-byte unit ((b*4 + j)*64 + h*32
-// + m), elem e.  Producers (GEMM epilogues, decode-attention combine,
+// + m), elem e.  Producers (GEMM epilogues, attention,
 // the embedding fragify kernel) write it; consumers stream it LINEARLY
 // exactly like packed weights — the per-iteration x machinery (32-line
 // scattered loads or LDS staging, measured 15-30% on top of the pure

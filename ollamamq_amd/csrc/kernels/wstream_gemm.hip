@@ -1,4 +1,4 @@
-// gfx950 weight-streaming decode GEMM: y[M,N] = x[M,K] @ W[N,K]^T, M <= 64
+// gfx950 weight-streaming GEMM of few rows: y[M,N] = x[M,K] @ W[N,K]^T, M <= 64
 // (128 with x in fragment layout).
 //
 // The decode projections are pure weight streaming (each weight byte is
@@ -408,8 +408,8 @@ void k_wstream_gemm(
                     sg += red8[wv][m][c];
                     su += red8[wv][m][c + 16];
                 }
-                if (rstd_parts) {              // MT==1 chain only
-                    const float rs = rstd_sh[gm];  // pre-silu: nonlinear
+                if (rstd_parts) {              // pre-silu: nonlinear
+                    const float rs = rstd_sh[gm];
                     sg *= rs;
                     su *= rs;
                 }

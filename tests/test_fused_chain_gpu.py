@@ -2,7 +2,7 @@
 
 The chain folds norm weights into the packs and carries rstd / residual /
 sum-of-squares through the GEMM epilogues (models/llama.py
-_forward_decode_fused); it must produce the same logits and the same
+_forward_fused); it must produce the same logits and the same
 greedy tokens as the generic path (explicit rmsnorm kernels + per-shape
 GEMM dispatch) within bf16 tolerance.
 """
