@@ -1,22 +1,22 @@
 #!/usr/bin/env python3
-"""Flagship serving benchmark — driver contract.
+"""Flagship serving benchmark.
 
-Measures the BASELINE.json headline: aggregate tokens/sec serving Llama-3-8B
+Measures the headline metric: aggregate tokens/sec serving Llama-3-8B
 to 32 concurrent users per GPU backend (weak scaling: each of the N ranks is
-one independent MI355X backend running the in-process HIP engine, exactly
-config 3 of BASELINE.json).  A "step" is one continuous-batching decode
+one independent MI355X backend running the in-process HIP engine, one
+worker per GPU).  A "step" is one continuous-batching decode
 iteration: every resident sequence advances one token through the full
 hand-written HIP path (fused RMSNorm, RoPE, paged attention, SwiGLU,
 sampler) + hipBLASLt projections.  Warmup admits + prefills the users, so
 the timed region is pure steady-state serving; p50 queue-wait (submit ->
 first token) is measured during warmup and reported in config.
 
-Launch (driver):
+Launch:
   python bench.py --gpus 1 --steps K --warmup W
   python -m torch.distributed.run --nnodes=1 --nproc-per-node N \
       --master-addr 127.0.0.1 bench.py --gpus N --steps K --warmup W
 
-The reference publishes no number for this metric (BASELINE.md) =>
+The reference publishes no number for this metric =>
 vs_baseline is null.
 """
 import argparse
@@ -32,7 +32,7 @@ import torch
 
 def run_stack(args):
     """Full-stack serving benchmark: native dispatcher + UDS engine
-    workers + HTTP streaming clients (VERDICT r01 item 3).  The timed
+    workers + HTTP streaming clients.  The timed
     region crosses the whole reference-parity path — HTTP ingress,
     per-user queues, scheduler, UDS hop, engine, token stream-out — and
     p50 queue-wait is the DISPATCHER's own /admin/stats definition

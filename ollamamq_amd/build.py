@@ -4,7 +4,7 @@
   python -m ollamamq_amd.build --kernels  # just the gfx950 kernel .so
 
 hipcc cross-compiles gfx950 without a GPU, so this runs in CPU-only CI.
-Artifacts (git-ignored, but shipped in gpurun snapshots):
+Artifacts (git-ignored):
   ollamamq_amd/csrc/kernels/_kernels_gfx950.so
   ollamamq_amd/csrc/dispatcher/_dispatch*.so  + ollamamq-server binary
 """
@@ -99,7 +99,7 @@ def build_dispatcher(force=False):
 
 
 def build_tsan_stress(force=False):
-    """TSan-instrumented concurrency hammer (SURVEY §5 race detection)."""
+    """TSan-instrumented concurrency hammer."""
     import glob
     srcs = sorted(glob.glob(os.path.join(DDIR, "*.cpp")))
     core = [s for s in srcs if not s.endswith("main.cpp")

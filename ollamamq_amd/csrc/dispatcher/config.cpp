@@ -62,9 +62,7 @@ bool load_config(const std::string& path, AppConfig* out, std::string* err) {
     // The parser accepts exactly the documented 3-section subset
     // (appconf.yaml.example).  Anything it cannot represent is a HARD
     // error with a line number — a config that silently parses to
-    // something else is worse than one that refuses to load (
-    // "parses the shipped examples; any real-world appconf fails
-    // silently or oddly").
+    // something else is worse than one that refuses to load.
     auto unsupported = [&](int ln, const std::string& what,
                            std::string* e) {
         if (e)

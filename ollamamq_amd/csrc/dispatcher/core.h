@@ -1,12 +1,11 @@
 // Core state of the ollamamq_amd dispatcher — native C++ rebuild of the
 // reference's AppState (reference src/dispatcher.rs:159-198) with the same
-// coarse-mutex discipline (SURVEY.md §5 "Race detection": coarse locks +
-// snapshot pattern; lock order: control_ops BEFORE backends, mirroring
+// coarse-mutex discipline (coarse locks + snapshot pattern; lock order: control_ops BEFORE backends, mirroring
 // reference src/control.rs:963-965).
 //
 // Where the reference's backends are external HTTP servers, ours are an
-// abstract Backend: HttpBackend (wire-compatible external mode, config 1 of
-// BASELINE.json), WorkerBackend (in-process MI355X GPU worker over a unix
+// abstract Backend: HttpBackend (wire-compatible external mode),
+// WorkerBackend (in-process MI355X GPU worker over a unix
 // socket) and MockBackend (tests).
 #pragma once
 
@@ -239,8 +238,7 @@ public:
 
     LogRing log;
 
-    // metrics surface beyond the reference (tokens/sec and
-    // queue-wait percentiles are the BASELINE headline): ring of recent
+    // metrics surface beyond the reference (queue-wait percentiles): ring of recent
     // queue waits (enqueue -> dispatch), sampled by the scheduler
     mutable std::mutex waits_mu;
     std::deque<int64_t> wait_samples_ms;   // cap 2048

@@ -1,5 +1,5 @@
 // C9/C11/C15: HTTP backend — the external-inference-server compatibility
-// mode (config 1 of BASELINE.json).  Probing order and control-call wire
+// mode.  Probing order and control-call wire
 // bodies follow the reference exactly (reference src/control.rs:128-334
 // probe; :762-936 load/unload executors) so real Ollama / LM Studio
 // servers and the E2E mocks work unchanged.

@@ -8,8 +8,8 @@
 //   flight, model routable or API-family supported), preferring backends
 //   that already have the model loaded; the backend is picked by least
 //   active_requests with a rotating next-index tiebreak.
-// Additionally enforced here (the reference declares but never enforces —
-// SURVEY.md §5 "latent"): tasks older than stuck_timeout with no eligible
+// Additionally enforced here (the reference declares but never enforces
+// it): tasks older than stuck_timeout with no eligible
 // backend are failed 503.
 #pragma once
 

@@ -121,8 +121,8 @@ void Server::handle(const HttpRequest& req, HttpConn& conn) {
         return;
     }
     if (req.path == "/metrics" && req.method == "GET") {
-        // Prometheus exposition (beyond the reference: SURVEY §5 calls for
-        // a first-class metrics surface for the tokens/queue-wait metric)
+        // Prometheus exposition (beyond the reference: tokens and
+        // queue waits as metrics)
         conn.send(200,
                   {{"Content-Type",
                     "text/plain; version=0.0.4; charset=utf-8"}},

@@ -1,5 +1,4 @@
-// Thread-sanitizer stress for the dispatcher core (SURVEY.md §5 "race
-// detection": the reference leans on Rust's type system; the C++ rebuild
+// Thread-sanitizer stress for the dispatcher core (the reference leans on Rust's type system; the C++ rebuild
 // runs this hammer under -fsanitize=thread in CI instead).
 //
 // Spawns ingress threads (enqueue tasks), a scheduler thread

@@ -7,7 +7,7 @@
 // model), newline-framed JSON control messages, raw byte streaming for
 // token output, cancellation by socket close (the worker aborts the
 // sequence and frees its KV when the dispatcher hangs up — the reference
-// merely dropped bytes, SURVEY.md §7 hard-part 4).
+// merely dropped bytes).
 #include <sys/socket.h>
 #include <sys/un.h>
 #include <unistd.h>
@@ -53,8 +53,8 @@ bool send_all(int fd, const std::string& s) {
 }
 
 // Buffered line reader: the old one-byte-per-recv() header read cost
-// ~60 syscalls per request on the token hot path's front door (ADVICE
-// r01); this reads in 16 KiB gulps and hands any overshoot back to the
+// ~60 syscalls per request on the token hot path's front
+// door; this reads in 16 KiB gulps and hands any overshoot back to the
 // caller via rest() so the byte stream after the header is preserved.
 class LineReader {
 public:

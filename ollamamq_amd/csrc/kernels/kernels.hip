@@ -1,15 +1,14 @@
 // gfx950 (MI355X / CDNA4) inference kernels for ollamamq_amd.
 //
 // Hand-written HIP for the hot ops the reference delegates to external
-// Ollama backends (the reference has zero GPU code; this is
-// new construction mandated by the north star): fused residual+RMSNorm,
+// Ollama backends (it has no GPU code): fused residual+RMSNorm,
 // RoPE, paged-KV append, paged decode/prefill attention with LDS-staged KV
 // tiles, SwiGLU, greedy sampler.
 //
-// Conventions (cdna_hip_programming.md):
+// Conventions:
 //  * wave = 64 lanes, block sizes are multiples of 64;
-//  * bf16 I/O, fp32 math; vectorized 16B loads (G13);
-//  * LDS rows padded to kill bank conflicts (G4);
+//  * bf16 I/O, fp32 math; vectorized 16B loads;
+//  * LDS rows padded to kill bank conflicts;
 //  * no CUDA-compat shims; compiled only for --offload-arch=gfx950.
 //
 // Exposed as extern "C" launchers taking raw device pointers + hipStream_t,

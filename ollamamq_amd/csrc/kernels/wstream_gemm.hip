@@ -3,14 +3,13 @@
 //
 // The decode projections are pure weight streaming (each weight byte is
 // used M times; compute is nothing next to the 8 TB/s HBM pull), and
-// round-1 measured hipBLASLt at 1.8-4.6 TB/s on these shapes with a
-// ~19 us floor on qkv/o (profiles/r01_decode_step_budget.md).  Two
-// hand-written attempts also lost:
+// hipBLASLt reaches 1.8-4.6 TB/s on these shapes with a ~19 us floor on
+// qkv/o (profiles/r01_decode_step_budget.md).  Two other hand-written
+// kernels lose too:
 //  * fragment-direct (skinny_gemm.hip): MFMA-layout loads are 16 B/lane at
 //    8 KB row stride -> cold misses over-fetched ~4x;
-//  * LDS-staged: full-line loads, but __syncthreads() carries a vmcnt(0)
-//    (cdna_hip_programming.md "Pipelining across barriers"), draining the
-//    prefetch ring every chunk -> 87% SQ_WAIT_ANY.
+//  * LDS-staged: full-line loads, but __syncthreads() carries a vmcnt(0),
+//    draining the prefetch ring every chunk -> 87% SQ_WAIT_ANY.
 //
 // This kernel removes the conflict at the source: the weights are OURS,
 // so they are stored pre-packed in MFMA fragment order (ops/hip.py
@@ -18,8 +17,7 @@
 // lives at packed uint4 index ((t*NB + b)*4 + j)*64 + (h*32 + r), e inside.
 // The stream is then PERFECTLY linear: each wave reads consecutive 1 KiB
 // vectors (full 128 B line use per instruction), tagged non-temporal
-// (MI355X_MICROARCH "nt-weights": one-time-read stream, -18% landed
-// traffic), with no LDS staging, no barriers, and a register prefetch of
+// (a stream read once: -18% landed traffic), with no LDS staging, no barriers, and a register prefetch of
 // one to four 4 KiB iterations per wave.
 //
 // Geometry: grid (N/32, ksplit) x 512 threads (8 waves).  The K/64
@@ -96,7 +94,7 @@ extern "C" int wstream_pure_bf16(void* sink, const void* wp, int N, int K,
 // block's 32-column output tile holds the (gate, up) pairs of 16 ffn
 // columns; the epilogue computes silu(g)*u (GU == 2: gelu_tanh(g)*u) and stores [M, 16] of the
 // activation directly.  Kills the separate swiglu kernel (9.7 us x 32
-// layers/step in the r02 trace) and the gate_up intermediate round-trip.
+// layers/step) and the gate_up intermediate round-trip.
 // Fused-rmsnorm chain extensions (all nullable; tp=1 decode path):
 //  * rstd_parts/rstd_nt: per-tile sum-of-squares partials of the RAW
 //    residual state x (written by the producing GEMM's epilogue).  The
@@ -111,8 +109,7 @@ extern "C" int wstream_pure_bf16(void* sink, const void* wp, int N, int K,
 // ops/hip.py pack_weight_qkv_rope), so each 32-col output tile holds
 // complete rotation pairs; the epilogue rotates q/k with the host
 // cos/sin tables and writes k/v straight into the paged KV pool —
-// the separate rope_append kernel (8.6 us x layers/step in the r02
-// trace) disappears from the decode step.
+// the separate rope_append kernel (8.6 us x layers/step) disappears from the decode step.
 struct RopeEpi {
     const float* cos_t;   // [max_ctx, 64]
     const float* sin_t;

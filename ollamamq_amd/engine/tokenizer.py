@@ -1,7 +1,7 @@
 """Byte-level synthetic tokenizer.
 
-There is no network to fetch real tokenizer vocabularies (
-synthetic prompts, random-init weights), so workers tokenize bytes 1:1
+Weights are random and prompts synthetic where no tokenizer's vocabulary is at
+hand, so workers tokenize bytes 1:1
 (token id = byte value) and render generated ids deterministically:
 ids < 256 decode to their byte, larger ids to a printable ⟨id⟩ marker.
 This keeps the wire contract exercised end-to-end (prompt in, streamed

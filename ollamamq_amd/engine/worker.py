@@ -3,8 +3,8 @@
 One worker owns one MI355X (or a TP group of them) and serves the
 dispatcher over a unix domain socket — the in-process replacement for the
 reference's HTTP hop to an external Ollama server (reference
-src/dispatcher.rs:742; SURVEY.md §5 "Distributed communication backend":
-the hop becomes a direct submit into the engine's continuous batch).
+src/dispatcher.rs:742):
+the hop becomes a direct submit into the engine's continuous batch.
 
 Protocol (newline-framed JSON in, framed stream out):
   {"cmd":"probe"}                  -> one JSON line of state
@@ -15,7 +15,7 @@ Protocol (newline-framed JSON in, framed stream out):
                                       then raw response bytes, EOF = done.
 Cancellation: the dispatcher closes the socket; the worker notices the
 write failure and cancels the sequence (KV pages freed) — the reference
-only dropped bytes, we stop the compute (SURVEY.md §7 hard-part 4).
+only dropped bytes, we stop the compute.
 
 Run:  python -m ollamamq_amd.engine.worker --socket /tmp/omq0.sock \
           --gpu 0 [--model llama3-8b --max-ctx 4096 --max-batch 64]
@@ -52,7 +52,7 @@ class Worker:
         # (and loads) these models, so the dispatcher's model routing
         # (smart/fuzzy match against available_models) steers each request
         # to the workers that carry its model (reference
-        # src/dispatcher.rs:599-620; BASELINE.json config 5 mixed fleet)
+        # src/dispatcher.rs:599-620): a mixed fleet
         self.model_filter = list(models) if models else None
         self.device = f"cuda:{gpu}" if torch.cuda.is_available() else "cpu"
         self.dtype = (torch.bfloat16 if torch.cuda.is_available()

@@ -45,7 +45,7 @@ def main():
     ap.add_argument("--max-ctx", type=int, default=4096)
     # 288 GB HBM3E leaves KV room far beyond batch 32; measured
     # continuous-batching throughput: 32/64/128 users = 5.5k/9.5k/13.2k
-    # tok/s on one MI355X (BASELINE.md) — 64 is the serving default
+    # tok/s on one MI355X — 64 is the serving default
     ap.add_argument("--max-batch", type=int, default=64)
     ap.add_argument("--port", type=int, default=11435)
     ap.add_argument("--host", type=str, default="127.0.0.1")
@@ -61,8 +61,8 @@ def main():
                          "--gpus/--tp/--model: comma list of "
                          "MODEL[*COUNT][/tpN], e.g. "
                          "'llama3-8b*4,llama3-70b/tp4' = four 1-GPU 8B "
-                         "backends + one TP4 70B backend (BASELINE.json "
-                         "config 5).  Each worker advertises ONLY its "
+                         "backends + one TP4 70B backend.  "
+                         "Each worker advertises ONLY its "
                          "model, so /api/tags routing steers requests "
                          "(reference src/dispatcher.rs:599-620).")
     ap.add_argument("--checkpoint", action="append", default=[],
@@ -128,7 +128,7 @@ def main():
                    "--model", model, "--max-ctx", str(args.max_ctx),
                    "--max-batch", str(args.max_batch)]
             # RCCL small-message tuning for the TP decode all-reduces
-            # (SURVEY.md §5: 16-64 KiB latency-bound messages over the
+            # (16-64 KiB latency-bound messages over the
             # 7-link point-to-point xGMI mesh).  OLLAMAMQ_RCCL_ALGO /
             # _PROTO map onto NCCL_ALGO / NCCL_PROTO for the worker
             # group only; unset, RCCL's own size-based tuning applies

@@ -2,8 +2,7 @@
 
 The reference (Chleba/ollamaMQ) delegates all model math to external Ollama
 servers over HTTP (reference src/dispatcher.rs:742-747); this module is the
-in-process compute contract those backends implicitly satisfied
-(SURVEY.md §2 "CUDA kernels ... There are none").
+in-process compute contract those backends implicitly satisfied.
 
 Design notes (MI355X):
 * weights live resident in HBM3E as bf16 (8B = ~16 GB of 288 GB);

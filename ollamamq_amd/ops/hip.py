@@ -1,7 +1,7 @@
 """ctypes bindings for the gfx950 HIP kernels (csrc/kernels/kernels.hip).
 
 The extension is built IN-TREE (csrc/kernels/_kernels_gfx950.so) so the
-.so travels with the repo snapshot to GPU boxes.  On a GPU box a missing
+.so travels with the source tree.  On a machine with a GPU a missing
 extension is a hard error — ops never fall back silently to eager PyTorch
 (the GPU tests must exercise the native path).
 """
@@ -174,7 +174,7 @@ def require():
     _try_load()
     if _lib is None:
         raise RuntimeError(
-            "ollamamq_amd HIP extension missing on a GPU box: "
+            "ollamamq_amd HIP extension missing on a machine with a GPU: "
             f"{_load_err}. Build it with `python -m ollamamq_amd.build` "
             "(hipcc --offload-arch=gfx950)."
         )
@@ -535,7 +535,7 @@ def pack_weight(w):
     n = t*32+r, k = b*64 + j*16 + h*8 + e goes to 16-byte unit
     ((t*NB + b)*4 + j)*64 + (h*32 + r).  The kernel's loads then walk the
     buffer LINEARLY (full 128 B line per instruction, nt-tagged) — the fix
-    for the 4x cold-line over-fetch of fragment-direct loads (NOTES r01).
+    for the 4x cold-line over-fetch of fragment-direct loads.
     Returns None when the shape doesn't qualify."""
     N, K = w.shape
     if N % 32 or K % 64 or w.dtype != torch.bfloat16 \
@@ -676,7 +676,7 @@ def _wstream_ksplit(N, K):
 _WS_DEPTH = int(os.environ.get("OLLAMAMQ_WS_DEPTH", "1"))
 _WS_XLDS = int(os.environ.get("OLLAMAMQ_WS_XLDS", "1"))
 _WS_KS = os.environ.get("OLLAMAMQ_WS_KS")   # sweep override
-# N above which the library GEMM wins (measured r02 sweep,
+# N above which the library GEMM wins (measured,
 # profiles/r02_gemm_sweep.md: wstream beats hipBLASLt on the
 # ramp-dominated small-N decode shapes qkv/o/down; on gate_up/logits the
 # lib's big-grid kernels are closer to the stream ceiling than our

@@ -1,6 +1,6 @@
 """Op dispatch: hand-written gfx950 HIP kernels on GPU, fp32 torch on CPU.
 
-Policy (task requirement): on a GPU box the HIP extension MUST be present —
+Policy: on a machine with a GPU the HIP extension MUST be present —
 ops fail loudly rather than falling back to eager PyTorch, so a passing GPU
 test is evidence the native path ran.  Set OLLAMAMQ_FORCE_REF=1 to force the
 reference path explicitly (used only by numerics tests to produce oracles).
@@ -24,7 +24,7 @@ def _use_hip(t: torch.Tensor) -> bool:
     if not t.is_cuda or force_ref():
         return False
     from . import hip  # deferred: imports/builds the extension
-    hip.require()      # raises if the extension is missing on a GPU box
+    hip.require()      # raises if the extension is missing on a GPU machine
     return True
 
 

@@ -2,8 +2,8 @@
 
 These are the numerics oracle for the gfx950 HIP kernels (tests compare the
 HIP path against these at fp32) and the CPU execution path for the
-dispatcher/scheduler test suite, which runs with no GPU (the
-reference's whole test strategy runs on loopback without real backends).
+dispatcher/scheduler test suite, which runs with no GPU (as the
+reference's tests run on loopback without real backends).
 """
 from __future__ import annotations
 

@@ -8,7 +8,7 @@ sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 
 def pytest_configure(config):
     config.addinivalue_line(
-        "markers", "gpu: test requires a real MI355X GPU (run via gpurun)"
+        "markers", "gpu: test requires a real MI355X GPU"
     )
 
 

@@ -1,7 +1,7 @@
 """Llama-3-70B end-to-end on ONE MI355X (weights ~141 GB bf16 of 288 GB
 HBM3E — the capacity the paged pool is sized against).  Opt-in
 (OLLAMAMQ_TEST_70B=1): the full-size init takes ~1-2 min, so the default
-GPU suite skips it; tools/run_70b.sh drives it via gpurun."""
+GPU suite skips it; tools/run_70b.sh drives it."""
 import os
 
 import pytest

@@ -1,5 +1,5 @@
-"""bench.py driver contract: single-process default run and the exact
-torchrun multi-rank launch shape the round-end driver uses (CPU/gloo here;
+"""bench.py contract: single-process default run and the exact
+torchrun multi-rank launch shape (CPU/gloo here;
 the same code path binds NCCL/RCCL per-GPU on an MI355X node)."""
 import json
 import os
@@ -61,7 +61,7 @@ def test_bench_torchrun_two_ranks():
 
 def test_bench_stack_mode():
     """--stack measures through the full dispatcher + UDS worker path and
-    reports the dispatcher's own queue-wait percentiles (VERDICT r01 #3)."""
+    reports the dispatcher's own queue-wait percentiles."""
     r = subprocess.run(
         [sys.executable, BENCH, "--stack", "--gpus", "1",
          "--steps", "36", "--warmup", "3"],

@@ -101,7 +101,7 @@ def test_url_normalization():
 
 def test_adversarial_yaml_refused(tmp_path):
     """Constructs outside the documented subset must refuse to load with
-    a line-numbered error, never silently misparse (ADVICE r01)."""
+    a line-numbered error, never silently misparse."""
     bad = [
         ("anchors", "backends:\n  - &b http://x\n"),
         ("alias value", "models:\n  - name: *b\n"),

@@ -1,4 +1,4 @@
-"""Failure detection + elastic recovery (SURVEY.md §5): a dead worker goes
+"""Failure detection + elastic recovery: a dead worker goes
 offline via the health loop, requests for it park/503, and a restarted
 worker rejoins automatically with learned state re-probed."""
 import os
@@ -113,8 +113,7 @@ def test_worker_death_and_rejoin(tmp_path):
 def test_midstream_worker_death_truncates_cleanly(tmp_path):
     """Worker dies while a response is STREAMING: the client's stream
     ends (truncated, no done marker), the dispatcher survives, and the
-    health loop flips the backend offline (SURVEY §5 mid-stream
-    failure semantics)."""
+    health loop flips the backend offline."""
     if not os.path.exists(BIN):
         subprocess.run([sys.executable, "-m", "ollamamq_amd.build"],
                        check=True)

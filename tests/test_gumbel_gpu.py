@@ -1,6 +1,6 @@
 """Gumbel-max sampler kernel + in-graph sampled decode (1 GPU).
 
-the stochastic sampler is a hand-written kernel and
+The stochastic sampler is a hand-written kernel and
 sampled workloads replay hipGraphs.  Exactness: with a supplied uniform
 noise buffer the kernel must equal the fp32 reference
 argmax(l/T - log(-log(u))) bit-for-bit in its argmax decision; without

@@ -1,6 +1,6 @@
 """Numerics: each gfx950 HIP kernel vs the plain-PyTorch fp32 reference.
 
-Runs only on a real MI355X (pytest -m gpu via gpurun).  Inputs are random
+Runs only on a real MI355X (pytest -m gpu).  Inputs are random
 bf16; the oracle computes in fp32 from the same bf16-rounded values, so
 tolerances cover only the kernel's own bf16 output rounding + fp32
 reduction-order differences.

@@ -102,7 +102,7 @@ def test_load_spreads_across_workers(node):
 # --------------------------------------------------------------- config 5
 @pytest.fixture(scope="module")
 def hetero_node(tmp_path_factory):
-    """Mixed-fleet rehearsal (BASELINE.json config 5 on CPU): two workers
+    """Mixed-fleet rehearsal on the CPU: two workers
     carrying ONLY tiny + one carrying ONLY tiny-qwen; requests must route
     by model (reference src/dispatcher.rs:599-620) and fair-share across
     users."""

@@ -1,4 +1,4 @@
-"""Checkpoint/resume semantics (SURVEY §5): the dispatcher's durable
+"""Checkpoint/resume semantics: the dispatcher's durable
 state is blocked_items.json + appconf.yaml.  Restarting the dispatcher
 while the worker keeps running must (a) reload the blocklist from disk,
 (b) re-discover the worker and its RESIDENT model via the probe (the

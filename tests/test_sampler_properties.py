@@ -42,7 +42,7 @@ def test_greedy_always_argmax(B, V, seed):
 @settings(derandomize=True, max_examples=30, deadline=None)
 @given(st.integers(2, 8), st.integers(8, 200), st.integers(0, 10 ** 6))
 def test_mixed_per_request_params(B, V, seed):
-    """VERDICT r01 item 6: rows carry DIFFERENT top_k/top_p in one batch;
+    """Rows carry DIFFERENT top_k/top_p in one batch;
     each row must honor its own filter (no engine-wide max/min bleed)."""
     g = torch.Generator().manual_seed(seed)
     logits = torch.randn(B, V, generator=g) * 4

@@ -1,6 +1,6 @@
 """hipGraph-captured decode step containing RCCL collectives (1 GPU).
 
-before an 8-GPU node runs TP decode graphs,
+Before an 8-GPU node runs TP decode graphs,
 prove the capture mechanics on a single MI355X with a 1-rank NCCL(=RCCL)
 group — the model's 2-per-layer all-reduces execute inside the captured
 graph (numerically no-ops at world 1) and the replayed tokens match the

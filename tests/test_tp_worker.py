@@ -76,8 +76,8 @@ def test_tp_worker_lockstep_matches_single():
 def _rank_uds(rank, world, port, sock_path, q):
     """Rank 0 serves the REAL UDS wire (worker.serve + Conn), exercising
     Conn._request -> TPWorker.generate(..., num_ctx=...) and the
-    keep_alive:0 -> unload(only_if_idle=True) path that ADVICE r01 found
-    untested (TPWorker signatures must match worker.Worker's)."""
+    keep_alive:0 -> unload(only_if_idle=True) path
+    (TPWorker signatures must match worker.Worker's)."""
     os.environ["MASTER_ADDR"] = "127.0.0.1"
     os.environ["MASTER_PORT"] = str(port)
     import json

@@ -1,4 +1,4 @@
-"""Race detection (SURVEY.md §5): the dispatcher core under
+"""Race detection: the dispatcher core under
 ThreadSanitizer — ingress/scheduler/health/control/TUI-snapshot threads
 hammering one AppState.  Any data race or lock-order violation fails."""
 import os

@@ -1,4 +1,4 @@
-"""Localize the MFMA prefill attention numerics error (GPU box)."""
+"""Localize the MFMA prefill attention numerics error (on a GPU)."""
 import os
 import sys
 

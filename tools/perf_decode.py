@@ -1,6 +1,6 @@
 """Microbench: decode attention old (unsplit) vs flash-decoding path.
 
-Run on a GPU box:  python tools/perf_decode.py [ctx] [batch]
+Run on a GPU machine:  python tools/perf_decode.py [ctx] [batch]
 """
 import os
 import sys

@@ -1,7 +1,7 @@
 """Decode-shape microbench for the small per-step kernels (rmsnorm,
 swiglu, rope_append, argmax): isolates each op at batch B with cold
 activations (cycled buffers) to see how far each sits above its
-latency floor.  Run on a GPU box: python tools/perf_elementwise.py [B]
+latency floor.  Run on a GPU machine: python tools/perf_elementwise.py [B]
 """
 import os
 import sys

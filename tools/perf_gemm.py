@@ -2,11 +2,11 @@
 shapes, with a ksplit x prefetch-depth sweep and a pure-stream arm (same
 grid/addressing, loads only) that shows each geometry's load-path ceiling.
 
-Run on a GPU box: python tools/perf_gemm.py [M] [--sweep]
+Run on a GPU machine: python tools/perf_gemm.py [M] [--sweep]
 
 COLD-weight protocol: cycles enough weight copies that the 256 MiB L3
 never serves a re-read (the serving loop streams weights from HBM once
-per step; r01's fragment-direct kernel won warm and lost cold)."""
+per step; the fragment-direct kernel wins warm and loses cold)."""
 import os
 import sys
 import time

@@ -1,5 +1,5 @@
 #!/bin/bash
-# Serving soak on a GPU box: bring up the full node (dispatcher + GPU
+# Serving soak on a GPU machine: bring up the full node (dispatcher + GPU
 # worker, Llama-3-8B), then drive repeated randomized stress waves for
 # $SOAK_SECS while watching VRAM and dispatcher RSS for drift.
 set -x

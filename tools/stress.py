@@ -6,7 +6,7 @@ parity: 50 users × 1-12 randomized requests over 4 endpoints × 2 models,
         --users 50 --models llama3-8b
 
 Prints aggregate tokens/sec and queue-wait percentiles at the end — the
-BASELINE.json serving metric, measured through the full HTTP stack.
+serving metric, measured through the full HTTP stack.
 """
 import argparse
 import concurrent.futures as cf

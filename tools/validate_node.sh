@@ -1,5 +1,5 @@
 #!/bin/bash
-# Full-stack validation on a GPU box: node launcher -> C++ dispatcher ->
+# Full-stack validation on a GPU machine: node launcher -> C++ dispatcher ->
 # UDS -> GPU engine worker serving Llama-3-8B over the Ollama/OpenAI wire,
 # plus multi-model routing (8B + tiny) and a small stress run.
 set -x
