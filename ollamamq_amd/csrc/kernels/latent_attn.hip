@@ -1008,8 +1008,8 @@ __global__ __launch_bounds__(256, 1) void k_flash(
 
 // ---------------------------------------------------------------------------
 // The same for bf16 keys of at most 192 and values of at most 128, see
-// flash32.h.  32 heads, 192 / 128 wide, prompts of 1024 and 3072 tokens: 192 us
-// within a model, 370 with k_flash; alone 136 (0.8 PFLOP/s).  Tiles of 128
+// flash32.h.  32 heads, 192 / 128 wide, prompts of 1024 and 3072 tokens: 203 us
+// within a model, 370 with k_flash; alone 138 (0.8 PFLOP/s).  Tiles of 128
 // queries leave a CU half its waves, as LDS holds one block: 67 us against 48
 // for 7 prompts, 2310 tokens together, and no gain for one of 37.
 // VEC: whole vectors of queries and keys.

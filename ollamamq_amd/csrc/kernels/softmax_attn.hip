@@ -280,8 +280,8 @@ __global__ __launch_bounds__(256) void k_softmax_flash(
 
 // ---------------------------------------------------------------------------
 // The same for bf16 heads of at most 128, see flash32.h.  32 heads of 128, 8 of
-// them key/value heads, prompts of 1024 and 3072 tokens: 135 us within a model,
-// 214 with k_softmax_flash; alone 124 (0.7 PFLOP/s).
+// them key/value heads, prompts of 1024 and 3072 tokens: 141 us within a model,
+// 214 with k_softmax_flash; alone 127 (0.7 PFLOP/s).
 // ---------------------------------------------------------------------------
 // EVEN: heads are DK and DV wide and eight keys are on one page.
 template <int DK, int DV, int NW, bool EVEN>
@@ -615,7 +615,7 @@ static int softmax_go(
 
 // rows of an item of the flash kernels, all of one sequence, for T_rows tokens
 // of R heads a key/value head.  256 rows a block stage a chunk once for twice
-// the work of 128 (2 x 2048 tokens, 32 heads: 106 us against 112), but 517 tokens
+// the work of 128 (2 x 2048 tokens, 32 heads: 108 us against 112), but 517 tokens
 // are 72 blocks of them (26 us against 20)
 extern "C" int softmax_rows(int f32, int Dp, int Vp, int T_rows, int R, int G)
 {
