@@ -1,0 +1,725 @@
+// gfx950 products of many rows: y[M, N] = x[M, K] @ W[N, K]^T, x in fragment
+// layout (tile_mma.h), W packed the same way (ops/hip.py pack_weight and its
+// kin), with what follows a product of the fused chain in the epilogue.
+//
+// What bounds it: at 256 CUs the matrix cores draw the card down to 1.5 to
+// 1.7 GHz, where this loop keeps them 95 % busy (1.5 PFLOP/s over the rows that
+// are there; 2.25 with operands that do not move).  So a product takes what its
+// padded tiles take, and what is left to gain is padding, passes beside the
+// product and, for few rows, CUs without a tile.
+//
+// * A block of four waves, one a SIMD, makes 32 HM x 32 HN of y; a wave keeps
+//   its quarter, HM x HN accumulators of 16 x 16.  Large tiles because every
+//   byte that a CU loads costs power and time: 288 x 224 loads 126 operations
+//   a byte.
+// * K goes by in slabs of 32 through four stages of LDS.  Both operands lie in
+//   fragment order, so a slab of 32 rows is 2 KB in a row, goes to LDS without
+//   passing registers (16 bytes a lane) and comes back without bank conflicts.
+//   Three slabs are under way while one is multiplied.
+// * A wave issues one instruction every four clocks, a 16x16x32 product takes
+//   16: no more than three other instructions may stand beside it.  Hence
+//   pointers per piece that move only with the tile, stages known at compile
+//   time, one barrier a slab, and loads and reads spread over a slab's products
+//   (300 instructions a slab of 63 products ran at 1.30 PFLOP/s, 183 at 1.43).
+// * Blocks stay and take the next tile, whose first slabs are on their way
+//   while the last one's results are stored.
+//
+// Within 32 rows or columns LDS holds groups of eight in the order 0 2 | 1 3: 16
+// columns of a tile are then 8 of the first and 8 of the last 16, so the gate and
+// up columns of pack_weight_gu and the rotation pairs of pack_weight_qkv_rope
+// meet in one accumulator, 32 lanes apart.
+//
+// us for 541, 2317 and 8100 rows, one after another on one card:
+//   28672 x 4096, gated   library product 140, 421, 1270 and norm and
+//                         activation 15, 50, 166; here 110, 442, 1370
+//   6144 x 4096, rotated  40, 88, 268 and norm and append 11, 28, 78; here 40,
+//                         114, 325
+//   4096 x 14336          112, 213, 610; here 80 (six parts), 228, 650
+#include <type_traits>
+#include <utility>
+#include "act.h"
+#include "tile_mma.h"
+
+namespace {
+
+enum { RESIDUAL, GATED, ROPE, PARTS };
+
+// where a rotated or plain key and value go (ROPE)
+struct Append {
+    const float* cos_t;   // [positions, 64]
+    const float* sin_t;
+    const int* pos;       // [M]
+    const int* slot;      // [M]
+    const int* ptab;      // page table [slots, maxp]
+    bf16* kp;             // this layer's pools
+    bf16* vp;
+    int nl, nkl, psz, maxp;
+};
+
+struct TileArgs {
+    bf16* y;              // RESIDUAL, GATED: fragment layout; ROPE: [M, N]
+    float* part;          // PARTS: see k_tile_fold; GATED, ROPE: [M] scratch
+    const bf16* x;
+    const bf16* w;
+    const bf16* bias;     // ROPE: [N] or null, in W's order
+    const bf16* res;      // RESIDUAL: the residual stream, may be y
+    float* sq;            // RESIDUAL: [M, tiles of columns] sums of squares
+    const float* rstd;    // GATED, ROPE: [M, rstd_nt] sums of squares of x
+    int rstd_nt;
+    float inv_h, eps;
+    int M, N, K;
+    int mt, nt, ks, gm;   // tiles of rows, of columns, parts of K, rows a group
+    int gelu;
+    Append ap;
+};
+
+// 1 KB pieces to LDS, a lane's 16 bytes at base + voff to lds + 16 * lane.  An
+// instruction's offset moves both addresses, so one M0 serves two.
+template <int O0, int O1>
+DEV void to_lds2(uint64_t b0, uint64_t b1, int voff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+                 "global_load_lds_dwordx4 %1, %2 offset:%4\n\t"
+                 "global_load_lds_dwordx4 %1, %3 offset:%5"
+                 :: "s"(lds), "v"(voff), "s"(b0), "s"(b1), "n"(O0), "n"(O1)
+                 : "memory");        // M0: the compiler keeps nothing there
+}
+template <int O0>
+DEV void to_lds1(uint64_t b0, int voff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+                 "global_load_lds_dwordx4 %1, %2 offset:%3"
+                 :: "s"(lds), "v"(voff), "s"(b0), "n"(O0) : "memory");
+}
+template <int N> DEV void wait_loads() {
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
+}
+
+template <int I> using ic = std::integral_constant<int, I>;
+template <int... I, class F>
+DEV void each_of(std::integer_sequence<int, I...>, F f) { (f(ic<I>{}), ...); }
+// f(0), .. f(N - 1), as constants
+template <int N, class F> DEV void each(F f) {
+    each_of(std::make_integer_sequence<int, N>{}, f);
+}
+
+// row or column of 32 that half h (16 of LDS's order) has at its place p
+DEV int in_strip(int h, int p) {
+    return (p >> 3) * 16 + h * 8 + (p & 7);
+}
+// element (row, col) of fragments of N columns
+DEV int64_t frag_at(int row, int col, int N) {
+    return (int64_t)(row >> 5) * 32 * N + (col >> 3) * 256 + (row & 31) * 8
+           + (col & 7);
+}
+DEV void put4(bf16* p, const f32x4& v) {
+    *reinterpret_cast<bf16x4*>(p) =
+        bf16x4{(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
+}
+DEV f32x4 get4(const bf16* p) {
+    const bf16x4 v = *reinterpret_cast<const bf16x4*>(p);
+    return f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+}
+// the upper lanes of a with the lower lanes of b
+DEV void swap32(f32x4& a, f32x4& b) {
+    #pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const auto r = __builtin_amdgcn_permlane32_swap(
+            __float_as_uint(a[i]), __float_as_uint(b[i]), false, false);
+        a[i] = __uint_as_float(r[0]);
+        b[i] = __uint_as_float(r[1]);
+    }
+}
+
+// stages of LDS; four keep three slabs of a large tile under way, small tiles
+// need more of their slabs for as many bytes
+constexpr int tile_stages(int hm, int hn) { return hm + hn <= 8 ? 8 : 4; }
+constexpr int tile_lds(int hm, int hn) {        // and three values per row
+    return tile_stages(hm, hn) * (hm + hn) * 2048 + hm * 32 * 12;
+}
+
+template <int HM, int HN, int EPI>
+__global__ __launch_bounds__(256, 1) void k_tile_gemm(const TileArgs a)
+{
+    constexpr int STRIPS = HM + HN, STAGE = STRIPS * 2048;
+    constexpr int STAGES = tile_stages(HM, HN);
+    constexpr int PER = STRIPS / 2;        // pieces per wave and slab
+    constexpr int PAIRS = (PER + 1) / 2;
+    static_assert(STRIPS % 2 == 0 && PER <= 8);
+    extern __shared__ __align__(1024) char smem[];
+    const uint32_t lds0 =
+        (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+    float* row_f = reinterpret_cast<float*>(smem + STAGES * STAGE);
+    int* row_pos = reinterpret_cast<int*>(row_f + HM * 32);
+    int* row_kv = row_pos + HM * 32;
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wid >> 1, wn = wid & 1;
+    const int r16 = lane & 15, g4 = lane >> 4;
+
+    // A round's tiles are dealt to the XCDs in runs, so that the blocks which
+    // share an L2 share rows and columns too; a last, short round as evenly.
+    const int items = a.mt * a.nt * a.ks, G = gridDim.x;
+    auto item_at = [&](int first) {
+        const int per = (min(G, items - first) + 7) >> 3;
+        const int j = blockIdx.x >> 3;
+        const int id = first + (blockIdx.x & 7) * per + j;
+        return first < items && j < per && id < items ? id : -1;
+    };
+    const int nq = a.K / (32 * STAGES);    // rounds of slabs
+    int m, n, k, q0, q1;
+    auto tile_at = [&](int id, int& m, int& n, int& k, int& q0, int& q1) {
+        const int mn = a.mt * a.nt;
+        k = id / mn;
+        id -= k * mn;
+        const int per = a.gm * a.nt, g = id / per, r = id - g * per;
+        const int rows = min(a.gm, a.mt - g * a.gm);
+        n = r / rows;
+        m = g * a.gm + r - n * rows;
+        q0 = nq * k / a.ks;
+        q1 = nq * (k + 1) / a.ks;
+    };
+    int first = 0, id = item_at(0);
+    if (id < 0) return;
+    tile_at(id, m, n, k, q0, q1);
+
+    // the order of LDS comes from which lane loads what
+    int voff;
+    const int lane_off = ((lane & 32) + in_strip(lane >> 4 & 1, r16)) * 16;
+    uint64_t base[PER];
+    const int strip_bytes = a.K * 64;
+    // strips past the last repeat it; nothing of theirs is stored
+    const int ms = (a.M + 31) >> 5, ns = a.N >> 5;
+    auto point = [&](int m, int n, int q0) {
+        #pragma unroll
+        for (int i = 0; i < PER; i++) {
+            const int d = wid * PER + i, s = d >> 1;
+            const uint64_t p = s < HM
+                ? (uint64_t)a.x
+                      + (int64_t)min(m * HM + s, ms - 1) * strip_bytes
+                : (uint64_t)a.w
+                      + (int64_t)min(n * HN + s - HM, ns - 1) * strip_bytes;
+            base[i] = p + (d & 1) * 1024 - (i - PER / 2) * 1024;
+        }
+        voff = lane_off + q0 * (STAGES * 2048);
+    };
+    point(m, n, q0);
+    const uint32_t lds_w = lds0 + (wid * PER + PER / 2) * 1024;
+    auto load = [&](auto p_, auto st_) {   // two pieces into a stage
+        constexpr int p = 2 * decltype(p_)::value, st = decltype(st_)::value;
+        constexpr int o = (p - PER / 2) * 1024;
+        if constexpr (p + 1 < PER)
+            to_lds2<o, o + 1024>(base[p], base[p + 1], voff,
+                                 lds_w + st * STAGE);
+        else
+            to_lds1<o>(base[p], voff, lds_w + st * STAGE);
+    };
+    each<STAGES>([&](auto st) {
+        each<PAIRS>([&](auto p) { load(p, st); });
+        voff += 2048;
+    });
+
+    // Operands of a slab: half h of an operand's strips, lanes 16 j .. of it
+    // its columns 8 j ..; a wave's halves may begin inside a strip.
+    constexpr int NF = HM + HN;
+    bf16x8 f[2][NF];
+    const int foff = (g4 >> 1) * 1024 + (g4 & 1) * 512 + r16 * 16;
+    const int h0[2] = {wm * HM, wn * HN};
+    // an instruction reaches 64 KB from its pointer
+    constexpr int REACH = 65536 / STAGE, POINTERS = (STAGES + REACH - 1) / REACH;
+    const char* at[2][2][POINTERS];        // operand, parity, stages
+    #pragma unroll
+    for (int o = 0; o < 2; o++)
+        #pragma unroll
+        for (int par = 0; par < 2; par++)
+            #pragma unroll
+            for (int s = 0; s < POINTERS; s++) {
+                const int h = h0[o] + par;
+                at[o][par][s] = smem + foff + o * HM * 2048
+                                + (h >> 1) * 2048 + (h & 1) * 256
+                                + s * REACH * STAGE;
+            }
+    auto read = [&](int buf, auto st_, int i) {
+        constexpr int st = decltype(st_)::value;
+        const int o = i >= HM, h = o ? i - HM : i;
+        f[buf][i] = *reinterpret_cast<const bf16x8*>(
+            at[o][h & 1][st / REACH] + st % REACH * STAGE + (h >> 1) * 2048);
+    };
+    f32x4 acc[HM][HN] = {};
+
+    // One slab: its operands are in registers.  Whoever passes the barrier
+    // knows that every wave has read this stage, which the slab four ahead may
+    // then take, and that the next slab has landed: of a wave's loads only
+    // those of the two after it are still under way.
+    auto slab = [&](auto st_) {
+        constexpr int st = decltype(st_)::value, cur = st & 1, MF = HM * HN;
+        constexpr ic<(st + 1) % STAGES> next{};
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier"
+                     :: "n"(PER * (STAGES - 2)) : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        each<MF>([&](auto i_) {
+            constexpr int i = decltype(i_)::value;
+            // reads over the first three quarters, loads over all of it
+            #pragma unroll
+            for (int q = 0; q < NF; q++)
+                if (q * MF * 3 / (4 * NF) == i) read(cur ^ 1, next, q);
+            each<PAIRS>([&](auto p) {
+                if constexpr ((decltype(p)::value * MF + MF / 4) / PAIRS == i)
+                    load(p, st_);
+            });
+            // to and fro, so that one operand stays
+            constexpr int r = i / HN, c = r & 1 ? HN - 1 - i % HN : i % HN;
+            acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                f[cur][HM + c], f[cur][r], acc[r][c], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        voff += 2048;
+    };
+
+    // What a row's results need, for the 32 HM rows of a tile: the scale of its
+    // norm, and where its keys and values go.  The loads are under way before
+    // the stores of the tile before, for which they would wait; sums of squares
+    // in parts are added up in place, eight lanes a row.
+    struct {
+        float sq[2];
+        int pos[2], slot[2];
+    } of_row;
+    auto ask_rows = [&](int m) {
+        #pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int r = min(m * HM * 32 + i * 256 + (int)threadIdx.x,
+                              a.M - 1);
+            if (EPI == GATED || EPI == ROPE)
+                if (a.rstd_nt == 1) of_row.sq[i] = a.rstd[r];
+            if (EPI == ROPE) {
+                of_row.pos[i] = a.ap.pos[r];
+                of_row.slot[i] = a.ap.slot[r];
+            }
+        }
+    };
+    auto keep_rows = [&](int m) {
+        #pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int r = i * 256 + threadIdx.x;
+            if (r >= HM * 32) continue;
+            if (EPI == GATED || EPI == ROPE)
+                if (a.rstd_nt == 1)
+                    row_f[r] = rsqrtf(of_row.sq[i] * a.inv_h + a.eps);
+            if (EPI == ROPE) {
+                const Append& ap = a.ap;
+                const int pos = of_row.pos[i];
+                const int page =
+                    ap.ptab[of_row.slot[i] * ap.maxp + pos / ap.psz];
+                row_pos[r] = pos;
+                row_kv[r] = page * ap.nkl * ap.psz + pos % ap.psz;
+            }
+        }
+        if (EPI == GATED || EPI == ROPE)
+            if (a.rstd_nt > 1)
+                for (int r = threadIdx.x >> 3; r < HM * 32; r += 32) {
+                    const float* p =
+                        a.rstd + (int64_t)min(m * HM * 32 + r, a.M - 1)
+                                     * a.rstd_nt;
+                    float s = 0.f;
+                    #pragma unroll 4
+                    for (int e = threadIdx.x & 7; e < a.rstd_nt; e += 8)
+                        s += p[e];
+                    s += __shfl_xor(s, 1, 64);
+                    s += __shfl_xor(s, 2, 64);
+                    s += __shfl_xor(s, 4, 64);
+                    if ((threadIdx.x & 7) == 0)
+                        row_f[r] = rsqrtf(s * a.inv_h + a.eps);
+                }
+    };
+    ask_rows(m);
+    keep_rows(m);
+    wait_loads<PER * (STAGES - 1)>();
+    asm volatile("s_barrier" ::: "memory");
+    #pragma unroll
+    for (int i = 0; i < NF; i++) read(0, ic<0>{}, i);
+
+    for (;;) {
+        const int next_id = item_at(first + G);
+        int m1 = m, n1 = n, k1 = k, p0 = q0, p1 = q1;
+        if (next_id >= 0) tile_at(next_id, m1, n1, k1, p0, p1);
+        for (int q = q0; q < q1; q++) {
+            if (q == q1 - 1) {
+                if (next_id >= 0) point(m1, n1, p0);
+                else voff -= STAGES * 2048;    // once more, for nobody
+            }
+            each<STAGES>(slab);
+        }
+
+        // A lane has row in_strip(.., r16) of every 16 rows and the columns
+        // from in_strip(.., 4 * g4) on of every 16 columns, four of them.
+        // Worked out anew for each tile: kept through the loop they would be
+        // spilled, and a reload waits for every store before it.
+        int here = lane;
+        asm volatile("" : "+v"(here));
+        const int r16 = here & 15, g4 = here >> 4;
+        if (next_id >= 0) ask_rows(m1);
+        auto row_in = [&](int i) {         // within the tile
+            const int h = wm * HM + i;
+            return (h >> 1) * 32 + in_strip(h & 1, r16);
+        };
+        const int nh = a.N >> 4;           // halves of columns
+        const int hj0 = n * HN * 2 + wn * HN;
+        const int live = min(HN, nh - hj0);    // of this wave's
+        if constexpr (EPI == PARTS) {
+            const int mh = ms * 2, hi0 = m * HM * 2 + wm * HM;
+            float* out = a.part + (((int64_t)k * mh + hi0) * nh + hj0) * 256
+                         + here * 4;
+            #pragma unroll
+            for (int i = 0; i < HM; i++, out += nh * 256)
+                if (hi0 + i < mh) {
+                    #pragma unroll
+                    for (int j = 0; j < HN; j++)
+                        if (j < live)
+                            *reinterpret_cast<f32x4*>(out + j * 256) =
+                                acc[i][j];
+                }
+        } else if constexpr (EPI == RESIDUAL) {
+            // halves of columns are 256 elements apart, strips 1024
+            const char* res = reinterpret_cast<const char*>(a.res);
+            char* y = reinterpret_cast<char*>(a.y);
+            // from a strip's first half; a wave without columns reads others'
+            const int rel = live > 0 ? hj0 & 1 : 0;
+            const int even = live > 0 ? hj0 - rel : 0;
+            auto offset = [&](int i) {
+                const int r = min(m * HM * 32 + row_in(i), a.M - 1);
+                return (uint32_t)(frag_at(r, even * 16
+                                          + in_strip(0, 4 * g4), a.N) * 2);
+            };
+            auto at = [&](int j) {
+                const int h = rel + j;
+                return (h >> 1) * 2048 + (h & 1) * 512;
+            };
+            constexpr int AHEAD = 3;
+            bf16x4 old[AHEAD][HN];
+            auto fetch = [&](int b, int i) {
+                const char* p = res + offset(i);
+                #pragma unroll
+                for (int j = 0; j < HN; j++)
+                    old[b][j] = *reinterpret_cast<const bf16x4*>(
+                        p + at(max(min(j, live - 1), 0)));
+            };
+            #pragma unroll
+            for (int i = 0; i + 1 < AHEAD; i++) fetch(i, i);
+            float sums[HM];
+            #pragma unroll
+            for (int i = 0; i < HM; i++) {
+                if (i + AHEAD - 1 < HM)
+                    fetch((i + AHEAD - 1) % AHEAD, i + AHEAD - 1);
+                const bool ok = m * HM * 32 + row_in(i) < a.M;
+                char* p = y + offset(i);
+                float s2 = 0.f;
+                #pragma unroll
+                for (int j = 0; j < HN; j++) {
+                    f32x4 v = acc[i][j];
+                    #pragma unroll
+                    for (int e = 0; e < 4; e++) v[e] += (float)old[i % AHEAD][j][e];
+                    if (ok && j < live) {
+                        put4(reinterpret_cast<bf16*>(p + at(j)), v);
+                        #pragma unroll
+                        for (int e = 0; e < 4; e++) s2 += v[e] * v[e];
+                    }
+                }
+                s2 += __shfl_xor(s2, 16, 64);
+                sums[i] = s2 + __shfl_xor(s2, 32, 64);
+                __builtin_amdgcn_sched_barrier(0);     // registers
+            }
+            // the two waves of a row
+            if (wn && g4 == 0)
+                #pragma unroll
+                for (int i = 0; i < HM; i++) row_f[row_in(i)] = sums[i];
+            lds_barrier();
+            if (!wn && g4 == 0)
+                #pragma unroll
+                for (int i = 0; i < HM; i++) {
+                    const int r = m * HM * 32 + row_in(i);
+                    if (r < a.M)
+                        a.sq[(int64_t)r * a.nt + n] =
+                            sums[i] + row_f[row_in(i)];
+                }
+        } else {
+            // Two accumulators at a time: after the swap one holds first
+            // halves (gates, low dimensions), the other the second, of the
+            // first accumulator on lower lanes and of the second on upper.
+            const int c4 = (g4 & 1) * 4;
+            const bool upper = g4 >> 1;
+            float rs[HM];
+            #pragma unroll
+            for (int i = 0; i < HM; i++) rs[i] = row_f[row_in(i)];
+            auto pair = [&](int i0, int j0, int i1, int j1, f32x4& lo,
+                            f32x4& hi) {
+                lo = acc[i0][j0] * rs[i0];
+                hi = acc[i1][j1] * rs[i1];
+                swap32(lo, hi);
+            };
+            // accumulators two by two: of a row, then the last of two rows
+            constexpr int ROW = HN / 2, ENDS = HN & 1 ? (HM + 1) / 2 : 0;
+            if constexpr (EPI == GATED) {
+                char* y = reinterpret_cast<char*>(a.y);
+                auto offset = [&](int i) {
+                    const int r = min(m * HM * 32 + row_in(i), a.M - 1);
+                    return (uint32_t)(frag_at(r, hj0 * 8 + c4, a.N >> 1) * 2);
+                };
+                auto put = [&](char* p, bool ok, const f32x4& lo,
+                               const f32x4& hi) {
+                    f32x4 v;
+                    #pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const float z = a.gelu ? gelu_arg(lo[e]) : lo[e];
+                        v[e] = lo[e] * __builtin_amdgcn_rcpf(1.f + __expf(-z))
+                               * hi[e];
+                    }
+                    if (ok) put4(reinterpret_cast<bf16*>(p), v);
+                };
+                #pragma unroll
+                for (int i = 0; i < HM; i++) {
+                    const bool ok = m * HM * 32 + row_in(i) < a.M;
+                    char* p = y + offset(i) + upper * 512;
+                    #pragma unroll
+                    for (int j = 0; j < 2 * ROW; j += 2) {
+                        f32x4 lo, hi;
+                        pair(i, j, i, j + 1, lo, hi);
+                        put(p + j * 512, ok && j + upper < live, lo, hi);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);     // registers
+                }
+                #pragma unroll
+                for (int e = 0; e < ENDS; e++) {
+                    const int i0 = 2 * e, i1 = min(i0 + 1, HM - 1);
+                    f32x4 lo, hi;
+                    pair(i0, HN - 1, i1, HN - 1, lo, hi);
+                    const int i = upper ? i1 : i0;
+                    put(y + (upper ? offset(i1) : offset(i0)) + (HN - 1) * 512,
+                        m * HM * 32 + (upper ? row_in(i1) : row_in(i0)) < a.M
+                            && HN <= live && !(upper && i1 == i0), lo, hi);
+                }
+            } else {
+                // A strip is one head's: a quarter of its pairs, or of its
+                // values.
+                static_assert(HN % 2 == 0);
+                const Append& ap = a.ap;
+                const int qt = ap.nl * 4, kt = ap.nkl * 4, t0 = hj0 >> 1;
+                const int c = upper * 8 + c4;
+                bf16x4 bias[ROW][2];
+                if (a.bias)
+                    #pragma unroll
+                    for (int j = 0; j < ROW; j++) {
+                        const bf16* b = a.bias + min(t0 + j, ns - 1) * 32 + c;
+                        bias[j][0] = *reinterpret_cast<const bf16x4*>(b);
+                        bias[j][1] = *reinterpret_cast<const bf16x4*>(b + 16);
+                    }
+                f32x4 turn[2][ROW][2];
+                auto fetch = [&](int b, int i) {
+                    const uint32_t o = row_pos[row_in(i)] * 64 + c;
+                    #pragma unroll
+                    for (int j = 0; j < ROW; j++) {
+                        const int d = (t0 + j & 3) * 16;
+                        turn[b][j][0] =
+                            *reinterpret_cast<const f32x4*>(ap.cos_t + d + o);
+                        turn[b][j][1] =
+                            *reinterpret_cast<const f32x4*>(ap.sin_t + d + o);
+                    }
+                };
+                fetch(0, 0);
+                #pragma unroll
+                for (int i = 0; i < HM; i++) {
+                    if (i + 1 < HM) fetch((i + 1) & 1, i + 1);
+                    const int row = m * HM * 32 + row_in(i);
+                    const int64_t kv = (int64_t)row_kv[row_in(i)] * 128 + c;
+                    const uint32_t q = row * a.N + c;
+                    #pragma unroll
+                    for (int j = 0; j < ROW; j++) {
+                        f32x4 lo, hi;
+                        pair(i, 2 * j, i, 2 * j + 1, lo, hi);
+                        if (a.bias)
+                            #pragma unroll
+                            for (int e = 0; e < 4; e++) {
+                                lo[e] += (float)bias[j][0][e];
+                                hi[e] += (float)bias[j][1][e];
+                            }
+                        const int t = t0 + j;
+                        if (t >= ns) continue;
+                        if (t >= qt + kt) {        // values as they are
+                            const int s = t - qt - kt;
+                            bf16* p = ap.vp + (s >> 2) * ap.psz * 128
+                                      + (s & 3) * 32;
+                            if (row < a.M) {
+                                put4(p + kv, lo);
+                                put4(p + kv + 16, hi);
+                            }
+                            continue;
+                        }
+                        const f32x4 co = turn[i & 1][j][0];
+                        const f32x4 si = turn[i & 1][j][1];
+                        const f32x4 u = lo * co - hi * si;
+                        const f32x4 v = hi * co + lo * si;
+                        const int s = t < qt ? t : t - qt, d = (s & 3) * 16;
+                        if (row >= a.M) continue;
+                        if (t < qt) {
+                            bf16* p = a.y + (s >> 2) * 128 + d;
+                            put4(p + q, u);
+                            put4(p + q + 64, v);
+                        } else {
+                            bf16* p = ap.kp + (s >> 2) * ap.psz * 128 + d;
+                            put4(p + kv, u);
+                            put4(p + kv + 64, v);
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);     // registers
+                }
+            }
+        }
+        if (next_id >= 0) {
+            lds_barrier();                 // every wave has read its rows
+            keep_rows(m1);
+        }
+        // Stores count as loads do: none may be under way when the next tile
+        // counts its own.  By then its first slabs have landed too.
+        wait_loads<0>();
+        if (next_id < 0) return;
+        first += G;
+        m = m1, n = n1, k = k1, q0 = p0, q1 = p1;
+        #pragma unroll
+        for (int i = 0; i < HM; i++)
+            #pragma unroll
+            for (int j = 0; j < HN; j++) acc[i][j] = f32x4{};
+        // read again: 4 (HM + HN) registers less to keep through the epilogue
+        #pragma unroll
+        for (int i = 0; i < NF; i++) read(0, ic<0>{}, i);
+    }
+}
+
+// Sums of a product in parts: y = res + sum of the parts, and sums of squares.
+// A part is [16 rows, in pairs to 32][16 columns] accumulators as k_tile_gemm's
+// lanes hold them.  A block takes 16 rows and a `pieces`-th of the columns:
+// 541 x 4096 in 4 parts, 8 pieces, is 272 blocks that read 35 MB.
+template <int BS>
+__global__ __launch_bounds__(BS) void k_tile_fold(
+    bf16* __restrict__ y, const bf16* __restrict__ res,
+    float* __restrict__ sq, const float* __restrict__ part, int M, int N,
+    int ks)
+{
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int r16 = lane & 15, g4 = lane >> 4;
+    const int hi = blockIdx.x, pieces = gridDim.y;
+    const int mh = gridDim.x, nh = N >> 4;
+    const int row = (hi >> 1) * 32 + in_strip(hi & 1, r16);
+    const int from = nh * blockIdx.y / pieces;
+    const int to = nh * (blockIdx.y + 1) / pieces;
+    float s2 = 0.f;
+    for (int j = from + wid; j < to; j += BS / 64) {
+        const float* p = part + ((int64_t)hi * nh + j) * 256 + lane * 4;
+        const int64_t step = (int64_t)mh * nh * 256;
+        f32x4 v = *reinterpret_cast<const f32x4*>(p);
+        for (int k = 1; k < ks; k++)
+            v += *reinterpret_cast<const f32x4*>(p + k * step);
+        if (row >= M) continue;
+        const int col = (j >> 1) * 32 + in_strip(j & 1, 4 * g4);
+        const int64_t o = frag_at(row, col, N);
+        v += get4(res + o);
+        put4(y + o, v);
+        #pragma unroll
+        for (int e = 0; e < 4; e++) s2 += v[e] * v[e];
+    }
+    s2 += __shfl_xor(s2, 16, 64);
+    s2 += __shfl_xor(s2, 32, 64);
+    __shared__ float sum[BS / 64][16];
+    if (lane < 16) sum[wid][lane] = s2;
+    __syncthreads();
+    if (threadIdx.x < 16 && row < M) {
+        float s = 0.f;
+        #pragma unroll
+        for (int w = 0; w < BS / 64; w++) s += sum[w][threadIdx.x];
+        sq[(int64_t)row * pieces + blockIdx.y] = s;
+    }
+}
+
+// parts of sums of squares of a row, added up: eight lanes a row
+__global__ __launch_bounds__(256) void k_row_sums(
+    float* __restrict__ out, const float* __restrict__ in, int M, int nt)
+{
+    const int r = blockIdx.x * 32 + (threadIdx.x >> 3);
+    float s = 0.f;
+    if (r < M)
+        #pragma unroll 4
+        for (int e = threadIdx.x & 7; e < nt; e += 8)
+            s += in[(int64_t)r * nt + e];
+    s += __shfl_xor(s, 1, 64);
+    s += __shfl_xor(s, 2, 64);
+    s += __shfl_xor(s, 4, 64);
+    if (r < M && (threadIdx.x & 7) == 0) out[r] = s;
+}
+
+template <int EPI>
+int launch(TileArgs a, int hm, int hn, int cus, hipStream_t stream)
+{
+    const int items = a.mt * a.nt * a.ks;
+    const int lds = tile_lds(hm, hn);
+    // blocks that live together: LDS holds two of the smallest tile
+    const int room = cus * (2 * lds <= 160 * 1024 ? 2 : 1);
+    const int grid = (items < room ? items + 7 : room) / 8 * 8;
+    auto go = [&](auto k) {
+        const hipError_t e = hipFuncSetAttribute(
+            (const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return (int)e;
+        // A block of several tiles waits for its rows' sums with each, 1.5 us; one
+        // launch for all of them takes 3.  Of one tile it waits for loads anyway.
+        if ((EPI == GATED || EPI == ROPE) && items > grid && a.rstd_nt > 1) {
+            k_row_sums<<<(a.M + 31) / 32, 256, 0, stream>>>(a.part, a.rstd, a.M,
+                                                            a.rstd_nt);
+            a.rstd = a.part;
+            a.rstd_nt = 1;
+        }
+        k<<<grid, 256, lds, stream>>>(a);
+        return (int)hipGetLastError();
+    };
+    #define TILE(A, B) \
+        if (hm == A && hn == B) return go(k_tile_gemm<A, B, EPI>)
+    TILE(8, 8);
+    if constexpr (EPI != ROPE) TILE(9, 7);
+    TILE(8, 6);
+    TILE(6, 6);
+    TILE(8, 4);
+    TILE(6, 4);
+    TILE(4, 4);
+    TILE(4, 2);
+    #undef TILE
+    return -110;                            // no such tile
+}
+
+}  // namespace
+
+// Tiles are hm x hn times 32 rows and columns.  epi: RESIDUAL (y = res + x W^T,
+// sq), GATED (y = act(gate) * up of normed x), ROPE (normed x, positions, keys
+// and values appended) or PARTS (y and sq come from part, ks parts of K).
+extern "C" int tile_gemm_bf16(
+    void* y, void* part, const void* x, const void* w, const void* bias,
+    const void* res, void* sq, const void* rstd, int rstd_nt, float inv_h,
+    float eps, int M, int N, int K, int epi, int hm, int hn, int ks, int gm,
+    int pieces, int gelu, int cus, const void* rcos, const void* rsin,
+    const void* pos, const void* slot, const void* ptab, void* kp, void* vp,
+    int nl, int nkl, int psz, int maxp, hipStream_t stream)
+{
+    const int unit = 32 * tile_stages(hm, hn);     // of K
+    if (M < 1 || N < 32 || N % 32 || K < unit || K % unit || ks < 1
+        || ks > K / unit || (int64_t)(M + 31) * N >= (int64_t)1 << 31 || gm < 1 || cus < 8 || (epi != PARTS && ks != 1)
+        || (epi == ROPE && N != (nl + 2 * nkl) * 128))
+        return -111;
+    TileArgs a{(bf16*)y, (float*)part, (const bf16*)x, (const bf16*)w,
+               (const bf16*)bias, (const bf16*)res, (float*)sq,
+               (const float*)rstd, rstd_nt, inv_h, eps, M, N, K,
+               (M + hm * 32 - 1) / (hm * 32), (N + hn * 32 - 1) / (hn * 32),
+               ks, gm, gelu,
+               {(const float*)rcos, (const float*)rsin, (const int*)pos,
+                (const int*)slot, (const int*)ptab, (bf16*)kp, (bf16*)vp,
+                nl, nkl, psz, maxp}};
+    if (epi == RESIDUAL) return launch<RESIDUAL>(a, hm, hn, cus, stream);
+    if (epi == GATED) return launch<GATED>(a, hm, hn, cus, stream);
+    if (epi == ROPE) return launch<ROPE>(a, hm, hn, cus, stream);
+    if (const int e = launch<PARTS>(a, hm, hn, cus, stream)) return e;
+    k_tile_fold<256><<<dim3((M + 31) / 32 * 2, pieces), 256, 0, stream>>>(
+        (bf16*)y, (const bf16*)res, (float*)sq, (const float*)part, M, N, ks);
+    return (int)hipGetLastError();
+}

@@ -395,6 +395,12 @@ class LlamaModel:
                      or 0 < idx.shape[0] <= ops.CHAIN_ROWS)):
             return self._forward_fused(tokens, positions, kv_cache,
                                        slot_ids, attn_meta)
+        if (chain and tokens.shape[0] > ops.CHAIN_ROWS
+                and not attn_meta.one_each and idx is not None
+                and 0 < idx.shape[0] <= ops.CHAIN_ROWS
+                and self._tiles_take(tokens.shape[0])):
+            return self._forward_tiles(tokens, positions, kv_cache,
+                                       slot_ids, attn_meta)
         x = ops.embedding(tokens, self.embed)
         residual = None
         for li, layer in enumerate(self.layers):
@@ -515,3 +521,41 @@ class LlamaModel:
                                 self.lm_head.shape[0], rstd=sq_a,
                                 rstd_nt=nt, inv_h=inv_h, eps=eps,
                                 K=H, xlds=2, M_frag=B)
+
+    def _tiles_take(self, T):
+        H, d, l = self.cfg.hidden, self.cfg.head_dim, self.layers[0]
+        return (ops.tiles_take(T, l.wqkv.shape[0], H)
+                and ops.tiles_take(T, H, self.n_local_heads * d)
+                and ops.tiles_take(T, l.wgate_up.shape[0], H)
+                and ops.tiles_take(T, H, l.wdown.shape[1]))
+
+    def _forward_tiles(self, tokens, positions, kv_cache, slot_ids,
+                       attn_meta):
+        """_forward_fused for prompts of more rows than its products take:
+        the same chain, its products over tiles of rows and columns."""
+        cfg = self.cfg
+        B, H = tokens.shape[0], cfg.hidden
+        nl, nkl, d = self.n_local_heads, self.n_local_kv_heads, cfg.head_dim
+        inv_h, eps = 1.0 / H, cfg.norm_eps
+        # tickets of single tokens' attention in parts
+        tickets = torch.empty(max(1, attn_meta.n_single * nkl),
+                              dtype=torch.int32, device=self.embed.device)
+        res, sq = ops.fragify_sumsq(self.embed, tokens=tokens, clear=tickets)
+        nt = 1
+        for li, layer in enumerate(self.layers):
+            qkv = ops.tile_qkv_rope(
+                res, layer.wqkv_pk, B, layer.wqkv.shape[0], H, layer.bqkv_rp,
+                kv_cache, li, positions, slot_ids, self.rope_cos,
+                self.rope_sin, nl, nkl, sq, nt, inv_h, eps)
+            q = qkv[:, :nl * d].view(-1, nl, d)
+            attn = ops.attention_frag(q, kv_cache, li, attn_meta, tickets)
+            sq, nt = ops.tile_residual(attn, layer.wo_pk, B, H, nl * d, res)
+            act = ops.tile_gu(res, layer.wgu_pk, B, layer.wgate_up.shape[0],
+                              H, sq, nt, inv_h, eps)
+            sq, nt = ops.tile_residual(act, layer.wdown_pk, B, H,
+                                       layer.wdown.shape[1], res)
+        res, sq = ops.frag_rows(res, attn_meta.logits_idx, H, B)
+        return ops.linear_fused(res, self.lm_head_pk, self.lm_head.shape[0],
+                                rstd=sq, rstd_nt=1, inv_h=inv_h, eps=eps,
+                                K=H, xlds=2,
+                                M_frag=attn_meta.logits_idx.shape[0])

@@ -8,6 +8,8 @@ extension is a hard error — ops never fall back silently to eager PyTorch
 from __future__ import annotations
 
 import ctypes
+import functools
+import math
 import os
 from typing import NamedTuple, Optional
 
@@ -63,6 +65,8 @@ def _try_load():
     lib.wstream_pure_bf16.argtypes = [vp, vp, i, i, i, vp]
     lib.wstream_gu_bf16.argtypes = [vp, vp, vp, i, i, i, i64, i,
                                     vp, i, f, f, i, i, vp]
+    lib.tile_gemm_bf16.argtypes = [*[vp] * 8, i, f, f, *[i] * 11, *[vp] * 7,
+                                   i, i, i, i, vp]
     lib.row_sumsq_bf16.argtypes = [vp, vp, i, i, vp]
     lib.frag_rows_bf16.argtypes = [vp, vp, vp, vp, i, i, i, vp]
     lib.fragify_sumsq_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i, i, i, vp, i,
@@ -636,6 +640,110 @@ def linear_qkv_rope(x, packed, N, bias_rp, cache, layer, positions,
         _p(cos), _p(sin), _p(pos32), _p(slot32), _p(cache.page_table),
         kp, vp, nl, nkl, cache.page_size, cache.page_table.shape[1],
         xf, _stream()), "wstream_qkv_rope")
+    return y
+
+
+# Products of many rows (tile_gemm.hip): tiles in units of 32 rows and columns
+TILES = ((8, 8), (9, 7), (8, 6), (6, 6), (8, 4), (6, 4), (4, 4), (4, 2))
+TILE_RESIDUAL, TILE_GATED, TILE_ROPE, TILE_PARTS = range(4)
+TILE_FOLD = 8             # blocks that add up the parts of a row
+
+
+@functools.lru_cache(maxsize=4096)
+def tile_plan(M, N, K, epi, cus=256):
+    """(rows, columns, parts of K) of the tiles for which the time of a product
+    is least, as estimated: the larger of what the busiest CU takes, a slab of
+    32 of K being bound by its products or its loads; of what all padded work
+    draws at the power limit; and of reading the weights.  Parts cost a second
+    launch, which reads them.  us, fitted to 2900 times of 65 to 8100 rows and
+    11 matrices (3584 to 37888 columns); what it chooses takes 1 % more than
+    the best choice on average."""
+    best, least = None, math.inf
+    for hm, hn in TILES:
+        unit = 256 if hm + hn <= 8 else 128
+        if K % unit or (epi == TILE_ROPE and hn % 2):
+            continue
+        tiles, area = -(-M // (32 * hm)) * -(-N // (32 * hn)), hm * hn
+        for ks in range(1, 9 if epi == TILE_RESIDUAL else 2):
+            if ks > 1 and (tiles * ks > 2.5 * cus or K // unit < 2 * ks):
+                break
+            slabs = -(-K // unit // ks) * unit / 32
+            rounds = -(-tiles * ks // cus)
+            slab = max(area * 0.0079, (hm + hn) * 0.0235)
+            t = max(rounds * (slabs * slab + 2.2 + area * 0.16),
+                    tiles * ks * area / cus * (slabs * 0.0088 + 0.16),
+                    N * K * 4e-7)
+            if ks > 1:
+                t += 10.6 + ks * M * N * 1.4e-6
+            if t < least:
+                best, least = (hm, hn, ks), t
+    return best
+
+
+def tiles_take(M, N, K):
+    """The products over tiles take M rows of x [M, K] and W [N, K]."""
+    return N % 64 == 0 and K % 128 == 0 and (M + 31) * max(N, K) < 2 ** 31
+
+
+def _tile_gemm(epi, y, x, packed, M, N, K, plan, part=None, bias=None,
+               res=None, sq=None, rstd=None, rstd_nt=0, inv_h=0.0, eps=0.0,
+               gelu=0, rope=(None,) * 7 + (0,) * 4):
+    hm, hn, ks = plan
+    if rstd_nt > 1:
+        part = torch.empty(M, dtype=torch.float32, device=x.device)
+    assert x.numel() >= -(-M // 32) * 32 * K and packed.numel() == N * K
+    _check(_lib.tile_gemm_bf16(
+        _p(y), _p(part), _p(x), _p(packed), _p(bias), _p(res), _p(sq),
+        _p(rstd), rstd_nt, float(inv_h), float(eps), M, N, K, epi, hm, hn, ks,
+        8, TILE_FOLD, gelu, _cus(x.device.index), *rope, _stream()),
+        "tile_gemm")
+
+
+@functools.lru_cache(maxsize=None)
+def _cus(index):
+    return torch.cuda.get_device_properties(index).multi_processor_count
+
+
+def tile_gu(x, packed, M, N, K, rstd, rstd_nt, inv_h, eps, glu="silu",
+            plan=None):
+    """As linear_gu over fragments, for many rows: act(gate) * up of the
+    normed rows of x."""
+    act = torch.empty(-(-M // 32) * 32 * (N // 2), dtype=x.dtype,
+                      device=x.device)
+    _tile_gemm(TILE_GATED, act, x, packed, M, N, K,
+               plan or tile_plan(M, N, K, TILE_GATED), rstd=rstd,
+               rstd_nt=rstd_nt, inv_h=inv_h, eps=eps, gelu=GELU[glu])
+    return act
+
+
+def tile_residual(x, packed, M, N, K, res, plan=None):
+    """res += x W^T in place, all in fragment layout, for many rows; returns
+    partial sums of squares of the new rows and how many a row has."""
+    plan = plan or tile_plan(M, N, K, TILE_RESIDUAL)
+    ks, part, epi = plan[2], None, TILE_RESIDUAL
+    if ks > 1:
+        part = torch.empty(ks * -(-M // 32) * 32 * N, dtype=torch.float32,
+                           device=x.device)
+        epi = TILE_PARTS
+    nt = TILE_FOLD if ks > 1 else -(-N // (plan[1] * 32))
+    sq = torch.empty(M, nt, dtype=torch.float32, device=x.device)
+    _tile_gemm(epi, res, x, packed, M, N, K, plan, part=part, res=res, sq=sq)
+    return sq, nt
+
+
+def tile_qkv_rope(x, packed, M, N, K, bias_rp, cache, layer, positions,
+                  slots, cos, sin, nl, nkl, rstd, rstd_nt, inv_h, eps,
+                  plan=None):
+    """As linear_qkv_rope over fragments, for many rows."""
+    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    kp, vp = _layer_ptrs(cache, layer)
+    pos32, slot32 = _i32(positions), _i32(slots)
+    _tile_gemm(TILE_ROPE, y, x, packed, M, N, K,
+               plan or tile_plan(M, N, K, TILE_ROPE), bias=bias_rp, rstd=rstd,
+               rstd_nt=rstd_nt, inv_h=inv_h, eps=eps,
+               rope=(_p(cos), _p(sin), _p(pos32), _p(slot32),
+                     _p(cache.page_table), kp, vp, nl, nkl, cache.page_size,
+                     cache.page_table.shape[1]))
     return y
 
 

@@ -828,6 +828,36 @@ def qkv_rope_fused(x, packed, N, bias_rp, cache, layer, positions, slots,
                                M_real=M_real)
 
 
+# ---- the same chain over tiles of many rows -----------------------------
+
+def tiles_take(M, N, K):
+    """Products over tiles take M rows of a product [M, K] x [N, K]."""
+    from . import hip
+    return hip.tiles_take(M, N, K)
+
+
+def tile_qkv_rope(x, packed, M, N, K, bias_rp, cache, layer, positions, slots,
+                  cos, sin, nl, nkl, rstd, rstd_nt, inv_h, eps):
+    """rmsnorm -> qkv GEMM -> RoPE -> paged KV append, one kernel."""
+    from . import hip
+    return hip.tile_qkv_rope(x, packed, M, N, K, bias_rp, cache, layer,
+                             positions, slots, cos, sin, nl, nkl, rstd,
+                             rstd_nt, inv_h, eps)
+
+
+def tile_residual(x, packed, M, N, K, res):
+    """res += x W^T; partial sums of squares of the new rows and how many a
+    row has."""
+    from . import hip
+    return hip.tile_residual(x, packed, M, N, K, res)
+
+
+def tile_gu(x, packed, M, N, K, rstd, rstd_nt, inv_h, eps):
+    """rmsnorm -> gate_up GEMM -> SwiGLU, one kernel."""
+    from . import hip
+    return hip.tile_gu(x, packed, M, N, K, rstd, rstd_nt, inv_h, eps)
+
+
 def sample(logits, temperature, top_k, top_p, generator=None):
     # Sampler: torch ops compose on-GPU; custom fused kernel in ops/hip.py
     # handles the greedy + temperature paths.

@@ -1,0 +1,152 @@
+"""Products of many rows over tiles (tile_gemm.hip) against float64."""
+import math
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from ollamamq_amd.ops import hip
+
+PLANS = [(*t, ks) for t in hip.TILES for ks in (1, 3)]
+
+
+def test_plans_are_possible():
+    """What is chosen is a tile that the kernel has and parts that K has."""
+    for M in (129, 130, 300, 541, 2317, 8192):
+        for N, K in ((64, 128), (448, 384), (4096, 14336), (37888, 3584)):
+            for epi in (hip.TILE_RESIDUAL, hip.TILE_GATED, hip.TILE_ROPE):
+                hm, hn, ks = hip.tile_plan(M, N, K, epi)
+                unit = 256 if hm + hn <= 8 else 128
+                assert (hm, hn) in hip.TILES and K % unit == 0
+                assert 1 <= ks <= K // unit
+                assert epi == hip.TILE_RESIDUAL or ks == 1
+                assert epi != hip.TILE_ROPE or hn % 2 == 0
+
+
+def frag(x):
+    rows = -(-x.shape[0] // 32) * 32
+    f = x.new_full((rows, x.shape[1]), math.nan)   # what no row may see
+    f[:len(x)] = x
+    return f.view(rows // 32, 32, -1, 8).transpose(1, 2).flatten()
+
+
+def unfrag(f, rows, cols):
+    return f.view(-1, cols // 8, 32, 8).transpose(1, 2).reshape(-1, cols)[:rows]
+
+
+def rand(*shape, scale=1.0):
+    return (torch.randn(*shape, device="cuda") * scale).bfloat16()
+
+
+def off(a, b):
+    return ((a.double() - b).norm() / b.norm()).item()
+
+
+# One rounding to bf16, half a step of 2^-7 at most of every value, of fp32 sums: K / 32 steps
+# of up to K terms, together sqrt(K) times the result, each rounded to 2^-24 of
+# it, are 2^-14 for K = 1024; twice that for the product of two such sums.
+ROUNDED = 2 ** -8 + 2 ** -13
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("plan", PLANS, ids=str)
+@pytest.mark.parametrize("M, N, K", [
+    (1, 64, 768), (32, 64, 768), (33, 448, 768), (129, 576, 768),
+    (577, 64, 1024), (2500, 3072, 768)])
+def test_product(plan, M, N, K):
+    """Rows and columns around the edges of tiles; the last in several rounds
+    of blocks."""
+    hip.require()
+    torch.manual_seed(M + N)
+    x, w, eps = rand(M, K), rand(N, K, scale=K ** -0.5), 1e-5
+    xf, y = frag(x), x.double() @ w.double().T
+    res = rand(M, N)
+    rf = frag(res)
+    sq, nt = hip.tile_residual(xf, hip.pack_weight(w), M, N, K, rf, plan=plan)
+    assert off(unfrag(rf, M, N), y + res.double()) < ROUNDED
+    # fp32 sums of squares of at most 2^12 values before their rounding
+    assert sq.shape == (M, nt)
+    assert off(sq.sum(1), (y + res.double()).square().sum(1)) < 2 ** -18
+    if plan[2] > 1:
+        return
+    for nt in (1, 3, 40):
+        sq = (torch.rand(M, nt, device="cuda") + 0.5) * (K / nt)
+        scale = (sq.double().sum(1) / K + eps).rsqrt()[:, None]
+        for glu in ("silu", "gelu_tanh"):
+            act = hip.tile_gu(xf, hip.pack_weight_gu(w), M, N, K, sq, nt,
+                              1.0 / K, eps, glu, plan=plan)
+            g, u = (y * scale).chunk(2, 1)
+            g = (torch.nn.functional.silu(g) if glu == "silu" else
+                 torch.nn.functional.gelu(g, approximate="tanh"))
+            assert off(unfrag(act, M, N // 2), g * u) < ROUNDED
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("plan", [p for p in hip.TILES if p[1] % 2 == 0],
+                         ids=str)
+@pytest.mark.parametrize("M, nl, nkl, page, bias", [
+    (1, 1, 1, 16, False), (131, 4, 2, 16, True), (300, 7, 1, 48, True),
+    (2500, 32, 4, 64, False)])
+def test_rotated(plan, M, nl, nkl, page, bias):
+    hip.require()
+    torch.manual_seed(M)
+    K, slots, eps = 256, 3, 1e-5
+    N, per = (nl + 2 * nkl) * 128, -(-(M // slots + 9) // page)
+    n_pages = slots * per + 1
+    w = rand(N, K, scale=K ** -0.5)
+    b = rand(N) if bias else None
+    x = rand(M, K)
+    # a buffer of its own for each, so that a stray write shows
+    cache = SimpleNamespace(
+        n_kv_heads=nkl, page_size=page,
+        k_pool=torch.zeros(2, n_pages, nkl, page, 128, device="cuda",
+                           dtype=torch.bfloat16),
+        page_table=torch.randperm(n_pages, device="cuda")[:slots * per]
+        .view(slots, per).int().contiguous())
+    cache.v_pool = torch.zeros_like(cache.k_pool)
+    pos = torch.arange(M, device="cuda").int() // slots + 5
+    slot = torch.arange(M, device="cuda").int() % slots
+    angle = torch.rand(per * page, 64, device="cuda") * 6
+    cos, sin = angle.cos(), angle.sin()
+    sq = (torch.rand(M, 9, device="cuda") + 0.5) * (K / 9)
+    order = torch.tensor(hip.qkv_rope_order(nl, nkl), device="cuda")
+    q = hip.tile_qkv_rope(
+        frag(x), hip.pack_weight_qkv_rope(w, nl, nkl), M, N, K,
+        b[order].contiguous() if bias else None, cache, 1, pos, slot, cos,
+        sin, nl, nkl, sq, 9, 1.0 / K, eps, plan=(*plan, 1))
+    y = x.double() @ w.double().T
+    y *= (sq.double().sum(1) / K + eps).rsqrt()[:, None]
+    if bias:
+        y += b.double()
+    wq, wk, wv = (t.unflatten(1, (-1, 128)) for t in
+                  y.split([nl * 128, nkl * 128, nkl * 128], 1))
+
+    def turn(t):
+        c, s = (f[pos.long()].double()[:, None] for f in (cos, sin))
+        lo, hi = t.chunk(2, -1)
+        return torch.cat([lo * c - hi * s, hi * c + lo * s], -1)
+
+    at = cache.page_table[slot.long(), pos.long() // page].long()
+    place = pos.long() % page
+    assert off(q[:, :nl * 128].unflatten(1, (-1, 128)), turn(wq)) < ROUNDED
+    assert off(cache.k_pool[1][at, :, place], turn(wk)) < ROUNDED
+    assert off(cache.v_pool[1][at, :, place], wv) < ROUNDED
+    for pool in (cache.k_pool, cache.v_pool):
+        assert not pool[0].any()
+        pool[1][at, :, place] = 0
+        assert not pool[1].any()
+
+
+def test_refused():
+    lib = hip._lib if hip.available() else None
+    if lib is None:
+        pytest.skip("the extension is not built")
+    none = [None] * 8
+
+    def call(M=129, N=64, K=256, epi=0, hm=4, hn=4, ks=1):
+        return lib.tile_gemm_bf16(*none, 1, 0.0, 0.0, M, N, K, epi, hm, hn,
+                                  ks, 8, 8, 0, 256, *none[:7], 1, 1, 16, 1,
+                                  None)
+    for bad in (dict(M=0), dict(N=48), dict(K=128), dict(K=192, hm=9, hn=7),
+                dict(ks=2), dict(epi=3, ks=2), dict(hm=5, hn=5), dict(epi=2)):
+        assert call(**bad) < 0
