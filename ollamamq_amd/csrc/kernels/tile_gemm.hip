@@ -228,30 +228,38 @@ __global__ __launch_bounds__(256, 1) void k_tile_gemm(const TileArgs a)
     });
 
     // Operands of a slab: half h of an operand's strips, lanes 16 j .. of it
-    // its columns 8 j ..; a wave's halves may begin inside a strip.
+    // its columns 8 j ..; a wave's halves may begin inside a strip.  Pointers
+    // that the compiler cannot derive from each other, or it adds up an address
+    // for each read between the products (8 x 8 tiles: 1238 clocks a slab of
+    // 1024 for its products, 1174 without).
     constexpr int NF = HM + HN;
     bf16x8 f[2][NF];
-    const int foff = (g4 >> 1) * 1024 + (g4 & 1) * 512 + r16 * 16;
-    const int h0[2] = {wm * HM, wn * HN};
+    typedef const __attribute__((address_space(3))) char* lds_ptr;
+    typedef const __attribute__((address_space(3))) bf16x8* lds_frag;
     // an instruction reaches 64 KB from its pointer
     constexpr int REACH = 65536 / STAGE, POINTERS = (STAGES + REACH - 1) / REACH;
-    const char* at[2][2][POINTERS];        // operand, parity, stages
+    lds_ptr at[2][2][POINTERS];            // operand, parity, stages
     #pragma unroll
     for (int o = 0; o < 2; o++)
         #pragma unroll
         for (int par = 0; par < 2; par++)
             #pragma unroll
             for (int s = 0; s < POINTERS; s++) {
-                const int h = h0[o] + par;
-                at[o][par][s] = smem + foff + o * HM * 2048
+                const int h = (o ? wn * HN : wm * HM) + par;
+                at[o][par][s] = (lds_ptr)smem + (g4 >> 1) * 1024
+                                + (g4 & 1) * 512 + r16 * 16 + o * HM * 2048
                                 + (h >> 1) * 2048 + (h & 1) * 256
                                 + s * REACH * STAGE;
+                if (par == 0 || (o ? HN : HM) & 1)
+                    asm volatile("" : "+v"(at[o][par][s]));
             }
     auto read = [&](int buf, auto st_, int i) {
         constexpr int st = decltype(st_)::value;
         const int o = i >= HM, h = o ? i - HM : i;
-        f[buf][i] = *reinterpret_cast<const bf16x8*>(
-            at[o][h & 1][st / REACH] + st % REACH * STAGE + (h >> 1) * 2048);
+        const bool even = (o ? HN : HM) % 2 == 0;
+        f[buf][i] = *(lds_frag)(
+            at[o][even ? 0 : h & 1][st / REACH] + (even ? (h & 1) * 256 : 0)
+            + st % REACH * STAGE + (h >> 1) * 2048);
     };
     f32x4 acc[HM][HN] = {};
 
