@@ -33,7 +33,10 @@ DEV float pair_max(float x) {
 struct Seen { int first, last, first_lo, first_hi, last_lo, last_hi; };
 
 template <int DK, int DV, int NW, bool VT> struct Flash32 {
-    static constexpr int KT = 64, KS = DK + 8, VS = VT ? KT + 4 : DV + 8;
+    // Rows of K are 4 banks apart from a multiple of 64, whole rows of V 16: a
+    // transpose load takes 64 bytes of each of four (with 4, 55 % of the cycles
+    // of LDS were conflicts).
+    static constexpr int KT = 64, KS = DK + 8, VS = VT ? KT + 4 : DV + 32;
     static constexpr int KB = KT * KS, VB = (VT ? DV : KT) * VS;
     static constexpr int LDS = 2 * (KB + VB) * 2;      // bytes
     static constexpr int NK = DK / 8 / NW, NV = DV / 8 / NW;
@@ -57,20 +60,31 @@ template <int DK, int DV, int NW, bool VT> struct Flash32 {
         }
     }
 
-    // Chunks c_lo .. c_hi - 1.  kat(base, w0, row, c), vat: eight values from
-    // column c of a row on, w0 the first row of the wave's piece (rows are
-    // keys, for transposed values columns); unit: of a score, in octaves.  m:
-    // the row's maximum; l: this lane's sum of weights.
-    template <class K, class V>
-    DEV void walk(bf16* lds, bf16x8* qf, int c_lo, int c_hi,
-                         float unit, K kat, V vat, const Seen& see, float& m,
-                         float& l, f32x16* o)
+    // Chunks c_lo .. c_hi - 1.  page(base, w0): of the wave's piece from row w0
+    // on, also past the last key; kat(base, page, row, c), vat: eight values
+    // from column c of a row on (rows are keys, for transposed values columns);
+    // unit: of a score, in octaves.  m: the row's maximum; l: this lane's sum
+    // of weights.  Pages are looked up a chunk before their loads, which would
+    // wait for them with the products behind them.
+    template <class P, class K, class V>
+    DEV void walk(bf16* lds, bf16x8* qf, int c_lo, int c_hi, float unit,
+                  P page, K kat, V vat, const Seen& see, float& m, float& l,
+                  f32x16* o)
     {
         const int tid = threadIdx.x, lane = tid & 63;
         const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int col = lane & 31, h = lane >> 5;
         constexpr int KC = DK / 8, VC = (VT ? KT : DV) / 8;
         u32x4 kp[NK], vp[NV];
+        int k_page[NK], v_page[NV];
+        auto ask = [&](int base) {
+            #pragma unroll
+            for (int j = 0; j < NK; j++)
+                k_page[j] = page(base, (wid * 64 + j * NW * 64) / KC);
+            #pragma unroll
+            for (int j = 0; j < NV; j++)
+                v_page[j] = page(base, (wid * 64 + j * NW * 64) / VC);
+        };
         // a row's maximum is taken before the unit: it has to be positive
         if (unit < 0.f)
             #pragma unroll
@@ -81,13 +95,13 @@ template <int DK, int DV, int NW, bool VT> struct Flash32 {
         auto load = [&](int base) {
             #pragma unroll
             for (int j = 0; j < NK; j++) {
-                const int u = tid + j * NW * 64, w = wid * 64 + j * NW * 64;
-                kp[j] = kat(base, w / KC, u / KC, u % KC * 8);
+                const int u = tid + j * NW * 64;
+                kp[j] = kat(base, k_page[j], u / KC, u % KC * 8);
             }
             #pragma unroll
             for (int j = 0; j < NV; j++) {
-                const int u = tid + j * NW * 64, w = wid * 64 + j * NW * 64;
-                vp[j] = vat(base, w / VC, u / VC, u % VC * 8);
+                const int u = tid + j * NW * 64;
+                vp[j] = vat(base, v_page[j], u / VC, u % VC * 8);
             }
         };
         auto store = [&](bf16* buf) {
@@ -110,14 +124,19 @@ template <int DK, int DV, int NW, bool VT> struct Flash32 {
                     *reinterpret_cast<u32x4*>(d) = vp[j];
             }
         };
+        ask(c_lo * KT);
         load(c_lo * KT);
+        ask(c_lo * KT + KT);
         store(lds);
         __syncthreads();
         for (int ch = c_lo; ch < c_hi; ch++) {
             const int base = ch * KT;
             const bf16* k_s = lds + ((ch - c_lo) & 1) * (KB + VB);
             const bf16* v_s = k_s + KB;
-            if (ch + 1 < c_hi) load(base + KT);
+            if (ch + 1 < c_hi) {
+                load(base + KT);
+                ask(base + 2 * KT);
+            }
             if (base <= see.last_hi && base + KT > see.first_lo) {
                 f32x16 s[2] = {};
                 #pragma unroll

@@ -1056,6 +1056,7 @@ __global__ __launch_bounds__(512, 2) void k_flash32(
     Flash32<DK, DV, 8, true>::walk(
         reinterpret_cast<bf16*>(smem), qf, first_seen(pos0) / 64,
         (kv_len + 63) / 64, scale * 1.4426950408889634f,
+        [](int, int) { return 0; },
         [&](int base, int, int key, int c) {
             const bf16* src = kh + (int64_t)(base + key) * H * D;
             const bf16* shared = krh + (base + key) * krs;

@@ -5,10 +5,12 @@
 // token * G + head), so a staged key serves all of them, whatever G is.
 // Before, a wave had one head's 32 tokens, weights went through LDS and values
 // were transposed by 2-byte stores (32 heads, 8 of them key/value heads):
-//   8100 tokens, window 4096     1288 us (315 TF), now 456 (891)
-//   2 x 2048                      334 us (205 TF), now 101 (680)
-//   7 prompts, 2310 together       68 us (103 TF), now 26 (270)
-//   2048, 32 / 32 heads          1781 us, now 67
+//   8100 tokens, window 4096     1288 us (315 TF), now 460 (883)
+//   2 x 2048                      334 us (205 TF), now 100 (690)
+//   7 prompts, 2310 together       68 us (103 TF), now 25 (278)
+//   2048, 32 / 32 heads          1781 us, now 66
+// of which values without bank conflicts and pages a chunk ahead are the last
+// steps, one after another on one card: 474, 103, 26 and 72 us before.
 #include "decode_attn.h"
 
 constexpr int D = 128;
@@ -48,11 +50,13 @@ DEV void prefill_block(
     #pragma unroll
     for (int c = 0; c < 8; c++) qf[c] = frag8(qr + c * 16);
     // a wave takes four keys at a time
-    auto at = [&](const bf16* pool, int base, int w0, int k, int c) {
+    auto page_of = [&](int base, int w0) {
+        return SH ? pt[min(base + w0, kv_len - 1) >> pshift] : 0;
+    };
+    auto at = [&](const bf16* pool, int base, int pg, int k, int c) {
         const int key = min(base + k, kv_len - 1);
         int64_t r;
         if (SH) {
-            const int pg = pt[min(base + w0, kv_len - 1) >> pshift];
             r = (((int64_t)pg * KVH + kvh) << pshift) * D
                 + ((key & ((1 << pshift) - 1)) * D + c);
         } else
@@ -67,9 +71,9 @@ DEV void prefill_block(
     f32x16 o[4] = {};
     Flash32<D, D, NW, false>::walk(
         reinterpret_cast<bf16*>(smem), qf, first_seen(p_lo) / KT,
-        (kv_len + KT - 1) / KT, unit,
-        [&](int base, int w, int k, int c) { return at(kpool, base, w, k, c); },
-        [&](int base, int w, int k, int c) { return at(vpool, base, w, k, c); },
+        (kv_len + KT - 1) / KT, unit, page_of,
+        [&](int base, int p, int k, int c) { return at(kpool, base, p, k, c); },
+        [&](int base, int p, int k, int c) { return at(vpool, base, p, k, c); },
         see, m, l, o);
     if (w0 + col > end) return;
     const float f = l > 0.f ? 1.f / l : 0.f;

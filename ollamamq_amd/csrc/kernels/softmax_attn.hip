@@ -317,9 +317,13 @@ __global__ __launch_bounds__(NW * 64, 2) void k_softmax_flash32(
         const int d = c * 16 + h * 8;
         qf[c] = EVEN || d < Dp ? frag8(qr + d) : frag_zero<bf16>();
     }
-    auto at = [&](const bf16* pool, int width, int base, int w, int k, int c) {
+    auto page_of = [&](int base, int w) {
+        return EVEN ? pt[min(base + w, kv_len - 1) >> pshift] : 0;
+    };
+    auto at = [&](const bf16* pool, int width, int base, int page, int k,
+                  int c) {
         const int key = min(base + k, kv_len - 1);
-        const int pg = pt[(EVEN ? min(base + w, kv_len - 1) : key) >> pshift];
+        const int pg = EVEN ? page : pt[key >> pshift];
         const int64_t r = (((int64_t)pg * G + kvh) << pshift)
                           + (key & ((1 << pshift) - 1));
         return EVEN || c < width
@@ -332,11 +336,11 @@ __global__ __launch_bounds__(NW * 64, 2) void k_softmax_flash32(
     Flash32<DK, DV, NW, false>::walk(
         reinterpret_cast<bf16*>(smem), qf,
         first_seen(rule, pos[row0 / R]) / 64, (kv_len + 63) / 64,
-        rule.scale * Expo<bf16>::unit,
-        [&](int base, int w, int k, int c) {
-            return at(kpool, Dp, base, w, k, c); },
-        [&](int base, int w, int k, int c) {
-            return at(vpool, Vp, base, w, k, c); },
+        rule.scale * Expo<bf16>::unit, page_of,
+        [&](int base, int p, int k, int c) {
+            return at(kpool, Dp, base, p, k, c); },
+        [&](int base, int p, int k, int c) {
+            return at(vpool, Vp, base, p, k, c); },
         see, m, l, o);
     if (w0 + col > end) return;
     const float f = finish<bf16>(m, l, rule.sink, head)
