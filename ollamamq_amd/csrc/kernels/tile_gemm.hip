@@ -697,7 +697,9 @@ int launch(TileArgs a, int hm, int hn, int cus, hipStream_t stream)
         if (hm == A && hn == B) return go(k_tile_gemm<A, B, EPI>)
     TILE(8, 8);
     if constexpr (EPI != ROPE) TILE(9, 7);
+    if constexpr (EPI != ROPE) TILE(7, 7);
     TILE(8, 6);
+    TILE(10, 4);
     TILE(6, 6);
     TILE(8, 4);
     TILE(6, 4);

@@ -644,7 +644,8 @@ def linear_qkv_rope(x, packed, N, bias_rp, cache, layer, positions,
 
 
 # Products of many rows (tile_gemm.hip): tiles in units of 32 rows and columns
-TILES = ((8, 8), (9, 7), (8, 6), (6, 6), (8, 4), (6, 4), (4, 4), (4, 2))
+TILES = ((8, 8), (9, 7), (7, 7), (8, 6), (10, 4), (6, 6), (8, 4), (6, 4),
+         (4, 4), (4, 2))
 TILE_RESIDUAL, TILE_GATED, TILE_ROPE, TILE_PARTS = range(4)
 TILE_FOLD = 8             # blocks that add up the parts of a row
 
@@ -652,12 +653,13 @@ TILE_FOLD = 8             # blocks that add up the parts of a row
 @functools.lru_cache(maxsize=4096)
 def tile_plan(M, N, K, epi, cus=256):
     """(rows, columns, parts of K) of the tiles for which the time of a product
-    is least, as estimated: the larger of what the busiest CU takes, a slab of
-    32 of K being bound by its products or its loads; of what all padded work
-    draws at the power limit; and of reading the weights.  Parts cost a second
-    launch, which reads them.  us, fitted to 2900 times of 65 to 8100 rows and
-    11 matrices (3584 to 37888 columns); what it chooses takes 1 % more than
-    the best choice on average."""
+    is least, as estimated: about the largest of what the busiest CU takes, a
+    slab of 32 of K being bound by its products or its loads; of what all
+    padded work draws at the power limit; and of reading the weights.  Parts
+    cost a second launch, which reads them.  us, fitted to 6700 times of every
+    tile at 24 numbers of rows from 129 to 8192 and 11 matrices (3584 to 37888
+    columns); at 25 others what it chooses for a layer takes 0.5 % more than
+    the best choice on average and 4 % at most."""
     best, least = None, math.inf
     for hm, hn in TILES:
         unit = 256 if hm + hn <= 8 else 128
@@ -669,12 +671,12 @@ def tile_plan(M, N, K, epi, cus=256):
                 break
             slabs = -(-K // unit // ks) * unit / 32
             rounds = -(-tiles * ks // cus)
-            slab = max(area * 0.0079, (hm + hn) * 0.0235)
-            t = max(rounds * (slabs * slab + 2.2 + area * 0.16),
-                    tiles * ks * area / cus * (slabs * 0.0088 + 0.16),
-                    N * K * 4e-7)
+            slab = max(area * 0.00715, hm * 0.0239 + hn * 0.0223)
+            busiest = rounds * (slabs * slab + 2.6 + area * 0.202)
+            power = tiles * ks * area / cus * (slabs * 0.0079 + 0.202)
+            t = (busiest ** 8 + power ** 8 + (N * K * 4e-7) ** 8) ** 0.125
             if ks > 1:
-                t += 10.6 + ks * M * N * 1.4e-6
+                t += 7.3 + ks * M * N * 1.5e-6
             if t < least:
                 best, least = (hm, hn, ks), t
     return best
