@@ -647,7 +647,7 @@ def linear_qkv_rope(x, packed, N, bias_rp, cache, layer, positions,
 TILES = ((8, 8), (9, 7), (7, 7), (8, 6), (10, 4), (6, 6), (8, 4), (6, 4),
          (4, 4), (4, 2))
 TILE_RESIDUAL, TILE_GATED, TILE_ROPE, TILE_PARTS = range(4)
-TILE_FOLD = 8             # blocks that add up the parts of a row
+TILE_FOLD = 16            # blocks that add up the parts of a row
 
 
 @functools.lru_cache(maxsize=4096)
