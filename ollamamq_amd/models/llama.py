@@ -487,30 +487,53 @@ class LlamaModel:
         nt = 1                      # embed stats = one partial tile
         inv_h = 1.0 / H
         eps = cfg.norm_eps
+        # From 65 rows on o and down go over tiles in parts of K: a block of
+        # k_wstream_gemm loads all rows for 32 columns (4096 x 4096 and 4096 x
+        # 14336, 128 rows: 20.5 and 46.2 us against 15.3 and 36.6; 72 rows: 17.0
+        # and 34.5 against 14.4 and 33.6; 64: 15.4 and 31.4 against 13.3 and
+        # 32.5).  So do rotated products with columns for 160 blocks of 64
+        # (12288 x 4096, 128 rows: 51 us against 40; 6144: 27 against 33).
+        tiles = B > 64 and self._tiles_take(B)
         for li, layer in enumerate(self.layers):
             # fused rmsnorm -> qkv -> RoPE -> paged KV append: q comes
             # back rotated in standard layout, k/v land in the pool
-            qkv = ops.qkv_rope_fused(
-                res, layer.wqkv_pk, layer.wqkv.shape[0], layer.bqkv_rp,
-                kv_cache, li, positions, slot_ids,
-                self.rope_cos, self.rope_sin, nl, nkl,
-                rstd=sq_a, rstd_nt=nt, inv_h=inv_h, eps=eps,
-                K=H, M_real=B)
+            if tiles and layer.wqkv.shape[0] >= 10240:
+                qkv = ops.tile_qkv_rope(
+                    res, layer.wqkv_pk, B, layer.wqkv.shape[0], H,
+                    layer.bqkv_rp, kv_cache, li, positions, slot_ids,
+                    self.rope_cos, self.rope_sin, nl, nkl, sq_a, nt, inv_h,
+                    eps)
+            else:
+                qkv = ops.qkv_rope_fused(
+                    res, layer.wqkv_pk, layer.wqkv.shape[0], layer.bqkv_rp,
+                    kv_cache, li, positions, slot_ids,
+                    self.rope_cos, self.rope_sin, nl, nkl,
+                    rstd=sq_a, rstd_nt=nt, inv_h=inv_h, eps=eps,
+                    K=H, M_real=B)
             q = qkv[:, :nl * d].view(-1, nl, d)
             attn = ops.attention_frag(q, kv_cache, li, attn_meta,
                                       tickets)
-            ops.linear_fused(attn, layer.wo_pk, H, res=res, sq_out=sq_b,
-                             y=res, yfrag=1, K=nl * d, xlds=2, M_frag=B,
-                             sem=tickets)
+            nb = tiles_h
+            if tiles:
+                sq_b, nb = ops.tile_residual(attn, layer.wo_pk, B, H, nl * d,
+                                             res)
+            else:
+                ops.linear_fused(attn, layer.wo_pk, H, res=res, sq_out=sq_b,
+                                 y=res, yfrag=1, K=nl * d, xlds=2, M_frag=B,
+                                 sem=tickets)
             act = ops.gu_fused(res, layer.wgu_pk,
                                layer.wgate_up.shape[0], rstd=sq_b,
-                               rstd_nt=tiles_h, inv_h=inv_h, eps=eps,
+                               rstd_nt=nb, inv_h=inv_h, eps=eps,
                                K=H, yfrag=1, M_frag=B)
-            ops.linear_fused(act, layer.wdown_pk, H, res=res,
-                             sq_out=sq_a, y=res, yfrag=1,
-                             K=layer.wdown.shape[1], xlds=2, M_frag=B,
-                             sem=tickets)
             nt = tiles_h
+            if tiles:
+                sq_a, nt = ops.tile_residual(act, layer.wdown_pk, B, H,
+                                             layer.wdown.shape[1], res)
+            else:
+                ops.linear_fused(act, layer.wdown_pk, H, res=res,
+                                 sq_out=sq_a, y=res, yfrag=1,
+                                 K=layer.wdown.shape[1], xlds=2, M_frag=B,
+                                 sem=tickets)
         idx = attn_meta.logits_idx
         if (idx is not None and 0 < idx.shape[0] <= ops.CHAIN_ROWS
                 and attn_meta.rows != list(range(B))):

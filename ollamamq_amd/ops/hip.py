@@ -676,7 +676,7 @@ def tile_plan(M, N, K, epi, cus=256):
             power = tiles * ks * area / cus * (slabs * 0.0079 + 0.202)
             t = (busiest ** 8 + power ** 8 + (N * K * 4e-7) ** 8) ** 0.125
             if ks > 1:
-                t += 7.3 + ks * M * N * 1.5e-6
+                t += 3.0 + ks * M * N * 1.5e-6
             if t < least:
                 best, least = (hm, hn, ks), t
     return best
