@@ -770,19 +770,25 @@ __global__ __launch_bounds__(512, 1) void k_wide(
     }
 }
 
-// Tiles a block: those with which the busiest CU loads least, counted in
-// units of 4 KB a step of K.  k_wstream_gemm (1) has two blocks a CU and reads
-// no rows past M; its loads may be a tenth more, for the steps' barriers
-// (37888 columns: 33 rows 70 us against 80, 45 rows 69 against 59; 16384: 33
-// rows 32 against 36).
+// Tiles a block: those with which the busiest CU is done first, in units of 4
+// KB a step of K.  A block of k_wide loads its tiles and all rows, or waits: two
+// tiles take what 4.8 + mt / 2 units take.  A tile of k_wstream_gemm (1), of
+// which a CU has several at a time, takes 0.8 (1 + mt), its rows coming from
+// L1 at times.  For 4096 columns of K a unit is 6 us.  us of 1, 2, 4 and 8:
+//   16384 x 4096,  40 rows  30  36  35  56      22016 x 4096,  40  42  56  37  58
+//                  96       41  39  43  63      37888 x 3584,  40  67  71  64  57
+//   11008 x 2048, 112       26  23  26  39                     64  75  72  65  57
+// Over 11 widths and 33 to 128 rows the choice takes 0.1 % more than the best
+// one; one by loads alone, k_wstream_gemm's counted by rows, 2.5 %.
 static int wide_tiles(int M, int N)
 {
     const int tiles = N / 32, mt = (M + 31) / 32;
     int best = 1;
-    double least = tiles / 256. * (1 + M / 32.) / 1.1;
+    double least = (tiles + 255) / 256 * 0.8 * (1 + mt);
     for (int cw = 2; cw <= 8; cw *= 2) {
         const int blocks = (tiles + cw - 1) / cw;
-        const double units = (blocks + 255) / 256 * (cw + mt);
+        const double units = (blocks + 255) / 256
+                             * (cw == 2 ? 4.8 + 0.5 * mt : cw + mt);
         if (units < least) {
             least = units;
             best = cw;
