@@ -3,15 +3,15 @@
 // kin), with what follows a product of the fused chain in the epilogue.
 //
 // What bounds it: at 256 CUs the matrix cores draw the card down to 1.5 to
-// 1.7 GHz, where this loop keeps them 95 % busy (1.5 PFLOP/s over the rows that
+// 1.7 GHz, where this loop keeps them 89 % busy (1.5 PFLOP/s over the rows that
 // are there; 2.25 with operands that do not move).  So a product takes what its
 // padded tiles take, and what is left to gain is padding, passes beside the
 // product and, for few rows, CUs without a tile.
 //
 // * A block of four waves, one a SIMD, makes 32 HM x 32 HN of y; a wave keeps
 //   its quarter, HM x HN accumulators of 16 x 16.  Large tiles because every
-//   byte that a CU loads costs power and time: 288 x 224 loads 126 operations
-//   a byte.
+//   byte that a CU loads costs power and time: 256 x 256 makes 128 operations
+//   of a byte.
 // * K goes by in slabs of 32 through four stages of LDS.  Both operands lie in
 //   fragment order, so a slab of 32 rows is 2 KB in a row, goes to LDS without
 //   passing registers (16 bytes a lane) and comes back without bank conflicts.
@@ -20,7 +20,8 @@
 //   16: no more than three other instructions may stand beside it.  Hence
 //   pointers per piece that move only with the tile, stages known at compile
 //   time, one barrier a slab, and loads and reads spread over a slab's products
-//   (300 instructions a slab of 63 products ran at 1.30 PFLOP/s, 183 at 1.43).
+//   (a slab of 63 products in 300 instructions ran at 1.30 PFLOP/s, in 183 at
+//   1.43).
 // * Blocks stay and take the next tile, whose first slabs are on their way
 //   while the last one's results are stored.
 //
@@ -31,10 +32,11 @@
 //
 // us for 541, 2317 and 8100 rows, one after another on one card:
 //   28672 x 4096, gated   library product 140, 421, 1270 and norm and
-//                         activation 15, 50, 166; here 110, 442, 1370
+//                         activation 15, 50, 166; here 107, 440, 1270
 //   6144 x 4096, rotated  40, 88, 268 and norm and append 11, 28, 78; here 40,
-//                         114, 325
-//   4096 x 14336          112, 213, 610; here 80 (six parts), 228, 650
+//                         114, 320
+//   4096 x 14336          112, 213, 610; here 76 (three parts and what adds
+//                         them up), 204, 626
 #include <type_traits>
 #include <utility>
 #include "act.h"
@@ -725,6 +727,7 @@ int launch(TileArgs a, int hm, int hn, int cus, hipStream_t stream)
     TILE(6, 4);
     TILE(4, 4);
     TILE(4, 2);
+    if constexpr (EPI != GATED) TILE(2, 2);
     #undef TILE
     return -110;                            // no such tile
 }

@@ -6,10 +6,11 @@ in-process compute contract those backends implicitly satisfied.
 
 Design notes (MI355X):
 * weights live resident in HBM3E as bf16 (8B = ~16 GB of 288 GB);
-* projection GEMMs go through torch F.linear (hipBLASLt/rocBLAS) — plain
-  library GEMMs; every fused hot op (fused residual+RMSNorm, RoPE,
-  prefill/decode attention over the paged KV pool, SwiGLU, sampler) is a
-  hand-written gfx950 HIP kernel behind ollamamq_amd.ops;
+* projections stream packed weights, a few rows at a time or over tiles of many
+  (ops.linear_fused, ops.tile_residual and their kin), with norms, rope, SwiGLU
+  and residual in their epilogues; without packed weights, tensor parallel or
+  with other shapes they are torch F.linear (hipBLASLt/rocBLAS) between
+  hand-written gfx950 HIP kernels behind ollamamq_amd.ops;
 * tensor parallelism: column-parallel QKV/gate-up, row-parallel o/down with
   one RCCL all-reduce each (2/layer), vocab-parallel logits with all-gather.
 """
@@ -296,7 +297,7 @@ class LlamaModel:
     def _pack_weights(self):
         """Build MFMA-fragment-order packed copies of every projection for
         the weight-streaming decode GEMM.  Doubles weight HBM (8B: 16->32
-        of 288 GB — prefill keeps the standard layout for hipBLASLt); on
+        of 288 GB — the general path keeps the standard layout); on
         models where the copy would not fit (70B on one GPU) packing is
         skipped wholesale and decode stays on the library GEMMs."""
         import os
@@ -487,13 +488,15 @@ class LlamaModel:
         nt = 1                      # embed stats = one partial tile
         inv_h = 1.0 / H
         eps = cfg.norm_eps
-        # From 65 rows on o and down go over tiles in parts of K: a block of
+        # From 49 rows on o and down go over tiles in parts of K: a block of
         # k_wstream_gemm loads all rows for 32 columns (4096 x 4096 and 4096 x
         # 14336, 128 rows: 20.5 and 46.2 us against 15.3 and 36.6; 72 rows: 17.0
-        # and 34.5 against 14.4 and 33.6; 64: 15.4 and 31.4 against 13.3 and
-        # 32.5).  So do rotated products with columns for 160 blocks of 64
-        # (12288 x 4096, 128 rows: 51 us against 40; 6144: 27 against 33).
-        tiles = B > 64 and self._tiles_take(B)
+        # and 34.5 against 14.4 and 33.6; 64: 14.9 and 31.1 against 12.5 and
+        # 29.1; 56: 15.0 and 30.1 against 13.4 and 29.5; 45: 14.4 and 28.5
+        # against 12.6 and 28.9).  So do rotated products with columns for 160
+        # blocks of 64 (12288 x 4096, 128 rows: 51 us against 40, 56: 33 against
+        # 29; 6144: 27 against 33, 18 against 22).
+        tiles = B > 48 and self._tiles_take(B)
         for li, layer in enumerate(self.layers):
             # fused rmsnorm -> qkv -> RoPE -> paged KV append: q comes
             # back rotated in standard layout, k/v land in the pool

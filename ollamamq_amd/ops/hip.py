@@ -646,6 +646,7 @@ def linear_qkv_rope(x, packed, N, bias_rp, cache, layer, positions,
 # Products of many rows (tile_gemm.hip): tiles in units of 32 rows and columns
 TILES = ((8, 8), (9, 7), (7, 7), (8, 6), (10, 4), (6, 6), (8, 4), (6, 4),
          (4, 4), (4, 2))
+TILE_LEAST = (2, 2)       # for 64 rows at most, not gated
 TILE_RESIDUAL, TILE_GATED, TILE_ROPE, TILE_PARTS = range(4)
 TILE_FOLD = 16            # blocks that add up the parts of a row
 
@@ -659,7 +660,14 @@ def tile_plan(M, N, K, epi, cus=256):
     cost a second launch, which reads them.  us, fitted to 6700 times of every
     tile at 24 numbers of rows from 129 to 8192 and 11 matrices (3584 to 37888
     columns); at 25 others what it chooses for a layer takes 0.5 % more than
-    the best choice on average and 4 % at most."""
+    the best choice on average and 4 % at most.  Few rows are weights' reads:
+    the smallest tiles, in as many parts as there are CUs but of no fewer than
+    1536 of K (64 rows of 4096 x 4096 and 4096 x 14336, parts: 1 14.4 and more
+    than 40, 2 12.5, 3 13.2 and 33.1, 4 13.3 and 29.1; at 128 rows 64 x 64 takes
+    a quarter more than 128 x 64)."""
+    if M <= 64 and epi != TILE_GATED and K % 256 == 0:
+        parts = min(cus // -(-N // 64), K // 1536, 8)
+        return (*TILE_LEAST, max(1, parts) if epi == TILE_RESIDUAL else 1)
     best, least = None, math.inf
     for hm, hn in TILES:
         unit = 256 if hm + hn <= 8 else 128

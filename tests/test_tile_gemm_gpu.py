@@ -7,17 +7,19 @@ import torch
 
 from ollamamq_amd.ops import hip
 
-PLANS = [(*t, ks) for t in hip.TILES for ks in (1, 3)]
+SMALL = hip.TILE_LEAST
+PLANS = [(*t, ks) for t in (*hip.TILES, SMALL) for ks in (1, 3)]
 
 
 def test_plans_are_possible():
     """What is chosen is a tile that the kernel has and parts that K has."""
-    for M in (129, 130, 300, 541, 2317, 8192):
+    for M in (1, 49, 64, 65, 129, 130, 300, 541, 2317, 8192):
         for N, K in ((64, 128), (448, 384), (4096, 14336), (37888, 3584)):
             for epi in (hip.TILE_RESIDUAL, hip.TILE_GATED, hip.TILE_ROPE):
                 hm, hn, ks = hip.tile_plan(M, N, K, epi)
                 unit = 256 if hm + hn <= 8 else 128
-                assert (hm, hn) in hip.TILES and K % unit == 0
+                assert (hm, hn) in (*hip.TILES, SMALL) and K % unit == 0
+                assert (hm, hn) != SMALL or epi != hip.TILE_GATED
                 assert 1 <= ks <= K // unit
                 assert epi == hip.TILE_RESIDUAL or ks == 1
                 assert epi != hip.TILE_ROPE or hn % 2 == 0
@@ -67,7 +69,7 @@ def test_product(plan, M, N, K):
     # fp32 sums of squares of at most 2^12 values before their rounding
     assert sq.shape == (M, nt)
     assert off(sq.sum(1), (y + res.double()).square().sum(1)) < 2 ** -18
-    if plan[2] > 1:
+    if plan[2] > 1 or plan[:2] == SMALL:
         return
     for nt in (1, 3, 40):
         sq = (torch.rand(M, nt, device="cuda") + 0.5) * (K / nt)
@@ -82,7 +84,8 @@ def test_product(plan, M, N, K):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("plan", [p for p in hip.TILES if p[1] % 2 == 0],
+@pytest.mark.parametrize("plan", [p for p in (*hip.TILES, SMALL)
+                                  if p[1] % 2 == 0],
                          ids=str)
 @pytest.mark.parametrize("M, nl, nkl, page, bias", [
     (1, 1, 1, 16, False), (131, 4, 2, 16, True), (300, 7, 1, 48, True),
