@@ -131,6 +131,17 @@ DEV void swap32(f32x4& a, f32x4& b) {
     }
 }
 
+// n / (1 + e), e not negative, as close as the division is: a reciprocal and
+// one step of Newton's method on the quotient, infinities and NaN as a division
+// has them.  In eighths, for reciprocals of 2^126 and more are flushed.  Prompts
+// take 0.4 % longer than with the reciprocal alone, 1.3 with the division.
+DEV float over_1_and(float n, float e) {
+    const float d = fmaf(e, 0.125f, 0.125f), r = __builtin_amdgcn_rcpf(d);
+    n *= 0.125f;
+    const float q = n * r;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, n), r, q), d, n);
+}
+
 // stages of LDS; four keep three slabs of a large tile under way, small tiles
 // need more of their slabs for as many bytes
 constexpr int tile_stages(int hm, int hn) { return hm + hn <= 8 ? 8 : 4; }
@@ -488,8 +499,7 @@ __global__ __launch_bounds__(256, 1) void k_tile_gemm(const TileArgs a)
                     #pragma unroll
                     for (int e = 0; e < 4; e++) {
                         const float z = a.gelu ? gelu_arg(lo[e]) : lo[e];
-                        v[e] = lo[e] * __builtin_amdgcn_rcpf(1.f + __expf(-z))
-                               * hi[e];
+                        v[e] = over_1_and(lo[e], __expf(-z)) * hi[e];
                     }
                     if (ok) put4(reinterpret_cast<bf16*>(p), v);
                 };

@@ -84,6 +84,27 @@ def test_product(plan, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("glu", ["silu", "gelu_tanh"])
+def test_activation_is_the_chains(glu):
+    """Sums of whole numbers are exact in any order, so what is left is the
+    epilogue: bit for bit that of the weight stream.  A reciprocal off by a
+    unit of fp32 turns one value of 2^16 to another bf16."""
+    hip.require()
+    torch.manual_seed(7)
+    M, N, K = 128, 28672, 256
+    x = torch.randint(-2, 3, (M, K), device="cuda").bfloat16()
+    w = torch.randint(-1, 2, (N, K), device="cuda").bfloat16()
+    # scales about 1/8, another for every row
+    sq = (torch.rand(M, device="cuda") + 0.5) * 64 * K
+    args = (frag(x), hip.pack_weight_gu(w))
+    norm = dict(rstd=sq, rstd_nt=1, inv_h=1.0 / K, eps=1e-5, glu=glu)
+    want = hip.linear_gu(*args, N, K=K, yfrag=1, M_frag=M, **norm)
+    for plan in ((8, 8, 1), (9, 7, 1)):
+        got = hip.tile_gu(*args, M, N, K, plan=plan, **norm)
+        assert torch.equal(unfrag(got, M, N // 2), unfrag(want, M, N // 2))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("plan", [p for p in (*hip.TILES, SMALL)
                                   if p[1] % 2 == 0],
                          ids=str)
