@@ -626,12 +626,12 @@ __global__ __launch_bounds__(256, 1) void k_tile_gemm(const TileArgs a)
 // lanes hold them.  A block takes 16 rows and a `pieces`-th of the columns, a
 // wave four accumulators at a time with the loads of all of them and of two
 // parts under way: 541 x 4096 in 3 parts, 16 pieces, reads 27 MB in 9.2 us
-// (one accumulator at a time in 8 pieces: 15.3).
+// (one accumulator at a time in 8 pieces: 15.3).  y may be res: a lane reads
+// only what it writes itself afterwards, and the padding of rows past M.
 template <int BS>
 __global__ __launch_bounds__(BS) void k_tile_fold(
-    bf16* __restrict__ y, const bf16* __restrict__ res,
-    float* __restrict__ sq, const float* __restrict__ part, int M, int N,
-    int ks)
+    bf16* y, const bf16* res, float* __restrict__ sq,
+    const float* __restrict__ part, int M, int N, int ks)
 {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const int r16 = lane & 15, g4 = lane >> 4;
@@ -650,10 +650,9 @@ __global__ __launch_bounds__(BS) void k_tile_fold(
         int64_t at[J];
         #pragma unroll
         for (int i = 0; i < J; i++) {
-            const int j = min(j0 + i * W, to - 1);
+            const int j = j0 + i * W < to ? j0 + i * W : j0;
             p[i] = part + ((int64_t)hi * nh + j) * 256 + lane * 4;
-            at[i] = frag_at(min(row, M - 1),
-                            (j >> 1) * 32 + in_strip(j & 1, 4 * g4), N);
+            at[i] = frag_at(row, (j >> 1) * 32 + in_strip(j & 1, 4 * g4), N);
             v[i] = *reinterpret_cast<const f32x4*>(p[i]);
             old[i] = *reinterpret_cast<const bf16x4*>(res + at[i]);
         }
