@@ -755,8 +755,15 @@ extern "C" int tile_gemm_bf16(
     int nl, int nkl, int psz, int maxp, hipStream_t stream)
 {
     const int unit = 32 * tile_stages(hm, hn);     // of K
-    if (M < 1 || N < 32 || N % 32 || K < unit || K % unit || ks < 1
-        || ks > K / unit || (int64_t)(M + 31) * N >= (int64_t)1 << 31 || gm < 1 || cus < 8 || (epi != PARTS && ks != 1)
+    const bool normed = epi == GATED || epi == ROPE;
+    // fp32 parts, or a sum per row, where it comes in several
+    const bool scratch = epi == PARTS || (normed && rstd_nt > 1);
+    if (epi < RESIDUAL || epi > PARTS || M < 1 || N < 32 || N % 32
+        || K < unit || K % unit || ks < 1 || ks > K / unit
+        || (int64_t)(M + 31) * N >= (int64_t)1 << 31
+        || gm < 1 || cus < 8 || (scratch && !part)
+        || (normed && (!rstd || rstd_nt < 1))
+        || (epi == PARTS ? pieces < 1 : ks != 1)
         || (epi == ROPE && N != (nl + 2 * nkl) * 128))
         return -111;
     TileArgs a{(bf16*)y, (float*)part, (const bf16*)x, (const bf16*)w,

@@ -174,3 +174,26 @@ def test_refused():
     for bad in (dict(M=0), dict(N=48), dict(K=128), dict(K=192, hm=9, hn=7),
                 dict(ks=2), dict(epi=3, ks=2), dict(hm=5, hn=5), dict(epi=2)):
         assert call(**bad) < 0
+
+
+def test_refused_scratch():
+    """Scratch, sums and pieces that a product cannot do without, and
+    epilogues that there are none of."""
+    lib = hip._lib if hip.available() else None
+    if lib is None:
+        pytest.skip("the extension is not built")
+    some = 1 << 20                      # nothing reads it
+
+    def call(epi, part=some, rstd=some, rstd_nt=1, pieces=16):
+        return lib.tile_gemm_bf16(
+            some, part, some, some, None, some, some, rstd, rstd_nt, 0.0, 0.0,
+            129, 384, 256, epi, 4, 4, 1, 8, pieces, 0, 256, *[some] * 7, 1, 1,
+            16, 1, None)
+    if not torch.cuda.is_available():   # nothing but the device is missing
+        for epi in range(4):
+            assert call(epi) > 0
+    for bad in (dict(epi=3, pieces=0), dict(epi=3, pieces=-1),
+                dict(epi=3, part=None), dict(epi=1, part=None, rstd_nt=3),
+                dict(epi=2, part=None, rstd_nt=3), dict(epi=1, rstd_nt=0),
+                dict(epi=2, rstd=None), dict(epi=-1), dict(epi=4)):
+        assert call(**bad) < 0, bad
