@@ -497,6 +497,10 @@ class LlamaModel:
         # blocks of 64 (12288 x 4096, 128 rows: 51 us against 40, 56: 33 against
         # 29; 6144: 27 against 33, 18 against 22).
         tiles = B > 48 and self._tiles_take(B)
+        # a switch that asks for parts means the streams'
+        o_tiles = tiles and ops.asked_parts(nl * d) is None
+        down_tiles = tiles and ops.asked_parts(
+            self.layers[0].wdown.shape[1]) is None
         for li, layer in enumerate(self.layers):
             # fused rmsnorm -> qkv -> RoPE -> paged KV append: q comes
             # back rotated in standard layout, k/v land in the pool
@@ -517,7 +521,7 @@ class LlamaModel:
             attn = ops.attention_frag(q, kv_cache, li, attn_meta,
                                       tickets)
             nb = tiles_h
-            if tiles:
+            if o_tiles:
                 sq_b, nb = ops.tile_residual(attn, layer.wo_pk, B, H, nl * d,
                                              res)
             else:
@@ -529,7 +533,7 @@ class LlamaModel:
                                rstd_nt=nb, inv_h=inv_h, eps=eps,
                                K=H, yfrag=1, M_frag=B)
             nt = tiles_h
-            if tiles:
+            if down_tiles:
                 sq_a, nt = ops.tile_residual(act, layer.wdown_pk, B, H,
                                              layer.wdown.shape[1], res)
             else:

@@ -814,6 +814,12 @@ def _frag_ksplit(N, K):
     return ks
 
 
+def asked_parts(K):
+    """The parts that a switch asks of streamed products over K, or None."""
+    ks = os.environ.get(f"OLLAMAMQ_WS_KS_{K}") or _WS_KS
+    return int(ks) if ks else None
+
+
 def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
                   rstd=None, rstd_nt=0, inv_h=0.0, eps=0.0,
                   res=None, sq_out=None, y=None, yfrag=0, K=None,
@@ -837,12 +843,8 @@ def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
         y = torch.empty((((M + 31) // 32) * 32 * N,) if yfrag
                         else (M, N), dtype=x.dtype, device=x.device)
     if ks is None:
-        per_k = os.environ.get(f"OLLAMAMQ_WS_KS_{K}")   # per-shape tuning
-        if per_k:
-            ks = int(per_k)
-        elif _WS_KS:
-            ks = int(_WS_KS)
-        else:
+        ks = asked_parts(K)
+        if ks is None:
             ks = _frag_ksplit(N, K) if xlds == 2 else _wstream_ksplit(N, K)
     if rstd is not None:
         ks = 1            # every part would have to scale its rows

@@ -836,6 +836,12 @@ def tiles_take(M, N, K):
     return hip.tiles_take(M, N, K)
 
 
+def asked_parts(K):
+    """The parts that a switch asks of streamed products over K, or None."""
+    from . import hip
+    return hip.asked_parts(K)
+
+
 def tile_qkv_rope(x, packed, M, N, K, bias_rp, cache, layer, positions, slots,
                   cos, sin, nl, nkl, rstd, rstd_nt, inv_h, eps):
     """rmsnorm -> qkv GEMM -> RoPE -> paged KV append, one kernel."""

@@ -75,6 +75,30 @@ def test_chain_and_general_path(name):
     assert torch.equal(k1 != 0, k2 != 0) and torch.equal(v1 != 0, v2 != 0)
 
 
+@pytest.mark.parametrize("env, every, over_tiles", [
+    ({}, None, {512, 1024}), ({"OLLAMAMQ_WS_KS_512": "1"}, None, {1024}),
+    ({"OLLAMAMQ_WS_KS_1024": "2"}, None, {512}), ({}, "1", set())])
+def test_parts_asked_for(env, every, over_tiles, monkeypatch):
+    """OLLAMAMQ_WS_KS and OLLAMAMQ_WS_KS_<K> reach o and down of a step of any
+    size: a product that they name is streamed."""
+    from ollamamq_amd.models import LlamaModel, PRESETS
+    from ollamamq_amd.ops import hip
+    cfg = PRESETS["tiny"]
+    model = LlamaModel(cfg, device="cuda:0", dtype=torch.bfloat16, seed=5)
+    assert (cfg.q_dim, cfg.ffn) == (512, 1024)
+    step = [[(0, range(64), [63])]]
+    want = _run(model, cfg, False, step)[0][0]
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    monkeypatch.setattr(hip, "_WS_KS", every)
+    seen, product = set(), hip.tile_residual
+    monkeypatch.setattr(hip, "tile_residual",
+                        lambda x, w, M, N, K, *a: seen.add(K)
+                        or product(x, w, M, N, K, *a))
+    _close(_run(model, cfg, True, step)[0][0].float(), want.float())
+    assert seen == over_tiles
+
+
 @pytest.mark.parametrize("H", [64, 512, 4096])
 def test_rows(H):
     from ollamamq_amd.ops import hip
