@@ -399,7 +399,8 @@ class LlamaModel:
         if (chain and tokens.shape[0] > ops.CHAIN_ROWS
                 and not attn_meta.one_each and idx is not None
                 and 0 < idx.shape[0] <= ops.CHAIN_ROWS
-                and self._tiles_take(tokens.shape[0])):
+                and self._tiles_take(tokens.shape[0])
+                and not ops.library_products()):
             return self._forward_tiles(tokens, positions, kv_cache,
                                        slot_ids, attn_meta)
         x = ops.embedding(tokens, self.embed)

@@ -836,6 +836,12 @@ def tiles_take(M, N, K):
     return hip.tiles_take(M, N, K)
 
 
+def library_products():
+    """A switch asks for the library's products where it has them."""
+    from . import hip
+    return not hip.USE_WSTREAM
+
+
 def asked_parts(K):
     """The parts that a switch asks of streamed products over K, or None."""
     from . import hip

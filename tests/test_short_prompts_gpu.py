@@ -99,6 +99,21 @@ def test_parts_asked_for(env, every, over_tiles, monkeypatch):
     assert seen == over_tiles
 
 
+@pytest.mark.parametrize("streams", [True, False])
+def test_library_products_asked_for(streams, monkeypatch):
+    """OLLAMAMQ_NO_WSTREAM reaches prompts of more rows than the chain's."""
+    from ollamamq_amd.models import LlamaModel, PRESETS
+    from ollamamq_amd.ops import hip
+    cfg = PRESETS["tiny"]
+    model = LlamaModel(cfg, device="cuda:0", dtype=torch.bfloat16, seed=5)
+    monkeypatch.setattr(hip, "USE_WSTREAM", streams)
+    seen, product = [], hip.tile_gu
+    monkeypatch.setattr(hip, "tile_gu",
+                        lambda *a: seen.append(a) or product(*a))
+    _run(model, cfg, True, [[(0, range(129), [128])]])
+    assert len(seen) == (cfg.n_layers if streams else 0)
+
+
 @pytest.mark.parametrize("H", [64, 512, 4096])
 def test_rows(H):
     from ollamamq_amd.ops import hip
