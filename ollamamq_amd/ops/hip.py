@@ -721,7 +721,8 @@ def tile_gu(x, packed, M, N, K, rstd, rstd_nt, inv_h, eps, glu="silu",
     act = torch.empty(-(-M // 32) * 32 * (N // 2), dtype=x.dtype,
                       device=x.device)
     _tile_gemm(TILE_GATED, act, x, packed, M, N, K,
-               plan or tile_plan(M, N, K, TILE_GATED), rstd=rstd,
+               plan or tile_plan(M, N, K, TILE_GATED, _cus(x.device.index)),
+               rstd=rstd,
                rstd_nt=rstd_nt, inv_h=inv_h, eps=eps, gelu=GELU[glu])
     return act
 
@@ -729,7 +730,7 @@ def tile_gu(x, packed, M, N, K, rstd, rstd_nt, inv_h, eps, glu="silu",
 def tile_residual(x, packed, M, N, K, res, plan=None):
     """res += x W^T in place, all in fragment layout, for many rows; returns
     partial sums of squares of the new rows and how many a row has."""
-    plan = plan or tile_plan(M, N, K, TILE_RESIDUAL)
+    plan = plan or tile_plan(M, N, K, TILE_RESIDUAL, _cus(x.device.index))
     ks, part, epi = plan[2], None, TILE_RESIDUAL
     if ks > 1:
         part = torch.empty(ks * -(-M // 32) * 32 * N, dtype=torch.float32,
@@ -749,8 +750,8 @@ def tile_qkv_rope(x, packed, M, N, K, bias_rp, cache, layer, positions,
     kp, vp = _layer_ptrs(cache, layer)
     pos32, slot32 = _i32(positions), _i32(slots)
     _tile_gemm(TILE_ROPE, y, x, packed, M, N, K,
-               plan or tile_plan(M, N, K, TILE_ROPE), bias=bias_rp, rstd=rstd,
-               rstd_nt=rstd_nt, inv_h=inv_h, eps=eps,
+               plan or tile_plan(M, N, K, TILE_ROPE, _cus(x.device.index)),
+               bias=bias_rp, rstd=rstd, rstd_nt=rstd_nt, inv_h=inv_h, eps=eps,
                rope=(_p(cos), _p(sin), _p(pos32), _p(slot32),
                      _p(cache.page_table), kp, vp, nl, nkl, cache.page_size,
                      cache.page_table.shape[1]))

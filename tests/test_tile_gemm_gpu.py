@@ -25,6 +25,29 @@ def test_plans_are_possible():
                 assert epi != hip.TILE_ROPE or hn % 2 == 0
 
 
+@pytest.mark.parametrize("cus", [32, 64, 256])
+def test_plans_are_the_devices(cus, monkeypatch):
+    """Tiles and parts are chosen for as many CUs as the device has, which is
+    what the grid is sized for: a partition of a card has fewer."""
+    seen = []
+    monkeypatch.setattr(hip, "_cus", lambda index: cus)
+    monkeypatch.setattr(
+        hip, "_tile_gemm", lambda epi, y, x, packed, M, N, K, plan, **k:
+        seen.append(plan))
+    M, N, K = 300, 384, 1536
+    x, w, y = torch.empty(320 * K), torch.empty(N * K), torch.empty(320 * N)
+    cache = SimpleNamespace(page_size=16, k_pool=torch.empty(1, 1),
+                            v_pool=torch.empty(1, 1),
+                            page_table=torch.empty(1, 1).int())
+    hip.tile_residual(x, w, M, N, K, y)
+    hip.tile_gu(x, w, M, N, K, None, 1, 0.0, 0.0)
+    hip.tile_qkv_rope(x, w, M, N, K, None, cache, 0, torch.empty(M).int(),
+                      torch.empty(M).int(), None, None, 1, 1, None, 1, 0.0,
+                      0.0)
+    assert seen == [hip.tile_plan(M, N, K, epi, cus) for epi in
+                    (hip.TILE_RESIDUAL, hip.TILE_GATED, hip.TILE_ROPE)]
+
+
 def frag(x):
     rows = -(-x.shape[0] // 32) * 32
     f = x.new_full((rows, x.shape[1]), math.nan)   # what no row may see
