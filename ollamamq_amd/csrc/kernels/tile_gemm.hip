@@ -37,6 +37,8 @@
 //                         114, 320
 //   4096 x 14336          112, 213, 610; here 76 (three parts and what adds
 //                         them up), 204, 626
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include <utility>
 #include "act.h"
@@ -741,7 +743,76 @@ int launch(TileArgs a, int hm, int hn, int cus, hipStream_t stream)
     return -110;                            // no such tile
 }
 
+// in units of 32 rows and columns
+constexpr int TILES[][2] = {{8, 8}, {9, 7}, {7, 7}, {8, 6}, {10, 4},
+                            {6, 6}, {8, 4}, {6, 4}, {4, 4}, {4, 2}};
+
+int div_up(int a, int b) { return (a + b - 1) / b; }
+double pow8(double x) { x *= x; x *= x; return x * x; }
+
+// us that a product takes, about the largest of what the busiest CU takes, a
+// slab of 32 of K being bound by its products or its loads; of what all padded
+// work draws at the power limit; and of reading the weights.  Parts cost a second
+// launch, which reads them.
+double estimate(int M, int N, int K, int hm, int hn, int ks, int cus)
+{
+    const int unit = 32 * tile_stages(hm, hn), area = hm * hn;
+    const int items = div_up(M, 32 * hm) * div_up(N, 32 * hn) * ks;
+    const double slabs = div_up(K / unit, ks) * unit / 32;
+    const double slab = std::max(area * 0.00715, hm * 0.0239 + hn * 0.0223);
+    const double busiest =
+        div_up(items, cus) * (slabs * slab + 2.6 + area * 0.202);
+    const double power =
+        (double)items * area / cus * (slabs * 0.0079 + 0.202);
+    const double t = sqrt(sqrt(sqrt(pow8(busiest) + pow8(power)
+                                    + pow8((double)N * K * 4e-7))));
+    return ks > 1 ? t + 3.0 + (double)ks * M * N * 1.5e-6 : t;
+}
+
 }  // namespace
+
+// The tiles of a product and its parts, hm | hn << 8 | ks << 16: those that the
+// estimate likes best.  It was fitted to 6700 times of every tile at 24 numbers
+// of rows from 129 to 8192 and the 11 matrices of the presets (3584 to 37888
+// columns); at 25 others what it chooses for a layer takes 0.5 % more than the
+// best choice on average and 4 % at most.  From 65 to 128 rows, weights not in
+// cache, o and down of 3584 to 8192 columns: down 0 to 7 % more than the best;
+// o of up to 4096 columns would take 5 to 15 % less over tiles of 64 x 64, which
+// are not weighed there.
+// Few rows are weights' reads: the smallest tiles, in as many parts as there are
+// CUs but of no fewer than 1536 of K (64 rows of 4096 x 4096 and 4096 x 14336
+// in cache, parts: 1 14.4 and more than 40, 2 12.5, 3 13.2 and 33.1, 4 13.3 and
+// 29.1; not in cache 2 16.5, 4 14.9 and 29.9).
+// On the host a choice takes 1.5 us; in Python it took 10 to 70, and a step of a
+// new number of rows 90 us longer than the next one (four layers, 301 to 399).
+extern "C" int tile_gemm_plan(int M, int N, int K, int epi, int cus)
+{
+    if (M < 1 || N < 32 || K < 128 || K % 128 || cus < 8 || epi < RESIDUAL
+        || epi > ROPE)
+        return -111;
+    auto plan = [](int hm, int hn, int ks) { return hm | hn << 8 | ks << 16; };
+    if (M <= 64 && epi != GATED && K % 256 == 0) {
+        const int parts = std::min({cus / div_up(N, 64), K / 1536, 8});
+        return plan(2, 2, epi == RESIDUAL ? std::max(1, parts) : 1);
+    }
+    int best = -110;
+    double least = INFINITY;
+    for (const auto& [hm, hn] : TILES) {
+        const int unit = 32 * tile_stages(hm, hn);
+        if (K % unit || (epi == ROPE && hn % 2)) continue;
+        const int64_t tiles =
+            (int64_t)div_up(M, 32 * hm) * div_up(N, 32 * hn);
+        for (int ks = 1; ks <= (epi == RESIDUAL ? 8 : 1); ks++) {
+            if (ks > 1 && (tiles * ks > 2.5 * cus || K / unit < 2 * ks)) break;
+            const double t = estimate(M, N, K, hm, hn, ks, cus);
+            if (t < least) {
+                least = t;
+                best = plan(hm, hn, ks);
+            }
+        }
+    }
+    return best;
+}
 
 // Tiles are hm x hn times 32 rows and columns.  epi: RESIDUAL (y = res + x W^T,
 // sq), GATED (y = act(gate) * up of normed x), ROPE (normed x, positions, keys

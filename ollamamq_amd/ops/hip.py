@@ -9,7 +9,6 @@ from __future__ import annotations
 
 import ctypes
 import functools
-import math
 import os
 from typing import NamedTuple, Optional
 
@@ -67,6 +66,7 @@ def _try_load():
                                     vp, i, f, f, i, i, vp]
     lib.tile_gemm_bf16.argtypes = [*[vp] * 8, i, f, f, *[i] * 11, *[vp] * 7,
                                    i, i, i, i, vp]
+    lib.tile_gemm_plan.argtypes = [i, i, i, i, i]
     lib.row_sumsq_bf16.argtypes = [vp, vp, i, i, vp]
     lib.frag_rows_bf16.argtypes = [vp, vp, vp, vp, i, i, i, vp]
     lib.fragify_sumsq_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i, i, i, vp, i,
@@ -653,41 +653,12 @@ TILE_FOLD = 16            # blocks that add up the parts of a row
 
 @functools.lru_cache(maxsize=4096)
 def tile_plan(M, N, K, epi, cus=256):
-    """(rows, columns, parts of K) of the tiles for which the time of a product
-    is least, as estimated: about the largest of what the busiest CU takes, a
-    slab of 32 of K being bound by its products or its loads; of what all
-    padded work draws at the power limit; and of reading the weights.  Parts
-    cost a second launch, which reads them.  us, fitted to 6700 times of every
-    tile at 24 numbers of rows from 129 to 8192 and 11 matrices (3584 to 37888
-    columns); at 25 others what it chooses for a layer takes 0.5 % more than
-    the best choice on average and 4 % at most.  Few rows are weights' reads:
-    the smallest tiles, in as many parts as there are CUs but of no fewer than
-    1536 of K (64 rows of 4096 x 4096 and 4096 x 14336, parts: 1 14.4 and more
-    than 40, 2 12.5, 3 13.2 and 33.1, 4 13.3 and 29.1; at 128 rows 64 x 64 takes
-    a quarter more than 128 x 64)."""
-    if M <= 64 and epi != TILE_GATED and K % 256 == 0:
-        parts = min(cus // -(-N // 64), K // 1536, 8)
-        return (*TILE_LEAST, max(1, parts) if epi == TILE_RESIDUAL else 1)
-    best, least = None, math.inf
-    for hm, hn in TILES:
-        unit = 256 if hm + hn <= 8 else 128
-        if K % unit or (epi == TILE_ROPE and hn % 2):
-            continue
-        tiles, area = -(-M // (32 * hm)) * -(-N // (32 * hn)), hm * hn
-        for ks in range(1, 9 if epi == TILE_RESIDUAL else 2):
-            if ks > 1 and (tiles * ks > 2.5 * cus or K // unit < 2 * ks):
-                break
-            slabs = -(-K // unit // ks) * unit / 32
-            rounds = -(-tiles * ks // cus)
-            slab = max(area * 0.00715, hm * 0.0239 + hn * 0.0223)
-            busiest = rounds * (slabs * slab + 2.6 + area * 0.202)
-            power = tiles * ks * area / cus * (slabs * 0.0079 + 0.202)
-            t = (busiest ** 8 + power ** 8 + (N * K * 4e-7) ** 8) ** 0.125
-            if ks > 1:
-                t += 3.0 + ks * M * N * 1.5e-6
-            if t < least:
-                best, least = (hm, hn, ks), t
-    return best
+    """(rows, columns, parts of K) of the tiles that a product takes."""
+    require()
+    plan = _lib.tile_gemm_plan(M, N, K, epi, cus)
+    if plan <= 0:
+        raise ValueError(f"no tiles for {M} rows of {N} x {K}")
+    return plan & 255, plan >> 8 & 255, plan >> 16
 
 
 def tiles_take(M, N, K):

@@ -1,5 +1,6 @@
 """Products of many rows over tiles (tile_gemm.hip) against float64."""
 import math
+import time
 from types import SimpleNamespace
 
 import pytest
@@ -23,6 +24,58 @@ def test_plans_are_possible():
                 assert 1 <= ks <= K // unit
                 assert epi == hip.TILE_RESIDUAL or ks == 1
                 assert epi != hip.TILE_ROPE or hn % 2 == 0
+
+
+def estimate(M, N, K, epi, cus):
+    """{(rows, columns, parts): us} of every plan that is weighed."""
+    took = {}
+    for hm, hn in hip.TILES:
+        unit = 256 if hm + hn <= 8 else 128
+        if K % unit or (epi == hip.TILE_ROPE and hn % 2):
+            continue
+        tiles, area = -(-M // (32 * hm)) * -(-N // (32 * hn)), hm * hn
+        for ks in range(1, 9 if epi == hip.TILE_RESIDUAL else 2):
+            if ks > 1 and (tiles * ks > 2.5 * cus or K // unit < 2 * ks):
+                break
+            slabs = -(-K // unit // ks) * unit / 32
+            slab = max(area * 0.00715, hm * 0.0239 + hn * 0.0223)
+            busiest = -(-tiles * ks // cus) * (slabs * slab + 2.6
+                                               + area * 0.202)
+            power = tiles * ks * area / cus * (slabs * 0.0079 + 0.202)
+            t = (busiest ** 8 + power ** 8 + (N * K * 4e-7) ** 8) ** 0.125
+            took[hm, hn, ks] = t + (3.0 + ks * M * N * 1.5e-6) * (ks > 1)
+    return took
+
+
+def test_plans_take_least():
+    """The choice is the one that the estimate likes best; for a new number of
+    rows it takes no more host time than a launch."""
+    for cus in (32, 256, 304):
+        for N, K in ((64, 128), (384, 1536), (4096, 14336), (6144, 4096),
+                     (37888, 3584), (5120, 13824)):
+            for M in (65, 129, 541, 1000, 2317, 8100):
+                for epi in range(3):
+                    took = estimate(M, N, K, epi, cus)
+                    plan = hip.tile_plan(M, N, K, epi, cus)
+                    assert took[plan] <= min(took.values()) * (1 + 1e-9)
+    for cus, N, K, parts in ((256, 4096, 4096, 2), (256, 4096, 14336, 4),
+                             (256, 64, 65536, 8), (64, 4096, 14336, 1),
+                             (256, 512, 512, 1)):
+        assert hip.tile_plan(64, N, K, hip.TILE_RESIDUAL, cus) == (
+            *SMALL, parts)
+        assert hip.tile_plan(64, N, K, hip.TILE_ROPE, cus) == (*SMALL, 1)
+    times = []                          # 1.6 us; in Python 68
+    for M in range(1000, 1301):
+        t0 = time.perf_counter()
+        hip.tile_plan(M, 4096, 14336, hip.TILE_RESIDUAL)
+        times.append(time.perf_counter() - t0)
+    assert sorted(times)[150] < 20e-6
+
+
+def test_plans_refused():
+    for bad in ((0, 64, 128), (129, 0, 128), (129, 64, 64), (129, 64, 192)):
+        with pytest.raises(ValueError):
+            hip.tile_plan(*bad, hip.TILE_GATED)
 
 
 @pytest.mark.parametrize("cus", [32, 64, 256])
