@@ -785,7 +785,8 @@ static int wide_tiles(int M, int N)
     const int tiles = N / 32, mt = (M + 31) / 32;
     int best = 1;
     double least = (tiles + 255) / 256 * 0.8 * (1 + mt);
-    for (int cw = 2; cw <= 8; cw *= 2) {
+    // two tiles of 64 rows are 5.8 units, one after the other 4.8 at most
+    for (int cw = mt == 2 ? 4 : 2; cw <= 8; cw *= 2) {
         const int blocks = (tiles + cw - 1) / cw;
         const double units = (blocks + 255) / 256
                              * (cw == 2 ? 4.8 + 0.5 * mt : cw + mt);
@@ -817,7 +818,7 @@ static int wide(int cw, void* y, const void* x, const void* wp, int M, int N,
         return cw == 8   ? go(k_wide<MT, 8, GU>)                           \
                : cw == 4 ? go(k_wide<MT, 4, GU>)                           \
                          : go(k_wide<MT, 2, GU>)
-    if (mt == 2) WIDE(2);
+    if (mt == 2) return cw == 8 ? go(k_wide<2, 8, GU>) : go(k_wide<2, 4, GU>);
     if (mt == 3) WIDE(3);
     WIDE(4);
     #undef WIDE
