@@ -490,14 +490,19 @@ class LlamaModel:
         inv_h = 1.0 / H
         eps = cfg.norm_eps
         # From 49 rows on o and down go over tiles in parts of K: a block of
-        # k_wstream_gemm loads all rows for 32 columns (4096 x 4096 and 4096 x
-        # 14336, 128 rows: 20.5 and 46.2 us against 15.3 and 36.6; 72 rows: 17.0
-        # and 34.5 against 14.4 and 33.6; 64: 14.9 and 31.1 against 12.5 and
-        # 29.1; 56: 15.0 and 30.1 against 13.4 and 29.5; 45: 14.4 and 28.5
-        # against 12.6 and 28.9).  So do rotated products with columns for 160
-        # blocks of 64 (12288 x 4096, 128 rows: 51 us against 40, 56: 33 against
-        # 29; 6144: 27 against 33, 18 against 22).
+        # k_wstream_gemm loads all rows for 32 columns.  us of a step, four
+        # layers, streams and tiles for o and down:
+        #                48 users      64         96         128
+        #   llama3-8b   531   546   559   560   662   646   740   711
+        #   qwen2-7b    586   592   618   608   731   709   816   777
+        #   llama2-13b  836   774   935   831  1163  1013  1360  1154
+        # So do rotated products of which the streams need a second round of
+        # blocks (49 and 128 rows: 9216 x 4096 31 and 50 us against 30 and 36,
+        # 12288 x 4096 33 and 51 against 31 and 37, 9216 x 2048 20 and 32 against
+        # 18 and 22; of one round 8192 x 4096 20 and 29 against 28 and 35).
         tiles = B > 48 and self._tiles_take(B)
+        qkv_tiles = tiles and not ops.streams_at_once(
+            self.layers[0].wqkv.shape[0], dev)
         # a switch that asks for parts means the streams'
         o_tiles = tiles and ops.asked_parts(nl * d) is None
         down_tiles = tiles and ops.asked_parts(
@@ -505,7 +510,7 @@ class LlamaModel:
         for li, layer in enumerate(self.layers):
             # fused rmsnorm -> qkv -> RoPE -> paged KV append: q comes
             # back rotated in standard layout, k/v land in the pool
-            if tiles and layer.wqkv.shape[0] >= 10240:
+            if qkv_tiles:
                 qkv = ops.tile_qkv_rope(
                     res, layer.wqkv_pk, B, layer.wqkv.shape[0], H,
                     layer.bqkv_rp, kv_cache, li, positions, slot_ids,

@@ -666,6 +666,12 @@ def tiles_take(M, N, K):
     return N % 64 == 0 and K % 128 == 0 and (M + 31) * max(N, K) < 2 ** 31
 
 
+def streams_at_once(N, device):
+    """Every block of a streamed product of more than 32 rows has a CU: each
+    takes 32 of N columns and a CU to itself."""
+    return N <= 32 * _cus(device.index)
+
+
 def _tile_gemm(epi, y, x, packed, M, N, K, plan, part=None, bias=None,
                res=None, sq=None, rstd=None, rstd_nt=0, inv_h=0.0, eps=0.0,
                gelu=0, rope=(None,) * 7 + (0,) * 4):

@@ -842,6 +842,12 @@ def library_products():
     return not hip.USE_WSTREAM
 
 
+def streams_at_once(N, device):
+    """Every block of a streamed product of N columns has a CU."""
+    from . import hip
+    return hip.streams_at_once(N, device)
+
+
 def asked_parts(K):
     """The parts that a switch asks of streamed products over K, or None."""
     from . import hip

@@ -99,6 +99,30 @@ def test_parts_asked_for(env, every, over_tiles, monkeypatch):
     assert seen == over_tiles
 
 
+@pytest.mark.parametrize("heads, rounds", [(48, 1), (56, 2), (64, 2)])
+def test_second_round_of_streams(heads, rounds, monkeypatch):
+    """Rotated products go over tiles where their streams' blocks of 32
+    columns are more than the CUs."""
+    import dataclasses
+    from ollamamq_amd.models import LlamaModel, PRESETS
+    from ollamamq_amd.ops import hip
+    cfg = dataclasses.replace(PRESETS["tiny"], n_heads=heads, n_kv_heads=8)
+    blocks = (cfg.q_dim + 2 * cfg.kv_dim) // 32
+    assert -(-blocks // hip._cus(0)) == rounds
+    model = LlamaModel(cfg, device="cuda:0", dtype=torch.bfloat16, seed=5)
+    seen, product = [], hip.tile_qkv_rope
+    monkeypatch.setattr(hip, "tile_qkv_rope",
+                        lambda *a: seen.append(a) or product(*a))
+    for n in (49, 128):
+        step = [[(0, range(n), [n - 1])]]
+        got, k1, v1 = _run(model, cfg, True, step)
+        want, k2, v2 = _run(model, cfg, False, step)
+        _close(got[0].float(), want[0].float())
+        for a, b in ((k1, k2), (v1, v2)):
+            _close(a[b != 0], b[b != 0])    # the pools hold zeros elsewhere
+    assert len(seen) == (2 * cfg.n_layers if rounds > 1 else 0)
+
+
 @pytest.mark.parametrize("streams", [True, False])
 def test_library_products_asked_for(streams, monkeypatch):
     """OLLAMAMQ_NO_WSTREAM reaches prompts of more rows than the chain's."""
