@@ -22,16 +22,17 @@ def _close(a, b):
     assert off.max() <= 10 * 2 ** -7 * size
 
 
-def _run(model, cfg, fused, steps):
+def _run(model, cfg, fused, steps, streams=5, ctx=256, pages=96):
     """Logits of every step, and the keys and values at the end; a step is a
     list of (stream, tokens, wanted places)."""
     from ollamamq_amd.engine import LlamaEngine, PagedKVCache
     model.fused_chain = fused
-    kv = PagedKVCache.for_model(cfg, n_pages=96, max_slots=6, max_ctx=256,
-                                device="cuda:0", dtype=torch.bfloat16)
+    kv = PagedKVCache.for_model(cfg, n_pages=pages, max_slots=streams + 1,
+                                max_ctx=ctx, device="cuda:0",
+                                dtype=torch.bfloat16)
     eng = LlamaEngine(model, kv, max_batch=4)
     eng.use_graphs = False
-    streams = [eng.open_stream() for _ in range(5)]
+    streams = [eng.open_stream() for _ in range(streams)]
     out = [eng.feed([(streams[i], list(t), list(w)) for i, t, w in step])
            for step in steps]
     return out, kv.k_pool.float(), kv.v_pool.float()
