@@ -870,10 +870,11 @@ def tile_residual(x, packed, M, N, K, res):
     return hip.tile_residual(x, packed, M, N, K, res)
 
 
-def tile_gu(x, packed, M, N, K, rstd, rstd_nt, inv_h, eps):
-    """rmsnorm -> gate_up GEMM -> SwiGLU, one kernel."""
+def tile_gu(x, packed, M, N, K, rstd, rstd_nt, inv_h, eps, act="silu"):
+    """rmsnorm -> gate_up GEMM -> SwiGLU, or with another activation of the
+    gate (see gateup_swiglu), one kernel."""
     from . import hip
-    return hip.tile_gu(x, packed, M, N, K, rstd, rstd_nt, inv_h, eps)
+    return hip.tile_gu(x, packed, M, N, K, rstd, rstd_nt, inv_h, eps, act)
 
 
 def sample(logits, temperature, top_k, top_p, generator=None):
