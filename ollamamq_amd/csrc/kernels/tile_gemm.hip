@@ -777,7 +777,7 @@ double estimate(int M, int N, int K, int hm, int hn, int ks, int cus)
 // columns); at 25 others what it chooses for a layer takes 0.5 % more than the
 // best choice on average and 4 % at most.  From 65 to 128 rows, weights not in
 // cache, o and down of 3584 to 8192 columns: down 0 to 7 % more than the best;
-// o of up to 4096 columns would take 5 to 15 % less over tiles of 64 x 64, which
+// o of up to 4096 columns would take 5 to 20 % less over tiles of 64 x 64, which
 // are not weighed there.
 // Few rows are weights' reads: the smallest tiles, in as many parts as there are
 // CUs but of no fewer than 1536 of K (64 rows of 4096 x 4096 and 4096 x 14336
