@@ -62,7 +62,8 @@ __global__ __launch_bounds__(BS) void k_rms_residual(
     int bare,                           // no x at all
     Route rt)
 {
-    const int o = blockIdx.x, tid = threadIdx.x;
+    const int o = FR ? frag_row_of(blockIdx.x, gridDim.x) : blockIdx.x;
+    const int tid = threadIdx.x;
     const int64_t r = rows ? rows[o] : o;
     __shared__ float red[2][BS / 64];
     float x[NV][VEC];
@@ -378,7 +379,7 @@ __global__ __launch_bounds__(BS) void k_rms_gate(
     T* __restrict__ out, const float* __restrict__ o,
     const float* __restrict__ w, Rows<P> gate, int og, int N, float eps)
 {
-    const int64_t t = blockIdx.x;
+    const int64_t t = FR ? frag_row_of(blockIdx.x, gridDim.x) : blockIdx.x;
     const int tid = threadIdx.x;
     const float* row = o + t * N;
     __shared__ float red[BS / 64];

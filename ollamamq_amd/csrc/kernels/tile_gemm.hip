@@ -37,6 +37,13 @@
 //                         114, 320
 //   4096 x 14336          112, 213, 610; here 76 (three parts and what adds
 //                         them up), 204, 626
+// Rows that are normed already (tile_rows_bf16), for 559, 1200 and 4096 rows:
+//   28672 x 4096, gated   library product and activation 147, 268, 747; here 105,
+//                         223, 722
+//   16384 x 4096          74, 142, 405; here 71, 131, 420
+//   10816 x 4096          54, 97, 399; here 52, 90, 290
+//   4096 x 14336          115, 157, 325; here 64, 115 (parts, left to the reader),
+//                         316
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -46,7 +53,7 @@
 
 namespace {
 
-enum { RESIDUAL, GATED, ROPE, PARTS };
+enum { RESIDUAL, GATED, ROPE, PARTS, ROWS, ROW_PARTS };
 
 // where a rotated or plain key and value go (ROPE)
 struct Append {
@@ -61,15 +68,16 @@ struct Append {
 };
 
 struct TileArgs {
-    bf16* y;              // RESIDUAL, GATED: fragment layout; ROPE: [M, N]
-    float* part;          // PARTS: see k_tile_fold; GATED, ROPE: [M] scratch
+    bf16* y;              // RESIDUAL, GATED: fragment layout; ROPE, ROWS: [M, N]
+    float* part;          // PARTS: see k_tile_fold; ROW_PARTS: [ks, M, N];
+                          // GATED, ROPE: [M] scratch
     const bf16* x;
     const bf16* w;
     const bf16* bias;     // ROPE: [N] or null, in W's order
     const bf16* res;      // RESIDUAL: the residual stream, may be y
     float* sq;            // RESIDUAL: [M, tiles of columns] sums of squares
     const float* rstd;    // GATED, ROPE: [M, rstd_nt] sums of squares of x
-    int rstd_nt;
+    int rstd_nt;          // GATED: 0 where x is normed already
     float inv_h, eps;
     int M, N, K;
     int mt, nt, ks, gm;   // tiles of rows, of columns, parts of K, rows a group
@@ -131,6 +139,21 @@ DEV void swap32(f32x4& a, f32x4& b) {
         a[i] = __uint_as_float(r[0]);
         b[i] = __uint_as_float(r[1]);
     }
+}
+
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+// Lanes 16 g of a and b hold four columns each; those of two such groups side by
+// side: a's eight on the first of them, b's on the second
+DEV u32x4 trade16(const f32x4& a, const f32x4& b) {
+    typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+    const auto pack = [](const f32x4& v) {
+        return __builtin_bit_cast(u32x2, bf16x4{(__bf16)v[0], (__bf16)v[1],
+                                                (__bf16)v[2], (__bf16)v[3]});
+    };
+    const u32x2 p = pack(a), q = pack(b);
+    const auto lo = __builtin_amdgcn_permlane16_swap(p[0], q[0], false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(p[1], q[1], false, false);
+    return u32x4{lo[0], hi[0], lo[1], hi[1]};
 }
 
 // n / (1 + e), e not negative, as close as the division is: a reciprocal and
@@ -334,8 +357,9 @@ __global__ __launch_bounds__(256, 1) void k_tile_gemm(const TileArgs a)
             const int r = i * 256 + threadIdx.x;
             if (r >= HM * 32) continue;
             if (EPI == GATED || EPI == ROPE)
-                if (a.rstd_nt == 1)
-                    row_f[r] = rsqrtf(of_row.sq[i] * a.inv_h + a.eps);
+                if (a.rstd_nt <= 1)
+                    row_f[r] = a.rstd_nt
+                        ? rsqrtf(of_row.sq[i] * a.inv_h + a.eps) : 1.f;
             if (EPI == ROPE) {
                 const Append& ap = a.ap;
                 const int pos = of_row.pos[i];
@@ -409,6 +433,46 @@ __global__ __launch_bounds__(256, 1) void k_tile_gemm(const TileArgs a)
                             *reinterpret_cast<f32x4*>(out + j * 256) =
                                 acc[i][j];
                 }
+        } else if constexpr (EPI == ROW_PARTS) {
+            #pragma unroll
+            for (int i = 0; i < HM; i++) {
+                const int row = m * HM * 32 + row_in(i);
+                float* p = a.part + ((int64_t)k * a.M + row) * a.N
+                           + in_strip(0, 4 * g4);
+                #pragma unroll
+                for (int j = 0; j < HN; j++) {
+                    const int h = hj0 + j;
+                    if (row < a.M && j < live)
+                        *reinterpret_cast<f32x4*>(p + (h >> 1) * 32
+                                                  + (h & 1) * 8) = acc[i][j];
+                }
+            }
+        } else if constexpr (EPI == ROWS) {
+            // Lanes that hold four columns of a row beside four others hold
+            // eight of it, and of the next 16 rows, after trading halves.
+            #pragma unroll
+            for (int i = 0; i < HM; i += 2) {
+                const bool two = i + 1 < HM;
+                const int mine = two && g4 & 1 ? row_in(min(i + 1, HM - 1))
+                                               : row_in(i);
+                const int row = m * HM * 32 + mine;
+                bf16* p = a.y + (int64_t)row * a.N
+                          + (two ? g4 >> 1 << 4 : in_strip(0, 4 * g4));
+                #pragma unroll
+                for (int j = 0; j < HN; j++) {
+                    const int h = hj0 + j;
+                    bf16* at = p + (h >> 1) * 32 + (h & 1) * 8;
+                    const bool ok = row < a.M && j < live;
+                    if (two) {
+                        const u32x4 v = trade16(acc[i][j],
+                                                acc[min(i + 1, HM - 1)][j]);
+                        if (ok) *reinterpret_cast<u32x4*>(at) = v;
+                    } else if (ok) {
+                        put4(at, acc[i][j]);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);     // registers
+            }
         } else if constexpr (EPI == RESIDUAL) {
             // halves of columns are 256 elements apart, strips 1024
             const char* res = reinterpret_cast<const char*>(a.res);
@@ -738,7 +802,7 @@ int launch(TileArgs a, int hm, int hn, int cus, hipStream_t stream)
     TILE(6, 4);
     TILE(4, 4);
     TILE(4, 2);
-    if constexpr (EPI != GATED) TILE(2, 2);
+    if constexpr (EPI == RESIDUAL || EPI == ROPE || EPI == PARTS) TILE(2, 2);
     #undef TILE
     return -110;                            // no such tile
 }
@@ -852,4 +916,28 @@ extern "C" int tile_gemm_bf16(
     k_tile_fold<256><<<dim3((M + 31) / 32 * 2, pieces), 256, 0, stream>>>(
         (bf16*)y, (const bf16*)res, (float*)sq, (const float*)part, M, N, ks);
     return (int)hipGetLastError();
+}
+
+// The same over rows that are normed already: y = act(gate) * up in fragment
+// layout (GATED), x W^T in rows (ROWS) or its ks parts in fp32 (ROW_PARTS).
+extern "C" int tile_rows_bf16(
+    void* y, void* part, const void* x, const void* w, int M, int N, int K,
+    int epi, int hm, int hn, int ks, int gm, int gelu, int cus,
+    hipStream_t stream)
+{
+    const int unit = 32 * tile_stages(hm, hn);     // of K
+    if ((epi != GATED && epi != ROWS && epi != ROW_PARTS) || M < 1 || N < 32
+        || N % 32 || K < unit || K % unit || ks < 1 || ks > K / unit
+        || (int64_t)(M + 31) * N >= (int64_t)1 << 31 || gm < 1 || cus < 8
+        || (epi != ROW_PARTS && ks != 1) || !(epi == ROW_PARTS ? part : y))
+        return -111;
+    TileArgs a{};
+    a.y = (bf16*)y, a.part = (float*)part;
+    a.x = (const bf16*)x, a.w = (const bf16*)w;
+    a.M = M, a.N = N, a.K = K;
+    a.mt = div_up(M, hm * 32), a.nt = div_up(N, hn * 32), a.ks = ks;
+    a.gm = gm, a.gelu = gelu;
+    if (epi == GATED) return launch<GATED>(a, hm, hn, cus, stream);
+    if (epi == ROWS) return launch<ROWS>(a, hm, hn, cus, stream);
+    return launch<ROW_PARTS>(a, hm, hn, cus, stream);
 }

@@ -166,6 +166,12 @@ class HybridModel:
             p is not None for owner in (self, *self.layers)
             for p in owner.packs.values())
 
+    def tiles_take(self, rows: int) -> bool:
+        """Products over tiles take this many rows of every matrix."""
+        return all(ops.tiles_take(rows, *w.shape)
+                   for owner in (self, *self.layers)
+                   for w in owner.matrices().values())
+
     def weight_bytes(self) -> int:
         n = self.embed.numel()
         if self.head is not self.embed:

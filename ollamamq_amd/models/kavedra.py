@@ -336,7 +336,9 @@ class KavedraModel(HybridModel):
         return {} if self.loop_in is None else {"loop_in": self.loop_in}
 
     def _mixer(self, layer, run, h, cache, slot_ids, positions, meta, frag):
-        p = ops.linear_parts(h, layer.w_in, layer.packs.get("w_in"))
+        # parts of many rows are more to read than whole sums are to wait for
+        p = ops.linear_parts(h, layer.w_in, layer.packs.get("w_in"),
+                             8 if slot_ids.shape[0] <= ops.CHAIN_ROWS else 1)
         s, w = layer.spec, layer.mix
         if s.type == "lightning":
             o = ops.lightning(p, w, cache.state[run]["lightning"], slot_ids,
@@ -370,10 +372,15 @@ class KavedraModel(HybridModel):
         run."""
         meta = attn_meta
         idx = meta.logits_idx
-        # few tokens, portions of prompts too: activations in fragment layout
-        frag = (self.frag_decode and 0 < tokens.shape[0] <= ops.CHAIN_ROWS
-                and (idx is None or 0 < idx.shape[0] <= ops.CHAIN_ROWS)
-                and (meta.one_each or self.whole_heads))
+        # Activations in fragment layout: few tokens, portions of prompts too,
+        # and prompts of many, whose products go over tiles
+        T = tokens.shape[0]
+        frag = self.frag_decode and (
+            0 < T <= ops.CHAIN_ROWS
+            and (idx is None or 0 < idx.shape[0] <= ops.CHAIN_ROWS)
+            and (meta.one_each or self.whole_heads)
+            or T > ops.CHAIN_ROWS and not meta.one_each and self.whole_heads
+            and self.tiles_take(T) and not ops.library_products())
 
         def join(x, y, pre, **kw):
             return ops.rms_residual(x, y, None, pre, 1.0, self.cfg.eps,
@@ -403,7 +410,7 @@ class KavedraModel(HybridModel):
         # the logits of few rows, of whatever step
         frag = (self.frag_decode and not return_hidden
                 and self.head_pk is not None
-                and 0 < (tokens if idx is None else idx).shape[0]
+                and 0 < (T if idx is None else idx.shape[0])
                 <= ops.CHAIN_ROWS)
         _, h = join(x, y, self.final_norm if return_hidden
                     else self.head_norm, rows=idx, need_x=False,

@@ -15,8 +15,8 @@ from typing import NamedTuple, Optional
 import torch
 
 from . import reference as ref
-from .interface import (LIGHTNING_CHUNK, AttnMeta, Branches, FragRows,
-                        Partials, Weighted)
+from .interface import (CHAIN_ROWS, LIGHTNING_CHUNK, AttnMeta, Branches,
+                        FragRows, Partials, Weighted)
 
 _LIB_PATH = os.path.join(
     os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
@@ -67,6 +67,7 @@ def _try_load():
     lib.tile_gemm_bf16.argtypes = [*[vp] * 8, i, f, f, *[i] * 11, *[vp] * 7,
                                    i, i, i, i, vp]
     lib.tile_gemm_plan.argtypes = [i, i, i, i, i]
+    lib.tile_rows_bf16.argtypes = [*[vp] * 4, *[i] * 10, vp]
     lib.row_sumsq_bf16.argtypes = [vp, vp, i, i, vp]
     lib.frag_rows_bf16.argtypes = [vp, vp, vp, vp, i, i, i, vp]
     lib.fragify_sumsq_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i, i, i, vp, i,
@@ -647,7 +648,8 @@ def linear_qkv_rope(x, packed, N, bias_rp, cache, layer, positions,
 TILES = ((8, 8), (9, 7), (7, 7), (8, 6), (10, 4), (6, 6), (8, 4), (6, 4),
          (4, 4), (4, 2))
 TILE_LEAST = (2, 2)       # for 64 rows at most, not gated
-TILE_RESIDUAL, TILE_GATED, TILE_ROPE, TILE_PARTS = range(4)
+(TILE_RESIDUAL, TILE_GATED, TILE_ROPE, TILE_PARTS, TILE_ROWS,
+ TILE_ROW_PARTS) = range(6)
 TILE_FOLD = 16            # blocks that add up the parts of a row
 
 
@@ -733,6 +735,42 @@ def tile_qkv_rope(x, packed, M, N, K, bias_rp, cache, layer, positions,
                      _p(cache.page_table), kp, vp, nl, nkl, cache.page_size,
                      cache.page_table.shape[1]))
     return y
+
+
+def _tile_rows(epi, y, x, packed, N, plan, part=None, gelu=0):
+    hm, hn, ks = plan
+    assert x.buf.numel() >= -(-x.rows // 32) * 32 * x.cols \
+        and packed.numel() == N * x.cols
+    _check(_lib.tile_rows_bf16(
+        _p(y), _p(part), _p(x.buf), _p(packed), x.rows, N, x.cols, epi, hm,
+        hn, ks, 8, gelu, _cus(x.buf.device.index), _stream()), "tile_rows")
+
+
+def tile_linear(x, packed, N, most=1, f32=False, plan=None):
+    """x W^T of many rows in fragment layout, in rows, or where it is faster
+    its parts of K, `most` of them at most; f32: parts, if only one."""
+    M, K, dev = x.rows, x.cols, x.buf.device
+    if plan is None:
+        # parts cost their consumer what adding them up costs a residual's
+        plan = tile_plan(M, N, K, TILE_RESIDUAL, _cus(dev.index))
+        if plan[2] > most:
+            plan = tile_plan(M, N, K, TILE_GATED, _cus(dev.index))
+    if plan[2] > 1 or f32:
+        part = torch.empty((plan[2], M, N), dtype=torch.float32, device=dev)
+        _tile_rows(TILE_ROW_PARTS, None, x, packed, N, plan, part)
+        return Partials(part)
+    y = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+    _tile_rows(TILE_ROWS, y, x, packed, N, plan)
+    return y
+
+
+def tile_act(x, packed, N, glu="silu", plan=None):
+    """tile_gu of rows that are normed already."""
+    act = _frag_rows(x.rows, N // 2, x.buf)
+    _tile_rows(TILE_GATED, act.buf, x, packed, N, plan or tile_plan(
+        x.rows, N, x.cols, TILE_GATED, _cus(x.buf.device.index)),
+        gelu=GELU[glu])
+    return act
 
 
 USE_WSTREAM = os.environ.get("OLLAMAMQ_NO_WSTREAM") != "1"
@@ -1004,8 +1042,11 @@ def _parts_ksplit(N, K, most=8):
 
 
 def _linear_frag(x, N, packed, parts, most=8):
-    """Weight-streaming product of an activation in fragment layout."""
+    """Weight-streaming product of an activation in fragment layout, or one
+    over tiles."""
     M, K = x.rows, x.cols
+    if M > CHAIN_ROWS:
+        return tile_linear(x, packed, N, most if parts else 1)
     ks = _parts_ksplit(N, K, most) if parts else _wstream_ksplit(N, K)
     y = part = None
     if ks > 1:
@@ -1026,6 +1067,8 @@ def linear_f32(x, weight, packed=None):
     N = weight.shape[0]
     if isinstance(x, FragRows):
         M, K = x.rows, x.cols
+        if M > CHAIN_ROWS:
+            return tile_linear(x, packed, N, 8, True)
         part = torch.empty((_parts_ksplit(N, K), M, N), dtype=torch.float32,
                            device=weight.device)
         _check(_lib.wstream_gemm_bf16(
@@ -1040,6 +1083,8 @@ def linear_f32(x, weight, packed=None):
 
 def linear_gu_frag(x, packed, N, glu="silu"):
     """linear_gu of an activation in fragment layout, and so its result."""
+    if x.rows > CHAIN_ROWS:
+        return tile_act(x, packed, N, glu)
     act = linear_gu(x.buf, packed, N, K=x.cols, yfrag=1, M_frag=x.rows,
                     glu=glu)
     return FragRows(act, x.rows, N // 2)

@@ -129,7 +129,8 @@ CHAIN_ROWS = 128
 
 class FragRows(NamedTuple):
     """A bf16 activation [rows, cols] in the layout in which the
-    weight-streaming product reads it (GPU, up to CHAIN_ROWS rows)."""
+    weight-streaming product reads it (GPU; from CHAIN_ROWS rows on the
+    product over tiles)."""
     buf: torch.Tensor
     rows: int
     cols: int
