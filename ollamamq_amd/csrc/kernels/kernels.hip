@@ -767,6 +767,26 @@ extern "C" int embed_gather_bf16(void* out, const void* table,
     return (int)hipGetLastError();
 }
 
+// Entries of an int32 table, the page table's new ones of a step.
+__global__ __launch_bounds__(256) void k_set_entries(
+    int* __restrict__ table, int64_t size, const int* __restrict__ place,
+    const int* __restrict__ value, int n)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const int p = place[i];
+    if (p >= 0 && p < size) table[p] = value[i];
+}
+
+extern "C" int set_entries(void* table, int64_t size, const void* place,
+                           const void* value, int n, hipStream_t stream)
+{
+    if (n < 1) return n ? (int)hipErrorInvalidValue : 0;
+    k_set_entries<<<(n + 255) / 256, 256, 0, stream>>>(
+        (int*)table, size, (const int*)place, (const int*)value, n);
+    return (int)hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------
 // Row sum-of-squares: sq[m] = sum_k x[m][k]^2 (fp32).  Seeds the fused
 // rmsnorm-in-GEMM decode chain after the embedding gather (wstream_gemm

@@ -17,12 +17,14 @@ from __future__ import annotations
 
 import itertools
 import time
+from array import array
 from dataclasses import dataclass, field
 from typing import Callable, Dict, List, Optional
 
+import numpy as np
 import torch
 
-from ..ops.interface import AttnMeta
+from ..ops.interface import AttnMeta, Stage
 from ..ops import interface as ops
 from .kvcache import PagedKVCache
 
@@ -366,39 +368,59 @@ class LlamaEngine:
                  n_decode=0, rows=None):
         """One forward of token_list, q_lens tokens per sequence from position
         starts on; logits of every sequence's last token, or of `rows`.  The
-        batch goes to the device in one piece."""
+        batch, the pages it takes and the model's plans for it go to the
+        device in one piece."""
         slots = [s.slot for s in seqs]
-        self.kv.ensure_all([(slot, self.kv.seq_lens[slot] + ql)
-                            for slot, ql in zip(slots, q_lens)])
+        places, values = [], []
+        try:
+            self.kv.grow([(slot, self.kv.seq_lens[slot] + ql)
+                          for slot, ql in zip(slots, q_lens)], places, values)
+            meta, tokens, positions, slot_per_tok = self._send(
+                slots, token_list, starts, q_lens, mode, n_decode, rows,
+                places, values)
+        except BaseException:
+            # whatever it was, pages that a sequence has are in the table
+            if places:
+                ops.set_entries(self.kv.page_table, *(
+                    torch.tensor(v, dtype=torch.int32, device=self.dev)
+                    for v in (places, values)))
+            raise
+        return self.model.forward(tokens, positions, self.kv, slot_per_tok,
+                                  meta)
+
+    def _send(self, slots, token_list, starts, q_lens, mode, n_decode, rows,
+              places, values):
+        """The batch on the device: (meta, tokens, their positions, their
+        slots); places, values: new entries of the page table."""
         kv_lens = [self.kv.seq_lens[slot] for slot in slots]
         cu = [0, *itertools.accumulate(q_lens)]
         want = [c - 1 for c in cu[1:]] if rows is None else rows
-        n, T = len(seqs), len(token_list)
-        host = torch.empty(2 * len(want) + 3 * T + 3 * n + 1,
-                           dtype=torch.int32,
-                           pin_memory=self.dev.type == "cuda")
-        sizes = [2 * len(want), T, T, T, n, n, n + 1]
-        i32 = torch.int32
-        for part, value in zip(host.split(sizes), (
-                torch.tensor(want, dtype=torch.long).view(i32),
-                torch.tensor(token_list, dtype=i32),
-                torch.cat([torch.arange(p, p + ql, dtype=i32)
-                           for p, ql in zip(starts, q_lens)]),
-                torch.repeat_interleave(torch.tensor(slots, dtype=i32),
-                                        torch.tensor(q_lens)),
-                *(torch.tensor(v, dtype=i32)
-                  for v in (slots, kv_lens, cu)))):
-            part.copy_(value)
-        idx, tokens, positions, slot_per_tok, slot_ids, seq_lens, cu_q = \
-            host.to(self.dev, non_blocking=True).split(sizes)
+        stage = Stage()
         meta = AttnMeta(
-            mode=mode, slot_ids=slot_ids, seq_lens=seq_lens, cu_q=cu_q,
-            logits_idx=idx.view(torch.long), max_q=max(q_lens),
-            max_kv=max(kv_lens), n_decode=n_decode,
+            mode=mode, slot_ids=None, seq_lens=None, cu_q=None,
+            logits_idx=None, max_q=max(q_lens), max_kv=max(kv_lens),
+            n_decode=n_decode,
             window=getattr(self.model.cfg, "sliding_window", 0),
-            q_lens=list(q_lens), kv_lens=kv_lens, slots=slots, rows=want)
-        return self.model.forward(tokens, positions, self.kv, slot_per_tok,
-                                  meta)
+            q_lens=list(q_lens), kv_lens=kv_lens, slots=slots, rows=want,
+            stage=stage)
+        first = np.array(starts) - np.array(cu[:-1])
+        for part in (np.array(want, dtype=np.int64).view(np.int32),
+                     array("i", token_list),
+                     np.arange(cu[-1]) + np.repeat(first, q_lens),
+                     np.repeat(slots, q_lens), slots, kv_lens, cu, places,
+                     values):
+            stage.add(part)
+        plan = getattr(self.model, "plan", None)
+        if plan is not None:
+            plan(self.kv, meta)
+        sent = stage.send(self.dev)
+        (idx, tokens, positions, slot_per_tok, meta.slot_ids, meta.seq_lens,
+         meta.cu_q, at, entries) = sent[:9]
+        meta.logits_idx = idx.view(torch.long)
+        meta.settle(sent)
+        if places:
+            ops.set_entries(self.kv.page_table, at, entries)
+        return meta, tokens, positions, slot_per_tok
 
     def _sample(self, seqs, logits):
         if all(s.params.temperature <= 0 for s in seqs):

@@ -74,24 +74,10 @@ class SequenceCache:
         """Grow page lists to cover new_len tokens each, (slot, new_len)
         pairs.  New entries of the page table go to the device together, and
         nothing waits for what it still has to do."""
-        width = self.page_table.shape[1]
         places: List[int] = []
         values: List[int] = []
         try:
-            for slot, new_len in wanted:
-                if new_len > self.max_ctx:
-                    raise RuntimeError(
-                        f"sequence exceeds max_ctx {self.max_ctx}")
-                need = (new_len + self.page_size - 1) // self.page_size
-                pages = self._slot_pages[slot]
-                had = len(pages)
-                if need - had > len(self._free_pages):
-                    raise RuntimeError("KV cache: out of pages")
-                while len(pages) < need:
-                    pages.append(self._free_pages.pop())
-                places.extend(range(slot * width + had, slot * width + need))
-                values.extend(pages[had:])
-                self.seq_lens[slot] = new_len
+            self.grow(wanted, places, values)
         finally:
             table = self.page_table.view(-1)
             if len(places) == 1:
@@ -102,6 +88,28 @@ class SequenceCache:
                     both = both.pin_memory()
                 both = both.to(table.device, non_blocking=True)
                 table.index_copy_(0, both[0], both[1].int())
+
+    def grow(self, wanted: List[Tuple[int, int]], places: List[int],
+             values: List[int]) -> None:
+        """ensure_all without the device: adds the page table's new entries
+        and where they go in the flat table.  What was grown before an error
+        stays, and its entries are there."""
+        width, size = self.page_table.shape[1], self.page_size
+        for slot, new_len in wanted:
+            if new_len > self.max_ctx:
+                raise RuntimeError(
+                    f"sequence exceeds max_ctx {self.max_ctx}")
+            pages = self._slot_pages[slot]
+            had = len(pages)
+            if new_len > had * size:
+                need = (new_len + size - 1) // size
+                if need - had > len(self._free_pages):
+                    raise RuntimeError("KV cache: out of pages")
+                while len(pages) < need:
+                    pages.append(self._free_pages.pop())
+                places.extend(range(slot * width + had, slot * width + need))
+                values.extend(pages[had:])
+            self.seq_lens[slot] = new_len
 
     def can_fit(self, extra_tokens: int) -> bool:
         return len(self._free_pages) * self.page_size >= extra_tokens

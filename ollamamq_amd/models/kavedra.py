@@ -331,9 +331,27 @@ class KavedraModel(HybridModel):
         self.head = put(get("head", (cfg.vocab, W))).contiguous()
         self._pack_weights()
         self.whole_heads = all(s.vdim % 8 == 0 for s in cfg.layers)
+        # a run of every kind of layer: those alike share a plan
+        kinds = {}
+        for run, (li, _) in enumerate(cfg.runs):
+            s = cfg.layers[li]
+            kinds[s.type, s.heads, s.dim, s.vdim, s.kv_heads, s.window,
+                  s.kv_rank, s.rot_dim] = self.layers[li], run
+        self.planned = list(kinds.values())
 
     def matrices(self):
         return {} if self.loop_in is None else {"loop_in": self.loop_in}
+
+    def plan(self, cache, meta):
+        """What the mixers have to know of a batch."""
+        for layer, run in self.planned:
+            s, w = layer.spec, layer.mix
+            if s.type == "lightning":
+                ops.plan_lightning(cache, meta, w)
+            elif s.type == "attention":
+                ops.plan_softmax(cache, run, meta, w, sum(meta.q_lens))
+            else:
+                ops.plan_latent(cache, run, meta, w)
 
     def _mixer(self, layer, run, h, cache, slot_ids, positions, meta, frag):
         # parts of many rows are more to read than whole sums are to wait for

@@ -370,6 +370,10 @@ class LlamaModel:
         return n * self.embed.element_size()
 
     # -- forward -----------------------------------------------------------
+    def plan(self, kv_cache, attn_meta):
+        """What a forward's attention has to know of its batch."""
+        ops.plan_attention(kv_cache, attn_meta, self.n_local_heads)
+
     def forward(
         self,
         tokens: torch.Tensor,      # [T] int32/int64 flat token ids

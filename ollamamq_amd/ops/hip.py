@@ -59,6 +59,7 @@ def _try_load():
     lib.mixed_attn_bf16.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, i, vp, vp,
                                     i, i, i, i, i, i, i, f, i64, i, i, vp]
     lib.embed_gather_bf16.argtypes = [vp, vp, vp, i, i, vp]
+    lib.set_entries.argtypes = [vp, i64, vp, vp, i, vp]
     lib.wstream_gemm_bf16.argtypes = [vp, vp, vp, vp, vp, i, i, i, i64, i,
                                       i, i, vp, i, f, f, vp, vp, i, vp, vp]
     lib.wstream_pure_bf16.argtypes = [vp, vp, i, i, i, vp]
@@ -176,6 +177,8 @@ def available() -> bool:
 
 
 def require():
+    if _lib is not None:
+        return
     _try_load()
     if _lib is None:
         raise RuntimeError(
@@ -408,6 +411,22 @@ def upload(values, dev):
     return t.pin_memory().to(dev, non_blocking=True)
 
 
+def _with_batch(values, dev, meta):
+    """upload, or with the batch itself where that has not been sent."""
+    return upload(values, dev) if meta.stage is None else meta.stage.add(values)
+
+
+def set_entries(table, places, values):
+    """Entries of an int32 table, in one launch."""
+    n = places.shape[0]
+    assert table.dtype == places.dtype == values.dtype == torch.int32 \
+        and table.is_contiguous() and places.is_contiguous() \
+        and values.is_contiguous() and values.shape == places.shape == (n,)
+    if n:
+        _check(_lib.set_entries(_p(table), table.numel(), _p(places),
+                                _p(values), n, _stream()), "set_entries")
+
+
 def _prefill_plan(meta, first, G, KVH, dev):
     """(tiles, waves a block) of the sequences from `first` on, the longest
     walks first; cached on the meta object (one build per forward, shared by
@@ -430,7 +449,7 @@ def _prefill_plan(meta, first, G, KVH, dev):
             items.append((slot, tok, kv - n, row, min(rows, n * G - row)))
         tok += n
     items.sort(key=lambda it: -(it[2] + (it[3] + it[4]) // G))
-    plan = (upload(items, dev) if items else None), waves
+    plan = (_with_batch(items, dev, meta) if items else None), waves
     setattr(meta, key, plan)
     return plan
 
@@ -776,6 +795,7 @@ def tile_act(x, packed, N, glu="silu", plan=None):
 USE_WSTREAM = os.environ.get("OLLAMAMQ_NO_WSTREAM") != "1"
 
 
+@functools.lru_cache(maxsize=1024)
 def _wstream_ksplit(N, K):
     """Measured rules (profiles/r02_gemm_sweep.md + in-graph A/B):
     * small weights (< 64 MB: qkv/o) are ramp/latency-floor-bound —
@@ -1026,6 +1046,7 @@ def _frag_rows(M, cols, like):
                     M, cols)
 
 
+@functools.lru_cache(maxsize=1024)
 def _parts_ksplit(N, K, most=8):
     """Split for a product whose consumer folds the partial sums: the one
     that loads the 256 CUs most evenly, smaller if nearly as good."""
@@ -1292,9 +1313,8 @@ def _latent_plan(meta, w, KW, f32, dev):
         if tiles:
             # the kernels take the last first: the longest walks
             tiles.sort(key=lambda t: t[1] + t[2])
-            groups.append((
-                torch.tensor(gather, dtype=torch.int32).to(dev),
-                torch.tensor(tiles, dtype=torch.int32).to(dev), kv0))
+            groups.append((_with_batch(gather, dev, meta),
+                           _with_batch(tiles, dev, meta), kv0))
         gather, tiles, kv0 = [], [], 0
 
     while i < len(slots):
@@ -1311,9 +1331,8 @@ def _latent_plan(meta, w, KW, f32, dev):
         if kv0 * H * (D + V) * esz > EXPAND_BYTES:
             flush()
     flush()
-    dev_items = torch.tensor(items, dtype=torch.int32).to(dev) \
-        if items else None
-    plan = (n_absorbed, dev_items, kv_absorbed, groups)
+    plan = (n_absorbed, _with_batch(items, dev, meta) if items else None,
+            kv_absorbed, groups)
     setattr(meta, key, plan)
     return plan
 
@@ -1447,7 +1466,7 @@ def _chunk_plan(meta, dev, step_tokens):
         seqs.append((len(chunks), (n + 63) // 64))
         chunks += [(row + t, min(64, n - t)) for t in range(0, n, 64)]
         row += n
-    t32 = lambda x: upload(x, dev) if x else None
+    t32 = lambda x: _with_batch(x, dev, meta) if x else None
     plan = (t32(spans), t32(chunks), t32(seqs), base, row - base)
     setattr(meta, key, plan)
     return plan
@@ -1497,6 +1516,11 @@ LIGHTNING_STEP_TOKENS = 4    # portions up to this walk token by token
 LIGHTNING_MAX_D = 256        # key width the chunk kernels take
 
 
+def lightning_plan(meta, w, dev):
+    return _chunk_plan(meta, dev, LIGHTNING_STEP_TOKENS
+                       if w.dim <= LIGHTNING_MAX_D else 1 << 62)
+
+
 def lightning(p, w, state, slot_ids, positions, meta, frag=False):
     H, D, V = w.heads, w.dim, w.vdim
     rows = _rows(p)
@@ -1520,9 +1544,7 @@ def lightning(p, w, state, slot_ids, positions, meta, frag=False):
         _check(_lib.lightning_step(f32, _p(o), *head, _p(None), nd, H, D, V,
                                    _stream()), "lightning_step")
     if not meta.one_each:
-        spans, chunks, seqs, base, n = _chunk_plan(
-            meta, t.device,
-            LIGHTNING_STEP_TOKENS if D <= LIGHTNING_MAX_D else 1 << 62)
+        spans, chunks, seqs, base, n = lightning_plan(meta, w, t.device)
         if spans is not None:
             _check(_lib.lightning_step(
                 f32, _p(o), *head, _p(spans), spans.shape[0], H, D, V,
@@ -1943,7 +1965,7 @@ def _tile_plan(meta, R, rows, dev):
         row += n
     # the kernels take the last first: the longest walks
     long_ = [item[1:] for item in sorted(long_, key=lambda item: item[0])]
-    t32 = lambda x: upload(x, dev) if x else None
+    t32 = lambda x: _with_batch(x, dev, meta) if x else None
     plan = (t32(short), n_short, kv, t32(long_))
     setattr(meta, key, plan)
     return plan
@@ -2051,6 +2073,13 @@ def qkv_norm_rope_append(p, norms, cache, run, w, rope, slot_ids, positions):
     return q
 
 
+def softmax_plan(meta, w, T, kp, vp):
+    R = w.heads // w.kv_heads
+    rows = _lib.softmax_rows(_is_f32(kp), kp.shape[3], vp.shape[3], T, R,
+                             w.kv_heads)
+    return rows, _tile_plan(meta, R, rows, kp.device)
+
+
 def softmax_attention(q, cache, run, w, slot_ids, positions, meta, frag,
                       gate=None):
     T, H, Dp = q.shape
@@ -2074,8 +2103,7 @@ def softmax_attention(q, cache, run, w, slot_ids, positions, meta, frag,
         n_items, n_tok, kv = T * -(-R // 16), T, meta.max_kv
         short = long_ = None
     else:
-        rows = _lib.softmax_rows(f32, Dp, Vp, T, R, G)
-        short, n_tok, kv, long_ = _tile_plan(meta, R, rows, q.device)
+        rows, (short, n_tok, kv, long_) = softmax_plan(meta, w, T, kp, vp)
         n_items = 0 if short is None else short.shape[0]
 
     def launch(item_rows, items, n, tokens, split, part, ml):

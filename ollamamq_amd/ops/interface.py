@@ -11,6 +11,7 @@ import os
 from dataclasses import dataclass
 from typing import List, NamedTuple, Optional, Union
 
+import numpy as np
 import torch
 
 from . import reference as ref
@@ -23,9 +24,44 @@ def force_ref() -> bool:
 def _use_hip(t: torch.Tensor) -> bool:
     if not t.is_cuda or force_ref():
         return False
-    from . import hip  # deferred: imports/builds the extension
     hip.require()      # raises if the extension is missing on a GPU machine
     return True
+
+
+class Later(NamedTuple):
+    """A tensor that a Stage will have."""
+    index: int
+
+
+class Stage:
+    """What a forward's host side has for the device, sent in one piece: each
+    copy of its own costs the step 10 us on the device and the host 15."""
+
+    ALIGN = 16                      # int32 values: a part is 64-byte aligned
+
+    def __init__(self):
+        self.parts = []
+
+    def add(self, values) -> Later:
+        """values: int32, or what makes an int32 array."""
+        self.parts.append(np.asarray(values, dtype=np.int32))
+        return Later(len(self.parts) - 1)
+
+    def send(self, dev) -> List[torch.Tensor]:
+        """Every part as a tensor, without waiting for what the device still
+        has to do."""
+        sizes = []
+        for part in self.parts:
+            sizes += part.size, -part.size % self.ALIGN
+        host = torch.empty(sum(sizes), dtype=torch.int32,
+                           pin_memory=dev.type == "cuda")
+        flat, at = host.numpy(), 0
+        for i, part in enumerate(self.parts):
+            flat[at:at + part.size] = part.ravel()
+            at += sizes[2 * i] + sizes[2 * i + 1]
+        there = host.to(dev, non_blocking=True).split(sizes)[::2]
+        return [t if part.ndim == 1 else t.view(part.shape)
+                for t, part in zip(there, self.parts)]
 
 
 @dataclass
@@ -59,6 +95,8 @@ class AttnMeta:
     slots: Optional[List[int]] = None
     # host copy of logits_idx
     rows: Optional[List[int]] = None
+    # while the batch has not been sent: what plans made now are sent with
+    stage: Optional[Stage] = None
 
     @property
     def one_each(self) -> bool:
@@ -79,6 +117,17 @@ class AttnMeta:
             self.kv_lens = self.seq_lens.tolist()
             self.slots = self.slot_ids.tolist()
         return self.slots, self.q_lens, self.kv_lens
+
+    def settle(self, sent: List[torch.Tensor]) -> None:
+        """The plans that were made for the stage have its tensors."""
+        def there(v):
+            if isinstance(v, Later):
+                return sent[v.index]
+            return type(v)(map(there, v)) if type(v) in (tuple, list) else v
+        for key, plan in vars(self).items():
+            if key[0] == "_":
+                setattr(self, key, there(plan))
+        self.stage = None
 
     def check_rows(self, n: int) -> None:
         """IndexError where logits_idx names a row that n tokens do not have.
@@ -253,7 +302,6 @@ class LowRank(NamedTuple):
 def low_rank(w: torch.Tensor) -> LowRank:
     if not w.is_cuda:
         return LowRank(w)
-    from . import hip
     return LowRank(w, hip.pack_operand(w))
 
 
@@ -356,21 +404,18 @@ def moe_weights(router, experts, top, put) -> MoeWeights:
 
 def embedding(tokens: torch.Tensor, table: torch.Tensor) -> torch.Tensor:
     if _use_hip(table):
-        from . import hip
         return hip.embedding(tokens, table)
     return table.index_select(0, tokens.long())
 
 
 def rmsnorm_residual(x, residual, weight, eps):
     if _use_hip(x):
-        from . import hip
         return hip.rmsnorm_residual(x, residual, weight, eps)
     return ref.rmsnorm_residual(x, residual, weight, eps)
 
 
 def rope(q, k, positions, cos, sin):
     if _use_hip(q):
-        from . import hip
         return hip.rope(q, k, positions, cos, sin)
     return ref.rope(q, k, positions, cos, sin)
 
@@ -379,7 +424,6 @@ def rope_append(cache, layer, q, k, v, positions, slot_ids, cos, sin):
     """Fused RoPE + KV append (one pass); falls back to the two reference
     ops on CPU."""
     if _use_hip(q):
-        from . import hip
         return hip.rope_append(cache, layer, q, k, v, positions, slot_ids,
                                cos, sin)
     ref.rope(q, k, positions, cos, sin)
@@ -388,14 +432,12 @@ def rope_append(cache, layer, q, k, v, positions, slot_ids, cos, sin):
 
 def kv_append(cache, layer, k, v, slot_ids, positions):
     if _use_hip(k):
-        from . import hip
         return hip.kv_append(cache, layer, k, v, slot_ids, positions)
     return ref.kv_append(cache, layer, k, v, slot_ids, positions)
 
 
 def attention(q, cache, layer, meta: AttnMeta):
     if _use_hip(q):
-        from . import hip
         if meta.mode == "decode":
             return hip.attention_decode(q, cache, layer, meta)
         if meta.mode == "mixed":
@@ -411,7 +453,6 @@ def linear(x, weight, bias=None, packed=None):
     over the pre-packed copy when `packed` is provided (hipBLASLt measured
     1.8-4.6 TB/s vs the ~6.3 TB/s streaming roofline on these shapes)."""
     if _use_hip(weight):
-        from . import hip
         return hip.linear(x, weight, bias, packed)
     return torch.nn.functional.linear(x, weight, bias)
 
@@ -422,7 +463,6 @@ def pack_weight(w):
     them (the per-shape lib-vs-stream policy only applies to the generic
     non-chain dispatch in hip.linear)."""
     if w.is_cuda:
-        from . import hip
         if hip.available():
             return hip.pack_weight(w)
     return None
@@ -433,7 +473,6 @@ def linear_parts(x, weight, packed=None,
     """As linear, but a split product may come back as its partial sums, at
     most `most` of them (few where several consumers add them up)."""
     if _use_hip(weight):
-        from . import hip
         return hip.linear_parts(x, weight, packed, most)
     return torch.nn.functional.linear(x, weight)
 
@@ -446,7 +485,6 @@ def dyt_residual(x, y, post: Optional[DyT], pre: DyT,
     of `tokens`; y a tensor, Partials or None; `rows` selects the rows to
     compute; frag returns h as FragRows.  Returns (x', h)."""
     if _use_hip(pre.w):
-        from . import hip
         return hip.dyt_residual(x, y, post, pre, shift, embed, tokens, rows,
                                 need_x, frag)
     return ref.dyt_residual(x, y, post, pre, shift, embed, tokens, rows)
@@ -455,7 +493,6 @@ def dyt_residual(x, y, post: Optional[DyT], pre: DyT,
 def linear_f32(x, weight, packed=None) -> Union[torch.Tensor, Partials]:
     """As linear_parts, the result fp32 whatever the operands' type."""
     if _use_hip(weight):
-        from . import hip
         return hip.linear_f32(x, weight, packed)
     return torch.nn.functional.linear(x.float(), weight.float())
 
@@ -465,7 +502,6 @@ def polynorm(z, coef, eps, frag=False):
     division by the row's root mean square."""
     t = z.parts if isinstance(z, Partials) else z
     if _use_hip(t):
-        from . import hip
         return hip.polynorm(z, coef, eps, frag)
     return ref.polynorm(z, coef, eps)
 
@@ -473,7 +509,6 @@ def polynorm(z, coef, eps, frag=False):
 def latent_append(cache, run, d, weight, slot_ids, positions, eps):
     """RMS norm of d [T, R] and append to the run's paged latent pool."""
     if _use_hip(d):
-        from . import hip
         return hip.latent_append(cache, run, d, weight, slot_ids, positions,
                                  eps)
     return ref.latent_append(cache, run, d, weight, slot_ids, positions, eps)
@@ -486,7 +521,6 @@ def latent_rope_append(p, cache, run, w: LatentWeights, norm, eps,
     and key part to the run's pool.  -> queries [T, H * (D + rot_dim)]."""
     t = p.parts if isinstance(p, Partials) else p
     if _use_hip(t):
-        from . import hip
         return hip.latent_rope_append(p, cache, run, w, norm, eps, rope,
                                       slot_ids, positions)
     return ref.latent_rope_append(p, cache, run, w, norm, eps, rope,
@@ -500,7 +534,6 @@ def latent_attention(q, cache, run, w: LatentWeights, slot_ids, positions,
     cached latent.  q [T, H*(D+rot_dim)] (rows may be strided) -> [T, H*V],
     times the sigmoid of the gate's columns."""
     if _use_hip(q):
-        from . import hip
         return hip.latent_attention(q, cache, run, w, slot_ids, positions,
                                     meta, frag, gate)
     return ref.latent_attention(q, cache, run, w, meta, gate)
@@ -514,7 +547,6 @@ def rope_qkv_append(p, bias, cache, run, w: SoftmaxAttn, rope: Rope,
     zeros as the pool's are."""
     t = p.parts if isinstance(p, Partials) else p
     if _use_hip(t):
-        from . import hip
         return hip.rope_qkv_append(p, bias, cache, run, w, rope, slot_ids,
                                    positions)
     return ref.rope_qkv_append(p, bias, cache, run, w, rope, slot_ids,
@@ -529,7 +561,6 @@ def qkv_norm_rope_append(p, norms: HeadNorms, cache, run, w: SoftmaxAttn,
     pool's are."""
     t = p.parts if isinstance(p, Partials) else p
     if _use_hip(t):
-        from . import hip
         return hip.qkv_norm_rope_append(p, norms, cache, run, w, rope,
                                         slot_ids, positions)
     return ref.qkv_norm_rope_append(p, norms, cache, run, w, rope, slot_ids,
@@ -543,7 +574,6 @@ def softmax_attention(q, cache, run, w: SoftmaxAttn, slot_ids, positions,
     rope_qkv_append returns it.  -> [T, H*V], a head's result times the
     sigmoid of its gate column."""
     if _use_hip(q):
-        from . import hip
         return hip.softmax_attention(q, cache, run, w, slot_ids, positions,
                                      meta, frag, gate)
     return ref.softmax_attention(q, cache, run, w, meta, gate)
@@ -555,7 +585,6 @@ def lightning(p, w: LightningWeights, state, slot_ids, positions,
     p [T, ...] (a tensor or Partials); state [slots, H, D, V] fp32 is read
     and advanced.  Norm and output gate included.  -> [T, H*V]."""
     if _use_hip(w.powers):
-        from . import hip
         return hip.lightning(p, w, state, slot_ids, positions, meta, frag)
     return ref.lightning(p, w, state, meta)
 
@@ -566,7 +595,6 @@ def gla(p, w: GlaWeights, state, slot_ids, positions, meta: AttnMeta,
     [slots, H, D, V] fp32 is read and advanced.  Head norm and output gate
     included.  -> [T, H*V]."""
     if _use_hip(p):
-        from . import hip
         return hip.gla(p, w, state, slot_ids, positions, meta, frag)
     return ref.gla(p, w, state, meta)
 
@@ -580,7 +608,6 @@ def gated_delta(p, w: GatedDeltaWeights, state, conv_state, slot_ids,
     fp32, are read and advanced.  Head norm and output gate included.
     -> [T, H*V]."""
     if _use_hip(w.norm):
-        from . import hip
         return hip.gated_delta(p, w, state, conv_state, slot_ids, positions,
                                meta, frag)
     return ref.gated_delta(p, w, state, conv_state, meta)
@@ -594,7 +621,6 @@ def general_delta(p, w: GeneralDeltaWeights, state, slot_ids, positions,
     state [slots, H, D, D] fp32 is read and advanced.  Head norm and output
     gate included.  -> [T, H*D]."""
     if _use_hip(w.norm):
-        from . import hip
         return hip.general_delta(p, w, state, slot_ids, positions, meta,
                                  frag)
     return ref.general_delta(p, w, state, meta)
@@ -610,7 +636,6 @@ def ln_residual(x, y, norm: Optional[LayerNorm], mult, eps, scale=None,
     `rows` selects the rows to compute; frag returns h as FragRows.
     Returns (x', h)."""
     if _use_hip(embed):
-        from . import hip
         return hip.ln_residual(x, y, norm, mult, eps, scale, embed, tokens,
                                rows, need_x, frag, then)
     return ref.ln_residual(x, y, norm, mult, eps, scale, embed, tokens, rows,
@@ -629,7 +654,6 @@ def rms_residual(x, y, post, pre, mult, eps, embed=None, tokens=None,
     appends the token's embedding row to h; frag returns h as FragRows.
     Returns (x', h)."""
     if _use_hip(embed):
-        from . import hip
         return hip.rms_residual(x, y, post, pre, mult, eps, embed, tokens,
                                 embed_scale, rows, need_x, frag, shift=shift,
                                 tail=tail, bare=bare)
@@ -642,7 +666,6 @@ def rms_residual_route(x, y, post, mult, eps, moe, embed=None, tokens=None,
     """rms_residual without `pre`, and moe_route of the new operand:
     (x', h, (chosen, share))."""
     if _use_hip(embed):
-        from . import hip
         return hip.rms_residual_route(x, y, post, mult, eps, moe, embed,
                                       tokens, embed_scale, frag)
     x, h = ref.rms_residual(x, y, post, None, mult, eps, embed, tokens,
@@ -658,7 +681,6 @@ def qk_norm_append(p, cache, run, w: SigmoidAttn, q_norm, k_norm, eps,
     filled up with zeros as the pool's are."""
     t = p.parts if isinstance(p, Partials) else p
     if _use_hip(t):
-        from . import hip
         return hip.qk_norm_append(p, cache, run, w, q_norm, k_norm, eps,
                                   slot_ids, positions)
     return ref.qk_norm_append(p, cache, run, w, q_norm, k_norm, eps,
@@ -670,7 +692,6 @@ def sigmoid_attention(q, cache, run, w: SigmoidAttn, slot_ids, positions,
     """Causal attention with independent key weights over the run's paged
     keys and values; q as qk_norm_append returns it.  -> [T, H*V]."""
     if _use_hip(q):
-        from . import hip
         return hip.sigmoid_attention(q, cache, run, w, slot_ids, positions,
                                      meta, frag)
     return ref.sigmoid_attention(q, cache, run, w, meta)
@@ -680,7 +701,6 @@ def moe_route(h, w: MoeWeights):
     """(experts int32 [T, top], strongest first; their shares fp32 of a
     softmax over all experts), router logits in fp32."""
     if _use_hip(w.router):
-        from . import hip
         return hip.moe_route(h, w)
     return ref.moe_route(h, w)
 
@@ -689,7 +709,6 @@ def moe_experts(h, w: MoeWeights, chosen, share, packs=None) -> Weighted:
     """The chosen experts' outputs for every token, not yet added up.
     packs: packed copies of gate_up and down for decode."""
     if _use_hip(w.router):
-        from . import hip
         return hip.moe_experts(h, w, chosen, share, packs or {})
     return ref.moe_experts(h, w, chosen, share)
 
@@ -697,7 +716,6 @@ def moe_experts(h, w: MoeWeights, chosen, share, packs=None) -> Weighted:
 def swiglu(gate_up, act="silu"):
     """act(gate) * up with act "silu" or "gelu_tanh"."""
     if _use_hip(gate_up):
-        from . import hip
         return hip.swiglu(gate_up, act)
     return ref.swiglu(gate_up, act)
 
@@ -711,10 +729,8 @@ def gateup_swiglu(x, weight, packed_gu=None, act="silu"):
     fragment x-loads double the scattered line traffic.)  FragRows go
     through the fused kernel at any batch and stay FragRows."""
     if isinstance(x, FragRows):
-        from . import hip
         return hip.linear_gu_frag(x, packed_gu, weight.shape[0], act)
     if packed_gu is not None and x.shape[0] <= 32 and _use_hip(x):
-        from . import hip
         if hip.USE_WSTREAM and x.dtype == torch.bfloat16 \
                 and x.stride(1) == 1:
             return hip.linear_gu(x, packed_gu, weight.shape[0], glu=act)
@@ -724,7 +740,6 @@ def gateup_swiglu(x, weight, packed_gu=None, act="silu"):
 def pack_weight_gu(w):
     """GU-interleaved packed copy for the fused gate_up+SwiGLU kernel."""
     if w.is_cuda:
-        from . import hip
         if hip.available():
             return hip.pack_weight_gu(w)
     return None
@@ -736,7 +751,6 @@ def pack_weight_gu(w):
 def row_sumsq(x, out=None):
     """sq[m] = sum(x[m]**2) in fp32 (seeds the chain after embedding)."""
     if _use_hip(x):
-        from . import hip
         return hip.row_sumsq(x, out)
     s = (x.float() ** 2).sum(-1)
     if out is not None:
@@ -755,7 +769,6 @@ def linear_fused(x, packed, N, bias=None, rstd=None, rstd_nt=0,
     K given => x is a 32-row frag-layout buffer streamed linearly;
     yfrag => the output is emitted in frag layout; sem: see
     hip.linear_packed."""
-    from . import hip
     return hip.linear_packed(x, packed, bias, N, rstd=rstd,
                              rstd_nt=rstd_nt, inv_h=inv_h, eps=eps,
                              res=res, sq_out=sq_out, y=y, yfrag=yfrag,
@@ -766,13 +779,11 @@ def fragify_sumsq(x, sq=None, tokens=None, rows=None, add=None, clear=None):
     """Standard [M, H] -> 32-row frag layout + per-row sum of squares; with
     tokens, of their rows of the embedding table x; with rows, of these rows
     of x + add; clear: int32 scratch to set to zero on the way."""
-    from . import hip
     return hip.fragify_sumsq(x, sq, tokens, rows, add, clear)
 
 
 def other_attention(meta) -> bool:
     """A triage switch has another attention take this step."""
-    from . import hip
     return force_ref() or (meta.mode == "prefill"
                            and hip.valu_prefill(meta))
 
@@ -780,7 +791,6 @@ def other_attention(meta) -> bool:
 def attention_frag(q, cache, layer, meta, sem=None):
     """Attention emitting its output in frag layout; sem: see
     hip.attention_decode."""
-    from . import hip
     if meta.one_each:
         return hip.attention_decode(q, cache, layer, meta, True, sem=sem)
     return hip.attention_mixed(q, cache, layer, meta, True, sem)
@@ -789,14 +799,12 @@ def attention_frag(q, cache, layer, meta, sem=None):
 def frag_rows(xf, rows, H, T=None):
     """Rows of an activation of T rows in frag layout, in that layout, and
     their sums of squares (NaN for a row that does not exist)."""
-    from . import hip
     return hip.frag_rows(xf, rows, H, T)
 
 
 def gu_fused(x, packed, N, rstd, rstd_nt, inv_h, eps, K=None, yfrag=0,
              M_frag=32):
     """rmsnorm -> gate_up GEMM -> SwiGLU, one kernel."""
-    from . import hip
     return hip.linear_gu(x, packed, N, rstd=rstd, rstd_nt=rstd_nt,
                          inv_h=inv_h, eps=eps, K=K, yfrag=yfrag,
                          M_frag=M_frag)
@@ -805,7 +813,6 @@ def gu_fused(x, packed, N, rstd, rstd_nt, inv_h, eps, K=None, yfrag=0,
 def pack_weight_qkv_rope(w, nl, nkl):
     """Pair-ordered qkv pack for the fused RoPE/KV-append epilogue."""
     if w.is_cuda and w.shape[1] % 64 == 0:
-        from . import hip
         if hip.available():
             return hip.pack_weight_qkv_rope(w, nl, nkl)
     return None
@@ -813,7 +820,6 @@ def pack_weight_qkv_rope(w, nl, nkl):
 
 def qkv_rope_bias_order(bias, nl, nkl):
     """Reorder a qkv bias to match the pair-ordered pack."""
-    from . import hip
     order = torch.tensor(hip.qkv_rope_order(nl, nkl), device=bias.device)
     return bias.index_select(0, order).contiguous()
 
@@ -822,7 +828,6 @@ def qkv_rope_fused(x, packed, N, bias_rp, cache, layer, positions, slots,
                    cos, sin, nl, nkl, rstd, rstd_nt, inv_h, eps,
                    K=None, M_real=32):
     """rmsnorm -> qkv GEMM -> RoPE -> paged KV append, one kernel."""
-    from . import hip
     return hip.linear_qkv_rope(x, packed, N, bias_rp, cache, layer,
                                positions, slots, cos, sin, nl, nkl,
                                rstd, rstd_nt, inv_h, eps, K=K,
@@ -833,32 +838,27 @@ def qkv_rope_fused(x, packed, N, bias_rp, cache, layer, positions, slots,
 
 def tiles_take(M, N, K):
     """Products over tiles take M rows of a product [M, K] x [N, K]."""
-    from . import hip
     return hip.tiles_take(M, N, K)
 
 
 def library_products():
     """A switch asks for the library's products where it has them."""
-    from . import hip
     return not hip.USE_WSTREAM
 
 
 def streams_at_once(N, device):
     """Every block of a streamed product of N columns has a CU."""
-    from . import hip
     return hip.streams_at_once(N, device)
 
 
 def asked_parts(K):
     """The parts that a switch asks of streamed products over K, or None."""
-    from . import hip
     return hip.asked_parts(K)
 
 
 def tile_qkv_rope(x, packed, M, N, K, bias_rp, cache, layer, positions, slots,
                   cos, sin, nl, nkl, rstd, rstd_nt, inv_h, eps):
     """rmsnorm -> qkv GEMM -> RoPE -> paged KV append, one kernel."""
-    from . import hip
     return hip.tile_qkv_rope(x, packed, M, N, K, bias_rp, cache, layer,
                              positions, slots, cos, sin, nl, nkl, rstd,
                              rstd_nt, inv_h, eps)
@@ -867,14 +867,12 @@ def tile_qkv_rope(x, packed, M, N, K, bias_rp, cache, layer, positions, slots,
 def tile_residual(x, packed, M, N, K, res):
     """res += x W^T; partial sums of squares of the new rows and how many a
     row has."""
-    from . import hip
     return hip.tile_residual(x, packed, M, N, K, res)
 
 
 def tile_gu(x, packed, M, N, K, rstd, rstd_nt, inv_h, eps, act="silu"):
     """rmsnorm -> gate_up GEMM -> SwiGLU, or with another activation of the
     gate (see gateup_swiglu), one kernel."""
-    from . import hip
     return hip.tile_gu(x, packed, M, N, K, rstd, rstd_nt, inv_h, eps, act)
 
 
@@ -882,6 +880,45 @@ def sample(logits, temperature, top_k, top_p, generator=None):
     # Sampler: torch ops compose on-GPU; custom fused kernel in ops/hip.py
     # handles the greedy + temperature paths.
     if _use_hip(logits):
-        from . import hip
         return hip.sample(logits, temperature, top_k, top_p, generator)
     return ref.sample(logits, temperature, top_k, top_p, generator)
+
+
+def set_entries(table, places, values):
+    """table.view(-1)[places] = values, all int32."""
+    if _use_hip(table):
+        hip.set_entries(table, places, values)
+    else:
+        table.view(-1).index_copy_(0, places.long(), values)
+
+
+def plan_attention(cache, meta, heads):
+    """The plan of `attention` made now, to be sent with the batch."""
+    if not meta.one_each and _use_hip(cache.page_table):
+        kvh = cache.n_kv_heads
+        hip._prefill_plan(meta, meta.n_single, heads // kvh, kvh,
+                          cache.page_table.device)
+
+
+def plan_lightning(cache, meta, w: LightningWeights):
+    """That of `lightning`."""
+    if not meta.one_each and _use_hip(cache.page_table):
+        hip.lightning_plan(meta, w, cache.page_table.device)
+
+
+def plan_softmax(cache, run, meta, w: SoftmaxAttn, rows):
+    """That of `softmax_attention` of as many rows."""
+    if not meta.one_each and _use_hip(cache.page_table):
+        kp, vp = cache.key_pool[run], cache.value_pool[run]
+        hip.softmax_plan(meta, w, rows, kp, vp)
+
+
+def plan_latent(cache, run, meta, w: LatentWeights):
+    """That of `latent_attention`."""
+    if not meta.one_each and _use_hip(cache.page_table):
+        pool = cache.latent_pool[run]
+        hip._latent_plan(meta, w, pool.shape[2], hip._is_f32(pool),
+                         pool.device)
+
+
+from . import hip  # noqa: E402  (it takes its types from here)
