@@ -76,8 +76,8 @@ extern "C" int wstream_pure_bf16(void* sink, const void* wp, int N, int K,
 // DEPTH: weights under way per wave, in 4 KiB iterations.
 // XLDS == 2: x in fragment layout (the decode chain).  A CU's loads are what
 // bounds it, x counted: rows past M repeat row M - 1, so few rows cost few
-// cache lines.  4 iterations ahead for 32 rows, in registers for two blocks a
-// CU; 2 for 64, where one block a CU with two of x under way beats two with
+// cache lines.  1 or 4 iterations ahead for 32 rows (frag_depth), in registers
+// for two blocks a CU; 2 for 64, where one block a CU with two of x under way beats two with
 // one (37888 x 3584: 70 us against 79).  28672 x 4096 with its norm and
 // activation: 46 us before for any M, now 44 for 32 rows, 39 for 1.
 // XLDS (requires MT==1): stage the x fragments through a wave-PRIVATE
@@ -824,12 +824,20 @@ static int wide(int cw, void* y, const void* x, const void* wp, int M, int N,
     #undef WIDE
 }
 
-// Iterations ahead for 32 rows in fragment layout: no more than a wave has,
-// as the slots of a first round that it does not have are loaded all the same
+// Iterations ahead for 32 rows in fragment layout: four where every wave has whole
+// rounds of four, or one.  Slots of a first round that a wave does not have are
+// loaded all the same, and 4 KB of each of 16 waves are already twice what a CU
+// can have under way (32 KB, 57 GB/s of weights).  us for 1 and 32 rows, two
+// iterations the same as one within 2 %:
+//                    one          four
+//   28672 x 4096     44.5  49.2   42.6  48.5      8 iterations a wave
+//   37888 x 3584     47.8  55.9   50.3  58.8      7
+//   18432 x 3072     23.5  27.6   26.9  31.9      6
+//   4096 x 14336     22.4  25.1   23.4  26.4      14, in two parts
+//   4096 x 11008     19.0  20.9   19.6  21.4      10 or 11
 static int frag_depth(int K, int ksplit)
 {
-    const int n = K / 64 / (8 * ksplit);
-    return n >= 4 ? 4 : n >= 2 ? 2 : 1;
+    return K % (64 * 8 * 4 * ksplit) ? 1 : 4;
 }
 
 // Fused gate_up @ SwiGLU over GU-interleaved packed weights.
@@ -869,9 +877,8 @@ static int wstream_gu(
         return (int)hipGetLastError();
     }
     const int d = frag_depth(K, 1);
-    auto go = xlds == 2 ? (d == 4   ? k_wstream_gemm<1, 4, 2, GU>
-                           : d == 2 ? k_wstream_gemm<1, 2, 2, GU>
-                                    : k_wstream_gemm<1, 1, 2, GU>)
+    auto go = xlds == 2 ? (d == 4 ? k_wstream_gemm<1, 4, 2, GU>
+                                  : k_wstream_gemm<1, 1, 2, GU>)
               : xlds == 1 ? k_wstream_gemm<1, 1, 1, GU>
                           : k_wstream_gemm<1, 1, 0, GU>;
     go<<<grid, 512, lds, stream>>>(
@@ -931,9 +938,7 @@ extern "C" int wstream_gemm_bf16(
     const int d = frag_depth(K, ksplit);
     if (M <= 32) {
         if (xlds == 2)
-            (d == 4   ? k_wstream_gemm<1, 4, 2>
-             : d == 2 ? k_wstream_gemm<1, 2, 2>
-                      : k_wstream_gemm<1, 1, 2>)
+            (d == 4 ? k_wstream_gemm<1, 4, 2> : k_wstream_gemm<1, 1, 2>)
                 <<<grid, 512, lds_red, stream>>>(
                 (bf16*)y, (float*)part, (const bf16*)x, (const u32x4*)wp,
                 (const bf16*)bias, M, N, K, xs, ksplit, rp, rstd_nt,
@@ -1018,9 +1023,8 @@ extern "C" int wstream_qkv_rope_bf16(
             (const bf16*)bias, M, N, K, xs, 1, (const float*)rstd_parts,
             rstd_nt, inv_h, eps, nullptr, nullptr, rp, 0, nullptr);
     else if (xf)
-        (d == 4   ? k_wstream_gemm<1, 4, 2, 0, 1>
-         : d == 2 ? k_wstream_gemm<1, 2, 2, 0, 1>
-                  : k_wstream_gemm<1, 1, 2, 0, 1>)
+        (d == 4 ? k_wstream_gemm<1, 4, 2, 0, 1>
+                : k_wstream_gemm<1, 1, 2, 0, 1>)
             <<<grid, 512, lds, stream>>>(
             (bf16*)y, nullptr, (const bf16*)x, (const u32x4*)wp,
             (const bf16*)bias, M, N, K, xs, 1, (const float*)rstd_parts,
