@@ -27,6 +27,7 @@
 // ksplit>1 writes fp32 partials; the consumer folds them, or the block that
 // arrives last at a tile (x in fragment layout, or with a fused epilogue), or
 // k_wstream_combine (+bias).
+#include <algorithm>
 #include "act.h"
 #include "tile_mma.h"
 
@@ -617,44 +618,55 @@ void k_wstream_gemm(
 }
 
 // ---------------------------------------------------------------------------
-// Many columns for 33 to 128 rows in fragment layout: gate-up and logits.  A
-// CU moves some 20 bytes a clock through its vector loads whatever they are,
-// and k_wstream_gemm reads all rows for every 32 columns: three units of 4 KB
-// a step of 64 with 64 rows, five with 128, of which one is weights.  Here a
-// block takes CW tiles of 32 columns and its waves share the activations
-// through LDS, CW + rows / 32 units for CW of weights: 8 / CW groups of CW
-// waves walk parts of K, a step of every group staged at a time, the next one
-// on its way in registers.  The barrier leaves loads in flight.  With norm and
-// activation, K 4096, us for 64 and 128 rows:
-//   16384   36 and 42 (k_wstream_gemm 36 and 50)
-//   28672   47 and 57 (64 and 93; library product, norm and activation 63)
-//  128256  179 and 200 (250 and 362)
+// Many columns for rows in fragment layout: gate-up and logits.  A CU has 32 KB
+// of loads under way, in order: rows that L2 has queue behind weights from
+// memory, 50 GB/s of both together, 136 of what L2 has alone.  So k_wstream_gemm,
+// which reads all rows for every 32 columns, loads three units of 4 KB a step of
+// 64 with 64 rows, five with 128, of which one is weights.  Here a block takes CW
+// tiles of 32 columns and its waves share the activations through LDS, CW + rows
+// / 32 units for CW of weights: groups of CW waves walk parts of K, a step of
+// every group staged at a time, the next one on its way in registers.  The
+// barrier leaves loads in flight.  With norm and activation, us for 64 and 128
+// rows:
+//   16384 x 4096   35 and 43 (k_wstream_gemm 35 and 48)
+//   28672 x 4096   46 and 53 (63 and 88; library product, norm and activation 63)
+//   37888 x 3584   52 and 58 (78 and 109; four and eight tiles 69 and 70)
+//  128256 x 4096  185 and 209 (265 and 380)
 // Products in parts stay with k_wstream_gemm: adding up the parts of several
 // tiles costs one block more than the loads saved (4096 x 14336, 128 rows:
 // 56 us against 49).  More weights or activations under way give nothing.
+
+// parts of K that a block's waves walk side by side: eight to twelve waves
+static constexpr __host__ __device__ int wide_parts(int cw)
+{
+    return cw == 3 ? 3 : cw == 2 ? 4 : cw == 8 ? 1 : 2;
+}
 // bytes for two stages of activations, or the sums that follow them
 static constexpr __host__ __device__ int wide_lds(int mt, int cw)
 {
-    const int x = 2 * (8 / cw) * mt * 4096, sums = 8 * 32 * 33 * 4;
+    const int kw = wide_parts(cw);
+    const int x = 2 * kw * mt * 4096, sums = cw * kw * 32 * 33 * 4;
     return x > sums ? x : sums;
 }
 
 template <int MT, int CW, int GU>
-__global__ __launch_bounds__(512, 1) void k_wide(
+__global__ __launch_bounds__(CW * wide_parts(CW) * 64, 1) void k_wide(
     bf16* __restrict__ y,            // [M, N], with GU [M, N / 2]
     const u32x4* __restrict__ x,     // [M, K] in fragment layout
     const u32x4* __restrict__ wp, int M, int N, int K,
     const float* __restrict__ rstd_parts, int rstd_nt, float inv_h,
     float eps, int yfrag)
 {
-    constexpr int KW = 8 / CW, DEPTH = CW == 4 ? 2 : 4;
+    constexpr int KW = wide_parts(CW), BS = CW * KW * 64;
+    constexpr int DEPTH = CW > 2 && CW < 8 ? 2 : 4;
+    static_assert(BS >= 512);                  // lanes for the rows' sums
     constexpr int STAGE = KW * MT * 256;               // 16-byte units
-    constexpr int NX = (STAGE + 511) / 512;
+    constexpr int NX = (STAGE + BS - 1) / BS;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int cw = wid % CW, kw = wid / CW;
     const int NB = K >> 6, tiles = N >> 5;
-    auto from = [&](int k) { return (int)((int64_t)k * NB / KW); };
+    auto from = [&](int k) { return k * NB / KW; };
     const int lo = from(kw), hi = from(kw + 1), steps = (NB + KW - 1) / KW;
     // tiles past the last repeat it and are not stored
     const int t0 = blockIdx.x * CW;
@@ -672,27 +684,33 @@ __global__ __launch_bounds__(512, 1) void k_wide(
             w[s][j].u = __builtin_nontemporal_load(
                 wq + (int64_t)min(b, max(hi, 1) - 1) * 256 + j * 64);
     };
+    const u32x4* xq[NX];
+    #pragma unroll
+    for (int i = 0; i < NX; i++) {
+        const int e = i * BS + tid, u = min(e >> 8, KW * MT - 1);
+        xq[i] = x + (int64_t)(u % MT) * K * 4 + (int64_t)from(u / MT) * 256
+                + (e & 255);
+    }
     auto ldx = [&](int r) {
         #pragma unroll
         for (int i = 0; i < NX; i++) {
-            const int u = (tid >> 8) + i * 2;          // group and row tile
-            if (u >= KW * MT) break;
-            const int b = min(from(u / MT) + r, NB - 1);
-            xr[i] = x[(int64_t)(u % MT) * K * 4 + (int64_t)b * 256
-                      + (tid & 255)];
+            if (STAGE % BS && i == NX - 1 && i * BS + tid >= STAGE) break;
+            const int u = (i * BS + tid) >> 8;
+            const int rr = min(r, NB - 1 - from(u / MT));
+            xr[i] = xq[i][(int64_t)rr * 256];
         }
     };
     auto stx = [&](int r) {
         #pragma unroll
         for (int i = 0; i < NX; i++)
-            if ((tid >> 8) + i * 2 < KW * MT)
-                x_s[(r & 1) * STAGE + i * 512 + tid] = xr[i];
+            if (i * BS + tid < STAGE)
+                x_s[(r & 1) * STAGE + i * BS + tid] = xr[i];
     };
     #pragma unroll
     for (int s = 0; s < DEPTH; s++) ldw(s, lo + s);
     ldx(0);
     // the norm's partial sums, FL lanes a row
-    constexpr int FL = MT == 2 ? 8 : 4;
+    constexpr int FL = MT == 1 ? 16 : MT == 2 ? 8 : 4;
     float rsum = 0.f;
     if (rstd_parts && tid / FL < M) {
         const float* p = rstd_parts + (int64_t)(tid / FL) * rstd_nt;
@@ -753,8 +771,7 @@ __global__ __launch_bounds__(512, 1) void k_wide(
         };
         constexpr int C = GU ? 16 : 32;                // columns of a tile
         const int cols = GU ? N / 2 : N;
-        #pragma unroll
-        for (int e = tid; e < CW * 32 * C; e += 512) {
+        for (int e = tid; e < CW * 32 * C; e += BS) {
             const int n = e % C, c = e / C % CW, mr = e / (C * CW);
             const int row = m * 32 + mr, col = (t0 + c) * C + n;
             if (row >= M || t0 + c >= tiles) continue;
@@ -774,22 +791,42 @@ __global__ __launch_bounds__(512, 1) void k_wide(
 // KB a step of K.  A block of k_wide loads its tiles and all rows, or waits: two
 // tiles take what 4.8 + mt / 2 units take.  A tile of k_wstream_gemm (1), of
 // which a CU has several at a time, takes 0.8 (1 + mt), its rows coming from
-// L1 at times.  For 4096 columns of K a unit is 6 us.  us of 1, 2, 4 and 8:
-//   16384 x 4096,  40 rows  30  36  35  56      22016 x 4096,  40  42  56  37  58
-//                  96       41  39  43  63      37888 x 3584,  40  67  71  64  57
-//   11008 x 2048, 112       26  23  26  39                     64  75  72  65  57
-// Over 11 widths and 33 to 128 rows the choice takes 0.1 % more than the best
-// one; one by loads alone, k_wstream_gemm's counted by rows, 2.5 %.
-static int wide_tiles(int M, int N)
+// L1 at times.  Numbers other than 2, 4 and 8 are for one round of blocks: of
+// several rounds the weights' reads are what is left.  us, K 4096 but for
+// 37888 x 3584 and 32000 x 2048 (the last two):
+//                 rows    1    2    3    4    5    6    8
+//   16384           40   30   36   34   35   43   46   56
+//   22016           48   46   58   38   40   44   49   58
+//                  128   68   70   45   49   54   57   72
+//   28672           64   63   65   66   46   48   52   61
+//   37888           48   71   74   64   67   51   53   60
+//                  128  109   95   78   86   58   60   70
+//   32000           48   39   39   40   34   30   31   36
+// Over 23 matrices and 33 to 128 rows the choice takes 1 % more than the best
+// one, with 2, 4 and 8 alone 2.8 %.
+// Up to 32 rows the stream's own blocks, two a CU, read at the memory's rate; 25
+// rows and more are all the cache lines that 32 are, and blocks that fill half
+// of a last round wait for them (32 rows, stream and k_wide: 22016 x 4096 37.0
+// and 35.1, 37888 x 3584 53.2 and 50.4, 128256 x 4096 191 and 177; 28672 x 4096
+// 46.5 and 47.0, 32000 x 2048 27.7 and 28.0).
+static int wide_tiles(int M, int N, int K)
 {
     const int tiles = N / 32, mt = (M + 31) / 32;
+    const int whole = (tiles + 255) / 256;     // of one round of blocks
+    if (M <= 32) {
+        if (M <= 24 || K < 3072) return 1;
+        if (tiles >= 2048) return 8;
+        return tiles > 512 && (-tiles & 511) > 256 ? whole : 1;
+    }
     int best = 1;
-    double least = (tiles + 255) / 256 * 0.8 * (1 + mt);
+    double least = whole * 0.8 * (1 + mt);
     // two tiles of 64 rows are 5.8 units, one after the other 4.8 at most
-    for (int cw = mt == 2 ? 4 : 2; cw <= 8; cw *= 2) {
+    for (int cw = mt == 2 ? 3 : 2; cw <= 8; cw++) {
+        if (cw < whole && (cw & (cw - 1))) continue;
         const int blocks = (tiles + cw - 1) / cw;
         const double units = (blocks + 255) / 256
-                             * (cw == 2 ? 4.8 + 0.5 * mt : cw + mt);
+                             * std::max<double>(cw + mt,
+                                                cw < 4 ? 4.8 + 0.5 * mt : 0);
         if (units < least) {
             least = units;
             best = cw;
@@ -809,19 +846,27 @@ static int wide(int cw, void* y, const void* x, const void* wp, int M, int N,
         const hipError_t e = hipFuncSetAttribute(
             (const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) return (int)e;
-        k<<<(N / 32 + cw - 1) / cw, 512, lds, stream>>>(
+        k<<<(N / 32 + cw - 1) / cw, cw * wide_parts(cw) * 64, lds, stream>>>(
             (bf16*)y, (const u32x4*)x, (const u32x4*)wp, M, N, K,
             (const float*)rstd_parts, rstd_nt, inv_h, eps, yfrag);
         return (int)hipGetLastError();
     };
-    #define WIDE(MT)                                                       \
-        return cw == 8   ? go(k_wide<MT, 8, GU>)                           \
-               : cw == 4 ? go(k_wide<MT, 4, GU>)                           \
-                         : go(k_wide<MT, 2, GU>)
-    if (mt == 2) return cw == 8 ? go(k_wide<2, 8, GU>) : go(k_wide<2, 4, GU>);
-    if (mt == 3) WIDE(3);
+    #define WIDE(CW)                                                       \
+        if (cw == CW)                                                      \
+            return mt == 1   ? go(k_wide<1, CW, GU>)                       \
+                   : mt == 2 ? go(k_wide<2, CW, GU>)                       \
+                   : mt == 3 ? go(k_wide<3, CW, GU>)                       \
+                             : go(k_wide<4, CW, GU>)
+    if (cw == 2 && mt > 2)
+        return mt == 3 ? go(k_wide<3, 2, GU>) : go(k_wide<4, 2, GU>);
+    WIDE(3);
     WIDE(4);
+    WIDE(5);
+    WIDE(6);
+    WIDE(7);
+    WIDE(8);
     #undef WIDE
+    return -105;                                       // no such tiles
 }
 
 // Iterations ahead for 32 rows in fragment layout: four where every wave has whole
@@ -852,12 +897,14 @@ static int wstream_gu(
     dim3 grid(N / 32, 1);
     const int lds = (xlds == 1 ? 16 * 4096 : 8 * 32 * 32 * 4) + 512;
     if (M > (xlds == 2 ? 128 : 64)) return -104;   // rows of a block
+    if (xlds == 2) {           // frag chain
+        const int cw = wide_tiles(M, N, K);
+        if (cw > 1)
+            return wide<GU>(cw, act, x, wp, M, N, K, rstd_parts, rstd_nt,
+                            inv_h, eps, yfrag, stream);
+    }
     if (M > 32) {
-        if (xlds == 2) {       // frag chain at batches 33..128
-            const int cw = wide_tiles(M, N);
-            if (cw > 1)
-                return wide<GU>(cw, act, x, wp, M, N, K, rstd_parts, rstd_nt,
-                                inv_h, eps, yfrag, stream);
+        if (xlds == 2) {
             (M <= 64   ? k_wstream_gemm<2, 2, 2, GU>
              : M <= 96 ? k_wstream_gemm<3, 2, 2, GU>
                        : k_wstream_gemm<4, 2, 2, GU>)
@@ -936,6 +983,12 @@ extern "C" int wstream_gemm_bf16(
     if (ksplit > 1 && !sem && (rstd_parts || res_in || sq_parts || yfrag))
         return -100;
     const int d = frag_depth(K, ksplit);
+    if (xlds == 2 && ksplit == 1 && y && !bias && !ri && !sq) {
+        const int cw = wide_tiles(M, N, K);
+        if (cw > 1)
+            return wide<0>(cw, y, x, wp, M, N, K, rp, rstd_nt, inv_h, eps,
+                           yfrag, stream);
+    }
     if (M <= 32) {
         if (xlds == 2)
             (d == 4 ? k_wstream_gemm<1, 4, 2> : k_wstream_gemm<1, 1, 2>)
@@ -960,10 +1013,6 @@ extern "C" int wstream_gemm_bf16(
                 inv_h, eps, ri, sq, {}, yfrag, sem);
     } else {
         if (xlds == 2) {
-            const int cw = wide_tiles(M, N);
-            if (ksplit == 1 && y && !bias && !ri && !sq && cw > 1)
-                return wide<0>(cw, y, x, wp, M, N, K, rp, rstd_nt, inv_h,
-                               eps, yfrag, stream);
             (M <= 64   ? k_wstream_gemm<2, 2, 2>
              : M <= 96 ? k_wstream_gemm<3, 2, 2>
                        : k_wstream_gemm<4, 2, 2>)
