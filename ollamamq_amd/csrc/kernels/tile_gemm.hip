@@ -83,6 +83,7 @@ struct TileArgs {
     int mt, nt, ks, gm;   // tiles of rows, of columns, parts of K, rows a group
     int gelu;
     Append ap;
+    int rows_at;          // bytes of LDS before what is kept of rows
 };
 
 // 1 KB pieces to LDS, a lane's 16 bytes at base + voff to lds + 16 * lane.  An
@@ -100,6 +101,11 @@ DEV void to_lds1(uint64_t b0, int voff, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
                  "global_load_lds_dwordx4 %1, %2 offset:%3"
                  :: "s"(lds), "v"(voff), "s"(b0), "n"(O0) : "memory");
+}
+DEV void to_lds4(const void* b0, int voff, uint32_t lds) {   // 256 bytes
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+                 "global_load_lds_dword %1, %2"
+                 :: "s"(lds), "v"(voff), "s"((uint64_t)b0) : "memory");
 }
 template <int N> DEV void wait_loads() {
     asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
@@ -170,8 +176,15 @@ DEV float over_1_and(float n, float e) {
 // stages of LDS; four keep three slabs of a large tile under way, small tiles
 // need more of their slabs for as many bytes
 constexpr int tile_stages(int hm, int hn) { return hm + hn <= 8 ? 8 : 4; }
-constexpr int tile_lds(int hm, int hn) {        // and three values per row
-    return tile_stages(hm, hn) * (hm + hn) * 2048 + hm * 32 * 12;
+// bytes before three values per row: the first tile's sums of squares, nt per
+// row, take the place of the last stage at first and may need more than that
+constexpr int tile_rows_at(int hm, int hn, int nt) {
+    const int stage = (hm + hn) * 2048, last = (tile_stages(hm, hn) - 1) * stage;
+    const int sums = (hm * 128 * nt + 1023) / 1024 * 1024;
+    return last + (sums > stage ? sums : stage);
+}
+constexpr int tile_lds(int hm, int hn, int nt) {
+    return tile_rows_at(hm, hn, nt) + hm * 32 * 12;
 }
 
 template <int HM, int HN, int EPI>
@@ -185,7 +198,7 @@ __global__ __launch_bounds__(256, 1) void k_tile_gemm(const TileArgs a)
     extern __shared__ __align__(1024) char smem[];
     const uint32_t lds0 =
         (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
-    float* row_f = reinterpret_cast<float*>(smem + STAGES * STAGE);
+    float* row_f = reinterpret_cast<float*>(smem + a.rows_at);
     int* row_pos = reinterpret_cast<int*>(row_f + HM * 32);
     int* row_kv = row_pos + HM * 32;
     const int lane = threadIdx.x & 63;
@@ -260,10 +273,73 @@ __global__ __launch_bounds__(256, 1) void k_tile_gemm(const TileArgs a)
         voff += st < STAGES - 1 ? ((st + 1 ^ turn) - (st ^ turn)) * 2048
                                 : (STAGES + turn - (st ^ turn)) * 2048;
     };
-    each<STAGES>([&](auto st) {
+    auto load_stage = [&](auto st) {
         each<PAIRS>([&](auto p) { load(p, st); });
         step(st);
+    };
+
+    // What the results of the first tile's rows need goes straight to LDS,
+    // ahead of the slabs.  Into registers it came behind all of theirs, sums
+    // of squares eight rows of a wave after the other and the page after the
+    // position and the slot.  K of 256, so little else, us with 1, 16 and 128
+    // sums a row: 541 x 28672 over 9 x 7, gated, 21.3, 24.4 and 30.1, now 20.7,
+    // 20.5 and 22.9; 1000 x 6144 over 8 x 4, rotated, 15.1, 18.3 and 22.3, now
+    // 15.5, 15.7 and 18.7 (128 there by the other kernel).
+    const bool sums = (EPI == GATED || EPI == ROPE) && a.rstd_nt > 0;
+    const float* sums_s =
+        reinterpret_cast<const float*>(smem + (STAGES - 1) * STAGE);
+    if (sums) {
+        const uint32_t to = lds0 + (STAGES - 1) * STAGE;
+        const int64_t from = (int64_t)m * HM * 32 * a.rstd_nt;
+        const float* p = a.rstd + from;
+        const int end = (int)min((int64_t)HM * 128 * a.rstd_nt,
+                                 ((int64_t)a.M * a.rstd_nt - from) * 4);
+        // past the end the last again
+        if (a.rstd_nt % 4 == 0 && (uint64_t)a.rstd % 16 == 0)
+            for (int i = wid * 1024; i < end; i += 4096)
+                to_lds1<0>((uint64_t)p, min(i + lane * 16, end - 16), to + i);
+        else
+            for (int i = wid * 256; i < end; i += 1024)
+                to_lds4(p, min(i + lane * 4, end - 4), to + i);
+    }
+    // every wave waits for those of its own rows alone
+    auto own_rows = [&](auto f) {
+        if constexpr (EPI == ROPE)
+            for (int i = wid; i < HM / 2; i += 4)
+                f(i * 64 + lane, lds0 + a.rows_at + i * 256);
+    };
+    own_rows([&](int r, uint32_t to) {
+        const int at = min(m * HM * 32 + r, a.M - 1) * 4;
+        to_lds4(a.ap.pos, at, to + HM * 128);
+        to_lds4(a.ap.slot, at, to + HM * 256);
     });
+    each<STAGES - 1>(load_stage);
+    if (sums || EPI == ROPE) {
+        wait_loads<PER * (STAGES - 1)>();
+        own_rows([&](int r, uint32_t to) {
+            const int at = row_kv[r] * a.ap.maxp + row_pos[r] / a.ap.psz;
+            to_lds4(a.ap.ptab, at * 4, to + HM * 256);
+        });
+    }
+    if (sums) {
+        lds_barrier();
+        for (int r = threadIdx.x; r < HM * 32; r += 256) {
+            const float* p = sums_s + r * a.rstd_nt;
+            f32x4 s{};
+            if (a.rstd_nt % 4 == 0)
+                #pragma unroll 4
+                for (int e = 0; e < a.rstd_nt; e += 4)
+                    s += *reinterpret_cast<const f32x4*>(p + e);
+            else
+                for (int e = 0; e < a.rstd_nt; e++) s[0] += p[e];
+            row_f[r] = rsqrtf((s[0] + s[1] + (s[2] + s[3])) * a.inv_h
+                              + a.eps);
+        }
+        lds_barrier();
+    } else if (EPI == GATED) {
+        for (int r = threadIdx.x; r < HM * 32; r += 256) row_f[r] = 1.f;
+    }
+    load_stage(ic<STAGES - 1>{});
 
     // Operands of a slab: half h of an operand's strips, lanes 16 j .. of it
     // its columns 8 j ..; a wave's halves may begin inside a strip.  Pointers
@@ -330,10 +406,9 @@ __global__ __launch_bounds__(256, 1) void k_tile_gemm(const TileArgs a)
         step(st_);
     };
 
-    // What a row's results need, for the 32 HM rows of a tile: the scale of its
-    // norm, and where its keys and values go.  The loads are under way before
-    // the stores of the tile before, for which they would wait; sums of squares
-    // in parts are added up in place, eight lanes a row.
+    // The same for a later tile: the loads are under way before the stores of
+    // the tile before, for which they would wait.  Sums of squares in parts are
+    // added up by another kernel then.
     struct {
         float sq[2];
         int pos[2], slot[2];
@@ -357,9 +432,8 @@ __global__ __launch_bounds__(256, 1) void k_tile_gemm(const TileArgs a)
             const int r = i * 256 + threadIdx.x;
             if (r >= HM * 32) continue;
             if (EPI == GATED || EPI == ROPE)
-                if (a.rstd_nt <= 1)
-                    row_f[r] = a.rstd_nt
-                        ? rsqrtf(of_row.sq[i] * a.inv_h + a.eps) : 1.f;
+                row_f[r] = a.rstd_nt
+                    ? rsqrtf(of_row.sq[i] * a.inv_h + a.eps) : 1.f;
             if (EPI == ROPE) {
                 const Append& ap = a.ap;
                 const int pos = of_row.pos[i];
@@ -369,25 +443,7 @@ __global__ __launch_bounds__(256, 1) void k_tile_gemm(const TileArgs a)
                 row_kv[r] = page * ap.nkl * ap.psz + pos % ap.psz;
             }
         }
-        if (EPI == GATED || EPI == ROPE)
-            if (a.rstd_nt > 1)
-                for (int r = threadIdx.x >> 3; r < HM * 32; r += 32) {
-                    const float* p =
-                        a.rstd + (int64_t)min(m * HM * 32 + r, a.M - 1)
-                                     * a.rstd_nt;
-                    float s = 0.f;
-                    #pragma unroll 4
-                    for (int e = threadIdx.x & 7; e < a.rstd_nt; e += 8)
-                        s += p[e];
-                    s += __shfl_xor(s, 1, 64);
-                    s += __shfl_xor(s, 2, 64);
-                    s += __shfl_xor(s, 4, 64);
-                    if ((threadIdx.x & 7) == 0)
-                        row_f[r] = rsqrtf(s * a.inv_h + a.eps);
-                }
     };
-    ask_rows(m);
-    keep_rows(m);
     wait_loads<PER * (STAGES - 1)>();
     asm volatile("s_barrier" ::: "memory");
     #pragma unroll
@@ -412,6 +468,12 @@ __global__ __launch_bounds__(256, 1) void k_tile_gemm(const TileArgs a)
         int here = lane;
         asm volatile("" : "+v"(here));
         const int r16 = here & 15, g4 = here >> 4;
+        if (EPI == ROPE && first == 0) {   // pages to places
+            for (int r = threadIdx.x; r < HM * 32; r += 256)
+                row_kv[r] = row_kv[r] * a.ap.nkl * a.ap.psz
+                            + row_pos[r] % a.ap.psz;
+            lds_barrier();
+        }
         if (next_id >= 0) ask_rows(m1);
         auto row_in = [&](int i) {         // within the tile
             const int h = wm * HM + i;
@@ -771,19 +833,26 @@ template <int EPI>
 int launch(TileArgs a, int hm, int hn, int cus, hipStream_t stream)
 {
     const int items = a.mt * a.nt * a.ks;
-    const int lds = tile_lds(hm, hn);
+    constexpr bool NORMED = EPI == GATED || EPI == ROPE;
     // blocks that live together: LDS holds two of the smallest tile
-    const int room = cus * (2 * lds <= 160 * 1024 ? 2 : 1);
+    constexpr int ALL = 160 * 1024;
+    const int each = 2 * tile_lds(hm, hn, 0) <= ALL ? 2 : 1;
+    const int room = cus * each;
     const int grid = (items < room ? items + 7 : room) / 8 * 8;
+    // A block of several tiles takes one sum per row, and so does one without
+    // room for more.  The launch that adds them up takes 3 us.
+    const bool add_up = NORMED && a.rstd_nt > 1
+        && (items > grid || a.rstd_nt > 256
+            || tile_lds(hm, hn, a.rstd_nt) > ALL / each);
+    a.rows_at = tile_rows_at(hm, hn, NORMED && !add_up ? a.rstd_nt : 1);
+    const int lds = a.rows_at + hm * 32 * 12;
     auto go = [&](auto k) {
         const hipError_t e = hipFuncSetAttribute(
             (const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) return (int)e;
-        // A block of several tiles waits for its rows' sums with each, 1.5 us; one
-        // launch for all of them takes 3.  Of one tile it waits for loads anyway.
-        if ((EPI == GATED || EPI == ROPE) && items > grid && a.rstd_nt > 1) {
-            k_row_sums<<<(a.M + 31) / 32, 256, 0, stream>>>(a.part, a.rstd, a.M,
-                                                            a.rstd_nt);
+        if (add_up) {
+            k_row_sums<<<(a.M + 31) / 32, 256, 0, stream>>>(a.part, a.rstd,
+                                                            a.M, a.rstd_nt);
             a.rstd = a.part;
             a.rstd_nt = 1;
         }
