@@ -752,11 +752,13 @@ __global__ __launch_bounds__(256, 1) void k_tile_gemm(const TileArgs a)
 // Sums of a product in parts: y = res + sum of the parts, and sums of squares.
 // A part is [16 rows, in pairs to 32][16 columns] accumulators as k_tile_gemm's
 // lanes hold them.  A block takes 16 rows and a `pieces`-th of the columns, a
-// wave four accumulators at a time with the loads of all of them and of two
-// parts under way: 541 x 4096 in 3 parts, 16 pieces, reads 27 MB in 9.2 us
-// (one accumulator at a time in 8 pieces: 15.3).  y may be res: a lane reads
+// wave four accumulators at a time with the loads of all of them and of the
+// first KS parts under way.  What bounds it is the wait for those: others' caches
+// held them.  us with the product, two parts under way before and all now: 128 x
+// 4096 x 4096 in 4 parts 17.8 and 16.2, 128 x 3584 x 18944 in 4 48.3 and 46.6,
+// 300 x 4096 x 14336 in 3 59.8 and 58.7.  y may be res: a lane reads
 // only what it writes itself afterwards, and the padding of rows past M.
-template <int BS>
+template <int BS, int KS>
 __global__ __launch_bounds__(BS) void k_tile_fold(
     bf16* y, const bf16* res, float* __restrict__ sq,
     const float* __restrict__ part, int M, int N, int ks)
@@ -772,7 +774,7 @@ __global__ __launch_bounds__(BS) void k_tile_fold(
     float s2 = 0.f;
     constexpr int J = 4, W = BS / 64;
     for (int j0 = from + wid; j0 < to; j0 += J * W) {
-        f32x4 v[J];
+        f32x4 v[KS][J];
         bf16x4 old[J];
         const float* p[J];
         int64_t at[J];
@@ -781,23 +783,26 @@ __global__ __launch_bounds__(BS) void k_tile_fold(
             const int j = j0 + i * W < to ? j0 + i * W : j0;
             p[i] = part + ((int64_t)hi * nh + j) * 256 + lane * 4;
             at[i] = frag_at(row, (j >> 1) * 32 + in_strip(j & 1, 4 * g4), N);
-            v[i] = *reinterpret_cast<const f32x4*>(p[i]);
+            #pragma unroll
+            for (int k = 0; k < KS; k++)
+                v[k][i] = *reinterpret_cast<const f32x4*>(p[i] + k * step);
             old[i] = *reinterpret_cast<const bf16x4*>(res + at[i]);
         }
-        #pragma unroll 2
-        for (int k = 1; k < ks; k++)
-            #pragma unroll
-            for (int i = 0; i < J; i++)
-                v[i] += *reinterpret_cast<const f32x4*>(p[i] + k * step);
+        __builtin_amdgcn_sched_barrier(0);     // all of them before any sum
         #pragma unroll
         for (int i = 0; i < J; i++) {
+            f32x4 t = v[0][i];
+            #pragma unroll
+            for (int k = 1; k < KS; k++) t += v[k][i];
+            for (int k = KS; k < ks; k++)
+                t += *reinterpret_cast<const f32x4*>(p[i] + k * step);
             if (row >= M || j0 + i * W >= to) continue;
             #pragma unroll
             for (int e = 0; e < 4; e++) {
-                v[i][e] += (float)old[i][e];
-                s2 += v[i][e] * v[i][e];
+                t[e] += (float)old[i][e];
+                s2 += t[e] * t[e];
             }
-            put4(y + at[i], v[i]);
+            put4(y + at[i], t);
         }
     }
     s2 += __shfl_xor(s2, 16, 64);
@@ -982,8 +987,15 @@ extern "C" int tile_gemm_bf16(
     if (epi == GATED) return launch<GATED>(a, hm, hn, cus, stream);
     if (epi == ROPE) return launch<ROPE>(a, hm, hn, cus, stream);
     if (const int e = launch<PARTS>(a, hm, hn, cus, stream)) return e;
-    k_tile_fold<256><<<dim3((M + 31) / 32 * 2, pieces), 256, 0, stream>>>(
-        (bf16*)y, (const bf16*)res, (float*)sq, (const float*)part, M, N, ks);
+    const dim3 grid((M + 31) / 32 * 2, pieces);
+    #define FOLD(KS) \
+        case KS: k_tile_fold<256, KS><<<grid, 256, 0, stream>>>( \
+            (bf16*)y, (const bf16*)res, (float*)sq, (const float*)part, M, N, \
+            ks); break
+    switch (std::min(ks, 8)) {
+        FOLD(1); FOLD(2); FOLD(3); FOLD(4); FOLD(5); FOLD(6); FOLD(7); FOLD(8);
+    }
+    #undef FOLD
     return (int)hipGetLastError();
 }
 
