@@ -818,6 +818,107 @@ __global__ __launch_bounds__(BS) void k_tile_fold(
     }
 }
 
+// The same for a rotated product: x W^T of normed rows with its bias, queries
+// rotated to y, keys and values to their pages.  A wave takes strips of 32
+// columns, two at a time: a head's 16 pairs of dimensions, or its values.  What
+// the 16 rows need is asked for ahead of the parts, every lane for its own row.
+// Waits bound it; with the product in parts, 128 rows, us, and k_wstream_gemm,
+// which rotates by itself: 6144 x 4096 22.9 and 25.0, 4608 x 3584 18.3 and 23.9.
+template <int BS, int KS>
+__global__ __launch_bounds__(BS) void k_tile_fold_rope(const TileArgs a)
+{
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int r16 = lane & 15, g4 = lane >> 4;
+    const bool upper = g4 >> 1;
+    const int c = upper * 8 + (g4 & 1) * 4;        // after the swap
+    const Append& ap = a.ap;
+    const int hi = blockIdx.x, mh = gridDim.x, nh = a.N >> 4, ns = a.N >> 5;
+    const int row = (hi >> 1) * 32 + in_strip(hi & 1, r16);
+    const int at = min(row, a.M - 1);
+    const int from = ns * blockIdx.y / gridDim.y;
+    const int to = ns * (blockIdx.y + 1) / gridDim.y;
+    const int64_t step = (int64_t)mh * nh * 256;
+    const int pos = ap.pos[at], slot = ap.slot[at];
+    float s2 = 0.f;
+    #pragma unroll 4
+    for (int e = g4; e < a.rstd_nt; e += 4)
+        s2 += a.rstd[(int64_t)at * a.rstd_nt + e];
+    int64_t kv = 0;
+    float rs = 0.f;
+    const int qt = ap.nl * 4, kt = ap.nkl * 4;
+    constexpr int J = 2, W = BS / 64;
+    for (int j0 = from + wid; j0 < to; j0 += J * W) {
+        f32x4 v[KS][J][2], turn[J][2];
+        bf16x4 bias[J][2];
+        const float* p[J];
+        #pragma unroll
+        for (int i = 0; i < J; i++) {
+            const int t = j0 + i * W < to ? j0 + i * W : j0;
+            p[i] = a.part + ((int64_t)hi * nh + 2 * t) * 256 + lane * 4;
+            #pragma unroll
+            for (int k = 0; k < KS; k++)
+                #pragma unroll
+                for (int h = 0; h < 2; h++)
+                    v[k][i][h] = *reinterpret_cast<const f32x4*>(
+                        p[i] + k * step + h * 256);
+            if (a.bias)
+                #pragma unroll
+                for (int h = 0; h < 2; h++)
+                    bias[i][h] = *reinterpret_cast<const bf16x4*>(
+                        a.bias + t * 32 + c + h * 16);
+            const int o = pos * 64 + (t & 3) * 16 + c;
+            turn[i][0] = *reinterpret_cast<const f32x4*>(ap.cos_t + o);
+            turn[i][1] = *reinterpret_cast<const f32x4*>(ap.sin_t + o);
+        }
+        if (j0 == from + wid) {            // the first time
+            const int page = ap.ptab[slot * ap.maxp + pos / ap.psz];
+            kv = ((int64_t)page * ap.nkl * ap.psz + pos % ap.psz) * 128 + c;
+            s2 += __shfl_xor(s2, 16, 64);
+            s2 += __shfl_xor(s2, 32, 64);
+            rs = rsqrtf(s2 * a.inv_h + a.eps);
+        }
+        #pragma unroll
+        for (int i = 0; i < J; i++) {
+            const int t = j0 + i * W;
+            f32x4 lo = v[0][i][0], hi2 = v[0][i][1];
+            #pragma unroll
+            for (int k = 1; k < KS; k++) {
+                lo += v[k][i][0];
+                hi2 += v[k][i][1];
+            }
+            for (int k = KS; k < a.ks; k++) {
+                lo += *reinterpret_cast<const f32x4*>(p[i] + k * step);
+                hi2 += *reinterpret_cast<const f32x4*>(p[i] + k * step + 256);
+            }
+            lo *= rs;
+            hi2 *= rs;
+            swap32(lo, hi2);
+            if (a.bias)
+                #pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    lo[e] += (float)bias[i][0][e];
+                    hi2[e] += (float)bias[i][1][e];
+                }
+            if (t >= to || row >= a.M) continue;
+            if (t >= qt + kt) {
+                const int s = t - qt - kt;
+                bf16* d = ap.vp + (s >> 2) * ap.psz * 128 + (s & 3) * 32 + kv;
+                put4(d, lo);
+                put4(d + 16, hi2);
+                continue;
+            }
+            const f32x4 u = lo * turn[i][0] - hi2 * turn[i][1];
+            const f32x4 w = hi2 * turn[i][0] + lo * turn[i][1];
+            const int s = t < qt ? t : t - qt, d = (s & 3) * 16;
+            bf16* q = t < qt
+                ? a.y + (int64_t)row * a.N + (s >> 2) * 128 + d + c
+                : ap.kp + (s >> 2) * ap.psz * 128 + d + kv;
+            put4(q, u);
+            put4(q + 64, w);
+        }
+    }
+}
+
 // parts of sums of squares of a row, added up: eight lanes a row
 __global__ __launch_bounds__(256) void k_row_sums(
     float* __restrict__ out, const float* __restrict__ in, int M, int nt)
@@ -1021,4 +1122,39 @@ extern "C" int tile_rows_bf16(
     if (epi == GATED) return launch<GATED>(a, hm, hn, cus, stream);
     if (epi == ROWS) return launch<ROWS>(a, hm, hn, cus, stream);
     return launch<ROW_PARTS>(a, hm, hn, cus, stream);
+}
+
+// As tile_gemm_bf16's ROPE, the product in ks parts of K.  part: ks times the
+// rows, in 32s, times N.
+extern "C" int tile_rope_parts_bf16(
+    void* y, void* part, const void* x, const void* w, const void* bias,
+    const void* rstd, int rstd_nt, float inv_h, float eps, int M, int N, int K,
+    int hm, int hn, int ks, int gm, int cus, const void* rcos,
+    const void* rsin, const void* pos, const void* slot, const void* ptab,
+    void* kp, void* vp, int nl, int nkl, int psz, int maxp,
+    hipStream_t stream)
+{
+    const int unit = 32 * tile_stages(hm, hn);     // of K
+    if (M < 1 || N != (nl + 2 * nkl) * 128 || N < 32 || K < unit || K % unit
+        || ks < 1 || ks > K / unit || (int64_t)(M + 31) * N >= (int64_t)1 << 31
+        || gm < 1 || cus < 8 || !part || !rstd || rstd_nt < 1)
+        return -111;
+    TileArgs a{};
+    a.y = (bf16*)y, a.part = (float*)part, a.x = (const bf16*)x;
+    a.w = (const bf16*)w, a.bias = (const bf16*)bias;
+    a.rstd = (const float*)rstd, a.rstd_nt = rstd_nt;
+    a.inv_h = inv_h, a.eps = eps, a.M = M, a.N = N, a.K = K;
+    a.mt = div_up(M, hm * 32), a.nt = div_up(N, hn * 32), a.ks = ks;
+    a.gm = gm;
+    a.ap = {(const float*)rcos, (const float*)rsin, (const int*)pos,
+            (const int*)slot, (const int*)ptab, (bf16*)kp, (bf16*)vp,
+            nl, nkl, psz, maxp};
+    if (const int e = launch<PARTS>(a, hm, hn, cus, stream)) return e;
+    // a wave's two strips at a time, once
+    const dim3 grid(div_up(M, 32) * 2, std::max(1, N / 256));
+    #define FOLD(KS) \
+        case KS: k_tile_fold_rope<256, KS><<<grid, 256, 0, stream>>>(a); break
+    switch (std::min(ks, 4)) { FOLD(1); FOLD(2); FOLD(3); FOLD(4); }
+    #undef FOLD
+    return (int)hipGetLastError();
 }

@@ -508,6 +508,9 @@ class LlamaModel:
         tiles = B > 48 and self._tiles_take(B)
         qkv_tiles = tiles and not ops.streams_at_once(
             self.layers[0].wqkv.shape[0], dev)
+        # of one round some take less time in parts
+        qkv_parts = ops.rope_parts(B, self.layers[0].wqkv.shape[0], H, dev) \
+            if tiles and not qkv_tiles else None
         # a switch that asks for parts means the streams'
         o_tiles = tiles and ops.asked_parts(nl * d) is None
         down_tiles = tiles and ops.asked_parts(
@@ -521,6 +524,12 @@ class LlamaModel:
                     layer.bqkv_rp, kv_cache, li, positions, slot_ids,
                     self.rope_cos, self.rope_sin, nl, nkl, sq_a, nt, inv_h,
                     eps)
+            elif qkv_parts is not None:
+                qkv = ops.tile_qkv_parts(
+                    res, layer.wqkv_pk, B, layer.wqkv.shape[0], H,
+                    layer.bqkv_rp, kv_cache, li, positions, slot_ids,
+                    self.rope_cos, self.rope_sin, nl, nkl, sq_a, nt, inv_h,
+                    eps, qkv_parts)
             else:
                 qkv = ops.qkv_rope_fused(
                     res, layer.wqkv_pk, layer.wqkv.shape[0], layer.bqkv_rp,

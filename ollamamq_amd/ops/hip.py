@@ -68,6 +68,8 @@ def _try_load():
     lib.tile_gemm_bf16.argtypes = [*[vp] * 8, i, f, f, *[i] * 11, *[vp] * 7,
                                    i, i, i, i, vp]
     lib.tile_gemm_plan.argtypes = [i, i, i, i, i]
+    lib.tile_rope_parts_bf16.argtypes = [
+        *[vp] * 6, i, f, f, *[i] * 8, *[vp] * 7, i, i, i, i, vp]
     lib.tile_rows_bf16.argtypes = [*[vp] * 4, *[i] * 10, vp]
     lib.row_sumsq_bf16.argtypes = [vp, vp, i, i, vp]
     lib.frag_rows_bf16.argtypes = [vp, vp, vp, vp, i, i, i, vp]
@@ -753,6 +755,48 @@ def tile_qkv_rope(x, packed, M, N, K, bias_rp, cache, layer, positions,
                rope=(_p(cos), _p(sin), _p(pos32), _p(slot32),
                      _p(cache.page_table), kp, vp, nl, nkl, cache.page_size,
                      cache.page_table.shape[1]))
+    return y
+
+
+@functools.lru_cache(maxsize=4096)
+def rope_parts(M, N, K, cus=256):
+    """(rows, columns, parts of K) of the tiles of a rotated product of 49 to
+    128 rows, or None where the stream of its weights is faster or its blocks
+    would not run at once.  A streaming block loads all rows for 32 columns,
+    for 65 rows and 97 a third and a fourth strip of 32, and has all of K to go
+    through; in parts all CUs load, a fold of 3 us follows.  us of a stream and
+    of parts, the fold included:
+                    64 rows       65           96          97..112      128
+      6144 x 4096  17.8 18.4   19.9 21.3   21.5 21.3   24.2 22.9   25.0 22.9
+      4608 x 3584  16.8 14.8   18.7 17.1   20.4 17.1   23.2 18.2   23.9 18.3
+      8192 x 4096  19.1 19.5   20.9 22.5   22.6 22.5   25.5 24.3   26.4 24.4
+      5120 x 4096  17.3 16.9   19.2 19.4   20.8 19.3   23.6 21.2   24.3 21.2
+      3072 x 2048  10.7 10.2   12.0 11.8   12.9 11.8   15.0 12.4   15.6 12.4
+    so parts from 97 rows on, and from 49 where there are three."""
+    parts = min(cus // -(-N // 64), K // 1024, 8)
+    if parts < 2 or K % 256 or not 48 < M <= 128 or (M <= 96 and parts < 3):
+        return None
+    return 2 if M <= 64 else 4, 2, parts
+
+
+def tile_qkv_parts(x, packed, M, N, K, bias_rp, cache, layer, positions,
+                   slots, cos, sin, nl, nkl, rstd, rstd_nt, inv_h, eps, plan):
+    """tile_qkv_rope in parts of K, which a second kernel adds up, rotates and
+    appends."""
+    dev = x.device
+    hm, hn, ks = plan
+    rows = -(-M // 32) * 32
+    assert x.numel() >= rows * K and packed.numel() == N * K
+    y = torch.empty((M, N), dtype=x.dtype, device=dev)
+    part = torch.empty(ks * rows * N, dtype=torch.float32, device=dev)
+    kp, vp = _layer_ptrs(cache, layer)
+    pos32, slot32 = _i32(positions), _i32(slots)
+    _check(_lib.tile_rope_parts_bf16(
+        _p(y), _p(part), _p(x), _p(packed), _p(bias_rp), _p(rstd), rstd_nt,
+        float(inv_h), float(eps), M, N, K, hm, hn, ks, 8, _cus(dev.index),
+        _p(cos), _p(sin), _p(pos32), _p(slot32), _p(cache.page_table), kp, vp,
+        nl, nkl, cache.page_size, cache.page_table.shape[1], _stream()),
+        "tile_rope_parts")
     return y
 
 

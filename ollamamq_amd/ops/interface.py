@@ -864,6 +864,19 @@ def tile_qkv_rope(x, packed, M, N, K, bias_rp, cache, layer, positions, slots,
                              rstd_nt, inv_h, eps)
 
 
+def rope_parts(M, N, K, device):
+    """The tiles of a qkv product in parts, or None where it is streamed."""
+    return hip.rope_parts(M, N, K, hip._cus(device.index))
+
+
+def tile_qkv_parts(x, packed, M, N, K, bias_rp, cache, layer, positions,
+                   slots, cos, sin, nl, nkl, rstd, rstd_nt, inv_h, eps, plan):
+    """tile_qkv_rope in parts of K and their sum, two kernels."""
+    return hip.tile_qkv_parts(x, packed, M, N, K, bias_rp, cache, layer,
+                              positions, slots, cos, sin, nl, nkl, rstd,
+                              rstd_nt, inv_h, eps, plan)
+
+
 def tile_residual(x, packed, M, N, K, res):
     """res += x W^T; partial sums of squares of the new rows and how many a
     row has."""
