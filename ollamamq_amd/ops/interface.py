@@ -17,6 +17,19 @@ import torch
 from . import reference as ref
 
 
+class _Deferred:
+    """ops.hip until it is first needed: it takes its types from here, and its
+    switches from the environment of that moment."""
+
+    def __getattr__(self, name):
+        global hip
+        from . import hip
+        return getattr(hip, name)
+
+
+hip = _Deferred()
+
+
 def force_ref() -> bool:
     return os.environ.get("OLLAMAMQ_FORCE_REF") == "1"
 
@@ -932,6 +945,3 @@ def plan_latent(cache, run, meta, w: LatentWeights):
         pool = cache.latent_pool[run]
         hip._latent_plan(meta, w, pool.shape[2], hip._is_f32(pool),
                          pool.device)
-
-
-from . import hip  # noqa: E402  (it takes its types from here)
