@@ -29,6 +29,15 @@ from ..ops import interface as ops
 from .kvcache import PagedKVCache
 
 
+def _ints(tokens):
+    """As int32; what is not whole or too large as a tensor takes it, which
+    costs ten times as much."""
+    try:
+        return array("i", tokens)
+    except (TypeError, OverflowError):
+        return torch.tensor(tokens, dtype=torch.int32).numpy()
+
+
 @dataclass
 class GenParams:
     max_tokens: int = 128
@@ -405,7 +414,7 @@ class LlamaEngine:
             stage=stage)
         first = np.array(starts) - np.array(cu[:-1])
         for part in (np.array(want, dtype=np.int64).view(np.int32),
-                     array("i", token_list),
+                     _ints(token_list),
                      np.arange(cu[-1]) + np.repeat(first, q_lens),
                      np.repeat(slots, q_lens), slots, kv_lens, cu, places,
                      values):

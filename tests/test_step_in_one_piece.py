@@ -2,6 +2,7 @@
 same tensors as one by one, also when something fails on the way."""
 from array import array
 
+import numpy as np
 import pytest
 import torch
 
@@ -103,3 +104,28 @@ def test_pages_are_in_the_table_after_an_error(fails, monkeypatch):
         pages = kv._slot_pages[s.slot]
         assert len(pages) == (2 if s is a else 0 if fails == "pages" else 3)
         assert kv.page_table[s.slot, :len(pages)].tolist() == pages
+
+
+@pytest.mark.parametrize("dev", WHERE)
+def test_tokens_are_what_a_tensor_takes(dev):
+    """Numbers of any type, of which the whole part counts; RuntimeError where
+    they are too large."""
+    cfg = PRESETS["tiny"]
+    dtype = torch.float32 if dev == "cpu" else torch.bfloat16
+    model = build_model(cfg, device=dev, dtype=dtype, seed=1)
+    kv = cache_for_model(cfg, n_pages=9, max_slots=4, max_ctx=64, device=dev,
+                         dtype=dtype)
+    eng = LlamaEngine(model, kv, max_batch=4)
+    want = None
+    for text in ([3, 1, 4], [3.0, 1.5, 4.0], list(np.array([3., 1., 4.])),
+                 [3, torch.tensor(1), True + 3]):
+        s = eng.open_stream()
+        got = eng.feed([(s, text, [0, 2])])
+        eng.close_stream(s)
+        want = got if want is None else want
+        assert torch.equal(got, want)
+    for bad in ([2 ** 31], [1.0, 2.0 ** 40]):
+        s = eng.open_stream()
+        with pytest.raises(RuntimeError):
+            eng._forward([s], bad, [0], [len(bad)], "prefill")
+        eng.close_stream(s)
