@@ -93,9 +93,13 @@ class SequenceCache:
              values: List[int]) -> None:
         """ensure_all without the device: adds the page table's new entries
         and where they go in the flat table.  What was grown before an error
-        stays, and its entries are there."""
+        stays, and its entries are there.  Whether a slot is one of the
+        cache's is asked here: on the device an entry outside the table is
+        left out without a word."""
         width, size = self.page_table.shape[1], self.page_size
         for slot, new_len in wanted:
+            if not 0 <= slot < self.max_slots:
+                raise IndexError(f"KV cache: no sequence slot {slot}")
             if new_len > self.max_ctx:
                 raise RuntimeError(
                     f"sequence exceeds max_ctx {self.max_ctx}")

@@ -911,7 +911,8 @@ def sample(logits, temperature, top_k, top_p, generator=None):
 
 
 def set_entries(table, places, values):
-    """table.view(-1)[places] = values, all int32."""
+    """table.view(-1)[places] = values, all int32.  Places are the caller's to
+    check: the kernel leaves out those outside the table."""
     if _use_hip(table):
         hip.set_entries(table, places, values)
     else:

@@ -37,3 +37,18 @@ def test_the_first_are_kept(last, message):
     assert c.free_page_count() == 7
     c.ensure(d, 28)
     assert c.page_table[d, :7].tolist() == c._slot_pages[d]
+
+
+@pytest.mark.parametrize("slot", [-1, 3, 4])
+def test_slots_that_there_are_none_of(slot):
+    """Refused before anything is taken: a closed stream has the slot -1, and
+    the last slot's pages are not its own."""
+    c, (a, b, d) = _cache()
+    c.ensure_all([(a, 6), (d, 4)])
+    table, lens, free = c.page_table.clone(), list(c.seq_lens), \
+        list(c._free_pages)
+    for grow in (c.ensure_all, lambda w: c.grow(w, [], [])):
+        with pytest.raises(IndexError):
+            grow([(slot, 20)])
+        assert torch.equal(c.page_table, table)
+        assert c.seq_lens == lens and c._free_pages == free
