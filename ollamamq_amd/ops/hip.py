@@ -910,9 +910,10 @@ def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
     apply rmsnorm scaling of the raw-residual input x (norm weight must
     be folded into the pack); `res` adds the residual stream into the
     output (pass y=res for the in-place residual update) and `sq_out`
-    emits per-tile sum-of-squares partials for the next GEMM.  `sem`: int32
-    zeros, one per 32 columns, for a split product that adds up its own parts;
-    they are zero again when it ends, so a stream's products can share them."""
+    emits per-tile sum-of-squares partials for the next GEMM, for whole tiles
+    of 32 rows.  `sem`: int32 zeros, one per 32 columns, for a split product
+    that adds up its own parts; they are zero again when it ends, so a stream's
+    products can share them."""
     if K is None:
         M, K = x.shape
         xs = x.stride(0)
@@ -934,6 +935,7 @@ def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
         # wins on the short ramp-bound ones (qkv/o)
         xlds = (_WS_XLDS if M <= 32 and N * K * 2 > (64 << 20) else 0)
     part = None
+    assert sq_out is None or sq_out.numel() >= -(-M // 32) * N
     # what is fused needs the finished sums: the product adds up its own parts
     if ks > 1 and (xlds == 2 or res is not None or sq_out is not None
                    or yfrag):
