@@ -816,7 +816,7 @@ def tile_linear(x, packed, N, most=1, f32=False, plan=None):
     if plan is None:
         # parts cost their consumer what adding them up costs a residual's
         plan = tile_plan(M, N, K, TILE_RESIDUAL, _cus(dev.index))
-        if plan[2] > most:
+        if plan[2] > most or plan[:2] == TILE_LEAST:     # none for rows
             plan = tile_plan(M, N, K, TILE_GATED, _cus(dev.index))
     if plan[2] > 1 or f32:
         part = torch.empty((plan[2], M, N), dtype=torch.float32, device=dev)

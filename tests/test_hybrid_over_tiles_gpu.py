@@ -48,6 +48,39 @@ def test_product(tile, M, N, K):
         near(unfrag(act.buf, M, N // 2), g * u)
 
 
+@pytest.mark.parametrize("dev", [
+    "cpu", pytest.param("cuda:0", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("M", [1, 64, 65, 128, 129])
+def test_own_plan(M, dev, monkeypatch):
+    """Without a plan a product takes tiles that there are for its results,
+    also of as few rows as others have smaller ones for."""
+    hip.require()
+    torch.manual_seed(M)
+    N, K = 576, 8192
+    x = torch.randn(M, K).bfloat16()
+    w = torch.randn(N, K).mul_(K ** -0.5).bfloat16()
+    plans, product = [], hip._tile_rows
+    if dev == "cpu":
+        monkeypatch.setattr(hip, "_cus", lambda index: 256)
+
+    def spy(epi, y, x, packed, N, plan, *a, **k):
+        plans.append(plan)
+        if dev != "cpu":
+            product(epi, y, x, packed, N, plan, *a, **k)
+    monkeypatch.setattr(hip, "_tile_rows", spy)
+    xf = FragRows(frag(x.to(dev)), M, K)
+    pk = hip.pack_weight(w.to(dev)) if dev != "cpu" else w.flatten()
+    got = [hip.tile_linear(xf, pk, N, most=8), hip.tile_linear(xf, pk, N),
+           hip.tile_linear(xf, pk, N, 8, True)]
+    assert len(plans) == 3 and all(p[:2] in hip.TILES for p in plans)
+    if dev != "cpu":
+        y = x.double() @ w.double().T
+        for out in got:
+            if not isinstance(out, torch.Tensor):
+                out = out.parts.sum(0)
+            near(out.cpu(), y)
+
+
 def test_refused():
     lib = hip._lib if hip.available() else None
     if lib is None:
