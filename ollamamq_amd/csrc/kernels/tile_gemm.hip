@@ -953,8 +953,11 @@ int launch(TileArgs a, int hm, int hn, int cus, hipStream_t stream)
     a.rows_at = tile_rows_at(hm, hn, NORMED && !add_up ? a.rstd_nt : 1);
     const int lds = a.rows_at + hm * 32 * 12;
     auto go = [&](auto k) {
+        // the same for every call: another thread may be between this and the
+        // launch
         const hipError_t e = hipFuncSetAttribute(
-            (const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+            (const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+            ALL / each);
         if (e != hipSuccess) return (int)e;
         if (add_up) {
             k_row_sums<<<(a.M + 31) / 32, 256, 0, stream>>>(a.part, a.rstd,
