@@ -64,3 +64,39 @@ def test_parts_of_rows(M, nt, shift):
         want = outputs(plan, sq, 1)
         for got, one in zip(outputs(plan, parts, nt), want):
             assert one.any() and torch.equal(got, one), plan
+
+
+def eight_side_by_side(parts):
+    """fp32 sums of rows as eight lanes add them up, and then the lanes."""
+    parts = parts.cpu()
+    lanes = torch.zeros(parts.shape[0], 8)
+    for e in range(parts.shape[1]):
+        lanes[:, e % 8] += parts[:, e]
+    while lanes.shape[1] > 1:
+        lanes = lanes[:, ::2] + lanes[:, 1::2]
+    return lanes[:, 0].contiguous().cuda()
+
+
+# 2^25 has no room for what is added to it before it is taken away again, so a
+# sum in another order is another sum: only every eighth part may be together.
+# Sums of 33 rows are added up by the product itself, of 20000, more than one
+# round of blocks of every tile, by a kernel of their own.
+@pytest.mark.gpu
+@pytest.mark.parametrize("nt", [2, 9, 12, 16, 19, 22, 32, 53])
+@pytest.mark.parametrize("M", [33, 20000])
+def test_order_of_sums(M, nt):
+    hip.require()
+    torch.manual_seed(nt)
+    N, K = 1024, 256
+    x = torch.randn((M + 31) // 32 * 32 * K, device="cuda").bfloat16()
+    w = torch.randn(N * K, device="cuda").mul_(K ** -0.5).bfloat16()
+    parts = torch.rand(M, nt, device="cuda") * 100
+    if nt > 8:
+        parts[:, 0], parts[:, 8] = 2 ** 25, -2 ** 25
+    for tile in hip.TILES:
+        one, got = (hip.tile_gu(x, w, M, N, K, rstd, n, 1.0 / K, 1e-5,
+                                plan=(*tile, 1)).view(-1, N // 16, 32, 8)
+                    .transpose(1, 2).reshape(-1, N // 2)[:M]
+                    for rstd, n in ((eight_side_by_side(parts), 1),
+                                    (parts, nt)))
+        assert one.any() and torch.equal(got, one), tile
