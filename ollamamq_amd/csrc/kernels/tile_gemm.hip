@@ -849,10 +849,15 @@ __global__ __launch_bounds__(BS) void k_tile_fold_rope(const TileArgs a)
     const int to = ns * (blockIdx.y + 1) / gridDim.y;
     const int64_t step = (int64_t)mh * nh * 256;
     const int pos = ap.pos[at], slot = ap.slot[at];
-    float s2 = 0.f;
-    #pragma unroll 4
-    for (int e = g4; e < a.rstd_nt; e += 4)
-        s2 += a.rstd[(int64_t)at * a.rstd_nt + e];
+    // sums of a row: eight side by side, as k_row_sums adds them up
+    const float* sums = a.rstd + (int64_t)at * a.rstd_nt;
+    float s2[2] = {};
+    #pragma unroll 2
+    for (int e = g4; e < a.rstd_nt; e += 8) {
+        const float v = sums[min(e + 4, a.rstd_nt - 1)];
+        s2[0] += sums[e];
+        s2[1] += e + 4 < a.rstd_nt ? v : 0.f;
+    }
     int64_t kv = 0;
     float rs = 0.f;
     const int qt = ap.nl * 4, kt = ap.nkl * 4;
@@ -883,9 +888,12 @@ __global__ __launch_bounds__(BS) void k_tile_fold_rope(const TileArgs a)
         if (j0 == from + wid) {            // the first time
             const int page = ap.ptab[slot * ap.maxp + pos / ap.psz];
             kv = ((int64_t)page * ap.nkl * ap.psz + pos % ap.psz) * 128 + c;
-            s2 += __shfl_xor(s2, 16, 64);
-            s2 += __shfl_xor(s2, 32, 64);
-            rs = rsqrtf(s2 * a.inv_h + a.eps);
+            #pragma unroll
+            for (int h = 0; h < 2; h++) {
+                s2[h] += __shfl_xor(s2[h], 16, 64);
+                s2[h] += __shfl_xor(s2[h], 32, 64);
+            }
+            rs = rsqrtf((s2[0] + s2[1]) * a.inv_h + a.eps);
         }
         #pragma unroll
         for (int i = 0; i < J; i++) {

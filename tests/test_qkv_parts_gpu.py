@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from ollamamq_amd.ops import hip
+from test_tile_row_sums_gpu import eight_side_by_side
 
 
 def test_rule():
@@ -69,6 +70,40 @@ def test_bits(M, nl, nkl, page, nt, bias, ks):
     for tile in ((4, 2), *([(2, 2)] if M <= 64 else [])):
         for got, one in zip(outputs(hip.tile_qkv_parts, (*tile, ks)), want):
             assert torch.equal(got, one)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nt", [2, 4, 7, 9, 16, 19, 32])
+def test_order_of_row_sums(nt):
+    """Eight sums side by side, however many a row comes in: 2^25 has no room
+    for what is added to it before it is taken away again."""
+    hip.require()
+    torch.manual_seed(nt)
+    M, K, nl, nkl, page = 65, 512, 4, 1, 16
+    N = (nl + 2 * nkl) * 128
+    x = torch.randn(96 * K, device="cuda").bfloat16()
+    w = torch.randn(N * K, device="cuda").mul_(K ** -0.5).bfloat16()
+    parts = torch.rand(M, nt, device="cuda") * 100
+    if nt > 8:
+        parts[:, 0], parts[:, 8] = 2 ** 25, -2 ** 25
+    pos = torch.arange(M, device="cuda").int()
+    slot = torch.zeros_like(pos)
+    table = torch.arange(5, device="cuda").int().view(1, 5)
+    cos, sin = torch.rand(2, 80, 64, device="cuda")
+
+    def outputs(sq, n):
+        cache = SimpleNamespace(
+            n_kv_heads=nkl, page_size=page, page_table=table,
+            k_pool=torch.zeros(1, 5, nkl, page, 128, device="cuda",
+                               dtype=torch.bfloat16))
+        cache.v_pool = torch.zeros_like(cache.k_pool)
+        q = hip.tile_qkv_parts(x, w, M, N, K, None, cache, 0, pos, slot, cos,
+                               sin, nl, nkl, sq, n, 1.0 / K, 1e-5, (4, 2, 2))
+        return q[:, :nl * 128], cache.k_pool, cache.v_pool
+
+    for got, one in zip(outputs(parts, nt),
+                        outputs(eight_side_by_side(parts), 1)):
+        assert one.any() and torch.equal(got, one)
 
 
 def test_refused():
