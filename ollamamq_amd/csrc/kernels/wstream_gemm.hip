@@ -806,16 +806,29 @@ __global__ __launch_bounds__(CW * wide_parts(CW) * 64, 1) void k_wide(
 // one, with 2, 4 and 8 alone 2.8 %.
 // Up to 32 rows the stream's own blocks, two a CU, read at the memory's rate; 25
 // rows and more are all the cache lines that 32 are, and blocks that fill half
-// of a last round wait for them (32 rows, stream and k_wide: 22016 x 4096 37.0
-// and 35.1, 37888 x 3584 53.2 and 50.4, 128256 x 4096 191 and 177; 28672 x 4096
-// 46.5 and 47.0, 32000 x 2048 27.7 and 28.0).
-static int wide_tiles(int M, int N, int K)
+// of a last round wait for them (32 rows, stream and k_wide: 22016 x 4096 34.6
+// and 31.7, 37888 x 3584 49.5 and 46.0; 28672 x 4096 43.3 and 43.8, 24576 x 3072
+// 27.6 and 28.2).  Eight tiles a block take rounds of a block a CU, and a last
+// round takes as long whatever it has, so it has to be nearly full: the more
+// so where the stream's waves have whole rounds of four (frag_depth).  Stream
+// and eight tiles, 32 rows:
+//   blocks            257      352      400      512      544      594
+//   x 4096         96  111  129  136  146  148  190  177  200  216  218  223
+//   x 3584         88   99  115  116  132  122  172  150  184  187  201  193
+// With norm and activation the stream writes less: 352 blocks x 4096 117 and 135,
+// 512 170 and 171, 594 x 3584 177 and 188.
+static int wide_tiles(int M, int N, int K, bool gated)
 {
     const int tiles = N / 32, mt = (M + 31) / 32;
     const int whole = (tiles + 255) / 256;     // of one round of blocks
     if (M <= 32) {
         if (M <= 24 || K < 3072) return 1;
-        if (tiles >= 2048) return 8;
+        if (tiles >= 2048) {
+            const int blocks = (tiles + 7) / 8, rounds = (blocks + 255) / 256;
+            const double full = blocks / (256. * rounds);
+            return (gated ? rounds == 1 : full >= (K % 2048 ? 0.77 : 0.85))
+                       ? 8 : 1;
+        }
         return tiles > 512 && (-tiles & 511) > 256 ? whole : 1;
     }
     int best = 1;
@@ -833,6 +846,13 @@ static int wide_tiles(int M, int N, int K)
         }
     }
     return best;
+}
+
+// tiles a block that a product takes, 1: k_wstream_gemm
+extern "C" int wstream_wide_tiles(int M, int N, int K, int gated)
+{
+    return M < 1 || M > 128 || N < 32 || K < 64 ? -104
+                                                : wide_tiles(M, N, K, gated);
 }
 
 template <int GU>
@@ -898,7 +918,7 @@ static int wstream_gu(
     const int lds = (xlds == 1 ? 16 * 4096 : 8 * 32 * 32 * 4) + 512;
     if (M > (xlds == 2 ? 128 : 64)) return -104;   // rows of a block
     if (xlds == 2) {           // frag chain
-        const int cw = wide_tiles(M, N, K);
+        const int cw = wide_tiles(M, N, K, true);
         if (cw > 1)
             return wide<GU>(cw, act, x, wp, M, N, K, rstd_parts, rstd_nt,
                             inv_h, eps, yfrag, stream);
@@ -984,7 +1004,7 @@ extern "C" int wstream_gemm_bf16(
         return -100;
     const int d = frag_depth(K, ksplit);
     if (xlds == 2 && ksplit == 1 && y && !bias && !ri && !sq) {
-        const int cw = wide_tiles(M, N, K);
+        const int cw = wide_tiles(M, N, K, false);
         if (cw > 1)
             return wide<0>(cw, y, x, wp, M, N, K, rp, rstd_nt, inv_h, eps,
                            yfrag, stream);

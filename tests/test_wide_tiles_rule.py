@@ -1,0 +1,31 @@
+"""Which streamed products share their rows between several tiles of columns:
+none that is slower for it than it was with the stream or with a power of two of
+tiles.  Each line was measured on both sides, us."""
+import pytest
+
+from ollamamq_amd.ops import hip
+
+
+@pytest.mark.parametrize("M, N, K, gated, tiles", [
+    # up to 32 rows: a last round of eight tiles a block that is nearly full
+    (32, 73728, 4096, True, 1),         # 97, with eight 126
+    (25, 65600, 4096, False, 1),        # 96, with eight 111
+    (32, 102400, 4096, True, 1),        # 135, with eight 144
+    (32, 81920, 3584, False, 1),        # 103, with eight 111
+    (32, 139264, 4096, False, 1),       # 200, with eight 216
+    (32, 128256, 4096, False, 8),       # 183, with eight 172
+    (32, 152064, 3584, False, 8),       # 201, with eight 193
+    (32, 102400, 3584, False, 8),       # 132, with eight 122
+    (32, 65536, 3584, True, 8),         # 77, with eight 75
+    (32, 22016, 4096, True, 3),         # 34, with three 32
+    (24, 22016, 4096, True, 1), (32, 28672, 4096, True, 1),
+])
+def test_choice(M, N, K, gated, tiles):
+    hip.require()
+    assert hip._lib.wstream_wide_tiles(M, N, K, gated) == tiles
+
+
+def test_none():
+    hip.require()
+    for bad in ((0, 64, 64), (129, 64, 64), (1, 16, 64), (1, 64, 32)):
+        assert hip._lib.wstream_wide_tiles(*bad, False) < 0
