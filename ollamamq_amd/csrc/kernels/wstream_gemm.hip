@@ -791,19 +791,27 @@ __global__ __launch_bounds__(CW * wide_parts(CW) * 64, 1) void k_wide(
 // KB a step of K.  A block of k_wide loads its tiles and all rows, or waits: two
 // tiles take what 4.8 + mt / 2 units take.  A tile of k_wstream_gemm (1), of
 // which a CU has several at a time, takes 0.8 (1 + mt), its rows coming from
-// L1 at times.  Numbers other than 2, 4 and 8 are for one round of blocks: of
-// several rounds the weights' reads are what is left.  us, K 4096 but for
-// 37888 x 3584 and 32000 x 2048 (the last two):
-//                 rows    1    2    3    4    5    6    8
-//   16384           40   30   36   34   35   43   46   56
-//   22016           48   46   58   38   40   44   49   58
-//                  128   68   70   45   49   54   57   72
-//   28672           64   63   65   66   46   48   52   61
-//   37888           48   71   74   64   67   51   53   60
-//                  128  109   95   78   86   58   60   70
-//   32000           48   39   39   40   34   30   31   36
-// Over 23 matrices and 33 to 128 rows the choice takes 1 % more than the best
-// one, with 2, 4 and 8 alone 2.8 %.
+// L1 at times.  All weights take 0.0068 units a tile at the memory's rate, so
+// where that is more, eight tiles load fewer rows for them; not for K of 1024,
+// which ends sooner in two parts side by side.  Numbers other than 2, 4 and 8 are
+// for one round of blocks: of several rounds the weights' reads are what is left;
+// three, whose parts of K do not divide it, from K of 2048 on.  us:
+//                     rows    1    2    3    4    5    6    7    8
+//   16384 x 4096        64   34        34   36   42   45   50   55
+//                      128   46   41   41   45   51   53   60   68
+//   22016 x 4096        64   47        37   38   44   47   52   57
+//                      128   64   68   44   47   53   55   62   69
+//   28672 x 4096        64   60        64   44   47   50   55   59
+//   37888 x 3584        64   75        61   66   49   50   54   56
+//                      128  105   92   75   82   55   57   62   68
+//   49152 x 4096        64   95        76   83   94   72   69   69
+//   57344 x 3584        64  107        90   72   86   96   72   69
+//                      128  151  127  113   94  102  109   77   78
+//   24576 x 1536        64   26        19   19   22   23   25   26
+//   32000 x 2048        64   37        39   32   28   30   32   34
+// Over 21 numbers of columns, 9 of K from 512 to 4096 and 33 to 128 rows the
+// choice takes 0.6 % more than the best one, with 2, 4 and 8 alone 4.8 %; 14 % for
+// the last line, where one round of five would do.
 // Up to 32 rows the stream's own blocks, two a CU, read at the memory's rate; 25
 // rows and more are all the cache lines that 32 are, and blocks that fill half
 // of a last round wait for them (32 rows, stream and k_wide: 22016 x 4096 34.6
@@ -835,12 +843,14 @@ static int wide_tiles(int M, int N, int K, bool gated)
     double least = whole * 0.8 * (1 + mt);
     // two tiles of 64 rows are 5.8 units, one after the other 4.8 at most
     for (int cw = mt == 2 ? 3 : 2; cw <= 8; cw++) {
-        if (cw < whole && (cw & (cw - 1))) continue;
+        const bool odd = cw & (cw - 1);
+        if (odd && (cw < whole || (cw == 3 && K < 2048))) continue;
         const int blocks = (tiles + cw - 1) / cw;
-        const double units = (blocks + 255) / 256
-                             * std::max<double>(cw + mt,
-                                                cw < 4 ? 4.8 + 0.5 * mt : 0);
-        if (units < least) {
+        const double units = std::max(
+            (blocks + 255) / 256
+                * std::max<double>(cw + mt, cw < 4 ? 4.8 + 0.5 * mt : 0),
+            K > 1024 ? tiles * 0.0068 : 0);
+        if (odd || cw == 2 ? units < least : units <= least) {
             least = units;
             best = cw;
         }

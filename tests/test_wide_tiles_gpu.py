@@ -17,6 +17,9 @@ pytestmark = pytest.mark.gpu
     (40, 2043, 192), (127, 1801, 64),                       # eight
     # up to 32 rows: the stream, and three, five, seven and eight
     (24, 577, 3072), (25, 577, 3072), (32, 1183, 3136), (28, 1540, 3072),
-    (32, 2051, 3072), (31, 1025, 3008)])
+    (32, 2051, 3072), (31, 1025, 3008),
+    # three of a K that takes them, and six and seven beside the others' limits
+    (33, 601, 2112), (128, 767, 2048), (64, 1460, 192), (96, 1610, 1088),
+    (128, 1790, 1088)])
 def test_tiles(M, tiles, K):
     many_columns(M, tiles, K)

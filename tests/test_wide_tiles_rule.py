@@ -19,6 +19,17 @@ from ollamamq_amd.ops import hip
     (32, 65536, 3584, True, 8),         # 77, with eight 75
     (32, 22016, 4096, True, 3),         # 34, with three 32
     (24, 22016, 4096, True, 1), (32, 28672, 4096, True, 1),
+    # more rows: three tiles only of a K that has them divided ...
+    (33, 24576, 512, True, 4),          # 9.9, with three 11.1
+    (64, 20480, 1024, True, 4),         # 14.3, with three 14.9
+    (33, 24576, 1792, True, 4),         # 20.3, with three 21.3
+    (64, 22016, 4096, True, 3),         # 36.9, with four 38.1
+    # ... and eight where the weights' reads are what is left
+    (64, 49152, 4096, True, 8),         # 68.6, with six 72.2
+    (33, 57344, 3584, True, 8),         # 68.3, with seven 71.8
+    (128, 53248, 4096, True, 7),        # 79.1, with eight 83.1
+    (64, 49152, 1024, True, 6),         # 23.6, with eight 28.3
+    (64, 37888, 3584, True, 5), (128, 28672, 4096, True, 4),
 ])
 def test_choice(M, N, K, gated, tiles):
     hip.require()
