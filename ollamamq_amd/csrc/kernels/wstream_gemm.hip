@@ -77,10 +77,10 @@ extern "C" int wstream_pure_bf16(void* sink, const void* wp, int N, int K,
 // DEPTH: weights under way per wave, in 4 KiB iterations.
 // XLDS == 2: x in fragment layout (the decode chain).  A CU's loads are what
 // bounds it, x counted: rows past M repeat row M - 1, so few rows cost few
-// cache lines.  1 or 4 iterations ahead for 32 rows (frag_depth), in registers
-// for two blocks a CU; 2 for 64, where one block a CU with two of x under way beats two with
-// one (37888 x 3584: 70 us against 79).  28672 x 4096 with its norm and
-// activation: 46 us before for any M, now 44 for 32 rows, 39 for 1.
+// cache lines.  1, 2 or 4 iterations ahead for 32 rows (frag_depth), in registers
+// for two blocks a CU; 2 for 64, where one block a CU with two of x under way
+// beats two with one (37888 x 3584: 70 us against 79).  28672 x 4096 with its
+// norm and activation: 46 us before for any M, now 44 for 32 rows, 39 for 1.
 // XLDS (requires MT==1): stage the x fragments through a wave-PRIVATE
 // LDS tile instead of loading them in MFMA layout.  The direct x
 // fragment load is 32 rows x 16 B at an 8 KB stride = 32 cache-line
@@ -902,17 +902,35 @@ static int wide(int cw, void* y, const void* x, const void* wp, int M, int N,
 // Iterations ahead for 32 rows in fragment layout: four where every wave has whole
 // rounds of four, or one.  Slots of a first round that a wave does not have are
 // loaded all the same, and 4 KB of each of 16 waves are already twice what a CU
-// can have under way (32 KB, 57 GB/s of weights).  us for 1 and 32 rows, two
-// iterations the same as one within 2 %:
+// can have under way (32 KB, 57 GB/s of weights).  us for 1 and 32 rows:
 //                    one          four
 //   28672 x 4096     44.5  49.2   42.6  48.5      8 iterations a wave
 //   37888 x 3584     47.8  55.9   50.3  58.8      7
 //   18432 x 3072     23.5  27.6   26.9  31.9      6
 //   4096 x 14336     22.4  25.1   23.4  26.4      14, in two parts
 //   4096 x 11008     19.0  20.9   19.6  21.4      10 or 11
-static int frag_depth(int K, int ksplit)
+// Two of 17 rows and more where a CU has no second block to load meanwhile and
+// the waves have no more than two or four iterations, or half of them three, us
+// of one and two for 12 and 32 rows:
+//   2048 x 2048       6.4   7.2    6.4   6.9      2, in two parts
+//   4096 x 1024       4.9   5.6    4.9   5.4      2
+//   3584 x 3584       8.8   9.9    8.8   9.7      3 or 4, in two parts
+// With 256 blocks (8192 x 1024, norm and activation) 5.3 and 5.9, two 5.5 and 6.1;
+// of 3 iterations (3072 x 3072, in two parts) 7.6 and 8.8, two 8.4 and 9.1.
+static int frag_depth(int M, int N, int K, int ksplit)
 {
-    return K % (64 * 8 * 4 * ksplit) ? 1 : 4;
+    const int its = K / 64, waves = 8 * ksplit;
+    if (its % (4 * waves) == 0) return 4;
+    return M > 16 && N / 32 * ksplit < 256
+                   && (its == 2 * waves
+                       || (2 * its >= 7 * waves && its < 4 * waves))
+               ? 2 : 1;
+}
+
+extern "C" int wstream_depth(int M, int N, int K, int ksplit)
+{
+    return M < 1 || M > 32 || N < 32 || K < 64 || ksplit < 1
+               ? -104 : frag_depth(M, N, K, ksplit);
 }
 
 // Fused gate_up @ SwiGLU over GU-interleaved packed weights.
@@ -953,9 +971,10 @@ static int wstream_gu(
             nullptr, nullptr, {}, 0);
         return (int)hipGetLastError();
     }
-    const int d = frag_depth(K, 1);
-    auto go = xlds == 2 ? (d == 4 ? k_wstream_gemm<1, 4, 2, GU>
-                                  : k_wstream_gemm<1, 1, 2, GU>)
+    const int d = frag_depth(M, N, K, 1);
+    auto go = xlds == 2 ? (d == 4   ? k_wstream_gemm<1, 4, 2, GU>
+                           : d == 2 ? k_wstream_gemm<1, 2, 2, GU>
+                                    : k_wstream_gemm<1, 1, 2, GU>)
               : xlds == 1 ? k_wstream_gemm<1, 1, 1, GU>
                           : k_wstream_gemm<1, 1, 0, GU>;
     go<<<grid, 512, lds, stream>>>(
@@ -1012,7 +1031,7 @@ extern "C" int wstream_gemm_bf16(
     // what is fused needs the finished sums, and k_wstream_combine writes rows
     if (ksplit > 1 && !sem && (rstd_parts || res_in || sq_parts || yfrag))
         return -100;
-    const int d = frag_depth(K, ksplit);
+    const int d = frag_depth(M, N, K, ksplit);
     if (xlds == 2 && ksplit == 1 && y && !bias && !ri && !sq) {
         const int cw = wide_tiles(M, N, K, false);
         if (cw > 1)
@@ -1021,7 +1040,9 @@ extern "C" int wstream_gemm_bf16(
     }
     if (M <= 32) {
         if (xlds == 2)
-            (d == 4 ? k_wstream_gemm<1, 4, 2> : k_wstream_gemm<1, 1, 2>)
+            (d == 4   ? k_wstream_gemm<1, 4, 2>
+             : d == 2 ? k_wstream_gemm<1, 2, 2>
+                      : k_wstream_gemm<1, 1, 2>)
                 <<<grid, 512, lds_red, stream>>>(
                 (bf16*)y, (float*)part, (const bf16*)x, (const u32x4*)wp,
                 (const bf16*)bias, M, N, K, xs, ksplit, rp, rstd_nt,
@@ -1091,7 +1112,7 @@ extern "C" int wstream_qkv_rope_bf16(
     RopeEpi rp{(const float*)rcos, (const float*)rsin, (const int*)pos,
                (const int*)slot, (const int*)ptab, (bf16*)kp, (bf16*)vp,
                nl, nkl, psz, maxp};
-    const int d = frag_depth(K, 1);
+    const int d = frag_depth(M, N, K, 1);
     if (M > (xf ? 128 : 32)) return -104;          // rows of a block
     if (xf && M > 32)
         (M <= 64   ? k_wstream_gemm<2, 2, 2, 0, 1>
@@ -1102,8 +1123,9 @@ extern "C" int wstream_qkv_rope_bf16(
             (const bf16*)bias, M, N, K, xs, 1, (const float*)rstd_parts,
             rstd_nt, inv_h, eps, nullptr, nullptr, rp, 0, nullptr);
     else if (xf)
-        (d == 4 ? k_wstream_gemm<1, 4, 2, 0, 1>
-                : k_wstream_gemm<1, 1, 2, 0, 1>)
+        (d == 4   ? k_wstream_gemm<1, 4, 2, 0, 1>
+         : d == 2 ? k_wstream_gemm<1, 2, 2, 0, 1>
+                  : k_wstream_gemm<1, 1, 2, 0, 1>)
             <<<grid, 512, lds, stream>>>(
             (bf16*)y, nullptr, (const bf16*)x, (const u32x4*)wp,
             (const bf16*)bias, M, N, K, xs, 1, (const float*)rstd_parts,

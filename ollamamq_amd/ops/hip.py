@@ -63,6 +63,7 @@ def _try_load():
     lib.wstream_gemm_bf16.argtypes = [vp, vp, vp, vp, vp, i, i, i, i64, i,
                                       i, i, vp, i, f, f, vp, vp, i, vp, vp]
     lib.wstream_wide_tiles.argtypes = [i, i, i, i]
+    lib.wstream_depth.argtypes = [i, i, i, i]
     lib.wstream_pure_bf16.argtypes = [vp, vp, i, i, i, vp]
     lib.wstream_gu_bf16.argtypes = [vp, vp, vp, i, i, i, i64, i,
                                     vp, i, f, f, i, i, vp]

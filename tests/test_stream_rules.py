@@ -1,6 +1,6 @@
-"""Which streamed products share their rows between several tiles of columns:
-none that is slower for it than it was with the stream or with a power of two of
-tiles.  Each line was measured on both sides, us."""
+"""Which streamed products share their rows between several tiles of columns,
+and how far ahead of its sums a wave loads: no choice that is slower than the one
+before it.  Each line was measured on both sides, us."""
 import pytest
 
 from ollamamq_amd.ops import hip
@@ -31,12 +31,29 @@ from ollamamq_amd.ops import hip
     (64, 49152, 1024, True, 6),         # 23.6, with eight 28.3
     (64, 37888, 3584, True, 5), (128, 28672, 4096, True, 4),
 ])
-def test_choice(M, N, K, gated, tiles):
+def test_tiles(M, N, K, gated, tiles):
     hip.require()
     assert hip._lib.wstream_wide_tiles(M, N, K, gated) == tiles
+
+
+@pytest.mark.parametrize("M, N, K, parts, ahead", [
+    (32, 3584, 3584, 2, 2),             # 9.7, one 9.9
+    (32, 2048, 2048, 2, 2),             # 6.9, one 7.2
+    (17, 4096, 1024, 1, 2), (32, 4096, 1920, 1, 2),
+    (32, 8192, 1024, 1, 1),             # 5.9, two 6.1: a block a CU
+    (32, 3072, 3072, 2, 1),             # 8.8, two 9.1: three iterations
+    (16, 3584, 3584, 2, 1), (32, 4096, 512, 1, 1), (32, 18432, 3072, 1, 1),
+    (1, 4096, 4096, 2, 4), (32, 28672, 4096, 1, 4),
+])
+def test_iterations_ahead(M, N, K, parts, ahead):
+    hip.require()
+    assert hip._lib.wstream_depth(M, N, K, parts) == ahead
 
 
 def test_none():
     hip.require()
     for bad in ((0, 64, 64), (129, 64, 64), (1, 16, 64), (1, 64, 32)):
         assert hip._lib.wstream_wide_tiles(*bad, False) < 0
+    for bad in ((0, 64, 64, 1), (33, 64, 64, 1), (1, 16, 64, 1),
+                (1, 64, 64, 0)):
+        assert hip._lib.wstream_depth(*bad) < 0
