@@ -774,9 +774,19 @@ def rope_parts(M, N, K, cus=256):
       8192 x 4096  19.1 19.5   20.9 22.5   22.6 22.5   25.5 24.3   26.4 24.4
       5120 x 4096  17.3 16.9   19.2 19.4   20.8 19.3   23.6 21.2   24.3 21.2
       3072 x 2048  10.7 10.2   12.0 11.8   12.9 11.8   15.0 12.4   15.6 12.4
-    so parts from 97 rows on, and from 49 where there are three."""
+    so parts from 97 rows on, and from 49 where there are three.  Two parts of
+    a short K gain less than the fold takes, the less so where they are not
+    alike (97 rows):
+      4096 x 2048  14.5 15.0    6144 x 2560  18.6 17.4    8192 x 2816  20.0 20.6
+      6144 x 2048  15.4 16.5    8192 x 2304  18.0 19.0    8192 x 3072  20.5 20.1
+    and so do three of up to 56 rows where the stream's waves have whole rounds
+    (5120 x 4096 15.7 and 16.2, 60 rows 16.4 and 16.3, x 3584 15.3 and 14.7)."""
     parts = min(cus // -(-N // 64), K // 1024, 8)
     if parts < 2 or K % 256 or not 48 < M <= 128 or (M <= 96 and parts < 3):
+        return None
+    if parts == 2 and N > 2560 and K < (3072 if K % 512 else 2560):
+        return None
+    if parts == 3 and M <= 56 and N > 4096 and K <= 4096 and K % 1024 == 0:
         return None
     return 2 if M <= 64 else 4, 2, parts
 

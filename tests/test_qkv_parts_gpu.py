@@ -28,6 +28,22 @@ def test_rule():
     assert hip.rope_parts(96, 6144, 4096) is None
 
 
+@pytest.mark.parametrize("M, N, K, parts", [
+    # streams and parts, us
+    (97, 6144, 2048, None),             # 15.4, 16.5
+    (128, 5120, 2048, None),            # 15.3, 15.9
+    (97, 8192, 2816, None),             # 20.0, 20.6
+    (49, 5120, 4096, None),             # 15.7, 16.2
+    (56, 4608, 3072, None),             # 13.1, 13.4
+    (97, 2560, 2048, (4, 2, 2)),        # 14.2, 14.0
+    (97, 6144, 2560, (4, 2, 2)),        # 18.6, 17.4
+    (97, 6144, 3328, (4, 2, 2)),        # 21.4, 21.0
+    (57, 5120, 4096, (2, 2, 3)), (49, 5120, 3584, (2, 2, 3)),
+    (49, 5120, 5120, (2, 2, 3)), (49, 2560, 3072, (2, 2, 3))])
+def test_no_slower_than_the_stream(M, N, K, parts):
+    assert hip.rope_parts(M, N, K) == parts
+
+
 # the fold loads up to four parts at once; strips of 32 columns by the eight, a
 # rest, and fewer than its waves
 @pytest.mark.gpu
