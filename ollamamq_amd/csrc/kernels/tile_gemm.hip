@@ -326,21 +326,27 @@ __global__ __launch_bounds__(256, 1) void k_tile_gemm(const TileArgs a)
         for (int r = threadIdx.x; r < HM * 32; r += 256) {
             const float* p = sums_s + r * a.rstd_nt;
             // eight side by side, so of n the chain is of n / 8 + 3, and the
-            // bits are those of k_row_sums
+            // bits are those of k_row_sums; loads behind conditions of their own
+            // would spill 95 registers (8 x 8 tiles, 400 bytes a lane)
             f32x4 s{}, t{};
-            if (a.rstd_nt % 4 == 0)
+            if (a.rstd_nt % 8 == 0)
                 #pragma unroll 2
                 for (int e = 0; e < a.rstd_nt; e += 8) {
                     s += *reinterpret_cast<const f32x4*>(p + e);
-                    if (e + 4 < a.rstd_nt)
-                        t += *reinterpret_cast<const f32x4*>(p + e + 4);
+                    t += *reinterpret_cast<const f32x4*>(p + e + 4);
                 }
             else
-                for (int e = 0; e < a.rstd_nt; e += 8)
+                #pragma unroll 1
+                for (int e = 0; e < a.rstd_nt; e += 8) {
+                    const int last = a.rstd_nt - 1 - e;
                     #pragma unroll
-                    for (int i = 0; i < 8; i++)
-                        if (e + i < a.rstd_nt)
-                            (i < 4 ? s : t)[i & 3] += p[e + i];
+                    for (int i = 0; i < 4; i++) {
+                        const float u = p[e + min(i, last)];
+                        const float v = p[e + min(i + 4, last)];
+                        s[i] += i <= last ? u : 0.f;
+                        t[i] += i + 4 <= last ? v : 0.f;
+                    }
+                }
             row_f[r] = rsqrtf((s[0] + s[1] + (s[2] + s[3])
                                + (t[0] + t[1] + (t[2] + t[3])))
                               * a.inv_h + a.eps);
