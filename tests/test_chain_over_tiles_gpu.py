@@ -77,3 +77,39 @@ def test_against_general_path(kv_heads, bias, window, monkeypatch):
     for a, b in ((k1, k2), (v1, v2)):
         _close(a[b != 0], b[b != 0])
         assert torch.equal(a != 0, b != 0)
+
+
+@pytest.mark.parametrize("hidden, heads, kv_heads, taken", [
+    (4096, 32, 8, {97, 128}),                   # two parts
+    (3584, 28, 4, {49, 64, 65, 96, 97, 128})])  # three
+def test_qkv_in_parts(hidden, heads, kv_heads, taken, monkeypatch):
+    """Which steps take them, and that their queries, keys and values are the
+    general path's: over tiles of 64 and of 128 rows, prompts and decode."""
+    from ollamamq_amd.models import LlamaModel, PRESETS
+    from ollamamq_amd.ops import hip
+    cfg = dataclasses.replace(
+        PRESETS["qwen2-7b"], name="wide", hidden=hidden, n_heads=heads,
+        n_kv_heads=kv_heads, n_layers=2, ffn=2048, vocab=512, max_ctx=256)
+    model = LlamaModel(cfg, device="cuda:0", dtype=torch.bfloat16, seed=5,
+                       fast_init=True)
+    rows, product = [], hip.tile_qkv_parts
+
+    def spy(x, packed, M, *a):
+        rows.append(M)
+        return product(x, packed, M, *a)
+    monkeypatch.setattr(hip, "tile_qkv_parts", spy)
+    steps = [[(i, _text(n, i), [n - 1])]
+             for i, n in enumerate((48, 49, 64, 65, 96, 97, 128))]
+    steps += [[(i, [i], [0]) for i in range(n)] for n in (49, 97)]
+    size = dict(streams=97, ctx=256, pages=400)
+    got, k1, v1 = _run(model, cfg, True, steps, **size)
+    assert set(rows) == taken
+    took = len(rows)
+    assert took == 2 * (len(taken) + len(taken & {49, 97}))
+    want, k2, v2 = _run(model, cfg, False, steps, **size)
+    assert len(rows) == took
+    for a, b in zip(got, want):
+        _close(a.float(), b.float())
+    for a, b in ((k1, k2), (v1, v2)):
+        _close(a[b != 0], b[b != 0])
+        assert torch.equal(a != 0, b != 0)

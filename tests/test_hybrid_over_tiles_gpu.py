@@ -187,3 +187,29 @@ def test_what_stays_general(change, monkeypatch):
     for a, b in zip(got[0], want[0]):
         # but for the logits' product: see test_hybrid_short_prompts_gpu.py
         torch.testing.assert_close(a, b, rtol=2 ** -7, atol=1e-4)
+
+
+@pytest.mark.gpu
+def test_heads_that_are_not_whole_vectors_stay_general(monkeypatch):
+    """All of whose products would go over tiles: 32 heads of 20 are 640."""
+    rope, wide = RopeSpec(16, 1e4), dict(ff=200)
+    decay = tuple(0.5 + 0.015 * i for i in range(32))
+    kinds = {
+        "s": KavedraLayerSpec("lightning", 32, 24, 20, decay=decay, **wide),
+        "a": KavedraLayerSpec("attention", 32, 32, 20, kv_heads=16, scale=0.2,
+                              rope=rope, **wide),
+        "l": KavedraLayerSpec("latent_attention", 32, 16, 20, kv_rank=48,
+                              rot_dim=16, scale=0.17, window=50, rope=rope,
+                              **wide)}
+    cfg = KavedraConfig(name="many", width=256, vocab=320,
+                        layers=[kinds[c] for c in "slsa"], logit_scale=0.5,
+                        loop=(1, 3, 2), max_ctx=512)
+    model = build_model(cfg, device="cuda:0", dtype=torch.bfloat16, seed=3)
+    assert model.frag_decode and model.tiles_take(129)
+    assert not model.whole_heads
+    monkeypatch.setattr(hip, "_tile_rows", None)
+    got = _run(model, cfg, True, STEPS[:1])
+    want = _run(model, cfg, False, STEPS[:1])
+    for a, b in zip(got[0], want[0]):
+        # but for the logits' product: see test_hybrid_short_prompts_gpu.py
+        torch.testing.assert_close(a, b, rtol=2 ** -7, atol=1e-4)
