@@ -636,7 +636,8 @@ void k_wstream_gemm(
 // tiles costs one block more than the loads saved (4096 x 14336, 128 rows:
 // 56 us against 49).  More weights or activations under way give nothing.
 
-// parts of K that a block's waves walk side by side: eight to twelve waves
+// parts of K that a block's waves walk side by side: eight to twelve waves, of
+// seven tiles fourteen
 static constexpr __host__ __device__ int wide_parts(int cw)
 {
     return cw == 3 ? 3 : cw == 2 ? 4 : cw == 8 ? 1 : 2;
@@ -787,8 +788,8 @@ __global__ __launch_bounds__(CW * wide_parts(CW) * 64, 1) void k_wide(
     }
 }
 
-// Tiles a block: those with which the busiest CU is done first, in units of 4
-// KB a step of K.  A block of k_wide loads its tiles and all rows, or waits: two
+// Tiles a block: those with which the busiest of 256 CUs is done first, in units
+// of 4 KB a step of K.  A block of k_wide loads its tiles and all rows, or waits: two
 // tiles take what 4.8 + mt / 2 units take.  A tile of k_wstream_gemm (1), of
 // which a CU has several at a time, takes 0.8 (1 + mt), its rows coming from
 // L1 at times.  All weights take 0.0068 units a tile at the memory's rate, so

@@ -464,8 +464,9 @@ class LlamaModel:
                        attn_meta):
         """A step of few tokens, decode or short portions of prompts, as a
         fused weight-streaming chain (tp=1, up to ops.CHAIN_ROWS rows): 4
-        products per layer, of which o and down are two kernels each where
-        they go over tiles in parts, zero rmsnorm/swiglu kernels.
+        products per layer, of which o and down, and of some sizes qkv, are
+        two kernels each where they go over tiles in parts, zero
+        rmsnorm/swiglu kernels.
         rmsnorm weights are folded into the packs; the rstd scale rides
         each consumer GEMM's epilogue from sum-of-squares partials the
         producer GEMM emitted; residual adds happen in place inside the

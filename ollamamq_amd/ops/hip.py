@@ -773,8 +773,8 @@ def rope_parts(M, N, K, cus=256):
       4608 x 3584  16.8 14.8   18.7 17.1   20.4 17.1   23.2 18.2   23.9 18.3
       8192 x 4096  19.1 19.5   20.9 22.5   22.6 22.5   25.5 24.3   26.4 24.4
       5120 x 4096  17.3 16.9   19.2 19.4   20.8 19.3   23.6 21.2   24.3 21.2
-      3072 x 2048  10.7 10.2   12.0 11.8   12.9 11.8   15.0 12.4   15.6 12.4
-    so parts from 97 rows on, and from 49 where there are three.  Two parts of
+    so parts from 97 rows on, and from 49 where there are three; to 128 rows,
+    above which the fold was not measured against whole tiles.  Two parts of
     a short K gain less than the fold takes, the less so where they are not
     alike (97 rows):
       4096 x 2048  14.5 15.0    6144 x 2560  18.6 17.4    8192 x 2816  20.0 20.6
