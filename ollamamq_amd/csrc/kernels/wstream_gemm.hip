@@ -840,19 +840,22 @@ static int wide_tiles(int M, int N, int K, bool gated)
         }
         return tiles > 512 && (-tiles & 511) > 256 ? whole : 1;
     }
+    // two tiles of 64 rows are 5.8 units, one after the other 4.8 at most
+    auto units = [&](int cw) {
+        const int blocks = (tiles + cw - 1) / cw;
+        return (blocks + 255) / 256
+               * std::max<double>(cw + mt, cw < 4 ? 4.8 + 0.5 * mt : 0);
+    };
     int best = 1;
     double least = whole * 0.8 * (1 + mt);
-    // two tiles of 64 rows are 5.8 units, one after the other 4.8 at most
-    for (int cw = mt == 2 ? 3 : 2; cw <= 8; cw++) {
-        const bool odd = cw & (cw - 1);
-        if (odd && (cw < whole || (cw == 3 && K < 2048))) continue;
-        const int blocks = (tiles + cw - 1) / cw;
-        const double units = std::max(
-            (blocks + 255) / 256
-                * std::max<double>(cw + mt, cw < 4 ? 4.8 + 0.5 * mt : 0),
-            K > 1024 ? tiles * 0.0068 : 0);
-        if (odd || cw == 2 ? units < least : units <= least) {
-            least = units;
+    for (int cw = mt == 2 ? 4 : 2; cw <= 8; cw *= 2)
+        if (units(cw) < least) least = units(best = cw);
+    const double reads = K > 1024 ? tiles * 0.0068 : 0;
+    for (int cw : {3, 5, 6, 7}) {
+        if (cw < whole || (cw == 3 && K < 2048)) continue;
+        const double u = std::max(units(cw), reads);
+        if (u < least) {
+            least = u;
             best = cw;
         }
     }

@@ -30,6 +30,8 @@ from ollamamq_amd.ops import hip
     (128, 53248, 4096, True, 7),        # 79.1, with eight 83.1
     (64, 49152, 1024, True, 6),         # 23.6, with eight 28.3
     (64, 37888, 3584, True, 5), (128, 28672, 4096, True, 4),
+    (97, 65568, 4096, False, 4),        # 144, with eight 172
+    (128, 73728, 3584, True, 4),        # 134, with eight 143
 ])
 def test_tiles(M, N, K, gated, tiles):
     hip.require()
