@@ -686,9 +686,9 @@ __global__ __launch_bounds__(CW * wide_parts(CW) * 64, 1) void k_wide(
                 wq + (int64_t)min(b, max(hi, 1) - 1) * 256 + j * 64);
     };
     // Where a wave's 64 come from is the same for all of them, so it is worked out
-    // in scalar registers, behind the first weights.  Pointers kept per lane took
-    // 0.5 us of 14 before those (11008 x 1024) and with 128 rows 170 us instead of
-    // 160 (57344 x 8192).
+    // in scalar registers.  Pointers kept per lane took 0.5 us of 14 before the
+    // first weights (11008 x 1024) and with 128 rows 170 us instead of 160 (57344 x
+    // 8192).
     auto ldx = [&](int r) {
         #pragma unroll
         for (int i = 0; i < NX; i++) {
@@ -707,7 +707,10 @@ __global__ __launch_bounds__(CW * wide_parts(CW) * 64, 1) void k_wide(
     };
     #pragma unroll
     for (int s = 0; s < DEPTH; s++) ldw(s, lo + s);
-    __builtin_amdgcn_sched_barrier(0);
+    // where four parts begin takes longer than the weights' (1 to 3 % of 11008 x
+    // 1024); of fewer the compiler's order is better, by 2 us of 490 in four layers
+    // of 37 rows
+    if constexpr (KW == 4) __builtin_amdgcn_sched_barrier(0);
     ldx(0);
     // the norm's partial sums, FL lanes a row
     constexpr int FL = MT == 1 ? 16 : MT == 2 ? 8 : 4;
