@@ -905,6 +905,214 @@ static int wide(int cw, void* y, const void* x, const void* wp, int M, int N,
     return -105;                                       // no such tiles
 }
 
+// ---------------------------------------------------------------------------
+// Blocks of 16 columns and all of K for few rows in fragment layout.
+// k_wstream_gemm's 32 columns make 128 blocks of 4096, so such products go in
+// parts of K, and adding those up (stores through to memory, a ticket, loads
+// back) takes 2.4 us at the end of each.  Half as wide, 256 blocks load the same
+// weights without parts; but each loads all rows, so the more rows, the less it
+// is worth (narrow_pays).  us in parts and here, with residual and sums:
+//               rows     1            8           16           24           32
+//   4096 x 4096      9.8  7.2     9.9  7.2    10.0  7.7    10.4  8.5    10.6  9.7
+//   3584 x 3584      8.9  6.4     8.6  6.4     8.8  6.9     9.4  8.1     9.9  9.2
+//   2048 x 2048      6.5  4.4     6.5  4.4     6.5  4.7     6.9  5.4     7.0  5.9
+//   4096 x 14336    22.6 21.5    22.8 21.3    23.0 22.8    23.9 25.9    25.7 31.3
+// (7.2 us are 4.7 TB/s.)  A line of 128 bytes of the pack has eight columns, so a
+// wave's load takes whole lines here too: columns 16 h to 16 h + 15 of a tile, or,
+// where a rotation pairs columns, 8 h to 8 h + 7 of both its halves.
+// Rows are asked for as far ahead as weights, as loads return in order; four
+// steps are as fast as six or eight, in registers for three blocks a CU.
+// ROPE: norm, rotation and append as k_wstream_gemm has them, else residual and
+// sums of squares.
+template <int RT, bool ROPE>
+__global__ __launch_bounds__(512, RT == 1 ? 6 : 4) void k_narrow(
+    bf16* y, const u32x4* __restrict__ x, const u32x4* __restrict__ wp,
+    const bf16* __restrict__ bias, int M, int N, int K,
+    const float* __restrict__ rstd_parts, int rstd_nt, float inv_h, float eps,
+    const bf16* res_in, float* __restrict__ sq_parts, RopeEpi rp = {})
+{
+    constexpr int D = 4;                      // steps of 64 under way
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t = blockIdx.x >> 1, half = blockIdx.x & 1;
+    const int NB = K >> 6, lo = wid * NB / 8, hi = (wid + 1) * NB / 8;
+    const int last = max(hi - 1, lo);
+    const int qt = rp.nl * 4, kt = rp.nkl * 4;         // tiles per section
+    const bool pairs = ROPE && t < qt + kt;
+    // a lane's unit of 16 bytes: eight of k of one column, or row
+    const unsigned unit = (g >> 1) * 64 + (g & 1) * 32;
+    const int c = pairs ? (r & 8) * 2 + half * 8 + (r & 7) : half * 16 + r;
+    typedef __attribute__((address_space(1))) const char* Global;
+    const uint64_t lw = (unit + c) * 16u;
+    uint64_t lx[RT];
+    #pragma unroll
+    for (int m = 0; m < RT; m++)
+        lx[m] = (unit + min(m * 16 + r, M - 1)) * 16u;
+    const Global wq = (Global)(wp + (int64_t)t * NB * 256), xq = (Global)x;
+    u4bf8 w[D][2], xr[D][RT][2];
+    f32x4 acc[RT] = {};
+    auto step = [](Global p, int b) {
+        Global q = p + (int64_t)b * 4096;
+        asm("" : "+s"(q));                    // no address per lane
+        return q;
+    };
+    auto load = [&](int s, int b) {
+        const Global q = step(wq, b), p = step(xq, b);
+        #pragma unroll
+        for (int a = 0; a < 2; a++)
+            w[s][a].u = __builtin_nontemporal_load(
+                (const u32x4*)(q + lw + a * 2048));
+        #pragma unroll
+        for (int m = 0; m < RT; m++)
+            #pragma unroll
+            for (int a = 0; a < 2; a++)
+                xr[s][m][a].u = *(const u32x4*)(p + lx[m] + a * 2048);
+    };
+    auto mul = [&](int s) {
+        #pragma unroll
+        for (int a = 0; a < 2; a++)
+            #pragma unroll
+            for (int m = 0; m < RT; m++)
+                acc[m] = mma(xr[s][m][a].v, w[s][a].v, acc[m]);
+    };
+    #pragma unroll
+    for (int s = 0; s < D; s++) load(s, min(lo + s, last));
+    // this thread's result, and what it needs besides the sum
+    const int row = threadIdx.x >> 4, col = threadIdx.x & 15;
+    float add = 0.f, rsum = 0.f;
+    if (!ROPE) {
+        if (row < min(M, RT * 16))
+            add = __bfloat162float(
+                res_in[frag_off(row, blockIdx.x * 16 + col)]);
+    } else {
+        // the norm's partial sums, FL lanes a row
+        constexpr int FL = 512 / (RT * 16);
+        const int m = threadIdx.x / FL;
+        if (m < M) {
+            const float* p = rstd_parts + (int64_t)m * rstd_nt;
+            int i = threadIdx.x % FL;
+            for (; i + 7 * FL < rstd_nt; i += 8 * FL) {
+                float v[8];
+                #pragma unroll
+                for (int k = 0; k < 8; k++) v[k] = p[i + k * FL];
+                #pragma unroll
+                for (int k = 0; k < 8; k++) rsum += v[k];
+            }
+            for (; i + FL < rstd_nt; i += 2 * FL) rsum += p[i] + p[i + FL];
+            if (i < rstd_nt) rsum += p[i];
+        }
+    }
+    int b = lo;
+    for (; b + 2 * D <= hi; b += D)
+        #pragma unroll
+        for (int s = 0; s < D; s++) {
+            mul(s);
+            load(s, b + s + D);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    #pragma unroll
+    for (int s = 0; s < D; s++) {
+        if (b + s < hi) mul(s);
+        if (b + s + D < hi) load(s, b + s + D);
+    }
+    #pragma unroll
+    for (int s = 0; s < D - 1; s++)
+        if (b + s + D < hi) mul(s);
+
+    // the waves' sums; rows of 20 are 16 banks apart four rows on
+    __shared__ float red[8][RT * 16][20];
+    __shared__ float rstd_s[RT * 16];
+    #pragma unroll
+    for (int m = 0; m < RT; m++)
+        #pragma unroll
+        for (int i = 0; i < 4; i++) red[wid][m * 16 + g * 4 + i][r] = acc[m][i];
+    if (ROPE) {
+        constexpr int FL = 512 / (RT * 16);
+        #pragma unroll
+        for (int o = FL / 2; o; o >>= 1) rsum += __shfl_down(rsum, o, 64);
+        if (threadIdx.x % FL == 0)
+            rstd_s[threadIdx.x / FL] = rsqrtf(rsum * inv_h + eps);
+    }
+    __syncthreads();
+    if (row >= RT * 16) return;
+    auto total = [&](int n) {
+        float s = 0.f;
+        #pragma unroll
+        for (int v = 0; v < 8; v++) s += red[v][row][n];
+        return s;
+    };
+    if (!ROPE) {
+        float s = total(col) + add;
+        if (row < M)
+            y[frag_off(row, blockIdx.x * 16 + col)] = __float2bfloat16(s);
+        s *= s;
+        #pragma unroll
+        for (int o = 8; o; o >>= 1) s += __shfl_xor(s, o, 64);
+        if (col == 0 && row < M)
+            sq_parts[(int64_t)row * gridDim.x + blockIdx.x] = s;
+        return;
+    }
+    if (row >= M || (pairs && col >= 8)) return;
+    const float rs = rstd_s[row];
+    float lo_v = total(col) * rs, hi_v = pairs ? total(col + 8) * rs : 0.f;
+    const int p = rp.pos[row], n0 = half * (pairs ? 8 : 16) + col;
+    if (bias) {
+        lo_v += __bfloat162float(bias[t * 32 + n0]);
+        if (pairs) hi_v += __bfloat162float(bias[t * 32 + 16 + n0]);
+    }
+    const int sec = t < qt ? t : pairs ? t - qt : t - qt - kt, head = sec >> 2;
+    bf16* dst = y + (int64_t)row * N + head * 128;
+    if (t >= qt) {
+        const int page = rp.ptab[rp.slot[row] * rp.maxp + p / rp.psz];
+        dst = (pairs ? rp.kp : rp.vp)
+              + (((int64_t)page * rp.nkl + head) * rp.psz + p % rp.psz) * 128;
+    }
+    if (pairs) {
+        const int d = (sec & 3) * 16 + n0;
+        const float co = rp.cos_t[p * 64 + d], si = rp.sin_t[p * 64 + d];
+        dst[d] = __float2bfloat16(lo_v * co - hi_v * si);
+        dst[64 + d] = __float2bfloat16(hi_v * co + lo_v * si);
+    } else
+        dst[(sec & 3) * 32 + n0] = __float2bfloat16(lo_v);
+}
+
+// Whether a product that would go in `ksplit` parts goes in blocks of 16 columns:
+// where the busiest of 256 CUs has less than 210 KB more to load, rows counted by
+// the eight of a cache line, which it does in the time that adding up the parts
+// takes; without parts where it has no more.  Over 11 numbers of columns from
+// 1024 to 8192, 11 of K from 1024 to 28672 and 1 to 32 rows the choice takes 0.6 %
+// more than the better one, parts alone 6 %, 16 columns alone 11 %.
+static bool narrow_pays(int M, int N, int K, int ksplit)
+{
+    const int rows = (M + 7) / 8 * 8;
+    auto busiest = [](int blocks) { return (int64_t)((blocks + 255) / 256); };
+    const int64_t more = busiest(N / 16) * K * (32 + 2 * rows)
+                         - busiest(N / 32 * ksplit) * (K / ksplit)
+                               * (64 + 2 * rows);
+    return M <= 32 && more <= (ksplit > 1 ? 210 << 10 : 0);
+}
+
+extern "C" int wstream_narrow(int M, int N, int K, int ksplit)
+{
+    return M < 1 || N < 32 || K < 64 || ksplit < 1
+               ? -104 : narrow_pays(M, N, K, ksplit);
+}
+
+// y = x W^T + res_in, both in fragment layout (they may be one); sq_parts: N / 16
+// sums of squares a row
+extern "C" int wstream_narrow_bf16(
+    void* y, const void* x, const void* wp, int M, int N, int K,
+    const void* res_in, void* sq_parts, hipStream_t stream)
+{
+    if (M < 1 || M > 32 || N < 32 || N % 32 || K < 64 || K % 64 || !res_in
+        || !sq_parts)
+        return -104;
+    (M <= 16 ? k_narrow<1, false> : k_narrow<2, false>)<<<N / 16, 512, 0, stream>>>(
+        (bf16*)y, (const u32x4*)x, (const u32x4*)wp, nullptr, M, N, K, nullptr,
+        0, 0.f, 0.f, (const bf16*)res_in, (float*)sq_parts, RopeEpi{});
+    return (int)hipGetLastError();
+}
+
 // Iterations ahead for 32 rows in fragment layout: four where every wave has whole
 // rounds of four, or one.  Slots of a first round that a wave does not have are
 // loaded all the same, and 4 KB of each of 16 waves are already twice what a CU
@@ -1120,6 +1328,15 @@ extern "C" int wstream_qkv_rope_bf16(
                nl, nkl, psz, maxp};
     const int d = frag_depth(M, N, K, 1);
     if (M > (xf ? 128 : 32)) return -104;          // rows of a block
+    // blocks of 32 columns that are more than the CUs leave some of them two (12288
+    // x 4096, 1 to 16 rows: 3.3 to 2.6 us less of 22; 6144 x 4096: none)
+    if (xf && M <= 16 && N > 256 * 32) {
+        k_narrow<1, true><<<N / 16, 512, 0, stream>>>(
+            (bf16*)y, (const u32x4*)x, (const u32x4*)wp, (const bf16*)bias, M, N,
+            K, (const float*)rstd_parts, rstd_nt, inv_h, eps, nullptr, nullptr,
+            rp);
+        return (int)hipGetLastError();
+    }
     if (xf && M > 32)
         (M <= 64   ? k_wstream_gemm<2, 2, 2, 0, 1>
          : M <= 96 ? k_wstream_gemm<3, 2, 2, 0, 1>

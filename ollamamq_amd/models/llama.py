@@ -482,7 +482,7 @@ class LlamaModel:
         tiles_h = H // 32
         dev = self.embed.device
         rows = -(-B // 32) * 32          # the products write these of sq
-        sq_a, sq_b = torch.empty((2, rows * tiles_h), dtype=torch.float32,
+        sq_a, sq_b = torch.empty((2, rows * H // 16), dtype=torch.float32,
                                  device=dev)
         tickets = torch.empty(max(tiles_h, B * nkl), dtype=torch.int32,
                               device=dev)
@@ -541,27 +541,23 @@ class LlamaModel:
             q = qkv[:, :nl * d].view(-1, nl, d)
             attn = ops.attention_frag(q, kv_cache, li, attn_meta,
                                       tickets)
-            nb = tiles_h
             if o_tiles:
                 sq_b, nb = ops.tile_residual(attn, layer.wo_pk, B, H, nl * d,
                                              res)
             else:
-                ops.linear_fused(attn, layer.wo_pk, H, res=res, sq_out=sq_b,
-                                 y=res, yfrag=1, K=nl * d, xlds=2, M_frag=B,
-                                 sem=tickets)
+                nb = ops.linear_residual(attn, layer.wo_pk, B, H, nl * d, res,
+                                         sq_b, tickets)
             act = ops.gu_fused(res, layer.wgu_pk,
                                layer.wgate_up.shape[0], rstd=sq_b,
                                rstd_nt=nb, inv_h=inv_h, eps=eps,
                                K=H, yfrag=1, M_frag=B)
-            nt = tiles_h
             if down_tiles:
                 sq_a, nt = ops.tile_residual(act, layer.wdown_pk, B, H,
                                              layer.wdown.shape[1], res)
             else:
-                ops.linear_fused(act, layer.wdown_pk, H, res=res,
-                                 sq_out=sq_a, y=res, yfrag=1,
-                                 K=layer.wdown.shape[1], xlds=2, M_frag=B,
-                                 sem=tickets)
+                nt = ops.linear_residual(act, layer.wdown_pk, B, H,
+                                         layer.wdown.shape[1], res, sq_a,
+                                         tickets)
         idx = attn_meta.logits_idx
         if (idx is not None and 0 < idx.shape[0] <= ops.CHAIN_ROWS
                 and attn_meta.rows != list(range(B))):

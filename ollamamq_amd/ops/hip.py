@@ -62,6 +62,8 @@ def _try_load():
     lib.set_entries.argtypes = [vp, i64, vp, vp, i, vp]
     lib.wstream_gemm_bf16.argtypes = [vp, vp, vp, vp, vp, i, i, i, i64, i,
                                       i, i, vp, i, f, f, vp, vp, i, vp, vp]
+    lib.wstream_narrow.argtypes = [i, i, i, i]
+    lib.wstream_narrow_bf16.argtypes = [vp, vp, vp, i, i, i, vp, vp, vp]
     lib.wstream_wide_tiles.argtypes = [i, i, i, i]
     lib.wstream_depth.argtypes = [i, i, i, i]
     lib.wstream_pure_bf16.argtypes = [vp, vp, i, i, i, vp]
@@ -967,6 +969,27 @@ def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
         _p(rstd), rstd_nt, float(inv_h), float(eps), _p(res), _p(sq_out),
         yfrag, _p(sem), _stream()), "wstream_gemm")
     return y
+
+
+@functools.lru_cache(maxsize=4096)
+def narrow_pays(M, N, K):
+    """Whether a residual product of M rows goes in blocks of 16 columns."""
+    return M <= 32 and _lib.wstream_narrow(M, N, K, _frag_ksplit(N, K)) == 1
+
+
+def linear_residual(x, packed, M, N, K, res, sq, sem):
+    """res += x @ W^T, x and res in fragment layout; sq gets sums of squares of
+    the result, m-major, and has room for N / 16 a row.  Returns how many there
+    are.  sem: see linear_packed."""
+    if asked_parts(K) is None and narrow_pays(M, N, K):
+        assert sq.numel() >= M * (N // 16)
+        _check(_lib.wstream_narrow_bf16(
+            _p(res), _p(x), _p(packed), M, N, K, _p(res), _p(sq), _stream()),
+            "wstream_narrow")
+        return N // 16
+    linear_packed(x, packed, None, N, res=res, sq_out=sq, y=res, yfrag=1, K=K,
+                  xlds=2, M_frag=M, sem=sem)
+    return N // 32
 
 
 def fragify_sumsq(x, sq=None, tokens=None, rows=None, add=None, clear=None):

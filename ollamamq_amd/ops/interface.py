@@ -788,6 +788,13 @@ def linear_fused(x, packed, N, bias=None, rstd=None, rstd_nt=0,
                              K=K, xlds=xlds, M_frag=M_frag, sem=sem)
 
 
+def linear_residual(x, packed, M, N, K, res, sq, sem):
+    """A streamed product's residual form in the fused chain: res += x @ W^T,
+    and its sums of squares for the next product's rstd; returns how many of
+    them a row has.  See hip.linear_residual."""
+    return hip.linear_residual(x, packed, M, N, K, res, sq, sem)
+
+
 def fragify_sumsq(x, sq=None, tokens=None, rows=None, add=None, clear=None):
     """Standard [M, H] -> 32-row frag layout + per-row sum of squares; with
     tokens, of their rows of the embedding table x; with rows, of these rows

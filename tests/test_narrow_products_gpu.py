@@ -1,0 +1,104 @@
+"""Products of up to 32 rows in blocks of 16 columns: residual and sums of squares,
+rotation and append.
+
+Tolerance: sums of up to K products of bf16 values in fp32, whose error is below
+K 2^-24 of the sum of magnitudes, then one rounding to bf16 (2^-9 of the value,
+doubled as the sum's error can cross a tie).  A row's sum of squares is taken of
+the values before that rounding: K 2^-22 of it at most, as values' errors count
+twice.
+"""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(flat, M, W):
+    """Rows of an activation in fragment layout."""
+    t = flat.view(W // 16, 2, 32, 8)                 # 16 and 8 of W, row
+    return t.permute(2, 0, 1, 3).reshape(32, W)[:M]
+
+
+# waves without a step, with one, with four and more than four; halves of a wave's
+# rows
+@pytest.mark.parametrize("N,K", [(32, 64), (96, 512), (64, 64 * 37),
+                                 (2048, 2048), (32, 64 * 71)])
+@pytest.mark.parametrize("M", [1, 7, 16, 17, 31, 32])
+def test_residual(M, N, K):
+    from ollamamq_amd.ops import hip
+    hip.require()
+    g = torch.Generator(device="cuda").manual_seed(M * N + K)
+
+    def rand(*shape):
+        return torch.randn(shape, generator=g, device="cuda").bfloat16()
+
+    x, w, r = rand(M, K), rand(N, K), rand(M, N)
+    xf, rf = (hip.fragify_sumsq(t)[0] for t in (x, r))
+    sq = torch.full((M * N // 16 + 64,), 7.0, device="cuda")
+    hip._check(hip._lib.wstream_narrow_bf16(
+        hip._p(rf), hip._p(xf), hip._p(hip.pack_weight(w)), M, N, K,
+        hip._p(rf), hip._p(sq), hip._stream()), "wstream_narrow")
+    want = x.double() @ w.double().T + r.double()
+    size = x.double().abs() @ w.double().abs().T + r.double().abs()
+    err = (_rows(rf, M, N).double() - want).abs()
+    assert (err <= 2 ** -8 * want.abs() + K * 2 ** -24 * size).all()
+    sums = sq[:M * N // 16].view(M, -1).double().sum(1)
+    torch.testing.assert_close(sums, want.square().sum(1), rtol=K * 2 ** -22,
+                               atol=0)
+    assert (sq[M * N // 16:] == 7).all()
+
+
+def test_residual_refused():
+    from ollamamq_amd.ops import hip
+    hip.require()
+    t = torch.zeros(64 * 64, device="cuda", dtype=torch.bfloat16)
+    p = hip._p(t)
+    for M, N, K, res in ((0, 32, 64, p), (33, 32, 64, p), (1, 16, 64, p),
+                         (1, 48, 64, p), (1, 32, 32, p), (1, 32, 64, None)):
+        assert hip._lib.wstream_narrow_bf16(p, p, p, M, N, K, res, p,
+                                            hip._stream())
+
+
+# more than 256 tiles of 32 columns: up to 16 rows in blocks of 16, above in
+# blocks of 32.  A row's results do not hang on the rows beside it.
+@pytest.mark.parametrize("nl,nkl,bias", [(66, 1, True), (22, 22, False)])
+@pytest.mark.parametrize("M", [1, 9, 16])
+def test_rotated(M, nl, nkl, bias):
+    from ollamamq_amd.engine import PagedKVCache
+    from ollamamq_amd.ops import hip
+    hip.require()
+    g = torch.Generator(device="cuda").manual_seed(M)
+    N, K, T = (nl + 2 * nkl) * 128, 64 * 11, 17
+    assert N > 256 * 32
+
+    def rand(*shape):
+        return torch.randn(shape, generator=g, device="cuda").bfloat16()
+
+    x, w = rand(T, K), rand(N, K)
+    b = rand(N) if bias else None                    # in the order of the pack
+    packed = hip.pack_weight_qkv_rope(w, nl, nkl)
+    ang = torch.rand(64, 64, generator=g, device="cuda") * 6.28
+    cos, sin = ang.cos(), ang.sin()
+    got = []
+    for m in (T, M):
+        cache = PagedKVCache(1, nkl, 128, n_pages=64, max_slots=T, max_ctx=64,
+                             device="cuda", dtype=torch.bfloat16)
+        slots = [cache.alloc_slot() for _ in range(m)]
+        for i, s in enumerate(slots):
+            cache.ensure(s, 2 * i + 1)
+        xf, sq = hip.fragify_sumsq(x[:m])
+        q = hip.linear_qkv_rope(
+            xf, packed, N, b, cache, 0,
+            torch.arange(m, device="cuda", dtype=torch.int32) * 2,
+            torch.tensor(slots, device="cuda", dtype=torch.int32), cos, sin,
+            nl, nkl, sq, 1, 1.0 / K, 1e-5, K=K, M_real=m)
+        pools = [torch.stack([
+            pool[0, cache.page_table[s, 2 * i // 16].long(), :, 2 * i % 16]
+            for i, s in enumerate(slots[:M])])
+            for pool in (cache.k_pool, cache.v_pool)]
+        got.append([q[:M, :nl * 128], *pools])
+    for a, c in zip(*got):
+        assert a.abs().max() > 0.1
+        # both round sums of the same terms, of size sqrt(K) in fp32
+        torch.testing.assert_close(a.float(), c.float(), rtol=2 ** -7,
+                                   atol=K * 2 ** -20)
