@@ -917,6 +917,11 @@ static int wide(int cw, void* y, const void* x, const void* wp, int M, int N,
 //   3584 x 3584      8.9  6.4     8.6  6.4     8.8  6.9     9.4  8.1     9.9  9.2
 //   2048 x 2048      6.5  4.4     6.5  4.4     6.5  4.7     6.9  5.4     7.0  5.9
 //   4096 x 14336    22.6 21.5    22.8 21.3    23.0 22.8    23.9 25.9    25.7 31.3
+// and over tiles from 49 rows on:
+//               rows    40           48           56                64
+//   4096 x 4096     13.0 12.1    13.9 12.3    13.3 15.7 12.6    13.6 15.7 13.7
+//   3584 x 3584     11.9 11.0    11.7 10.7    12.3 14.3 11.8    12.6 14.2 12.4
+//   2048 x 2048      8.5  6.7     8.6  7.0     8.9 12.1  7.8     9.1 12.2  8.4
 // (7.2 us are 4.7 TB/s.)  A line of 128 bytes of the pack has eight columns, so a
 // wave's load takes whole lines here too: columns 16 h to 16 h + 15 of a tile, or,
 // where a rotation pairs columns, 8 h to 8 h + 7 of both its halves.
@@ -925,7 +930,7 @@ static int wide(int cw, void* y, const void* x, const void* wp, int M, int N,
 // ROPE: norm, rotation and append as k_wstream_gemm has them, else residual and
 // sums of squares.
 template <int RT, bool ROPE>
-__global__ __launch_bounds__(512, RT == 1 ? 6 : 4) void k_narrow(
+__global__ __launch_bounds__(512, RT == 1 ? 6 : RT == 2 ? 4 : 2) void k_narrow(
     bf16* y, const u32x4* __restrict__ x, const u32x4* __restrict__ wp,
     const bf16* __restrict__ bias, int M, int N, int K,
     const float* __restrict__ rstd_parts, int rstd_nt, float inv_h, float eps,
@@ -946,8 +951,10 @@ __global__ __launch_bounds__(512, RT == 1 ? 6 : 4) void k_narrow(
     const uint64_t lw = (unit + c) * 16u;
     uint64_t lx[RT];
     #pragma unroll
-    for (int m = 0; m < RT; m++)
-        lx[m] = (unit + min(m * 16 + r, M - 1)) * 16u;
+    for (int m = 0; m < RT; m++) {
+        const int at = min(m * 16 + r, M - 1);
+        lx[m] = (uint64_t)(at >> 5) * K * 64 + (unit + (at & 31)) * 16u;
+    }
     const Global wq = (Global)(wp + (int64_t)t * NB * 256), xq = (Global)x;
     u4bf8 w[D][2], xr[D][RT][2];
     f32x4 acc[RT] = {};
@@ -977,16 +984,19 @@ __global__ __launch_bounds__(512, RT == 1 ? 6 : 4) void k_narrow(
     };
     #pragma unroll
     for (int s = 0; s < D; s++) load(s, min(lo + s, last));
-    // this thread's result, and what it needs besides the sum
+    // this thread's results, of rows 32 apart, and what they need besides the sums
+    constexpr int RR = (RT + 1) / 2, FL = RT > 2 ? 8 : 512 / (RT * 16);
     const int row = threadIdx.x >> 4, col = threadIdx.x & 15;
-    float add = 0.f, rsum = 0.f;
+    const int n16 = blockIdx.x * 16 + col;
+    float add[RR] = {}, rsum = 0.f;
     if (!ROPE) {
-        if (row < min(M, RT * 16))
-            add = __bfloat162float(
-                res_in[frag_off(row, blockIdx.x * 16 + col)]);
+        #pragma unroll
+        for (int i = 0; i < RR; i++)
+            if (row + i * 32 < min(M, RT * 16))
+                add[i] = __bfloat162float(
+                    res_in[frag_row_off(row + i * 32, n16, N)]);
     } else {
         // the norm's partial sums, FL lanes a row
-        constexpr int FL = 512 / (RT * 16);
         const int m = threadIdx.x / FL;
         if (m < M) {
             const float* p = rstd_parts + (int64_t)m * rstd_nt;
@@ -1027,34 +1037,37 @@ __global__ __launch_bounds__(512, RT == 1 ? 6 : 4) void k_narrow(
         #pragma unroll
         for (int i = 0; i < 4; i++) red[wid][m * 16 + g * 4 + i][r] = acc[m][i];
     if (ROPE) {
-        constexpr int FL = 512 / (RT * 16);
         #pragma unroll
         for (int o = FL / 2; o; o >>= 1) rsum += __shfl_down(rsum, o, 64);
         if (threadIdx.x % FL == 0)
             rstd_s[threadIdx.x / FL] = rsqrtf(rsum * inv_h + eps);
     }
     __syncthreads();
-    if (row >= RT * 16) return;
-    auto total = [&](int n) {
+    auto total = [&](int m, int n) {
         float s = 0.f;
         #pragma unroll
-        for (int v = 0; v < 8; v++) s += red[v][row][n];
+        for (int v = 0; v < 8; v++) s += red[v][m][n];
         return s;
     };
     if (!ROPE) {
-        float s = total(col) + add;
-        if (row < M)
-            y[frag_off(row, blockIdx.x * 16 + col)] = __float2bfloat16(s);
-        s *= s;
         #pragma unroll
-        for (int o = 8; o; o >>= 1) s += __shfl_xor(s, o, 64);
-        if (col == 0 && row < M)
-            sq_parts[(int64_t)row * gridDim.x + blockIdx.x] = s;
+        for (int i = 0; i < RR; i++) {
+            const int m = row + i * 32;
+            if (m >= RT * 16) return;
+            float s = total(m, col) + add[i];
+            if (m < M) y[frag_row_off(m, n16, N)] = __float2bfloat16(s);
+            s *= s;
+            #pragma unroll
+            for (int o = 8; o; o >>= 1) s += __shfl_xor(s, o, 64);
+            if (col == 0 && m < M)
+                sq_parts[(int64_t)m * gridDim.x + blockIdx.x] = s;
+        }
         return;
     }
-    if (row >= M || (pairs && col >= 8)) return;
+    if (row >= min(M, RT * 16) || (pairs && col >= 8)) return;
     const float rs = rstd_s[row];
-    float lo_v = total(col) * rs, hi_v = pairs ? total(col + 8) * rs : 0.f;
+    float lo_v = total(row, col) * rs;
+    float hi_v = pairs ? total(row, col + 8) * rs : 0.f;
     const int p = rp.pos[row], n0 = half * (pairs ? 8 : 16) + col;
     if (bias) {
         lo_v += __bfloat162float(bias[t * 32 + n0]);
@@ -1077,11 +1090,12 @@ __global__ __launch_bounds__(512, RT == 1 ? 6 : 4) void k_narrow(
 }
 
 // Whether a product that would go in `ksplit` parts goes in blocks of 16 columns:
-// where the busiest of 256 CUs has less than 210 KB more to load, rows counted by
+// where the busiest of 256 CUs has at most 256 KB more to load, rows counted by
 // the eight of a cache line, which it does in the time that adding up the parts
 // takes; without parts where it has no more.  Over 11 numbers of columns from
 // 1024 to 8192, 11 of K from 1024 to 28672 and 1 to 32 rows the choice takes 0.6 %
-// more than the better one, parts alone 6 %, 16 columns alone 11 %.
+// more than the better one, parts alone 6 %, 16 columns alone 11 %; of 33 to 64
+// rows, over 4 of columns and 5 of K from 1024 to 5632, 0.6, 5 and 5 %.
 static bool narrow_pays(int M, int N, int K, int ksplit)
 {
     const int rows = (M + 7) / 8 * 8;
@@ -1089,7 +1103,7 @@ static bool narrow_pays(int M, int N, int K, int ksplit)
     const int64_t more = busiest(N / 16) * K * (32 + 2 * rows)
                          - busiest(N / 32 * ksplit) * (K / ksplit)
                                * (64 + 2 * rows);
-    return M <= 32 && more <= (ksplit > 1 ? 210 << 10 : 0);
+    return M <= 64 && more <= (ksplit > 1 ? 256 << 10 : 0);
 }
 
 extern "C" int wstream_narrow(int M, int N, int K, int ksplit)
@@ -1104,10 +1118,13 @@ extern "C" int wstream_narrow_bf16(
     void* y, const void* x, const void* wp, int M, int N, int K,
     const void* res_in, void* sq_parts, hipStream_t stream)
 {
-    if (M < 1 || M > 32 || N < 32 || N % 32 || K < 64 || K % 64 || !res_in
+    if (M < 1 || M > 64 || N < 32 || N % 32 || K < 64 || K % 64 || !res_in
         || !sq_parts)
         return -104;
-    (M <= 16 ? k_narrow<1, false> : k_narrow<2, false>)<<<N / 16, 512, 0, stream>>>(
+    (M <= 16   ? k_narrow<1, false>
+     : M <= 32 ? k_narrow<2, false>
+     : M <= 48 ? k_narrow<3, false>
+               : k_narrow<4, false>)<<<N / 16, 512, 0, stream>>>(
         (bf16*)y, (const u32x4*)x, (const u32x4*)wp, nullptr, M, N, K, nullptr,
         0, 0.f, 0.f, (const bf16*)res_in, (float*)sq_parts, RopeEpi{});
     return (int)hipGetLastError();

@@ -512,10 +512,13 @@ class LlamaModel:
         # of one round some take less time in parts
         qkv_parts = ops.rope_parts(B, self.layers[0].wqkv.shape[0], H, dev) \
             if tiles and not qkv_tiles else None
-        # a switch that asks for parts means the streams'
-        o_tiles = tiles and ops.asked_parts(nl * d) is None
-        down_tiles = tiles and ops.asked_parts(
-            self.layers[0].wdown.shape[1]) is None
+        # a switch that asks for parts means the streams'; blocks of 16 columns
+        # are before tiles where they pay
+        def over_tiles(K):
+            return (tiles and ops.asked_parts(K) is None
+                    and not ops.narrow_pays(B, H, K))
+        o_tiles = over_tiles(nl * d)
+        down_tiles = over_tiles(self.layers[0].wdown.shape[1])
         for li, layer in enumerate(self.layers):
             # fused rmsnorm -> qkv -> RoPE -> paged KV append: q comes
             # back rotated in standard layout, k/v land in the pool

@@ -974,7 +974,7 @@ def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
 @functools.lru_cache(maxsize=4096)
 def narrow_pays(M, N, K):
     """Whether a residual product of M rows goes in blocks of 16 columns."""
-    return M <= 32 and _lib.wstream_narrow(M, N, K, _frag_ksplit(N, K)) == 1
+    return M <= 64 and _lib.wstream_narrow(M, N, K, _frag_ksplit(N, K)) == 1
 
 
 def linear_residual(x, packed, M, N, K, res, sq, sem):

@@ -788,6 +788,12 @@ def linear_fused(x, packed, N, bias=None, rstd=None, rstd_nt=0,
                              K=K, xlds=xlds, M_frag=M_frag, sem=sem)
 
 
+def narrow_pays(M, N, K) -> bool:
+    """A residual product of M rows goes in blocks of 16 columns: see
+    hip.narrow_pays."""
+    return hip.narrow_pays(M, N, K)
+
+
 def linear_residual(x, packed, M, N, K, res, sq, sem):
     """A streamed product's residual form in the fused chain: res += x @ W^T,
     and its sums of squares for the next product's rstd; returns how many of

@@ -1,4 +1,4 @@
-"""Products of up to 32 rows in blocks of 16 columns: residual and sums of squares,
+"""Products of up to 64 rows in blocks of 16 columns: residual and sums of squares,
 rotation and append.
 
 Tolerance: sums of up to K products of bf16 values in fp32, whose error is below
@@ -15,15 +15,15 @@ pytestmark = pytest.mark.gpu
 
 def _rows(flat, M, W):
     """Rows of an activation in fragment layout."""
-    t = flat.view(W // 16, 2, 32, 8)                 # 16 and 8 of W, row
-    return t.permute(2, 0, 1, 3).reshape(32, W)[:M]
+    t = flat.view(-1, W // 16, 2, 32, 8)             # 32 rows, 16 and 8 of W
+    return t.permute(0, 3, 1, 2, 4).reshape(-1, W)[:M]
 
 
 # waves without a step, with one, with four and more than four; halves of a wave's
 # rows
 @pytest.mark.parametrize("N,K", [(32, 64), (96, 512), (64, 64 * 37),
                                  (2048, 2048), (32, 64 * 71)])
-@pytest.mark.parametrize("M", [1, 7, 16, 17, 31, 32])
+@pytest.mark.parametrize("M", [1, 7, 16, 17, 32, 33, 48, 49, 64])
 def test_residual(M, N, K):
     from ollamamq_amd.ops import hip
     hip.require()
@@ -53,7 +53,7 @@ def test_residual_refused():
     hip.require()
     t = torch.zeros(64 * 64, device="cuda", dtype=torch.bfloat16)
     p = hip._p(t)
-    for M, N, K, res in ((0, 32, 64, p), (33, 32, 64, p), (1, 16, 64, p),
+    for M, N, K, res in ((0, 32, 64, p), (65, 32, 64, p), (1, 16, 64, p),
                          (1, 48, 64, p), (1, 32, 32, p), (1, 32, 64, None)):
         assert hip._lib.wstream_narrow_bf16(p, p, p, M, N, K, res, p,
                                             hip._stream())

@@ -66,9 +66,11 @@ def test_none():
     (1, 4096, 4096, 2, 1), (32, 4096, 4096, 2, 1),      # 9.8 7.2, 10.6 9.7
     (8, 4096, 14336, 2, 1), (24, 4096, 14336, 2, 0),    # 22.8 21.3, 23.9 25.9
     (8, 3584, 18944, 2, 1), (16, 3584, 18944, 2, 0),    # 26.0 25.7, 26.6 28.5
-    (16, 2048, 5632, 4, 0), (32, 2048, 2048, 2, 1),     # 7.0 5.9
+    (32, 2048, 5632, 4, 0), (32, 2048, 2048, 2, 1),     # 9.6 11.8, 7.0 5.9
     (1, 4608, 1024, 1, 0), (16, 4096, 1024, 1, 1),      # 5.1 5.4, 5.2 4.4
-    (33, 4096, 4096, 2, 0),
+    (48, 4096, 4096, 2, 1), (64, 2048, 2048, 2, 1),     # 13.9 12.3, 9.1 8.4
+    (48, 2048, 5632, 4, 0), (64, 5120, 3584, 2, 0),     # 11.9 13.9, 20.5 22.2
+    (65, 2048, 2048, 2, 0),
 ])
 def test_narrow(M, N, K, ks, narrow):
     hip.require()
