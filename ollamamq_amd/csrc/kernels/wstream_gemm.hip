@@ -1095,9 +1095,12 @@ __global__ __launch_bounds__(512, RT == 1 ? 6 : RT == 2 ? 4 : 2) void k_narrow(
 // takes; without parts where it has no more.  Over 11 numbers of columns from
 // 1024 to 8192, 11 of K from 1024 to 28672 and 1 to 32 rows the choice takes 0.6 %
 // more than the better one, parts alone 6 %, 16 columns alone 11 %; of 33 to 64
-// rows, over 4 of columns and 5 of K from 1024 to 5632, 0.6, 5 and 5 %.
+// rows, over 4 of columns from 2048 to 5120 and 5 of K from 1024 to 5632, 0.6, 5
+// and 5 %.  Fewer columns leave CUs without a block, and from 49 rows on tiles in
+// parts do not.
 static bool narrow_pays(int M, int N, int K, int ksplit)
 {
+    if (M > 48 && N < 2048) return false;
     const int rows = (M + 7) / 8 * 8;
     auto busiest = [](int blocks) { return (int64_t)((blocks + 255) / 256); };
     const int64_t more = busiest(N / 16) * K * (32 + 2 * rows)

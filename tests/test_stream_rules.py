@@ -70,7 +70,7 @@ def test_none():
     (1, 4608, 1024, 1, 0), (16, 4096, 1024, 1, 1),      # 5.1 5.4, 5.2 4.4
     (48, 4096, 4096, 2, 1), (64, 2048, 2048, 2, 1),     # 13.9 12.3, 9.1 8.4
     (48, 2048, 5632, 4, 0), (64, 5120, 3584, 2, 0),     # 11.9 13.9, 20.5 22.2
-    (65, 2048, 2048, 2, 0),
+    (65, 2048, 2048, 2, 0), (49, 1024, 1024, 1, 0), (48, 1024, 1024, 1, 1),
 ])
 def test_narrow(M, N, K, ks, narrow):
     hip.require()
