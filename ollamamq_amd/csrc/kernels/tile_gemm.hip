@@ -1036,6 +1036,30 @@ double estimate(int M, int N, int K, int hm, int hn, int ks, int cus)
     return ks > 1 ? t + 3.0 + (double)ks * M * N * 1.5e-6 : t;
 }
 
+bool takes(int K, int epi, int hm, int hn)
+{
+    return K % (32 * tile_stages(hm, hn)) == 0 && !(epi == ROPE && hn % 2);
+}
+
+struct Choice { int hm, hn, ks; double us; };
+
+Choice choose(int M, int N, int K, int epi, int cus)
+{
+    Choice best{0, 0, 0, INFINITY};
+    for (const auto& [hm, hn] : TILES) {
+        if (!takes(K, epi, hm, hn)) continue;
+        const int unit = 32 * tile_stages(hm, hn);
+        const int64_t tiles =
+            (int64_t)div_up(M, 32 * hm) * div_up(N, 32 * hn);
+        for (int ks = 1; ks <= (epi == RESIDUAL ? 8 : 1); ks++) {
+            if (ks > 1 && (tiles * ks > 2.5 * cus || K / unit < 2 * ks)) break;
+            const double t = estimate(M, N, K, hm, hn, ks, cus);
+            if (t < best.us) best = {hm, hn, ks, t};
+        }
+    }
+    return best;
+}
+
 }  // namespace
 
 // The tiles of a product and its parts, hm | hn << 8 | ks << 16: those that the
@@ -1062,20 +1086,46 @@ extern "C" int tile_gemm_plan(int M, int N, int K, int epi, int cus)
         const int parts = std::min({cus / div_up(N, 64), K / 1536, 8});
         return plan(2, 2, epi == RESIDUAL ? std::max(1, parts) : 1);
     }
-    int best = -110;
-    double least = INFINITY;
+    const Choice c = choose(M, N, K, epi, cus);
+    return c.hm ? plan(c.hm, c.hn, c.ks) : -110;
+}
+
+// A gated or rotated product of several rounds of tiles in two: as many of its
+// rows as fill whole rounds of one size of tile, and the others over tiles of
+// their own.  In one a last round takes as long whatever it has (2310 rows of
+// 28672 x 4096 over 7 x 7 tiles: 5.5 rounds, 429 us; 1792 rows, four rounds, and
+// 518 over 9 x 7, one: 399).  us in one and in two:
+//                    rows   1000       1600       2310       3000       4500
+//   28672 x 4096          189 182    284 271    429 399    522 502    746 726
+//   37888 x 3584          244 233               495 474               913 883
+//   22016 x 4096                     237 225               406 395    618 589
+// A second launch takes 9 us by the estimate's measure: over 37 random numbers of
+// rows and four matrices, those of 9 us and 1 % less take 4 % less on average, the
+// others between 3 % more and 3 % less.
+// Rows of the first | its tile << 24 | the others' tile << 40, each hm | hn << 8,
+// or 0 for one launch.
+extern "C" int64_t tile_gemm_split(int M, int N, int K, int epi, int cus)
+{
+    if (M <= 128 || N < 32 || K < 128 || K % 128 || cus < 8
+        || (epi != GATED && epi != ROPE))
+        return 0;
+    const Choice one = choose(M, N, K, epi, cus);
+    double least = one.us / 1.01 - 9.0;
+    int64_t best = 0;
     for (const auto& [hm, hn] : TILES) {
-        const int unit = 32 * tile_stages(hm, hn);
-        if (K % unit || (epi == ROPE && hn % 2)) continue;
-        const int64_t tiles =
-            (int64_t)div_up(M, 32 * hm) * div_up(N, 32 * hn);
-        for (int ks = 1; ks <= (epi == RESIDUAL ? 8 : 1); ks++) {
-            if (ks > 1 && (tiles * ks > 2.5 * cus || K / unit < 2 * ks)) break;
-            const double t = estimate(M, N, K, hm, hn, ks, cus);
-            if (t < least) {
-                least = t;
-                best = plan(hm, hn, ks);
-            }
+        if (hm * hn < 40) break;               // no rounds of small tiles
+        if (!takes(K, epi, hm, hn)) continue;
+        const int columns = div_up(N, 32 * hn);
+        for (int rows = 32 * hm, n = columns; rows < M;
+             rows += 32 * hm, n += columns) {
+            if (n < 0.92 * div_up(n, cus) * cus) continue;
+            const double t = estimate(rows, N, K, hm, hn, 1, cus);
+            if (t >= least) break;
+            const Choice rest = choose(M - rows, N, K, epi, cus);
+            if (t + rest.us >= least) continue;
+            least = t + rest.us;
+            best = rows | (int64_t)(hm | hn << 8) << 24
+                   | (int64_t)(rest.hm | rest.hn << 8) << 40;
         }
     }
     return best;

@@ -72,6 +72,8 @@ def _try_load():
     lib.tile_gemm_bf16.argtypes = [*[vp] * 8, i, f, f, *[i] * 11, *[vp] * 7,
                                    i, i, i, i, vp]
     lib.tile_gemm_plan.argtypes = [i, i, i, i, i]
+    lib.tile_gemm_split.argtypes = [i, i, i, i, i]
+    lib.tile_gemm_split.restype = i64
     lib.tile_rope_parts_bf16.argtypes = [
         *[vp] * 6, i, f, f, *[i] * 8, *[vp] * 7, i, i, i, i, vp]
     lib.tile_rows_bf16.argtypes = [*[vp] * 4, *[i] * 10, vp]
@@ -688,6 +690,20 @@ def tile_plan(M, N, K, epi, cus=256):
     return plan & 255, plan >> 8 & 255, plan >> 16
 
 
+@functools.lru_cache(maxsize=4096)
+def tile_plans(M, N, K, epi, cus=256):
+    """[(first row, rows, tiles as tile_plan has them)] of the launches that a
+    gated or rotated product takes: one, or two where a last round of tiles
+    would be half empty."""
+    require()
+    two = _lib.tile_gemm_split(M, N, K, epi, cus)
+    if not two:
+        return [(0, M, tile_plan(M, N, K, epi, cus))]
+    rows = two & (1 << 24) - 1
+    return [(at, n, (two >> to & 255, two >> to + 8 & 255, 1))
+            for at, n, to in ((0, rows, 24), (rows, M - rows, 40))]
+
+
 def tiles_take(M, N, K):
     """The products over tiles take M rows of x [M, K] and W [N, K]."""
     return N % 64 == 0 and K % 128 == 0 and (M + 31) * max(N, K) < 2 ** 31
@@ -701,14 +717,21 @@ def streams_at_once(N, device):
 
 def _tile_gemm(epi, y, x, packed, M, N, K, plan, part=None, bias=None,
                res=None, sq=None, rstd=None, rstd_nt=0, inv_h=0.0, eps=0.0,
-               gelu=0, rope=(None,) * 7 + (0,) * 4):
+               gelu=0, rope=(None,) * 7 + (0,) * 4, at=0):
+    """M rows from row `at` on (a multiple of 32), of y too."""
     hm, hn, ks = plan
     if rstd_nt > 1:
         part = torch.empty(M, dtype=torch.float32, device=x.device)
-    assert x.numel() >= -(-M // 32) * 32 * K and packed.numel() == N * K
+    assert x.numel() >= (at + -(-M // 32) * 32) * K and packed.numel() == N * K
+    yp, xp, rp = _p(y), _p(x), _p(rstd)
+    if at:
+        cols = N // 2 if epi == TILE_GATED else N
+        yp, xp, rp = yp + at * cols * 2, xp + at * K * 2, rp + at * rstd_nt * 4
+        if epi == TILE_ROPE:
+            rope = (*rope[:2], rope[2] + at * 4, rope[3] + at * 4, *rope[4:])
     _check(_lib.tile_gemm_bf16(
-        _p(y), _p(part), _p(x), _p(packed), _p(bias), _p(res), _p(sq),
-        _p(rstd), rstd_nt, float(inv_h), float(eps), M, N, K, epi, hm, hn, ks,
+        yp, _p(part), xp, _p(packed), _p(bias), _p(res), _p(sq),
+        rp, rstd_nt, float(inv_h), float(eps), M, N, K, epi, hm, hn, ks,
         8, TILE_FOLD, gelu, _cus(x.device.index), *rope, _stream()),
         "tile_gemm")
 
@@ -724,10 +747,11 @@ def tile_gu(x, packed, M, N, K, rstd, rstd_nt, inv_h, eps, glu="silu",
     normed rows of x."""
     act = torch.empty(-(-M // 32) * 32 * (N // 2), dtype=x.dtype,
                       device=x.device)
-    _tile_gemm(TILE_GATED, act, x, packed, M, N, K,
-               plan or tile_plan(M, N, K, TILE_GATED, _cus(x.device.index)),
-               rstd=rstd,
-               rstd_nt=rstd_nt, inv_h=inv_h, eps=eps, gelu=GELU[glu])
+    for at, rows, tiles in [(0, M, plan)] if plan else tile_plans(
+            M, N, K, TILE_GATED, _cus(x.device.index)):
+        _tile_gemm(TILE_GATED, act, x, packed, rows, N, K, tiles, rstd=rstd,
+                   rstd_nt=rstd_nt, inv_h=inv_h, eps=eps, gelu=GELU[glu],
+                   at=at)
     return act
 
 
@@ -753,12 +777,13 @@ def tile_qkv_rope(x, packed, M, N, K, bias_rp, cache, layer, positions,
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
     kp, vp = _layer_ptrs(cache, layer)
     pos32, slot32 = _i32(positions), _i32(slots)
-    _tile_gemm(TILE_ROPE, y, x, packed, M, N, K,
-               plan or tile_plan(M, N, K, TILE_ROPE, _cus(x.device.index)),
-               bias=bias_rp, rstd=rstd, rstd_nt=rstd_nt, inv_h=inv_h, eps=eps,
-               rope=(_p(cos), _p(sin), _p(pos32), _p(slot32),
-                     _p(cache.page_table), kp, vp, nl, nkl, cache.page_size,
-                     cache.page_table.shape[1]))
+    for at, rows, tiles in [(0, M, plan)] if plan else tile_plans(
+            M, N, K, TILE_ROPE, _cus(x.device.index)):
+        _tile_gemm(TILE_ROPE, y, x, packed, rows, N, K, tiles, bias=bias_rp,
+                   rstd=rstd, rstd_nt=rstd_nt, inv_h=inv_h, eps=eps,
+                   rope=(_p(cos), _p(sin), _p(pos32), _p(slot32),
+                         _p(cache.page_table), kp, vp, nl, nkl,
+                         cache.page_size, cache.page_table.shape[1]), at=at)
     return y
 
 
@@ -814,12 +839,16 @@ def tile_qkv_parts(x, packed, M, N, K, bias_rp, cache, layer, positions,
     return y
 
 
-def _tile_rows(epi, y, x, packed, N, plan, part=None, gelu=0):
+def _tile_rows(epi, y, x, packed, N, plan, part=None, gelu=0, at=0, rows=None):
+    """Gated: `rows` from row `at` on (a multiple of 32), of y too."""
     hm, hn, ks = plan
     assert x.buf.numel() >= -(-x.rows // 32) * 32 * x.cols \
         and packed.numel() == N * x.cols
+    yp, xp = _p(y), _p(x.buf)
+    if at:
+        yp, xp = yp + at * (N // 2) * 2, xp + at * x.cols * 2
     _check(_lib.tile_rows_bf16(
-        _p(y), _p(part), _p(x.buf), _p(packed), x.rows, N, x.cols, epi, hm,
+        yp, _p(part), xp, _p(packed), rows or x.rows, N, x.cols, epi, hm,
         hn, ks, 8, gelu, _cus(x.buf.device.index), _stream()), "tile_rows")
 
 
@@ -844,9 +873,10 @@ def tile_linear(x, packed, N, most=1, f32=False, plan=None):
 def tile_act(x, packed, N, glu="silu", plan=None):
     """tile_gu of rows that are normed already."""
     act = _frag_rows(x.rows, N // 2, x.buf)
-    _tile_rows(TILE_GATED, act.buf, x, packed, N, plan or tile_plan(
-        x.rows, N, x.cols, TILE_GATED, _cus(x.buf.device.index)),
-        gelu=GELU[glu])
+    for at, rows, tiles in [(0, x.rows, plan)] if plan else tile_plans(
+            x.rows, N, x.cols, TILE_GATED, _cus(x.buf.device.index)):
+        _tile_rows(TILE_GATED, act.buf, x, packed, N, tiles, gelu=GELU[glu],
+                   at=at, rows=rows)
     return act
 
 
