@@ -911,7 +911,7 @@ static int wide(int cw, void* y, const void* x, const void* wp, int M, int N,
 // parts of K, and adding those up (stores through to memory, a ticket, loads
 // back) takes 2.4 us at the end of each.  Half as wide, 256 blocks load the same
 // weights without parts; but each loads all rows, so the more rows, the less it
-// is worth (narrow_pays).  us in parts and here, with residual and sums:
+// is worth (wstream_residual).  us in parts and here, with residual and sums:
 //               rows     1            8           16           24           32
 //   4096 x 4096      9.8  7.2     9.9  7.2    10.0  7.7    10.4  8.5    10.6  9.7
 //   3584 x 3584      8.9  6.4     8.6  6.4     8.8  6.9     9.4  8.1     9.9  9.2
@@ -1089,32 +1089,6 @@ __global__ __launch_bounds__(512, RT == 1 ? 6 : RT == 2 ? 4 : 2) void k_narrow(
         dst[(sec & 3) * 32 + n0] = __float2bfloat16(lo_v);
 }
 
-// Whether a product that would go in `ksplit` parts goes in blocks of 16 columns:
-// where the busiest of 256 CUs has at most 256 KB more to load, rows counted by
-// the eight of a cache line, which it does in the time that adding up the parts
-// takes; without parts where it has no more.  Over 11 numbers of columns from
-// 1024 to 8192, 11 of K from 1024 to 28672 and 1 to 32 rows the choice takes 0.6 %
-// more than the better one, parts alone 6 %, 16 columns alone 11 %; of 33 to 64
-// rows, over 4 of columns from 2048 to 5120 and 5 of K from 1024 to 5632, 0.6, 5
-// and 5 %.  Fewer columns leave CUs without a block, and from 49 rows on tiles in
-// parts do not.
-static bool narrow_pays(int M, int N, int K, int ksplit)
-{
-    if (M > 48 && N < 2048) return false;
-    const int rows = (M + 7) / 8 * 8;
-    auto busiest = [](int blocks) { return (int64_t)((blocks + 255) / 256); };
-    const int64_t more = busiest(N / 16) * K * (32 + 2 * rows)
-                         - busiest(N / 32 * ksplit) * (K / ksplit)
-                               * (64 + 2 * rows);
-    return M <= 64 && more <= (ksplit > 1 ? 256 << 10 : 0);
-}
-
-extern "C" int wstream_narrow(int M, int N, int K, int ksplit)
-{
-    return M < 1 || N < 32 || K < 64 || ksplit < 1
-               ? -104 : narrow_pays(M, N, K, ksplit);
-}
-
 // y = x W^T + res_in, both in fragment layout (they may be one); sq_parts: N / 16
 // sums of squares a row
 extern "C" int wstream_narrow_bf16(
@@ -1131,6 +1105,238 @@ extern "C" int wstream_narrow_bf16(
         (bf16*)y, (const u32x4*)x, (const u32x4*)wp, nullptr, M, N, K, nullptr,
         0, 0.f, 0.f, (const bf16*)res_in, (float*)sq_parts, RopeEpi{});
     return (int)hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Blocks of 64 columns in parts of K, a wave two tiles of 32, for long K and 17 to
+// 48 rows in fragment layout.  A block of k_wstream_gemm loads all rows of its K for
+// 32 columns, with 48 rows 1.5 bytes of them for a byte of weights; here half, in
+// twice as many parts, whose sums take longer to meet.  us, with residual and sums:
+//               rows     16           24           32           45
+//   4096 x 14336     21.9 22.7    22.7 22.7    24.3 23.1    28.4 25.8
+//   3584 x 18944     26.9 25.9    27.2 26.0    29.7 26.8    35.2 30.6
+//   4096 x 11008     18.9 19.5    19.7 19.7    20.5 20.1    24.4 22.3
+//   5120 x 13824     34.9 27.2    35.4 26.0    38.5 26.8    48.0 30.1
+//   8192 x 28672     72.5 75.5    75.0 74.7    80.7 75.3    93.4 81.6
+// (117 MB in 23.1 us are 5.1 TB/s; two, three and four steps ahead are alike.)  From
+// 49 rows on tiles are as fast.
+template <int MT>
+__global__ __launch_bounds__(512, 1) void k_duo(
+    bf16* y, float* __restrict__ part, const u32x4* __restrict__ x,
+    const u32x4* __restrict__ wp, int M, int N, int K, int ksplit,
+    const bf16* res_in, float* __restrict__ sq_parts, int* __restrict__ sem)
+{
+    constexpr int D = MT == 1 ? 3 : 2;        // steps of 64 under way
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int t = blockIdx.x, ks = blockIdx.y;
+    const int NB = K >> 6, GW = ksplit * 8, gw = ks * 8 + wid;
+    const int lo = gw * NB / GW, hi = (gw + 1) * NB / GW;
+    const int last = max(hi - 1, lo);
+    typedef __attribute__((address_space(1))) const char* Global;
+    const Global wq = (Global)(wp + (int64_t)t * 2 * NB * 256), xq = (Global)x;
+    const int64_t next = (int64_t)NB * 4096;          // the second tile
+    const uint64_t lw = lane * 16u;
+    uint64_t lx[MT];
+    #pragma unroll
+    for (int m = 0; m < MT; m++)
+        lx[m] = (uint64_t)m * K * 64 + (lane & 32) * 16u
+                + min(lane & 31, max(M - m * 32, 1) - 1) * 16u;
+    u4bf8 w[D][2][4], xr[D][MT][4];
+    f32x16 acc[2][MT] = {};
+    auto step = [](Global p, int64_t at) {
+        Global q = p + at;
+        asm("" : "+s"(q));                    // no address per lane
+        return q;
+    };
+    auto load = [&](int s, int b) {
+        const Global p = step(xq, (int64_t)b * 4096);
+        #pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const Global q = step(wq, (int64_t)b * 4096 + c * next);
+            #pragma unroll
+            for (int j = 0; j < 4; j++)
+                w[s][c][j].u = __builtin_nontemporal_load(
+                    (const u32x4*)(q + lw + j * 1024));
+        }
+        #pragma unroll
+        for (int m = 0; m < MT; m++)
+            #pragma unroll
+            for (int j = 0; j < 4; j++)
+                xr[s][m][j].u = *(const u32x4*)(p + lx[m] + j * 1024);
+    };
+    auto mul = [&](int s) {
+        #pragma unroll
+        for (int j = 0; j < 4; j++)
+            #pragma unroll
+            for (int m = 0; m < MT; m++)
+                #pragma unroll
+                for (int c = 0; c < 2; c++)
+                    acc[c][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        xr[s][m][j].v, w[s][c][j].v, acc[c][m], 0, 0, 0);
+    };
+    #pragma unroll
+    for (int s = 0; s < D; s++) load(s, min(lo + s, last));
+    int b = lo;
+    for (; b + 2 * D <= hi; b += D)
+        #pragma unroll
+        for (int s = 0; s < D; s++) {
+            mul(s);
+            load(s, b + s + D);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    #pragma unroll
+    for (int s = 0; s < D; s++) {
+        if (b + s < hi) mul(s);
+        if (b + s + D < hi) load(s, b + s + D);
+    }
+    #pragma unroll
+    for (int s = 0; s < D - 1; s++)
+        if (b + s + D < hi) mul(s);
+
+    // 32 rows of 64 columns at a time: a thread has four columns of one row
+    extern __shared__ __align__(16) char smem[];
+    float (*red)[32][64] = reinterpret_cast<float (*)[32][64]>(smem);
+    const int row = tid >> 4, col = (tid & 15) * 4;
+    f32x4 v[MT];
+    #pragma unroll
+    for (int m = 0; m < MT; m++) {
+        if (m) __syncthreads();
+        #pragma unroll
+        for (int c = 0; c < 2; c++)
+            #pragma unroll
+            for (int r = 0; r < 16; r++)
+                red[wid][(r & 3) + 8 * (r >> 2) + 4 * (lane >> 5)]
+                   [c * 32 + (lane & 31)] = acc[c][m][r];
+        __syncthreads();
+        v[m] = f32x4{};
+        #pragma unroll
+        for (int u = 0; u < 8; u++)
+            v[m] += *reinterpret_cast<const f32x4*>(&red[u][row][col]);
+    }
+    const int tiles = gridDim.x;
+    if (ksplit > 1) {
+        // The block that arrives last adds up the parts, in their order, as in
+        // k_wstream_gemm: written through, read past the caches.
+        #pragma unroll
+        for (int m = 0; m < MT; m++) {
+            float* p = part + (((int64_t)ks * tiles + t) * MT + m) * 2048 + tid * 4;
+            #pragma unroll
+            for (int e = 0; e < 4; e += 2) {
+                const uint64_t u = (uint64_t)__float_as_uint(v[m][e + 1]) << 32
+                                   | __float_as_uint(v[m][e]);
+                __hip_atomic_store(reinterpret_cast<uint64_t*>(p + e), u,
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        int* drawn = reinterpret_cast<int*>(smem);
+        if (tid == 0)
+            *drawn = __hip_atomic_fetch_add(sem + t, 1, __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (*drawn != ksplit - 1) return;
+        if (tid == 0)
+            __hip_atomic_store(sem + t, 0, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        #pragma unroll
+        for (int m = 0; m < MT; m++) v[m] = f32x4{};
+        for (int k = 0; k < ksplit; k += 4) {
+            uint64_t u[4][MT][2];
+            #pragma unroll
+            for (int q = 0; q < 4; q++)
+                #pragma unroll
+                for (int m = 0; m < MT; m++)
+                    #pragma unroll
+                    for (int e = 0; e < 2; e++)
+                        u[q][m][e] = __hip_atomic_load(
+                            reinterpret_cast<const uint64_t*>(
+                                part + (((int64_t)min(k + q, ksplit - 1) * tiles
+                                         + t) * MT + m) * 2048 + tid * 4) + e,
+                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            #pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (k + q < ksplit)
+                    #pragma unroll
+                    for (int m = 0; m < MT; m++)
+                        #pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            v[m][e] += __uint_as_float(
+                                (unsigned)(u[q][m][e >> 1] >> 32 * (e & 1)));
+        }
+    }
+    #pragma unroll
+    for (int m = 0; m < MT; m++) {
+        const int at = m * 32 + row;
+        const int64_t o = frag_row_off(at, t * 64 + col, N);
+        float s = 0.f;
+        if (at < M) {
+            const bf16x4 r = *reinterpret_cast<const bf16x4*>(res_in + o);
+            bf16x4 q;
+            #pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float f = v[m][e] + (float)r[e];
+                q[e] = (__bf16)f;
+                s += f * f;
+            }
+            *reinterpret_cast<bf16x4*>(y + o) = q;
+        }
+        #pragma unroll
+        for (int o = 8; o; o >>= 1) s += __shfl_xor(s, o, 64);
+        if ((tid & 15) == 0 && at < M) sq_parts[(int64_t)at * tiles + t] = s;
+    }
+}
+
+// y = x W^T + res_in, both in fragment layout (they may be one), in `ksplit` parts
+// of K; part: as many times the floats of N columns of whole row tiles; sem: zeros,
+// one per 64 columns, zero again at the end; sq_parts: N / 64 sums of squares a row
+extern "C" int wstream_duo_bf16(
+    void* y, void* part, const void* x, const void* wp, int M, int N, int K,
+    int ksplit, const void* res_in, void* sq_parts, void* sem,
+    hipStream_t stream)
+{
+    if (M < 1 || M > 64 || N < 64 || N % 64 || K < 64 || K % 64 || ksplit < 1
+        || !res_in || !sq_parts || (ksplit > 1 && (!part || !sem)))
+        return -104;
+    constexpr int lds = 8 * 32 * 64 * 4;
+    auto go = M <= 32 ? k_duo<1> : k_duo<2>;
+    const hipError_t e = hipFuncSetAttribute(
+        (const void*)go, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return (int)e;
+    go<<<dim3(N / 64, ksplit), 512, lds, stream>>>(
+        (bf16*)y, (float*)part, (const u32x4*)x, (const u32x4*)wp, M, N, K,
+        ksplit, (const bf16*)res_in, (float*)sq_parts, (int*)sem);
+    return (int)hipGetLastError();
+}
+
+// How a residual product of few rows goes: 0 streamed in `ksplit` parts, 1 in
+// blocks of 16 columns, or in blocks of 64 in as many parts as are returned, two
+// or more.  What has least to load on the busiest of 256 CUs, rows counted by the
+// eight of a cache line, where adding up parts takes the time of 256 KB, of 64
+// columns 400 KB.  Over 11 numbers of columns from 1024 to 8192, 11 of K from
+// 1024 to 28672 and 1 to 32 rows the choice of the first two takes 0.6 % more than
+// the better one, parts alone 6 %, 16 columns alone 11 %; of 33 to 64 rows, over
+// 4 of columns from 2048 to 5120 and 5 of K from 1024 to 5632, 0.6, 5 and 5 %.
+// From 49 rows on tiles in parts are the other way: they use CUs that fewer than
+// 2048 columns leave without a block, and are no slower than 64 columns.
+extern "C" int wstream_residual(int M, int N, int K, int ksplit)
+{
+    if (M < 1 || N < 32 || N % 32 || K < 64 || K % 64 || ksplit < 1) return -104;
+    if (M > 64 || (M > 48 && N < 2048)) return 0;
+    const int rows = (M + 7) / 8 * 8;
+    // bytes: of a column's, and all rows'
+    auto load = [&](int columns, int parts) {
+        const int64_t blocks = N / columns * parts;
+        return (blocks + 255) / 256 * (K / parts) * 2 * (columns + rows);
+    };
+    const int64_t whole = load(16, 1);
+    const int64_t parts = load(32, ksplit) + (ksplit > 1 ? 256 << 10 : 0);
+    int64_t least = std::min(whole, parts);
+    int best = whole <= parts;
+    const int ks = N % 64 ? 0 : std::min(256 / (N / 64), K / 512);
+    if (M <= 48 && ks > 1 && load(64, ks) + (400 << 10) < least) best = ks;
+    return best;
 }
 
 // Iterations ahead for 32 rows in fragment layout: four where every wave has whole

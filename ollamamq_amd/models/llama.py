@@ -512,11 +512,11 @@ class LlamaModel:
         # of one round some take less time in parts
         qkv_parts = ops.rope_parts(B, self.layers[0].wqkv.shape[0], H, dev) \
             if tiles and not qkv_tiles else None
-        # a switch that asks for parts means the streams'; blocks of 16 columns
-        # are before tiles where they pay
+        # a switch that asks for parts means the streams', and some go in blocks
+        # of 16 columns
         def over_tiles(K):
             return (tiles and ops.asked_parts(K) is None
-                    and not ops.narrow_pays(B, H, K))
+                    and not ops.residual_parts(B, H, K))
         o_tiles = over_tiles(nl * d)
         down_tiles = over_tiles(self.layers[0].wdown.shape[1])
         for li, layer in enumerate(self.layers):

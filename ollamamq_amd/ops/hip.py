@@ -62,7 +62,9 @@ def _try_load():
     lib.set_entries.argtypes = [vp, i64, vp, vp, i, vp]
     lib.wstream_gemm_bf16.argtypes = [vp, vp, vp, vp, vp, i, i, i, i64, i,
                                       i, i, vp, i, f, f, vp, vp, i, vp, vp]
-    lib.wstream_narrow.argtypes = [i, i, i, i]
+    lib.wstream_residual.argtypes = [i, i, i, i]
+    lib.wstream_duo_bf16.argtypes = [vp, vp, vp, vp, i, i, i, i, vp, vp, vp,
+                                     vp]
     lib.wstream_narrow_bf16.argtypes = [vp, vp, vp, i, i, i, vp, vp, vp]
     lib.wstream_wide_tiles.argtypes = [i, i, i, i]
     lib.wstream_depth.argtypes = [i, i, i, i]
@@ -1002,24 +1004,34 @@ def linear_packed(x, packed, bias, N, ks=None, depth=None, xlds=None,
 
 
 @functools.lru_cache(maxsize=4096)
-def narrow_pays(M, N, K):
-    """Whether a residual product of M rows goes in blocks of 16 columns."""
-    return M <= 64 and _lib.wstream_narrow(M, N, K, _frag_ksplit(N, K)) == 1
+def residual_parts(M, N, K):
+    """How a residual product of M rows is streamed: 0 by linear_packed, 1 in
+    blocks of 16 columns, else in blocks of 64 in so many parts of K."""
+    return _lib.wstream_residual(M, N, K, _frag_ksplit(N, K))
 
 
 def linear_residual(x, packed, M, N, K, res, sq, sem):
     """res += x @ W^T, x and res in fragment layout; sq gets sums of squares of
     the result, m-major, and has room for N / 16 a row.  Returns how many there
     are.  sem: see linear_packed."""
-    if asked_parts(K) is None and narrow_pays(M, N, K):
+    ks = residual_parts(M, N, K) if asked_parts(K) is None else 0
+    if ks == 0:
+        linear_packed(x, packed, None, N, res=res, sq_out=sq, y=res, yfrag=1,
+                      K=K, xlds=2, M_frag=M, sem=sem)
+        return N // 32
+    if ks == 1:
         assert sq.numel() >= M * (N // 16)
         _check(_lib.wstream_narrow_bf16(
             _p(res), _p(x), _p(packed), M, N, K, _p(res), _p(sq), _stream()),
             "wstream_narrow")
         return N // 16
-    linear_packed(x, packed, None, N, res=res, sq_out=sq, y=res, yfrag=1, K=K,
-                  xlds=2, M_frag=M, sem=sem)
-    return N // 32
+    assert sq.numel() >= M * (N // 64) and sem.numel() >= N // 64
+    part = torch.empty(ks * -(-M // 32) * 32 * N, dtype=torch.float32,
+                       device=x.device)
+    _check(_lib.wstream_duo_bf16(
+        _p(res), _p(part), _p(x), _p(packed), M, N, K, ks, _p(res), _p(sq),
+        _p(sem), _stream()), "wstream_duo")
+    return N // 64
 
 
 def fragify_sumsq(x, sq=None, tokens=None, rows=None, add=None, clear=None):

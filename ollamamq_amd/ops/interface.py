@@ -788,10 +788,9 @@ def linear_fused(x, packed, N, bias=None, rstd=None, rstd_nt=0,
                              K=K, xlds=xlds, M_frag=M_frag, sem=sem)
 
 
-def narrow_pays(M, N, K) -> bool:
-    """A residual product of M rows goes in blocks of 16 columns: see
-    hip.narrow_pays."""
-    return hip.narrow_pays(M, N, K)
+def residual_parts(M, N, K) -> int:
+    """How a residual product of M rows is streamed: see hip.residual_parts."""
+    return hip.residual_parts(M, N, K)
 
 
 def linear_residual(x, packed, M, N, K, res, sq, sem):

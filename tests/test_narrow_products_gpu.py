@@ -1,5 +1,5 @@
-"""Products of up to 64 rows in blocks of 16 columns: residual and sums of squares,
-rotation and append.
+"""Products of up to 64 rows in blocks of 16 columns, or of 64 in parts of K:
+residual and sums of squares, rotation and append.
 
 Tolerance: sums of up to K products of bf16 values in fp32, whose error is below
 K 2^-24 of the sum of magnitudes, then one rounding to bf16 (2^-9 of the value,
@@ -10,6 +10,8 @@ twice.
 import pytest
 import torch
 
+from ollamamq_amd.ops import hip
+
 pytestmark = pytest.mark.gpu
 
 
@@ -19,13 +21,37 @@ def _rows(flat, M, W):
     return t.permute(0, 3, 1, 2, 4).reshape(-1, W)[:M]
 
 
-# waves without a step, with one, with four and more than four; halves of a wave's
-# rows
-@pytest.mark.parametrize("N,K", [(32, 64), (96, 512), (64, 64 * 37),
-                                 (2048, 2048), (32, 64 * 71)])
+def _residual(ks, x, w, r):
+    """x w^T + r and its sums of squares a row, in blocks of 16 columns or in ks
+    parts of 64; what is beside them stays as it is."""
+    (M, K), N = x.shape, len(w)
+    xf, rf = (hip.fragify_sumsq(t)[0] for t in (x, r))
+    packed, n = hip.pack_weight(w), M * N // (64 if ks else 16)
+    sq = torch.full((n + 64,), 7.0, device="cuda")
+    if ks:
+        rows = -(-M // 32) * 32
+        part = torch.full((ks * rows * N + 64,), 7.0, device="cuda")
+        sem = torch.zeros(N // 64 + 1, dtype=torch.int32, device="cuda")
+        hip._check(hip._lib.wstream_duo_bf16(
+            hip._p(rf), hip._p(part), hip._p(xf), hip._p(packed), M, N, K, ks,
+            hip._p(rf), hip._p(sq), hip._p(sem), hip._stream()), "duo")
+        assert not sem.any() and (part[ks * rows * N:] == 7).all()
+    else:
+        hip._check(hip._lib.wstream_narrow_bf16(
+            hip._p(rf), hip._p(xf), hip._p(packed), M, N, K, hip._p(rf),
+            hip._p(sq), hip._stream()), "narrow")
+    assert (sq[n:] == 7).all()
+    return _rows(rf, M, N), sq[:n].view(M, -1).double().sum(1)
+
+
+# waves without a step, with one, with whole rounds of those under way and with
+# more; halves of a wave's rows
+@pytest.mark.parametrize("ks,N,K", [
+    (0, 32, 64), (0, 96, 512), (0, 64, 64 * 37), (0, 2048, 2048),
+    (0, 32, 64 * 71), (1, 64, 64), (1, 128, 64 * 61), (2, 64, 1024),
+    (3, 192, 64 * 71), (4, 256, 64 * 225), (5, 64, 64 * 83), (9, 128, 64 * 80)])
 @pytest.mark.parametrize("M", [1, 7, 16, 17, 32, 33, 48, 49, 64])
-def test_residual(M, N, K):
-    from ollamamq_amd.ops import hip
+def test_residual(M, ks, N, K):
     hip.require()
     g = torch.Generator(device="cuda").manual_seed(M * N + K)
 
@@ -33,23 +59,16 @@ def test_residual(M, N, K):
         return torch.randn(shape, generator=g, device="cuda").bfloat16()
 
     x, w, r = rand(M, K), rand(N, K), rand(M, N)
-    xf, rf = (hip.fragify_sumsq(t)[0] for t in (x, r))
-    sq = torch.full((M * N // 16 + 64,), 7.0, device="cuda")
-    hip._check(hip._lib.wstream_narrow_bf16(
-        hip._p(rf), hip._p(xf), hip._p(hip.pack_weight(w)), M, N, K,
-        hip._p(rf), hip._p(sq), hip._stream()), "wstream_narrow")
+    got, sums = _residual(ks, x, w, r)
     want = x.double() @ w.double().T + r.double()
     size = x.double().abs() @ w.double().abs().T + r.double().abs()
-    err = (_rows(rf, M, N).double() - want).abs()
+    err = (got.double() - want).abs()
     assert (err <= 2 ** -8 * want.abs() + K * 2 ** -24 * size).all()
-    sums = sq[:M * N // 16].view(M, -1).double().sum(1)
     torch.testing.assert_close(sums, want.square().sum(1), rtol=K * 2 ** -22,
                                atol=0)
-    assert (sq[M * N // 16:] == 7).all()
 
 
-def test_residual_refused():
-    from ollamamq_amd.ops import hip
+def test_refused():
     hip.require()
     t = torch.zeros(64 * 64, device="cuda", dtype=torch.bfloat16)
     p = hip._p(t)
@@ -57,6 +76,14 @@ def test_residual_refused():
                          (1, 48, 64, p), (1, 32, 32, p), (1, 32, 64, None)):
         assert hip._lib.wstream_narrow_bf16(p, p, p, M, N, K, res, p,
                                             hip._stream())
+    for M, N, K, ks, part, res, sem in (
+            (0, 64, 64, 1, p, p, p), (65, 64, 64, 1, p, p, p),
+            (1, 32, 64, 1, p, p, p), (1, 96, 64, 1, p, p, p),
+            (1, 64, 96, 1, p, p, p), (1, 64, 64, 0, p, p, p),
+            (1, 64, 1024, 2, None, p, p), (1, 64, 1024, 2, p, None, p),
+            (1, 64, 1024, 2, p, p, None)):
+        assert hip._lib.wstream_duo_bf16(p, part, p, p, M, N, K, ks, res, p,
+                                         sem, hip._stream())
 
 
 # more than 256 tiles of 32 columns: up to 16 rows in blocks of 16, above in
@@ -65,7 +92,6 @@ def test_residual_refused():
 @pytest.mark.parametrize("M", [1, 9, 16])
 def test_rotated(M, nl, nkl, bias):
     from ollamamq_amd.engine import PagedKVCache
-    from ollamamq_amd.ops import hip
     hip.require()
     g = torch.Generator(device="cuda").manual_seed(M)
     N, K, T = (nl + 2 * nkl) * 128, 64 * 11, 17

@@ -61,17 +61,24 @@ def test_none():
         assert hip._lib.wstream_depth(*bad) < 0
 
 
-@pytest.mark.parametrize("M,N,K,ks,narrow", [
-    # us in parts and in blocks of 16 columns
+@pytest.mark.parametrize("M,N,K,ks,how", [
+    # us in parts and in blocks of 16 columns ...
     (1, 4096, 4096, 2, 1), (32, 4096, 4096, 2, 1),      # 9.8 7.2, 10.6 9.7
-    (8, 4096, 14336, 2, 1), (24, 4096, 14336, 2, 0),    # 22.8 21.3, 23.9 25.9
-    (8, 3584, 18944, 2, 1), (16, 3584, 18944, 2, 0),    # 26.0 25.7, 26.6 28.5
+    (8, 4096, 14336, 2, 1),                             # 22.8 21.3
+    (8, 3584, 18944, 2, 1),                             # 26.0 25.7
     (32, 2048, 5632, 4, 0), (32, 2048, 2048, 2, 1),     # 9.6 11.8, 7.0 5.9
     (1, 4608, 1024, 1, 0), (16, 4096, 1024, 1, 1),      # 5.1 5.4, 5.2 4.4
     (48, 4096, 4096, 2, 1), (64, 2048, 2048, 2, 1),     # 13.9 12.3, 9.1 8.4
     (48, 2048, 5632, 4, 0), (64, 5120, 3584, 2, 0),     # 11.9 13.9, 20.5 22.2
     (65, 2048, 2048, 2, 0), (49, 1024, 1024, 1, 0), (48, 1024, 1024, 1, 1),
+    # ... and of 64
+    (32, 4096, 14336, 2, 4), (45, 4096, 14336, 2, 4),   # 24.3 23.1, 28.4 25.8
+    (16, 3584, 18944, 2, 4), (45, 3584, 18944, 2, 4),   # 26.9 25.9, 35.2 30.6
+    (1, 5120, 13824, 2, 3), (45, 4096, 11008, 2, 4),    # 33.9 27.2, 24.4 22.3
+    (8, 8192, 28672, 1, 0), (32, 8192, 28672, 1, 2),    # 75.9 77.8, 80.7 75.3
+    (32, 2048, 8192, 4, 0), (49, 4096, 14336, 2, 0),    # 11.5 11.7
+    (32, 4128, 14336, 2, 0),
 ])
-def test_narrow(M, N, K, ks, narrow):
+def test_residual(M, N, K, ks, how):
     hip.require()
-    assert hip._lib.wstream_narrow(M, N, K, ks) == narrow
+    assert hip._lib.wstream_residual(M, N, K, ks) == how
