@@ -7,27 +7,34 @@
 // 16-wide matrix tile, so a byte is read once for all of them.
 //
 // Every wave walks its own steps of 32 keys with its own maximum and sum, and
-// nothing passes through LDS before the one merge at the end:
-//  * a key row is the row operand of mfma_16x16x32 as it lies in memory;
-//  * values are loaded as whole rows (four of them per instruction) and
-//    turned in registers: a lane holds columns 8c..8c+7 of the eight keys
-//    whose weights it holds, and 32 byte permutes make of them the operands
-//    of eight value tiles (tile v has the columns 8c + v);
-//  * both are requested a step ahead, 16 KB in flight per wave.
+// nothing is shared before the one merge at the end:
+//  * keys and values go straight to LDS of the wave's own, a step ahead, 16 KB
+//    under way per wave, in whole rows, four of them an instruction.  A key row is
+//    the row operand of mfma_16x16x32; loaded to registers in that form, 16 lanes
+//    touch 16 lines for 16 bytes each;
+//  * values are read as they were loaded and turned in registers: a lane holds
+//    columns 8c..8c+7 of the eight keys whose weights it holds, and 32 byte
+//    permutes make of them the operands of eight value tiles (tile v has the
+//    columns 8c + v);
+//  * page numbers are looked up for many steps at once, a lane each.
 // Weights stay fp32: they enter the product with the values as three bf16
 // terms, which hold all 24 bits.
 //
-// Bound by memory: 5.2 TB/s over large caches, where a device copy makes 4.7.
-// Before, keys and values went through LDS for products on the vector units,
-// one head a wave (32 heads, 8 of them key/value heads, unless said):
-//   32 users, 256 to 768 tokens                34.2 us, now 17.5
-//   128 users, 350 to 1050                      131 us, now 70
-//   12 users, 4096 to 12288                     144 us, now 83
-//   45 users, 300 to 900, 28 / 4 heads           46 us, now 18.5
-//   20 users, 550 to 1650, 32 / 32 heads        282 us, now 69
-// Loading values through wave-private LDS tiles instead is no faster and
-// costs 70 KB of LDS; non-temporal loads gain 2 us at 128 users and lose as
-// much at 45.
+// Bound by memory: 4.9 to 5.3 TB/s over large caches, where a device copy makes
+// 4.7; the loads alone take 1 to 2 % less.  us, with keys and values loaded to
+// registers in operand order, and so (32 heads, 8 of them key/value heads, unless
+// said):
+//   one user, 300 tokens                        7.4, now 6.4
+//   32 users, 256 to 768                       18.1, now 17.3
+//   128 users, 350 to 1050                     72.2, now 71.1
+//   12 users, 4096 to 12288                    86.2, now 82.6
+//   24 users, 1000 to 3000                     47.7, now 45.0
+//   48 users, 300 to 900, 28 / 4 heads         19.0, now 18.1
+//   24 users, 550 to 1650, 32 / 32 heads       81.1, now 81
+//   24 users, 1000 to 3000, pages of 24 tokens  54.7, now 48.4
+// A wave's steps one after the other and heads dealt to the XCDs in turn are 1 to
+// 3 % slower; whole lines of 8 rows an instruction, put right in registers, no
+// faster than operand order.
 #pragma once
 #include "flash32.h"
 
@@ -47,13 +54,13 @@ DEV float2 get2(const float* p) {
 
 // Pages: with SH they are 1 << pshift tokens and no smaller than a tile of
 // 16 keys, so a tile's page number is the same for the whole wave; otherwise
-// any number of tokens, looked up key by key.
-// s: DECODE_LDS bytes
-constexpr int DECODE_LDS = 8 * 8 * (128 + 2) * 4;
+// any number of tokens, and every key has its own.
+// smem: DECODE_LDS bytes
+constexpr int DECODE_LDS = 8 * 2 * 32 * 128 * 2;
 
 template <bool SH>
 DEV void decode_block(
-    float* s, int kvh, int seq, int z, int split, int least,
+    char* smem, int kvh, int seq, int z, int split, int least,
     bf16* __restrict__ out,               // [S, Hq, D] (split == 1)
     float* __restrict__ o_part,           // [S, Hq, split, D]
     float* __restrict__ ml_part,          // [S, Hq, split, 2] maximum, sum
@@ -71,82 +78,118 @@ DEV void decode_block(
     const int Hq = G * KVH;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, lr = lane & 15, g = lane >> 4;
-    const int kv_len = seq_lens[seq], last = kv_len - 1;
-    const int* pt = page_table + (int64_t)slot_ids[seq] * max_pages;
+    int kv_len = seq_lens[seq], slot = slot_ids[seq];
+    asm volatile("" : "+s"(kv_len), "+s"(slot));      // asked for together
+    const int last = kv_len - 1;
+    const int* pt = page_table + (int64_t)slot * max_pages;
     // first key that the query, at kv_len - 1, sees
     const int lo = window > 0 ? max(0, kv_len - window) : 0;
     const int first = lo / KT, steps = (kv_len + KT - 1) / KT - first;
-    // parts in use: each has `least` steps, at least one a wave (300 tokens of
-    // one user: 7.3 us in one part, 8.2 in two)
+    // parts in use: each has `least` steps, at least one a wave (two parts cost
+    // 300 tokens of one user 0.9 us)
     const int parts = max(1, min(split, steps / least));
     if (z >= parts) return;
     const int GW = parts * NW;            // a wave's steps: every GW-th
 
-    float* o_s = s;                       // [NW * 8][D]
-    float* ml_s = s + NW * 8 * D;         // [NW * 8][2]
+    // a wave's own: 32 keys and values, in the end its G results, maxima and sums
+    constexpr int OWN = KT * D;           // floats
+    float* o_s = reinterpret_cast<float*>(smem);
+    char* keys = smem + wid * OWN * 4;
+    char* values = keys + KT * D * 2;
 
-    bf16x8 qf[4], kf[2][4];
-    u32x4 vr[8];
+    bf16x8 qf[4];
     const bf16* qr = q + seq * qs + (kvh * G + min(lr, G - 1)) * D + g * 8;
     #pragma unroll
     for (int d = 0; d < 4; d++) qf[d] = frag8(qr + d * 32);
 
-    // SH: pages of a step's tiles, looked up a step before they are needed
-    int pg[2], next[2];
-    auto pages = [&](int st) {
-        #pragma unroll
-        for (int t = 0; SH && t < 2; t++) {
-            pg[t] = next[t];
-            next[t] = pt[min((first + st) * KT + t * 16, last) >> pshift];
+    int st = z * NW + wid;
+    // the key of instruction e; past the last the last again, with no weight
+    auto key_of = [&](int st, int e) {
+        return min((first + st) * KT + e * 4 + g, last);
+    };
+    // Pages are looked up for many of a wave's steps at once, one a lane: of a
+    // step's two tiles, or as many as its keys can lie in.
+    const int per = SH ? 2 : (KT - 1) / page + 2, many = 64 / per;
+    int book = 0, pg[SH ? 2 : 8];
+    auto pages = [&](int st, int j) {
+        if (j == 0) {
+            const int b = lane / per, p = lane - b * per;
+            const int key = (first + st + b * GW) * KT;
+            book = pt[SH ? min(key + p * 16, last) >> pshift
+                         : min(min(key, last) / page + p, last / page)];
+            asm volatile("" : "+v"(book));    // waited for here alone
         }
+        #pragma unroll
+        for (int t = 0; SH && t < 2; t++)
+            pg[t] = __builtin_amdgcn_readlane(book, j * 2 + t);
+        #pragma unroll
+        for (int e = 0; !SH && e < 8; e++)
+            pg[e] = __shfl(book, j * per + key_of(st, e) / page
+                                     - (first + st) * KT / page, 64);
     };
-    // row of a key within one of the pools
-    auto row = [&](const bf16* pool, int t, int key) {
-        if (SH)
-            return pool + (((int64_t)pg[t] * KVH + kvh) << pshift) * D
-                   + (key & ((1 << pshift) - 1)) * D;
-        return pool + (((int64_t)pt[key / page] * KVH + kvh) * page
-                       + key % page) * D;
+    auto to_lds = [&](const bf16* pool, int st, int e, int piece, char* to) {
+        const int key = key_of(st, e);
+        const bf16* row = SH
+            ? pool + (((int64_t)pg[e >> 2] * KVH + kvh) << pshift) * D
+                  + (key & ((1 << pshift) - 1)) * D
+            : pool + (((int64_t)pg[e] * KVH + kvh) * page + key % page) * D;
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) void*)(row + piece * 8),
+            (__attribute__((address_space(3))) void*)(to + e * 1024), 16, 0, 0);
     };
-    // keys past the last are the last again, with a weight of zero
+    // The loads of keys and of values take turns and their waits count them, so
+    // none may pass another; and a buffer has been read before it is loaded again.
+    auto in_order = [] {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
     auto load_k = [&](int st) {
+        in_order();
+        // pieces of 16 bytes where 16 rows are read without bank conflicts
         #pragma unroll
-        for (int t = 0; t < 2; t++) {
-            const int key = min((first + st) * KT + t * 16 + lr, last);
-            const bf16* r = row(kpool, t, key) + g * 8;
-            #pragma unroll
-            for (int d = 0; d < 4; d++) kf[t][d] = frag8(r + d * 32);
-        }
+        for (int e = 0; e < 8; e++)
+            to_lds(kpool, st, e, lr ^ ((e & 3) * 4 + g), keys);
+        in_order();
+    };
+    auto key_at = [&](int t, int d) {
+        return *reinterpret_cast<const bf16x8*>(
+            keys + t * 4096 + lr * 256 + ((d * 4 + g) ^ lr) * 16);
     };
     auto load_v = [&](int st) {
+        in_order();
         #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const int key = min((first + st) * KT + (e >> 2) * 16 + g * 4
-                                + (e & 3), last);
-            vr[e] = *reinterpret_cast<const u32x4*>(
-                row(vpool, e >> 2, key) + lr * 8);
-        }
+        for (int e = 0; e < 8; e++) to_lds(vpool, st, e, lr, values);
+        in_order();
     };
+    // all but the last n loads have come
+    #define ARRIVED(n)                                                     \
+        do {                                                               \
+            __builtin_amdgcn_sched_barrier(0);                             \
+            asm volatile("s_waitcnt vmcnt(" #n ")" ::: "memory");          \
+            __builtin_amdgcn_sched_barrier(0);                             \
+        } while (0)
 
     float m = NEG, l = 0.f;
     f32x4 acc[8] = {};
-    int st = z * NW + wid;
     if (st < steps) {
-        pages(st);
-        pages(st + GW);
+        pages(st, 0);
+        // what the loop takes from registers is there before its loads
+        #pragma unroll
+        for (int d = 0; d < 4; d++) asm volatile("" : "+v"(qf[d]));
         load_k(st);
         load_v(st);
     }
-    for (; st < steps; st += GW) {
+    for (int j = 1 % many; st < steps; st += GW, j = j + 1 < many ? j + 1 : 0) {
         const bool more = st + GW < steps;
+        ARRIVED(8);                // keys
         f32x4 s[2] = {};           // scores
         #pragma unroll
         for (int d = 0; d < 4; d++) {
-            s[0] = mma(kf[0][d], qf[d], s[0]);
-            s[1] = mma(kf[1][d], qf[d], s[1]);
+            s[0] = mma(key_at(0, d), qf[d], s[0]);
+            s[1] = mma(key_at(1, d), qf[d], s[1]);
         }
         if (more) {
-            pages(st + 2 * GW);
+            pages(st + GW, j);
             load_k(st + GW);
         }
         // scores of the keys base + 16 j + 4 g + i for head lr
@@ -182,6 +225,13 @@ DEV void decode_block(
         l = l * f + sum;                  // of this lane's keys only
         #pragma unroll
         for (int v = 0; v < 8; v++) acc[v] *= f;
+        if (more) ARRIVED(8);
+        else ARRIVED(0);
+        u32x4 vr[8];
+        #pragma unroll
+        for (int e = 0; e < 8; e++)
+            vr[e] = *reinterpret_cast<const u32x4*>(
+                values + ((e >> 2) * 16 + g * 4 + (e & 3)) * 256 + lr * 16);
         #pragma unroll
         for (int v = 0; v < 8; v++) {
             u32x4 a;
@@ -197,6 +247,7 @@ DEV void decode_block(
         }
         if (more) load_v(st + GW);
     }
+    #undef ARRIVED
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
 
@@ -205,13 +256,13 @@ DEV void decode_block(
         #pragma unroll
         for (int i = 0; i < 4; i++) {
             f32x4* d = reinterpret_cast<f32x4*>(
-                o_s + (wid * G + lr) * D + (g * 4 + i) * 8);
+                o_s + wid * OWN + lr * D + (g * 4 + i) * 8);
             d[0] = f32x4{acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
             d[1] = f32x4{acc[4][i], acc[5][i], acc[6][i], acc[7][i]};
         }
         if (g == 0) {
-            ml_s[(wid * G + lr) * 2] = m;
-            ml_s[(wid * G + lr) * 2 + 1] = l;
+            o_s[wid * OWN + 8 * D + lr * 2] = m;
+            o_s[wid * OWN + 8 * D + lr * 2 + 1] = l;
         }
     }
     __syncthreads();
@@ -220,13 +271,15 @@ DEV void decode_block(
     const int c = (threadIdx.x % (D / 4)) * 4, hq = kvh * G + h;
     float top = NEG, den = 0.f;
     #pragma unroll
-    for (int w = 0; w < NW; w++) top = fmaxf(top, ml_s[(w * G + h) * 2]);
+    for (int w = 0; w < NW; w++)
+        top = fmaxf(top, o_s[w * OWN + 8 * D + h * 2]);
     f32x4 sum = {};
     #pragma unroll
     for (int w = 0; w < NW; w++) {
-        const float f = __builtin_amdgcn_exp2f(ml_s[(w * G + h) * 2] - top);
-        den += f * ml_s[(w * G + h) * 2 + 1];
-        sum += f * *reinterpret_cast<const f32x4*>(o_s + (w * G + h) * D + c);
+        const float* ml = o_s + w * OWN + 8 * D + h * 2;
+        const float f = __builtin_amdgcn_exp2f(ml[0] - top);
+        den += f * ml[1];
+        sum += f * *reinterpret_cast<const f32x4*>(o_s + w * OWN + h * D + c);
     }
     if (parts > 1) {
         // The block that arrives last merges the parts, in their order.  They

@@ -12,7 +12,7 @@ __global__ __launch_bounds__(512, 2) void k_decode_attn(
     int64_t qs, int window, int fragout, int least)
 {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    decode_block<SH>(reinterpret_cast<float*>(smem), blockIdx.x, blockIdx.y,
+    decode_block<SH>(smem, blockIdx.x, blockIdx.y,
                      blockIdx.z, gridDim.z, least, out, o_part, ml_part, sem, q,
                      kpool, vpool, page_table, slot_ids, seq_lens, G, KVH,
                      page, pshift, max_pages, unit, qs, window, fragout);
@@ -35,6 +35,9 @@ extern "C" int decode_attn_bf16(
     const bool sh = page >= 16 && !(page & (page - 1));
     const float unit = scale * 1.4426950408889634f;
     auto go = sh ? k_decode_attn<true> : k_decode_attn<false>;
+    const hipError_t ok = hipFuncSetAttribute(
+        (const void*)go, hipFuncAttributeMaxDynamicSharedMemorySize, DECODE_LDS);
+    if (ok != hipSuccess) return (int)ok;
     go<<<dim3(KVH, S, split), 512, DECODE_LDS, stream>>>(
         (bf16*)out, (float*)part, (float*)part + (int64_t)S * Hq * split * 128,
         (int*)sem, (const bf16*)q, (const bf16*)kpool, (const bf16*)vpool,

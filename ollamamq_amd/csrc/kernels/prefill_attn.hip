@@ -124,7 +124,7 @@ __global__ __launch_bounds__(512, 2) void k_mixed_attn(
                              kpool, vpool, page_table, G, KVH, page, pshift,
                              max_pages, unit, qs, window, fragout);
     else
-        decode_block<SH>(reinterpret_cast<float*>(smem), blockIdx.x, b % S,
+        decode_block<SH>(smem, blockIdx.x, b % S,
                          b / S, split, least, out, o_part, ml_part, sem, q,
                          kpool, vpool, page_table, slot_ids, seq_lens, G, KVH,
                          page, pshift, max_pages, unit, qs, window, fragout);

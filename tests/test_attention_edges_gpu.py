@@ -99,6 +99,22 @@ def test_decode(heads, kv_heads, page, window):
                        got.flatten(1))
 
 
+@pytest.mark.parametrize("page,window", [(16, 0), (64, 0), (5, 0), (24, 0),
+                                         (33, 0), (16, 8225), (24, 8225)])
+def test_decode_long_walks(page, window, monkeypatch):
+    """More steps a wave than it looks up pages for at once, and as many."""
+    hip = _hip()
+    lens = [8160, 8192, 8193, 8225, 16385, 16640]
+    cache, slots = _cache(lens, 2, page, 9)
+    monkeypatch.setenv("OLLAMAMQ_DECODE_SPLIT", "1")
+    q = torch.randn(len(lens), 8, D, device="cuda").bfloat16()
+    ones = [1] * len(lens)
+    want = _exact(q, cache, 1, slots, lens, ones, window)
+    got = hip.attention_decode(q, cache, 1,
+                               _meta(slots, lens, ones, window, "decode"))
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=1e-5)
+
+
 @pytest.mark.parametrize("split", [1, 2, 3, 32])
 def test_decode_parts(split, monkeypatch):
     """Any number of parts, some of them without keys, and queries that lie
