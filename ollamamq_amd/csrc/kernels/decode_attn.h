@@ -61,6 +61,7 @@ constexpr int DECODE_LDS = 8 * 2 * 32 * 128 * 2;
 template <bool SH>
 DEV void decode_block(
     char* smem, int kvh, int seq, int z, int split, int least,
+    int S, int cus,
     bf16* __restrict__ out,               // [S, Hq, D] (split == 1)
     float* __restrict__ o_part,           // [S, Hq, split, D]
     float* __restrict__ ml_part,          // [S, Hq, split, 2] maximum, sum
@@ -79,14 +80,37 @@ DEV void decode_block(
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, lr = lane & 15, g = lane >> 4;
     int kv_len = seq_lens[seq], slot = slot_ids[seq];
-    asm volatile("" : "+s"(kv_len), "+s"(slot));      // asked for together
+    int other = split > 1 && cus ? seq_lens[min(lane, S - 1)] : 0;
+    // asked for together
+    asm volatile("" : "+s"(kv_len), "+s"(slot), "+v"(other));
     const int last = kv_len - 1;
     const int* pt = page_table + (int64_t)slot * max_pages;
     // first key that the query, at kv_len - 1, sees
     const int lo = window > 0 ? max(0, kv_len - window) : 0;
     const int first = lo / KT, steps = (kv_len + KT - 1) / KT - first;
-    // parts in use: each has `least` steps, at least one a wave (two parts cost
-    // 300 tokens of one user 0.9 us)
+    // Parts in use: each has `least` steps, at least one a wave (two parts cost
+    // 300 tokens of one user 0.9 us).  With cus, an even share, for a block a CU,
+    // of what all sequences have: short contexts stay whole, where parts of 8
+    // steps made up to 768 blocks with as many ends, and long ones take no longer
+    // than the rest.  us with 8 steps and so (ragged, key/value heads): 12 users of
+    // 800 tokens, 8 heads 16.8, 14.1; 16 of 1500 27.7, 24.7; 20 of 600 18.4, 15.0;
+    // 45 of 600, 4 heads 20.3, 16.2; 5 of 1000, 32 heads 23.9, 20.1.  Shares of 36
+    // and more end too far apart: 12 of 8192 took 88 us for 82.  Finding the share
+    // takes 0.4 us, so contexts of less than two parts and of 100 steps and more,
+    // whose share is seldom less than that, go without.
+    if (z > 0 && z >= steps / least) return;
+    if (split > 1 && cus && steps >= 2 * least && steps < 100) {
+        auto steps_of = [&](int n) {
+            return (n + KT - 1) / KT - (window > 0 ? max(0, n - window) / KT : 0);
+        };
+        int all = lane < S ? steps_of(other) : 0;
+        for (int i = lane + 64; i < S; i += 64) all += steps_of(seq_lens[i]);
+        #pragma unroll
+        for (int d = 32; d; d >>= 1) all += __shfl_xor(all, d, 64);
+        all = __builtin_amdgcn_readfirstlane(all);
+        const int share = (all * KVH + cus - 1) / cus;
+        if (share < 36) least = max(least, share);
+    }
     const int parts = max(1, min(split, steps / least));
     if (z >= parts) return;
     const int GW = parts * NW;            // a wave's steps: every GW-th

@@ -114,8 +114,8 @@ __global__ __launch_bounds__(512, 2) void k_mixed_attn(
     const bf16* __restrict__ vpool, const int* __restrict__ page_table,
     const Item* __restrict__ items, int n_items,
     const int* __restrict__ slot_ids, const int* __restrict__ seq_lens,
-    int S, int split, int least, int G, int KVH, int page, int pshift,
-    int max_pages, float unit, int64_t qs, int window, int fragout)
+    int S, int split, int least, int cus, int G, int KVH, int page,
+    int pshift, int max_pages, float unit, int64_t qs, int window, int fragout)
 {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int b = blockIdx.y - n_items;
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(512, 2) void k_mixed_attn(
                              max_pages, unit, qs, window, fragout);
     else
         decode_block<SH>(smem, blockIdx.x, b % S,
-                         b / S, split, least, out, o_part, ml_part, sem, q,
+                         b / S, split, least, S, cus, out, o_part, ml_part, sem, q,
                          kpool, vpool, page_table, slot_ids, seq_lens, G, KVH,
                          page, pshift, max_pages, unit, qs, window, fragout);
 }
@@ -180,13 +180,13 @@ extern "C" int mixed_attn_bf16(
     void* out, void* part, void* sem, const void* q, const void* kpool,
     const void* vpool, const void* page_table, const void* items, int n_items,
     const void* slot_ids, const void* seq_lens, int S, int split, int least,
-    int Hq, int KVH, int page, int max_pages, float scale, int64_t q_stride,
+    int cus, int Hq, int KVH, int page, int max_pages, float scale, int64_t q_stride,
     int window, int fragout, hipStream_t stream)
 {
     const int G = Hq / KVH;
     if (G < 1 || G > 8 || G * KVH != Hq || page < 1 || S < 1 || n_items < 1
         || (reinterpret_cast<uintptr_t>(q) & 15) || q_stride % 8
-        || split < 1 || least < 8 || (split > 1 && (!part || !sem)))
+        || split < 1 || least < 8 || cus < 0 || (split > 1 && (!part || !sem)))
         return (int)hipErrorInvalidValue;
     const bool sh = page >= 16 && !(page & (page - 1));
     constexpr int flash = Flash32<D, D, 8, false>::LDS;
@@ -199,7 +199,7 @@ extern "C" int mixed_attn_bf16(
         (bf16*)out, (float*)part, (float*)part + (int64_t)S * Hq * split * D,
         (int*)sem, (const bf16*)q, (const bf16*)kpool, (const bf16*)vpool,
         (const int*)page_table, (const Item*)items, n_items,
-        (const int*)slot_ids, (const int*)seq_lens, S, split, least, G, KVH,
+        (const int*)slot_ids, (const int*)seq_lens, S, split, least, cus, G, KVH,
         page, sh ? __builtin_ctz(page) : 0, max_pages,
         scale * 1.4426950408889634f, q_stride, window, fragout);
     return (int)hipGetLastError();

@@ -49,7 +49,7 @@ def _try_load():
     lib.argmax_bf16.argtypes = [vp, vp, i, i, vp, vp, i, *[vp] * 6]
     lib.argmax_f32.argtypes = lib.argmax_bf16.argtypes
     lib.decode_attn_bf16.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp,
-                                     i, i, i, i, i, f, i64, i, i, i, i, vp]
+                                     i, i, i, i, i, f, i64, i, i, i, i, i, vp]
     lib.skinny_gemm_bf16.argtypes = [vp, vp, vp, vp, i, i, i, i64, i, vp]
     lib.skinny_direct_bf16.argtypes = [vp, vp, vp, vp, i, i, i, i64, i, vp]
     lib.rope_append_bf16.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp, vp,
@@ -57,7 +57,7 @@ def _try_load():
     lib.prefill_attn_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i, i, i, i, i,
                                       i, f, i64, i, i, vp]
     lib.mixed_attn_bf16.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, i, vp, vp,
-                                    i, i, i, i, i, i, i, f, i64, i, i, vp]
+                                    i, i, i, i, i, i, i, i, f, i64, i, i, vp]
     lib.embed_gather_bf16.argtypes = [vp, vp, vp, i, i, vp]
     lib.set_entries.argtypes = [vp, i64, vp, vp, i, vp]
     lib.wstream_gemm_bf16.argtypes = [vp, vp, vp, vp, vp, i, i, i, i64, i,
@@ -342,16 +342,15 @@ def _attention(q, cache, layer, meta, qt):
 
 
 def _decode_split(pairs, max_kv):
-    """Parts of a context, for `pairs` (sequence, key/value head) pairs, each
-    of at least _decode_least steps of 32 keys.  Up to 64 pairs, a block a CU
-    in all: more parts are more to add up (4 users of 10000 tokens, 8 key/value
-    heads: 40 us in 8, 47 in 24; 8 of 2000: 18 in 4, 25 in 12).  Up to 191, 768
-    blocks even out ragged contexts (12 users of 4096 to 12288: 149 us whole,
-    91 in two, 80 in eight).  From 192 on one part is best where its blocks
-    fill whole rounds of the 256 CUs (32 users of about 512 tokens: 17 us
-    against 20 in two short ones); where they do not, long parts fill the last
-    round (34 users of 2500: 73 us against 88 whole, 24 of 4000: 82 against
-    92)."""
+    """Most parts of a context, for `pairs` (sequence, key/value head) pairs; how
+    many it takes the kernel says, from all lengths.  Up to 64 pairs, a block a CU
+    in all: more parts are more to add up (8 users of 3500 tokens, 8 key/value
+    heads: 28 us in 4, 34 in 16).  Up to 191, 768 blocks even out ragged contexts
+    (12 users of 4096 to 12288: 84 us in two, 73 in eight).  From 192 on one part
+    is best where its blocks fill whole rounds of the 256 CUs (32 users of about
+    512 tokens: 17 us against 20 in two short ones); where they do not, long parts
+    fill the last round (34 users of 2500: 73 us against 88 whole, 24 of 4000: 82
+    against 94)."""
     env = os.environ.get("OLLAMAMQ_DECODE_SPLIT")
     if env:                       # tuning override (tools/perf_decode.py)
         want = int(env)
@@ -362,14 +361,19 @@ def _decode_split(pairs, max_kv):
     return min(want, max(1, (max_kv + 255) // 256), 32)
 
 
-def _decode_least(pairs):
-    """Steps of a part: one for each of its eight waves, or so many that short
-    contexts stay whole (24, 32 and 48 tried)."""
-    return 48 if pairs >= 192 else 8
+def _decode_least(pairs, dev):
+    """(steps of 32 keys that a part has at least, CUs to share all steps by, or
+    0): one for each of its eight waves; from 192 pairs on so many that short
+    contexts stay whole (24, 32 and 48 tried).  Shares pay where the parts may be
+    more than a block a CU, so not up to 64 pairs."""
+    if pairs >= 192:
+        return 48, 0
+    return 8, _cus(dev.index) if pairs > 64 else 0
 
 
 def _decode_parts(S, Hq, kvh, meta, sem, dev):
-    """(parts of a context, steps of one, scratch, tickets, slots, lengths)"""
+    """(most parts of a context, steps of one and CUs to share by, scratch,
+    tickets, slots, lengths)"""
     split = _decode_split(S * kvh, meta.max_kv)
     part = None
     if split > 1:
@@ -378,7 +382,7 @@ def _decode_parts(S, Hq, kvh, meta, sem, dev):
         if sem is None:
             sem = torch.zeros(S * kvh, dtype=torch.int32, device=dev)
         assert sem.numel() >= S * kvh
-    return (split, _decode_least(S * kvh), part, sem, _i32(meta.slot_ids),
+    return (split, _decode_least(S * kvh, dev), part, sem, _i32(meta.slot_ids),
             _i32(meta.seq_lens))
 
 
@@ -403,13 +407,13 @@ def attention_decode(q, cache, layer, meta, fragout=False, out=None,
         q = q.clone(memory_format=torch.contiguous_format)
     kp, vp = _layer_ptrs(cache, layer)
     kvh = cache.n_kv_heads
-    split, least, part, sem, slot32, len32 = _decode_parts(
+    split, (least, cus), part, sem, slot32, len32 = _decode_parts(
         S, Hq, kvh, meta, sem, q.device)
     _check(_lib.decode_attn_bf16(
         _p(out), _p(part), _p(sem), _p(q), kp, vp, _p(cache.page_table),
         _p(slot32), _p(len32), S, Hq, kvh, cache.page_size,
         cache.page_table.shape[1], 1.0 / (D ** 0.5), _row_stride(q, D),
-        split, least, meta.window, 1 if fragout else 0, _stream()),
+        split, least, cus, meta.window, 1 if fragout else 0, _stream()),
         "decode_attn")
     return out
 
@@ -512,13 +516,14 @@ def attention_mixed(q, cache, layer, meta, fragout=False, sem=None):
         if q.data_ptr() % 16 or _row_stride(q, D) % 8:
             q = q.clone(memory_format=torch.contiguous_format)
         kp, vp = _layer_ptrs(cache, layer)
-        split, least, part, sem, slots, lens = _decode_parts(
+        split, (least, cus), part, sem, slots, lens = _decode_parts(
             nd, Hq, kvh, sub, sem, q.device)
         _check(_lib.mixed_attn_bf16(
             _p(out), _p(part), _p(sem), _p(q), kp, vp, _p(cache.page_table),
             _p(items), items.shape[0], _p(slots), _p(lens), nd, split, least,
-            Hq, kvh, cache.page_size, cache.page_table.shape[1], D ** -0.5,
-            _row_stride(q, D), meta.window, int(fragout), _stream()),
+            cus, Hq, kvh, cache.page_size,
+            cache.page_table.shape[1], D ** -0.5, _row_stride(q, D),
+            meta.window, int(fragout), _stream()),
             "mixed_attn")
     return out
 

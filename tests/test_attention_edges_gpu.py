@@ -115,6 +115,28 @@ def test_decode_long_walks(page, window, monkeypatch):
     torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=1e-5)
 
 
+@pytest.mark.parametrize("S,heads,window", [
+    (2, 2, 0), (64, 1, 0), (65, 1, 0), (129, 1, 0), (90, 2, 700), (30, 4, 0)])
+def test_decode_even_shares(S, heads, window):
+    """Parts by the lengths of all sequences, more than a wave has lanes too;
+    tickets are zero again."""
+    hip = _hip()
+    lens = [(3000, 31, 1, 256, 257, 600, 1500, 33)[i * 3 % 8]
+            for i in range(S)]
+    cache, slots = _cache(lens, heads, 16, 11)
+    assert hip._decode_split(S * heads, max(lens)) > 1
+    q = torch.randn(S, 4 * heads, D, device="cuda").bfloat16()
+    ones = [1] * S
+    want = _exact(q, cache, 1, slots, lens, ones, window)
+    sem = torch.zeros(S * heads, dtype=torch.int32, device="cuda")
+    for _ in range(2):
+        got = hip.attention_decode(
+            q, cache, 1, _meta(slots, lens, ones, window, "decode"), sem=sem)
+        torch.testing.assert_close(got.double(), want, rtol=2 ** -8,
+                                   atol=1e-5)
+        assert not sem.any()
+
+
 @pytest.mark.parametrize("split", [1, 2, 3, 32])
 def test_decode_parts(split, monkeypatch):
     """Any number of parts, some of them without keys, and queries that lie
