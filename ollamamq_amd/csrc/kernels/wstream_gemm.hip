@@ -927,8 +927,8 @@ static int wide(int cw, void* y, const void* x, const void* wp, int M, int N,
 // where a rotation pairs columns, 8 h to 8 h + 7 of both its halves.
 // Rows are asked for as far ahead as weights, as loads return in order; four
 // steps are as fast as six or eight, in registers for three blocks a CU.
-// ROPE: norm, rotation and append as k_wstream_gemm has them, else residual and
-// sums of squares.
+// ROPE: norm (none without rstd_parts), rotation and append as k_wstream_gemm has
+// them, else residual and sums of squares.
 template <int RT, bool ROPE>
 __global__ __launch_bounds__(512, RT == 1 ? 6 : RT == 2 ? 4 : 2) void k_narrow(
     bf16* y, const u32x4* __restrict__ x, const u32x4* __restrict__ wp,
@@ -998,7 +998,7 @@ __global__ __launch_bounds__(512, RT == 1 ? 6 : RT == 2 ? 4 : 2) void k_narrow(
     } else {
         // the norm's partial sums, FL lanes a row
         const int m = threadIdx.x / FL;
-        if (m < M) {
+        if (rstd_parts && m < M) {
             const float* p = rstd_parts + (int64_t)m * rstd_nt;
             int i = threadIdx.x % FL;
             for (; i + 7 * FL < rstd_nt; i += 8 * FL) {
@@ -1040,7 +1040,8 @@ __global__ __launch_bounds__(512, RT == 1 ? 6 : RT == 2 ? 4 : 2) void k_narrow(
         #pragma unroll
         for (int o = FL / 2; o; o >>= 1) rsum += __shfl_down(rsum, o, 64);
         if (threadIdx.x % FL == 0)
-            rstd_s[threadIdx.x / FL] = rsqrtf(rsum * inv_h + eps);
+            rstd_s[threadIdx.x / FL] =
+                rstd_parts ? rsqrtf(rsum * inv_h + eps) : 1.f;
     }
     __syncthreads();
     auto total = [&](int m, int n) {

@@ -128,3 +128,64 @@ def test_rotated(M, nl, nkl, bias):
         # both round sums of the same terms, of size sqrt(K) in fp32
         torch.testing.assert_close(a.float(), c.float(), rtol=2 ** -7,
                                    atol=K * 2 ** -20)
+
+
+def _halves(head, angle):
+    """A head's rotation in 64 bits."""
+    lo, hi = head.chunk(2, -1)
+    return torch.cat([lo * angle.cos() - hi * angle.sin(),
+                      hi * angle.cos() + lo * angle.sin()], -1)
+
+
+# Sums of squares come in any number: none (rows are taken as they are), and ones
+# that 32 lanes a row read in eights, in twos and singly.
+@pytest.mark.parametrize("nt", [None, 1, 31, 33, 256, 257, 300])
+@pytest.mark.parametrize("M", [1, 16, 17])
+def test_rotated_norms(M, nt):
+    from ollamamq_amd.engine import PagedKVCache
+    hip.require()
+    nl, nkl, K, page = 60, 3, 64 * 9, 16
+    N, eps = (nl + 2 * nkl) * 128, 0.0 if nt is None else 1e-5
+    assert N > 256 * 32
+    g = torch.Generator(device="cuda").manual_seed(M + (nt or 0))
+
+    def rand(*shape):
+        return torch.randn(shape, generator=g, device="cuda").bfloat16()
+
+    x, w, b = rand(M, K), rand(N, K), rand(N)
+    sq = None if nt is None else \
+        torch.rand(M, nt, generator=g, device="cuda") * 2 * K / nt
+    scale = 1.0 if nt is None else \
+        (sq.double().sum(1, keepdim=True) / K + eps).rsqrt()
+    angle = torch.rand(64, 64, generator=g, device="cuda") * 6.28
+    pos = torch.arange(M, device="cuda", dtype=torch.int32) * 3
+    cache = PagedKVCache(1, nkl, 128, page_size=page, n_pages=80, max_slots=M,
+                         max_ctx=64, device="cuda", dtype=torch.bfloat16)
+    slots = [cache.alloc_slot() for _ in range(M)]
+    for i, s in enumerate(slots):
+        cache.ensure(s, 3 * i + 1)
+    order = torch.tensor(hip.qkv_rope_order(nl, nkl), device="cuda")
+    got = hip.linear_qkv_rope(
+        hip.fragify_sumsq(x)[0], hip.pack_weight_qkv_rope(w, nl, nkl), N,
+        b[order], cache, 0, pos,
+        torch.tensor(slots, device="cuda", dtype=torch.int32), angle.cos(),
+        angle.sin(), nl, nkl, sq, nt or 0, 0.0 if nt is None else 1.0 / K,
+        eps, K=K, M_real=M)
+    at = [(cache.page_table[s, 3 * i // page].long(), 3 * i % page)
+          for i, s in enumerate(slots)]
+    got = torch.cat([got[:, :nl * 128].unflatten(1, (nl, 128)), *(
+        torch.stack([pool[0, p, :, o] for p, o in at])
+        for pool in (cache.k_pool, cache.v_pool))], 1)
+    want = (x.double() @ w.double().T * scale + b.double()) \
+        .unflatten(1, (-1, 128))
+    size = (x.double().abs() @ w.double().abs().T * scale + b.double().abs()) \
+        .unflatten(1, (-1, 128))
+    turned = nl + nkl                        # values are not
+    want[:, :turned] = _halves(want[:, :turned],
+                               angle.double()[pos.long()][:, None])
+    size[:, :turned] = size[:, :turned] + size[:, :turned].roll(64, -1)
+    # as above, and the scale: nt sums and a reciprocal root; sines and cosines
+    # are rounded to 24 bits
+    err = (got.double() - want).abs()
+    assert (err <= 2 ** -8 * want.abs()
+            + (K + (nt or 0) + 8) * 2 ** -24 * size).all()
