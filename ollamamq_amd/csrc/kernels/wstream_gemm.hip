@@ -996,17 +996,18 @@ __global__ __launch_bounds__(512, RT == 1 ? 6 : RT == 2 ? 4 : 2) void k_narrow(
                 add[i] = __bfloat162float(
                     res_in[frag_row_off(row + i * 32, n16, N)]);
     } else {
-        // the norm's partial sums, FL lanes a row
+        // the norm's partial sums, FL lanes a row; eight at a time do not fit 80
+        // registers beside the loads under way (12288 x 4096: 17.6 us, 17.5 so)
         const int m = threadIdx.x / FL;
         if (rstd_parts && m < M) {
             const float* p = rstd_parts + (int64_t)m * rstd_nt;
             int i = threadIdx.x % FL;
-            for (; i + 7 * FL < rstd_nt; i += 8 * FL) {
-                float v[8];
+            for (; i + 3 * FL < rstd_nt; i += 4 * FL) {
+                float v[4];
                 #pragma unroll
-                for (int k = 0; k < 8; k++) v[k] = p[i + k * FL];
+                for (int k = 0; k < 4; k++) v[k] = p[i + k * FL];
                 #pragma unroll
-                for (int k = 0; k < 8; k++) rsum += v[k];
+                for (int k = 0; k < 4; k++) rsum += v[k];
             }
             for (; i + FL < rstd_nt; i += 2 * FL) rsum += p[i] + p[i + FL];
             if (i < rstd_nt) rsum += p[i];

@@ -1,6 +1,8 @@
 """What a product asks of its buffers, on the host: a kernel cannot know how
 long they are."""
 import os
+import re
+import shutil
 import subprocess
 import sys
 
@@ -64,3 +66,29 @@ def test_a_kernel_has_one_limit_of_lds(tmp_path):
         limits.setdefault(kernel, set()).add(int(value))
     assert len(limits) > 15
     assert all(len(v) == 1 and max(v) <= 160 * 1024 for v in limits.values())
+
+
+LLVM = "/opt/rocm/llvm/bin"
+
+
+@pytest.mark.skipif(not os.path.exists(f"{LLVM}/llvm-readelf"),
+                    reason="needs ROCm's object tools")
+def test_narrow_blocks_keep_their_sums_in_registers(tmp_path):
+    """Three blocks a CU leave a lane of k_narrow 80 registers; what does not fit
+    would go through memory in the loop that memory bounds."""
+    if not hip.available():
+        pytest.skip("the extension is not built")
+    lib = tmp_path / "kernels.so"
+    shutil.copy(hip._lib._name, lib)
+    subprocess.run([f"{LLVM}/llvm-objdump", "--offloading", lib], check=True,
+                   capture_output=True)
+    found = 0
+    for part in tmp_path.glob("*gfx950"):
+        notes = subprocess.run([f"{LLVM}/llvm-readelf", "--notes", part],
+                               check=True, capture_output=True, text=True)
+        for kernel in notes.stdout.split("- .agpr_count:")[1:]:
+            if "k_narrow" in kernel:
+                found += 1
+                assert re.search(r"\.private_segment_fixed_size: 0\n", kernel)
+                assert re.search(r"\.vgpr_spill_count: 0\n", kernel), kernel
+    assert found >= 5
