@@ -997,7 +997,8 @@ __global__ __launch_bounds__(512, RT == 1 ? 6 : RT == 2 ? 4 : 2) void k_narrow(
                     res_in[frag_row_off(row + i * 32, n16, N)]);
     } else {
         // the norm's partial sums, FL lanes a row; eight at a time do not fit 80
-        // registers beside the loads under way (12288 x 4096: 17.6 us, 17.5 so)
+        // registers beside the loads under way (12288 x 4096, one row: 22.9 us with 12
+        // of them spilled, 17.9 so)
         const int m = threadIdx.x / FL;
         if (rstd_parts && m < M) {
             const float* p = rstd_parts + (int64_t)m * rstd_nt;
