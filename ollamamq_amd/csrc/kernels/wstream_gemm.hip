@@ -1540,6 +1540,33 @@ extern "C" int wstream_gemm_bf16(
 
 
 
+// Rotated products of up to 16 rows go in blocks of 16 columns where blocks of 32
+// are more than the 256 CUs, which leaves some of them two; where those of 16 are
+// no more than three a CU, all that fit at once; and where a wave has most of the
+// four steps that it asks for at first.  us in blocks of 32 and of 16:
+//   columns               8448       10240       12288       13312       16384
+//   x 1024,  1 row      6.9  7.7    7.2  8.0    7.4  8.2    7.5  9.6    8.0 10.1
+//           16          7.6  9.1    7.7  9.4    8.0  9.8    8.0 11.3    8.6 12.1
+//   x 1792,  1          9.9  8.8   10.4  9.2   10.9  9.8
+//           16         10.8 10.5   11.2 11.3   11.5 11.5
+//   x 2048,  1         10.9  9.4   11.3  9.6   11.6 10.2   11.9 11.6   13.1 12.6
+//           16         11.7 11.0   12.2 11.3   12.6 11.8   12.8 13.4   13.8 14.9
+//   x 4096,  1         18.8 15.6   19.7 16.6   20.3 17.5   20.8 20.5   24.0 22.5
+//           16         20.2 18.0   20.7 19.5   21.4 20.1   21.6 23.8   24.5 25.8
+//   x 8192,  1         34.5 29.1   36.4 31.0   38.4 33.7   38.9 39.5   44.9 43.2
+//           16         36.8 33.0   38.4 35.2   40.0 36.9   40.3 44.5   45.6 47.7
+// 6144 x 4096 gains nothing.
+static bool rope_narrow(int M, int N, int K)
+{
+    return M >= 1 && M <= 16 && N % 32 == 0 && N > 256 * 32 && N <= 3 * 256 * 16
+           && K >= 1792;
+}
+
+extern "C" int wstream_rope_narrow(int M, int N, int K)
+{
+    return rope_narrow(M, N, K);
+}
+
 // qkv GEMM with fused RoPE + paged KV append (fused decode chain):
 // q lands rotated in y's standard layout; k/v land in the paged pool.
 extern "C" int wstream_qkv_rope_bf16(
@@ -1557,9 +1584,7 @@ extern "C" int wstream_qkv_rope_bf16(
                nl, nkl, psz, maxp};
     const int d = frag_depth(M, N, K, 1);
     if (M > (xf ? 128 : 32)) return -104;          // rows of a block
-    // blocks of 32 columns that are more than the CUs leave some of them two (12288
-    // x 4096, 1 to 16 rows: 3.3 to 2.6 us less of 22; 6144 x 4096: none)
-    if (xf && M <= 16 && N > 256 * 32) {
+    if (xf && rope_narrow(M, N, K)) {
         k_narrow<1, true><<<N / 16, 512, 0, stream>>>(
             (bf16*)y, (const u32x4*)x, (const u32x4*)wp, (const bf16*)bias, M, N,
             K, (const float*)rstd_parts, rstd_nt, inv_h, eps, nullptr, nullptr,

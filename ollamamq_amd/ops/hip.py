@@ -63,6 +63,7 @@ def _try_load():
     lib.wstream_gemm_bf16.argtypes = [vp, vp, vp, vp, vp, i, i, i, i64, i,
                                       i, i, vp, i, f, f, vp, vp, i, vp, vp]
     lib.wstream_residual.argtypes = [i, i, i, i]
+    lib.wstream_rope_narrow.argtypes = [i, i, i]
     lib.wstream_duo_bf16.argtypes = [vp, vp, vp, vp, i, i, i, i, vp, vp, vp,
                                      vp]
     lib.wstream_narrow_bf16.argtypes = [vp, vp, vp, i, i, i, vp, vp, vp]

@@ -94,8 +94,8 @@ def test_rotated(M, nl, nkl, bias):
     from ollamamq_amd.engine import PagedKVCache
     hip.require()
     g = torch.Generator(device="cuda").manual_seed(M)
-    N, K, T = (nl + 2 * nkl) * 128, 64 * 11, 17
-    assert N > 256 * 32
+    N, K, T = (nl + 2 * nkl) * 128, 64 * 29, 17
+    assert hip._lib.wstream_rope_narrow(M, N, K)
 
     def rand(*shape):
         return torch.randn(shape, generator=g, device="cuda").bfloat16()
@@ -140,13 +140,14 @@ def _halves(head, angle):
 # Sums of squares come in any number: none (rows are taken as they are), and ones
 # that 32 lanes a row read in eights, in twos and singly.
 @pytest.mark.parametrize("nt", [None, 1, 31, 33, 256, 257, 300])
-@pytest.mark.parametrize("M", [1, 16, 17])
-def test_rotated_norms(M, nt):
+@pytest.mark.parametrize("M,K", [(1, 64 * 29), (16, 64 * 29), (5, 64 * 75),
+                                 (17, 64 * 29), (16, 64 * 9)])
+def test_rotated_norms(M, K, nt):
     from ollamamq_amd.engine import PagedKVCache
     hip.require()
-    nl, nkl, K, page = 60, 3, 64 * 9, 16
+    nl, nkl, page = 60, 3, 16
     N, eps = (nl + 2 * nkl) * 128, 0.0 if nt is None else 1e-5
-    assert N > 256 * 32
+    assert hip._lib.wstream_rope_narrow(M, N, K) == (M < 17 and K > 64 * 9)
     g = torch.Generator(device="cuda").manual_seed(M + (nt or 0))
 
     def rand(*shape):

@@ -82,3 +82,21 @@ def test_none():
 def test_residual(M, N, K, ks, how):
     hip.require()
     assert hip._lib.wstream_residual(M, N, K, ks) == how
+
+
+@pytest.mark.parametrize("M,N,K,narrow", [
+    # us in blocks of 32 columns and of 16
+    (1, 8448, 4096, True), (16, 8448, 4096, True),      # 18.8 15.6, 20.2 18.0
+    (1, 12288, 4096, True), (16, 12288, 8192, True),    # 20.3 17.5, 40.0 36.9
+    (1, 8448, 1792, True), (16, 12288, 2048, True),     # 9.9 8.8, 12.6 11.8
+    (1, 8448, 512, False), (16, 12288, 512, False),     # 4.9 7.1, 6.0 8.7
+    (1, 8448, 1024, False), (16, 12288, 1024, False),   # 6.9 7.7, 8.0 9.8
+    (16, 10240, 1536, False),                           # 10.3 10.6
+    (16, 13312, 4096, False), (8, 15360, 5120, False),  # 21.6 23.8, 26.8 28.1
+    (16, 16384, 8192, False), (8, 12416, 4096, False),  # 45.6 47.7
+    (1, 8192, 4096, False), (17, 12288, 4096, False), (0, 8448, 4096, False),
+    (1, 8464, 4096, False),                             # no whole tiles
+])
+def test_rotated(M, N, K, narrow):
+    hip.require()
+    assert hip._lib.wstream_rope_narrow(M, N, K) == narrow
