@@ -1316,29 +1316,40 @@ extern "C" int wstream_duo_bf16(
 // How a residual product of few rows goes: 0 streamed in `ksplit` parts, 1 in
 // blocks of 16 columns, or in blocks of 64 in as many parts as are returned, two
 // or more.  What has least to load on the busiest of 256 CUs, rows counted by the
-// eight of a cache line, where adding up parts takes the time of 256 KB, of 64
-// columns 400 KB.  Over 11 numbers of columns from 1024 to 8192, 11 of K from
-// 1024 to 28672 and 1 to 32 rows the choice of the first two takes 0.6 % more than
-// the better one, parts alone 6 %, 16 columns alone 11 %; of 33 to 64 rows, over
-// 4 of columns from 2048 to 5120 and 5 of K from 1024 to 5632, 0.6, 5 and 5 %.
-// From 49 rows on tiles in parts are the other way: they use CUs that fewer than
-// 2048 columns leave without a block, and are no slower than 64 columns.
+// eight of a cache line, but no less than 1.4 times its share of the weights, which
+// is what memory takes (8192 x 28672, 16 rows: 69.9 us streamed, 72.4 in blocks of
+// 64).  Adding up parts takes the time of 200 KB, of more than 32 rows 270, of
+// blocks of 64 columns 300 and 20 more for each part beyond four (512 x 18944, 48
+// rows: 15.1 us in 8 parts, 22.1 in 32 of 64 columns).  Blocks of 16 columns load
+// what K of 768 takes even if it is less (4096 x 256, 32 rows: 4.5 us streamed,
+// 5.1).  Over 12 numbers of columns from 512 to 8192, 16 of K from 128 to 28672 and
+// 8 of rows from 1 to 64 the choice takes 1.8 % more than the best of the three,
+// parts (tiles in parts from 49 rows on) alone 13 %, 16 columns alone 21 %, and at
+// most 2.7 % more than parts.
+// From 49 rows on the parts are of tiles, which take the time of 360 KB more: they
+// use CUs that fewer than 2048 columns leave without a block, and are no slower
+// than 64 columns.
 extern "C" int wstream_residual(int M, int N, int K, int ksplit)
 {
     if (M < 1 || N < 32 || N % 32 || K < 64 || K % 64 || ksplit < 1) return -104;
     if (M > 64 || (M > 48 && N < 2048)) return 0;
     const int rows = (M + 7) / 8 * 8;
     // bytes: of a column's, and all rows'
-    auto load = [&](int columns, int parts) {
+    auto load = [&](int columns, int parts, int k) {
         const int64_t blocks = N / columns * parts;
-        return (blocks + 255) / 256 * (K / parts) * 2 * (columns + rows);
+        return std::max<int64_t>(
+            (blocks + 255) / 256 * (k / parts) * 2 * (columns + rows),
+            1.4 / 128 * N * K);
     };
-    const int64_t whole = load(16, 1);
-    const int64_t parts = load(32, ksplit) + (ksplit > 1 ? 256 << 10 : 0);
+    const int sums = M > 48 ? 360 : M > 32 ? 270 : 200;
+    const int64_t whole = load(16, 1, std::max(K, 768));
+    const int64_t parts = load(32, ksplit, K) + (ksplit > 1 ? sums << 10 : 0);
     int64_t least = std::min(whole, parts);
     int best = whole <= parts;
     const int ks = N % 64 ? 0 : std::min(256 / (N / 64), K / 512);
-    if (M <= 48 && ks > 1 && load(64, ks) + (400 << 10) < least) best = ks;
+    if (M <= 48 && ks > 1
+        && load(64, ks, K) + ((300 + 20 * std::max(ks - 4, 0)) << 10) < least)
+        best = ks;
     return best;
 }
 

@@ -100,3 +100,22 @@ def test_residual(M, N, K, ks, how):
 def test_rotated(M, N, K, narrow):
     hip.require()
     assert hip._lib.wstream_rope_narrow(M, N, K) == narrow
+
+
+@pytest.mark.parametrize("M,N,K,ks,how", [
+    # where the weights' own time is what is left: us streamed and in 64 columns
+    (9, 8192, 28672, 1, 0), (16, 8192, 28672, 1, 0),    # 69.7 71.9, 69.9 72.4
+    (24, 8192, 28672, 1, 2), (16, 3584, 18944, 2, 4),   # 72.1 71.4, 24.9 25.0
+    # more parts of 64 columns are more to add up
+    (48, 512, 18944, 8, 0), (24, 512, 18944, 8, 0),     # 15.1 22.1, 11.7 15.9
+    (48, 1024, 28672, 8, 0), (45, 1536, 8960, 8, 10),   # 20.2 22.7, 17.3 15.5
+    # short K: us streamed and in 16 columns; over tiles and in 16 columns
+    (32, 4096, 256, 1, 0), (24, 1536, 128, 1, 0),       # 4.5 5.1, 4.1 4.8
+    (32, 3584, 512, 1, 0), (32, 1024, 1024, 1, 1),      # 5.0 5.8, 5.3 5.2
+    (64, 3584, 256, 1, 0), (64, 3584, 3584, 2, 1),      # 5.2 6.8, 14.1 11.0
+    # few rows: parts of few tiles
+    (1, 1536, 8960, 8, 0), (9, 2048, 5632, 4, 0),       # 10.6 10.9, 9.0 9.2
+])
+def test_residual_sizes(M, N, K, ks, how):
+    hip.require()
+    assert hip._lib.wstream_residual(M, N, K, ks) == how
