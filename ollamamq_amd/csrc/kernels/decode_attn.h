@@ -81,8 +81,9 @@ DEV void decode_block(
     const int lane = threadIdx.x & 63, lr = lane & 15, g = lane >> 4;
     int kv_len = seq_lens[seq], slot = slot_ids[seq];
     int other = split > 1 && cus ? seq_lens[min(lane, S - 1)] : 0;
-    // asked for together
-    asm volatile("" : "+s"(kv_len), "+s"(slot), "+v"(other));
+    // asked for together; scalars by themselves, or they count as a lane's own
+    asm volatile("" : "+s"(kv_len), "+s"(slot));
+    asm volatile("" : "+v"(other));
     const int last = kv_len - 1;
     const int* pt = page_table + (int64_t)slot * max_pages;
     // first key that the query, at kv_len - 1, sees
@@ -152,13 +153,26 @@ DEV void decode_block(
                                      - (first + st) * KT / page, 64);
     };
     auto to_lds = [&](const bf16* pool, int st, int e, int piece, char* to) {
-        const int key = key_of(st, e);
-        const bf16* row = SH
-            ? pool + (((int64_t)pg[e >> 2] * KVH + kvh) << pshift) * D
-                  + (key & ((1 << pshift) - 1)) * D
-            : pool + (((int64_t)pg[e] * KVH + kvh) * page + key % page) * D;
+        typedef __attribute__((address_space(1))) const char* Global;
+        Global from;
+        if (SH) {
+            // A tile of 16 keys lies in one page: an address of the wave's and
+            // 32 bits a lane (64 bits a lane, many users of 150 to 600 tokens:
+            // 2 % slower).  One past the last key takes the last's tile.
+            const int at = (first + st) * KT + (e >> 2) * 16;
+            const int tile = min(at, last & ~15);
+            from = (Global)(pool + ((((int64_t)pg[e >> 2] * KVH + kvh) << pshift)
+                                    + (tile & ((1 << pshift) - 1))) * D);
+            asm("" : "+s"(from));
+            const unsigned row = min((e & 3) * 4 + g + at - tile, last - tile);
+            from += row * 256u + piece * 16u;
+        } else {
+            const int key = key_of(st, e);
+            from = (Global)(pool + (((int64_t)pg[e] * KVH + kvh) * page
+                                    + key % page) * D + piece * 8);
+        }
         __builtin_amdgcn_global_load_lds(
-            (const __attribute__((address_space(1))) void*)(row + piece * 8),
+            (const __attribute__((address_space(1))) void*)from,
             (__attribute__((address_space(3))) void*)(to + e * 1024), 16, 0, 0);
     };
     // The loads of keys and of values take turns and their waits count them, so
@@ -196,14 +210,20 @@ DEV void decode_block(
     float m = NEG, l = 0.f;
     f32x4 acc[8] = {};
     if (st < steps) {
-        pages(st, 0);
+        if (SH) {
+            // the first step's pages as scalars: a short context has no others
+            #pragma unroll
+            for (int t = 0; t < 2; t++)
+                pg[t] = pt[min((first + st) * KT + t * 16, last) >> pshift];
+        } else
+            pages(st, 0);
         // what the loop takes from registers is there before its loads
         #pragma unroll
         for (int d = 0; d < 4; d++) asm volatile("" : "+v"(qf[d]));
         load_k(st);
         load_v(st);
     }
-    for (int j = 1 % many; st < steps; st += GW, j = j + 1 < many ? j + 1 : 0) {
+    for (int j = SH ? 0 : 1 % many; st < steps; st += GW, j = j + 1 < many ? j + 1 : 0) {
         const bool more = st + GW < steps;
         ARRIVED(8);                // keys
         f32x4 s[2] = {};           // scores

@@ -137,6 +137,29 @@ def test_decode_even_shares(S, heads, window):
         assert not sem.any()
 
 
+@pytest.mark.parametrize("page", [16, 32, 64, 256, 8, 24])
+@pytest.mark.parametrize("window", [0, 20])
+def test_decode_reads_no_row_past_the_end(page, window):
+    """What lies behind a context, in its last page and in others, is not a
+    number; contexts end in every part of a step."""
+    hip = _hip()
+    lens = [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 250, 257, 300]
+    cache, slots = _cache(lens, 2, page, 13)
+    for pool in (cache.k_pool, cache.v_pool):
+        held = pool[1].clone()
+        pool.fill_(float("nan"))
+        for slot, n in zip(slots, lens):
+            for at in range(0, n, page):
+                p, m = cache.page_table[slot, at // page].long(), n - at
+                pool[1, p, :, :m] = held[p, :, :m]
+    q = torch.randn(len(lens), 8, D, device="cuda").bfloat16()
+    ones = [1] * len(lens)
+    want = _exact(q, cache, 1, slots, lens, ones, window)
+    got = hip.attention_decode(q, cache, 1,
+                               _meta(slots, lens, ones, window, "decode"))
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=1e-5)
+
+
 @pytest.mark.parametrize("split", [1, 2, 3, 32])
 def test_decode_parts(split, monkeypatch):
     """Any number of parts, some of them without keys, and queries that lie
