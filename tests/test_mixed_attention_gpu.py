@@ -126,3 +126,47 @@ def test_long_parts_of_many_users(S, KVH, window):
         # one rounding to bf16, and fp32 sums
         torch.testing.assert_close(got[i].double(), want.flatten(0, 1),
                                    rtol=2 ** -8, atol=1e-5)
+
+
+@pytest.mark.parametrize("singles,KVH", [(12, 8), (3, 32), (33, 4)])
+@pytest.mark.parametrize("window", [0, 1600])
+def test_even_shares_beside_a_prompt(singles, KVH, window):
+    """Single tokens of 65 to 191 pairs beside a prompt: parts by the lengths of
+    all single tokens, against float64; tickets are zero again."""
+    from ollamamq_amd.ops import hip
+    hip.require()
+    torch.manual_seed(8)
+    G, page = 2, 16
+    lens = [300 + i * 2700 // (singles - 1) for i in range(singles)]
+    q_lens, kv_lens = [1] * singles + [70], lens + [200]
+    assert 64 < singles * KVH < 192
+    assert hip._decode_split(singles * KVH, max(kv_lens)) > 1
+    cache = PagedKVCache(1, KVH, D, page_size=page,
+                         n_pages=sum(n // page + 1 for n in kv_lens),
+                         max_slots=len(kv_lens), max_ctx=3072, device="cuda",
+                         dtype=torch.bfloat16)
+    slots = [cache.alloc_slot() for _ in kv_lens]
+    for s, n in zip(slots, kv_lens):
+        cache.ensure(s, n)
+    cache.k_pool.normal_()
+    cache.v_pool.normal_()
+    q = torch.randn(sum(q_lens), G * KVH, D, device="cuda").bfloat16()
+    sem = torch.zeros(len(kv_lens) * KVH, dtype=torch.int32, device="cuda")
+    first = None
+    for _ in range(2):
+        got = hip.attention_mixed(q, cache, 0, _meta(
+            slots, q_lens, kv_lens, singles, window), sem=sem)
+        assert not sem.any()
+        assert first is None or torch.equal(first, got)
+        first = got
+    for i, n in enumerate(lens):
+        pages = cache.page_table[slots[i], :-(-n // page)].long()
+        k, v = (p[0][pages].transpose(1, 2).flatten(0, 1)[:n].double()
+                for p in (cache.k_pool, cache.v_pool))
+        lo = max(0, n - window) if window else 0
+        s = torch.einsum("hgd,nhd->hgn", q[i].double().view(KVH, G, D),
+                         k[lo:]) / D ** 0.5
+        want = torch.einsum("hgn,nhd->hgd", s.softmax(-1), v[lo:])
+        # one rounding to bf16, and fp32 sums
+        torch.testing.assert_close(got[i].double(), want.flatten(0, 1),
+                                   rtol=2 ** -8, atol=1e-5)
