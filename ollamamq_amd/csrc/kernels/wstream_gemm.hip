@@ -1323,12 +1323,13 @@ extern "C" int wstream_duo_bf16(
 // rows: 15.1 us in 8 parts, 22.1 in 32 of 64 columns).  Blocks of 16 columns load
 // what K of 768 takes even if it is less (4096 x 256, 32 rows: 4.5 us streamed,
 // 5.1).  Over 12 numbers of columns from 512 to 8192, 16 of K from 128 to 28672 and
-// 8 of rows from 1 to 64 the choice takes 1.8 % more than the best of the three,
+// 8 of rows from 1 to 64 the choice takes 1.9 % more than the best of the three,
 // parts (tiles in parts from 49 rows on) alone 13 %, 16 columns alone 21 %, and at
 // most 2.7 % more than parts.
-// From 49 rows on the parts are of tiles, which take the time of 360 KB more: they
-// use CUs that fewer than 2048 columns leave without a block, and are no slower
-// than 64 columns.
+// From 49 rows on the parts are of tiles, which use CUs that fewer than 2048
+// columns leave without a block, and are no slower than 64 columns; at the price
+// of 256 KB the choice keeps tiles for 4096 x 5632, 56 rows, of 17.1 us where 16
+// columns take 15.1, and takes 16 columns nowhere that they are slower.
 extern "C" int wstream_residual(int M, int N, int K, int ksplit)
 {
     if (M < 1 || N < 32 || N % 32 || K < 64 || K % 64 || ksplit < 1) return -104;
@@ -1341,7 +1342,7 @@ extern "C" int wstream_residual(int M, int N, int K, int ksplit)
             (blocks + 255) / 256 * (k / parts) * 2 * (columns + rows),
             1.4 / 128 * N * K);
     };
-    const int sums = M > 48 ? 360 : M > 32 ? 270 : 200;
+    const int sums = M > 48 ? 256 : M > 32 ? 270 : 200;
     const int64_t whole = load(16, 1, std::max(K, 768));
     const int64_t parts = load(32, ksplit, K) + (ksplit > 1 ? sums << 10 : 0);
     int64_t least = std::min(whole, parts);
