@@ -926,11 +926,17 @@ static int wide(int cw, void* y, const void* x, const void* wp, int M, int N,
 // wave's load takes whole lines here too: columns 16 h to 16 h + 15 of a tile, or,
 // where a rotation pairs columns, 8 h to 8 h + 7 of both its halves.
 // Rows are asked for as far ahead as weights, as loads return in order; four
-// steps are as fast as six or eight, in registers for three blocks a CU.
+// steps are as fast as six or eight, in registers for two blocks a CU of up to 32
+// rows, with rotation for three.
 // ROPE: norm (none without rstd_parts), rotation and append as k_wstream_gemm has
 // them, else residual and sums of squares.
-template <int RT, bool ROPE>
-__global__ __launch_bounds__(512, RT == 1 ? 6 : RT == 2 ? 4 : 2) void k_narrow(
+// A sums a wave, of every A-th step: with those of eight waves no fewer than the
+// parts of a stream have, as a longer sum rounds more.  rms of what sums of K
+// products of size one are off by, 4096 columns, streamed, with one sum a wave and
+// with four: K of 4096 6.0e-6, 7.8e-6, 4.8e-6; of 14336 2.0e-5, 2.8e-5, 1.5e-5.
+// Neither is faster than the other.
+template <int RT, int A, bool ROPE>
+__global__ __launch_bounds__(512, ROPE ? 6 : RT == 1 || A == 2 ? 4 : 2) void k_narrow(
     bf16* y, const u32x4* __restrict__ x, const u32x4* __restrict__ wp,
     const bf16* __restrict__ bias, int M, int N, int K,
     const float* __restrict__ rstd_parts, int rstd_nt, float inv_h, float eps,
@@ -957,7 +963,7 @@ __global__ __launch_bounds__(512, RT == 1 ? 6 : RT == 2 ? 4 : 2) void k_narrow(
     }
     const Global wq = (Global)(wp + (int64_t)t * NB * 256), xq = (Global)x;
     u4bf8 w[D][2], xr[D][RT][2];
-    f32x4 acc[RT] = {};
+    f32x4 acc[A][RT] = {};
     auto step = [](Global p, int b) {
         Global q = p + (int64_t)b * 4096;
         asm("" : "+s"(q));                    // no address per lane
@@ -980,12 +986,14 @@ __global__ __launch_bounds__(512, RT == 1 ? 6 : RT == 2 ? 4 : 2) void k_narrow(
         for (int a = 0; a < 2; a++)
             #pragma unroll
             for (int m = 0; m < RT; m++)
-                acc[m] = mma(xr[s][m][a].v, w[s][a].v, acc[m]);
+                acc[s % A][m] = mma(xr[s][m][a].v, w[s][a].v,
+                                    acc[s % A][m]);
     };
     #pragma unroll
     for (int s = 0; s < D; s++) load(s, min(lo + s, last));
     // this thread's results, of rows 32 apart, and what they need besides the sums
-    constexpr int RR = (RT + 1) / 2, FL = RT > 2 ? 8 : 512 / (RT * 16);
+    static_assert(RT == 1 || !ROPE);
+    constexpr int RR = (RT + 1) / 2, FL = 32;
     const int row = threadIdx.x >> 4, col = threadIdx.x & 15;
     const int n16 = blockIdx.x * 16 + col;
     float add[RR] = {}, rsum = 0.f;
@@ -1035,9 +1043,15 @@ __global__ __launch_bounds__(512, RT == 1 ? 6 : RT == 2 ? 4 : 2) void k_narrow(
     __shared__ float red[8][RT * 16][20];
     __shared__ float rstd_s[RT * 16];
     #pragma unroll
-    for (int m = 0; m < RT; m++)
+    for (int m = 0; m < RT; m++) {
         #pragma unroll
-        for (int i = 0; i < 4; i++) red[wid][m * 16 + g * 4 + i][r] = acc[m][i];
+        for (int n = 1; n < A; n *= 2)
+            #pragma unroll
+            for (int s = 0; s + n < A; s += 2 * n) acc[s][m] += acc[s + n][m];
+        #pragma unroll
+        for (int i = 0; i < 4; i++)
+            red[wid][m * 16 + g * 4 + i][r] = acc[0][m][i];
+    }
     if (ROPE) {
         #pragma unroll
         for (int o = FL / 2; o; o >>= 1) rsum += __shfl_down(rsum, o, 64);
@@ -1101,10 +1115,11 @@ extern "C" int wstream_narrow_bf16(
     if (M < 1 || M > 64 || N < 32 || N % 32 || K < 64 || K % 64 || !res_in
         || !sq_parts)
         return -104;
-    (M <= 16   ? k_narrow<1, false>
-     : M <= 32 ? k_narrow<2, false>
-     : M <= 48 ? k_narrow<3, false>
-               : k_narrow<4, false>)<<<N / 16, 512, 0, stream>>>(
+    // of more than 4096 columns, a block a CU, streams have two parts at most
+    (M <= 16   ? k_narrow<1, 4, false>
+     : M <= 32 ? N > 4096 ? k_narrow<2, 2, false> : k_narrow<2, 4, false>
+     : M <= 48 ? k_narrow<3, 4, false>
+               : k_narrow<4, 4, false>)<<<N / 16, 512, 0, stream>>>(
         (bf16*)y, (const u32x4*)x, (const u32x4*)wp, nullptr, M, N, K, nullptr,
         0, 0.f, 0.f, (const bf16*)res_in, (float*)sq_parts, RopeEpi{});
     return (int)hipGetLastError();
@@ -1597,7 +1612,7 @@ extern "C" int wstream_qkv_rope_bf16(
     const int d = frag_depth(M, N, K, 1);
     if (M > (xf ? 128 : 32)) return -104;          // rows of a block
     if (xf && rope_narrow(M, N, K)) {
-        k_narrow<1, true><<<N / 16, 512, 0, stream>>>(
+        k_narrow<1, 1, true><<<N / 16, 512, 0, stream>>>(
             (bf16*)y, (const u32x4*)x, (const u32x4*)wp, (const bf16*)bias, M, N,
             K, (const float*)rstd_parts, rstd_nt, inv_h, eps, nullptr, nullptr,
             rp);
