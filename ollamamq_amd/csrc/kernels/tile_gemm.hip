@@ -1093,15 +1093,15 @@ extern "C" int tile_gemm_plan(int M, int N, int K, int epi, int cus)
 // A gated or rotated product of several rounds of tiles in two: as many of its
 // rows as fill whole rounds of one size of tile, and the others over tiles of
 // their own.  In one a last round takes as long whatever it has (2310 rows of
-// 28672 x 4096 over 7 x 7 tiles: 5.5 rounds, 429 us; 1792 rows, four rounds, and
-// 518 over 9 x 7, one: 399).  us in one and in two:
-//                    rows   1000       1600       2310       3000       4500
-//   28672 x 4096          189 182    284 271    429 399    522 502    746 726
-//   37888 x 3584          244 233               495 474               913 883
-//   22016 x 4096                     237 225               406 395    618 589
-// A second launch takes 9 us by the estimate's measure: over 37 random numbers of
-// rows and four matrices, those of 9 us and 1 % less take 4 % less on average, the
-// others between 3 % more and 3 % less.
+// 28672 x 4096 over 7 x 7 tiles: 5.5 rounds, 449 us; 576 rows over 9 x 7, one
+// round, and 1734 over 7 x 7, four: 412).  us in one and in two:
+//                    rows   1600       2310       3000       4500
+//   28672 x 4096          296 283    449 412    539 522
+//   37888 x 3584                     510 488
+//   22016 x 4096          247 232               436 417    633 610
+// A second launch takes 9 us by the estimate's measure, and two are to take 1 %
+// less.  Over 96 random numbers of rows from 129 to 8192 and 12 matrices, 156 go in
+// two and take 4.5 % less on average; five take 0.6 to 3.7 % more.
 // Rows of the first | its tile << 24 | the others' tile << 40, each hm | hn << 8,
 // or 0 for one launch.
 extern "C" int64_t tile_gemm_split(int M, int N, int K, int epi, int cus)

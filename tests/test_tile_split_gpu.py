@@ -16,8 +16,8 @@ M, K = 301, 256
 
 @pytest.mark.parametrize("cus", [32, 256, 304])
 def test_plans_cover_the_rows(cus):
-    """What is chosen has every row once, tiles that there are, whole tiles in
-    the first launch, and not more rounds of them than one launch has."""
+    """What is chosen has every row once, tiles that there are, and in the first
+    launch whole tiles and rounds that are nearly full."""
     hip.require()
     two = 0
     for N, K in ((28672, 4096), (37888, 3584), (16384, 2048), (12288, 4096),
@@ -46,6 +46,28 @@ def test_plans_cover_the_rows(cus):
                 (129, 64, 128, 0, 256), (0, 64, 128, 1, 256),
                 (129, 64, 128, 1, 0)):
         assert hip._lib.tile_gemm_split(*bad) == 0
+
+
+@pytest.mark.parametrize("N, K, epi, M, plans", [
+    # us in one launch and in two
+    (28672, 4096, 1, 1600, [(9, 7), (7, 7)]),              # 296 283
+    (28672, 4096, 1, 2310, [(9, 7), (7, 7)]),              # 449 412
+    (28672, 4096, 1, 3000, [(9, 7), (8, 6)]),              # 539 522
+    (37888, 3584, 1, 2310, [(9, 7), (7, 7)]),              # 510 488
+    (22016, 4096, 1, 1600, [(7, 7), (8, 6)]),              # 247 232
+    (22016, 4096, 1, 4500, [(7, 7), (8, 6)]),              # 633 610
+    (6144, 4096, 2, 6451, [(8, 8), (8, 6)]),               # 9 % less in two
+    # last rounds that are nearly full, or a launch's price
+    (28672, 4096, 1, 541, [(9, 7)]), (28672, 4096, 1, 2048, [(8, 6)]),
+    (28672, 4096, 1, 4500, [(9, 7)]), (28672, 4096, 1, 8100, [(8, 8)]),
+    (37888, 3584, 1, 1600, [(9, 7)]), (37888, 3584, 1, 8100, [(8, 8)]),
+    (22016, 4096, 1, 2310, [(6, 6)]), (6144, 4096, 2, 2310, [(8, 8)]),
+    (12288, 4096, 2, 1600, [(10, 4)]), (12288, 4096, 2, 8100, [(8, 8)]),
+])
+def test_which_go_in_two(N, K, epi, M, plans):
+    hip.require()
+    assert (hip.TILE_GATED, hip.TILE_ROPE) == (1, 2)
+    assert [p[2][:2] for p in hip.tile_plans(M, N, K, epi, 256)] == plans
 
 
 def frag(x):
