@@ -772,20 +772,15 @@ def row_sumsq(x, out=None):
     return s
 
 
-def linear_fused(x, packed, N, bias=None, rstd=None, rstd_nt=0,
-                 inv_h=0.0, eps=0.0, res=None, sq_out=None, y=None,
-                 yfrag=0, K=None, xlds=None, M_frag=32, sem=None):
-    """Weight-streaming GEMM with the fused-chain epilogue/prologue:
-    optional rmsnorm scaling of the raw-residual input (norm weight
-    folded into the pack), in-place residual add (pass y=res) and
-    sum-of-squares partial emission for the next GEMM's rstd.
-    K given => x is a 32-row frag-layout buffer streamed linearly;
-    yfrag => the output is emitted in frag layout; sem: see
-    hip.linear_packed."""
-    return hip.linear_packed(x, packed, bias, N, rstd=rstd,
-                             rstd_nt=rstd_nt, inv_h=inv_h, eps=eps,
-                             res=res, sq_out=sq_out, y=y, yfrag=yfrag,
-                             K=K, xlds=xlds, M_frag=M_frag, sem=sem)
+def linear_fused(x, packed, N, rstd=None, rstd_nt=0, inv_h=0.0, eps=0.0,
+                 K=None, xlds=None, M_frag=32):
+    """Streamed product of normed rows, the head's in the fused chain: rstd,
+    rstd_nt, inv_h and eps scale the rows of the raw residual stream x (the
+    norm's weight is folded into the pack).  K given => x is a 32-row
+    frag-layout buffer."""
+    return hip.linear_packed(x, packed, None, N, rstd=rstd, rstd_nt=rstd_nt,
+                             inv_h=inv_h, eps=eps, K=K, xlds=xlds,
+                             M_frag=M_frag)
 
 
 def residual_parts(M, N, K) -> int:
