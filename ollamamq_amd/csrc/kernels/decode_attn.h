@@ -20,18 +20,21 @@
 // Weights stay fp32: they enter the product with the values as three bf16
 // terms, which hold all 24 bits.
 //
-// Bound by memory: 4.9 to 5.3 TB/s over large caches, where a device copy makes
-// 4.7; the loads alone take 1 to 2 % less.  us, with keys and values loaded to
-// registers in operand order, and so (32 heads, 8 of them key/value heads, unless
-// said):
+// Bound by memory: 4.9 to 5.4 TB/s over large caches, where a device copy makes
+// 4.7.  us, with keys and values loaded to registers in operand order, and so (32
+// heads, 8 of them key/value heads, unless said):
 //   one user, 300 tokens                        7.4, now 6.4
-//   32 users, 256 to 768                       18.1, now 17.3
-//   128 users, 350 to 1050                     72.2, now 71.1
-//   12 users, 4096 to 12288                    86.2, now 82.6
-//   24 users, 1000 to 3000                     47.7, now 45.0
-//   48 users, 300 to 900, 28 / 4 heads         19.0, now 18.1
-//   24 users, 550 to 1650, 32 / 32 heads       81.1, now 81
-//   24 users, 1000 to 3000, pages of 24 tokens  54.7, now 48.4
+//   32 users, 256 to 768                       17.8, now 16.7
+//   128 users, 350 to 1050                     70.2, now 68.3
+//   12 users, 4096 to 12288                    84.8, now 81.5
+//   24 users, 1000 to 3000                     46.6, now 43.2
+//   48 users, 300 to 900, 28 / 4 heads         18.7, now 17.4
+//   24 users, 550 to 1650, 32 / 32 heads       78.7, now 77.1
+//   24 users, 1000 to 3000, pages of 24 tokens  52.8, now 46.2
+// Contexts of one step lose: 16 tokens, one user 3.9, now 4.2, 128 users 12.3, now
+// 13.0.  A block's 128 KB of LDS keep the next one from starting while the last
+// waves merge (the other kernel with as much: 12.8); the rest is not known, and
+// is neither the loads' way through LDS nor what comes before them.
 // A wave's steps one after the other and heads dealt to the XCDs in turn are 1 to
 // 3 % slower; whole lines of 8 rows an instruction, put right in registers, no
 // faster than operand order.
@@ -93,12 +96,18 @@ DEV void decode_block(
     // 300 tokens of one user 0.9 us).  With cus, an even share, for a block a CU,
     // of what all sequences have: short contexts stay whole, where parts of 8
     // steps made up to 768 blocks with as many ends, and long ones take no longer
-    // than the rest.  us with 8 steps and so (ragged, key/value heads): 12 users of
-    // 800 tokens, 8 heads 16.8, 14.1; 16 of 1500 27.7, 24.7; 20 of 600 18.4, 15.0;
-    // 45 of 600, 4 heads 20.3, 16.2; 5 of 1000, 32 heads 23.9, 20.1.  Shares of 36
-    // and more end too far apart: 12 of 8192 took 88 us for 82.  Finding the share
-    // takes 0.4 us, so contexts of less than two parts and of 100 steps and more,
-    // whose share is seldom less than that, go without.
+    // than the rest.  So the order of a sequence's sums depends on the lengths of
+    // those beside it, as the most parts do on their number and longest context.
+    // us with 8 steps and so (ragged, key/value heads), of batches as decode steps
+    // pad them: 12 users of 800 tokens, 8 heads 17.2, 14.2; 16 of 600 16.7, 14.1;
+    // 16 of 1500 28.1, 25.5; 24 of 800, 4 heads 17.7, 14.5; 32 of 1500 28.8, 25.9;
+    // 3 of 1000, 32 heads 18.0, 15.3; beside prompts, where they are not padded, 20
+    // of 600, 8 heads 18.4, 15.0; 45 of 600, 4 heads 20.0, 15.7.  Over 17 batches
+    // and 15 lengths from 100 to 4000 5 % less on average, and more in one case
+    // (4 of 500, 32 heads 12.2, 13.7).  Shares of 36 and more end too far apart: 12
+    // of 8192 took 88 us for 82.  Finding the share takes 0.2 to 0.4 us, so contexts
+    // of less than two parts and of 100 steps and more, whose share is seldom less
+    // than that, go without.
     if (z > 0 && z >= steps / least) return;
     if (split > 1 && cus && steps >= 2 * least && steps < 100) {
         auto steps_of = [&](int n) {

@@ -104,8 +104,9 @@ __global__ __launch_bounds__(NW * 64, 2) void k_prefill_attn(
 // prompt joins a few users, and each is a latency of its own (24 users of 400
 // to 1200 tokens and a prompt of 517 within a step: 24 and 19 us one after the
 // other, 30 together).  Blocks of prompts come first, the longest walks, and
-// the later parts of a context, of which there may be none, last; registers
-// leave one block of eight waves a CU, as decode alone has.
+// the later parts of a context, of which there may be none, last; registers and
+// the 128 KB of LDS that decode takes leave one block of eight waves a CU, as
+// decode alone has.
 template <bool SH>
 __global__ __launch_bounds__(512, 2) void k_mixed_attn(
     bf16* __restrict__ out, float* __restrict__ o_part,

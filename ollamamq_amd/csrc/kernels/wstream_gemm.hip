@@ -1308,7 +1308,8 @@ __global__ __launch_bounds__(512, 1) void k_duo(
 
 // y = x W^T + res_in, both in fragment layout (they may be one), in `ksplit` parts
 // of K; part: as many times the floats of N columns of whole row tiles; sem: zeros,
-// one per 64 columns, zero again at the end; sq_parts: N / 64 sums of squares a row
+// one per 64 columns, zero again at the end; sq_parts: N / 64 sums of squares a row.
+// wstream_residual takes it for up to 48 rows in two parts and more.
 extern "C" int wstream_duo_bf16(
     void* y, void* part, const void* x, const void* wp, int M, int N, int K,
     int ksplit, const void* res_in, void* sq_parts, void* sem,

@@ -495,13 +495,15 @@ class LlamaModel:
         nt = 1                      # embed stats = one partial tile
         inv_h = 1.0 / H
         eps = cfg.norm_eps
-        # From 49 rows on o and down go over tiles in parts of K: a block of
-        # k_wstream_gemm loads all rows for 32 columns.  us of a step, four
-        # layers, streams and tiles for o and down:
-        #                48 users      64         96         128
-        #   llama3-8b   531   546   559   560   662   646   740   711
-        #   qwen2-7b    586   592   618   608   731   709   816   777
-        #   llama2-13b  836   774   935   831  1163  1013  1360  1154
+        # From 49 rows on o and down go over tiles in parts of K, as a block of
+        # k_wstream_gemm loads all rows for 32 columns; of up to 64 rows some go in
+        # blocks of 16 columns and no parts (4096 x 4096, 64 rows: 13.6 us
+        # streamed, 15.7 over tiles, 12.8 so).  us of a step, four layers,
+        # streams and tiles for o and down:
+        #                96 users      128
+        #   llama3-8b   662   646   740   711
+        #   qwen2-7b    731   709   816   777
+        #   llama2-13b 1163  1013  1360  1154
         # So do rotated products of which the streams need a second round of
         # blocks (49 and 128 rows: 9216 x 4096 31 and 50 us against 30 and 36,
         # 12288 x 4096 33 and 51 against 31 and 37, 9216 x 2048 20 and 32 against
