@@ -8,14 +8,16 @@
 //
 // Every wave walks its own steps of 32 keys with its own maximum and sum, and
 // nothing is shared before the one merge at the end:
-//  * keys and values go straight to LDS of the wave's own, a step ahead, 16 KB
-//    under way per wave, in whole rows, four of them an instruction.  A key row is
-//    the row operand of mfma_16x16x32; loaded to registers in that form, 16 lanes
-//    touch 16 lines for 16 bytes each;
-//  * values are read as they were loaded and turned in registers: a lane holds
-//    columns 8c..8c+7 of the eight keys whose weights it holds, and 32 byte
-//    permutes make of them the operands of eight value tiles (tile v has the
-//    columns 8c + v);
+//  * keys and values are loaded a step ahead, 16 KB under way per wave, in whole
+//    rows, four of them an instruction: keys straight to LDS of the wave's own.  A
+//    key row is the row operand of mfma_16x16x32; loaded to registers in that
+//    form, 16 lanes touch 16 lines for 16 bytes each;
+//  * values are turned in registers: a lane holds columns 8c..8c+7 of the eight
+//    keys whose weights it holds, and 32 byte permutes make of them the operands
+//    of eight value tiles (tile v has the columns 8c + v).  With pages of 16, 32,
+//    64, ... tokens they come as they lie; with others through LDS as well, as
+//    the compiler waits for all loads to LDS by 64 bit addresses before it uses a
+//    register that was loaded;
 //  * page numbers are looked up for many steps at once, a lane each.
 // Weights stay fp32: they enter the product with the values as three bf16
 // terms, which hold all 24 bits.
@@ -23,22 +25,24 @@
 // Bound by memory: 4.9 to 5.4 TB/s over large caches, where a device copy makes
 // 4.7.  us, with keys and values loaded to registers in operand order, and so (32
 // heads, 8 of them key/value heads, unless said):
-//   one user, 300 tokens                        7.4, now 6.4
-//   32 users, 256 to 768                       17.8, now 16.7
-//   128 users, 350 to 1050                     70.2, now 68.3
-//   12 users, 4096 to 12288                    84.8, now 81.5
-//   24 users, 1000 to 3000                     46.6, now 43.2
-//   48 users, 300 to 900, 28 / 4 heads         18.7, now 17.4
-//   24 users, 550 to 1650, 32 / 32 heads       78.7, now 77.1
-//   24 users, 1000 to 3000, pages of 24 tokens  52.8, now 46.2
-// Contexts of one step lose: 16 tokens, one user 3.9, now 4.2, 128 users 12.3, now
-// 13.0.  A block's 128 KB of LDS keep the next one from starting while the last
-// waves merge (the other kernel with as much: 12.8); the rest is not known, and
-// is neither the loads' way through LDS nor what comes before them.
+//   one user, 300 tokens                        7.4, now 5.9
+//   32 users, 256 to 768                       17.8, now 16.4
+//   128 users, 350 to 1050                     70.6, now 68.0
+//   12 users, 4096 to 12288                    84.4, now 81.0
+//   24 users, 1000 to 3000                     46.6, now 42.7
+//   48 users, 300 to 900, 28 / 4 heads         18.7, now 16.9
+//   24 users, 550 to 1650, 32 / 32 heads       78.4, now 77.4
+//   24 users, 1000 to 3000, pages of 24 tokens  52.7, now 45.0
+// With values through LDS too, 128 KB a block, the next one does not start while
+// the last waves merge (128 users of 8 to 24 tokens 13.0, now 11.8, loaded to
+// registers 12.3; 32 heads, 68 users of 86 to 257 53.6, 50.7, 53.3).  Contexts of
+// one step are up to 0.2 us slower than with loads to registers where only few
+// blocks have them (28 / 4 heads, one user 3.9, now 4.1).
 // A wave's steps one after the other and heads dealt to the XCDs in turn are 1 to
 // 3 % slower; whole lines of 8 rows an instruction, put right in registers, no
 // faster than operand order.
 #pragma once
+#include <type_traits>
 #include "flash32.h"
 
 // two floats that other blocks write or read in the same launch
@@ -58,8 +62,8 @@ DEV float2 get2(const float* p) {
 // Pages: with SH they are 1 << pshift tokens and no smaller than a tile of
 // 16 keys, so a tile's page number is the same for the whole wave; otherwise
 // any number of tokens, and every key has its own.
-// smem: DECODE_LDS bytes
-constexpr int DECODE_LDS = 8 * 2 * 32 * 128 * 2;
+// smem: decode_lds bytes, for a wave 32 keys and, without SH, values
+constexpr int decode_lds(bool sh) { return 8 * (sh ? 1 : 2) * 32 * 128 * 2; }
 
 template <bool SH>
 DEV void decode_block(
@@ -99,12 +103,12 @@ DEV void decode_block(
     // than the rest.  So the order of a sequence's sums depends on the lengths of
     // those beside it, as the most parts do on their number and longest context.
     // us with 8 steps and so (ragged, key/value heads), of batches as decode steps
-    // pad them: 12 users of 800 tokens, 8 heads 17.2, 14.2; 16 of 600 16.7, 14.1;
-    // 16 of 1500 28.1, 25.5; 24 of 800, 4 heads 17.7, 14.5; 32 of 1500 28.8, 25.9;
-    // 3 of 1000, 32 heads 18.0, 15.3; beside prompts, where they are not padded, 20
-    // of 600, 8 heads 18.4, 15.0; 45 of 600, 4 heads 20.0, 15.7.  Over 17 batches
+    // pad them: 12 users of 800 tokens, 8 heads 16.7, 13.9; 16 of 600 16.5, 13.8;
+    // 16 of 1500 27.6, 25.2; 24 of 800, 4 heads 17.1, 14.2; 32 of 1500 28.2, 25.6;
+    // 3 of 1000, 32 heads 17.9, 15.1; beside prompts, where they are not padded, 20
+    // of 600, 8 heads 18.0, 14.6; 45 of 600, 4 heads 19.6, 15.4.  Over 17 batches
     // and 15 lengths from 100 to 4000 5 % less on average, and more in one case
-    // (4 of 500, 32 heads 12.2, 13.7).  Shares of 36 and more end too far apart: 12
+    // (4 of 500, 32 heads 12.0, 13.3).  Shares of 36 and more end too far apart: 12
     // of 8192 took 88 us for 82.  Finding the share takes 0.2 to 0.4 us, so contexts
     // of less than two parts and of 100 steps and more, whose share is seldom less
     // than that, go without.
@@ -126,12 +130,13 @@ DEV void decode_block(
     const int GW = parts * NW;            // a wave's steps: every GW-th
 
     // a wave's own: 32 keys and values, in the end its G results, maxima and sums
-    constexpr int OWN = KT * D;           // floats
+    constexpr int OWN = decode_lds(SH) / NW / 4;      // floats
     float* o_s = reinterpret_cast<float*>(smem);
     char* keys = smem + wid * OWN * 4;
     char* values = keys + KT * D * 2;
 
     bf16x8 qf[4];
+    u32x4 vr[8];
     const bf16* qr = q + seq * qs + (kvh * G + min(lr, G - 1)) * D + g * 8;
     #pragma unroll
     for (int d = 0; d < 4; d++) qf[d] = frag8(qr + d * 32);
@@ -161,28 +166,36 @@ DEV void decode_block(
             pg[e] = __shfl(book, j * per + key_of(st, e) / page
                                      - (first + st) * KT / page, 64);
     };
+    // SH: tile t of a step, 16 keys of one page, has an address of the wave's and
+    // 32 bits a lane (64 bits a lane, many users of 150 to 600 tokens: 2 %
+    // slower).  One past the last key takes the last's tile.
+    auto tile_of = [&](int st, int t) {
+        return min((first + st) * KT + t * 16, last & ~15);
+    };
+    auto tile_at = [&](const bf16* pool, int st, int t) {
+        return pool + ((((int64_t)pg[t] * KVH + kvh) << pshift)
+                       + (tile_of(st, t) & ((1 << pshift) - 1))) * D;
+    };
+    auto row_of = [&](int st, int t, int i) -> unsigned {
+        const int tile = tile_of(st, t);
+        return min((first + st) * KT + t * 16 + i - tile, last - tile);
+    };
     auto to_lds = [&](const bf16* pool, int st, int e, int piece, char* to) {
-        typedef __attribute__((address_space(1))) const char* Global;
-        Global from;
-        if (SH) {
-            // A tile of 16 keys lies in one page: an address of the wave's and
-            // 32 bits a lane (64 bits a lane, many users of 150 to 600 tokens:
-            // 2 % slower).  One past the last key takes the last's tile.
-            const int at = (first + st) * KT + (e >> 2) * 16;
-            const int tile = min(at, last & ~15);
-            from = (Global)(pool + ((((int64_t)pg[e >> 2] * KVH + kvh) << pshift)
-                                    + (tile & ((1 << pshift) - 1))) * D);
-            asm("" : "+s"(from));
-            const unsigned row = min((e & 3) * 4 + g + at - tile, last - tile);
-            from += row * 256u + piece * 16u;
-        } else {
+        auto* lds = (__attribute__((address_space(3))) void*)(to + e * 1024);
+        if constexpr (SH)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                __builtin_amdgcn_make_buffer_rsrc(
+                    (void*)tile_at(pool, st, e >> 2), 0, 16 * D * 2, 0x27000),
+                lds, 16, row_of(st, e >> 2, (e & 3) * 4 + g) * 256 + piece * 16,
+                0, 0, 0);
+        else {
             const int key = key_of(st, e);
-            from = (Global)(pool + (((int64_t)pg[e] * KVH + kvh) * page
-                                    + key % page) * D + piece * 8);
+            __builtin_amdgcn_global_load_lds(
+                (const __attribute__((address_space(1))) void*)(
+                    pool + (((int64_t)pg[e] * KVH + kvh) * page + key % page) * D
+                    + piece * 8),
+                lds, 16, 0, 0);
         }
-        __builtin_amdgcn_global_load_lds(
-            (const __attribute__((address_space(1))) void*)from,
-            (__attribute__((address_space(3))) void*)(to + e * 1024), 16, 0, 0);
     };
     // The loads of keys and of values take turns and their waits count them, so
     // none may pass another; and a buffer has been read before it is loaded again.
@@ -204,8 +217,22 @@ DEV void decode_block(
     };
     auto load_v = [&](int st) {
         in_order();
-        #pragma unroll
-        for (int e = 0; e < 8; e++) to_lds(vpool, st, e, lr, values);
+        if constexpr (SH) {
+            typedef __attribute__((address_space(1))) const char* Global;
+            typedef __attribute__((address_space(1))) const u32x4* Global16;
+            #pragma unroll
+            for (int t = 0; t < 2; t++) {
+                Global from = (Global)tile_at(vpool, st, t);
+                asm volatile("" : "+s"(from));        // known after the keys
+                #pragma unroll
+                for (int e = 0; e < 4; e++)
+                    vr[t * 4 + e] = *(Global16)(
+                        from + (row_of(st, t, g * 4 + e) * 256 + lr * 16));
+            }
+        } else {
+            #pragma unroll
+            for (int e = 0; e < 8; e++) to_lds(vpool, st, e, lr, values);
+        }
         in_order();
     };
     // all but the last n loads have come
@@ -218,22 +245,10 @@ DEV void decode_block(
 
     float m = NEG, l = 0.f;
     f32x4 acc[8] = {};
-    if (st < steps) {
-        if (SH) {
-            // the first step's pages as scalars: a short context has no others
-            #pragma unroll
-            for (int t = 0; t < 2; t++)
-                pg[t] = pt[min((first + st) * KT + t * 16, last) >> pshift];
-        } else
-            pages(st, 0);
-        // what the loop takes from registers is there before its loads
-        #pragma unroll
-        for (int d = 0; d < 4; d++) asm volatile("" : "+v"(qf[d]));
-        load_k(st);
-        load_v(st);
-    }
-    for (int j = SH ? 0 : 1 % many; st < steps; st += GW, j = j + 1 < many ? j + 1 : 0) {
-        const bool more = st + GW < steps;
+    // The last step has code of its own, so that the compiler knows what is under
+    // way behind the values: its waits for them count too.
+    auto step = [&](auto another, int j) {
+        constexpr bool more = decltype(another)::value;
         ARRIVED(8);                // keys
         f32x4 s[2] = {};           // scores
         #pragma unroll
@@ -241,7 +256,7 @@ DEV void decode_block(
             s[0] = mma(key_at(0, d), qf[d], s[0]);
             s[1] = mma(key_at(1, d), qf[d], s[1]);
         }
-        if (more) {
+        if constexpr (more) {
             pages(st + GW, j);
             load_k(st + GW);
         }
@@ -278,13 +293,14 @@ DEV void decode_block(
         l = l * f + sum;                  // of this lane's keys only
         #pragma unroll
         for (int v = 0; v < 8; v++) acc[v] *= f;
-        if (more) ARRIVED(8);
-        else ARRIVED(0);
-        u32x4 vr[8];
-        #pragma unroll
-        for (int e = 0; e < 8; e++)
-            vr[e] = *reinterpret_cast<const u32x4*>(
-                values + ((e >> 2) * 16 + g * 4 + (e & 3)) * 256 + lr * 16);
+        if constexpr (!SH) {
+            if constexpr (more) ARRIVED(8);
+            else ARRIVED(0);
+            #pragma unroll
+            for (int e = 0; e < 8; e++)
+                vr[e] = *reinterpret_cast<const u32x4*>(
+                    values + ((e >> 2) * 16 + g * 4 + (e & 3)) * 256 + lr * 16);
+        }
         #pragma unroll
         for (int v = 0; v < 8; v++) {
             u32x4 a;
@@ -298,7 +314,25 @@ DEV void decode_block(
             acc[v] = mma(af, w1, acc[v]);
             acc[v] = mma(af, w0, acc[v]);
         }
-        if (more) load_v(st + GW);
+        if constexpr (more) load_v(st + GW);
+    };
+    if (st < steps) {
+        if (SH) {
+            // the first step's pages as scalars: a short context has no others
+            #pragma unroll
+            for (int t = 0; t < 2; t++)
+                pg[t] = pt[min((first + st) * KT + t * 16, last) >> pshift];
+        } else
+            pages(st, 0);
+        // what the loop takes from registers is there before its loads
+        #pragma unroll
+        for (int d = 0; d < 4; d++) asm volatile("" : "+v"(qf[d]));
+        load_k(st);
+        load_v(st);
+        for (int j = SH ? 0 : 1 % many; st + GW < steps;
+             st += GW, j = j + 1 < many ? j + 1 : 0)
+            step(std::true_type{}, j);
+        step(std::false_type{}, 0);
     }
     #undef ARRIVED
     l += __shfl_xor(l, 16, 64);

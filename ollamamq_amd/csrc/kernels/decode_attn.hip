@@ -36,9 +36,9 @@ extern "C" int decode_attn_bf16(
     const float unit = scale * 1.4426950408889634f;
     auto go = sh ? k_decode_attn<true> : k_decode_attn<false>;
     const hipError_t ok = hipFuncSetAttribute(
-        (const void*)go, hipFuncAttributeMaxDynamicSharedMemorySize, DECODE_LDS);
+        (const void*)go, hipFuncAttributeMaxDynamicSharedMemorySize, decode_lds(sh));
     if (ok != hipSuccess) return (int)ok;
-    go<<<dim3(KVH, S, split), 512, DECODE_LDS, stream>>>(
+    go<<<dim3(KVH, S, split), 512, decode_lds(sh), stream>>>(
         (bf16*)out, (float*)part, (float*)part + (int64_t)S * Hq * split * 128,
         (int*)sem, (const bf16*)q, (const bf16*)kpool, (const bf16*)vpool,
         (const int*)page_table,

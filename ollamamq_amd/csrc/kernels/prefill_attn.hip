@@ -11,6 +11,7 @@
 //   2048, 32 / 32 heads          1781 us, now 66
 // of which values without bank conflicts and pages a chunk ahead are the last
 // steps, one after another on one card: 474, 103, 26 and 72 us before.
+#include <algorithm>
 #include "decode_attn.h"
 
 constexpr int D = 128;
@@ -104,9 +105,8 @@ __global__ __launch_bounds__(NW * 64, 2) void k_prefill_attn(
 // prompt joins a few users, and each is a latency of its own (24 users of 400
 // to 1200 tokens and a prompt of 517 within a step: 24 and 19 us one after the
 // other, 30 together).  Blocks of prompts come first, the longest walks, and
-// the later parts of a context, of which there may be none, last; registers and
-// the 128 KB of LDS that decode takes leave one block of eight waves a CU, as
-// decode alone has.
+// the later parts of a context, of which there may be none, last; registers
+// leave one block of eight waves a CU, as decode alone has.
 template <bool SH>
 __global__ __launch_bounds__(512, 2) void k_mixed_attn(
     bf16* __restrict__ out, float* __restrict__ o_part,
@@ -190,8 +190,8 @@ extern "C" int mixed_attn_bf16(
         || split < 1 || least < 8 || cus < 0 || (split > 1 && (!part || !sem)))
         return (int)hipErrorInvalidValue;
     const bool sh = page >= 16 && !(page & (page - 1));
-    constexpr int flash = Flash32<D, D, 8, false>::LDS;
-    const int lds = flash > DECODE_LDS ? flash : DECODE_LDS;
+    const int flash = Flash32<D, D, 8, false>::LDS;
+    const int lds = std::max(flash, decode_lds(sh));
     auto go = sh ? k_mixed_attn<true> : k_mixed_attn<false>;
     const hipError_t ok = hipFuncSetAttribute(
         (const void*)go, hipFuncAttributeMaxDynamicSharedMemorySize, lds);

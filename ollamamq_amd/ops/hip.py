@@ -347,11 +347,11 @@ def _decode_split(pairs, max_kv):
     many it takes the kernel says, from all lengths.  Up to 64 pairs, a block a CU
     in all: more parts are more to add up (8 users of 3500 tokens, 8 key/value
     heads: 29 us in 4, 35 in 16).  Up to 191, 768 blocks even out ragged contexts
-    (12 users of 4096 to 12288: 130 us whole, 87 in two, 82 in eight).  From 192
+    (12 users of 4096 to 12288: 128 us whole, 86 in two, 81 in eight).  From 192
     on one part is best where its blocks fill whole rounds of the 256 CUs (32
-    users of about 512 tokens: 17 us); where they do not, long parts fill the last
-    round (34 users of 2500: 68 us against 79 whole, 24 of 4000: 75 against
-    82)."""
+    users of about 512 tokens: 16 us); where they do not, long parts fill the last
+    round (34 users of 2500: 68 us against 78 whole, 24 of 4000: 75 against
+    81)."""
     env = os.environ.get("OLLAMAMQ_DECODE_SPLIT")
     if env:                       # tuning override (tools/perf_decode.py)
         want = int(env)
