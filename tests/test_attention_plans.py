@@ -1,7 +1,9 @@
 """Tiles of prompt attention, built on the host: every grouping of heads and
 every first sequence has its own on one batch."""
+import pytest
 import torch
 
+from ollamamq_amd.engine import PagedKVCache
 from ollamamq_amd.ops import hip
 from ollamamq_amd.ops.interface import AttnMeta
 
@@ -38,3 +40,33 @@ def test_groupings_and_first_sequences_share_a_batch(monkeypatch):
         assert sum(n for *_, n in tiles.tolist()) == len(rows)
         again, _ = hip._prefill_plan(meta, first, G, KVH, "cpu")
         assert again is tiles
+
+
+@pytest.mark.parametrize("singles, KVH, prompt, cus", [
+    (12, 8, 40, 248), (12, 8, 200, 224),    # blocks of 256 rows of four heads
+    (5, 32, 100, 192), (12, 8, 2047, 0),    # as many as there are CUs
+    (8, 8, 40, 0), (24, 8, 40, 0)])         # no shares
+def test_single_tokens_share_what_prompts_leave(singles, KVH, prompt, cus,
+                                                monkeypatch):
+    hip.require()
+    seen = []
+
+    class Spy:
+        def mixed_attn_bf16(self, *args):
+            seen.append(args)
+            return 0
+    monkeypatch.setattr(hip, "_lib", Spy())
+    monkeypatch.setattr(hip, "_cus", lambda index: 256)
+    monkeypatch.setattr(hip, "_stream", lambda: None)
+    monkeypatch.setattr(hip, "upload", lambda values, dev: torch.tensor(
+        values, dtype=torch.int32, device=dev))
+    lens = [300 + 50 * i for i in range(singles)] + [prompt]
+    meta = _meta([1] * singles + [prompt], lens, singles)
+    cache = PagedKVCache(1, KVH, 128, page_size=16, n_pages=4, max_slots=64,
+                         max_ctx=4096, device="cpu", dtype=torch.bfloat16)
+    q = torch.zeros(singles + prompt, 4 * KVH, 128, dtype=torch.bfloat16)
+    hip.attention_mixed(q, cache, 0, meta)
+    n_items, S, split, least, got = seen[0][8], *seen[0][11:15]
+    assert S == singles and least == (48 if singles * KVH >= 192 else 8)
+    assert got == cus
+    assert got in (0, 256 - n_items * KVH)
