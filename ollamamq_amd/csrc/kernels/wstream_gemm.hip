@@ -926,8 +926,9 @@ static int wide(int cw, void* y, const void* x, const void* wp, int M, int N,
 // wave's load takes whole lines here too: columns 16 h to 16 h + 15 of a tile, or,
 // where a rotation pairs columns, 8 h to 8 h + 7 of both its halves.
 // Rows are asked for as far ahead as weights, as loads return in order; four
-// steps are as fast as six or eight, in registers for two blocks a CU of up to 32
-// rows, with rotation for three.
+// steps are as fast as six or eight.  Registers are for two blocks a CU, with
+// rotation for three, and from 33 rows on, and of 17 on up to 4096 columns (no
+// more blocks than CUs), for one.
 // ROPE: norm (none without rstd_parts), rotation and append as k_wstream_gemm has
 // them, else residual and sums of squares.
 // A sums a wave, of every A-th step: with those of eight waves no fewer than the
